@@ -1,0 +1,324 @@
+// 32-bit matrix products on the matrix cores' 32-bit multiply-adds (v_mfma_f32_16x16x4_f32):
+//     C[M,N] = A[M,K] * W[N,K]^T (+ bias[N]) (+ residual[M,N])
+// for row-major operands whose rows start at multiples of 16 bytes (K and the stride of A
+// multiples of 4; gemm_generic.hip has the kernels for any others).  Products and sums are
+// 32-bit throughout: the instruction multiplies and adds 32-bit numbers, unsplit.
+//
+// A wavefront owns TM x TN blocks of 16 tokens x 16 weight rows.  In a block of 16 elements of K lane l holds elements
+// 4 * (l / 16) .. + 3 of weight row l % 16 and of token l % 16; instruction s of the block then multiplies element s of
+// every lane, so it sums the elements 4 q + s, q < 4, which is a permutation of K that both operands share.  Weights as
+// the first operand: acc[j] of lane (r, q) = C[token r][weight row 4 q + j], a 16-byte store.
+//
+// Two kernels:
+//   gemm_f32_few_kernel (up to 16 tokens, bound by reading W once): a workgroup's wavefronts cut K between them and add up
+//     in the order of K; operands straight from memory to registers, two sets of them, so that one set's loads are in
+//     flight while the other is multiplied.  Sixteen sums a result (one an instruction of a set) keep every chain of
+//     additions at 32 to 64 elements: with one chain a wavefront the error is three times as large, at no gain.
+//   gemm_f32_kernel (more tokens, bound by the matrix cores): four wavefronts share a tile's rows through local memory.
+//     A compute unit's caches bring about 18 bytes a cycle: wavefronts that each load the operands of 32 x 32 results for
+//     themselves need 32 and reach half of the matrix cores' rate (2 048 x 16 384 x 2 048: 76 TFLOP/s, straight from
+//     memory or through local memory of their own); a shared tile of 64 x 64 needs 16, of 128 x 128 8.  Where the tiles are
+//     too few to fill the chip K is cut among workgroups, whose sums a second kernel adds in the order of K.
+// Measured against the plain kernels that this replaces (us; floors at 5.05 TB/s and 153 TFLOP/s): 4 tokens 2 048 x 2 048 8.4
+// (floor 3.3), 2 048 x 8 192 28 (13), 16 384 x 2 048 29.5 (27); before 36 for the first two in the mean, and 33.  301
+// tokens 2 048 x 2 048 38 (17), 2 048 x 8 192 116 (66), 3 072 x 2 048 53 (25), 16 384 x 2 048 207 (132); before 746 for
+// the first two in the mean, 301 and 643.  2 048 tokens 16 384 x 2 048 1 115 (898, 123 TFLOP/s).  Errors against 64-bit
+// sums: up to 32 tokens those of the plain kernel (1.2e-7 of the norm at 2 048 elements), beyond at most the plain kernel's.
+#include "common.h"
+
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+struct GemmF32Args {
+  const float* A;
+  int lda;
+  const float* W;
+  float* C;
+  int ldc;
+  const float* residual;
+  int ldr;
+  const float* bias;
+  int M, N, K;
+  float* part;  // [cuts][M][N] sums of K's parts, or null: one part, finished here
+};
+
+// bias and residual, and the store of four neighbouring outputs of a token
+__device__ __forceinline__ void gf_store(const GemmF32Args& a, f4 v, int token, int n) {
+  float* c = a.C + (size_t)token * a.ldc + n;
+  float o[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    o[j] = v[j];
+    if (n + j < a.N) {
+      if (a.bias) o[j] += a.bias[n + j];
+      if (a.residual) o[j] += a.residual[(size_t)token * a.ldr + n + j];
+    }
+  }
+  if (n + 3 < a.N && ((uintptr_t)c & 15) == 0) {
+    *(f4*)c = (f4){o[0], o[1], o[2], o[3]};
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (n + j < a.N) c[j] = o[j];
+  }
+}
+
+#define GF_UNROLL 4  // blocks of 16 elements a set of loads
+
+__global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a) {
+  extern __shared__ __align__(16) f4 sums[];  // [wavefronts - 1][64]
+  // (the wavefront's number as one value for all its lanes, so that its loop counts in scalar registers)
+  const int lane = threadIdx.x & 63, kw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), KS = blockDim.x >> 6;
+  const int r = lane & 15, q = lane >> 4;
+  const int n0 = blockIdx.x * 16;
+  const int blocks = (a.K + 15) >> 4;
+  const int b0 = (int)((long)blocks * kw / KS), b1 = (int)((long)blocks * (kw + 1) / KS);
+  const float* wp = a.W + (size_t)min(n0 + r, a.N - 1) * a.K + 4 * q;
+  const float* ap = a.A + (size_t)min(r, a.M - 1) * a.lda + 4 * q;
+  f4 acc[GF_UNROLL][4];
+#pragma unroll
+  for (int u = 0; u < GF_UNROLL; ++u)
+#pragma unroll
+    for (int s = 0; s < 4; ++s) acc[u][s] = (f4){0.f, 0.f, 0.f, 0.f};
+  f4 w[2][GF_UNROLL], x[2][GF_UNROLL];
+  // (nothing moves across the end of a set's loads: the compiler would else sink each load to its first use and wait there)
+#define GF_LOAD(set, b)                                                                             \
+  do {                                                                                              \
+    _Pragma("unroll") for (int u = 0; u < GF_UNROLL; ++u) {                                         \
+      w[set][u] = *(const f4*)(wp + (size_t)((b) + u) * 16);                                        \
+      x[set][u] = *(const f4*)(ap + (size_t)((b) + u) * 16);                                        \
+    }                                                                                               \
+    __builtin_amdgcn_sched_barrier(0);                                                              \
+  } while (0)
+#define GF_MULTIPLY(set)                                                                            \
+  _Pragma("unroll") for (int u = 0; u < GF_UNROLL; ++u) _Pragma("unroll") for (int s = 0; s < 4; ++s) \
+      acc[u][s] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[set][u][s], x[set][u][s], acc[u][s], 0, 0, 0)
+  const int exact = (a.K & 15) == 0 ? b1 : min(b1, blocks - 1);  // blocks up to here lie inside K whole
+  const int sets = max(exact - b0, 0) / GF_UNROLL;
+  int b = b0;
+  if (sets > 0) {
+    GF_LOAD(0, b);
+    int s = 0;
+#pragma unroll 1
+    for (; s + 2 < sets; s += 2, b += 2 * GF_UNROLL) {
+      GF_LOAD(1, b + GF_UNROLL);
+      GF_MULTIPLY(0);
+      GF_LOAD(0, b + 2 * GF_UNROLL);
+      GF_MULTIPLY(1);
+    }
+    if (s + 1 < sets) {
+      GF_LOAD(1, b + GF_UNROLL);
+      GF_MULTIPLY(0);
+      GF_MULTIPLY(1);
+      b += 2 * GF_UNROLL;
+    } else {
+      GF_MULTIPLY(0);
+      b += GF_UNROLL;
+    }
+  }
+#undef GF_LOAD
+#undef GF_MULTIPLY
+#pragma unroll 1
+  for (; b < b1; ++b) {  // what is left, the last block perhaps cut by K: zeros behind it
+    const bool in = b * 16 + 4 * q < a.K;
+    const long off = in ? (long)b * 16 : -4L * q;
+    f4 wv = *(const f4*)(wp + off), xv = *(const f4*)(ap + off);
+    if (!in) wv = xv = (f4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) acc[0][s] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[s], xv[s], acc[0][s], 0, 0, 0);
+  }
+  f4 part[GF_UNROLL];
+#pragma unroll
+  for (int u = 0; u < GF_UNROLL; ++u) part[u] = (acc[u][0] + acc[u][1]) + (acc[u][2] + acc[u][3]);
+  f4 sum = (part[0] + part[1]) + (part[2] + part[3]);
+  if (KS > 1) {
+    if (kw > 0) sums[(kw - 1) * 64 + lane] = sum;
+    __syncthreads();
+    if (kw > 0) return;
+    for (int k = 0; k < KS - 1; ++k) sum += sums[k * 64 + lane];
+  }
+  if (r < a.M && n0 + 4 * q < a.N) gf_store(a, sum, r, n0 + 4 * q);
+}
+
+#define GS_ROW 36  // floats a row of 32 takes in local memory: 16 lanes that read 16 rows at one place meet 64 different banks
+
+// A workgroup: a tile of 32 TM tokens x 32 TN weight rows, its four wavefronts a quarter each, over the steps of 32 elements
+// of K that its cut (blockIdx.y) has.  A load brings 8 rows' 128 bytes.  Two tiles' rows in local memory: while one is read
+// the next step's, which have been in flight for a step, are written to the other, and the step after that is asked for.
+// CHAINS sums a result, added at the end: 8 for the smallest tile, which then is as exact as the few-row kernel (registers
+// are free there), else 1.
+template <int TM, int TN, int CHAINS>
+__global__ __launch_bounds__(256) void gemm_f32_kernel(GemmF32Args a) {
+  extern __shared__ __align__(16) float tile[];  // [2][32 * (TN + TM)][GS_ROW], weight rows first
+  constexpr int ROWS = 32 * (TN + TM), LOADS = ROWS / 32;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  // Workgroups that share weight rows run on one die (the hardware deals workgroups to the eight dies in turn), so that
+  // those rows pass through one L2: the number is [groups of 8 column tiles][row tiles][column tile within the 8].
+  const int mt = (a.M + 32 * TM - 1) / (32 * TM);
+  const int g = blockIdx.x / 8;
+  const int n0 = ((g / mt) * 8 + blockIdx.x % 8) * 32 * TN, m0 = (g % mt) * 32 * TM;
+  if (n0 >= a.N) return;  // the same for the whole workgroup
+  const int steps = (a.K + 31) >> 5;
+  const int s0 = (int)((long)steps * blockIdx.y / gridDim.y), s1 = (int)((long)steps * (blockIdx.y + 1) / gridDim.y);
+  const int lr = tid >> 3, lc = (tid & 7) * 4;  // load i brings rows 32 i + lr, 16 bytes a lane
+  const float* src[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i)
+    src[i] = i < TN ? a.W + (size_t)min(n0 + 32 * i + lr, a.N - 1) * a.K + lc
+                    : a.A + (size_t)min(m0 + 32 * (i - TN) + lr, a.M - 1) * a.lda + lc;
+  f4 acc[CHAINS][TN][TM];
+#pragma unroll
+  for (int c = 0; c < CHAINS; ++c)
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+      for (int u = 0; u < TM; ++u) acc[c][t][u] = (f4){0.f, 0.f, 0.f, 0.f};
+  f4 next[LOADS];
+  auto load = [&](int s) {
+    if (s * 32 + 32 <= a.K) {
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) next[i] = *(const f4*)(src[i] + (size_t)s * 32);
+    } else {  // K ends inside the step: zeros behind it
+      const bool in = s * 32 + lc < a.K;
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        next[i] = *(const f4*)(src[i] + (in ? (long)s * 32 : -(long)lc));
+        if (!in) next[i] = (f4){0.f, 0.f, 0.f, 0.f};
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // (the compiler would else sink the loads to where they are stored)
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) *(f4*)(tile + ((size_t)buf * ROWS + 32 * i + lr) * GS_ROW + lc) = next[i];
+  };
+  const float* wrow = tile + ((wave & 1) * 16 * TN + r) * GS_ROW + 4 * q;
+  const float* xrow = tile + (32 * TN + (wave >> 1) * 16 * TM + r) * GS_ROW + 4 * q;
+  load(s0);
+  store(0);
+  load(min(s0 + 1, s1 - 1));
+  __syncthreads();
+#pragma unroll 1
+  for (int s = s0; s < s1; ++s) {
+    const int buf = (s - s0) & 1;
+    f4 w[2][TN], x[2][TM];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+      for (int t = 0; t < TN; ++t) w[b][t] = *(const f4*)(wrow + (buf * ROWS + 16 * t) * GS_ROW + 16 * b);
+#pragma unroll
+      for (int t = 0; t < TM; ++t) x[b][t] = *(const f4*)(xrow + (buf * ROWS + 16 * t) * GS_ROW + 16 * b);
+    }
+    store(buf ^ 1);
+    load(min(s + 2, s1 - 1));  // (the last two steps load one again that nobody reads)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t = 0; t < TN; ++t)
+#pragma unroll
+          for (int u = 0; u < TM; ++u) {
+            const int c = (4 * b + e) % CHAINS;
+            acc[c][t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[b][t][e], x[b][u][e], acc[c][t][u], 0, 0, 0);
+          }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int half = CHAINS / 2; half > 0; half /= 2)
+#pragma unroll
+    for (int c = 0; c < half; ++c)
+#pragma unroll
+      for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int u = 0; u < TM; ++u) acc[c][t][u] += acc[c + half][t][u];
+#pragma unroll
+  for (int u = 0; u < TM; ++u) {
+    const int token = m0 + (wave >> 1) * 16 * TM + 16 * u + r;
+    if (token >= a.M) continue;
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+      const int n = n0 + (wave & 1) * 16 * TN + 16 * t + 4 * q;
+      if (n >= a.N) continue;
+      if (a.part) {  // (N is a multiple of 4 then)
+        *(f4*)(a.part + ((size_t)blockIdx.y * a.M + token) * a.N + n) = acc[0][t][u];
+      } else {
+        gf_store(a, acc[0][t][u], token, n);
+      }
+    }
+  }
+}
+
+// The sums of K's parts added in the order of K: a thread four neighbouring outputs.
+__global__ __launch_bounds__(256) void gemm_f32_sum_kernel(GemmF32Args a, int cuts) {
+  const int n = (blockIdx.x * blockDim.x + threadIdx.x) * 4, token = blockIdx.y;
+  if (n >= a.N) return;
+  const float* p = a.part + (size_t)token * a.N + n;
+  f4 v = *(const f4*)p;
+#pragma unroll 8
+  for (int c = 1; c < cuts; ++c) v += *(const f4*)(p + (size_t)c * a.M * a.N);
+  gf_store(a, v, token, n);
+}
+
+// Whether the kernels take the operands: rows at multiples of 16 bytes.
+TK_API int tk_gemm_f32_takes(const void* A, int lda, const void* W, int K) {
+  return ((((uintptr_t)A | (uintptr_t)W) & 15) == 0 && (lda & 3) == 0 && (K & 3) == 0) ? 1 : 0;
+}
+
+// workgroups of tiles of 32 tm tokens x 32 tn weight rows (their number over the columns is filled up to eights, see the kernel)
+static long gf_tiles(int M, int N, int tm, int tn) {
+  return (((long)N + 32 * tn - 1) / (32 * tn) + 7) / 8 * 8 * (((long)M + 32 * tm - 1) / (32 * tm));
+}
+
+// How many parts K is cut into among workgroups (the caller brings M * N floats for each where there is more than one):
+// so many that the tiles times the parts are about five workgroups a compute unit, of 256 elements of K at least.  In us at
+// 1 / 2 / 4 / 8 / 16 parts: 301 tokens 2 048 x 8 192 (160 tiles) 188 / 170 / 124 / 108 / 111; 600 tokens (320 tiles) 329 / 240 /
+// 199 / 199 / 207; 301 tokens 3 072 x 2 048 (240 tiles) 49 / 50 / 48 / 51 / 59; 16 384 x 2 048 (1 280 tiles) 203 / 202 / 216.
+TK_API int tk_gemm_f32_cuts(int M, int N, int K) {
+  if (M <= 16 || (N & 3) != 0) return 1;
+  long cuts = 1280 / gf_tiles(M, N, M <= 32 ? 1 : 2, 2);
+  const long most = K / 256;
+  if (cuts > most || M <= 32) cuts = most;  // (few tokens: chains of 32 elements in every part)
+  if (cuts > 32) cuts = 32;
+  return cuts < 1 ? 1 : (int)cuts;
+}
+
+template <int TM, int TN, int CHAINS>
+static bool gf_launch(const GemmF32Args& a, int cuts, hipStream_t stream) {
+  const long grid = gf_tiles(a.M, a.N, TM, TN);
+  if (grid > 0x7fffffffL) return false;
+  const size_t lds = (size_t)2 * 32 * (TM + TN) * GS_ROW * sizeof(float);
+  auto kernel = gemm_f32_kernel<TM, TN, CHAINS>;
+  if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return false;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid, cuts), dim3(256), lds, stream, a);
+  return true;
+}
+
+TK_API int tk_gemm_f32(const void* A, int lda, const void* W, void* C, int ldc, const void* residual, int ldr,
+                       const void* bias, int M, int N, int K, int cuts, void* part, hipStream_t stream) {
+  TK_REQUIRE(M >= 0 && N > 0 && K > 0 && lda >= K && ldc >= N, "gemm_f32: bad sizes M=%d N=%d K=%d lda=%d ldc=%d", M, N, K, lda, ldc);
+  TK_REQUIRE(!residual || ldr >= N, "gemm_f32: residual stride %d < N %d", ldr, N);
+  TK_REQUIRE(tk_gemm_f32_takes(A, lda, W, K), "gemm_f32: rows of A and W must start at multiples of 16 bytes");
+  TK_REQUIRE(cuts >= 1 && cuts <= (K + 31) / 32 && cuts < 65536 && (cuts == 1 || (part && (N & 3) == 0 && M > 16 && M < 65536)),
+             "gemm_f32: K=%d in %d parts", K, cuts);
+  if (M == 0) return 0;
+  GemmF32Args a = {(const float*)A, lda, (const float*)W, (float*)C, ldc, (const float*)residual, ldr, (const float*)bias, M, N, K,
+                   cuts > 1 ? (float*)part : nullptr};
+  if (M <= 16) {
+    // (2, 4, 8 wavefronts at 4 tokens, 2 048 x 2 048: 9.0, 8.2, 9.0 us, 2 048 x 8 192: 34, 25, 26, 16 384 x 2 048: 33, 30, 30)
+    const int KS = K < 64 ? 1 : (K < 4096 ? 4 : 8);
+    hipLaunchKernelGGL(gemm_f32_few_kernel, dim3((N + 15) / 16), dim3(64 * KS), (KS - 1) * 64 * sizeof(f4), stream, a);
+    TK_CHECK_LAUNCH("gemm_f32");
+    return 0;
+  }
+  // tiles of 128 x 128 read the operands half as often, where they still fill the chip twice over; up to 32 tokens leave half
+  // of a 64-token tile empty
+  bool ok;
+  if (M <= 32) ok = gf_launch<1, 2, 8>(a, cuts, stream);
+  else if (gf_tiles(M, N, 4, 4) >= 512) ok = gf_launch<4, 4, 1>(a, cuts, stream);
+  else ok = gf_launch<2, 2, 1>(a, cuts, stream);
+  TK_REQUIRE(ok, "gemm_f32: M=%d N=%d take too many workgroups, or their local memory could not be reserved", M, N);
+  if (cuts > 1) hipLaunchKernelGGL(gemm_f32_sum_kernel, dim3((N / 4 + 255) / 256, M), dim3(256), 0, stream, a, cuts);
+  TK_CHECK_LAUNCH("gemm_f32");
+  return 0;
+}

@@ -1,7 +1,7 @@
 // C[M,N] = A[M,K] * W[N,K]^T (+ residual[M,N]) with plain 32-bit multiply-adds:
-// the matrix product of the true 32-bit path, and the fallback of the bfloat16
-// path for shapes the MFMA kernels refuse.  Operands are row-major with K
-// contiguous; any M, N, K.  A bias (one value an output, of the storage type, or null) is added
+// the matrix product of operands whose rows do not start at multiples of 16 bytes, in either
+// storage type (the matrix-core kernels take the others: gemm_f32.hip, gemm_mfma.hip).
+// Operands are row-major with K contiguous; any M, N, K.  A bias (one value an output, of the storage type, or null) is added
 // to the product in 32-bit before it is rounded.  Two kernels: tiles of 64 x 64 through LDS, each output
 // summing its K products in ascending k; and, for up to GR_MAX_ROWS rows (decode), one
 // that streams the weights: a wavefront owns GR_COLS output columns, its lanes cut K
@@ -13,20 +13,14 @@
 #define GR_COLS 4
 #define GR_MAX_ROWS 32
 
-// Four consecutive elements as 32-bit floats: one 16-byte load where T is float and the
-// caller found sizes and addresses aligned, else element by element (k may run past K).
-template <typename T, bool VEC>
+// Four consecutive elements as 32-bit floats (k may run past K).
+template <typename T>
 __device__ __forceinline__ void load4(const T* row, int k, int K, float out[4]) {
-  if constexpr (VEC) {
-    const float4 v = *(const float4*)(row + k);
-    out[0] = v.x; out[1] = v.y; out[2] = v.z; out[3] = v.w;
-  } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) out[i] = (k + i < K) ? to_f32<T>(row[k + i]) : 0.f;
-  }
+  for (int i = 0; i < 4; ++i) out[i] = (k + i < K) ? to_f32<T>(row[k + i]) : 0.f;
 }
 
-template <typename T, typename TO, int MB, bool VEC>
+template <typename T, typename TO, int MB>
 __global__ __launch_bounds__(256) void gemm_rows_kernel(const T* __restrict__ A, int lda,
                                                         const T* __restrict__ W,
                                                         TO* __restrict__ C, int ldc,
@@ -44,12 +38,12 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const T* __restrict__ A,
   for (int k = lane * 4; k < K; k += TK_WAVE * 4) {
     float w[GR_COLS][4];
 #pragma unroll
-    for (int c = 0; c < GR_COLS; ++c) load4<T, VEC>(W + (size_t)min(n0 + c, N - 1) * K, k, K, w[c]);
+    for (int c = 0; c < GR_COLS; ++c) load4<T>(W + (size_t)min(n0 + c, N - 1) * K, k, K, w[c]);
 #pragma unroll
     for (int m = 0; m < MB; ++m) {
       if (m0 + m < M) {  // the same for every lane
         float a[4];
-        load4<T, VEC>(A + (size_t)(m0 + m) * lda, k, K, a);
+        load4<T>(A + (size_t)(m0 + m) * lda, k, K, a);
 #pragma unroll
         for (int c = 0; c < GR_COLS; ++c)
 #pragma unroll
@@ -77,17 +71,13 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(const T* __restrict__ A,
 template <typename T, typename TO>
 static void launch_rows(const T* A, int lda, const T* W, TO* C, int ldc, const T* residual, int ldr, const T* bias,
                         int M, int N, int K, hipStream_t stream) {
-  const bool vec = sizeof(T) == 4 && K % 4 == 0 && lda % 4 == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0;
   const int cols_per_block = (256 / TK_WAVE) * GR_COLS;
   const unsigned gx = (unsigned)((N + cols_per_block - 1) / cols_per_block);
-#define TK_ROWS_LAUNCH(MB, VEC)                                                                        \
-  hipLaunchKernelGGL((gemm_rows_kernel<T, TO, MB, VEC>), dim3(gx, (M + MB - 1) / MB), dim3(256), 0, stream, \
+#define TK_ROWS_LAUNCH(MB)                                                                             \
+  hipLaunchKernelGGL((gemm_rows_kernel<T, TO, MB>), dim3(gx, (M + MB - 1) / MB), dim3(256), 0, stream, \
                      A, lda, W, C, ldc, residual, ldr, bias, M, N, K)
-  if (M <= 4) {
-    if (vec) TK_ROWS_LAUNCH(4, true); else TK_ROWS_LAUNCH(4, false);
-  } else {
-    if (vec) TK_ROWS_LAUNCH(16, true); else TK_ROWS_LAUNCH(16, false);
-  }
+  if (M <= 4) TK_ROWS_LAUNCH(4);
+  else TK_ROWS_LAUNCH(16);
 #undef TK_ROWS_LAUNCH
 }
 

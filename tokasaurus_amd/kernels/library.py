@@ -31,6 +31,9 @@ _SIGNATURES: dict[str, dict[str, list]] = {
         "tk_rope_append": [c_int, _P, c_int, _P, _P, _P, c_int, _P, _P, _P, _P] + [c_int] * 7 + [_P],
         "tk_fill_u32": [_P, c_uint32, c_size_t, _P],
         "tk_gemm_generic": [c_int, _P, c_int, _P, _P, c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, _P],
+        "tk_gemm_f32": [_P, c_int, _P, _P, c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, _P, _P],
+        "tk_gemm_f32_takes": [_P, c_int, _P, c_int],
+        "tk_gemm_f32_cuts": [c_int, c_int, c_int],
         "tk_add_bias": [c_int, _P, _P, c_int, c_int, _P],
         "tk_head_rmsnorm": [c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_float, _P],
         "tk_paged_attention_generic": [c_int, _P, c_int, _P, c_int, _P, _P, _P, c_int, _P, _P]

@@ -278,7 +278,8 @@ def gemm_generic(
     out: torch.Tensor | None = None,
     bias: torch.Tensor | None = None,
 ) -> torch.Tensor:
-    """a [M, K] times w [N, K] transposed (+ bias [N]) (+ residual [M, N]), 32-bit multiply-adds.
+    """a [M, K] times w [N, K] transposed (+ bias [N]) (+ residual [M, N]), 32-bit multiply-adds: on the matrix cores
+    (``gemm_f32.hip``) for 32-bit operands whose rows start at multiples of 16 bytes, else on the plain kernels.
     ``out``: where the result goes (contiguous [M, N] of the result's type) instead of new memory."""
     _gpu(a, w, residual, bias)
     _check_bias(bias, w, "gemm")
@@ -296,6 +297,13 @@ def gemm_generic(
         _need(residual.shape == (m, n) and residual.stride(1) == 1 and residual.dtype == a.dtype,
               "gemm: residual must be [M, N] of the operand type")
         ldr = residual.stride(0)
+    if a.dtype == torch.float32 and m > 0 and load("core").tk_gemm_f32_takes(a.data_ptr(), a.stride(0), w.data_ptr(), k):
+        cuts = load("core").tk_gemm_f32_cuts(m, n, k)
+        part = torch.empty((cuts * m * n,), dtype=torch.float32, device=a.device) if cuts > 1 else None
+        call("tk_gemm_f32", a.data_ptr(), a.stride(0), w.data_ptr(), out.data_ptr(), n,
+             residual.data_ptr() if residual is not None else None, ldr, bias.data_ptr() if bias is not None else None,
+             m, n, k, cuts, part.data_ptr() if part is not None else None, _stream())
+        return out
     call(
         "tk_gemm_generic",
         dtype_code(a.dtype),
