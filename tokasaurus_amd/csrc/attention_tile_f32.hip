@@ -258,6 +258,12 @@ __global__ __launch_bounds__(NW * TK_WAVE) void attention_tile_f32_kernel(
         const bool seen = live && kp <= pos && kp >= lo_col && (window <= 0 || pos - kp < window);
         sc[i] = seen ? (shaped ? shaped_score(shape, s[i] * scale, pos - kp, head, nq) : s[i] * scale) : -INFINITY;
         tmax = fmaxf(tmax, sc[i]);
+        // a key that no column sees may be anything (a page's places behind the request's last token, a page given back):
+        // its weight is zero, and so must its values be, or a NaN there would reach the sums
+        if (kp > last_all || kp < first_seen) {
+#pragma unroll
+          for (int t = 0; t < VT; ++t) vr[t].v[i] = from_f32<T>(0.f);
+        }
       }
     }
     float p[4];

@@ -1863,7 +1863,7 @@ def attention_tile_f32(
     sink: torch.Tensor | None = None, split: bool | None = None, key_chunk: int = 0, longest: int = 0, first_row: int = 0,
     score_bias: torch.Tensor | None = None, value_freq: torch.Tensor | None = None,
     value_pair_halves: bool = False, gate: torch.Tensor | None = None, softcap: float = 0.0,
-    distance_bias: "DistanceBias | None" = None, section: int = 0,
+    distance_bias: "DistanceBias | None" = None, section: int = 0, out: torch.Tensor | None = None,
 ) -> torch.Tensor:
     """Attention in 32-bit arithmetic on the matrix cores: every token of the step over its
     request's pages; ``tile_req`` / ``tile_row0`` name each tile's request and its first token's
@@ -1877,7 +1877,8 @@ def attention_tile_f32(
     ``first_row``: ``q`` holds the step's rows from this one on only (the tiles name none before it), and so
     does the result.  ``score_bias``: sigmoid weights as in ``paged_attention_generic``.  ``value_freq``,
     ``value_pair_halves``, ``gate``: what ``unrotate_gate_`` does, in the kernel's own epilogue (halves only where
-    ``attention_tile_turns_halves``).  ``section`` as in ``paged_attention_generic``."""
+    ``attention_tile_turns_halves``).  ``section`` as in ``paged_attention_generic``.  ``out``: [tokens, nq * value_dim]
+    for the result instead of new memory; only the tiles' rows are written."""
     _gpu(q, kcache, vcache, block_table, q_start, kv_len, tile_req, tile_row0, sink, score_bias, value_freq, gate)
     db = _checked_distance_bias(distance_bias, nq)
     _f32_vector(value_freq, value_dim // 2, "attention: the values' frequencies")
@@ -1897,7 +1898,10 @@ def attention_tile_f32(
     _need(sink is None or (sink.shape == (nq,) and sink.dtype == torch.float32 and sink.is_contiguous()),
           f"attention: the sinks must be contiguous float32 [{nq}]")
     _check_pages(kcache, vcache, nkv, page_size, key_dim, q.dtype, "attention", value_dim)
-    out = torch.empty((q.shape[0], nq * value_dim), dtype=q.dtype, device=q.device)
+    if out is None:
+        out = torch.empty((q.shape[0], nq * value_dim), dtype=q.dtype, device=q.device)
+    _need(out.shape == (q.shape[0], nq * value_dim) and out.dtype == q.dtype and out.is_contiguous(),
+          "attention: the result's buffer must be contiguous [tokens, nq * value_dim] of the queries' type")
     chunks, part = 0, None
     if split and key_chunk > 0 and longest > key_chunk:
         # longer chunks where the step has workgroups enough without short ones: a chunk's walk should be long

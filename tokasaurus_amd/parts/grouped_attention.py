@@ -42,15 +42,16 @@ from tokasaurus_amd.parts.linear import Linear, Placer
 from tokasaurus_amd.parts.position import InterleavedRotary
 
 
-def tile_plan(ctx: StepContext, tokens_a_tile: int) -> tuple[torch.Tensor, torch.Tensor]:
-    """The step's rows cut into tiles of up to ``tokens_a_tile`` neighbouring tokens of one
-    request: for every tile its request and its first row.  Made once a step and shared by
-    the layers; a step that is recorded keeps it for its replays."""
-    key = ("tile_plan", tokens_a_tile)
+def tile_plan(ctx: StepContext, tokens_a_tile: int, first_request: int = 0, end_request: int | None = None) -> tuple[torch.Tensor, torch.Tensor]:
+    """The step's rows (those of requests ``first_request`` up to ``end_request``; all by default) cut into tiles of up to
+    ``tokens_a_tile`` neighbouring tokens of one request: for every tile its request and its first row.  Made once a step
+    and shared by the layers; a step that is recorded keeps it for its replays."""
+    end_request = ctx.num_requests if end_request is None else end_request
+    key = ("tile_plan", tokens_a_tile, first_request, end_request)
     plan = ctx.extras.get(key)
     if plan is None:
         req, row0 = [], []
-        for r in range(ctx.num_requests):
+        for r in range(first_request, end_request):
             a, b = ctx.host_q_start[r], ctx.host_q_start[r + 1]
             for first in range(a, b, tokens_a_tile):
                 req.append(r)
