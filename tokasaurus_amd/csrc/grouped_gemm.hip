@@ -2,18 +2,18 @@
 // v_mfma_f32_16x16x32_bf16: the experts of a mixture (rows sorted by expert) and a matrix a head.
 //
 //   tk_expert_sort        pairs (token, chosen expert) sorted by expert into slots, every expert's
-//                         run of slots filled up to whole tiles of GG_TM or GS_M slots
+//                         run of slots filled up to whole tiles of GS_M slots
 //   tk_grouped_gemm_bf16  C[c_row(slot), g * c_cols + n] = sum_k W[g][n][k] * A[a_row(slot), g * a_cols + k]
 //                         for the slots of every tile, g the tile's group; optionally the gated form
 //                         silu(gate) * up of two halves of W[g], or the gated form with clamps
 //   tk_expert_sum         per token the weighted sum of its pairs' rows, identity experts, shared expert
 //
-// A wavefront owns GG_TM = 64 slots x 64 outputs (32 in the gated form, for each of gate and up): weight rows
-// are the first operand of the matrix core, read straight from memory 16 bytes a lane, the slots' rows the
-// second; a lane ends up with 4 neighbouring outputs of one slot.  The next step's operands are asked for
-// before the current step's products.  Where an expert has many rows, tiles of GS_M = 128 slots x 128 weight rows go
-// through LDS instead (grouped_gemm_staged_kernel).  Sums are 32-bit and run over k in ascending order for every output:
-// a row's result does not depend on which other rows share its tile.
+// Two kernels.  A matrix a head (grouped_gemm_kernel): a wavefront owns GG_TM = 64 rows x 64 outputs: weight rows are the
+// first operand of the matrix core, read straight from memory 16 bytes a lane, the rows of A the second; a lane ends up with
+// 4 neighbouring outputs of one row.  The next step's operands are asked for before the current step's products.
+// Experts (grouped_gemm_staged_kernel): tiles of GS_M = 128 slots x 128 weight rows through local memory, however few slots a
+// tile holds (see there).  Sums are 32-bit and run over k in ascending steps for every output: a row's result does not
+// depend on which other rows share its tile.
 #include <math.h>
 
 #include "common.h"
@@ -37,8 +37,8 @@ struct GroupedArgs {
   const int* a_row;       // [slots] the row of A a slot reads, < 0: an empty slot; null: the slot's own number
   const int* c_row;       // [slots] the row of C a slot writes, < 0: none; null: the slot's own number
   const int* tile_group;  // [tiles] the group of every tile of slots, < 0: an unused tile, and [tiles] the number of used ones, which come
-                          // first; null: blockIdx.z (tiles of GG_TM only)
-  int a_cols, c_cols;     // columns of A and C that a group is offset by
+                          // first; null: blockIdx.z, and rows instead of slots
+  int a_cols, c_cols;     // (a group a blockIdx.z) columns of A and C that a group is offset by
   const bf16_t* W;        // [groups][N (2 N in the gated form: gate rows, then up rows)][K]
   size_t w_stride;        // elements from one group's matrix to the next
   void* C;
@@ -52,47 +52,38 @@ __device__ __forceinline__ float gg_gated(const GroupedArgs& a, float g, float u
   return a.limit > 0.f ? clamped_glu<bf16_t>(g, u, a.limit, a.alpha) : silu_mul_bf16(g, u);
 }
 
-// NT: blocks of 16 outputs a wavefront; GLU: the gated form; F32: 32-bit output
-template <int NT, bool GLU, bool F32>
+// NT: blocks of 16 outputs a wavefront; F32: 32-bit output
+template <int NT, bool F32>
 __global__ __launch_bounds__(GG_WAVES * TK_WAVE) void grouped_gemm_kernel(GroupedArgs a) {
   constexpr int MB = GG_TM / 16;
-  constexpr int WT = GLU ? 2 * NT : NT;  // weight blocks a wavefront reads a step
   const int lane = threadIdx.x & (TK_WAVE - 1), wave = threadIdx.x / TK_WAVE;
   const int tile = blockIdx.x;
-  const int g = a.tile_group ? a.tile_group[tile] : (int)blockIdx.z;
-  if (g < 0) return;
+  const int g = (int)blockIdx.z;
   const int n0 = (blockIdx.y * GG_WAVES + wave) * NT * 16;
   if (n0 >= a.N) return;
   const int r = lane & 15, q = lane >> 4;
   const bf16_t* Wg = a.W + (size_t)g * a.w_stride;
-  const bf16_t* wp[WT];
+  const bf16_t* wp[NT];
 #pragma unroll
-  for (int t = 0; t < WT; ++t) {
-    const int blk = GLU ? t % NT : t;
-    const int row = min(n0 + blk * 16 + r, a.N - 1) + ((GLU && t >= NT) ? a.N : 0);
-    wp[t] = Wg + (size_t)row * a.K + q * 8;
-  }
+  for (int t = 0; t < NT; ++t) wp[t] = Wg + (size_t)min(n0 + t * 16 + r, a.N - 1) * a.K + q * 8;
   const bf16_t* ap[MB];
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    const int slot = tile * GG_TM + mb * 16 + r;
-    int row = slot < a.slots ? (a.a_row ? a.a_row[slot] : slot) : -1;
-    ap[mb] = a.A + (size_t)max(row, 0) * a.lda + (size_t)g * a.a_cols + q * 8;
-  }
-  f32x4_t acc[WT][MB];
+  for (int mb = 0; mb < MB; ++mb)
+    ap[mb] = a.A + (size_t)min(tile * GG_TM + mb * 16 + r, a.slots - 1) * a.lda + (size_t)g * a.a_cols + q * 8;
+  f32x4_t acc[NT][MB];
 #pragma unroll
-  for (int t = 0; t < WT; ++t)
+  for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) acc[t][mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   const int steps = (a.K + 31) / 32;
-  bf16x8_t w[WT], av[MB];
-  auto load = [&](int ks, bf16x8_t (&wv)[WT], bf16x8_t (&xv)[MB]) {
+  bf16x8_t w[NT], av[MB];
+  auto load = [&](int ks, bf16x8_t (&wv)[NT], bf16x8_t (&xv)[MB]) {
     // a step may reach past K (a multiple of 8): read a valid chunk and zero the weight
     const bool k_ok = ks * 32 + q * 8 < a.K;
     const long off = k_ok ? (long)ks * 32 : -(long)(q * 8);
 #pragma unroll
-    for (int t = 0; t < WT; ++t) {
+    for (int t = 0; t < NT; ++t) {
       wv[t] = *(const bf16x8_t*)(wp[t] + off);
       if (!k_ok) wv[t] = gg_zero8();
     }
@@ -101,41 +92,34 @@ __global__ __launch_bounds__(GG_WAVES * TK_WAVE) void grouped_gemm_kernel(Groupe
   };
   load(0, w, av);
   for (int ks = 0; ks < steps; ++ks) {
-    bf16x8_t wn[WT], an[MB];
+    bf16x8_t wn[NT], an[MB];
     if (ks + 1 < steps) load(ks + 1, wn, an);
 #pragma unroll
-    for (int t = 0; t < WT; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
         acc[t][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], av[mb], acc[t][mb], 0, 0, 0);
     if (ks + 1 < steps) {
 #pragma unroll
-      for (int t = 0; t < WT; ++t) w[t] = wn[t];
+      for (int t = 0; t < NT; ++t) w[t] = wn[t];
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) av[mb] = an[mb];
     }
   }
-  // lane: slot mb * 16 + r, outputs n0 + t * 16 + 4 q + j
+  // lane: row mb * 16 + r, outputs n0 + t * 16 + 4 q + j
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
-    const int slot = tile * GG_TM + mb * 16 + r;
-    if (slot >= a.slots) continue;
-    if (a.a_row && a.a_row[slot] < 0) continue;
-    const int crow = a.c_row ? a.c_row[slot] : slot;
-    if (crow < 0) continue;
-    const float f = GLU && a.row_scale ? a.row_scale[a.scale_row[slot]] : 1.f;  // (a slot that is filled names its row)
+    const int row = tile * GG_TM + mb * 16 + r;
+    if (row >= a.slots) continue;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const int n = n0 + t * 16 + 4 * q;
-      float y[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) y[j] = GLU ? gg_gated(a, acc[t][mb][j] * f, acc[t + (GLU ? NT : 0)][mb][j] * f) : acc[t][mb][j];
-      const size_t at = (size_t)crow * a.ldc + (size_t)g * a.c_cols + n;
+      const size_t at = (size_t)row * a.ldc + (size_t)g * a.c_cols + n;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         if (n + j < a.N) {
-          if (F32) ((float*)a.C)[at + j] = y[j];
-          else ((bf16_t*)a.C)[at + j] = __float2bfloat16(y[j]);
+          if (F32) ((float*)a.C)[at + j] = acc[t][mb][j];
+          else ((bf16_t*)a.C)[at + j] = __float2bfloat16(acc[t][mb][j]);
         }
       }
     }
@@ -143,140 +127,230 @@ __global__ __launch_bounds__(GG_WAVES * TK_WAVE) void grouped_gemm_kernel(Groupe
 }
 
 // --------------------------------------------------------------------------
-// The same product for groups of many slots: a workgroup owns GS_M slots x 128 weight rows (in the gated form 64 of
-// gate and the 64 of up that belong to them), its four wavefronts 64 x 64 each.  64 elements of K a step go through LDS in
-// two buffers with one barrier a step, 16 bytes a thread and load, the 16-byte pieces of a row exchanged by its number
-// (piece ^ (row & 7)) so that the lanes that read one piece of sixteen rows spread over the banks; the next step's
-// pieces are on their way to registers meanwhile.  Workgroups go to the chip's dies in turn: each die takes a run of
-// neighbouring tiles (an expert's tiles mostly share a die, and its cache the expert's weights), GS_TILES of them at a
-// time through all outputs.  Every output's sum runs over k in the order of the kernel above: the same bits.
+// Experts: a workgroup owns GS_M slots x 128 weight rows (in the gated form 64 of
+// gate and the 64 of up that belong to them), its four wavefronts 64 x 64 each, on v_mfma_f32_32x32x16_bf16 (1.86 PFLOP/s
+// in a loop of nothing else; the 16 x 16 x 32 form 1.23 to 1.57).  Steps of 32 elements of K go straight from memory to
+// local memory into GS_STAGES buffers: two steps' rows are on their way while one is multiplied (48 KB a workgroup, three
+// workgroups a compute unit; four buffers and two workgroups: 228 against 210 us), with one barrier a step.  16-byte pieces of a row lie exchanged by (row / 4) & 3, made on the
+// side of the address, so that any 16 of the 32 rows that the lanes read at a time meet 64 different banks.
+// What bounds it is memory: an expert's weights (8 MB for 2 x 1 024 rows of 2 048) pass a die's L2 once for every time that its
+// tiles are taken up.  So workgroups come in the order of the runs: up to GS_TILES tiles of one group through all outputs,
+// then the next, each die a stretch of that order (the hardware deals workgroups to the eight dies in turn).
+// The results leave through local memory, 16 bytes a lane (8 scattered bytes a lane took 40 us of 290).
+// Experts of few rows take the same tiles: their products are priced by the weights, which a tile reads once (32 experts of 2 048 x
+// 1 024, 403 MB; tokens x 8 chosen, 13 / 64 / 300 tokens: 108 / 110 / 115 us for both products and the sum, 176 / 194 / 317
+// with 64 slots a wavefront straight from memory).
+// 2 048 tokens x 8 of 32 experts (143 tiles), gate and up: 290 us through registers into two buffers of 64
+// elements with tiles taken four at a time whatever their group (634 MB past the L2), 210 us so (474 MB; 343 are needed);
+// the loads alone take 180, the products alone 140.
 // --------------------------------------------------------------------------
 #define GS_M 128
-#define GS_K 64
+#define GS_K 32
+#define GS_STAGES 3
 #define GS_DIES 8
-#define GS_TILES 4
+#define GS_TILES 8
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
-__device__ __forceinline__ void gg_store4(bf16_t* dst, const float (&y)[4], int left) {
-  union { bf16_t v[4]; uint2 raw; } o;
+// 16 bytes a lane from memory to local memory, lane l to `lds` (the same for the wavefront) + 16 l.  Counted in vmcnt, which
+// the caller waits for: the compiler knows nothing of the load.
+__device__ __forceinline__ void load_to_lds(const bf16_t* src, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
+}
+
+// Tiles in a row before and behind `tile` that belong to its group `g` (both sides' first 64 asked for at once).
+__device__ __forceinline__ void gg_run(const int* tile_group, int used, int tile, int& g, int& before, int& behind) {
+  const int lane = threadIdx.x & (TK_WAVE - 1);
+  int at[2] = {0, 0};
+  bool open[2] = {true, true};
+  g = tile_group[tile];
+  while (open[0] || open[1]) {
+    int t[2], v[2];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) o.v[j] = __float2bfloat16(y[j]);
-  if (left >= 4 && ((uintptr_t)dst & 7) == 0) {
-    *(uint2*)dst = o.raw;
-  } else {
+    for (int side = 0; side < 2; ++side) {
+      t[side] = side == 0 ? tile - 1 - at[0] - lane : tile + 1 + at[1] + lane;
+      v[side] = tile_group[min(max(t[side], 0), used - 1)];
+    }
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j < left) dst[j] = o.v[j];
+    for (int side = 0; side < 2; ++side) {
+      if (!open[side]) continue;
+      const unsigned long long other = ~__ballot(t[side] >= 0 && t[side] < used && v[side] == g);
+      if (other != 0) {
+        at[side] += __ffsll(other) - 1;
+        open[side] = false;
+      } else {
+        at[side] += TK_WAVE;
+      }
+    }
+  }
+  before = at[0];
+  behind = at[1];
+}
+
+template <bool GLU>
+__global__ __launch_bounds__(256, 3) void grouped_gemm_staged_kernel(GroupedArgs a, int tiles, int n_blocks) {
+  extern __shared__ __align__(16) bf16_t rows[];  // [GS_STAGES][128 slots, 128 weight rows][GS_K]; then the results [GS_M][OUT]
+  constexpr int OUT = GLU ? 64 : 128;             // outputs of a workgroup
+  const int used = a.tile_group[tiles];           // the tiles that hold slots come first
+  const int items = used * n_blocks, per = (items + GS_DIES - 1) / GS_DIES;
+  const int seq = blockIdx.x / GS_DIES, item = blockIdx.x % GS_DIES * per + seq;
+  if (seq >= per || item >= items) return;
+  // the run of tiles of one group that the item lies in, and in it the chunk of up to GS_TILES tiles
+  const int some = item / n_blocks;
+  int g, before, behind;
+  gg_run(a.tile_group, used, some, g, before, behind);
+  const int chunk = some - before + before / GS_TILES * GS_TILES;  // its first tile
+  const int len = min(GS_TILES, some + behind + 1 - chunk);
+  const int off = item - chunk * n_blocks;
+  const int tile = chunk + off % len;
+  const int n0 = off / len * OUT;
+  const int lane = threadIdx.x & (TK_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TK_WAVE);
+  // A load brings 16 rows of 32 elements; wavefront w brings slots 32 w .. 32 w + 31 and as many weight rows.  Lane l writes
+  // piece l % 4 of row l / 4, which holds the row's piece (l % 4) ^ ((row / 4) & 3).
+  const int lrow = lane >> 2, piece = (lane & 3) ^ (lane >> 4);
+  // what this thread stores at the end: 16-byte pieces of rows, their places in C
+  constexpr int PIECES = OUT / 8, PASSES = GS_M * PIECES / 256;
+  const int orow = threadIdx.x / PIECES, ocol = threadIdx.x % PIECES * 8;
+  const int r = lane & 31, h = lane >> 5;
+  const int wm = wave & 1, wn = wave >> 1;
+  // (all numbers of rows are asked for before the first is used)
+  const int top = a.slots - 1;
+  int from[2], crow[PASSES], filled[PASSES], frow[2] = {0, 0};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) from[i] = tile * GS_M + wave * 32 + i * 16 + lrow;
+#pragma unroll
+  for (int i = 0; i < PASSES; ++i) crow[i] = filled[i] = tile * GS_M + orow + i * (256 / PIECES);
+  if (a.a_row) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) from[i] = a.a_row[min(from[i], top)];
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) filled[i] = a.a_row[min(filled[i], top)];
+  }
+  const bool scaled = GLU && a.row_scale;
+  if (scaled) {
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) frow[mb] = a.scale_row[min(tile * GS_M + wm * 64 + mb * 32 + r, top)];  // (< 0: an empty slot)
+  }
+  if (a.c_row) {
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) crow[i] = a.c_row[min(crow[i], top)];
+  }
+  const bf16_t* src[4];  // slots, then weight rows (a row that is not stored may read any)
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = wave * 32 + i * 16 + lrow;
+    const int wrow = GLU ? min(n0 + (row & 63), a.N - 1) + (row >= 64 ? a.N : 0) : min(n0 + row, a.N - 1);
+    src[2 + i] = a.W + (size_t)g * a.w_stride + (size_t)wrow * a.K + piece * 8;
+    src[i] = a.A + (size_t)max(tile * GS_M + row <= top ? from[i] : 0, 0) * a.lda + piece * 8;
+  }
+  float factor[2] = {1.f, 1.f};
+  if (scaled) {
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb) factor[mb] = a.row_scale[max(frow[mb], 0)];
+  }
+#pragma unroll
+  for (int i = 0; i < PASSES; ++i)
+    if (tile * GS_M + orow + i * (256 / PIECES) > top || filled[i] < 0) crow[i] = -1;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (nothing but the rows' loads is counted from here on)
+  const unsigned lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) bf16_t*)rows;
+  const int steps = (a.K + GS_K - 1) / GS_K;
+  auto ask = [&](int step) {
+    const int at = (step % GS_STAGES * 256 + wave * 32) * GS_K;  // elements
+    const size_t k = (size_t)step * GS_K;
+    if (step * GS_K + piece * 8 < a.K) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) load_to_lds(src[i] + k, lds + (at + ((i >> 1) * 128 + (i & 1) * 16) * GS_K) * 2);
+    } else {  // K (a multiple of 8) ends inside the step: zeros behind it (the step's first piece is always there)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *(bf16x8_t*)(rows + at + ((i >> 1) * 128 + (i & 1) * 16) * GS_K + lane * 8) = gg_zero8();
+    }
+  };
+  f32x16_t acc[2][2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) acc[t][mb][j] = 0.f;
+#pragma unroll
+  for (int s = 0; s < GS_STAGES - 1; ++s)
+    if (s < steps) ask(s);
+#pragma unroll 1
+  for (int s = 0; s < steps; ++s) {
+    // the step's rows are there when only those of the steps behind it (four loads each) are left, and every wavefront's are
+    // behind the barrier; every wavefront is through with the step before then, whose buffer is filled again
+    if (s + 1 < steps) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (s + GS_STAGES - 1 < steps) ask(s + GS_STAGES - 1);
+    const bf16_t* sa = rows + (size_t)(s % GS_STAGES) * 256 * GS_K;
+    const bf16_t* sw = sa + 128 * GS_K;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      bf16x8_t w[2], x[2];
+      const int swz = ((kk * 2 + h) ^ ((r >> 2) & 3)) * 8;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) w[t] = *(const bf16x8_t*)(sw + ((GLU ? t * 64 + wn * 32 : wn * 64 + t * 32) + r) * GS_K + swz);
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb) x[mb] = *(const bf16x8_t*)(sa + (wm * 64 + mb * 32 + r) * GS_K + swz);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb) acc[t][mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[t], x[mb], acc[t][mb], 0, 0, 0);
+    }
+  }
+  __syncthreads();
+  // A lane holds of slot wm * 64 + mb * 32 + r the outputs 8 (j / 4) + 4 h + j % 4 of a block of 32.  They pass through local
+  // memory (a row's 8-byte pieces exchanged by its number) so that a slot's outputs leave 16 bytes a lane, side by side.
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb) {
+    const int row = wm * 64 + mb * 32 + r;
+#pragma unroll
+    for (int t = 0; t < (GLU ? 1 : 2); ++t) {
+#pragma unroll
+      for (int j4 = 0; j4 < 4; ++j4) {
+        union { bf16_t v[4]; uint2 raw; } o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float y = GLU ? gg_gated(a, acc[0][mb][4 * j4 + j] * factor[mb], acc[1][mb][4 * j4 + j] * factor[mb]) : acc[t][mb][4 * j4 + j];
+          o.v[j] = __float2bfloat16(y);
+        }
+        const int unit = (GLU ? wn * 8 : wn * 16 + t * 8) + 2 * j4 + h;  // of 4 outputs
+        *(uint2*)(rows + row * OUT + ((unit >> 1) ^ (row & 7)) * 8 + (unit & 1) * 4) = o.raw;
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < PASSES; ++i) {
+    if (crow[i] < 0) continue;
+    const int row = orow + i * (256 / PIECES);
+    const uint4 v = *(const uint4*)(rows + row * OUT + ((ocol >> 3) ^ (row & 7)) * 8);
+    bf16_t* dst = (bf16_t*)a.C + (size_t)crow[i] * a.ldc + n0 + ocol;
+    const int left = a.N - n0 - ocol;
+    if (left >= 8 && ((uintptr_t)dst & 15) == 0) {
+      *(uint4*)dst = v;
+    } else {
+      const bf16_t* e = (const bf16_t*)&v;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (j < left) dst[j] = e[j];
+    }
   }
 }
 
 template <bool GLU>
-__global__ __launch_bounds__(256, 2) void grouped_gemm_staged_kernel(GroupedArgs a, int tiles, int n_blocks) {
-  __shared__ __align__(16) bf16_t sa[2][GS_M * GS_K], sw[2][128 * GS_K];
-  const int used = a.tile_group[tiles];  // the tiles that hold slots come first
-  const int per = (used + GS_DIES - 1) / GS_DIES;
-  const int die = blockIdx.x % GS_DIES, seq = blockIdx.x / GS_DIES;
-  const int local = seq / (GS_TILES * n_blocks) * GS_TILES + seq % GS_TILES;
-  const int tile = die * per + local;
-  if (local >= per || tile >= used) return;
-  const int g = a.tile_group[tile];
-  if (g < 0) return;
-  constexpr int OUT = GLU ? 64 : 128;  // outputs of a workgroup
-  const int n0 = seq / GS_TILES % n_blocks * OUT;
-  const int lane = threadIdx.x & (TK_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TK_WAVE);
-  const int r = lane & 15, q = lane >> 4;
-  // what this thread moves: piece `piece` of rows first_row + 32 i
-  const int first_row = threadIdx.x / 8, piece = threadIdx.x % 8;
-  const bf16_t *ap[4], *wp[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = first_row + 32 * i;
-    const int slot = tile * GS_M + row;
-    const int src = slot < a.slots ? (a.a_row ? a.a_row[slot] : slot) : -1;
-    ap[i] = a.A + (size_t)max(src, 0) * a.lda + piece * 8;
-    const int wrow = GLU ? min(n0 + (row & 63), a.N - 1) + (row >= 64 ? a.N : 0) : min(n0 + row, a.N - 1);
-    wp[i] = a.W + (size_t)g * a.w_stride + (size_t)wrow * a.K + piece * 8;
-  }
-  const int at = first_row * GS_K + ((piece ^ (first_row & 7)) * 8);  // (the rows 32 apart have the same exchange)
-  bf16x8_t pa[4], pw[4];
-  auto ask = [&](int k0) {
-    // a step may reach past K (a multiple of 8): a valid piece is read and replaced by zeros
-    const bool in = k0 + piece * 8 < a.K;
-    const long off = in ? (long)k0 : -(long)(piece * 8);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      pa[i] = *(const bf16x8_t*)(ap[i] + off);
-      pw[i] = *(const bf16x8_t*)(wp[i] + off);
-      if (!in) pw[i] = gg_zero8();
-    }
-  };
-  auto put = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      *(bf16x8_t*)(sa[buf] + at + 32 * i * GS_K) = pa[i];
-      *(bf16x8_t*)(sw[buf] + at + 32 * i * GS_K) = pw[i];
-    }
-  };
-  const int wm = wave & 1, wn = wave >> 1;
-  f32x4_t acc[4][4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb) acc[t][mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  auto multiply = [&](int buf) {
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      bf16x8_t w[4], x[4];
-      const int swz = ((kk * 4 + q) ^ (r & 7)) * 8;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        // gated: blocks 0, 1 of gate and 2, 3 of up
-        const int row = GLU ? (t >> 1) * 64 + wn * 32 + (t & 1) * 16 + r : wn * 64 + t * 16 + r;
-        w[t] = *(const bf16x8_t*)(sw[buf] + row * GS_K + swz);
-      }
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) x[mb] = *(const bf16x8_t*)(sa[buf] + (wm * 64 + mb * 16 + r) * GS_K + swz);
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int mb = 0; mb < 4; ++mb) acc[t][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], x[mb], acc[t][mb], 0, 0, 0);
-    }
-  };
-  ask(0);
-  put(0);
-  __syncthreads();
-  int buf = 0;
-  for (int k0 = 0; k0 < a.K; k0 += GS_K, buf ^= 1) {
-    const bool more = k0 + GS_K < a.K;
-    if (more) ask(k0 + GS_K);
-    multiply(buf);
-    if (more) put(buf ^ 1);
-    __syncthreads();
-  }
-  // lane: slot wm * 64 + mb * 16 + r, outputs 4 q + j of a block
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
-    const int slot = tile * GS_M + wm * 64 + mb * 16 + r;
-    if (slot >= a.slots) continue;
-    if (a.a_row && a.a_row[slot] < 0) continue;
-    const int crow = a.c_row ? a.c_row[slot] : slot;
-    if (crow < 0) continue;
-    const float f = GLU && a.row_scale ? a.row_scale[a.scale_row[slot]] : 1.f;
-    bf16_t* dst = (bf16_t*)a.C + (size_t)crow * a.ldc;
-#pragma unroll
-    for (int t = 0; t < (GLU ? 2 : 4); ++t) {
-      const int n = n0 + (GLU ? wn * 32 + t * 16 : wn * 64 + t * 16) + 4 * q;
-      float y[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) y[j] = GLU ? gg_gated(a, acc[t][mb][j] * f, acc[t + (GLU ? 2 : 0)][mb][j] * f) : acc[t][mb][j];
-      if (n < a.N) gg_store4(dst + n, y, a.N - n);
-    }
-  }
+static bool launch_staged(const GroupedArgs& a, int tiles, hipStream_t stream) {
+  const int outs = GLU ? 64 : 128, n_blocks = (a.N + outs - 1) / outs;
+  const long items = (long)tiles * n_blocks, groups = (items + GS_DIES - 1) / GS_DIES * GS_DIES;
+  if (groups >= (1l << 31)) return false;
+  const int lds = GS_STAGES * 256 * GS_K * (int)sizeof(bf16_t);  // 64 KB, at least the results' place
+  hipLaunchKernelGGL(grouped_gemm_staged_kernel<GLU>, dim3((unsigned)groups), dim3(256), lds, stream, a, tiles, n_blocks);
+  return true;
 }
 
 TK_API int tk_grouped_gemm_bf16(const void* A, int lda, const int* a_row, const int* c_row, const int* tile_group, int tiles,
                                 int groups_z, int a_cols, int c_cols, const void* W, size_t w_stride, void* C, int ldc,
                                 int N, int K, int slots, int glu, int out_f32, const float* row_scale, const int* scale_row,
-                                int tile_slots, float limit, float alpha, hipStream_t stream) {
+                                float limit, float alpha, hipStream_t stream) {
   TK_REQUIRE(A && W && C && N > 0 && K > 0 && slots >= 0 && tiles >= 0, "grouped_gemm: bad arguments");
   TK_REQUIRE(K % 8 == 0 && lda % 8 == 0 && a_cols % 8 == 0 && w_stride % 8 == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0,
              "grouped_gemm: rows of A and W must start at multiples of 16 bytes (K=%d lda=%d)", K, lda);
@@ -286,27 +360,19 @@ TK_API int tk_grouped_gemm_bf16(const void* A, int lda, const int* a_row, const 
   if (tiles == 0 || slots == 0) return 0;
   GroupedArgs a{(const bf16_t*)A, lda, a_row, c_row, tile_group, a_cols, c_cols, (const bf16_t*)W, w_stride, C, ldc, N, K, slots,
                 row_scale, scale_row, limit, alpha};
-  TK_REQUIRE(tile_slots == GG_TM || (tile_slots == GS_M && tile_group && !out_f32 && a_cols == 0 && c_cols == 0),
-             "grouped_gemm: tiles of %d slots, or of %d with groups by tile and storage-type output", GG_TM, GS_M);
-  if (tile_slots == GS_M) {
-    const int outs = glu ? 64 : 128;
-    const int n_blocks = (N + outs - 1) / outs, per = (tiles + GS_DIES - 1) / GS_DIES;
-    const long groups = (long)GS_DIES * ((per + GS_TILES - 1) / GS_TILES) * GS_TILES * n_blocks;
-    TK_REQUIRE(groups < (1l << 31), "grouped_gemm: too many outputs");
-    if (glu) hipLaunchKernelGGL(grouped_gemm_staged_kernel<true>, dim3((unsigned)groups), dim3(256), 0, stream, a, tiles, n_blocks);
-    else hipLaunchKernelGGL(grouped_gemm_staged_kernel<false>, dim3((unsigned)groups), dim3(256), 0, stream, a, tiles, n_blocks);
+  if (tile_group) {
+    TK_REQUIRE(!out_f32 && a_cols == 0 && c_cols == 0, "grouped_gemm: groups by tile write the storage type and have no columns of their own");
+    TK_REQUIRE(glu ? launch_staged<true>(a, tiles, stream) : launch_staged<false>(a, tiles, stream), "grouped_gemm: too many outputs");
     TK_CHECK_LAUNCH("grouped_gemm");
     return 0;
   }
-  const int nt = glu ? 2 : 4;
-  const dim3 grid(tiles, (N + GG_WAVES * nt * 16 - 1) / (GG_WAVES * nt * 16), groups_z > 0 ? groups_z : 1);
-  TK_REQUIRE(grid.y < 65536 && grid.z < 65536, "grouped_gemm: too many outputs or groups");
-  if (glu)
-    hipLaunchKernelGGL((grouped_gemm_kernel<2, true, false>), grid, dim3(GG_WAVES * TK_WAVE), 0, stream, a);
-  else if (out_f32)
-    hipLaunchKernelGGL((grouped_gemm_kernel<4, false, true>), grid, dim3(GG_WAVES * TK_WAVE), 0, stream, a);
+  TK_REQUIRE(!glu && !a_row && !c_row, "grouped_gemm: groups by the grid take plain rows and have no gated form");
+  const dim3 grid(tiles, (N + GG_WAVES * 64 - 1) / (GG_WAVES * 64), groups_z);
+  TK_REQUIRE((long)tiles * GG_TM >= slots && grid.y < 65536 && grid.z < 65536, "grouped_gemm: too few tiles, or too many outputs or groups");
+  if (out_f32)
+    hipLaunchKernelGGL((grouped_gemm_kernel<4, true>), grid, dim3(GG_WAVES * TK_WAVE), 0, stream, a);
   else
-    hipLaunchKernelGGL((grouped_gemm_kernel<4, false, false>), grid, dim3(GG_WAVES * TK_WAVE), 0, stream, a);
+    hipLaunchKernelGGL((grouped_gemm_kernel<4, false>), grid, dim3(GG_WAVES * TK_WAVE), 0, stream, a);
   TK_CHECK_LAUNCH("grouped_gemm");
   return 0;
 }
@@ -314,7 +380,7 @@ TK_API int tk_grouped_gemm_bf16(const void* A, int lda, const int* a_row, const 
 // --------------------------------------------------------------------------
 // Pairs (token, place) -> slots sorted by expert.  A workgroup a job: a layer's choice, or (where the choice of several layers
 // is known before the first of them runs) all layers' in one launch.  Expert e's pairs take the slots
-// first[e] .. first[e] + count[e] - 1 with first[e] a multiple of tm; the slots between a run's end and the
+// first[e] .. first[e] + count[e] - 1 with first[e] a multiple of GS_M; the slots between a run's end and the
 // next multiple are empty.  slot_pair[slot] = the pair (or -1), slot_token[slot] = its token (or -1),
 // tile_group[tile] = the expert whose run the tile lies in (or -1), tile_group[max_tiles] = the tiles in use.  Pairs of identity experts (ids >= experts)
 // and empty places (ids < 0) get no slot.  Which of an expert's slots a pair gets depends on the order of
@@ -323,7 +389,7 @@ TK_API int tk_grouped_gemm_bf16(const void* A, int lda, const int* a_row, const 
 struct SortJob {
   const int* ids;
   int *slot_pair, *slot_token, *tile_group;
-  int pairs, top, experts, max_tiles, tm;
+  int pairs, top, experts, max_tiles;
 };
 #define SORT_JOBS 48
 struct SortJobs {
@@ -332,7 +398,7 @@ struct SortJobs {
 __global__ __launch_bounds__(1024) void expert_sort_kernel(SortJobs jobs) {
   const SortJob& jb = jobs.job[blockIdx.x];
   const int* __restrict__ ids = jb.ids;
-  const int pairs = jb.pairs, top = jb.top, experts = jb.experts, max_tiles = jb.max_tiles, tm = jb.tm;
+  const int pairs = jb.pairs, top = jb.top, experts = jb.experts, max_tiles = jb.max_tiles, tm = GS_M;
   int* __restrict__ slot_pair = jb.slot_pair;
   int* __restrict__ slot_token = jb.slot_token;
   int* __restrict__ tile_group = jb.tile_group;
@@ -379,8 +445,7 @@ TK_API int tk_expert_sort(const SortJob* jobs, int n_jobs, hipStream_t stream) {
     for (int k = 0; k < n; ++k) {
       const SortJob& j = all.job[k] = jobs[first + k];
       TK_REQUIRE(j.ids && j.slot_pair && j.slot_token && j.tile_group && j.pairs >= 0 && j.top > 0 && j.experts > 0, "expert_sort: bad arguments");
-      TK_REQUIRE(j.tm == GG_TM || j.tm == GS_M, "expert_sort: tiles of %d slots", j.tm);
-      TK_REQUIRE(j.max_tiles >= (j.pairs + j.tm - 1) / j.tm + j.experts, "expert_sort: %d tiles cannot hold %d pairs of %d experts", j.max_tiles,
+      TK_REQUIRE(j.max_tiles >= (j.pairs + GS_M - 1) / GS_M + j.experts, "expert_sort: %d tiles cannot hold %d pairs of %d experts", j.max_tiles,
                  j.pairs, j.experts);
       TK_REQUIRE(3 * j.experts * sizeof(int) <= 48 * 1024, "expert_sort: too many experts");
       most = max(most, j.experts);

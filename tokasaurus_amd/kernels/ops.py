@@ -2109,9 +2109,13 @@ def squared_relu_(x: torch.Tensor) -> torch.Tensor:
 # a matrix a head; experts of which a token uses a few
 # --------------------------------------------------------------------------
 
-GROUPED_TILE = 64  # slots a tile of the grouped matrix-core product (GG_TM of grouped_gemm.hip)
-GROUPED_LARGE_TILE = 128  # of the one that goes through local memory (GS_M)
-GROUPED_LARGE_FROM = 96  # pairs an expert has on average from which on the experts' products take the large tiles
+HEAD_TILE = 64  # rows a tile of the product with a matrix a head (GG_TM of grouped_gemm.hip)
+EXPERT_TILE = 128  # slots a tile of the experts' products (GS_M)
+# Pairs (token, chosen expert) below which the experts' products stay with the kernels of a workgroup a pair, which read an
+# expert's weights for every pair that names it: 32 experts of 2,048 x 1,024, 8 chosen, in us a pair each / in tiles: 8 tokens
+# 112 / 99, 6 tokens 90 / 98; 64 experts of 1,024 x 512, 2 chosen: 24 tokens 29 / 42, 32 tokens 36 / 41.  (And from
+# GROUPED_FROM_ROWS rows on only: the tiles round an expert's rows before they are added.)
+EXPERT_TILES_FROM_PAIRS = 64
 GROUPED_FROM_ROWS = 12  # rows above which the products of experts and of heads run in tiles on the matrix cores
 
 
@@ -2144,9 +2148,9 @@ def head_linear(x: torch.Tensor, w: torch.Tensor, out_f32: bool = False, positio
     if not head_linear_is_fused(x, w):
         _need(freq is None and gate is None, "head_linear: so many rows are rotated and gated in passes of their own")
         # many rows: tiles of 32 rows on the matrix cores, the head as the tile's group
-        tiles = -(-x.shape[0] // GROUPED_TILE)
+        tiles = -(-x.shape[0] // HEAD_TILE)
         call("tk_grouped_gemm_bf16", x.data_ptr(), x.stride(0), None, None, None, tiles, heads, n_in, n_out, w.data_ptr(),
-             n_out * n_in, y.data_ptr(), y.stride(0), n_out, n_in, x.shape[0], 0, 1 if out_f32 else 0, None, None, GROUPED_TILE, 0.0, 0.0,
+             n_out * n_in, y.data_ptr(), y.stride(0), n_out, n_in, x.shape[0], 0, 1 if out_f32 else 0, None, None, 0.0, 0.0,
              _stream())
         return y
     if freq is not None:
@@ -2232,7 +2236,7 @@ class _SortJob(ctypes.Structure):
     """One choice to be sorted by expert (struct SortJob of grouped_gemm.hip)."""
 
     _fields_ = [("ids", ctypes.c_void_p), ("slot_pair", ctypes.c_void_p), ("slot_token", ctypes.c_void_p), ("tile_group", ctypes.c_void_p),
-                ("pairs", ctypes.c_int), ("top", ctypes.c_int), ("experts", ctypes.c_int), ("max_tiles", ctypes.c_int), ("tm", ctypes.c_int)]
+                ("pairs", ctypes.c_int), ("top", ctypes.c_int), ("experts", ctypes.c_int), ("max_tiles", ctypes.c_int)]
 
 
 @dataclass
@@ -2242,7 +2246,6 @@ class SortedPairs:
     slot_pair: torch.Tensor
     slot_token: torch.Tensor
     tile_group: torch.Tensor
-    tile: int
     max_tiles: int
     shape: tuple  # of the ids
 
@@ -2254,22 +2257,21 @@ def expert_sort(choices: "list[tuple[torch.Tensor, int]]") -> "list[SortedPairs]
         _gpu(ids)
         _i32(ids, "ids")
         n, top = ids.shape
-        tile = GROUPED_LARGE_TILE if n * top >= GROUPED_LARGE_FROM * experts else GROUPED_TILE
-        max_tiles = -(-(n * top) // tile) + experts
-        slots = max_tiles * tile
+        max_tiles = -(-(n * top) // EXPERT_TILE) + experts
+        slots = max_tiles * EXPERT_TILE
         book = torch.empty((2 * slots + max_tiles + 1,), dtype=torch.int32, device=ids.device)
-        s = SortedPairs(book[:slots], book[slots : 2 * slots], book[2 * slots :], tile, max_tiles, (n, top))
+        s = SortedPairs(book[:slots], book[slots : 2 * slots], book[2 * slots :], max_tiles, (n, top))
         job.ids, job.slot_pair, job.slot_token, job.tile_group = (t.data_ptr() for t in (ids, s.slot_pair, s.slot_token, s.tile_group))
-        job.pairs, job.top, job.experts, job.max_tiles, job.tm = n * top, top, int(experts), max_tiles, tile
+        job.pairs, job.top, job.experts, job.max_tiles = n * top, top, int(experts), max_tiles
         out.append(s)
     call("tk_expert_sort", ctypes.addressof(jobs), len(choices), _stream())
     return out
 
 
-def experts_go_in_tiles(rows: int, dtype: torch.dtype, width: int, ff: int) -> bool:
-    """Whether ``expert_mix`` sorts the pairs of so many tokens and runs the experts' products in tiles on the matrix cores
-    (for contiguous rows and weights)."""
-    return rows > GROUPED_FROM_ROWS and dtype == torch.bfloat16 and width % 8 == 0 and ff % 8 == 0
+def experts_go_in_tiles(rows: int, top: int, dtype: torch.dtype, width: int, ff: int) -> bool:
+    """Whether ``expert_mix`` sorts the pairs of so many tokens, ``top`` each, and runs the experts' products in tiles on the
+    matrix cores (for contiguous rows and weights)."""
+    return rows > GROUPED_FROM_ROWS and rows * top >= EXPERT_TILES_FROM_PAIRS and dtype == torch.bfloat16 and width % 8 == 0 and ff % 8 == 0
 
 
 def expert_mix(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor | None,
@@ -2305,20 +2307,20 @@ def expert_mix(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, i
     weight_ptr = weights.data_ptr() if weights is not None else None
     if n == 0:
         return out
-    if n > GROUPED_FROM_ROWS and _grouped_takes(h, w_gate_up, width) and ff % 8 == 0 and w_down.data_ptr() % 16 == 0:
+    if experts_go_in_tiles(n, top, h.dtype, width, ff) and _grouped_takes(h, w_gate_up, width) and w_down.data_ptr() % 16 == 0:
         # many tokens: the pairs sorted by expert, every expert's rows in tiles on the matrix cores
         if pairs is None:
             pairs = expert_sort([(ids, experts)])[0]
         _need(pairs.shape == (n, top), "expert_mix: pairs of another choice")
-        slot_pair, slot_token, tile_group, tile, max_tiles = pairs.slot_pair, pairs.slot_token, pairs.tile_group, pairs.tile, pairs.max_tiles
-        slots = max_tiles * tile
+        slot_pair, slot_token, tile_group, max_tiles = pairs.slot_pair, pairs.slot_token, pairs.tile_group, pairs.max_tiles
+        slots = max_tiles * EXPERT_TILE
         inter = torch.empty((slots, ff), dtype=h.dtype, device=h.device)
         call("tk_grouped_gemm_bf16", h.data_ptr(), h.stride(0), slot_token.data_ptr(), None, tile_group.data_ptr(), max_tiles, 0,
              0, 0, w_gate_up.data_ptr(), 2 * ff * width, inter.data_ptr(), ff, ff, width, slots, 1, 0, on_input,
-             slot_pair.data_ptr() if weights_on_input else None, tile, limit, alpha, _stream())
+             slot_pair.data_ptr() if weights_on_input else None, limit, alpha, _stream())
         y = torch.empty((n * top, width), dtype=h.dtype, device=h.device)
         call("tk_grouped_gemm_bf16", inter.data_ptr(), ff, None, slot_pair.data_ptr(), tile_group.data_ptr(), max_tiles, 0,
-             0, 0, w_down.data_ptr(), width * ff, y.data_ptr(), width, width, ff, slots, 0, 0, None, None, tile, 0.0, 0.0, _stream())
+             0, 0, w_down.data_ptr(), width * ff, y.data_ptr(), width, width, ff, slots, 0, 0, None, None, 0.0, 0.0, _stream())
         call("tk_expert_sum", h.data_ptr(), h.stride(0), y.data_ptr(), ids.data_ptr(), weight_ptr,
              shared.data_ptr() if shared is not None else None, shared_gate.data_ptr() if shared is not None else None,
              out.data_ptr(), n, width, experts, top, unit, _stream())
