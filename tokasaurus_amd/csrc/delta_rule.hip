@@ -14,15 +14,11 @@
 // The columns of S (one a value channel) do not meet: a column is owned by DR_LANES lanes that
 // cut dk between them and add up through the wavefront, always in the same order, so a token's
 // result does not depend on how its request's tokens were cut into steps or what shares the batch.
-#include "common.h"
+#include "delta_rule.h"
 
 #define DR_LANES 16    // lanes that share a column of the state (a row of the wavefront's data paths)
 #define DR_TOKENS 16   // most tokens staged in LDS at a time
-#define DR_MAX_TAPS 16
 
-__device__ __forceinline__ float silu_f32(float x) { return x / (1.0f + expf(-x)); }
-__device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + expf(-x)); }
-__device__ __forceinline__ float softplus_f32(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
 // --------------------------------------------------------------------------
 // Before the recurrence.  A token's work is cut into units, one a wavefront: a q head or a k head
@@ -315,6 +311,23 @@ __global__ __launch_bounds__(256) void gated_head_norm_kernel(const float* __res
     out[(size_t)unit * dv + i] = from_f32<T>(x[i] * rstd * w[i] * sigmoid_f32(g[i]));
 }
 
+// The tails of `C` channels moved on by the step's rows (after whoever reads the old ones).
+TK_API int tk_delta_tail(int dt, const void* proj, int ld, int taps, float* state, size_t state_stride, size_t tail_off,
+                         const int* q_start, const int* slots, int n_requests, int C, hipStream_t stream) {
+  TK_REQUIRE(taps >= 1 && taps <= DR_MAX_TAPS && ld >= C && tail_off + (size_t)(taps - 1) * C <= state_stride && n_requests < 65536,
+             "delta_tail: bad sizes taps=%d channels=%d requests=%d", taps, C, n_requests);
+  if (taps == 1 || n_requests <= 0) return 0;
+  const dim3 grid((C + 255) / 256, n_requests);
+  if (dt == TK_F32)
+    hipLaunchKernelGGL(delta_tail_kernel<float>, grid, dim3(256), 0, stream, (const float*)proj, ld, taps, state, state_stride,
+                       tail_off, q_start, slots, C);
+  else
+    hipLaunchKernelGGL(delta_tail_kernel<bf16_t>, grid, dim3(256), 0, stream, (const bf16_t*)proj, ld, taps, state, state_stride,
+                       tail_off, q_start, slots, C);
+  TK_CHECK_LAUNCH("delta_tail");
+  return 0;
+}
+
 TK_API int tk_delta_prepare(int dt, const void* proj, int ld, int col_b, const float* a_pre, int ld_a,
                             const float* conv_w, int taps, const float* a_log, const float* dt_bias,
                             float* state, size_t state_stride, size_t tail_off, const int* q_start,
@@ -347,17 +360,7 @@ TK_API int tk_delta_prepare(int dt, const void* proj, int ld, int col_b, const f
   }
 #undef DP_LAUNCH
   TK_CHECK_LAUNCH("delta_prepare");
-  if (taps > 1 && n_requests > 0 && !fuse_tail) {
-    TK_REQUIRE(n_requests < 65536, "delta_prepare: too many requests");
-    const dim3 tgrid((C + 255) / 256, n_requests);
-    if (dt == TK_F32)
-      hipLaunchKernelGGL(delta_tail_kernel<float>, tgrid, dim3(256), 0, stream, (const float*)proj, ld, taps, state,
-                         state_stride, tail_off, q_start, slots, C);
-    else
-      hipLaunchKernelGGL(delta_tail_kernel<bf16_t>, tgrid, dim3(256), 0, stream, (const bf16_t*)proj, ld, taps, state,
-                         state_stride, tail_off, q_start, slots, C);
-    TK_CHECK_LAUNCH("delta_tail");
-  }
+  if (taps > 1 && !fuse_tail) return tk_delta_tail(dt, proj, ld, taps, state, state_stride, tail_off, q_start, slots, n_requests, C, stream);
   return 0;
 }
 

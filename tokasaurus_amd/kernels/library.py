@@ -82,6 +82,11 @@ _SIGNATURES: dict[str, dict[str, list]] = {
         "tk_delta_prepare": [c_int, _P, c_int, c_int, _P, c_int, _P, c_int, _P, _P, _P, c_size_t, c_size_t, _P, _P, _P, _P]
         + [c_int] * 7 + [_P],
         "tk_delta_rule": [_P, c_int, _P, c_size_t, _P, _P, _P] + [c_int] * 6 + [_P],
+        "tk_delta_tail": [c_int, _P, c_int, c_int, _P, c_size_t, c_size_t, _P, _P, c_int, c_int, _P],
+        "tk_delta_chunks": [c_int, _P, c_int, c_int, _P, c_int, _P, c_int, _P, _P, _P, c_size_t, c_size_t, _P, _P, _P, _P, _P, _P, _P]
+        + [c_int] * 6 + [_P],
+        "tk_delta_chunk_tokens": [],
+        "tk_delta_chunk_words": [c_int, c_int],
         "tk_gated_head_norm": [c_int, _P, _P, c_int, _P, c_float, _P, c_int, c_int, c_int, _P],
         "tk_sample": [_P, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P],
         "tk_sample_static": [_P, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, _P],

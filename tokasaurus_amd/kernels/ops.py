@@ -1271,8 +1271,8 @@ def linear_attention_state_words(heads: int, key_dim: int, value_dim: int, memor
 
 @dataclass
 class ChunkPlan:
-    """A step's rows cut into chunks of ``linear_attention_chunk_tokens`` neighbouring tokens of one request, in the requests'
-    order: every chunk's request and first row, and every request's first chunk (and, last, the number of chunks), int32."""
+    """A step's rows cut into chunks of so many neighbouring tokens of one request (``linear_attention_chunk_tokens``,
+    ``delta_chunk_tokens``), in the requests' order: every chunk's request and first row, and every request's first chunk (and, last, the number of chunks), int32."""
 
     req: torch.Tensor
     row0: torch.Tensor
@@ -1949,6 +1949,63 @@ def delta_rec_width(heads: int, kv_heads: int, key_dim: int, value_dim: int) -> 
     return -(-(2 * kv_heads * key_dim + heads * value_dim + heads * key_dim + heads) // 4) * 4
 
 
+def _check_delta(proj, a_pre, conv_w, a_log, dt_bias, state, q_start, slots, heads, kv_heads, key_dim, value_dim) -> tuple[int, int]:
+    """What the delta rule reads, checked; (tokens, taps)."""
+    n = proj.shape[0]
+    channels = 2 * kv_heads * key_dim + heads * value_dim
+    _need(proj.dim() == 2 and proj.stride(1) == 1 and proj.dtype in _DT, "delta rule: rows must be 2-d with unit inner stride")
+    _need(conv_w.dim() == 2 and conv_w.shape[0] == channels and conv_w.dtype == torch.float32 and conv_w.is_contiguous(),
+          f"delta rule: the convolutions' weights must be contiguous float32 [{channels}, taps]")
+    taps = conv_w.shape[1]
+    _need(a_pre.shape == (n, heads * key_dim) and a_pre.dtype == torch.float32 and a_pre.stride(1) == 1,
+          "delta rule: the decay's projection must be float32 [tokens, heads * key_dim] with unit inner stride")
+    _f32_vector(a_log, heads, "delta rule: a_log")
+    _f32_vector(dt_bias, heads * key_dim, "delta rule: dt_bias")
+    _need(state.dim() == 2 and state.dtype == torch.float32 and state.is_contiguous()
+          and state.shape[1] >= delta_state_size(heads, kv_heads, key_dim, value_dim, taps), "delta rule: state rows too short")
+    _i32(q_start, "q_start")
+    _i32(slots, "slots")
+    _need(q_start.numel() == slots.numel() + 1, "delta rule: one slot a request")
+    return n, taps
+
+
+# Tokens of a step's longest portion from which on the delta rule goes in chunks (a step of 33 tokens takes 1.44 ms either way,
+# bound by the host; of 2,048 tokens 6.4 ms token by token and 4.4 in chunks)
+DELTA_CHUNKS_FROM = 32
+
+
+def delta_chunk_tokens(key_dim: int, value_dim: int, longest: int) -> int:
+    """Tokens of a chunk where a step whose longest portion has ``longest`` tokens goes in chunks (and so needs a
+    ``ChunkPlan`` of them), else 0."""
+    takes = longest >= DELTA_CHUNKS_FROM and load("core").tk_delta_chunk_words(int(key_dim), int(value_dim)) > 0
+    return load("core").tk_delta_chunk_tokens() if takes else 0
+
+
+def delta_rule_chunks(proj: torch.Tensor, col_b: int, a_pre: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor,
+                      dt_bias: torch.Tensor, state: torch.Tensor, q_start: torch.Tensor, slots: torch.Tensor, chunks: "ChunkPlan",
+                      heads: int, kv_heads: int, key_dim: int, value_dim: int) -> torch.Tensor:
+    """``delta_rule(delta_prepare(..))`` in chunks on the matrix cores (delta_rule_chunks.hip): o [tokens, heads * value_dim] in
+    32-bit, the matrices and tails in ``state`` moved on by the step's rows."""
+    _gpu(proj, a_pre, conv_w, a_log, dt_bias, state, q_start, slots, chunks.req)
+    n, taps = _check_delta(proj, a_pre, conv_w, a_log, dt_bias, state, q_start, slots, heads, kv_heads, key_dim, value_dim)
+    for t, name in ((chunks.req, "chunks"), (chunks.row0, "chunks"), (chunks.first, "chunks")):
+        _i32(t, name)
+    count = chunks.req.numel()
+    _need(chunks.row0.numel() == count and chunks.first.numel() == slots.numel() + 1, "delta rule: chunks of another step")
+    words = load("core").tk_delta_chunk_words(key_dim, value_dim)
+    o = torch.empty((n, heads * value_dim), dtype=torch.float32, device=proj.device)
+    rec = torch.empty((count * heads * words,), dtype=torch.float32, device=proj.device)
+    tail = heads * key_dim * value_dim
+    call("tk_delta_chunks", dtype_code(proj.dtype), proj.data_ptr(), proj.stride(0), int(col_b), a_pre.data_ptr(),
+         a_pre.stride(0) if n > 1 else heads * key_dim, conv_w.data_ptr(), taps, a_log.data_ptr(), dt_bias.data_ptr(),
+         state.data_ptr(), state.stride(0), tail, q_start.data_ptr(), slots.data_ptr(), chunks.req.data_ptr(),
+         chunks.row0.data_ptr(), chunks.first.data_ptr(), rec.data_ptr(), o.data_ptr(), count, slots.numel(), heads, kv_heads,
+         key_dim, value_dim, _stream())
+    call("tk_delta_tail", dtype_code(proj.dtype), proj.data_ptr(), proj.stride(0), taps, state.data_ptr(), state.stride(0), tail,
+         q_start.data_ptr(), slots.data_ptr(), slots.numel(), conv_w.shape[0], _stream())
+    return o
+
+
 def delta_prepare(
     proj: torch.Tensor,
     col_b: int,
@@ -1972,21 +2029,9 @@ def delta_prepare(
     softplus(a_pre + dt_bias)); beta = sigmoid(proj[:, col_b + head]).  The tails in ``state``
     are then moved on by this step's rows."""
     _gpu(proj, a_pre, conv_w, a_log, dt_bias, state, q_start, token_req, slots)
-    n = proj.shape[0]
-    channels = 2 * kv_heads * key_dim + heads * value_dim
-    _need(proj.dim() == 2 and proj.stride(1) == 1 and proj.dtype in _DT, "delta_prepare: rows must be 2-d with unit inner stride")
-    _need(conv_w.dim() == 2 and conv_w.shape[0] == channels and conv_w.dtype == torch.float32 and conv_w.is_contiguous(),
-          f"delta_prepare: the convolutions' weights must be contiguous float32 [{channels}, taps]")
-    taps = conv_w.shape[1]
-    _need(a_pre.shape == (n, heads * key_dim) and a_pre.dtype == torch.float32 and a_pre.stride(1) == 1,
-          "delta_prepare: the decay's projection must be float32 [tokens, heads * key_dim] with unit inner stride")
-    _f32_vector(a_log, heads, "delta_prepare: a_log")
-    _f32_vector(dt_bias, heads * key_dim, "delta_prepare: dt_bias")
-    _need(state.dim() == 2 and state.dtype == torch.float32 and state.is_contiguous()
-          and state.shape[1] >= delta_state_size(heads, kv_heads, key_dim, value_dim, taps), "delta_prepare: state rows too short")
-    for t, name in ((q_start, "q_start"), (token_req, "token_req"), (slots, "slots")):
-        _i32(t, name)
-    _need(token_req.numel() == n and q_start.numel() == slots.numel() + 1, "delta_prepare: one request a token, one slot a request")
+    n, taps = _check_delta(proj, a_pre, conv_w, a_log, dt_bias, state, q_start, slots, heads, kv_heads, key_dim, value_dim)
+    _i32(token_req, "token_req")
+    _need(token_req.numel() == n, "delta_prepare: one request a token")
     width = delta_rec_width(heads, kv_heads, key_dim, value_dim)
     rec = torch.empty((n, width), dtype=torch.float32, device=proj.device)
     call("tk_delta_prepare", dtype_code(proj.dtype), proj.data_ptr(), proj.stride(0), int(col_b), a_pre.data_ptr(),

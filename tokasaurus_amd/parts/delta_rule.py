@@ -22,6 +22,7 @@ import torch
 from tokasaurus_amd.kernels import ops
 from tokasaurus_amd.parts.base import CONV, MATRIX, MIXERS, NORM_WEIGHT, VECTOR, Mixer, StateNeed, StepContext, TensorSpec
 from tokasaurus_amd.parts.linear import Linear, Placer
+from tokasaurus_amd.parts.linear_attention import chunks_of
 
 
 @MIXERS.register("channel_delta_rule")
@@ -108,9 +109,14 @@ class ChannelDeltaRule(Mixer):
         proj = self.inp(h)
         low = self.low(self._columns(proj, self.col_a1, self.decay_rank + self.gate_rank), out_f32=True)
         a_pre, gate = low[:, : H * dk], low[:, H * dk :]  # 32-bit, rows a stride apart
-        rec = ops.delta_prepare(proj, self.col_b, a_pre, self.conv_w, self.a_log, self.dt_bias, state,
-                                ctx.q_start, ctx.token_req, ctx.slots, H, G, dk, dv)
-        o = ops.delta_rule(rec, state, ctx.q_start, ctx.slots, H, G, dk, dv)
+        size = ops.delta_chunk_tokens(dk, dv, ctx.max_q_len)
+        if size:
+            o = ops.delta_rule_chunks(proj, self.col_b, a_pre, self.conv_w, self.a_log, self.dt_bias, state, ctx.q_start,
+                                      ctx.slots, chunks_of(ctx, size), H, G, dk, dv)
+        else:
+            rec = ops.delta_prepare(proj, self.col_b, a_pre, self.conv_w, self.a_log, self.dt_bias, state,
+                                    ctx.q_start, ctx.token_req, ctx.slots, H, G, dk, dv)
+            o = ops.delta_rule(rec, state, ctx.q_start, ctx.slots, H, G, dk, dv)
         y = ops.gated_head_norm(o, gate, self.norm_w, self.norm_eps, H, dv, h.dtype)
         return y if rows is None else ops.gather_rows(y, rows)
 

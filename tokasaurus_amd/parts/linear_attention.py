@@ -37,13 +37,11 @@ from tokasaurus_amd.parts.base import BIAS, MATRIX, MIXERS, NORM_WEIGHT, UNIT_IN
 from tokasaurus_amd.parts.linear import Linear, Placer
 
 
-def chunk_plan(ctx: StepContext, memory: bool, key_dim: int) -> "ops.ChunkPlan | None":
-    """The step's rows in chunks, made once a step and shared by the layers; None for steps of short portions."""
-    if not ops.linear_attention_takes_chunks(memory, key_dim, ctx.max_q_len):
-        return None
-    plan = ctx.extras.get("chunk_plan")
+def chunks_of(ctx: StepContext, size: int) -> "ops.ChunkPlan":
+    """The step's rows in chunks of ``size`` tokens, made once a step and shared by the layers."""
+    key = ("chunk_plan", size)
+    plan = ctx.extras.get(key)
     if plan is None:
-        size = ops.linear_attention_chunk_tokens()
         req, row0, first = [], [], [0]
         for r in range(ctx.num_requests):
             rows = range(ctx.host_q_start[r], ctx.host_q_start[r + 1], size)
@@ -51,8 +49,15 @@ def chunk_plan(ctx: StepContext, memory: bool, key_dim: int) -> "ops.ChunkPlan |
             row0 += rows
             first.append(len(req))
         dev, n = upload(req + row0 + first, torch.int32, ctx.device), len(req)
-        plan = ctx.extras["chunk_plan"] = ops.ChunkPlan(dev[:n], dev[n : 2 * n], dev[2 * n :])
+        plan = ctx.extras[key] = ops.ChunkPlan(dev[:n], dev[n : 2 * n], dev[2 * n :])
     return plan
+
+
+def chunk_plan(ctx: StepContext, memory: bool, key_dim: int) -> "ops.ChunkPlan | None":
+    """The step's rows in linear attention's chunks; None for steps of short portions."""
+    if not ops.linear_attention_takes_chunks(memory, key_dim, ctx.max_q_len):
+        return None
+    return chunks_of(ctx, ops.linear_attention_chunk_tokens())
 
 
 class _LinearAttention(Mixer):
