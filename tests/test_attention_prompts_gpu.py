@@ -1,0 +1,122 @@
+"""Prompts in bfloat16 through the matrix-core attention of 32-bit arithmetic, one tile of 16 tokens a wavefront: steps of two
+blocks of 16 keys, the weights in three exact bfloat16 pieces, tiles dealt to the workgroups by length.  Against sums in
+64-bit."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _paged(lens, nkv, dk, dv, page, gen):
+    """Keys and values of requests of these lengths, in pages in shuffled order; every place behind a request's end is NaN."""
+    pages = [-(-n // page) for n in lens]
+    order = (torch.randperm(sum(pages), generator=gen) + 1).tolist()
+    table = torch.zeros((len(lens), max(pages)), dtype=torch.int32)
+    kc = torch.full((sum(pages) + 1, nkv, dk // 8, page, 8), float("nan"), dtype=torch.bfloat16)
+    vc = torch.full((sum(pages) + 1, nkv, page // 4, dv, 4), float("nan"), dtype=torch.bfloat16)
+    keys = [torch.randn((n, nkv, dk), generator=gen).bfloat16() for n in lens]
+    values = [torch.randn((n, nkv, dv), generator=gen).bfloat16() for n in lens]
+    for r, n in enumerate(lens):
+        for i in range(pages[r]):
+            p = table[r, i] = order.pop()
+            m = min(page, n - i * page)
+            k = torch.full((page, nkv, dk), float("nan"), dtype=torch.bfloat16)
+            v = torch.full((page, nkv, dv), float("nan"), dtype=torch.bfloat16)
+            k[:m], v[:m] = keys[r][i * page: i * page + m], values[r][i * page: i * page + m]
+            kc[p] = k.view(page, nkv, dk // 8, 8).permute(1, 2, 0, 3)
+            vc[p] = v.view(page // 4, 4, nkv, dv).permute(2, 0, 3, 1)
+    return keys, values, kc, vc, table
+
+
+def _run(q, kc, vc, table, portions, lens, nq, nkv, dk, dv, page, **options):
+    from tokasaurus_amd.kernels import ops
+
+    start = [0]
+    for n in portions:
+        start.append(start[-1] + n)
+    tiles = [(r, a) for r in range(len(lens)) for a in range(start[r], start[r + 1], 16)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    out = ops.attention_tile_f32(q.cuda().view(start[-1], nq * dk), kc.cuda(), vc.cuda(), table.cuda(), i32(start), i32(lens),
+                                 i32([r for r, _ in tiles]), i32([a for _, a in tiles]), nq, nkv, dk, dv, page, 1, **options)
+    return out.cpu().view(start[-1], nq, dv), start
+
+
+@pytest.mark.parametrize("lens,portions,nq,nkv,dk,dv,page,options", [
+    ([1], [1], 2, 1, 8, 16, 16, {}),
+    ([31, 32, 33], [31, 32, 33], 8, 2, 64, 64, 16, {}),  # the second block of a step in another page, or beyond the end
+    ([17, 300], [17, 40], 4, 2, 40, 48, 48, {}),  # a later portion of a prompt; sizes that fill no block
+    ([200], [200], 4, 4, 64, 32, 16, {"window": 40}),
+    ([200], [200], 4, 1, 32, 64, 64, {"section": 50}),
+    ([150], [150], 8, 8, 128, 128, 32, {"softcap": 5.0}),
+    ([150], [150], 4, 2, 64, 64, 32, {"score_bias": True}),
+    ([40], [40], 2, 2, 256, 256, 16, {}),  # heads too wide for two blocks a step
+    ([700, 65], [700, 65], 32, 8, 64, 64, 64, {}),  # 49 tiles x 8 workgroups: one round of 256 and a part of the next
+    ([400, 900], [400, 900], 28, 4, 64, 64, 64, {}),  # 82 tiles x 7: rounds in both directions, heads that leave wavefronts idle
+])
+def test_prompts_against_64_bit_sums(lens, portions, nq, nkv, dk, dv, page, options):
+    gen = torch.Generator().manual_seed(sum(lens) + dk)
+    keys, values, kc, vc, table = _paged(lens, nkv, dk, dv, page, gen)
+    q = torch.randn((sum(portions), nq, dk), generator=gen).bfloat16()
+    bias = torch.randn((nq,), generator=gen) if options.get("score_bias") else None
+    given = dict(options, **({"score_bias": bias.cuda()} if bias is not None else {}))
+    scale = dk ** -0.5
+    out, start = _run(q, kc, vc, table, portions, lens, nq, nkv, dk, dv, page, scale=scale, split=False, **given)
+    for r, n in enumerate(lens):
+        Q = q[start[r]: start[r + 1]].double()
+        K = keys[r].double().repeat_interleave(nq // nkv, 1)
+        V = values[r].double().repeat_interleave(nq // nkv, 1)
+        s = torch.einsum("thd,khd->htk", Q, K) * float(torch.tensor(scale, dtype=torch.float32))
+        if "softcap" in options:
+            s = options["softcap"] * torch.tanh(s / options["softcap"])
+        pos = torch.arange(n - portions[r], n)[:, None]
+        key = torch.arange(n)[None]
+        seen = key <= pos
+        if "window" in options:
+            seen = seen & (pos - key < options["window"])
+        if "section" in options:
+            seen = seen & (pos // options["section"] == key // options["section"])
+        if bias is None:
+            w = torch.softmax(s.masked_fill(~seen, float("-inf")), -1)
+        else:
+            w = torch.sigmoid(s + bias.double()[:, None, None]) * seen
+        want = torch.einsum("htk,khd->thd", w, V)
+        # the result is rounded once to bfloat16 (8 bits: up to 2^-8 of it); scores are 32-bit sums of dk products (their error moves
+        # a weight by as much, relatively), and the sums over the keys 32-bit sums of n
+        size = torch.einsum("htk,khd->thd", w, V.abs())
+        reach = float((torch.einsum("thd,khd->htk", Q.abs(), K.abs()) * scale).max())
+        limit = want.abs() * 2.0 ** -8 + size * (n + 64 + dk * reach) * 2.0 ** -23
+        assert ((out[start[r]: start[r + 1]].double() - want).abs() <= limit).all()
+
+
+def test_infinite_values_stay_infinite():
+    """A value that is infinite meets a weight's pieces that are zero: the sum must be what the 32-bit product gives."""
+    gen = torch.Generator().manual_seed(5)
+    n, page = 130, 16
+    keys, values, kc, vc, table = _paged([n], 1, 64, 64, page, gen)
+    at = 37
+    vc[table[0, at // page], 0, at % page // 4, 3, at % 4] = float("inf")
+    vc[table[0, at // page], 0, at % page // 4, 5, at % 4] = float("-inf")
+    q = torch.randn((n, 2, 64), generator=gen).bfloat16()
+    out, _ = _run(q, kc, vc, table, [n], [n], 2, 1, 64, 64, page, scale=0.125, split=False)
+    both, _ = _run(q, kc, vc, table, [n], [n], 2, 1, 64, 64, page, scale=0.125, split=True)  # 32-bit products
+    assert (out[48:, :, 3] == float("inf")).all() and (out[48:, :, 5] == float("-inf")).all()
+    assert torch.isfinite(out[:32]).all()
+    assert torch.equal(torch.isfinite(out), torch.isfinite(both)) and torch.equal(torch.isnan(out), torch.isnan(both))
+
+
+def test_which_prompts_take_a_tile_a_wavefront():
+    """With the step's longest request given, bfloat16 prompts leave the split form from 512 pairs on; single tokens do not."""
+    gen = torch.Generator().manual_seed(9)
+    lens = [300]
+    keys, values, kc, vc, table = _paged(lens, 8, 64, 64, 64, gen)
+    q = torch.randn((300, 32, 64), generator=gen).bfloat16()
+    args = (q, kc, vc, table, lens, lens, 32, 8, 64, 64, 64)
+    chosen, _ = _run(*args, longest=300)
+    plain, _ = _run(*args, split=False)
+    split, _ = _run(*args, split=True)
+    assert torch.equal(chosen, plain)
+    unknown, _ = _run(*args)  # 608 pairs, nothing known of the lengths
+    assert torch.equal(unknown, split)

@@ -19,6 +19,11 @@
 // The sum over a head's elements is permuted the same way: a lane loads whole 8-element pieces
 // of its key (the page layout's unit) and of its query, piece lane / 16 + 4 m.
 //   K pages: [page][kv head][dk / 8][P][8]    V pages: [page][kv head][P / 4][dv][4]
+// With bfloat16 storage and a tile a wavefront (prompts) a step is 32 keys and the weighted values go through the bfloat16
+// matrix cores in three exact pieces (at_pieces).  Measured, one prompt of 2,048 tokens with 32 heads of 64: 339 us with
+// 32-bit products of the weights and tiles in launch order, 101 us now; with a window of 1,024 and a soft cap 228 / 101;
+// one of 8,192 tokens 2,899 / 1,035; 32 heads of 128 780 / 303.  Results that differ from the rounded 64-bit ones: 2.9e-4
+// (3.8e-4 before).  What is left is the softmax's vector arithmetic.
 // Needs dk % 8 == 0, dv % 16 == 0, P % 16 == 0 (a step of 16 keys lies inside one page).
 #include "common.h"
 
@@ -81,10 +86,53 @@ struct ScoreShape {
   int far;
   const float* rel;
 };
-__device__ __forceinline__ float shaped_score(const ScoreShape& sh, float s, int dist, int head, int nq) {
-  if (sh.softcap > 0.f) s = sh.softcap * tanhf(s / sh.softcap);
+// `in_caps`: scale / softcap, so that the product of the stored numbers is rounded once on its way to the tanh (a
+// product and a division a score before, of which the division is ten instructions).
+__device__ __forceinline__ float shaped_score(const ScoreShape& sh, float product, float scale, float in_caps, int dist, int head, int nq) {
+  float s = sh.softcap > 0.f ? sh.softcap * tanhf(product * in_caps) : product * scale;
   if (sh.rel) s += sh.rel[(size_t)sh.bucket_of[min(max(dist, 0), sh.far)] * nq + head];
   return s;
+}
+
+// Blocks of 16 keys that a wavefront takes a step: two where the weighted values go through the bfloat16 matrix cores
+// (at_pieces) and the registers hold two blocks' keys and values twice.
+template <typename T, int KM, int VT, bool SPLIT>
+__device__ constexpr int at_halves() { return ScoresFromStorage<T>::value && !SPLIT && KM <= 4 && VT <= 8 ? 2 : 1; }
+
+// A 32-bit weight as the sum of three bfloat16 numbers, exactly (its 24 bits, 8 at a time): a bfloat16 value times each
+// is exact in 32-bit, so three products of v_mfma_f32_16x16x32_bf16 add what eight of v_mfma_f32_16x16x4_f32 add, in a
+// quarter of their time.  piece[n] holds what a lane's operand needs: the pieces of its 8 keys' weights.
+// An infinite value would meet pieces that are zero (NaN where the 32-bit product is infinite): a wavefront that ends
+// with a sum that is not finite walks its keys again with 32-bit products.
+__device__ __forceinline__ void at_pieces(const float (&p)[8], bf16x8_t (&piece)[3]) {
+  uint32_t packed[3][4];
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) {
+    float a = p[i], b = p[i + 1];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+      const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
+      packed[n][i / 2] = __builtin_amdgcn_perm(ub, ua, 0x07060302);  // the upper halves, a's below
+      a -= __uint_as_float(ua & 0xffff0000u);
+      b -= __uint_as_float(ub & 0xffff0000u);
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < 3; ++n) __builtin_memcpy(&piece[n], packed[n], sizeof(piece[n]));
+}
+
+// Which (tile, block of heads) a workgroup takes.  Causal tiles late in a prompt see many keys, early ones few, and
+// workgroups land on the compute units in turn: with tiles in launch order a unit gets the same place of the prompt
+// again and again (2,048 tokens and 8 blocks of heads: every 256th workgroup is the same tile).
+// So the late tiles go first, and every other round of 256 workgroups runs the other way; blocks of heads vary fastest, so that those of one number meet in one
+// chiplet's cache (workgroups go round the 8 chiplets) where their count is 8.
+__device__ __forceinline__ void at_place(int& tile, int& hy) {
+  const int nx = gridDim.x, ny = gridDim.y, all = nx * ny;
+  int id = blockIdx.x + nx * blockIdx.y;
+  const int base = id & ~255;
+  if ((base & 256) && base + 256 <= all) id = base + ((31 - ((id & 255) >> 3)) << 3) + (id & 7);
+  tile = nx - 1 - id / ny;
+  hy = id % ny;
 }
 
 // SPLIT: the NW wavefronts of a workgroup share one tile and take its key steps in turn
@@ -95,8 +143,10 @@ __device__ __forceinline__ float shaped_score(const ScoreShape& sh, float s, int
 // (tile, head block, chunk): blockIdx.z names the chunk.  A workgroup leaves its maxima, sums and weighted values
 // unnormalised in `part`; attention_tile_merge_kernel adds the chunks in ascending order.  For single decoded
 // tokens after long contexts, where a tile's walk would else keep one workgroup busy and the chip idle.
+//
+// (Four wavefronts a SIMD for heads up to 64 elements: one hides the loads and the exponentials of another.)
 template <typename T, int KM, int VT, bool SPLIT, int NW, bool PART = false>
-__global__ __launch_bounds__(NW * TK_WAVE) void attention_tile_f32_kernel(
+__global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 1) void attention_tile_f32_kernel(
     const T* __restrict__ q, int q_stride, T* __restrict__ out, int out_stride, const T* __restrict__ kcache,
     const T* __restrict__ vcache, const int* __restrict__ block_table, int table_stride,
     const int* __restrict__ q_start, const int* __restrict__ kv_len, const int* __restrict__ tile_req,
@@ -107,11 +157,12 @@ __global__ __launch_bounds__(NW * TK_WAVE) void attention_tile_f32_kernel(
   const int lane = threadIdx.x & (TK_WAVE - 1), wave = threadIdx.x / TK_WAVE;
   const int group = nq / nkv;
   const int blocks_per_kv = group / gg;  // head blocks of gg heads
-  const int hb = SPLIT ? blockIdx.y : blockIdx.y * NW + wave;
+  int tile = blockIdx.x, hy = blockIdx.y;
+  if constexpr (!SPLIT) at_place(tile, hy);
+  const int hb = SPLIT ? hy : hy * NW + wave;
   if (hb >= nkv * blocks_per_kv) return;
   const int kvh = hb / blocks_per_kv;
   const int head0 = kvh * group + (hb % blocks_per_kv) * gg;
-  const int tile = blockIdx.x;
   const int r = tile_req[tile];
   const int row0 = tile_row0[tile];
   const int tt = 16 / gg;
@@ -157,13 +208,12 @@ __global__ __launch_bounds__(NW * TK_WAVE) void attention_tile_f32_kernel(
   }
 
   v4f o[VT];
-#pragma unroll
-  for (int t = 0; t < VT; ++t) o[t] = (v4f){0.f, 0.f, 0.f, 0.f};
   const bool sig = score_bias != nullptr;
+  const float in_caps = shape.softcap > 0.f ? scale / shape.softcap : 0.f;
   const bool shaped = shape.softcap > 0.f || shape.rel != nullptr;
   const float pb = sig && live ? score_bias[head] : 0.f;
   // (sigmoid weights have no maximum to follow: it stays 0, so every merge below multiplies by exp(0))
-  float m_run = sig ? 0.f : -INFINITY, l_run = 0.f;  // l_run: this lane's share of the column's sum
+  float m_run, l_run;  // l_run: this lane's share of the column's sum
 
   // where this lane's pieces of a key and its values lie inside a page, for the page's first key: both offsets
   // grow linearly with the key's place in the page (8 elements a key, dv a key)
@@ -172,138 +222,177 @@ __global__ __launch_bounds__(NW * TK_WAVE) void attention_tile_f32_kernel(
   for (int m = 0; m < KM; ++m) koff[m] = (int)key_offset(P, col, (c + 4 * m < pieces ? c + 4 * m : 0) * 8);
 #pragma unroll
   for (int t = 0; t < VT; ++t) voff[t] = (int)value_offset(dv, 4 * c, 16 * t < dv ? 16 * t + col : 0);
-  const int step = SPLIT ? 16 * NW : 16;
-  int k0 = (lo_tile / 16) * 16 + (SPLIT ? 16 * wave : 0);
-  // The pages of this wavefront's steps, 64 steps at a time: lane j asks for the page of step `base + j`, and a
-  // step reads its page's number from that lane.  So no load of keys or values waits for a load of a page number.
-  const int k_first = k0;
+  constexpr int H = at_halves<T, KM, VT, SPLIT>();  // blocks of 16 keys a step
+  const int step = SPLIT ? 16 * NW : 16 * H;
+  const int k_first = (lo_tile / (16 * H)) * (16 * H) + (SPLIT ? 16 * wave : 0);
+  // The pages of this wavefront's blocks of keys, 64 blocks at a time: lane j asks for the page of block `base + j`, and
+  // a step reads its pages' numbers from those lanes.  So no load of keys or values waits for a load of a page number.
   int pv = 0;
 #define AT_PAGES(BASE)                                                  \
   do {                                                                  \
-    const int kj = k_first + ((BASE) + lane) * step;                    \
+    const int kj = k_first + ((BASE) + lane) * (step / H);              \
     pv = kj <= last ? max(table[kj / P], 0) : 0;                        \
   } while (0)
-  AT_PAGES(0);
-  // this lane's pieces of key k0 + col and its values (element 16 t + col of keys k0 + 4 c + i); the keys are
-  // asked for a step ahead, and (SPLIT, where nothing else hides the wait) the values too
-  Raw8<T> kr[KM];
-  Raw4<T> vr[VT];
-  if (k0 <= last) {
-    const int page = __builtin_amdgcn_readlane(pv, 0);
-    const T* kbase = kcache + ((size_t)page * nkv + kvh) * key_page + (k0 % P) * 8;
+  // `wide`: the weighted values as 32-bit products (see at_pieces)
+  auto walk = [&](auto wide) {
 #pragma unroll
-    for (int m = 0; m < KM; ++m) kr[m] = *(const Raw8<T>*)(kbase + koff[m]);
-    if constexpr (SPLIT) {
-      const T* vbase = vcache + ((size_t)page * nkv + kvh) * P * dv + (k0 % P) * dv;
+  for (int t = 0; t < VT; ++t) o[t] = (v4f){0.f, 0.f, 0.f, 0.f};
+  m_run = sig ? 0.f : -INFINITY;
+  l_run = 0.f;
+  int k0 = k_first;
+  AT_PAGES(0);
+  // this lane's pieces of key k0 + 16 h + col and its values (element 16 t + col of keys k0 + 16 h + 4 c + i); the keys
+  // are asked for a step ahead, and (SPLIT, where nothing else hides the wait) the values too
+  Raw8<T> kr[H][KM];
+  Raw4<T> vr[H][VT];
+  auto load_keys = [&](Raw8<T>(&dst)[H][KM], int at, int block) {
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const int page = __builtin_amdgcn_readlane(pv, (block + h) & 63);
+      const T* kbase = kcache + ((size_t)page * nkv + kvh) * key_page + ((at + 16 * h) % P) * 8;
+#pragma unroll
+      for (int m = 0; m < KM; ++m) dst[h][m] = *(const Raw8<T>*)(kbase + koff[m]);
+    }
+  };
+  auto load_values = [&](Raw4<T>(&dst)[H][VT], int at, int block) {
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const int page = __builtin_amdgcn_readlane(pv, (block + h) & 63);
+      const T* vbase = vcache + ((size_t)page * nkv + kvh) * P * dv + ((at + 16 * h) % P) * dv;
 #pragma unroll
       for (int t = 0; t < VT; ++t)
-        if (16 * t < dv) vr[t] = *(const Raw4<T>*)(vbase + voff[t]);
+        if (16 * t < dv) dst[h][t] = *(const Raw4<T>*)(vbase + voff[t]);
     }
+  };
+  if (k0 <= last) {
+    load_keys(kr, k0, 0);
+    if constexpr (SPLIT) load_values(vr, k0, 0);
   }
   int j = 0;
 #pragma unroll 1
-  for (; k0 <= last; k0 += step, ++j) {
-    if constexpr (!SPLIT) {
-      const int page = __builtin_amdgcn_readlane(pv, j & 63);
-      const T* vbase = vcache + ((size_t)page * nkv + kvh) * P * dv + (k0 % P) * dv;
-#pragma unroll
-      for (int t = 0; t < VT; ++t)
-        if (16 * t < dv) vr[t] = *(const Raw4<T>*)(vbase + voff[t]);
-    }
-    Raw8<T> kn[KM];
-    Raw4<T> vn[VT];
+  for (; k0 <= last; k0 += step, j += H) {
+    if constexpr (!SPLIT) load_values(vr, k0, j);
+    Raw8<T> kn[H][KM];
+    Raw4<T> vn[H][VT];
     const int k1 = k0 + step;
     if (k1 <= last) {
-      if (((j + 1) & 63) == 0) AT_PAGES(j + 1);
-      const int page1 = __builtin_amdgcn_readlane(pv, (j + 1) & 63);
-      const T* kbase = kcache + ((size_t)page1 * nkv + kvh) * key_page + (k1 % P) * 8;
-#pragma unroll
-      for (int m = 0; m < KM; ++m) kn[m] = *(const Raw8<T>*)(kbase + koff[m]);
-      if constexpr (SPLIT) {
-        const T* vbase = vcache + ((size_t)page1 * nkv + kvh) * P * dv + (k1 % P) * dv;
-#pragma unroll
-        for (int t = 0; t < VT; ++t)
-          if (16 * t < dv) vn[t] = *(const Raw4<T>*)(vbase + voff[t]);
-      }
+      if (((j + H) & 63) == 0) AT_PAGES(j + H);
+      load_keys(kn, k1, j + H);
+      if constexpr (SPLIT) load_values(vn, k1, j + H);
     }
     // S^T = K Q^T (a piece beyond the head's size meets zeros of the query)
-    v4f s = (v4f){0.f, 0.f, 0.f, 0.f};
-    if constexpr (STORED) {
+    v4f s[H];
 #pragma unroll
-      for (int m = 0; m < KM; ++m)
-        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kr[m]), as_bf16x8(qraw[m]), s, 0, 0, 0);
-    } else {
+    for (int h = 0; h < H; ++h) {
+      s[h] = (v4f){0.f, 0.f, 0.f, 0.f};
+      if constexpr (STORED) {
 #pragma unroll
-      for (int m = 0; m < KM; ++m)
+        for (int m = 0; m < KM; ++m)
+          s[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kr[h][m]), as_bf16x8(qraw[m]), s[h], 0, 0, 0);
+      } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          s = __builtin_amdgcn_mfma_f32_16x16x4f32(to_f32<T>(kr[m].v[e]), qv[m][e], s, 0, 0, 0);
+        for (int m = 0; m < KM; ++m)
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            s[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_f32<T>(kr[h][m].v[e]), qv[m][e], s[h], 0, 0, 0);
+      }
     }
-    // this lane now holds, for its column, keys k0 + 4 c + i
-    float sc[4];
+    // this lane now holds, for its column, keys k0 + 16 h + 4 c + i: number 4 h + i below
+    float sc[4 * H];
     float tmax = -INFINITY;
     // a step that every column of the tile sees whole needs no masks (the same for all lanes)
-    const bool whole = k0 + 15 <= pos0 && (window <= 0 || last_all - k0 < window) && k0 >= lo_last && n_tok * gg == 16;
+    const bool whole = k0 + 16 * H - 1 <= pos0 && (window <= 0 || last_all - k0 < window) && k0 >= lo_last && n_tok * gg == 16;
     if (whole) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        sc[i] = s[i] * scale;
-        if (shaped) sc[i] = shaped_score(shape, sc[i], pos - (k0 + 4 * c + i), head, nq);
+      for (int i = 0; i < 4 * H; ++i) {
+        const int kp = k0 + 16 * (i / 4) + 4 * c + i % 4;
+        sc[i] = shaped ? shaped_score(shape, s[i / 4][i % 4], scale, in_caps, pos - kp, head, nq) : s[i / 4][i % 4] * scale;
         tmax = fmaxf(tmax, sc[i]);
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int kp = k0 + 4 * c + i;
+      for (int i = 0; i < 4 * H; ++i) {
+        const int kp = k0 + 16 * (i / 4) + 4 * c + i % 4;
+        const float si = s[i / 4][i % 4];
         const bool seen = live && kp <= pos && kp >= lo_col && (window <= 0 || pos - kp < window);
-        sc[i] = seen ? (shaped ? shaped_score(shape, s[i] * scale, pos - kp, head, nq) : s[i] * scale) : -INFINITY;
+        sc[i] = seen ? (shaped ? shaped_score(shape, si, scale, in_caps, pos - kp, head, nq) : si * scale) : -INFINITY;
         tmax = fmaxf(tmax, sc[i]);
         // a key that no column sees may be anything (a page's places behind the request's last token, a page given back):
         // its weight is zero, and so must its values be, or a NaN there would reach the sums
         if (kp > last_all || kp < first_seen) {
 #pragma unroll
-          for (int t = 0; t < VT; ++t) vr[t].v[i] = from_f32<T>(0.f);
+          for (int t = 0; t < VT; ++t) vr[i / 4][t].v[i % 4] = from_f32<T>(0.f);
         }
       }
     }
-    float p[4];
+    float p[4 * H];
     float alpha = 1.f;
     if (sig) {
       // 1 / (1 + exp(-(score + bias))); a masked score gives 1 / (1 + inf) = 0
 #pragma unroll
-      for (int i = 0; i < 4; ++i) p[i] = 1.0f / (1.0f + exp2f(-(sc[i] + pb) * 1.44269504088896341f));
+      for (int i = 0; i < 4 * H; ++i) p[i] = 1.0f / (1.0f + exp2f(-(sc[i] + pb) * 1.44269504088896341f));
     } else {
       tmax = fmaxf(tmax, __shfl_xor(tmax, 16, TK_WAVE));
       tmax = fmaxf(tmax, __shfl_xor(tmax, 32, TK_WAVE));
       const float m_new = fmaxf(m_run, tmax);
       if (m_new == -INFINITY) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) p[i] = 0.f;
+        for (int i = 0; i < 4 * H; ++i) p[i] = 0.f;
       } else {
         // exp2 of the difference times log2(e): the hardware's own exponential (a masked score gives exp2(-inf) = 0)
         alpha = exp2f((m_run - m_new) * 1.44269504088896341f);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) p[i] = exp2f((sc[i] - m_new) * 1.44269504088896341f);
+        for (int i = 0; i < 4 * H; ++i) p[i] = exp2f((sc[i] - m_new) * 1.44269504088896341f);
       }
       m_run = m_new;
       l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
+      if constexpr (H == 2) l_run += (p[4] + p[5]) + (p[6] + p[7]);
     }
     // O^T += V^T P^T
 #pragma unroll
-    for (int t = 0; t < VT; ++t) {
-      if (16 * t < dv) {
-        v4f acc = o[t] * alpha;
+    for (int t = 0; t < VT; ++t) o[t] = o[t] * alpha;
+    if constexpr (decltype(wide)::value) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(to_f32<T>(vr[t].v[i]), p[i], acc, 0, 0, 0);
-        o[t] = acc;
+      for (int t = 0; t < VT; ++t) {
+        if (16 * t < dv) {
+#pragma unroll
+          for (int i = 0; i < 4 * H; ++i)
+            o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_f32<T>(vr[i / 4][t].v[i % 4]), p[i], o[t], 0, 0, 0);
+        }
+      }
+    } else if constexpr (H == 2) {
+      bf16x8_t piece[3];
+      at_pieces(p, piece);
+#pragma unroll
+      for (int n = 2; n >= 0; --n)
+#pragma unroll
+        for (int t = 0; t < VT; ++t)
+          if (16 * t < dv) {
+            Raw8<T> v8;
+            __builtin_memcpy(&v8.v[0], &vr[0][t], sizeof(vr[0][t]));
+            __builtin_memcpy(&v8.v[4], &vr[1][t], sizeof(vr[1][t]));
+            o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v8), piece[n], o[t], 0, 0, 0);
+          }
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+#pragma unroll
+      for (int m = 0; m < KM; ++m) kr[h][m] = kn[h][m];
+      if constexpr (SPLIT) {
+#pragma unroll
+        for (int t = 0; t < VT; ++t) vr[h][t] = vn[h][t];
       }
     }
+  }
+  };
+  walk(std::integral_constant<bool, H == 1>{});
+  if constexpr (H == 2) {
+    bool finite = true;
 #pragma unroll
-    for (int m = 0; m < KM; ++m) kr[m] = kn[m];
-    if constexpr (SPLIT) {
+    for (int t = 0; t < VT; ++t)
 #pragma unroll
-      for (int t = 0; t < VT; ++t) vr[t] = vn[t];
-    }
+      for (int i = 0; i < 4; ++i) finite = finite && fabsf(o[t][i]) < INFINITY;
+    if (!__all(finite)) walk(std::integral_constant<bool, true>{});
   }
 #undef AT_PAGES
   // the column's sum, from the four lanes that share it (always in this order)

@@ -1840,6 +1840,12 @@ def attention_tile_turns_halves(value_dim: int) -> bool:
 
 
 ATTENTION_TILE_SPLIT_BELOW = 2048  # (tile, head block) pairs of a step below which the wavefronts share tiles
+# The same for bfloat16 prompts, whose wavefronts walk two blocks of keys a step when each has a tile of its own: where no
+# token sees more keys than the step has tokens.  Split / one tile a wavefront on an MI355X, 32 heads of 64: 256 tokens
+# (512 pairs) 20.7 / 17.4 us, 512 tokens 48.6 / 27.8, 1,024 tokens 124 / 50, four prompts of 100 (896 pairs) 28 / 16; 16
+# heads of 128: 384 tokens (384 pairs) 37 / 33, 256 tokens 18.8 / 25.8; 8 heads of 64: 768 tokens (384 pairs) 29 / 37,
+# 1,024 tokens 39 / 46, 2,048 tokens 102 / 85.  Single tokens after long contexts are one long walk each: they stay split.
+ATTENTION_TILE_SPLIT_PROMPTS_BELOW = 512
 ATTENTION_TILE_WORKGROUPS = 512  # workgroups a step with key chunks should have before its chunks grow
 ATTENTION_TILE_LONGEST_CHUNK = 2048
 
@@ -1888,7 +1894,10 @@ def attention_tile_f32(
                            and gate.shape[0] == q.shape[0]), "attention: one gate a token and head, of the rows' type")
     _f32_vector(score_bias, nq, "attention: the scores' biases")
     if split is None:
-        split = tile_req.numel() * nkv * ((nq // nkv) // int(heads_a_tile)) < ATTENTION_TILE_SPLIT_BELOW
+        pairs = tile_req.numel() * nkv * ((nq // nkv) // int(heads_a_tile))
+        seen = min(int(longest), window) if window > 0 else int(longest)
+        prompts = q.dtype == torch.bfloat16 and 0 < seen <= q.shape[0]
+        split = pairs < (ATTENTION_TILE_SPLIT_PROMPTS_BELOW if prompts else ATTENTION_TILE_SPLIT_BELOW)
     _need(q.dim() == 2 and q.stride(1) == 1 and q.shape[1] >= nq * key_dim,
           "attention: q must be 2-d with unit inner stride and nq*d leading columns")
     for t, name in ((block_table, "block_table"), (q_start, "q_start"), (kv_len, "kv_len"), (tile_req, "tile_req"), (tile_row0, "tile_row0")):
