@@ -179,3 +179,9 @@ __device__ __forceinline__ float row_sum16(float v) {
   v += dpp_row_mirror(v);
   return v;
 }
+
+// 16 bytes a lane from memory to local memory, lane l to `lds` (the same for the wavefront) + 16 l.  Counted in vmcnt, which
+// the caller waits for: the compiler knows nothing of the load.
+__device__ __forceinline__ void load_to_lds(const bf16_t* src, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
+}

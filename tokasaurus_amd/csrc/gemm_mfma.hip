@@ -11,8 +11,8 @@
 // No workgroup talks to another and partial sums inside a workgroup are added in
 // wavefront order through LDS, so every output has one fixed order of summation.
 //
-// Two kernels (the entry point chooses; the engine calls it for up to 16 rows, for the
-// stacked q, k, v product up to 32):
+// Three kernels (the entry point chooses; the engine calls it for up to 16 rows, for the
+// stacked q, k, v product up to 32, for gate and up up to 64):
 //   gemm_skinny_kernel: a workgroup owns NT tiles and all of K; its wavefronts split K
 //     and read A straight from memory.
 //   gemm_staged_kernel (a wide output, the head, from 5 rows on): a workgroup is
@@ -20,6 +20,8 @@
 //     range of their row, whose part of A passes through LDS (double buffered, 4 steps
 //     of 32 a round) so that A is read from the caches once per workgroup and not once
 //     per wavefront.
+//   gemm_glu_stream_kernel (gate and up, up to 64 rows): W and A both go straight to LDS,
+//     several steps ahead; K is walked by every wavefront.
 //
 // Norm in front (sumsq_in != null).  The product of RMSNorm(x) is rstd[row] * ((x * w) W^T).
 // The kernel that produced x (the residual epilogue below, when emit_w is given) has
@@ -598,6 +600,85 @@ __global__ __launch_bounds__(1024) void gemm_staged_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------------
+// Gate and up projections for up to 64 rows (SwiGLU epilogue; glu_streams says when): a workgroup of 4 wavefronts owns 32 pairs of weight rows
+// and all of K.  In steps of 64 elements the 64 rows of W and the rows of A (16 * MB, the last one again behind M) go
+// straight from memory to local memory, ST_STAGES - 1 steps ahead, so that a compute unit has 40 KB and more of W on the
+// way whatever the wavefronts do; two workgroups share a unit.  Wavefront w takes 8 gate rows and their 8 up rows as one
+// tile of 16: the halves of a pair meet in lanes l and l + 32.
+// LDS: [stage][64 W rows, then 16 * MB A rows][64 elements], the 16-byte piece c of row r at place c ^ (r % 8): a load
+// instruction writes 8 whole rows in lane order, and 16 rows read at one K meet in all banks.
+// Bound by reading W.  Measured against the library's product and the pass behind it (us): N = 14,336, K = 4,096 (235 MB)
+// 66 / 47.5 at 16 rows (4.9 TB/s), 55.6 / 49.7 at 32, 65 / 52.7 at 48, 54.6 / 55.4 at 64; 8,192 x 3,072 25.1 / 19.9 at 16, 27.8 / 25.2
+// at 64; 8,192 x 2,048 20.3 / 17.0 at 16, 21.1 / 18.9 at 64.
+// ---------------------------------------------------------------------------------
+#define GL_K 64
+
+template <int MB>
+__host__ __device__ constexpr int gl_stages() { return MB == 2 ? 6 : 4; }
+
+// (NB: the blocks of 16 rows that are multiplied, a constant so that a step's reads of local memory go out together.)
+template <int MB, int NB, bool NORM>
+__global__ __launch_bounds__(256, 2) void gemm_glu_stream_kernel(GemmArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int S = gl_stages<MB>(), ROWS = 64 + 16 * MB, LOADS = 2 + MB / 2;  // loads a wavefront and step
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int first = blockIdx.x * 32 + wave * 8;  // this wavefront's gate rows
+  bf16_t* rows = (bf16_t*)smem;
+  float* scales = (float*)(smem + (size_t)S * ROWS * GL_K * sizeof(bf16_t));
+  const unsigned lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) bf16_t*)rows;
+  // what this lane brings: 16 bytes of row lane / 8 of each of its wavefront's groups of 8 rows
+  const int lr = lane >> 3, piece = ((lane & 7) ^ lr) * 8;
+  const bf16_t* src[LOADS];
+  src[0] = a.W + (size_t)min(first + lr, a.N - 1) * a.K + piece;
+  src[1] = a.W + (size_t)(a.N + min(first + lr, a.N - 1)) * a.K + piece;
+#pragma unroll
+  for (int i = 0; i < MB / 2; ++i) src[2 + i] = a.A + (size_t)min((wave * (MB / 2) + i) * 8 + lr, a.M - 1) * a.lda + piece;
+  const int steps = a.K / GL_K;
+  auto ask = [&](int step) {
+    const unsigned base = lds + (unsigned)(step % S * ROWS * GL_K * sizeof(bf16_t));
+    const size_t k = (size_t)step * GL_K;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int row = i < 2 ? wave * 16 + i * 8 : 64 + (wave * (MB / 2) + i - 2) * 8;
+      load_to_lds(src[i] + k, base + (unsigned)(row * GL_K * sizeof(bf16_t)));
+    }
+  };
+  for (int s = 0; s < S - 1 && s < steps; ++s) ask(s);
+  if (NORM) row_scales<MB>(a, scales);
+  f32x4_t acc[NB];
+#pragma unroll
+  for (int mb = 0; mb < NB; ++mb) acc[mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < steps; ++s) {
+    // the step is there when only the loads of the S - 2 behind it are left; behind the barrier every wavefront's are, and
+    // every wavefront is through with the step before, whose place is filled again
+    if (s + S - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (s + S - 1 < steps) ask(s + S - 1);
+    const bf16_t* at = rows + (size_t)(s % S) * ROWS * GL_K;
+#pragma unroll
+    for (int kk = 0; kk < GL_K / 32; ++kk) {
+      const int place = ((4 * kk + q) ^ (r & 7)) * 8;
+      const bf16x8_t wv = *(const bf16x8_t*)(at + (wave * 16 + r) * GL_K + place);
+#pragma unroll
+      for (int mb = 0; mb < NB; ++mb) {
+        const bf16x8_t av = *(const bf16x8_t*)(at + (64 + 16 * mb + r) * GL_K + place);
+        acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, av, acc[mb], 0, 0, 0);
+      }
+    }
+  }
+  // lanes of q < 2 hold gate rows 4 q + j, those of q + 2 the same rows of up
+#pragma unroll
+  for (int mb = 0; mb < NB; ++mb) {
+    f32x4_t up;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) up[j] = __shfl_xor(acc[mb][j], 32, 64);
+    const int token = 16 * mb + r;
+    if (q < 2) store4<EPI_SWIGLU>(a, acc[mb], up, NORM && token < a.M ? scales[token] : 1.0f, token, first + 4 * q);
+  }
+}
+
+// ---------------------------------------------------------------------------------
 // launch
 // ---------------------------------------------------------------------------------
 template <typename Kernel>
@@ -640,6 +721,26 @@ static bool launch_staged_one(const GemmArgs& a, int groups, int WK, hipStream_t
   auto kernel = gemm_staged_kernel<MB, NT, EPI, NORM>;
   if (!allow_lds(kernel, lds)) return false;
   hipLaunchKernelGGL(kernel, dim3(groups), dim3(WK * ST_WN * 64), lds, stream, a);
+  return true;
+}
+
+// Where gate and up are streamed through local memory instead of into the wavefronts' registers.  Measured on an MI355X
+// (us, weights from memory; skinny / streamed): N = 14,336, K = 4,096: 50.5 / 47.0 at 2 rows, 55.6 / 47.1 at 8, 63.5 / 47.5 at
+// 16; 8,192 x 3,072: 24.2 / 21.1 at 2, 30.2 / 19.9 at 16; 8,192 x 2,048: 17.1 / 18.2 at 4, 18.4 / 17.0 at 16 (at 8 alone 18.1 /
+// 17.5, but a whole 1B step, with the norm in front, 1,318 / 1,347);
+// with fewer workgroups than compute units 4,096 x 2,048: 10.3 / 10.3 at 16, 11.9 / 11.7 at 20, 13.6 / 11.6 at 32; 1,000 x 1,024:
+// 6.6 / 7.0 at 32, 9.4 / 9.1 at 48.
+static bool glu_streams(int M, int N, int K) {
+  if (N >= 32 * 256) return M >= (K >= 3072 ? 2 : 16);
+  return (long)M * K >= 40000;
+}
+
+template <int MB, int NB>
+static bool launch_glu_stream(const GemmArgs& a, bool norm, hipStream_t stream) {
+  const size_t lds = (size_t)gl_stages<MB>() * (64 + 16 * MB) * GL_K * sizeof(bf16_t) + (norm ? 16 * MB * sizeof(float) : 0);
+  auto kernel = norm ? gemm_glu_stream_kernel<MB, NB, true> : gemm_glu_stream_kernel<MB, NB, false>;
+  if (!allow_lds(kernel, lds)) return false;
+  hipLaunchKernelGGL(kernel, dim3((a.N + 31) / 32), dim3(256), lds, stream, a);
   return true;
 }
 
@@ -741,7 +842,7 @@ TK_API int tk_gemm_skinny_parts(int M, int N, int tile_rows) {
 // norm in front, the outputs for a following norm and the rotation's operands.
 // waves_k: wavefronts (skinny) or wavefront rows (staged) that split K inside a workgroup
 // (0 = choose); tiles: weight tiles per wavefront, 1 or 2 (0 = choose; SwiGLU and the rotation
-// always pair); staged: -1 = choose, 0 = skinny, 1 = staged; tile_rows: weight rows of a
+// always pair); staged: -1 = choose, 0 = skinny, 1 = staged, 2 = streamed gate and up; tile_rows: weight rows of a
 // tile that the skinny kernel uses, 16 or 8 (0 = choose; tk_gemm_skinny_parts tells the
 // choice to whoever sizes emit_sumsq); fold: 0 = never fold K into the unused half of the matrix
 // core, else where it can be done (tiles of 8 weight rows, up to 8 rows of A: gemm_skinny_kernel).
@@ -803,7 +904,12 @@ TK_API int tk_gemm_skinny_bf16(const void* A, int lda, const void* W, void* C, i
   int NT = paired ? 2 : (tiles > 0 ? tiles : 1);
   TK_REQUIRE(NT == 1 || NT == 2, "gemm_skinny: tiles=%d outside 1..2", NT);
   bool ok;
-  if (use_staged) {
+  const bool stream_fits = epi == EPI_SWIGLU && M <= 64 && K % GL_K == 0;
+  TK_REQUIRE(staged != 2 || stream_fits, "gemm_skinny: the streamed gate and up product takes 64 rows and a K of a multiple of 64");
+  if (staged == 2 || (staged < 0 && stream_fits && glu_streams(M, N, K))) {
+    ok = M <= 16 ? launch_glu_stream<2, 1>(a, norm, stream)
+                 : (M <= 32 ? launch_glu_stream<2, 2>(a, norm, stream) : launch_glu_stream<4, 4>(a, norm, stream));
+  } else if (use_staged) {
     const int units = paired ? n16 : (n16 + NT - 1) / NT;  // what one wavefront row owns
     const int groups = (units + ST_WN - 1) / ST_WN;
     int WK = waves_k;

@@ -151,12 +151,6 @@ __global__ __launch_bounds__(GG_WAVES * TK_WAVE) void grouped_gemm_kernel(Groupe
 #define GS_TILES 8
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
-// 16 bytes a lane from memory to local memory, lane l to `lds` (the same for the wavefront) + 16 l.  Counted in vmcnt, which
-// the caller waits for: the compiler knows nothing of the load.
-__device__ __forceinline__ void load_to_lds(const bf16_t* src, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
-}
-
 // Tiles in a row before and behind `tile` that belong to its group `g` (both sides' first 64 asked for at once).
 __device__ __forceinline__ void gg_run(const int* tile_group, int used, int tile, int& g, int& before, int& behind) {
   const int lane = threadIdx.x & (TK_WAVE - 1);

@@ -876,6 +876,19 @@ SKINNY_A_ELEMENTS = 80_000
 def skinny_rows(inner: int, paired: bool = False) -> int:
     """Rows up to which the weight-streaming product is taken for a weight of this inner size."""
     return max(1, min(SKINNY_MAX_ROWS, SKINNY_A_ELEMENTS // (inner * (2 if paired else 1))))
+
+
+GLU_STREAM_ROWS = 64  # rows that the streamed gate and up product takes
+
+
+def glu_rows(inner: int) -> int:
+    """Rows up to which gate and up (with the gated activation behind them) take the hand-written product.  At an inner size
+    of a multiple of 64 its streamed form is ahead of the library's product and the pass behind it up to 64 rows (16 / 32 / 64
+    rows on an MI355X: 14,336 x 4,096 66 / 47.5, 55.6 / 49.7, 54.6 / 55.4 us; 8,192 x 2,048 20.3 / 17.0, 20.3 / 17.9, 21.1 / 18.9;
+    1,000 x 1,024 at 64 10.4 / 9.8); at others the crossing is that of the weight-streaming product."""
+    return GLU_STREAM_ROWS if inner % 64 == 0 else skinny_rows(inner, paired=True)
+
+
 # The stacked q, k, v product with rotation and append in its epilogue replaces two kernels of
 # the library path and has a short inner size: it stays ahead up to 32 rows (4 % of a step) at an
 # inner size of 2 048, and up to twice the rows of an ordinary paired product at wider ones.

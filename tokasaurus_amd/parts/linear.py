@@ -6,9 +6,9 @@ may be stacked along the output rows into one product (q|k|v, gate|up).  The bia
 to the 32-bit sums, before the product is rounded.
 
 Which kernel runs is decided by the storage type and the number of rows:
-  * float32: 32-bit multiply-adds throughout (the true 32-bit path);
-  * bfloat16, few rows (decode; how many depends on the inner size, ``ops.skinny_rows``): the hand-written matrix-core
-    kernel that streams the weight once and fuses the epilogue; it can also fold in the
+  * float32: 32-bit multiply-adds throughout (the true 32-bit path), on the matrix cores where the sizes fit them;
+  * bfloat16, few rows (decode; how many depends on the inner size, ``ops.skinny_rows``, and ``ops.glu_rows`` for gate and
+    up): the hand-written matrix-core kernels that stream the weight once and fuses the epilogue; it can also fold in the
     norm in front (``Normed`` input), leave what the norm behind it needs
     (``emit_norm``), and rotate and append q, k and v (``rope_append``);
   * bfloat16, more rows (large decode batches, prefill): the library's matrix product,
@@ -85,10 +85,10 @@ class Linear:
         return self.weight.shape[1] % 8 == 0
 
     def _fast(self, m: int, paired: bool = False, out_f32: bool = False) -> bool:
-        """Whether ``m`` rows take the weight-streaming kernel: up to a number of rows that
-        depends on the inner size (``ops.skinny_rows``); a 32-bit result (the head) up to
-        ``ops.SKINNY_ROWS``."""
-        limit = ops.SKINNY_ROWS if out_f32 else ops.skinny_rows(self.in_features, paired)
+        """Whether ``m`` rows take the weight-streaming kernels: up to a number of rows that
+        depends on the inner size (``ops.skinny_rows``; gate and up: ``ops.glu_rows``); a
+        32-bit result (the head) up to ``ops.SKINNY_ROWS``."""
+        limit = ops.SKINNY_ROWS if out_f32 else (ops.glu_rows if paired else ops.skinny_rows)(self.in_features)
         return self.weight.dtype == torch.bfloat16 and 0 < m <= limit and self._aligned()
 
     def __call__(
