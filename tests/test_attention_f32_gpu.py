@@ -13,7 +13,8 @@ from tokasaurus_amd.parts.linear import Placer
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("heads", [(4, 4, 16), (6, 2, 64), (8, 1, 32), (8, 2, 128)])  # groups of 1, 3, 8 and 4
+@pytest.mark.parametrize("heads", [(4, 4, 16), (6, 2, 64), (8, 1, 32), (8, 2, 128),  # groups of 1, 3, 8 and 4
+                                   (9, 3, 112), (4, 2, 48), (8, 2, 80), (4, 4, 96), (4, 1, 144)])  # heads that fill no power of two of blocks
 @pytest.mark.parametrize("page,window", [(16, 0), (32, 21), (64, 300)])
 @pytest.mark.parametrize("step", [([40, 17], [0, 9]), ([1, 1, 1], [0, 15, 700]), ([33, 2, 1, 1], [0, 290, 31, 512])])
 def test_matches_the_plain_kernel(heads, page, window, step, monkeypatch):

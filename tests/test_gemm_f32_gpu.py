@@ -23,7 +23,7 @@ def check(got, a, w, bias=None, residual=None):
 
 # tokens at the edges of the few-row kernel (16), of tiles of 32, 64 and 128 tokens; columns and K at the edges of blocks
 @pytest.mark.parametrize("m", [1, 4, 15, 16, 17, 32, 33, 64, 65, 129, 300])
-@pytest.mark.parametrize("nk", [(1, 4), (4, 12), (18, 16), (63, 36), (64, 260), (77, 512), (260, 516), (1000, 2052)])
+@pytest.mark.parametrize("nk", [(1, 4), (4, 12), (18, 16), (63, 36), (64, 260), (77, 512), (260, 516), (1000, 2052), (1133, 1008), (1008, 276)])
 def test_sizes(m, nk):
     n, k = nk
     g = torch.Generator(device="cuda").manual_seed(m * 1000 + n + k)

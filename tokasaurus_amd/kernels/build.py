@@ -4,8 +4,8 @@ There are three shared objects, loaded through ctypes (no Python headers, no tor
 headers): ``core`` holds the kernels every model needs in either storage type,
 ``mfma`` the bfloat16 matrix-core kernels and ``library`` the calls of the matrix
 product library (hipBLASLt) for many rows of bfloat16, both of which a 32-bit run
-never loads and so never compiles.  A fresh checkout builds what it needs at its first call in
-well under a minute.  ``ensure_built`` is what the loader calls: it compiles only
+never loads and so never compiles.  A fresh checkout builds what it needs at its first call, in
+about two minutes on eight processors.  ``ensure_built`` is what the loader calls: it compiles only
 when no library matching the current sources exists, and prints a line per file
 meanwhile.  The libraries live in ``tokasaurus_amd/kernels/_build``; when that
 folder cannot be written (a checkout owned by someone else) they are built in a
@@ -28,7 +28,7 @@ CSRC = Path(__file__).resolve().parent.parent / "csrc"
 IN_TREE_DIR = Path(__file__).resolve().parent / "_build"
 GROUPS = {
     "core": ["errors.hip", "elementwise.hip", "attention_generic.hip", "gemm_generic.hip", "gemm_f32.hip", "sample.hip", "step_io.hip",
-             "stream_f32.hip", "attention_prepare.hip", "attention_tile_f32.hip", "delta_rule.hip", "delta_rule_chunks.hip", "routed_experts.hip", "gated_recurrence.hip", "linear_attention.hip", "linear_attention_chunks.hip", "state_space.hip"],
+             "stream_f32.hip", "attention_prepare.hip", "attention_tile_f32.hip", "attention_tile_bf16.hip", "delta_rule.hip", "delta_rule_chunks.hip", "routed_experts.hip", "gated_recurrence.hip", "linear_attention.hip", "linear_attention_chunks.hip", "state_space.hip"],
     "mfma": ["errors.hip", "attention_mfma.hip", "gemm_mfma.hip", "grouped_gemm.hip"],
     "library": ["errors.hip", "gemm_library.hip"],
 }
