@@ -123,6 +123,12 @@ __device__ __forceinline__ void at_pieces(const float (&p)[8], bf16x8_t (&piece)
   for (int n = 0; n < 3; ++n) __builtin_memcpy(&piece[n], packed[n], sizeof(piece[n]));
 }
 
+// The result of matrix products moved to ordinary registers at this place, in front of any branch.  The compiler waits for a
+// product that is read in its own stretch of code; a read of an accumulation register behind a branch it has placed one to
+// three instructions behind the product, which then was lost (with a branch around the products of a value head's last block,
+// heads of 112 and 240 missed one key in four of their last but one).
+__device__ __forceinline__ void at_settle(v4f& x) { asm volatile("" : "+v"(x)); }
+
 // Which (tile, block of heads) a workgroup takes.  Causal tiles late in a prompt see many keys, early ones few, and
 // workgroups land on the compute units in turn: with tiles in launch order a unit gets the same place of the prompt
 // again and again (2,048 tokens and 8 blocks of heads: every 256th workgroup is the same tile).
@@ -298,6 +304,8 @@ __global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 
             s[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_f32<T>(kr[h][m].v[e]), qv[m][e], s[h], 0, 0, 0);
       }
     }
+#pragma unroll
+    for (int h = 0; h < H; ++h) at_settle(s[h]);
     // this lane now holds, for its column, keys k0 + 16 h + 4 c + i: number 4 h + i below
     float sc[4 * H];
     float tmax = -INFINITY;
@@ -350,9 +358,7 @@ __global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 
       if constexpr (H == 2) l_run += (p[4] + p[5]) + (p[6] + p[7]);
     }
     // O^T += V^T P^T
-    // (for all VT blocks, also those behind dv, whose lanes hold some of the head's first values and are never stored: with a
-    // branch around a block's products the compiler has read the accumulators of the block in front of it, on the way that
-    // skips the last one, before its last product was through, and lost that product)
+    // (for all VT blocks, also those behind dv, whose lanes hold some of the head's first values and are never stored)
 #pragma unroll
     for (int t = 0; t < VT; ++t) o[t] = o[t] * alpha;
     if constexpr (decltype(wide)::value) {
@@ -374,6 +380,8 @@ __global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 
           o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(v8), piece[n], o[t], 0, 0, 0);
         }
     }
+#pragma unroll
+    for (int t = 0; t < VT; ++t) at_settle(o[t]);
 #pragma unroll
     for (int h = 0; h < H; ++h) {
 #pragma unroll
