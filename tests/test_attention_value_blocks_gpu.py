@@ -65,3 +65,37 @@ def test_every_number_of_value_blocks(dk, dv, dtype, form):
         limit = size * (n + 64 + dk * reach) * 2.0 ** -23 + (want.abs() * 2.0 ** -8 if dtype == torch.bfloat16 else 0)
         worst = ((out[start[r]: start[r + 1]] - want).abs() - limit).amax((0, 1))
         assert float(worst.max()) <= 0, f"request {r}: element {int(worst.argmax())} of {dv}"
+
+
+@pytest.mark.parametrize("form", [{"split": False}, {"split": True}, {"split": True, "key_chunk": 128, "longest": max(LENS)}],
+                         ids=["tile a wavefront", "shared tiles", "keys cut"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["float32", "bfloat16"])
+@pytest.mark.parametrize("mask", [{}, {"window": 21}, {"section": 25}], ids=["all", "window", "sections"])
+def test_what_is_not_finite_stays_with_those_who_see_it(mask, dtype, form):
+    """An infinite value, a NaN among the values and keys that are all NaN reach the tokens that see them and no others of their
+    tile, as in the plain kernel."""
+    gen = torch.Generator().manual_seed(3)
+    d = 64
+    _, _, kc, vc, table = _paged(d, d, dtype, gen)
+    for r, at, x in ((0, 37, float("inf")), (1, 285, float("nan"))):
+        vc[table[r, at // PAGE], :, at % PAGE // 4, 5, at % 4] = x
+    for at in range(16):
+        kc[table[0, 0], 1, :, at] = float("nan")
+    q = torch.randn((sum(PORTIONS), NQ * d), generator=gen).to(dtype).cuda()
+    start = [0, PORTIONS[0], sum(PORTIONS)]
+    tiles = [(r, a) for r in range(2) for a in range(start[r], start[r + 1], 16)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    req = i32([r for r in range(2) for _ in range(PORTIONS[r])])
+    pos = i32([p for r in range(2) for p in range(LENS[r] - PORTIONS[r], LENS[r])])
+    kc, vc, table = kc.cuda(), vc.cuda(), table.cuda()
+    want = ops.paged_attention_generic(q, kc, vc, table, req, pos, NQ, NKV, d, PAGE, scale=0.125, **mask)
+    got = ops.attention_tile_f32(q, kc, vc, table, i32(start), i32(LENS), i32([r for r, _ in tiles]), i32([a for _, a in tiles]),
+                                 NQ, NKV, d, d, PAGE, 1, scale=0.125, **mask, **form)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    assert bool(torch.isinf(want).any()) and bool(torch.isnan(want).any())
+    held = torch.isfinite(want)
+    # each kernel within the bound of the test above, with a result's size below the largest value's
+    reach = float((q.float().abs().view(-1, NQ, d).sum(-1).max() * kc.float().nan_to_num(0).abs().max())) * 0.125
+    largest = float(vc.float().nan_to_num(0, 0, 0).abs().max())
+    limit = 2 * largest * (max(LENS) + 64 + d * reach) * 2.0 ** -23 + (largest * 2.0 ** -8 if dtype == torch.bfloat16 else 0)
+    assert float((got[held].double() - want[held].double()).abs().max()) <= limit

@@ -231,6 +231,12 @@ __global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 
 #pragma unroll
   for (int t = 0; t < VT; ++t) voff[t] = (int)value_offset(dv, 4 * c, 16 * t < dv ? 16 * t + col : 0);
   constexpr int H = at_halves<T, KM, VT, SPLIT>();  // blocks of 16 keys a step
+  // a step that every column of the tile sees whole needs no masks (the same for all lanes)
+  auto seen_whole = [&](int k0) {
+    return k0 + 16 * H - 1 <= pos0 && (window <= 0 || last_all - k0 < window) && k0 >= lo_last && n_tok * gg == 16;
+  };
+  auto sees = [&](int kp) { return live && kp <= pos && kp >= lo_col && (window <= 0 || pos - kp < window); };
+  bool odd = false;  // the wavefront has met a value that is not finite in a step with masks
   const int step = SPLIT ? 16 * NW : 16 * H;
   const int k_first = (lo_tile / (16 * H)) * (16 * H) + (SPLIT ? 16 * wave : 0);
   // The pages of this wavefront's blocks of keys, 64 blocks at a time: lane j asks for the page of block `base + j`, and
@@ -309,9 +315,7 @@ __global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 
     // this lane now holds, for its column, keys k0 + 16 h + 4 c + i: number 4 h + i below
     float sc[4 * H];
     float tmax = -INFINITY;
-    // a step that every column of the tile sees whole needs no masks (the same for all lanes)
-    const bool whole = k0 + 16 * H - 1 <= pos0 && (window <= 0 || last_all - k0 < window) && k0 >= lo_last && n_tok * gg == 16;
-    if (whole) {
+    if (seen_whole(k0)) {
 #pragma unroll
       for (int i = 0; i < 4 * H; ++i) {
         const int kp = k0 + 16 * (i / 4) + 4 * c + i % 4;
@@ -323,14 +327,32 @@ __global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 
       for (int i = 0; i < 4 * H; ++i) {
         const int kp = k0 + 16 * (i / 4) + 4 * c + i % 4;
         const float si = s[i / 4][i % 4];
-        const bool seen = live && kp <= pos && kp >= lo_col && (window <= 0 || pos - kp < window);
-        sc[i] = seen ? (shaped ? shaped_score(shape, si, scale, in_caps, pos - kp, head, nq) : si * scale) : -INFINITY;
+        sc[i] = sees(kp) ? (shaped ? shaped_score(shape, si, scale, in_caps, pos - kp, head, nq) : si * scale) : -INFINITY;
         tmax = fmaxf(tmax, sc[i]);
         // a key that no column sees may be anything (a page's places behind the request's last token, a page given back):
         // its weight is zero, and so must its values be, or a NaN there would reach the sums
         if (kp > last_all || kp < first_seen) {
 #pragma unroll
           for (int t = 0; t < VT; ++t) vr[i / 4][t].v[i % 4] = from_f32<T>(0.f);
+        }
+      }
+      // the same for a value that is not finite where some columns see its key and others do not; those that do get it below
+      // (the heads of one token see the same keys)
+      if (decltype(wide)::value && n_tok > 1) {
+        float zero = 0.f;  // or NaN
+#pragma unroll
+        for (int t = 0; t < VT; ++t)
+#pragma unroll
+          for (int i = 0; i < 4 * H; ++i) zero = fmaf(to_f32<T>(vr[i / 4][t].v[i % 4]), 0.f, zero);
+        if (__builtin_expect(__any(zero != 0.f), 0)) {
+          odd = true;
+#pragma unroll
+          for (int t = 0; t < VT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4 * H; ++i) {
+              T& v = vr[i / 4][t].v[i % 4];
+              v = fabsf(to_f32<T>(v)) < INFINITY ? v : from_f32<T>(0.f);
+            }
         }
       }
     }
@@ -346,7 +368,7 @@ __global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 
       const float m_new = fmaxf(m_run, tmax);
       if (m_new == -INFINITY) {
 #pragma unroll
-        for (int i = 0; i < 4 * H; ++i) p[i] = 0.f;
+        for (int i = 0; i < 4 * H; ++i) p[i] = sc[i] == -INFINITY ? 0.f : sc[i];  // (no key seen, or scores that are all NaN)
       } else {
         // exp2 of the difference times log2(e): the hardware's own exponential (a masked score gives exp2(-inf) = 0)
         alpha = exp2f((m_run - m_new) * 1.44269504088896341f);
@@ -403,6 +425,26 @@ __global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 
     if (!__all(finite)) walk(std::integral_constant<bool, true>{});
   }
 #undef AT_PAGES
+  if (__builtin_expect(odd, 0)) {
+    // the values left out of the steps with masks, each for the columns that see its key: their sums are not finite
+    int places = P, size = dv;
+    asm volatile("" : "+s"(places), "+s"(size));  // (nothing of this is made ready in front of the walk, whose registers are full)
+#pragma unroll 1
+    for (int k0 = k_first; k0 <= last; k0 += step) {
+      if (seen_whole(k0)) continue;
+#pragma unroll 1
+      for (int kp = max(k0, first_seen); kp < k0 + 16 * H && kp <= last; ++kp) {
+        const T* vbase = vcache + ((size_t)max(table[kp / places], 0) * nkv + kvh) * places * size;
+#pragma unroll
+        for (int t = 0; t < VT; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float v = 16 * t < size ? to_f32<T>(vbase[value_offset(size, kp % places, 16 * t + 4 * c + e)]) : 0.f;
+            if (sees(kp) && !(fabsf(v) < INFINITY)) o[t][e] += v;
+          }
+      }
+    }
+  }
   // the column's sum, from the four lanes that share it (always in this order)
   float l = l_run;
   l += __shfl_xor(l, 16, TK_WAVE);
