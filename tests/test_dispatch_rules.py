@@ -62,3 +62,24 @@ def test_keys_of_short_portions_after_long_pasts_are_cut():
         for keys in (100, 1000, 5000, 200000):
             s = split(w, 64, keys)
             assert s == 0 or (s % 128 == 0 and 512 <= s < keys and -(-keys // s) <= 64)
+
+
+def test_chunks_of_split_attention_take_bounded_room_and_reach_every_key():
+    words = 16 * 130
+    for groups in (1, 8, 500, 2000, 70_000):
+        for bound in (1024, 16384, 131072):
+            for longest in (1, 255, 256, 257, 1000, bound):
+                if longest > bound:
+                    continue
+                for reach in (0, 64, 300, 5000):
+                    key_chunk, chunks = ops.attention_tile_chunks(groups, 256, bound, longest, reach, words)
+                    whole, most = ops.attention_tile_chunks(groups, 256, bound, bound, reach, words)
+                    # a chunk is as long as in a recorded step of this bound, whatever the step's own requests
+                    assert key_chunk == whole and key_chunk % 256 == 0 and 1 <= chunks <= most
+                    assert groups * most * words * 4 <= ops.ATTENTION_TILE_PART_BYTES or most == 1
+                    # every tile's keys lie in its chunks: those of the tile that starts at any place of a chunk
+                    seen = min(longest, reach + 15) if reach else longest
+                    worst = (longest - 1) // key_chunk if not reach else min((longest - 1) // key_chunk, (key_chunk - 1 + seen - 1) // key_chunk)
+                    assert chunks >= worst + 1
+    # (32-bit prompts of 2,000 pairs in a step planned for 131,072 keys: one chunk where the requests are short)
+    assert ops.attention_tile_chunks(2000, 256, 131072, 500, 0, words)[1] == 1

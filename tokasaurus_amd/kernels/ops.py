@@ -1861,6 +1861,32 @@ ATTENTION_TILE_SPLIT_BELOW = 2048  # (tile, head block) pairs of a step below wh
 ATTENTION_TILE_SPLIT_PROMPTS_BELOW = 512
 ATTENTION_TILE_WORKGROUPS = 512  # workgroups a step with key chunks should have before its chunks grow
 ATTENTION_TILE_LONGEST_CHUNK = 2048
+# Room for partial results a call may take at most; a step of so many workgroups (61 000 with values of 64) has longer chunks
+ATTENTION_TILE_PART_BYTES = 256 << 20
+
+
+def attention_tile_chunks(groups: int, key_chunk: int, bound: int, longest: int, reach: int, words: int) -> tuple[int, int]:
+    """(keys a chunk, chunks a tile) of a split step of so many workgroups without chunks.  ``bound``: what the step is planned
+    for, by which a chunk's length is chosen, so that a recorded step and one launched by itself add up alike; ``longest``: the
+    step's own longest request, behind which no chunk is laid out; ``reach``: a window or a section, or 0; ``words``: 32-bit
+    numbers of a partial result."""
+    # longer chunks where the step has workgroups enough without short ones: a chunk's walk should be long
+    # enough to hide its first loads
+    # (behind a window a tile sees at most window + 15 keys, whatever the request's length: they lie in
+    # `seen // chunk + 1` chunks at most, one more when they start inside one, and the kernel counts a tile's
+    # chunks from the first it sees)
+    # (the same for a tile whose first token is the last of its section)
+    seen = min(int(bound), reach + 15) if reach > 0 else int(bound)
+    while key_chunk < ATTENTION_TILE_LONGEST_CHUNK and groups * -(-seen // (2 * key_chunk)) >= ATTENTION_TILE_WORKGROUPS:
+        key_chunk *= 2
+
+    def count(of: int) -> int:
+        chunks = -(-int(of) // key_chunk)
+        return min(chunks, -(-min(int(of), seen) // key_chunk) + 1) if reach > 0 else chunks
+
+    while count(bound) > 1 and groups * count(bound) * words * 4 > ATTENTION_TILE_PART_BYTES:
+        key_chunk *= 2
+    return key_chunk, max(1, count(min(int(longest), int(bound))))
 
 
 def attention_tile_heads(group: int, max_q_len: int) -> int:
@@ -1882,7 +1908,7 @@ def attention_tile_f32(
     sink: torch.Tensor | None = None, split: bool | None = None, key_chunk: int = 0, longest: int = 0, first_row: int = 0,
     score_bias: torch.Tensor | None = None, value_freq: torch.Tensor | None = None,
     value_pair_halves: bool = False, gate: torch.Tensor | None = None, softcap: float = 0.0,
-    distance_bias: "DistanceBias | None" = None, section: int = 0, out: torch.Tensor | None = None,
+    distance_bias: "DistanceBias | None" = None, section: int = 0, out: torch.Tensor | None = None, step_longest: int = 0,
 ) -> torch.Tensor:
     """Attention in 32-bit arithmetic on the matrix cores: every token of the step over its
     request's pages; ``tile_req`` / ``tile_row0`` name each tile's request and its first token's
@@ -1897,7 +1923,8 @@ def attention_tile_f32(
     does the result.  ``score_bias``: sigmoid weights as in ``paged_attention_generic``.  ``value_freq``,
     ``value_pair_halves``, ``gate``: what ``unrotate_gate_`` does, in the kernel's own epilogue (halves only where
     ``attention_tile_turns_halves``).  ``section`` as in ``paged_attention_generic``.  ``out``: [tokens, nq * value_dim]
-    for the result instead of new memory; only the tiles' rows are written."""
+    for the result instead of new memory; only the tiles' rows are written.  ``step_longest``: the longest request of this very
+    step (0: ``longest`` says it), see ``attention_tile_chunks``."""
     _gpu(q, kcache, vcache, block_table, q_start, kv_len, tile_req, tile_row0, sink, score_bias, value_freq, gate)
     db = _checked_distance_bias(distance_bias, nq)
     _f32_vector(value_freq, value_dim // 2, "attention: the values' frequencies")
@@ -1906,8 +1933,9 @@ def attention_tile_f32(
     _need(gate is None or (gate.dim() == 2 and gate.stride(1) == 1 and gate.shape[1] == nq and gate.dtype == q.dtype
                            and gate.shape[0] == q.shape[0]), "attention: one gate a token and head, of the rows' type")
     _f32_vector(score_bias, nq, "attention: the scores' biases")
+    pairs = tile_req.numel() * nkv * ((nq // nkv) // int(heads_a_tile))
+    own = int(step_longest) or int(longest)
     if split is None:
-        pairs = tile_req.numel() * nkv * ((nq // nkv) // int(heads_a_tile))
         seen = min(int(longest), window) if window > 0 else int(longest)
         prompts = q.dtype == torch.bfloat16 and 0 < seen <= q.shape[0]
         split = pairs < (ATTENTION_TILE_SPLIT_PROMPTS_BELOW if prompts else ATTENTION_TILE_SPLIT_BELOW)
@@ -1926,22 +1954,9 @@ def attention_tile_f32(
           "attention: the result's buffer must be contiguous [tokens, nq * value_dim] of the queries' type")
     chunks, part = 0, None
     if split and key_chunk > 0 and longest > key_chunk:
-        # longer chunks where the step has workgroups enough without short ones: a chunk's walk should be long
-        # enough to hide its first loads
-        groups = tile_req.numel() * nkv * ((nq // nkv) // int(heads_a_tile))
-        # (behind a window a tile sees at most window + 15 keys, whatever the request's length: they lie in
-        # `seen // chunk + 1` chunks at most, one more when they start inside one, and the kernel counts a tile's
-        # chunks from the first it sees)
-        # (the same for a tile whose first token is the last of its section)
-        reach = int(section) or int(window)
-        seen = min(int(longest), reach + 15) if reach > 0 else int(longest)
-        while key_chunk < ATTENTION_TILE_LONGEST_CHUNK and groups * -(-seen // (2 * key_chunk)) >= ATTENTION_TILE_WORKGROUPS:
-            key_chunk *= 2
-        chunks = -(-int(longest) // int(key_chunk))
-        if reach > 0:
-            chunks = min(chunks, -(-seen // int(key_chunk)) + 1)
         words = load("core").tk_attention_tile_part_words(value_dim)
-        part = torch.empty((tile_req.numel() * nkv * ((nq // nkv) // int(heads_a_tile)) * chunks * words,), dtype=torch.float32, device=q.device)
+        key_chunk, chunks = attention_tile_chunks(pairs, int(key_chunk), int(longest), own, int(section) or int(window), words)
+        part = torch.empty((pairs * chunks * words,), dtype=torch.float32, device=q.device)
     # the kernel finds a tile's rows by their place in the step
     q_base = q.data_ptr() - int(first_row) * q.stride(0) * q.element_size()
     out_base = out.data_ptr() - int(first_row) * out.stride(0) * out.element_size()

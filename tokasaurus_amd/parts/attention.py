@@ -255,7 +255,8 @@ class PagedAttention(Mixer):
                 tile_req, tile_row0 = tile_plan(ctx, 16 // gg, first, end)
                 ops.attention_tile_f32(
                     q, cache.keys, cache.values, cache.block_table, ctx.q_start, ctx.kv_len, tile_req, tile_row0, nq, nkv, d, d,
-                    cache.page_size, gg, window=self.window, scale=self.scale, key_chunk=256, longest=bound, out=attn)
+                    cache.page_size, gg, window=self.window, scale=self.scale, key_chunk=256, longest=bound, out=attn,
+                    step_longest=ctx.max_kv_len)
         else:
             # shapes that neither matrix-core kernel takes
             attn = ops.paged_attention_generic(

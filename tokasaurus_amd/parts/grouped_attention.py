@@ -274,8 +274,8 @@ class GroupedAttention(Mixer):
             attn = ops.attention_tile_f32(qkv, cache.keys, cache.values, cache.block_table, ctx.q_start, ctx.kv_len,
                                           tile_req, tile_row0, nq, nkv, dk, dv, cache.page_size, gg,
                                           window=self.window, scale=self.scale, sink=self.sink, key_chunk=self.key_chunk,
-                                          longest=ctx.extras.get("kv_bound", ctx.max_kv_len), score_bias=self.score_bias,
-                                          value_freq=self.value_freq if fused else None, value_pair_halves=v_halves,
+                                          longest=ctx.extras.get("kv_bound", ctx.max_kv_len), step_longest=ctx.max_kv_len,
+                                          score_bias=self.score_bias, value_freq=self.value_freq if fused else None, value_pair_halves=v_halves,
                                           gate=gate if fused else None, softcap=self.softcap, distance_bias=self.rel,
                                           section=self.section)
             after = after and not fused

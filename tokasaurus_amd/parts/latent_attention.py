@@ -258,7 +258,7 @@ class LatentAttention(Mixer):
             o = ops.attention_tile_f32(ql, cache.keys, cache.values, cache.block_table, ctx.q_start, ctx.kv_len,
                                        tile_req, tile_row0, H, 1, dc, r, cache.page_size, gg, scale=self.scale, window=self.window, sink=self.sink,
                                        key_chunk=self.key_chunk, longest=ctx.extras.get("kv_bound", ctx.max_kv_len),
-                                       first_row=first_row)
+                                       step_longest=ctx.max_kv_len, first_row=first_row)
         else:
             o = torch.empty((ql.shape[0], H * r), dtype=ql.dtype, device=ql.device)
             for h0 in range(0, H, self.heads_a_call):
