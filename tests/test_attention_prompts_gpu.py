@@ -120,3 +120,28 @@ def test_which_prompts_take_a_tile_a_wavefront():
     assert torch.equal(chosen, plain)
     unknown, _ = _run(*args)  # 608 pairs, nothing known of the lengths
     assert torch.equal(unknown, split)
+
+
+def test_an_engines_prompt_takes_a_tile_a_wavefront(tmp_path, monkeypatch):
+    """Through the runner with its default planning bound (1,024 keys), which says nothing of the step's own lengths."""
+    from kupuzen_models import TOL, attention_layer, compare_rows, make_folder, plain_rows
+    from tokasaurus_amd.engine.batch import StepEntry
+    from tokasaurus_amd.engine.runner import ModelRunner
+    from tokasaurus_amd.kernels import ops
+
+    cfg = {"architecture": "Kupuzen", "vocab": 120, "width": 64, "embedding": {"scale": 2.0}, "norm": {"eps": 1e-5}, "residual_mult": 0.7,
+           "layers": [attention_layer(32, 2, 8, 16, 0.3, rot={"base": 100.0, "dims": 8})]}
+    folder = make_folder(tmp_path / "wide", cfg, seed=4)
+    runner = ModelRunner.from_folder(str(folder), "bfloat16", page_size=16, num_pages=160, max_slots=4)
+    assert runner.kv_bound(260) == 1024
+    chosen = []
+    rule = ops.attention_tile_splits
+    monkeypatch.setattr(ops, "attention_tile_splits", lambda *a, **kw: chosen.append(rule(*a, **kw)) or chosen[-1])
+    tokens = [(7 * i + 3) % 120 for i in range(300)]
+    out = runner.run([StepEntry("a", tokens[:260], [259])])
+    assert chosen == [False]  # 17 tiles x 32 heads
+    got = {("a", 259): out.logits[0].float().cpu()}
+    runner.run([StepEntry("a", tokens[260:290], [])])  # after a past longer than the step: shared tiles
+    runner.run([StepEntry("a", tokens[290:291], [])])
+    assert len(chosen) >= 3 and all(chosen[1:])
+    compare_rows(got, plain_rows(folder, {"a": tokens}), TOL["bfloat16"])

@@ -64,6 +64,17 @@ def test_keys_of_short_portions_after_long_pasts_are_cut():
             assert s == 0 or (s % 128 == 0 and 512 <= s < keys and -(-keys // s) <= 64)
 
 
+def test_prompts_leave_the_split_attention_by_their_own_length():
+    splits = ops.attention_tile_splits
+    # 32 heads, tiles of 16 tokens: the step's own longest request decides, whatever the step is planned for
+    assert not splits(512, True, 256, 256) and splits(480, True, 240, 240)
+    assert splits(512, True, 256, 1024) and splits(512, True, 256, 0) and splits(512, False, 256, 256)
+    assert not splits(2048, False, 64, 100_000)
+    # tokens of a section or behind a window see no more than it holds, however long the request
+    assert not splits(512, True, 256, 5000, section=200) and not splits(512, True, 256, 5000, window=200)
+    assert splits(512, True, 256, 5000, section=300) and splits(512, True, 256, 5000, window=300)
+
+
 def test_chunks_of_split_attention_take_bounded_room_and_reach_every_key():
     words = 16 * 130
     for groups in (1, 8, 500, 2000, 70_000):

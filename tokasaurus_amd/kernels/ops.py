@@ -1865,6 +1865,15 @@ ATTENTION_TILE_LONGEST_CHUNK = 2048
 ATTENTION_TILE_PART_BYTES = 256 << 20
 
 
+def attention_tile_splits(pairs: int, prompts: bool, rows: int, longest: int, window: int = 0, section: int = 0) -> bool:
+    """Whether a step of so many (tile, head block) pairs takes the form whose wavefronts share a tile.  ``prompts``: bfloat16
+    rows of portions (a step of single tokens does not depend on its own lengths: it is recorded for others); ``longest``: the
+    step's own longest request (0: not known), whose tokens see at most ``window`` keys or those of their ``section``."""
+    reach = int(section) or int(window)
+    seen = min(int(longest), reach) if reach > 0 else int(longest)
+    return pairs < (ATTENTION_TILE_SPLIT_PROMPTS_BELOW if prompts and 0 < seen <= rows else ATTENTION_TILE_SPLIT_BELOW)
+
+
 def attention_tile_chunks(groups: int, key_chunk: int, bound: int, longest: int, reach: int, words: int) -> tuple[int, int]:
     """(keys a chunk, chunks a tile) of a split step of so many workgroups without chunks.  ``bound``: what the step is planned
     for, by which a chunk's length is chosen, so that a recorded step and one launched by itself add up alike; ``longest``: the
@@ -1924,7 +1933,7 @@ def attention_tile_f32(
     ``value_pair_halves``, ``gate``: what ``unrotate_gate_`` does, in the kernel's own epilogue (halves only where
     ``attention_tile_turns_halves``).  ``section`` as in ``paged_attention_generic``.  ``out``: [tokens, nq * value_dim]
     for the result instead of new memory; only the tiles' rows are written.  ``step_longest``: the longest request of this very
-    step (0: ``longest`` says it), see ``attention_tile_chunks``."""
+    step (0: ``longest`` says it), see ``attention_tile_splits`` and ``attention_tile_chunks``."""
     _gpu(q, kcache, vcache, block_table, q_start, kv_len, tile_req, tile_row0, sink, score_bias, value_freq, gate)
     db = _checked_distance_bias(distance_bias, nq)
     _f32_vector(value_freq, value_dim // 2, "attention: the values' frequencies")
@@ -1936,9 +1945,8 @@ def attention_tile_f32(
     pairs = tile_req.numel() * nkv * ((nq // nkv) // int(heads_a_tile))
     own = int(step_longest) or int(longest)
     if split is None:
-        seen = min(int(longest), window) if window > 0 else int(longest)
-        prompts = q.dtype == torch.bfloat16 and 0 < seen <= q.shape[0]
-        split = pairs < (ATTENTION_TILE_SPLIT_PROMPTS_BELOW if prompts else ATTENTION_TILE_SPLIT_BELOW)
+        prompts = q.dtype == torch.bfloat16 and tile_req.numel() < q.shape[0]
+        split = attention_tile_splits(pairs, prompts, q.shape[0], own, window, section)
     _need(q.dim() == 2 and q.stride(1) == 1 and q.shape[1] >= nq * key_dim,
           "attention: q must be 2-d with unit inner stride and nq*d leading columns")
     for t, name in ((block_table, "block_table"), (q_start, "q_start"), (kv_len, "kv_len"), (tile_req, "tile_req"), (tile_row0, "tile_row0")):
