@@ -84,3 +84,57 @@ def test_chunks_follow_the_recurrence(heads, groups, dk, dv, taps, lengths, deca
     assert torch.equal(state[untouched], before[untouched])
     tails = heads * dk * dv
     assert torch.equal(state[:, tails:], plain_state[:, tails:])
+
+
+@pytest.mark.parametrize("lengths", [[40, 5, 100, 1, 31, 1], [1, 32], [33, 1, 1, 1], [31, 64]])
+@pytest.mark.parametrize("heads,groups,dk,dv,taps", [(2, 1, 64, 72, 4), (2, 2, 20, 8, 1), (1, 1, 128, 128, 6)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_what_a_request_shares_its_step_with_changes_nothing(lengths, heads, groups, dk, dv, taps, dtype):
+    """Requests of few tokens have the recurrence's bits, those of many the chunks', whoever shares the step."""
+    g = torch.Generator(device="cuda").manual_seed(sum(lengths) + dk)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    n, C, least = sum(lengths), 2 * groups * dk + heads * dv, ops.DELTA_CHUNKS_FROM
+    starts = [sum(lengths[:i]) for i in range(len(lengths) + 1)]
+    proj = rand(n, C + heads).to(dtype)
+    a_pre, conv_w, a_log, dt_bias = rand(n, heads * dk), rand(C, taps) * 0.5, rand(heads) * 0.5, rand(heads * dk) * 0.5
+    before = rand(len(lengths) + 1, ops.delta_state_size(heads, groups, dk, dv, taps)) * 0.3
+    slots = list(range(len(lengths), 0, -1))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    args, sizes = (proj, C, a_pre, conv_w, a_log, dt_bias), (heads, groups, dk, dv)
+    req = i32([r for r, m in enumerate(lengths) for _ in range(m)])
+    one, two, both = before.clone(), before.clone(), before.clone()
+    chunked = ops.delta_rule_chunks(*args, one, i32(starts), i32(slots), cut(starts, 16), *sizes)
+    plain = ops.delta_rule(ops.delta_prepare(*args, two, i32(starts), req, i32(slots), *sizes), two, i32(starts), i32(slots), *sizes)
+    all_chunks = cut(starts, 16)
+    keep = [i for i, r in enumerate(all_chunks.req.tolist()) if lengths[r] >= least]
+    counts = [-(-m // 16) if m >= least else 0 for m in lengths]
+    plan = ops.ChunkPlan(all_chunks.req[keep].contiguous(), all_chunks.row0[keep].contiguous(),
+                         i32([sum(counts[:i]) for i in range(len(counts) + 1)]))
+    few = next((r, starts[r]) for r, m in enumerate(lengths) if m < least)
+    got = ops.delta_rule_chunks(*args, both, i32(starts), i32(slots), plan, *sizes, req, least, few)
+    for r, m in enumerate(lengths):
+        rows, slot = slice(starts[r], starts[r + 1]), slots[r]
+        want, state = (chunked, one) if m >= least else (plain, two)
+        assert torch.equal(got[rows], want[rows]) and torch.equal(both[slot], state[slot]), r
+    assert torch.equal(both[0], before[0])
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_a_model_step_of_both_kinds_of_requests(tmp_path, dtype):
+    from kupuzen_models import TOL, compare_rows, delta_layer, make_folder, plain_rows
+    from tokasaurus_amd.engine.batch import StepEntry
+    from tokasaurus_amd.engine.runner import ModelRunner
+
+    cfg = {"architecture": "Kupuzen", "vocab": 120, "width": 64, "embedding": {"scale": 2.0}, "norm": {"eps": 1e-5}, "residual_mult": 0.7,
+           "layers": [delta_layer(4, 2, 16, 24, 4, 8, 8), delta_layer(2, 2, 16, 16, 4, 8, 8)]}
+    folder = make_folder(tmp_path / "delta", cfg, seed=6)
+    tokens = {r: [(k * i + 3) % 120 for i in range(230)] for r, k in (("a", 7), ("b", 11), ("c", 13))}
+    runner = ModelRunner.from_folder(str(folder), dtype, page_size=16, num_pages=64, max_slots=4)
+    at, got = {r: 0 for r in tokens}, {}
+    for step in ({"a": 40}, {"a": 1, "b": 170, "c": 20}, {"a": 150, "b": 1, "c": 34}, {"a": 1, "b": 2, "c": 1}):
+        entries = [StepEntry(r, tokens[r][at[r] : at[r] + n], list(range(n))) for r, n in step.items()]
+        rows = runner.run(entries).logits.float().cpu()
+        places = [(r, at[r] + i) for r, n in step.items() for i in range(n)]
+        got.update(zip(places, rows))
+        at = {r: at[r] + step.get(r, 0) for r in at}
+    compare_rows(got, plain_rows(folder, tokens), TOL[dtype])

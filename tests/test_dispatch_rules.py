@@ -94,3 +94,11 @@ def test_chunks_of_split_attention_take_bounded_room_and_reach_every_key():
                     assert chunks >= worst + 1
     # (32-bit prompts of 2,000 pairs in a step planned for 131,072 keys: one chunk where the requests are short)
     assert ops.attention_tile_chunks(2000, 256, 131072, 500, 0, words)[1] == 1
+
+
+def test_which_portions_take_the_delta_rule_in_chunks():
+    chunks = ops.delta_portions_in_chunks
+    assert chunks([1]) == [False] and chunks([159]) == [False] and chunks([160]) == [True] and chunks([]) == []
+    # single tokens and short portions keep the recurrence whatever shares their step; many portions count together
+    assert chunks([300, 31, 1, 1]) == [True, False, False, False]
+    assert chunks([48] * 8 + [1]) == [True] * 8 + [False] and chunks([32, 96, 31, 1]) == [False] * 4

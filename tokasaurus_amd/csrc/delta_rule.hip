@@ -12,13 +12,14 @@
 // Per token and head, with decay g (dk), write strength beta, unit k, scaled unit q, value v:
 //   S <- diag(g) S;  u = beta * (v - S^T k);  S <- S + k u^T;  o = S^T q.
 // The columns of S (one a value channel) do not meet: a column is owned by DR_LANES lanes that
-// cut dk between them and add up through the wavefront, always in the same order, so a token's
-// result does not depend on how its request's tokens were cut into steps or what shares the batch.
+// cut dk between them and add up through the wavefront, always in the same order: among the tokens that
+// run here a result does not depend on how its request's tokens were cut into steps or what shares the batch.
+// Portions of many tokens run in delta_rule_chunks.hip instead, whose sums stand in another order: a prompt's
+// results depend in their last bits on how it was cut, single tokens' on nothing.
 #include "delta_rule.h"
 
 #define DR_LANES 16    // lanes that share a column of the state (a row of the wavefront's data paths)
 #define DR_TOKENS 16   // most tokens staged in LDS at a time
-
 
 // --------------------------------------------------------------------------
 // Before the recurrence.  A token's work is cut into units, one a wavefront: a q head or a k head
@@ -29,6 +30,7 @@
 //   rec row (32-bit): [q: G*dk | k: G*dk | v: H*dv | decay: H*dk | beta: H]
 // FUSE_TAIL (every request of the step brings one token): the lane that convolves a channel also
 // moves the channel's tail on, which it alone reads; else the kernel below does it afterwards.
+// `below` > 0: only the tokens from `first_row` on, of requests that bring fewer than `below`; rec starts at that row.
 // --------------------------------------------------------------------------
 #define DP_MAX_PER_LANE 8  // dk, dv <= 512
 
@@ -38,14 +40,18 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
     const float* __restrict__ conv_w, int taps, const float* __restrict__ a_log,
     const float* __restrict__ dt_bias, float* __restrict__ state, size_t state_stride,
     size_t tail_off, const int* __restrict__ q_start, const int* __restrict__ token_req,
-    const int* __restrict__ slots, float* __restrict__ rec, int ld_rec, int H, int G, int dk, int dv) {
-  const int t = blockIdx.x;
+    const int* __restrict__ slots, float* __restrict__ rec, int ld_rec, int H, int G, int dk, int dv, int first_row, int below) {
+  const int t = first_row + blockIdx.x;
+  if (below > 0) {
+    const int r = token_req[t];
+    if (q_start[r + 1] - q_start[r] >= below) return;
+  }
   const int lane = threadIdx.x & (TK_WAVE - 1);
   const int unit = blockIdx.y * (blockDim.x / TK_WAVE) + threadIdx.x / TK_WAVE;
   const int n_units = 2 * G + 2 * H + 1;
   if (unit >= n_units) return;
   const int C = 2 * G * dk + H * dv;
-  float* out = rec + (size_t)t * ld_rec;
+  float* out = rec + (size_t)blockIdx.x * ld_rec;
   const int v_off = 2 * G * dk, decay_off = v_off + H * dv, beta_off = decay_off + H * dk;
   if (unit < 2 * G + H) {
     // a head's channels through the convolution: q head, k head or v head
@@ -202,7 +208,7 @@ template <int NQ, bool VEC>
 __global__ __launch_bounds__(NQ > 2 ? 384 : 1024) void delta_rule_kernel(
     const float* __restrict__ rec, int ld_rec, float* __restrict__ state, size_t state_stride,
     const int* __restrict__ q_start, const int* __restrict__ slots, float* __restrict__ o, int H, int G,
-    int dk, int dv, int cols, int tok) {
+    int dk, int dv, int cols, int tok, int below) {
   // two buffers of [tok][3][dkp] q, k, decay; [tok][cols] v; [tok] beta
   extern __shared__ __align__(16) float stage[];
   const int h = blockIdx.x, r = blockIdx.y;
@@ -215,6 +221,7 @@ __global__ __launch_bounds__(NQ > 2 ? 384 : 1024) void delta_rule_kernel(
   constexpr int dkp = NQ * DR_LANES * 4;  // dk rounded up to what the lanes of a column hold
   const int gk = h / (H / G);
   const int first = q_start[r], last = q_start[r + 1];
+  if (below > 0 && last - first >= below) return;  // the same for the whole workgroup
   float* s_col = state + (size_t)slots[r] * state_stride + ((size_t)h * dv + (live ? col : 0)) * dk;
 
   float s[NQ][4];
@@ -328,11 +335,15 @@ TK_API int tk_delta_tail(int dt, const void* proj, int ld, int taps, float* stat
   return 0;
 }
 
+// below > 0: only the rows from first_row on, of requests that bring fewer tokens; the tails stay as they are (tk_delta_tail
+// moves them on afterwards).  rec: [n_tokens - first_row] rows.
 TK_API int tk_delta_prepare(int dt, const void* proj, int ld, int col_b, const float* a_pre, int ld_a,
                             const float* conv_w, int taps, const float* a_log, const float* dt_bias,
                             float* state, size_t state_stride, size_t tail_off, const int* q_start,
                             const int* token_req, const int* slots, float* rec, int ld_rec, int n_tokens,
-                            int n_requests, int H, int G, int dk, int dv, hipStream_t stream) {
+                            int n_requests, int H, int G, int dk, int dv, int first_row, int below, hipStream_t stream) {
+  TK_REQUIRE(first_row >= 0 && below >= 0 && (below > 0 || first_row == 0) && first_row <= n_tokens,
+             "delta_prepare: rows from %d on of requests of fewer than %d tokens", first_row, below);
   TK_REQUIRE(n_tokens >= 0 && n_requests >= 0 && H > 0 && G > 0 && H % G == 0 && dk > 0 && dv > 0,
              "delta_prepare: bad sizes tokens=%d heads=%d kv heads=%d dk=%d dv=%d", n_tokens, H, G, dk, dv);
   TK_REQUIRE(taps >= 1 && taps <= DR_MAX_TAPS, "delta_prepare: %d taps (1..%d)", taps, DR_MAX_TAPS);
@@ -343,16 +354,16 @@ TK_API int tk_delta_prepare(int dt, const void* proj, int ld, int col_b, const f
   TK_REQUIRE(tail_off + (size_t)(taps - 1) * C <= state_stride, "delta_prepare: the state row is too short");
   TK_REQUIRE(dk <= DP_MAX_PER_LANE * TK_WAVE && dv <= DP_MAX_PER_LANE * TK_WAVE, "delta_prepare: head sizes %d, %d (at most %d)",
              dk, dv, DP_MAX_PER_LANE * TK_WAVE);
-  if (n_tokens == 0) return 0;
+  if (n_tokens == first_row) return 0;
   const int units = 2 * G + 2 * H + 1;
-  const dim3 grid(n_tokens, (units + 3) / 4);
+  const dim3 grid(n_tokens - first_row, (units + 3) / 4);
   TK_REQUIRE(grid.y < 65536, "delta_prepare: too many heads");
   // every request brings one token: the convolving lane moves its channel's tail on itself
-  const bool fuse_tail = n_tokens == n_requests && taps > 1;
+  const bool fuse_tail = n_tokens == n_requests && taps > 1 && below == 0;
 #define DP_LAUNCH(T, FUSE)                                                                                         \
   hipLaunchKernelGGL((delta_prepare_kernel<T, FUSE>), grid, dim3(256), 0, stream, (const T*)proj, ld, col_b, a_pre, ld_a, \
                      conv_w, taps, a_log, dt_bias, state, state_stride, tail_off, q_start, token_req, slots, rec,  \
-                     ld_rec, H, G, dk, dv)
+                     ld_rec, H, G, dk, dv, first_row, below)
   if (dt == TK_F32) {
     if (fuse_tail) DP_LAUNCH(float, true); else DP_LAUNCH(float, false);
   } else {
@@ -360,13 +371,14 @@ TK_API int tk_delta_prepare(int dt, const void* proj, int ld, int col_b, const f
   }
 #undef DP_LAUNCH
   TK_CHECK_LAUNCH("delta_prepare");
-  if (taps > 1 && !fuse_tail) return tk_delta_tail(dt, proj, ld, taps, state, state_stride, tail_off, q_start, slots, n_requests, C, stream);
+  if (taps > 1 && !fuse_tail && below == 0) return tk_delta_tail(dt, proj, ld, taps, state, state_stride, tail_off, q_start, slots, n_requests, C, stream);
   return 0;
 }
 
+// rec, o: of the step's first row.  below > 0: only the requests that bring fewer tokens.
 TK_API int tk_delta_rule(const float* rec, int ld_rec, float* state, size_t state_stride, const int* q_start,
                          const int* slots, float* o, int n_requests, int H, int G, int dk, int dv, int cols,
-                         hipStream_t stream) {
+                         int below, hipStream_t stream) {
   TK_REQUIRE(n_requests >= 0 && H > 0 && G > 0 && H % G == 0 && dk > 0 && dv > 0,
              "delta_rule: bad sizes heads=%d kv heads=%d dk=%d dv=%d", H, G, dk, dv);
   TK_REQUIRE(dk <= 512, "delta_rule: key size %d (at most 512)", dk);
@@ -392,10 +404,10 @@ TK_API int tk_delta_rule(const float* rec, int ld_rec, float* state, size_t stat
   do {                                                                                                           \
     if (vec)                                                                                                     \
       hipLaunchKernelGGL((delta_rule_kernel<NQ, true>), grid, block, smem, stream, rec, ld_rec, state,           \
-                         state_stride, q_start, slots, o, H, G, dk, dv, cols, tok);                              \
+                         state_stride, q_start, slots, o, H, G, dk, dv, cols, tok, below);                            \
     else                                                                                                         \
       hipLaunchKernelGGL((delta_rule_kernel<NQ, false>), grid, block, smem, stream, rec, ld_rec, state,          \
-                         state_stride, q_start, slots, o, H, G, dk, dv, cols, tok);                              \
+                         state_stride, q_start, slots, o, H, G, dk, dv, cols, tok, below);                            \
   } while (0)
   if (nq == 1) DR_CASE(1);
   else if (nq == 2) DR_CASE(2);

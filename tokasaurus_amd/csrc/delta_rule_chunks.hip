@@ -16,6 +16,8 @@
 // wavefronts hold a quarter of S's rows each in registers: two products on what the first left (their quarters added
 // through local memory, one barrier a chunk) and one update.  The result of a product lies in the lanes as the next needs
 // its operand (row 4 * (lane / 16) + j of column lane % 16), so S never leaves the registers.
+// A step's portions of many tokens come here (delta_portions_in_chunks in ops.py), its other requests run in delta_rule.hip: how a
+// request is cut into portions changes the order of the sums.
 // The recurrence token by token is one chain of 270 ns a token; here it is one of about 1 us a chunk of 16, and the first
 // kernel, bound by its vector instructions, has no chain.  Two prompts of 562 and 938 tokens, 16 heads of 128 x 128: 72 us of
 // delta_prepare and 256 us of delta_rule before, 99 and 58 us now.
@@ -263,7 +265,8 @@ __global__ __launch_bounds__(256) void delta_chunk_walk_kernel(DeltaChunkArgs a)
   const int dkp = a.dkp, dvp = a.dvp;
   const int first = a.q_start[r], last = a.q_start[r + 1];
   if (first >= last) return;
-  const int c0 = a.chunk_first[r], chunks = (last - first + DC_CHUNK - 1) / DC_CHUNK;
+  const int c0 = a.chunk_first[r], chunks = a.chunk_first[r + 1] - c0;  // none: a request that the recurrence takes
+  if (chunks <= 0) return;
   const size_t words = dc_words(dkp, dvp), step = (size_t)a.H * words;
   const int col = nb * 16 + lr;
   float* s_col = a.state + (size_t)a.slots[r] * a.state_stride + ((size_t)h * a.dv + (col < a.dv ? col : 0)) * a.dk;
@@ -349,7 +352,7 @@ TK_API int tk_delta_chunk_words(int dk, int dv) {
 }
 
 // proj, a_pre, conv_w, a_log, dt_bias, state: as tk_delta_prepare takes them; chunk_req, chunk_row0 [n_chunks], chunk_first
-// [n_requests]: the step's rows in chunks of 16 in the requests' order; rec: [n_chunks][H][tk_delta_chunk_words]; o: [tokens][H * dv].
+// [n_requests + 1]: the step's rows in chunks of 16 in the requests' order (none for a request that is left out); rec: [n_chunks][H][tk_delta_chunk_words]; o: [tokens][H * dv].
 // The convolutions' tails stay as they are (tk_delta_tail moves them on afterwards).
 TK_API int tk_delta_chunks(int dt, const void* proj, int ld, int col_b, const float* a_pre, int ld_a, const float* conv_w, int taps,
                            const float* a_log, const float* dt_bias, float* state, size_t state_stride, size_t tail_off,

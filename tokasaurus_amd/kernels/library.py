@@ -80,8 +80,8 @@ _SIGNATURES: dict[str, dict[str, list]] = {
         "tk_attention_tile_part_words": [c_int],
         "tk_attention_tile_f32_fits": [c_int] * 5,
         "tk_delta_prepare": [c_int, _P, c_int, c_int, _P, c_int, _P, c_int, _P, _P, _P, c_size_t, c_size_t, _P, _P, _P, _P]
-        + [c_int] * 7 + [_P],
-        "tk_delta_rule": [_P, c_int, _P, c_size_t, _P, _P, _P] + [c_int] * 6 + [_P],
+        + [c_int] * 9 + [_P],
+        "tk_delta_rule": [_P, c_int, _P, c_size_t, _P, _P, _P] + [c_int] * 7 + [_P],
         "tk_delta_tail": [c_int, _P, c_int, c_int, _P, c_size_t, c_size_t, _P, _P, c_int, c_int, _P],
         "tk_delta_chunks": [c_int, _P, c_int, c_int, _P, c_int, _P, c_int, _P, _P, _P, c_size_t, c_size_t, _P, _P, _P, _P, _P, _P, _P]
         + [c_int] * 6 + [_P],

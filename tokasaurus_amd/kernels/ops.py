@@ -1284,8 +1284,9 @@ def linear_attention_state_words(heads: int, key_dim: int, value_dim: int, memor
 
 @dataclass
 class ChunkPlan:
-    """A step's rows cut into chunks of so many neighbouring tokens of one request (``linear_attention_chunk_tokens``,
-    ``delta_chunk_tokens``), in the requests' order: every chunk's request and first row, and every request's first chunk (and, last, the number of chunks), int32."""
+    """A step's rows (those of the requests that go in chunks) cut into chunks of so many neighbouring tokens of one request
+    (``linear_attention_chunk_tokens``, ``delta_chunk_tokens``), in the requests' order: every chunk's request and first row, and
+    every request's first chunk (and, last, the number of chunks), int32."""
 
     req: torch.Tensor
     row0: torch.Tensor
@@ -2014,23 +2015,36 @@ def _check_delta(proj, a_pre, conv_w, a_log, dt_bias, state, q_start, slots, hea
     return n, taps
 
 
-# Tokens of a step's longest portion from which on the delta rule goes in chunks (a step of 33 tokens takes 1.44 ms either way,
-# bound by the host; of 2,048 tokens 6.4 ms token by token and 4.4 in chunks)
+# Tokens of a portion from which on the delta rule may take it in chunks, where a step's portions of that length have
+# DELTA_CHUNKS_TOKENS together.  The requests of a step that bring fewer, its single tokens above all, stay with the recurrence.
+# 16 heads of 128 x 128, a layer on an MI355X in us, all by the recurrence / all in chunks / portions in chunks beside the
+# recurrence: 64 tokens alone 29 / 40, 128: 47 / 44, 256: 84 / 54, eight of 48: 76 / 61; beside 8 single tokens 96: 53 / 56 / 65,
+# 160: 77 / 66 / 72, 256: 110 / 75 / 82; beside 64 single tokens 96: 85 / 146 / 107, 160: 111 / 149 / 112, 256: 149 / 159 / 121.
 DELTA_CHUNKS_FROM = 32
+DELTA_CHUNKS_TOKENS = 160
+
+
+def delta_portions_in_chunks(lengths: "list[int]") -> "list[bool]":
+    """For the requests of a step, by the tokens that each brings: which take the delta rule in chunks."""
+    together = sum(n for n in lengths if n >= DELTA_CHUNKS_FROM)
+    return [n >= DELTA_CHUNKS_FROM and together >= DELTA_CHUNKS_TOKENS for n in lengths]
 
 
 def delta_chunk_tokens(key_dim: int, value_dim: int, longest: int) -> int:
-    """Tokens of a chunk where a step whose longest portion has ``longest`` tokens goes in chunks (and so needs a
-    ``ChunkPlan`` of them), else 0."""
+    """Tokens of a chunk where a step whose longest portion has ``longest`` tokens has portions that go in chunks (and so needs
+    a ``ChunkPlan`` of them), else 0."""
     takes = longest >= DELTA_CHUNKS_FROM and load("core").tk_delta_chunk_words(int(key_dim), int(value_dim)) > 0
     return load("core").tk_delta_chunk_tokens() if takes else 0
 
 
 def delta_rule_chunks(proj: torch.Tensor, col_b: int, a_pre: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor,
                       dt_bias: torch.Tensor, state: torch.Tensor, q_start: torch.Tensor, slots: torch.Tensor, chunks: "ChunkPlan",
-                      heads: int, kv_heads: int, key_dim: int, value_dim: int) -> torch.Tensor:
+                      heads: int, kv_heads: int, key_dim: int, value_dim: int, token_req: torch.Tensor | None = None,
+                      below: int = 0, first_below: "tuple[int, int] | None" = None) -> torch.Tensor:
     """``delta_rule(delta_prepare(..))`` in chunks on the matrix cores (delta_rule_chunks.hip): o [tokens, heads * value_dim] in
-    32-bit, the matrices and tails in ``state`` moved on by the step's rows."""
+    32-bit, the matrices and tails in ``state`` moved on by the step's rows.  ``first_below`` (with ``token_req``, every
+    row's request): the first request of fewer than ``below`` tokens and its first row; such requests, of which ``chunks``
+    has none, take the recurrence."""
     _gpu(proj, a_pre, conv_w, a_log, dt_bias, state, q_start, slots, chunks.req)
     n, taps = _check_delta(proj, a_pre, conv_w, a_log, dt_bias, state, q_start, slots, heads, kv_heads, key_dim, value_dim)
     for t, name in ((chunks.req, "chunks"), (chunks.row0, "chunks"), (chunks.first, "chunks")):
@@ -2041,6 +2055,12 @@ def delta_rule_chunks(proj: torch.Tensor, col_b: int, a_pre: torch.Tensor, conv_
     o = torch.empty((n, heads * value_dim), dtype=torch.float32, device=proj.device)
     rec = torch.empty((count * heads * words,), dtype=torch.float32, device=proj.device)
     tail = heads * key_dim * value_dim
+    if first_below is not None:
+        request, row = first_below
+        _need(token_req is not None and below > 0, "delta rule: requests left to the recurrence need every row's request")
+        few = delta_prepare(proj, col_b, a_pre, conv_w, a_log, dt_bias, state, q_start, token_req, slots, heads, kv_heads,
+                            key_dim, value_dim, first_row=row, below=below)
+        delta_rule(few, state, q_start[request:], slots[request:], heads, kv_heads, key_dim, value_dim, first_row=row, below=below, out=o)
     call("tk_delta_chunks", dtype_code(proj.dtype), proj.data_ptr(), proj.stride(0), int(col_b), a_pre.data_ptr(),
          a_pre.stride(0) if n > 1 else heads * key_dim, conv_w.data_ptr(), taps, a_log.data_ptr(), dt_bias.data_ptr(),
          state.data_ptr(), state.stride(0), tail, q_start.data_ptr(), slots.data_ptr(), chunks.req.data_ptr(),
@@ -2066,23 +2086,26 @@ def delta_prepare(
     kv_heads: int,
     key_dim: int,
     value_dim: int,
+    first_row: int = 0,
+    below: int = 0,
 ) -> torch.Tensor:
     """What the recurrence reads, in 32-bit [tokens, q | k | v | decay | beta]: the rows
     ``proj`` [q | k | v | ...] pass their short causal convolutions (``conv_w`` [channels, taps],
     earlier inputs from this step's rows or the tail in the request's ``state`` row) and silu; q
     and k become unit vectors per head (q also times key_dim^-1/2); decay = exp(-exp(a_log) *
     softplus(a_pre + dt_bias)); beta = sigmoid(proj[:, col_b + head]).  The tails in ``state``
-    are then moved on by this step's rows."""
+    are then moved on by this step's rows.  ``below`` > 0: only the rows
+    from ``first_row`` on (the result holds those), of requests of fewer tokens, and the tails stay as they are."""
     _gpu(proj, a_pre, conv_w, a_log, dt_bias, state, q_start, token_req, slots)
     n, taps = _check_delta(proj, a_pre, conv_w, a_log, dt_bias, state, q_start, slots, heads, kv_heads, key_dim, value_dim)
     _i32(token_req, "token_req")
     _need(token_req.numel() == n, "delta_prepare: one request a token")
     width = delta_rec_width(heads, kv_heads, key_dim, value_dim)
-    rec = torch.empty((n, width), dtype=torch.float32, device=proj.device)
+    rec = torch.empty((n - first_row, width), dtype=torch.float32, device=proj.device)
     call("tk_delta_prepare", dtype_code(proj.dtype), proj.data_ptr(), proj.stride(0), int(col_b), a_pre.data_ptr(),
          a_pre.stride(0) if n > 1 else heads * key_dim, conv_w.data_ptr(), taps, a_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(), state.stride(0),
          heads * key_dim * value_dim, q_start.data_ptr(), token_req.data_ptr(), slots.data_ptr(), rec.data_ptr(), width,
-         n, slots.numel(), heads, kv_heads, key_dim, value_dim, _stream())
+         n, slots.numel(), heads, kv_heads, key_dim, value_dim, int(first_row), int(below), _stream())
     return rec
 
 
@@ -2099,9 +2122,11 @@ def delta_rule_columns(requests: int, heads: int, key_dim: int, value_dim: int) 
 
 
 def delta_rule(rec: torch.Tensor, state: torch.Tensor, q_start: torch.Tensor, slots: torch.Tensor,
-               heads: int, kv_heads: int, key_dim: int, value_dim: int) -> torch.Tensor:
+               heads: int, kv_heads: int, key_dim: int, value_dim: int, first_row: int = 0, below: int = 0,
+               out: torch.Tensor | None = None) -> torch.Tensor:
     """The recurrence over every request's tokens of this step, from and to the matrices in the
-    requests' ``state`` rows: o [tokens, heads * value_dim] in 32-bit."""
+    requests' ``state`` rows: o [tokens, heads * value_dim] in 32-bit.  ``below`` > 0: only over the requests of fewer tokens,
+    ``rec`` holding the step's rows from ``first_row`` on; the other rows of ``out`` stay as they are."""
     _gpu(rec, state, q_start, slots)
     n = rec.shape[0]
     _need(rec.dim() == 2 and rec.dtype == torch.float32 and rec.is_contiguous()
@@ -2111,10 +2136,13 @@ def delta_rule(rec: torch.Tensor, state: torch.Tensor, q_start: torch.Tensor, sl
     _i32(q_start, "q_start")
     _i32(slots, "slots")
     _need(q_start.numel() == slots.numel() + 1, "delta_rule: one slot a request")
-    o = torch.empty((n, heads * value_dim), dtype=torch.float32, device=rec.device)
+    o = out if out is not None else torch.empty((first_row + n, heads * value_dim), dtype=torch.float32, device=rec.device)
+    _need(o.shape == (first_row + n, heads * value_dim) and o.dtype == torch.float32 and o.is_contiguous(),
+          "delta_rule: the result's buffer must be contiguous float32 [tokens, heads * value_dim]")
     cols = delta_rule_columns(slots.numel(), heads, key_dim, value_dim)
-    call("tk_delta_rule", rec.data_ptr(), rec.stride(0), state.data_ptr(), state.stride(0), q_start.data_ptr(),
-         slots.data_ptr(), o.data_ptr(), slots.numel(), heads, kv_heads, key_dim, value_dim, cols, _stream())
+    # the kernel finds a token's row by its place in the step
+    call("tk_delta_rule", rec.data_ptr() - int(first_row) * rec.stride(0) * rec.element_size(), rec.stride(0), state.data_ptr(), state.stride(0), q_start.data_ptr(),
+         slots.data_ptr(), o.data_ptr(), slots.numel(), heads, kv_heads, key_dim, value_dim, cols, int(below), _stream())
     return o
 
 

@@ -103,16 +103,31 @@ class ChannelDeltaRule(Mixer):
         # (a new buffer: a one-row view counts as contiguous whatever its stride says)
         return torch.empty((x.shape[0], count), dtype=x.dtype, device=x.device).copy_(part)
 
+    def _chunks(self, ctx: StepContext) -> "tuple[int, tuple[int, int] | None]":
+        """(tokens of a chunk where portions of this step go in chunks, else 0; the first request that does not and its row).
+        Decided once a step and shared by the layers."""
+        key = ("delta_chunks", self.key_dim, self.value_dim)
+        if key not in ctx.extras:
+            start = ctx.host_q_start
+            size, few = ops.delta_chunk_tokens(self.key_dim, self.value_dim, ctx.max_q_len), None
+            if size:
+                taken = ops.delta_portions_in_chunks([b - a for a, b in zip(start, start[1:])])
+                size = size if any(taken) else 0
+                few = next(((r, start[r]) for r, t in enumerate(taken) if not t), None)
+            ctx.extras[key] = size, few
+        return ctx.extras[key]
+
     def _run(self, h: torch.Tensor, ctx: StepContext, state: torch.Tensor, rows: torch.Tensor | None) -> torch.Tensor:
         assert state is not None, "the delta rule keeps its state in the request's slot"
         H, G, dk, dv = self.num_heads, self.num_kv_heads, self.key_dim, self.value_dim
         proj = self.inp(h)
         low = self.low(self._columns(proj, self.col_a1, self.decay_rank + self.gate_rank), out_f32=True)
         a_pre, gate = low[:, : H * dk], low[:, H * dk :]  # 32-bit, rows a stride apart
-        size = ops.delta_chunk_tokens(dk, dv, ctx.max_q_len)
+        size, few = self._chunks(ctx)
         if size:
+            least = ops.DELTA_CHUNKS_FROM
             o = ops.delta_rule_chunks(proj, self.col_b, a_pre, self.conv_w, self.a_log, self.dt_bias, state, ctx.q_start,
-                                      ctx.slots, chunks_of(ctx, size), H, G, dk, dv)
+                                      ctx.slots, chunks_of(ctx, size, least), H, G, dk, dv, ctx.token_req, least, few)
         else:
             rec = ops.delta_prepare(proj, self.col_b, a_pre, self.conv_w, self.a_log, self.dt_bias, state,
                                     ctx.q_start, ctx.token_req, ctx.slots, H, G, dk, dv)

@@ -37,14 +37,16 @@ from tokasaurus_amd.parts.base import BIAS, MATRIX, MIXERS, NORM_WEIGHT, UNIT_IN
 from tokasaurus_amd.parts.linear import Linear, Placer
 
 
-def chunks_of(ctx: StepContext, size: int) -> "ops.ChunkPlan":
-    """The step's rows in chunks of ``size`` tokens, made once a step and shared by the layers."""
-    key = ("chunk_plan", size)
+def chunks_of(ctx: StepContext, size: int, shortest: int = 1) -> "ops.ChunkPlan":
+    """The step's rows (of requests that bring ``shortest`` tokens and more) in chunks of ``size`` tokens, made once a step
+    and shared by the layers."""
+    key = ("chunk_plan", size, shortest)
     plan = ctx.extras.get(key)
     if plan is None:
         req, row0, first = [], [], [0]
         for r in range(ctx.num_requests):
-            rows = range(ctx.host_q_start[r], ctx.host_q_start[r + 1], size)
+            a, b = ctx.host_q_start[r], ctx.host_q_start[r + 1]
+            rows = range(a, b, size) if b - a >= shortest else ()
             req += [r] * len(rows)
             row0 += rows
             first.append(len(req))
