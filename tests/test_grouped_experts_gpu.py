@@ -51,3 +51,41 @@ def test_experts_in_tiles(tokens, experts, top, width, ff, form):
     # error is then within 5 * 2^-9 of its terms, and these add like independent ones
     assert float((got.double() - want).norm() / want.norm()) <= 5 * 2.0 ** -9
     assert torch.isfinite(got).all()
+
+
+@pytest.mark.parametrize("tokens,top,experts", [(1, 1, 300), (13, 8, 256), (130, 1, 2), (129, 1, 1), (400, 3, 5), (64, 2, 64)])
+@pytest.mark.parametrize("spread", ["one expert", "all", "each its own"])
+def test_tiles_hold_every_choice(tokens, top, experts, spread):
+    """The fewest tiles that can hold any choice: all pairs on one expert, on all alike, and a pair an expert as far as they go."""
+    pairs = tokens * top
+    if spread == "one expert":
+        ids = torch.full((tokens, top), experts - 1, dtype=torch.int32)
+    elif spread == "all":
+        ids = (torch.arange(pairs, dtype=torch.int32) % experts).view(tokens, top)
+    else:  # every expert but one has one pair, the last all others
+        ids = torch.arange(pairs, dtype=torch.int32).clamp(max=min(experts, pairs) - 1).view(tokens, top)
+    s = ops.expert_sort([(ids.cuda(), experts)])[0]
+    assert s.max_tiles == ops.expert_tiles(pairs, experts) <= pairs
+    used = int(s.tile_group[-1])
+    count = torch.bincount(ids.flatten().long(), minlength=experts)
+    assert used == int((-(-count // ops.EXPERT_TILE)).sum()) <= s.max_tiles
+    slot_pair, group = s.slot_pair.cpu().view(-1, ops.EXPERT_TILE), s.tile_group.cpu()
+    assert sorted(slot_pair[slot_pair >= 0].tolist()) == list(range(pairs))
+    for t in range(s.max_tiles):
+        mine = slot_pair[t][slot_pair[t] >= 0].long()
+        assert (t < used) == (mine.numel() > 0) and (ids.flatten()[mine] == group[t]).all()
+
+
+def test_room_for_the_experts_is_that_of_the_pairs():
+    """256 experts of inner size 2,048, 64 pairs: rows between the two products are the pairs', not those of tiles an expert."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    h = torch.randn((32, 64), generator=g, device="cuda").bfloat16()
+    gu = torch.randn((256, 4096, 64), generator=g, device="cuda").bfloat16()
+    dn = torch.randn((256, 64, 2048), generator=g, device="cuda").bfloat16()
+    ids, weights = torch.randint(0, 256, (32, 2), generator=g, device="cuda", dtype=torch.int32), torch.rand((32, 2), generator=g, device="cuda")
+    pairs = ops.expert_sort([(ids, 256)])[0]
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = ops.expert_mix(h, gu, dn, ids, weights, pairs=pairs)
+    assert torch.isfinite(out).all() and torch.cuda.max_memory_allocated() - before < 4 << 20

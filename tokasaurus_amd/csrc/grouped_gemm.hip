@@ -336,7 +336,7 @@ static bool launch_staged(const GroupedArgs& a, int tiles, hipStream_t stream) {
   const int outs = GLU ? 64 : 128, n_blocks = (a.N + outs - 1) / outs;
   const long items = (long)tiles * n_blocks, groups = (items + GS_DIES - 1) / GS_DIES * GS_DIES;
   if (groups >= (1l << 31)) return false;
-  const int lds = GS_STAGES * 256 * GS_K * (int)sizeof(bf16_t);  // 64 KB, at least the results' place
+  const int lds = GS_STAGES * 256 * GS_K * (int)sizeof(bf16_t);  // 48 KB; the results' place is 32 at most
   hipLaunchKernelGGL(grouped_gemm_staged_kernel<GLU>, dim3((unsigned)groups), dim3(256), lds, stream, a, tiles, n_blocks);
   return true;
 }
@@ -439,7 +439,8 @@ TK_API int tk_expert_sort(const SortJob* jobs, int n_jobs, hipStream_t stream) {
     for (int k = 0; k < n; ++k) {
       const SortJob& j = all.job[k] = jobs[first + k];
       TK_REQUIRE(j.ids && j.slot_pair && j.slot_token && j.tile_group && j.pairs >= 0 && j.top > 0 && j.experts > 0, "expert_sort: bad arguments");
-      TK_REQUIRE(j.max_tiles >= (j.pairs + GS_M - 1) / GS_M + j.experts, "expert_sort: %d tiles cannot hold %d pairs of %d experts", j.max_tiles,
+      // (each expert that has pairs leaves at most one tile partly empty)
+      TK_REQUIRE(j.max_tiles >= (j.pairs + (long)(GS_M - 1) * min(j.experts, j.pairs)) / GS_M, "expert_sort: %d tiles cannot hold %d pairs of %d experts", j.max_tiles,
                  j.pairs, j.experts);
       TK_REQUIRE(3 * j.experts * sizeof(int) <= 48 * 1024, "expert_sort: too many experts");
       most = max(most, j.experts);

@@ -2368,6 +2368,11 @@ class SortedPairs:
     shape: tuple  # of the ids
 
 
+def expert_tiles(pairs: int, experts: int) -> int:
+    """Tiles that so many pairs can fill: each expert that has any, at most min(experts, pairs), leaves one tile partly empty."""
+    return (pairs + (EXPERT_TILE - 1) * min(experts, pairs)) // EXPERT_TILE
+
+
 def expert_sort(choices: "list[tuple[torch.Tensor, int]]") -> "list[SortedPairs]":
     """(ids [tokens, top], number of experts) of one or several choices -> their pairs sorted, in one launch."""
     out, jobs = [], (_SortJob * len(choices))()
@@ -2375,7 +2380,7 @@ def expert_sort(choices: "list[tuple[torch.Tensor, int]]") -> "list[SortedPairs]
         _gpu(ids)
         _i32(ids, "ids")
         n, top = ids.shape
-        max_tiles = -(-(n * top) // EXPERT_TILE) + experts
+        max_tiles = expert_tiles(n * top, int(experts))
         slots = max_tiles * EXPERT_TILE
         book = torch.empty((2 * slots + max_tiles + 1,), dtype=torch.int32, device=ids.device)
         s = SortedPairs(book[:slots], book[slots : 2 * slots], book[2 * slots :], max_tiles, (n, top))
@@ -2432,12 +2437,12 @@ def expert_mix(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, i
         _need(pairs.shape == (n, top), "expert_mix: pairs of another choice")
         slot_pair, slot_token, tile_group, max_tiles = pairs.slot_pair, pairs.slot_token, pairs.tile_group, pairs.max_tiles
         slots = max_tiles * EXPERT_TILE
-        inter = torch.empty((slots, ff), dtype=h.dtype, device=h.device)
-        call("tk_grouped_gemm_bf16", h.data_ptr(), h.stride(0), slot_token.data_ptr(), None, tile_group.data_ptr(), max_tiles, 0,
+        inter = torch.empty((n * top, ff), dtype=h.dtype, device=h.device)  # a row a pair: slots are many more where experts have few
+        call("tk_grouped_gemm_bf16", h.data_ptr(), h.stride(0), slot_token.data_ptr(), slot_pair.data_ptr(), tile_group.data_ptr(), max_tiles, 0,
              0, 0, w_gate_up.data_ptr(), 2 * ff * width, inter.data_ptr(), ff, ff, width, slots, 1, 0, on_input,
              slot_pair.data_ptr() if weights_on_input else None, limit, alpha, _stream())
         y = torch.empty((n * top, width), dtype=h.dtype, device=h.device)
-        call("tk_grouped_gemm_bf16", inter.data_ptr(), ff, None, slot_pair.data_ptr(), tile_group.data_ptr(), max_tiles, 0,
+        call("tk_grouped_gemm_bf16", inter.data_ptr(), ff, slot_pair.data_ptr(), slot_pair.data_ptr(), tile_group.data_ptr(), max_tiles, 0,
              0, 0, w_down.data_ptr(), width * ff, y.data_ptr(), width, width, ff, slots, 0, 0, None, None, 0.0, 0.0, _stream())
         call("tk_expert_sum", h.data_ptr(), h.stride(0), y.data_ptr(), ids.data_ptr(), weight_ptr,
              shared.data_ptr() if shared is not None else None, shared_gate.data_ptr() if shared is not None else None,
