@@ -102,3 +102,14 @@ def test_which_portions_take_the_delta_rule_in_chunks():
     # single tokens and short portions keep the recurrence whatever shares their step; many portions count together
     assert chunks([300, 31, 1, 1]) == [True, False, False, False]
     assert chunks([48] * 8 + [1]) == [True] * 8 + [False] and chunks([32, 96, 31, 1]) == [False] * 4
+
+
+def test_which_experts_products_run_in_tiles():
+    import torch
+
+    tiles = lambda rows, top, experts, ff=512: ops.experts_go_in_tiles(rows, top, torch.bfloat16, 1024, ff, experts)
+    # from 64 pairs on, and five pairs for four experts, in steps of more than a dozen rows
+    assert tiles(32, 2, 16) and not tiles(31, 2, 16) and not tiles(12, 8, 16)
+    assert not tiles(32, 2, 64) and not tiles(39, 2, 64) and tiles(40, 2, 64)
+    assert not tiles(39, 8, 256) and tiles(40, 8, 256)
+    assert not tiles(64, 2, 16, ff=12)

@@ -2230,9 +2230,13 @@ def squared_relu_(x: torch.Tensor) -> torch.Tensor:
 HEAD_TILE = 64  # rows a tile of the product with a matrix a head (GG_TM of grouped_gemm.hip)
 EXPERT_TILE = 128  # slots a tile of the experts' products (GS_M)
 # Pairs (token, chosen expert) below which the experts' products stay with the kernels of a workgroup a pair, which read an
-# expert's weights for every pair that names it: 32 experts of 2,048 x 1,024, 8 chosen, in us a pair each / in tiles: 8 tokens
-# 112 / 99, 6 tokens 90 / 98; 64 experts of 1,024 x 512, 2 chosen: 24 tokens 29 / 42, 32 tokens 36 / 41.  (And from
-# GROUPED_FROM_ROWS rows on only: the tiles round an expert's rows before they are added.)
+# expert's weights for every pair that names it, where tiles read them once: the pairs must be more than the experts by enough
+# (``experts_go_in_tiles``: five for four experts) and fill the chip.  In us a pair each / in tiles, all three kernels:
+# 16 experts of 2,048 x 2,048: 26 pairs 97 / 98, 64 pairs 196 / 109; 32 of 1,024 x 512: 64 pairs 36 / 41, 96 pairs 48 / 42; 32 of
+# 2,048 x 1,024: 48 pairs 90 / 98, 104 pairs 171 / 108; 64 of 1,024 x 512: 64 pairs 39 / 52, 96 pairs 53 / 54, 128 pairs 66 / 56; 64 of
+# 2,048 x 1,408: 78 pairs 186 / 179; 128 of 2,048 x 768: 96 pairs 146 / 159, 128 pairs 184 / 176, 192 pairs 256 / 200; 256 of
+# 2,048 x 512: 192 pairs 183 / 190, 256 pairs 232 / 217, 384 pairs 332 / 266.  (And from GROUPED_FROM_ROWS rows on only: the tiles
+# round an expert's rows before they are added.)
 EXPERT_TILES_FROM_PAIRS = 64
 GROUPED_FROM_ROWS = 12  # rows above which the products of experts and of heads run in tiles on the matrix cores
 
@@ -2391,10 +2395,12 @@ def expert_sort(choices: "list[tuple[torch.Tensor, int]]") -> "list[SortedPairs]
     return out
 
 
-def experts_go_in_tiles(rows: int, top: int, dtype: torch.dtype, width: int, ff: int) -> bool:
-    """Whether ``expert_mix`` sorts the pairs of so many tokens, ``top`` each, and runs the experts' products in tiles on the
-    matrix cores (for contiguous rows and weights)."""
-    return rows > GROUPED_FROM_ROWS and rows * top >= EXPERT_TILES_FROM_PAIRS and dtype == torch.bfloat16 and width % 8 == 0 and ff % 8 == 0
+def experts_go_in_tiles(rows: int, top: int, dtype: torch.dtype, width: int, ff: int, experts: int = 0) -> bool:
+    """Whether ``expert_mix`` sorts the pairs of so many tokens, ``top`` of so many experts each, and runs the experts' products
+    in tiles on the matrix cores (for contiguous rows and weights)."""
+    pairs = rows * top
+    many = pairs >= EXPERT_TILES_FROM_PAIRS and 4 * pairs >= 5 * experts
+    return rows > GROUPED_FROM_ROWS and many and dtype == torch.bfloat16 and width % 8 == 0 and ff % 8 == 0
 
 
 def expert_mix(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor | None,
@@ -2430,7 +2436,7 @@ def expert_mix(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, i
     weight_ptr = weights.data_ptr() if weights is not None else None
     if n == 0:
         return out
-    if experts_go_in_tiles(n, top, h.dtype, width, ff) and _grouped_takes(h, w_gate_up, width) and w_down.data_ptr() % 16 == 0:
+    if experts_go_in_tiles(n, top, h.dtype, width, ff, experts) and _grouped_takes(h, w_gate_up, width) and w_down.data_ptr() % 16 == 0:
         # many tokens: the pairs sorted by expert, every expert's rows in tiles on the matrix cores
         if pairs is None:
             pairs = expert_sort([(ids, experts)])[0]

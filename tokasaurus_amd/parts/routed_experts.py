@@ -147,7 +147,7 @@ class TokenTables:
         if self._ready is None:
             self._ready = ops.ExpertTables([x.table for x in self.layers])
         ids = ops.expert_lookup(ctx.token_ids, ctx.last_token, self._ready)
-        tiled = [i for i, x in enumerate(self.layers) if ops.experts_go_in_tiles(ctx.num_tokens, x.top, ctx.dtype, x.hidden_size, x.expert_size)]
+        tiled = [i for i, x in enumerate(self.layers) if ops.experts_go_in_tiles(ctx.num_tokens, x.top, ctx.dtype, x.hidden_size, x.expert_size, x.num_experts)]
         made = dict(zip(tiled, ops.expert_sort([(ids[i], self.layers[i].num_experts) for i in tiled]))) if tiled else {}
         ctx.extras[self.KEY] = [(x, made.get(i)) for i, x in enumerate(ids)]
 
