@@ -113,3 +113,11 @@ def test_which_experts_products_run_in_tiles():
     assert not tiles(32, 2, 64) and not tiles(39, 2, 64) and tiles(40, 2, 64)
     assert not tiles(39, 8, 256) and tiles(40, 8, 256)
     assert not tiles(64, 2, 16, ff=12)
+
+
+def test_rows_that_gate_and_up_take_in_the_hand_written_product():
+    # up to 64 where the streamed form is ahead: inner sizes up to 4,096, workgroups of 32 outputs in well filled rounds of 256
+    assert [ops.glu_rows(2048, n) for n in (1000, 8192, 8224, 12288, 14336, 16416, 24576)] == [64, 64, 16, 16, 64, 16, 64]
+    assert ops.glu_rows(4096, 14336) == 64 and ops.glu_rows(4096, 11008) == 16
+    assert ops.glu_rows(5120, 13824) == ops.glu_rows(8192, 28672) == 16
+    assert ops.glu_rows(2080, 8192) == ops.skinny_rows(2080, paired=True)

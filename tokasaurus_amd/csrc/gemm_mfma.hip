@@ -727,11 +727,12 @@ static bool launch_staged_one(const GemmArgs& a, int groups, int WK, hipStream_t
 // Where gate and up are streamed through local memory instead of into the wavefronts' registers.  Measured on an MI355X
 // (us, weights from memory; skinny / streamed): N = 14,336, K = 4,096: 50.5 / 47.0 at 2 rows, 55.6 / 47.1 at 8, 63.5 / 47.5 at
 // 16; 8,192 x 3,072: 24.2 / 21.1 at 2, 30.2 / 19.9 at 16; 8,192 x 2,048: 17.1 / 18.2 at 4, 18.4 / 17.0 at 16 (at 8 alone 18.1 /
-// 17.5, but a whole 1B step, with the norm in front, 1,318 / 1,347);
+// 17.5, but a whole 1B step, with the norm in front, 1,318 / 1,347); 8,192 x 2,304: 20.2 / 17.4 at 2, 22.5 / 16.3 at 16; 8,192 x
+// 2,560: 23.1 / 19.1 at 2; 8,192 x 2,816: 23.6 / 20.7 at 2;
 // with fewer workgroups than compute units 4,096 x 2,048: 10.3 / 10.3 at 16, 11.9 / 11.7 at 20, 13.6 / 11.6 at 32; 1,000 x 1,024:
 // 6.6 / 7.0 at 32, 9.4 / 9.1 at 48.
 static bool glu_streams(int M, int N, int K) {
-  if (N >= 32 * 256) return M >= (K >= 3072 ? 2 : 16);
+  if (N >= 32 * 256) return M >= (K >= 2304 ? 2 : 16);
   return (long)M * K >= 40000;
 }
 

@@ -879,14 +879,25 @@ def skinny_rows(inner: int, paired: bool = False) -> int:
 
 
 GLU_STREAM_ROWS = 64  # rows that the streamed gate and up product takes
+GLU_STREAM_DEEP_ROWS = 16  # and those up to which it is ahead whatever the sizes
 
 
-def glu_rows(inner: int) -> int:
-    """Rows up to which gate and up (with the gated activation behind them) take the hand-written product.  At an inner size
-    of a multiple of 64 its streamed form is ahead of the library's product and the pass behind it up to 64 rows (16 / 32 / 64
-    rows on an MI355X: 14,336 x 4,096 66 / 47.5, 55.6 / 49.7, 54.6 / 55.4 us; 8,192 x 2,048 20.3 / 17.0, 20.3 / 17.9, 21.1 / 18.9;
-    1,000 x 1,024 at 64 10.4 / 9.8); at others the crossing is that of the weight-streaming product."""
-    return GLU_STREAM_ROWS if inner % 64 == 0 else skinny_rows(inner, paired=True)
+def glu_rows(inner: int, outputs: int = 0) -> int:
+    """Rows up to which gate and up (with the gated activation behind them; ``outputs`` of each, 0: not known) take the
+    hand-written product.  At an inner size of a multiple of 64 that is its streamed form, a workgroup 32 outputs.  Library's product
+    and the pass behind it / streamed on an MI355X, us, at 16, 32 and 64 rows: 8,192 x 2,048 20.3 / 18.0, 20.4 / 18.7, 21.6 / 20.3;
+    8,192 x 3,072 25.3 / 20.6, 25.6 / 22.0, 28.2 / 25.3; 14,336 x 4,096 66.7 / 49.6, 60.6 / 51.9, 60.7 / 58.2; 1,000 x 1,024 9.9 / 6.8,
+    13.8 / 7.9, 14.0 / 10.4; 24,576 x 2,048 54.9 / 45.1, 53.0 / 45.5, 55.8 / 50.4: ahead up to 64 rows.  Not where the last round of
+    workgroups leaves more than an eighth of the compute units idle, 9,216 x 2,048 60.7 / 23.1, 24.5 / 25.2, 26.9 / 29.5; 10,240 x 2,560
+    50.9 / 29.3, 29.2 / 32.2, 34.3 / 40.4; 11,008 x 4,096 55.0 / 44.7, 44.9 / 46.6, 47.8 / 52.4; 12,288 x 4,096 50.3 / 48.7, 48.4 / 50.3,
+    50.0 / 55.5, nor at inner sizes above 4,096, 13,824 x 5,120 84.2 / 58.2, 57.0 / 62.0, 61.4 / 73.0; 12,288 x 6,144 72.0 / 72.9, 78.5 /
+    73.9, 81.4 / 84.4; 28,672 x 8,192 218 / 202, 200 / 200, 222 / 213: there up to 16.
+    At other inner sizes the crossing is that of the weight-streaming product."""
+    if inner % 64 != 0:
+        return skinny_rows(inner, paired=True)
+    groups = -(-outputs // 32)
+    rounds = -(-groups // 256)
+    return GLU_STREAM_ROWS if inner <= 4096 and (rounds <= 1 or 8 * groups >= 7 * 256 * rounds) else GLU_STREAM_DEEP_ROWS
 
 
 # The stacked q, k, v product with rotation and append in its epilogue replaces two kernels of

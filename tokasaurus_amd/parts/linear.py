@@ -88,7 +88,12 @@ class Linear:
         """Whether ``m`` rows take the weight-streaming kernels: up to a number of rows that
         depends on the inner size (``ops.skinny_rows``; gate and up: ``ops.glu_rows``); a
         32-bit result (the head) up to ``ops.SKINNY_ROWS``."""
-        limit = ops.SKINNY_ROWS if out_f32 else (ops.glu_rows if paired else ops.skinny_rows)(self.in_features)
+        if out_f32:
+            limit = ops.SKINNY_ROWS
+        else:
+            limit = ops.skinny_rows(self.in_features, paired)
+            if paired:
+                limit = max(limit, ops.glu_rows(self.in_features, self.total_out // 2))
         return self.weight.dtype == torch.bfloat16 and 0 < m <= limit and self._aligned()
 
     def __call__(
