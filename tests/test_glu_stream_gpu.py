@@ -85,3 +85,21 @@ def test_rows_of_gate_and_up():
     from tokasaurus_amd.kernels import ops
 
     assert ops.glu_rows(2048) == ops.glu_rows(64) == 64 and ops.glu_rows(2080) == ops.skinny_rows(2080, paired=True)
+
+
+@pytest.mark.parametrize("m", [20, 40, 64])
+@pytest.mark.parametrize("layout", ["odd stride", "odd start", "columns"])
+def test_rows_that_lie_anywhere_take_the_librarys_product(m, layout):
+    """Rows of 20 and more were the library's, which reads them wherever they lie."""
+    from tokasaurus_amd.kernels import ops
+    from tokasaurus_amd.parts.linear import Linear
+
+    n, k = 72, 4096
+    x, w, _ = _case(m, n, k, m)
+    buf = torch.zeros((m, k + 9), dtype=torch.bfloat16, device="cuda")
+    rows = {"odd stride": buf[:, :k], "odd start": buf.view(-1)[1 : 1 + m * k].view(m, k), "columns": buf.view(-1)[: m * k].view(k, m).t()}[layout]
+    rows.copy_(x)
+    lin = Linear(k, ["gate", "up"], [n, n])
+    lin.weight = w.cuda()
+    assert ops.skinny_rows(k, paired=True) < m <= ops.glu_rows(k, n) and not ops.rows_at_16_bytes(rows)
+    _check(lin(rows, swiglu=True), x.double(), w, _silu, k)

@@ -900,6 +900,11 @@ def glu_rows(inner: int, outputs: int = 0) -> int:
     return GLU_STREAM_ROWS if inner <= 4096 and (rounds <= 1 or 8 * groups >= 7 * 256 * rounds) else GLU_STREAM_DEEP_ROWS
 
 
+def rows_at_16_bytes(x: torch.Tensor) -> bool:
+    """Whether bfloat16 rows start where the hand-written products read them, at multiples of 16 bytes."""
+    return x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+
+
 # The stacked q, k, v product with rotation and append in its epilogue replaces two kernels of
 # the library path and has a short inner size: it stays ahead up to 32 rows (4 % of a step) at an
 # inner size of 2 048, and up to twice the rows of an ordinary paired product at wider ones.

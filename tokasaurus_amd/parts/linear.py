@@ -135,7 +135,9 @@ class Linear:
                 x = x.materialize()
         m = x.shape[0]
         if w.dtype == torch.bfloat16 and m > 0 and (m > ops.SKINNY_ROWS or self._aligned()):
-            if self._fast(m, swiglu, out_f32):
+            # (so many rows may lie anywhere: where the streamed gate and up cannot read them, the library's product does)
+            anywhere = swiglu and m > ops.skinny_rows(self.in_features, paired=True)
+            if self._fast(m, swiglu, out_f32) and (not anywhere or ops.rows_at_16_bytes(x)):
                 return ops.gemm_skinny_bf16(x, w, residual=residual, out_f32=out_f32, swiglu=swiglu,
                                             prenorm=prenorm, norm_eps=eps, out=out, bias=bias, glu=glu if swiglu else None,
                                             out_scale=out_scale)
