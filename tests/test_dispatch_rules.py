@@ -70,6 +70,8 @@ def test_prompts_leave_the_split_attention_by_their_own_length():
     assert not splits(512, True, 256, 256) and splits(480, True, 240, 240)
     assert splits(512, True, 256, 1024) and splits(512, True, 256, 0) and splits(512, False, 256, 256)
     assert not splits(2048, False, 64, 100_000)
+    # heads wider than 128 are walked one block of keys a step
+    assert splits(1023, True, 512, 512, widest=256) and not splits(1024, True, 512, 512, widest=256) and not splits(512, True, 512, 512, widest=128)
     # tokens of a section or behind a window see no more than it holds, however long the request
     assert not splits(512, True, 256, 5000, section=200) and not splits(512, True, 256, 5000, window=200)
     assert splits(512, True, 256, 5000, section=300) and splits(512, True, 256, 5000, window=300)

@@ -1870,25 +1870,32 @@ def attention_tile_turns_halves(value_dim: int) -> bool:
 
 
 ATTENTION_TILE_SPLIT_BELOW = 2048  # (tile, head block) pairs of a step below which the wavefronts share tiles
-# The same for bfloat16 prompts, whose wavefronts walk two blocks of keys a step when each has a tile of its own: where no
-# token sees more keys than the step has tokens.  Split / one tile a wavefront on an MI355X, 32 heads of 64: 256 tokens
-# (512 pairs) 20.7 / 17.4 us, 512 tokens 48.6 / 27.8, 1,024 tokens 124 / 50, four prompts of 100 (896 pairs) 28 / 16; 16
-# heads of 128: 384 tokens (384 pairs) 37 / 33, 256 tokens 18.8 / 25.8; 8 heads of 64: 768 tokens (384 pairs) 29 / 37,
-# 1,024 tokens 39 / 46, 2,048 tokens 102 / 85.  Single tokens after long contexts are one long walk each: they stay split.
+# The same for bfloat16 prompts, whose wavefronts walk two blocks of keys a step when each has a tile of its own (heads of up to
+# 128; one block where keys or values are wider): where no token sees more keys than the step has tokens.  Split / one tile a
+# wavefront on an MI355X, 32 heads of 64: 256 tokens (512 pairs) 19 / 15 us, 512 tokens 47 / 24, 1,024 tokens 119 / 44, four prompts
+# of 100 (896 pairs) 27 / 12; 16 heads of 128: 256 tokens (256 pairs) 18.8 / 25.8, 512 tokens 33 / 35, 768 tokens 59 / 48; 8 heads of
+# 64: 768 tokens (384 pairs) 29 / 37, 1,024 tokens 39 / 46, 2,048 tokens 102 / 85.  16 heads of 256: 512 tokens 76 / 100, 768 tokens
+# 133 / 144, 1,024 tokens 212 / 188; keys of 64 beside values of 256 58 / 88, 105 / 127, 174 / 165; keys of 192 beside values of 128
+# 53 / 61, 92 / 86, 145 / 113.  Single tokens after long contexts are one long walk each: they stay split.
 ATTENTION_TILE_SPLIT_PROMPTS_BELOW = 512
+ATTENTION_TILE_SPLIT_WIDE_PROMPTS_BELOW = 1024
 ATTENTION_TILE_WORKGROUPS = 512  # workgroups a step with key chunks should have before its chunks grow
 ATTENTION_TILE_LONGEST_CHUNK = 2048
 # Room for partial results a call may take at most; a step of so many workgroups (61 000 with values of 64) has longer chunks
 ATTENTION_TILE_PART_BYTES = 256 << 20
 
 
-def attention_tile_splits(pairs: int, prompts: bool, rows: int, longest: int, window: int = 0, section: int = 0) -> bool:
+def attention_tile_splits(pairs: int, prompts: bool, rows: int, longest: int, window: int = 0, section: int = 0,
+                          widest: int = 0) -> bool:
     """Whether a step of so many (tile, head block) pairs takes the form whose wavefronts share a tile.  ``prompts``: bfloat16
     rows of portions (a step of single tokens does not depend on its own lengths: it is recorded for others); ``longest``: the
-    step's own longest request (0: not known), whose tokens see at most ``window`` keys or those of their ``section``."""
+    step's own longest request (0: not known), whose tokens see at most ``window`` keys or those of their ``section``;
+    ``widest``: the larger of a key's and a value's size."""
     reach = int(section) or int(window)
     seen = min(int(longest), reach) if reach > 0 else int(longest)
-    return pairs < (ATTENTION_TILE_SPLIT_PROMPTS_BELOW if prompts and 0 < seen <= rows else ATTENTION_TILE_SPLIT_BELOW)
+    if not (prompts and 0 < seen <= rows):
+        return pairs < ATTENTION_TILE_SPLIT_BELOW
+    return pairs < (ATTENTION_TILE_SPLIT_PROMPTS_BELOW if widest <= 128 else ATTENTION_TILE_SPLIT_WIDE_PROMPTS_BELOW)
 
 
 def attention_tile_chunks(groups: int, key_chunk: int, bound: int, longest: int, reach: int, words: int) -> tuple[int, int]:
@@ -1963,7 +1970,7 @@ def attention_tile_f32(
     own = int(step_longest) or int(longest)
     if split is None:
         prompts = q.dtype == torch.bfloat16 and tile_req.numel() < q.shape[0]
-        split = attention_tile_splits(pairs, prompts, q.shape[0], own, window, section)
+        split = attention_tile_splits(pairs, prompts, q.shape[0], own, window, section, max(key_dim, value_dim))
     _need(q.dim() == 2 and q.stride(1) == 1 and q.shape[1] >= nq * key_dim,
           "attention: q must be 2-d with unit inner stride and nq*d leading columns")
     for t, name in ((block_table, "block_table"), (q_start, "q_start"), (kv_len, "kv_len"), (tile_req, "tile_req"), (tile_row0, "tile_row0")):
