@@ -88,13 +88,12 @@ class Linear:
         """Whether ``m`` rows take the weight-streaming kernels: up to a number of rows that
         depends on the inner size (``ops.skinny_rows``; gate and up: ``ops.glu_rows``); a
         32-bit result (the head) up to ``ops.SKINNY_ROWS``."""
+        if self.weight.dtype != torch.bfloat16 or not 0 < m <= ops.SKINNY_MAX_ROWS or not self._aligned():
+            return False
         if out_f32:
-            limit = ops.SKINNY_ROWS
-        else:
-            limit = ops.skinny_rows(self.in_features, paired)
-            if paired:
-                limit = max(limit, ops.glu_rows(self.in_features, self.total_out // 2))
-        return self.weight.dtype == torch.bfloat16 and 0 < m <= limit and self._aligned()
+            return m <= ops.SKINNY_ROWS
+        return (m <= ops.skinny_rows(self.in_features, paired)
+                or (paired and m <= ops.GLU_STREAM_ROWS and m <= ops.glu_rows(self.in_features, self.total_out // 2)))
 
     def __call__(
         self,
@@ -135,9 +134,9 @@ class Linear:
                 x = x.materialize()
         m = x.shape[0]
         if w.dtype == torch.bfloat16 and m > 0 and (m > ops.SKINNY_ROWS or self._aligned()):
-            # (so many rows may lie anywhere: where the streamed gate and up cannot read them, the library's product does)
-            anywhere = swiglu and m > ops.skinny_rows(self.in_features, paired=True)
-            if self._fast(m, swiglu, out_f32) and (not anywhere or ops.rows_at_16_bytes(x)):
+            # (more rows than the weight-streaming product's may lie anywhere: where the streamed gate and up cannot read them,
+            # the library's product does)
+            if self._fast(m, swiglu, out_f32) and (not swiglu or ops.rows_at_16_bytes(x) or m <= ops.skinny_rows(self.in_features, paired=True)):
                 return ops.gemm_skinny_bf16(x, w, residual=residual, out_f32=out_f32, swiglu=swiglu,
                                             prenorm=prenorm, norm_eps=eps, out=out, bias=bias, glu=glu if swiglu else None,
                                             out_scale=out_scale)
