@@ -145,3 +145,16 @@ def test_an_engines_prompt_takes_a_tile_a_wavefront(tmp_path, monkeypatch):
     runner.run([StepEntry("a", tokens[290:291], [])])
     assert len(chosen) >= 3 and all(chosen[1:])
     compare_rows(got, plain_rows(folder, {"a": tokens}), TOL["bfloat16"])
+
+
+@pytest.mark.parametrize("options", [{}, {"window": 100}, {"section": 150}])
+def test_chunks_end_with_the_steps_own_longest_request(options):
+    """The chunks behind it hold nothing: without them the sums are the same, bit by bit."""
+    gen = torch.Generator().manual_seed(11)
+    lens, portions = [200, 1100], [16, 40]
+    keys, values, kc, vc, table = _paged(lens, 2, 64, 64, 16, gen)
+    q = torch.randn((sum(portions), 4, 64), generator=gen).bfloat16()
+    args = (q, kc, vc, table, portions, lens, 4, 2, 64, 64, 16)
+    planned, _ = _run(*args, split=True, key_chunk=256, longest=8192, scale=0.125, **options)
+    own, _ = _run(*args, split=True, key_chunk=256, longest=8192, step_longest=1100, scale=0.125, **options)
+    assert torch.isfinite(own).all() and torch.equal(own, planned)

@@ -1,6 +1,6 @@
 // Paged attention for any head size, group size, page size and window, in
-// 32-bit arithmetic: the attention of the true 32-bit path, and of the bfloat16
-// path for shapes the MFMA kernels refuse.
+// 32-bit arithmetic: the attention of shapes the matrix-core kernels refuse
+// (attention_mfma.hip, attention_tile_f32.h).
 //
 // One workgroup per (query token, kv head).  It serves the `group` query heads
 // that share the kv head, walks the token's keys in chunks of CH positions

@@ -1,6 +1,7 @@
 // Paged attention in 32-bit arithmetic on the matrix cores (v_mfma_f32_16x16x4_f32): scores,
-// softmax weights and the weighted values are 32-bit products of 32-bit operands, whatever the
-// storage type of queries, keys and values.  For mixers that ask for exactly that: a sliding
+// softmax weights and the weighted values are 32-bit numbers and 32-bit sums, whatever the
+// storage type of queries, keys and values (from bfloat16 storage some of the products run on the bfloat16 matrix cores,
+// exactly: ScoresFromStorage, at_pieces).  For the 32-bit path, and for mixers that ask for exactly that: a sliding
 // window, key and value heads of different sizes, a scale of the model's choosing and a
 // learned sink per query head in the softmax's denominator; or, with `score_bias` (one number a
 // query head), no softmax at all: a visible key's weight is sigmoid(score + score_bias[head]), not
@@ -36,7 +37,8 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 // bfloat16 product with 32-bit sums (v_mfma_f32_16x16x32_bf16) gives 32-bit scores of the stored queries and keys
 // like the 32-bit product of the converted operands, at an eighth of the instructions and without the conversions.
 // Its operands are what a lane holds anyway: 8 neighbouring elements of key lane % 16 (of the column's query) from
-// element 8 * (lane / 16) of every 32 on.  The weighted values stay 32-bit products: the weights are 32-bit numbers.
+// element 8 * (lane / 16) of every 32 on.  The weights are 32-bit numbers: weighted values are 32-bit products, or where a step
+// is two blocks of keys (at_halves) products of the weights' three exact pieces.
 template <typename T>
 struct ScoresFromStorage { static constexpr bool value = false; };
 template <>

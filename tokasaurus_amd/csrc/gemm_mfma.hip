@@ -602,14 +602,14 @@ __global__ __launch_bounds__(1024) void gemm_staged_kernel(GemmArgs a) {
 // ---------------------------------------------------------------------------------
 // Gate and up projections for up to 64 rows (SwiGLU epilogue; glu_streams says when): a workgroup of 4 wavefronts owns 32 pairs of weight rows
 // and all of K.  In steps of 64 elements the 64 rows of W and the rows of A (16 * MB, the last one again behind M) go
-// straight from memory to local memory, ST_STAGES - 1 steps ahead, so that a compute unit has 40 KB and more of W on the
+// straight from memory to local memory, gl_stages - 1 steps ahead, so that a compute unit has 40 KB and more of W on the
 // way whatever the wavefronts do; two workgroups share a unit.  Wavefront w takes 8 gate rows and their 8 up rows as one
 // tile of 16: the halves of a pair meet in lanes l and l + 32.
 // LDS: [stage][64 W rows, then 16 * MB A rows][64 elements], the 16-byte piece c of row r at place c ^ (r % 8): a load
 // instruction writes 8 whole rows in lane order, and 16 rows read at one K meet in all banks.
 // Bound by reading W.  Measured against the library's product and the pass behind it (us): N = 14,336, K = 4,096 (235 MB)
-// 66 / 47.5 at 16 rows (4.9 TB/s), 55.6 / 49.7 at 32, 65 / 52.7 at 48, 54.6 / 55.4 at 64; 8,192 x 3,072 25.1 / 19.9 at 16, 27.8 / 25.2
-// at 64; 8,192 x 2,048 20.3 / 17.0 at 16, 21.1 / 18.9 at 64.
+// 66.7 / 49.6 at 16 rows (4.7 TB/s), 60.6 / 51.9 at 32, 67.4 / 54.9 at 48, 60.7 / 58.2 at 64; 8,192 x 3,072 25.3 / 20.6 at 16, 28.2 /
+// 25.3 at 64; 8,192 x 2,048 20.3 / 18.0 at 16, 21.6 / 20.3 at 64 (ops.glu_rows has more, and where the library is ahead).
 // ---------------------------------------------------------------------------------
 #define GL_K 64
 
