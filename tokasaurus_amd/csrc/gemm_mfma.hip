@@ -608,8 +608,9 @@ __global__ __launch_bounds__(1024) void gemm_staged_kernel(GemmArgs a) {
 // LDS: [stage][64 W rows, then 16 * MB A rows][64 elements], the 16-byte piece c of row r at place c ^ (r % 8): a load
 // instruction writes 8 whole rows in lane order, and 16 rows read at one K meet in all banks.
 // Bound by reading W.  Measured against the library's product and the pass behind it (us): N = 14,336, K = 4,096 (235 MB)
-// 66.7 / 49.6 at 16 rows (4.7 TB/s), 60.6 / 51.9 at 32, 67.4 / 54.9 at 48, 60.7 / 58.2 at 64; 8,192 x 3,072 25.3 / 20.6 at 16, 28.2 /
-// 25.3 at 64; 8,192 x 2,048 20.3 / 18.0 at 16, 21.6 / 20.3 at 64 (ops.glu_rows has more, and where the library is ahead).
+// 62.3 / 42.3 at 16 rows (5.6 TB/s), 60.5 / 45.5 at 32, 64.2 / 49.0 at 48, 55.9 / 52.9 at 64; 8,192 x 3,072 24.0 / 20.4 at 16, 25.9 /
+// 25.0 at 64; 8,192 x 2,048 19.2 / 14.2 at 16, 20.0 / 17.1 at 64 (ops.glu_rows has more, and where the library is ahead).
+// With all workgroups at the same step of K: 46.3, 48.6, 52.0 and 54.8; 20.1 and 24.9; 17.2 and 19.4.
 // ---------------------------------------------------------------------------------
 #define GL_K 64
 
@@ -635,9 +636,12 @@ __global__ __launch_bounds__(256, 2) void gemm_glu_stream_kernel(GemmArgs a) {
 #pragma unroll
   for (int i = 0; i < MB / 2; ++i) src[2 + i] = a.A + (size_t)min((wave * (MB / 2) + i) * 8 + lr, a.M - 1) * a.lda + piece;
   const int steps = a.K / GL_K;
+  // a workgroup begins its walk over K 7 steps behind its neighbour's beginning and comes round: in step, 256 workgroups would
+  // read the same columns of rows that lie 2 K bytes apart, which for a K of a power of two are few of the memory's channels
+  const int turn = (int)(blockIdx.x * 7u % (unsigned)steps);
   auto ask = [&](int step) {
     const unsigned base = lds + (unsigned)(step % S * ROWS * GL_K * sizeof(bf16_t));
-    const size_t k = (size_t)step * GL_K;
+    const size_t k = (size_t)(step + turn < steps ? step + turn : step + turn - steps) * GL_K;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       const int row = i < 2 ? wave * 16 + i * 8 : 64 + (wave * (MB / 2) + i - 2) * 8;

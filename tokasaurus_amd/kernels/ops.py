@@ -885,8 +885,9 @@ GLU_STREAM_DEEP_ROWS = 16  # and those up to which it is ahead whatever the size
 def glu_rows(inner: int, outputs: int = 0) -> int:
     """Rows up to which gate and up (with the gated activation behind them; ``outputs`` of each, 0: not known) take the
     hand-written product.  At an inner size of a multiple of 64 that is its streamed form, a workgroup 32 outputs.  Library's product
-    and the pass behind it / streamed on an MI355X, us, at 16, 32 and 64 rows: 8,192 x 2,048 20.3 / 18.0, 20.4 / 18.7, 21.6 / 20.3;
-    8,192 x 3,072 25.3 / 20.6, 25.6 / 22.0, 28.2 / 25.3; 14,336 x 4,096 66.7 / 49.6, 60.6 / 51.9, 60.7 / 58.2; 1,000 x 1,024 9.9 / 6.8,
+    and the pass behind it / streamed on an MI355X, us, at 16, 32 and 64 rows: 8,192 x 2,048 19.2 / 14.2, 19.2 / 15.0, 20.0 / 17.1;
+    8,192 x 3,072 24.0 / 20.4, 24.3 / 21.6, 25.9 / 25.0; 14,336 x 4,096 62.3 / 42.3, 60.5 / 45.5, 55.9 / 52.9; the next ones before the
+    workgroups began their walks apart (the streamed form gains where K is a power of two) 1,000 x 1,024 9.9 / 6.8,
     13.8 / 7.9, 14.0 / 10.4; 24,576 x 2,048 54.9 / 45.1, 53.0 / 45.5, 55.8 / 50.4: ahead up to 64 rows.  Not where the last round of
     workgroups leaves more than an eighth of the compute units idle, 9,216 x 2,048 60.7 / 23.1, 24.5 / 25.2, 26.9 / 29.5; 10,240 x 2,560
     50.9 / 29.3, 29.2 / 32.2, 34.3 / 40.4; 11,008 x 4,096 55.0 / 44.7, 44.9 / 46.6, 47.8 / 52.4; 12,288 x 4,096 50.3 / 48.7, 48.4 / 50.3,
@@ -898,6 +899,13 @@ def glu_rows(inner: int, outputs: int = 0) -> int:
     groups = -(-outputs // 32)
     rounds = -(-groups // 256)
     return GLU_STREAM_ROWS if inner <= 4096 and (rounds <= 1 or 8 * groups >= 7 * 256 * rounds) else GLU_STREAM_DEEP_ROWS
+
+
+def glu_streams(rows: int, outputs: int, inner: int) -> bool:
+    """Whether gate and up are asked for in their streamed form whatever the product itself would choose: where there is a workgroup
+    for every compute unit.  Weight-streaming / streamed on an MI355X since its workgroups begin their walks apart, us: 8,192 x 2,048
+    15.8 / 14.9 at one row, 16.8 / 14.1 at 8; 8,192 x 3,072 24.0 / 21.5 at one; 14,336 x 4,096 49.6 / 42.3 at one."""
+    return outputs >= 32 * 256 and inner % 64 == 0 and 0 < rows <= GLU_STREAM_ROWS
 
 
 def rows_at_16_bytes(x: torch.Tensor) -> bool:

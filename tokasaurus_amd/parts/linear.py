@@ -139,7 +139,8 @@ class Linear:
             if self._fast(m, swiglu, out_f32) and (not swiglu or ops.rows_at_16_bytes(x) or m <= ops.skinny_rows(self.in_features, paired=True)):
                 return ops.gemm_skinny_bf16(x, w, residual=residual, out_f32=out_f32, swiglu=swiglu,
                                             prenorm=prenorm, norm_eps=eps, out=out, bias=bias, glu=glu if swiglu else None,
-                                            out_scale=out_scale)
+                                            out_scale=out_scale,
+                                            staged=2 if swiglu and ops.glu_streams(m, self.total_out // 2, self.in_features) else -1)
             # library matrix product (hipBLASLt), 32-bit accumulation; with a bias through the tensor
             # library, whose call adds it to the 32-bit sums in the product's own epilogue (addmm)
             direct = ops.gemm_library_direct(x, w)
