@@ -1,0 +1,87 @@
+"""Products with K cut among workgroups and the passes that add the cuts, at the edges of the kernel's blocks of rows, tiles of
+weight rows and ring of steps, against sums in 64-bit and against the passes behind a whole product."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from tokasaurus_amd.kernels import ops
+from tokasaurus_amd.kernels.library import call
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(m, n, k, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    wide = torch.randn((m, k + 64), generator=gen, device="cuda").bfloat16()
+    return wide[:, 32 : k + 32], (torch.randn((n, k), generator=gen, device="cuda") / k ** 0.5).bfloat16(), gen
+
+
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 32, 33, 64, 65, 96, 97, 128])
+@pytest.mark.parametrize("n,k", [(8, 64), (72, 192), (64, 256), (200, 1088), (2048, 2048), (3000, 960)])
+def test_cuts_against_64_bit_sums(m, n, k):
+    """Every cut is 32-bit sums of at most k products, and their sum has as many terms as there are cuts: (k + 16) 2^-24 of the
+    sum of the magnitudes."""
+    x, w, _ = _case(m, n, k, m + n + k)
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    part = ops.gemm_split(x, w)
+    assert part.shape == (ops.split_cuts(n, k), m, n)
+    for cuts in {1, 2, 3, k // 64}:
+        if cuts > k // 64:
+            continue
+        own = torch.full((cuts, m, n), float("nan"), device="cuda")
+        call("tk_gemm_split_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), own.data_ptr(), m, n, k, cuts, torch.cuda.current_stream().cuda_stream)
+        for got in (part, own):
+            assert float(((got.double().sum(0) - want).abs() / (size + 1e-30)).max()) <= (k + 16) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("rows,hidden,cuts", [(1, 8, 1), (3, 72, 5), (17, 2048, 8), (5, 4096, 4), (2, 8192, 3), (2, 9000, 2)])
+@pytest.mark.parametrize("w32", [False, True])
+def test_residual_sum_and_norm(rows, hidden, cuts, w32):
+    """The very bits of the pass behind a whole product, for a product that is the cuts' sum in ascending order."""
+    gen = torch.Generator(device="cuda").manual_seed(hidden + cuts)
+    part = torch.randn((cuts, rows, hidden), generator=gen, device="cuda")
+    residual = torch.randn((rows, hidden), generator=gen, device="cuda").bfloat16()
+    weight = torch.randn((hidden,), generator=gen, device="cuda")
+    weight = weight if w32 else weight.bfloat16()
+    whole = part[0].clone()
+    for c in range(1, cuts):
+        whole += part[c]
+    for got, want in zip(ops.split_add_rmsnorm(part, residual, weight, 1e-5), ops.add_rmsnorm(whole.bfloat16(), residual, weight, 1e-5)):
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("nq,nkv,d,page", [(4, 2, 16, 16), (32, 8, 64, 16), (5, 5, 80, 4), (16, 2, 128, 32)])
+@pytest.mark.parametrize("tables", [True, False])
+def test_rotation_and_append(nq, nkv, d, page, tables):
+    rows, cuts, width = 19, 3, (nq + 2 * nkv) * d
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    part = torch.randn((cuts, rows, width), generator=gen, device="cuda")
+    whole = (part[0] + part[1]) + part[2]
+    positions = torch.randperm(3 * page, generator=gen, device="cuda")[:rows].to(torch.int32) if 3 * page >= rows else torch.arange(rows, device="cuda", dtype=torch.int32) % (3 * page)
+    req = torch.arange(rows, device="cuda", dtype=torch.int32)
+    table = torch.randperm(rows * 3, generator=gen, device="cuda").to(torch.int32).view(rows, 3)
+    cos, sin = ops.rope_table(1.0 / 10000 ** (torch.arange(0, d, 2, device="cuda").float() / d), 3 * page) if tables else (None, None)
+    pages = [[torch.zeros(shape(rows * 3, nkv, page, d), dtype=torch.bfloat16, device="cuda") for shape in (ops.key_pages_shape, ops.value_pages_shape)]
+             for _ in range(2)]
+    got = ops.split_rope_append(part, ops.RopeAppend(positions, req, table, cos, sin, *pages[0], nq, nkv, d, page))
+    stacked = whole.bfloat16()
+    ops.rope_append(stacked, positions, req, table, cos, sin, *pages[1], nq, nkv, d, page)
+    assert torch.equal(got, stacked[:, : nq * d])
+    assert torch.equal(pages[0][0], pages[1][0]) and torch.equal(pages[0][1], pages[1][1])
+    assert pages[0][0].count_nonzero() > 0
+
+
+def test_what_is_refused():
+    x, w, _ = _case(4, 64, 128, 1)
+    for bad in ((x[:, :96], w[:, :96].contiguous()), (x, w[:60]), (torch.cat([x] * 33), w), (x.float(), w.float()), (x[:, 1:65], w[:, :64].contiguous())):
+        with pytest.raises(ops.KernelError):
+            ops.gemm_split(*bad)
+
+
+def test_cuts_fill_the_compute_units():
+    for n in range(64, 16384, 192):
+        for k in (64, 512, 2048, 8192):
+            cuts = ops.split_cuts(n, k)
+            assert 1 <= cuts <= max(1, min(16, k // 256))

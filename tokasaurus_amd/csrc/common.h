@@ -180,6 +180,17 @@ __device__ __forceinline__ float row_sum16(float v) {
   return v;
 }
 
+// --------------------------------------------------------------------------
+// 16 bytes of the storage type at a time, where sizes and addresses allow it
+// --------------------------------------------------------------------------
+template <typename T>
+struct Pack {
+  static constexpr int N = 16 / sizeof(T);
+  union { uint4 raw; T v[N]; };
+  __device__ __forceinline__ void load(const T* p) { raw = *(const uint4*)p; }
+  __device__ __forceinline__ void store(T* p) const { *(uint4*)p = raw; }
+};
+
 // 16 bytes a lane from memory to local memory, lane l to `lds` (the same for the wavefront) + 16 l.  Counted in vmcnt, which
 // the caller waits for: the compiler knows nothing of the load.
 __device__ __forceinline__ void load_to_lds(const bf16_t* src, unsigned lds) {

@@ -36,17 +36,6 @@ TK_API int tk_embed_gather(int dt, const int* ids, const int* last_token, const 
   return 0;
 }
 
-// --------------------------------------------------------------------------
-// 16 bytes of the storage type at a time, where sizes and addresses allow it
-// --------------------------------------------------------------------------
-template <typename T>
-struct Pack {
-  static constexpr int N = 16 / sizeof(T);
-  union { uint4 raw; T v[N]; };
-  __device__ __forceinline__ void load(const T* p) { raw = *(const uint4*)p; }
-  __device__ __forceinline__ void store(T* p) const { *(uint4*)p = raw; }
-};
-
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 // --------------------------------------------------------------------------

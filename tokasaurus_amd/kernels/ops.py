@@ -7,6 +7,7 @@ step can be recorded into a HIP graph.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from dataclasses import dataclass
 
@@ -1090,6 +1091,105 @@ def gemm_skinny_bf16(
         m, n, k, epi, waves_k, tiles, staged, tile_rows, 1 if fold else 0, _stream(),
     )
     return (out, emitted) if emit_weight is not None else out
+
+
+# --------------------------------------------------------------------------
+# bfloat16 products with K cut among workgroups, and the passes that add the cuts
+# --------------------------------------------------------------------------
+
+SPLIT_ROWS = 128  # rows the split product takes
+SPLIT_TILE, SPLIT_STEP = 64, 64  # weight rows a workgroup, elements of K a step
+# Elements of x (rows x inner size) from which the split product and the pass that adds its cuts are ahead of the
+# weight-streaming kernel, whose workgroups each read all of x.  Measured on an MI355X, weights from memory, us:
+#   residual sum and norm behind it, weight-streaming / split: 2,048 x 2,048 8.5 / 8.7 at 20 rows, 8.9 / 8.7 at 24, 12.3 / 9.4 at
+#   40; 3,072 x 3,072 10.2 / 10.5 at 12, 10.9 / 10.5 at 16; 4,096 x 4,096 12.9 / 13.3 at 10, 13.6 / 13.4 at 12, 14.7 / 13.4 at 16;
+#   2,048 x 8,192 12.1 / 12.4 at 2, 13.8 / 12.6 at 6, 18.4 / 13.0 at 16; 3,072 x 8,192 15.5 / 16.1 at 4, 17.4 / 16.4 at 8;
+#   4,096 x 14,336 28.9 / 27.8 at 2, 31.6 / 26.9 at 8 (and the library's product with its pass: 2,048 x 8,192 16.6 at 16, 25.9 /
+#   14.0 at 64, 25.0 / 17.7 at 128; 2,048 x 2,048 12.2 / 10.4 at 64, 12.0 / 13.2 at 128; 4,096 x 14,336 42.6 / 30.7 at 64, 78.8 /
+#   39.1 at 128)
+#   rotation and append: 3,072 x 2,048 8.1 / 8.0 at 12 rows, 9.2 / 8.2 at 20; 5,120 x 3,072 11.7 / 11.8 at 8, 12.8 / 11.9 at 12;
+#   6,144 x 4,096 16.1 / 14.9 at 6, 18.2 / 15.2 at 16 (library 16.1 / 10.2 at 64 and 18.9 / 13.8 at 128 for the first, 25.7 / 18.4
+#   and 33.6 / 25.7 for the last)
+SPLIT_NORM_ELEMENTS = 48_000
+SPLIT_ROPE_ELEMENTS = 24_000
+# Elements of w from which: it pays below too (1,024 x 1,024 8.8 / 7.4 at 48 rows, 512 x 512 7.3 / 6.5 at 64), but little, and there a
+# step keeps one kernel, hence its bits, whether it is padded to a recorded size or not.
+SPLIT_WEIGHT_ELEMENTS = 1 << 20
+
+
+@functools.lru_cache(maxsize=None)
+def split_cuts(n: int, k: int) -> int:
+    """Cuts of K for a weight [n, k]: the fewest for which the 256 compute units' rounds of workgroups are filled to nine tenths,
+    a workgroup keeping four steps of K."""
+    tiles = -(-n // SPLIT_TILE)
+    most = max(1, min(16, k // (4 * SPLIT_STEP)))
+    filled = lambda c: tiles * c / (256 * -(-tiles * c // 256))  # noqa: E731
+    return next((c for c in range(1, most + 1) if filled(c) >= 0.9), max(range(1, most + 1), key=filled))
+
+
+def split_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``gemm_split`` takes this product."""
+    n, k = w.shape
+    return (0 < x.shape[0] <= SPLIT_ROWS and x.dtype == w.dtype == torch.bfloat16 and k % SPLIT_STEP == 0 and n % 8 == 0
+            and rows_at_16_bytes(x) and w.data_ptr() % 16 == 0)
+
+
+def split_norm_takes(residual: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether ``split_add_rmsnorm`` reads these: rows and a weight that start at multiples of 16 bytes."""
+    return residual.dtype == torch.bfloat16 and residual.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and residual.shape[1] % 8 == 0
+
+
+def gemm_split(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x [M <= 128, K] . w [N, K]^T in bfloat16 with K cut among workgroups: the cuts' 32-bit sums [cuts, M, N], which
+    ``split_add_rmsnorm`` or ``split_rope_append`` adds in ascending order."""
+    _gpu(x, w)
+    _need(x.dim() == 2 and w.dim() == 2 and w.is_contiguous() and x.shape[1] == w.shape[1] and split_takes(x, w),
+          "gemm_split: x [M, K] (up to 128 rows at multiples of 16 bytes) and w [N, K] must be bfloat16, K a multiple of 64, N of 8")
+    m, (n, k) = x.shape[0], w.shape
+    cuts = split_cuts(n, k)
+    part = torch.empty((cuts, m, n), dtype=torch.float32, device=x.device)
+    call("tk_gemm_split_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), part.data_ptr(), m, n, k, cuts, _stream())
+    return part
+
+
+def split_add_rmsnorm(part: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float) -> tuple[torch.Tensor, torch.Tensor]:
+    """``add_rmsnorm`` of a split product: (product rounded, + residual, rounded; its RMSNorm times ``weight``) in one pass."""
+    _gpu(part, residual, weight)
+    _need(part.dim() == 3 and part.dtype == torch.float32 and part.is_contiguous() and residual.shape == part.shape[1:]
+          and residual.is_contiguous() and residual.dtype == torch.bfloat16,
+          "split_add_rmsnorm: the sums must be float32 [cuts, rows, H], the residual contiguous bfloat16 [rows, H]")
+    cuts, rows, hidden = part.shape
+    if weight.shape != (hidden,) or not weight.is_contiguous() or weight.dtype not in (torch.bfloat16, torch.float32):
+        raise KernelError("split_add_rmsnorm: the weight must be [H] of bfloat16 or float32")
+    stream_out, out = torch.empty_like(residual), torch.empty_like(residual)
+    call("tk_split_add_rmsnorm", part.data_ptr(), cuts, residual.data_ptr(), weight.data_ptr(), 1 if weight.dtype == torch.float32 else 0,
+         stream_out.data_ptr(), out.data_ptr(), rows, hidden, float(eps), _stream())
+    return stream_out, out
+
+
+def split_rope_append(part: torch.Tensor, r: RopeAppend) -> torch.Tensor:
+    """``rope_append`` of a split [q | k | v] product (whole heads rotated): the cuts added and rounded, q and k rotated, k and v
+    stored in the tokens' pages; returns q [rows, nq * d]."""
+    _gpu(part, r.positions, r.token_req, r.block_table, r.cos, r.sin, r.kcache, r.vcache)
+    _need(part.dim() == 3 and part.dtype == torch.float32 and part.is_contiguous() and part.shape[2] == (r.nq + 2 * r.nkv) * r.head_dim,
+          "split_rope_append: the sums must be float32 [cuts, rows, (nq + 2 nkv) d]")
+    _need(r.rotary_dim is None or r.rotary_dim == r.head_dim, "split_rope_append rotates whole heads")
+    cuts, rows, _ = part.shape
+    for t, name in ((r.positions, "positions"), (r.token_req, "token_req"), (r.block_table, "block_table")):
+        _i32(t, name)
+    _need(r.positions.numel() == rows and r.token_req.numel() == rows and r.block_table.dim() == 2,
+          "split_rope_append: positions/token_req need one entry a row, block_table [requests, width]")
+    _check_pages(r.kcache, r.vcache, r.nkv, r.page_size, r.head_dim, torch.bfloat16, "split_rope_append")
+    if r.cos is not None:
+        _need(r.sin is not None and r.cos.dtype == r.sin.dtype == torch.float32 and r.cos.shape == r.sin.shape
+              and r.cos.shape[1] == r.head_dim // 2 and r.cos.is_contiguous() and r.sin.is_contiguous(),
+              "split_rope_append: cos/sin tables must be contiguous float32 [positions, d/2]")
+    q = torch.empty((rows, r.nq * r.head_dim), dtype=torch.bfloat16, device=part.device)
+    call("tk_split_rope_append", part.data_ptr(), cuts, q.data_ptr(), r.positions.data_ptr(), r.token_req.data_ptr(),
+         r.block_table.data_ptr(), r.block_table.stride(0), r.cos.data_ptr() if r.cos is not None else None,
+         r.sin.data_ptr() if r.sin is not None else None, r.kcache.data_ptr(), r.vcache.data_ptr(), rows, r.nq, r.nkv, r.head_dim,
+         r.page_size, _stream())
+    return q
 
 
 def add(x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:

@@ -164,15 +164,25 @@ class Linear:
         prod = ops.gemm_generic(x, w, residual=residual, out_f32=out_f32, out=out, bias=bias)
         return gated(prod) if swiglu else scaled(prod)
 
+    def _splits(self, x: torch.Tensor, least: int) -> bool:
+        """Whether the product takes the form with K cut among workgroups (``ops.gemm_split``), for a pass behind it that adds
+        the cuts: from ``least`` elements of x on, where the weight-streaming kernel's reads of x show."""
+        return (self.bias is None and x.shape[0] * self.in_features >= least
+                and self.in_features * self.total_out >= ops.SPLIT_WEIGHT_ELEMENTS and ops.split_takes(x, self.weight))
+
     def with_residual(
         self, x: torch.Tensor, residual: torch.Tensor, emit_norm: Norm | None
     ) -> tuple[torch.Tensor, Prepared | None]:
         """residual + product and, where the kernel can, what ``emit_norm`` (the norm
         that will be applied to the result) needs so that it costs no kernel of its own."""
-        if emit_norm is not None and getattr(emit_norm, "fusable_rms", False) and self._fast(x.shape[0]):
+        fusable = emit_norm is not None and getattr(emit_norm, "fusable_rms", False)
+        if fusable and residual.is_contiguous() and self._splits(x, ops.SPLIT_NORM_ELEMENTS) and ops.split_norm_takes(residual, emit_norm.weight):
+            out, normed = ops.split_add_rmsnorm(ops.gemm_split(x, self.weight), residual, emit_norm.weight, emit_norm.eps)
+            return out, Prepared(None, emit_norm, normed)
+        if fusable and self._fast(x.shape[0]):
             out, data = ops.gemm_skinny_bf16(x, self.weight, residual=residual, emit_weight=emit_norm.weight, bias=self.bias)
             return out, Prepared(data, emit_norm)
-        if emit_norm is not None and getattr(emit_norm, "fusable_rms", False) and x.shape[0] > 0:
+        if fusable and x.shape[0] > 0:
             # one pass adds the residual and norms the sum
             out, normed = ops.add_rmsnorm(self(x), residual.contiguous(), emit_norm.weight, emit_norm.eps)
             return out, Prepared(None, emit_norm, normed)
@@ -183,6 +193,12 @@ class Linear:
         append of k and v to the pages in its epilogue; returns q [M, nq*d], or None when
         that kernel does not take this case (the caller then does the steps one by one)."""
         m = (x.x if isinstance(x, Normed) else x).shape[0]
+        whole = rope.head_dim % 8 == 0 and (rope.rotary_dim is None or rope.rotary_dim == rope.head_dim)
+        stream = x.x if isinstance(x, Normed) else x
+        if whole and self._splits(stream, ops.SPLIT_ROPE_ELEMENTS):
+            rows = x.materialize() if isinstance(x, Normed) else x  # (a norm's rows lie as their stream does, or from their own start)
+            if ops.split_takes(rows, self.weight):
+                return ops.split_rope_append(ops.gemm_split(rows, self.weight), rope)
         most = min(ops.SKINNY_ROPE_ROWS, 2 * ops.skinny_rows(self.in_features, paired=True))
         fits = self.weight.dtype == torch.bfloat16 and 0 < m <= most and self._aligned()
         if not fits or rope.head_dim % 2 or (rope.rotary_dim is not None and rope.rotary_dim != rope.head_dim):
