@@ -53,6 +53,17 @@ def test_experts_in_tiles(tokens, experts, top, width, ff, form):
     assert torch.isfinite(got).all()
 
 
+@pytest.mark.parametrize("tokens", [40, 257, 700])
+@pytest.mark.parametrize("experts,top", [(5, 3), (2, 2), (1, 1)])
+@pytest.mark.parametrize("width,ff", [(64, 64), (320, 192), (512, 1088)])
+@pytest.mark.parametrize("form", ["silu", "clamps", "on input"])
+def test_experts_in_pairs_of_tiles(monkeypatch, tokens, experts, top, width, ff, form):
+    """One step of K, fewer than local memory holds, and more; outputs that end inside a block; no, one and several pairs."""
+    monkeypatch.setattr(ops, "EXPERT_PAIRS_FROM_ROWS", 1)
+    assert ops.experts_go_in_pairs_of_tiles(tokens * top, experts, width + 8, width, ff)
+    test_experts_in_tiles(tokens, experts, top, width, ff, form)
+
+
 @pytest.mark.parametrize("tokens,top,experts", [(1, 1, 300), (13, 8, 256), (130, 1, 2), (129, 1, 1), (400, 3, 5), (64, 2, 64)])
 @pytest.mark.parametrize("spread", ["one expert", "all", "each its own"])
 def test_tiles_hold_every_choice(tokens, top, experts, spread):
@@ -71,6 +82,10 @@ def test_tiles_hold_every_choice(tokens, top, experts, spread):
     assert used == int((-(-count // ops.EXPERT_TILE)).sum()) <= s.max_tiles
     slot_pair, group = s.slot_pair.cpu().view(-1, ops.EXPERT_TILE), s.tile_group.cpu()
     assert sorted(slot_pair[slot_pair >= 0].tolist()) == list(range(pairs))
+    runs = s.runs.cpu().view(-1, 4).tolist()  # every used tile in one pair of its expert or alone
+    twos, ones = runs[1 : 1 + runs[0][0]], runs[1 + s.max_tiles // 2 :][: runs[0][1]]
+    mine = [(t + 2 * (i - first) + j, e) for i, (t, e, first, _) in enumerate(twos) for j in range(2)] + [(t, e) for t, e, _, _ in ones]
+    assert sorted(mine) == list(enumerate(group[:used].tolist()))
     for t in range(s.max_tiles):
         mine = slot_pair[t][slot_pair[t] >= 0].long()
         assert (t < used) == (mine.numel() > 0) and (ids.flatten()[mine] == group[t]).all()

@@ -12,11 +12,11 @@
 // first operand of the matrix core, read straight from memory 16 bytes a lane, the rows of A the second; a lane ends up with
 // 4 neighbouring outputs of one row.  The next step's operands are asked for before the current step's products.
 // Experts (grouped_gemm_staged_kernel): tiles of GS_M = 128 slots x 128 weight rows through local memory, however few slots a
-// tile holds (see there).  Sums are 32-bit and run over k in ascending steps for every output: a row's result does not
+// tile holds (see there); experts of many rows take two such tiles as one of 256 x 256 (grouped_gemm_wide_kernel).  Sums are 32-bit and run over k in ascending steps for every output: a row's result does not
 // depend on which other rows share its tile.
 #include <math.h>
 
-#include "common.h"
+#include "gemm_tile.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
@@ -331,19 +331,123 @@ __global__ __launch_bounds__(256, 3) void grouped_gemm_staged_kernel(GroupedArgs
   }
 }
 
+// Experts of many rows: two neighbouring tiles of a group as one of 256 slots x 256 weight rows (in the gated form 128 of gate and
+// 128 of up), the odd last tile of a group 128 x 128 (gemm_tile.h).  The path from the L2 to a compute unit bounds these products,
+// and a tile of 256 x 256 asks for half as many bytes a product; pairs keep an expert's rows filled up to 128 and not to 256.
+// All pairs come before the first single tile, so that the short work fills what the last round of pairs leaves free.
+// 32 experts of 2,048 x 1,024, 2,048 tokens x 8: gate and up 206 to 182 us, down 114 to 93 (with 512 rows for every expert 158
+// and 79: the single tiles cost the rest); 64 x (1,024 x 512) 8,192 tokens x 4: 130 and 66.  With single tiles of 128 x 256 190 and
+// 96; every tile 128 x 256, without pairs, 185 and 105.
+template <class S, bool GLU>
+__device__ __forceinline__ void wide_tile(const GroupedArgs& a, char* smem, int g, int first, int n0) {
+  constexpr int OUT = GLU ? S::BN / 2 : S::BN;
+  static_assert(S::BM <= 256 && S::BM * S::BN * 2 + S::BM * 4 <= S::LDS, "");
+  const int lane = threadIdx.x & (TK_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TK_WAVE);
+  const int wm = wave & 1, wn = wave >> 1, top = a.slots - 1;
+  TileLoop<S, GLU> t;
+  t.wave = wave;
+  t.lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  t.a = (const char*)a.A;
+  t.w = (const char*)(a.W + (size_t)g * a.w_stride + (size_t)n0 * a.K);
+  // (all numbers of rows are asked for before the first is used)
+  const int lr = lane >> 3;
+  int from[S::LA], frow[S::TM], to = -1;
+#pragma unroll
+  for (int i = 0; i < S::LA; ++i) {
+    const int slot = min(first + wave * (16 * S::TM) + i * 8 + lr, top);
+    from[i] = a.a_row ? a.a_row[slot] : slot;
+  }
+  const int own = first + (int)threadIdx.x;  // of the first BM threads
+  if (threadIdx.x < S::BM && own <= top) {
+    to = a.c_row ? a.c_row[own] : own;
+    if (a.a_row && a.a_row[own] < 0) to = -1;
+  }
+  float factor[S::TM];
+#pragma unroll
+  for (int m = 0; m < S::TM; ++m) factor[m] = 1.f;
+  if (GLU && a.row_scale) {
+#pragma unroll
+    for (int m = 0; m < S::TM; ++m) frow[m] = a.scale_row[min(first + wm * (32 * S::TM) + m * 32 + (lane & 31), top)];  // (< 0: an empty slot)
+#pragma unroll
+    for (int m = 0; m < S::TM; ++m) factor[m] = a.row_scale[max(frow[m], 0)];
+  }
+#pragma unroll
+  for (int i = 0; i < S::LA; ++i)
+    t.off[i] = (unsigned)max(from[i], 0) * (unsigned)a.lda * 2 + ((lane & 7) ^ tile_swizzle(i * 8 + lr)) * 16;
+#pragma unroll
+  for (int i = 0; i < S::LW; ++i) {
+    const int row = wave * (16 * S::TN) + i * 8 + lr;  // (a row that is not stored may read any)
+    const int wrow = GLU ? min(row % OUT, a.N - 1 - n0) + (row >= OUT ? a.N : 0) : min(row, a.N - 1 - n0);
+    t.off[S::LA + i] = (unsigned)wrow * (unsigned)a.K * 2 + ((lane & 7) ^ tile_swizzle(i * 8 + lr)) * 16;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (nothing but the rows' loads is counted from here on)
+  t.run(smem, a.K / TILE_K, wm, wn, lane);
+  __syncthreads();
+  int* dst = (int*)(smem + S::BM * S::BN * 2);  // behind the results
+  if (threadIdx.x < S::BM) dst[threadIdx.x] = to;
+  t.deliver(smem, wm, wn, lane, n0, a.N, [&](float gate, float up, int m) { return gg_gated(a, gate * factor[m], up * factor[m]); },
+            [&](int row) -> bf16_t* { return dst[row] < 0 ? nullptr : (bf16_t*)a.C + (size_t)dst[row] * a.ldc; });
+}
+
+#define WIDE_OUT(glu) ((glu) ? 128 : 256)
+#define WIDE_PAIRS (GS_TILES / 2)
+using PairShape = TileShape<4, 4, 2, 3>;
+using SingleShape = TileShape<2, 2, 5, 5>;
+// A pair of tiles or a single one, as a workgroup reads it: the group's first tile (a single: its own), the group, the number of the
+// group's first pair and how many it has.
+struct TileRun {
+  int tile, group, first, count;
+};
+// runs: the numbers of pairs and of single tiles (as TileRun's first two), the pairs, the single tiles
 template <bool GLU>
-static bool launch_staged(const GroupedArgs& a, int tiles, hipStream_t stream) {
+__global__ __launch_bounds__(256, 1) void grouped_gemm_wide_kernel(GroupedArgs a, const TileRun* __restrict__ runs, int max_pairs, int n_blocks,
+                                                                   int single_blocks) {
+  extern __shared__ __align__(16) char smem[];
+  const int pairs = runs->tile, singles = runs->group;
+  int seq = blockIdx.x / GS_DIES;
+  const int per = (pairs * n_blocks + GS_DIES - 1) / GS_DIES;
+  if (seq < per) {
+    const int item = blockIdx.x % GS_DIES * per + seq;
+    if (item >= pairs * n_blocks) return;
+    const int some = item / n_blocks;
+    const TileRun r = runs[1 + some];
+    // the chunk of up to WIDE_PAIRS pairs of the group that the item lies in
+    const int chunk = r.first + (some - r.first) / WIDE_PAIRS * WIDE_PAIRS, len = min(WIDE_PAIRS, r.first + r.count - chunk);
+    const int off = item - chunk * n_blocks, pair = chunk + off % len;
+    wide_tile<PairShape, GLU>(a, smem, r.group, (r.tile + 2 * (pair - r.first)) * GS_M, off / len * WIDE_OUT(GLU));
+    return;
+  }
+  seq -= per;
+  const int per1 = (singles * single_blocks + GS_DIES - 1) / GS_DIES, item = blockIdx.x % GS_DIES * per1 + seq;
+  if (seq >= per1 || item >= singles * single_blocks) return;
+  const TileRun r = runs[1 + max_pairs + item / single_blocks];
+  wide_tile<SingleShape, GLU>(a, smem, r.group, r.tile * GS_M, item % single_blocks * (WIDE_OUT(GLU) / 2));
+}
+
+template <bool GLU>
+static bool launch_by_tile(const GroupedArgs& a, int tiles, const TileRun* runs, int max_singles, hipStream_t stream) {
+  const auto groups = [](long n) { return (n + GS_DIES - 1) / GS_DIES * GS_DIES; };
   const int outs = GLU ? 64 : 128, n_blocks = (a.N + outs - 1) / outs;
-  const long items = (long)tiles * n_blocks, groups = (items + GS_DIES - 1) / GS_DIES * GS_DIES;
-  if (groups >= (1l << 31)) return false;
+  if (runs) {
+    const int max_pairs = tiles / 2, wide_blocks = (a.N + WIDE_OUT(GLU) - 1) / WIDE_OUT(GLU);
+    const long grid = groups((long)max_pairs * wide_blocks) + groups((long)max_singles * n_blocks);
+    constexpr int lds = PairShape::LDS;
+    static_assert(lds >= SingleShape::LDS && SingleShape::BM == GS_M && PairShape::BM == 2 * GS_M, "");
+    auto kernel = grouped_gemm_wide_kernel<GLU>;
+    if (grid >= (1l << 31) || hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return false;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), lds, stream, a, runs, max_pairs, wide_blocks, n_blocks);
+    return true;
+  }
+  const long grid = groups((long)tiles * n_blocks);
+  if (grid >= (1l << 31)) return false;
   const int lds = GS_STAGES * 256 * GS_K * (int)sizeof(bf16_t);  // 48 KB; the results' place is 32 at most
-  hipLaunchKernelGGL(grouped_gemm_staged_kernel<GLU>, dim3((unsigned)groups), dim3(256), lds, stream, a, tiles, n_blocks);
+  hipLaunchKernelGGL(grouped_gemm_staged_kernel<GLU>, dim3((unsigned)grid), dim3(256), lds, stream, a, tiles, n_blocks);
   return true;
 }
 
 TK_API int tk_grouped_gemm_bf16(const void* A, int lda, const int* a_row, const int* c_row, const int* tile_group, int tiles,
                                 int groups_z, int a_cols, int c_cols, const void* W, size_t w_stride, void* C, int ldc,
-                                int N, int K, int slots, int glu, int out_f32, const float* row_scale, const int* scale_row,
+                                int N, int K, int slots, const TileRun* runs, int max_singles, long a_rows, int glu, int out_f32, const float* row_scale, const int* scale_row,
                                 float limit, float alpha, hipStream_t stream) {
   TK_REQUIRE(A && W && C && N > 0 && K > 0 && slots >= 0 && tiles >= 0, "grouped_gemm: bad arguments");
   TK_REQUIRE(K % 8 == 0 && lda % 8 == 0 && a_cols % 8 == 0 && w_stride % 8 == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0,
@@ -356,7 +460,9 @@ TK_API int tk_grouped_gemm_bf16(const void* A, int lda, const int* a_row, const 
                 row_scale, scale_row, limit, alpha};
   if (tile_group) {
     TK_REQUIRE(!out_f32 && a_cols == 0 && c_cols == 0, "grouped_gemm: groups by tile write the storage type and have no columns of their own");
-    TK_REQUIRE(glu ? launch_staged<true>(a, tiles, stream) : launch_staged<false>(a, tiles, stream), "grouped_gemm: too many outputs");
+    TK_REQUIRE(!runs || (((uintptr_t)runs & 15) == 0 && K % TILE_K == 0 && a_rows * lda * 2 < (1l << 32) && (glu ? 2l : 1l) * N * K * 2 < (1l << 32) && max_singles > 0),
+               "grouped_gemm: pairs of tiles take whole steps of %d of K, and rows that 32-bit offsets reach", TILE_K);
+    TK_REQUIRE(glu ? launch_by_tile<true>(a, tiles, runs, max_singles, stream) : launch_by_tile<false>(a, tiles, runs, max_singles, stream), "grouped_gemm: too many outputs");
     TK_CHECK_LAUNCH("grouped_gemm");
     return 0;
   }
@@ -383,7 +489,8 @@ TK_API int tk_grouped_gemm_bf16(const void* A, int lda, const int* a_row, const 
 struct SortJob {
   const int* ids;
   int *slot_pair, *slot_token, *tile_group;
-  int pairs, top, experts, max_tiles;
+  TileRun* runs;  // (grouped_gemm_wide_kernel: room for the numbers, max_tiles / 2 pairs and max_singles single tiles)
+  int pairs, top, experts, max_tiles, max_singles;
 };
 #define SORT_JOBS 48
 struct SortJobs {
@@ -396,10 +503,14 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(SortJobs jobs) {
   int* __restrict__ slot_pair = jb.slot_pair;
   int* __restrict__ slot_token = jb.slot_token;
   int* __restrict__ tile_group = jb.tile_group;
-  extern __shared__ int sh[];  // [experts] counts, [experts] first slots, [experts] cursors
+  extern __shared__ int sh[];  // [experts] each: counts, first slots, cursors, first pairs of tiles, first single tiles
   int* count = sh;
   int* first = sh + experts;
   int* cursor = sh + 2 * experts;
+  int* first_pair = sh + 3 * experts;
+  int* first_single = sh + 4 * experts;
+  TileRun* run_of_pair = jb.runs + 1;
+  TileRun* run_of_single = run_of_pair + max_tiles / 2;
   for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = cursor[e] = 0;
   for (int s = threadIdx.x; s < max_tiles * tm; s += blockDim.x) slot_pair[s] = slot_token[s] = -1;
   for (int t = threadIdx.x; t < max_tiles; t += blockDim.x) tile_group[t] = -1;
@@ -410,16 +521,26 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(SortJobs jobs) {
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    int at = 0;
+    int at = 0, twos = 0, ones = 0;
     for (int e = 0; e < experts; ++e) {
+      const int n = (count[e] + tm - 1) / tm;
       first[e] = at;
-      at += (count[e] + tm - 1) / tm * tm;
+      first_pair[e] = twos;
+      first_single[e] = ones;
+      at += n * tm;
+      twos += n / 2;
+      ones += n & 1;
     }
     tile_group[max_tiles] = at / tm;
+    jb.runs[0] = {twos, ones, 0, 0};
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < experts; e += blockDim.x)
-    for (int t = first[e] / tm; t < (first[e] + count[e] + tm - 1) / tm; ++t) tile_group[t] = e;
+  for (int e = threadIdx.x; e < experts; e += blockDim.x) {
+    const int t0 = first[e] / tm, n = (count[e] + tm - 1) / tm;
+    for (int t = 0; t < n; ++t) tile_group[t0 + t] = e;
+    for (int p = 0; p < n / 2; ++p) run_of_pair[first_pair[e] + p] = {t0, e, first_pair[e], n / 2};
+    if (n & 1) run_of_single[first_single[e]] = {t0 + n - 1, e, first_single[e], 1};
+  }
   for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
     const int e = ids[p];
     if (e >= 0 && e < experts) {
@@ -438,14 +559,15 @@ TK_API int tk_expert_sort(const SortJob* jobs, int n_jobs, hipStream_t stream) {
     int most = 0;
     for (int k = 0; k < n; ++k) {
       const SortJob& j = all.job[k] = jobs[first + k];
-      TK_REQUIRE(j.ids && j.slot_pair && j.slot_token && j.tile_group && j.pairs >= 0 && j.top > 0 && j.experts > 0, "expert_sort: bad arguments");
+      TK_REQUIRE(j.ids && j.slot_pair && j.slot_token && j.tile_group && j.runs && j.pairs >= 0 && j.top > 0 && j.experts > 0, "expert_sort: bad arguments");
       // (each expert that has pairs leaves at most one tile partly empty)
       TK_REQUIRE(j.max_tiles >= (j.pairs + (long)(GS_M - 1) * min(j.experts, j.pairs)) / GS_M, "expert_sort: %d tiles cannot hold %d pairs of %d experts", j.max_tiles,
                  j.pairs, j.experts);
-      TK_REQUIRE(3 * j.experts * sizeof(int) <= 48 * 1024, "expert_sort: too many experts");
+      TK_REQUIRE(j.max_singles >= min(j.experts, j.max_tiles), "expert_sort: %d single tiles cannot hold those of %d experts", j.max_singles, j.experts);
+      TK_REQUIRE(5 * j.experts * sizeof(int) <= 80 * 1024, "expert_sort: too many experts");
       most = max(most, j.experts);
     }
-    hipLaunchKernelGGL(expert_sort_kernel, dim3(n), dim3(1024), 3 * most * sizeof(int), stream, all);
+    hipLaunchKernelGGL(expert_sort_kernel, dim3(n), dim3(1024), 5 * most * sizeof(int), stream, all);
     TK_CHECK_LAUNCH("expert_sort");
   }
   return 0;

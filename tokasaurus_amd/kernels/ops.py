@@ -2403,7 +2403,7 @@ def head_linear(x: torch.Tensor, w: torch.Tensor, out_f32: bool = False, positio
         # many rows: tiles of 32 rows on the matrix cores, the head as the tile's group
         tiles = -(-x.shape[0] // HEAD_TILE)
         call("tk_grouped_gemm_bf16", x.data_ptr(), x.stride(0), None, None, None, tiles, heads, n_in, n_out, w.data_ptr(),
-             n_out * n_in, y.data_ptr(), y.stride(0), n_out, n_in, x.shape[0], 0, 1 if out_f32 else 0, None, None, 0.0, 0.0,
+             n_out * n_in, y.data_ptr(), y.stride(0), n_out, n_in, x.shape[0], None, 0, 0, 0, 1 if out_f32 else 0, None, None, 0.0, 0.0,
              _stream())
         return y
     if freq is not None:
@@ -2489,7 +2489,8 @@ class _SortJob(ctypes.Structure):
     """One choice to be sorted by expert (struct SortJob of grouped_gemm.hip)."""
 
     _fields_ = [("ids", ctypes.c_void_p), ("slot_pair", ctypes.c_void_p), ("slot_token", ctypes.c_void_p), ("tile_group", ctypes.c_void_p),
-                ("pairs", ctypes.c_int), ("top", ctypes.c_int), ("experts", ctypes.c_int), ("max_tiles", ctypes.c_int)]
+                ("runs", ctypes.c_void_p), ("pairs", ctypes.c_int), ("top", ctypes.c_int), ("experts", ctypes.c_int), ("max_tiles", ctypes.c_int),
+                ("max_singles", ctypes.c_int)]
 
 
 @dataclass
@@ -2499,7 +2500,9 @@ class SortedPairs:
     slot_pair: torch.Tensor
     slot_token: torch.Tensor
     tile_group: torch.Tensor
+    runs: torch.Tensor  # two neighbouring tiles of an expert each, and the odd last ones
     max_tiles: int
+    max_singles: int
     shape: tuple  # of the ids
 
 
@@ -2517,10 +2520,12 @@ def expert_sort(choices: "list[tuple[torch.Tensor, int]]") -> "list[SortedPairs]
         n, top = ids.shape
         max_tiles = expert_tiles(n * top, int(experts))
         slots = max_tiles * EXPERT_TILE
-        book = torch.empty((2 * slots + max_tiles + 1,), dtype=torch.int32, device=ids.device)
-        s = SortedPairs(book[:slots], book[slots : 2 * slots], book[2 * slots :], max_tiles, (n, top))
-        job.ids, job.slot_pair, job.slot_token, job.tile_group = (t.data_ptr() for t in (ids, s.slot_pair, s.slot_token, s.tile_group))
-        job.pairs, job.top, job.experts, job.max_tiles = n * top, top, int(experts), max_tiles
+        singles, end = min(int(experts), max_tiles), 2 * slots + max_tiles + 1
+        at = -(-end // 4) * 4  # (a run is 16 bytes)
+        book = torch.empty((at + 4 * (1 + max_tiles // 2 + singles),), dtype=torch.int32, device=ids.device)
+        s = SortedPairs(book[:slots], book[slots : 2 * slots], book[2 * slots : end], book[at:], max_tiles, singles, (n, top))
+        job.ids, job.slot_pair, job.slot_token, job.tile_group, job.runs = (t.data_ptr() for t in (ids, s.slot_pair, s.slot_token, s.tile_group, s.runs))
+        job.pairs, job.top, job.experts, job.max_tiles, job.max_singles = n * top, top, int(experts), max_tiles, singles
         out.append(s)
     call("tk_expert_sort", ctypes.addressof(jobs), len(choices), _stream())
     return out
@@ -2532,6 +2537,20 @@ def experts_go_in_tiles(rows: int, top: int, dtype: torch.dtype, width: int, ff:
     pairs = rows * top
     many = pairs >= EXPERT_TILES_FROM_PAIRS and 4 * pairs >= 5 * experts
     return rows > GROUPED_FROM_ROWS and many and dtype == torch.bfloat16 and width % 8 == 0 and ff % 8 == 0
+
+
+# Rows an expert, on average, from which two neighbouring tiles of an expert are multiplied as one of 256 x 256: with fewer, too
+# many of the tiles are odd ones or nearly empty.  In us by single tiles / in pairs, both products and the sum: 32 experts of
+# 2,048 x 1,024, 256 rows an expert 227 / 201, 375 rows 268 / 260, 512 rows 360 / 298, 1,024 rows 659 / 517; 16 of 2,048 x 2,048, 256 rows
+# 211 / 215, 375 rows 274 / 233, 512 rows 360 / 273; 64 of 1,024 x 512, 256 rows 125 / 137, 512 rows 211 / 209; 128 of 2,048 x 768,
+# 187 rows 489 / 436, 256 rows 616 / 602, 512 rows 1,074 / 910.
+EXPERT_PAIRS_FROM_ROWS = 320
+
+
+def experts_go_in_pairs_of_tiles(pairs: int, experts: int, stride: int, width: int, ff: int) -> bool:
+    """Whether two neighbouring tiles of an expert's rows are multiplied as one."""
+    reach = 2 * max(pairs * max(stride, ff), 2 * ff * width) < 2 ** 32  # (the kernel's offsets are 32-bit bytes)
+    return pairs >= EXPERT_PAIRS_FROM_ROWS * experts and width % 64 == 0 and ff % 64 == 0 and reach
 
 
 def expert_mix(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor | None,
@@ -2573,14 +2592,15 @@ def expert_mix(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, i
             pairs = expert_sort([(ids, experts)])[0]
         _need(pairs.shape == (n, top), "expert_mix: pairs of another choice")
         slot_pair, slot_token, tile_group, max_tiles = pairs.slot_pair, pairs.slot_token, pairs.tile_group, pairs.max_tiles
-        slots = max_tiles * EXPERT_TILE
+        slots, singles = max_tiles * EXPERT_TILE, pairs.max_singles
+        wide = pairs.runs.data_ptr() if experts_go_in_pairs_of_tiles(n * top, experts, h.stride(0), width, ff) else None
         inter = torch.empty((n * top, ff), dtype=h.dtype, device=h.device)  # a row a pair: slots are many more where experts have few
         call("tk_grouped_gemm_bf16", h.data_ptr(), h.stride(0), slot_token.data_ptr(), slot_pair.data_ptr(), tile_group.data_ptr(), max_tiles, 0,
-             0, 0, w_gate_up.data_ptr(), 2 * ff * width, inter.data_ptr(), ff, ff, width, slots, 1, 0, on_input,
+             0, 0, w_gate_up.data_ptr(), 2 * ff * width, inter.data_ptr(), ff, ff, width, slots, wide, singles, n, 1, 0, on_input,
              slot_pair.data_ptr() if weights_on_input else None, limit, alpha, _stream())
         y = torch.empty((n * top, width), dtype=h.dtype, device=h.device)
         call("tk_grouped_gemm_bf16", inter.data_ptr(), ff, slot_pair.data_ptr(), slot_pair.data_ptr(), tile_group.data_ptr(), max_tiles, 0,
-             0, 0, w_down.data_ptr(), width * ff, y.data_ptr(), width, width, ff, slots, 0, 0, None, None, 0.0, 0.0, _stream())
+             0, 0, w_down.data_ptr(), width * ff, y.data_ptr(), width, width, ff, slots, wide, singles, n * top, 0, 0, None, None, 0.0, 0.0, _stream())
         call("tk_expert_sum", h.data_ptr(), h.stride(0), y.data_ptr(), ids.data_ptr(), weight_ptr,
              shared.data_ptr() if shared is not None else None, shared_gate.data_ptr() if shared is not None else None,
              out.data_ptr(), n, width, experts, top, unit, _stream())
