@@ -1,0 +1,60 @@
+"""Products of many rows in tiles: every tile, rows and outputs that end inside one, as many steps of K as local memory holds and
+fewer and more, rows a stride apart, the plain and the gated form, against sums in 64-bit."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from test_glu_stream_gpu import _case, _check, _silu
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape", range(5))
+@pytest.mark.parametrize("m", [1, 127, 200, 577])
+@pytest.mark.parametrize("n,k", [(8, 64), (136, 128), (72, 192), (520, 256), (1000, 320), (264, 448), (1288, 1024)])
+def test_against_64_bit_sums(shape, m, n, k):
+    from tokasaurus_amd.kernels import ops
+
+    x, w, _ = _case(m, n, k, 7 * m + n + k + shape)
+    wide = torch.zeros((m, k + 8), dtype=torch.bfloat16)  # rows apart
+    wide[:, :k] = x
+    rows = wide.cuda()[:, :k]
+    _check(ops.gemm_tiles_bf16(rows, w.cuda(), shape, glu=True), x.double(), w, _silu, k)
+    plain = ops.gemm_tiles_bf16(rows, w.cuda(), shape)
+    want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    # 32-bit sums of k products (k 2^-24 of their sizes), rounded once to bfloat16 (8 bits: 2^-8 of the value at most)
+    assert ((plain.cpu().double() - want).abs() <= want.abs() * 2.0 ** -8 + size * (k + 8) * 2.0 ** -23).all()
+
+
+@pytest.mark.parametrize("m,n,k,glu", [(65, 8192, 2048, True), (101, 8192, 2048, True), (1000, 2048, 1024, True), (1270, 3072, 512, False), (1800, 2048, 192, False)])
+def test_linear_takes_them(m, n, k, glu):
+    """The rule's tiles through the linear map, and its other products."""
+    from tokasaurus_amd.kernels import ops
+    from tokasaurus_amd.parts.linear import Linear
+
+    assert ops.tiles_choice(m, n, k, glu) >= 0 and ops.tiles_choice(m, n, k - 8, glu) == -1
+    x, w, gen = _case(m, n, k, m + n)
+    w = w if glu else w[:n]
+    lin = Linear(k, ["w"], [w.shape[0]])
+    lin.weight = w.cuda()
+    if glu:
+        return _check(lin(x.cuda(), swiglu=True), x.double(), w, _silu, k)
+    res = torch.randn((m, n), generator=gen).bfloat16()
+    prod = x.double() @ w.double().t()
+    want = prod + res.double()
+    got = lin(x.cuda(), residual=res.cuda()).cpu().double()
+    # the product rounded (2^-8 of it at most), then the sum; 32-bit sums of products of size 1 / sqrt(k), a few of them
+    assert ((got - want).abs() <= (want.abs() + 1.01 * prod.abs()) * 2.0 ** -8 + 1e-4).all()
+
+
+def test_refused():
+    from tokasaurus_amd.kernels import ops
+    from tokasaurus_amd.kernels.library import KernelError
+
+    x, w, _ = _case(200, 64, 128, 1)
+    for bad in (lambda: ops.gemm_tiles_bf16(x.cuda()[:, :96], w.cuda()[:, :96].contiguous(), 0),  # a step of K cut short
+                lambda: ops.gemm_tiles_bf16(x.cuda(), w.cuda(), 5), lambda: ops.gemm_tiles_bf16(x.cuda()[:, 4:68], w.cuda()[:, :64].contiguous(), 0)):
+        with pytest.raises(KernelError):
+            bad()

@@ -1,21 +1,25 @@
 // A tile of a bfloat16 matrix product through local memory, for products of many rows:  C[m, n] = sum_k A[m, k] W[n, k].
 //
-// A workgroup of 4 wavefronts owns 64 TM rows of A and 64 TN rows of W, a wavefront 32 TM x 32 TN of them on
-// v_mfma_f32_32x32x16_bf16 with W as the first operand.  What bounds it is the path from the L2 to a compute unit (about 35
-// bytes a clock, whatever the tile: 32 KB take 920 clocks for a tile of 128 x 128, whose products take 512), so a tile is as
-// large as the shape of the product lets it be and the sums stay in the accumulation registers (256 for 256 x 256: one
-// wavefront a SIMD).  Steps of 64 elements of K (128 bytes of a row, a whole cache line: steps of 32 elements in twice the
-// buffers took 10 to 30 % longer) go straight from memory to local memory; of W, which comes from memory, a step more is on
-// its way than of A, which the L2 holds (256 x 256: two steps of A and three of W are all of the 160 KB; with two of each a step
-// waits for its loads, 148 against 132 us for 2,048 x 2,048 x 8,192 rows from memory).  A wavefront is alone on its SIMD, so the order
-// within a step is written down: between a block's products (16 elements of K) come the reads of the next block's operands and
-// the loads of the steps ahead, a few at a time; one barrier a step, in front of its last block, when all of the step's operands
-// are in registers or on their way there.
+// A workgroup of 4 wavefronts owns 64 TM rows of A and 64 TN rows of W, a wavefront 32 TM x 32 TN of them.  Two things bound it.
+// The path from the L2 to a compute unit gives about 35 bytes a clock whatever the tile (32 KB take 920 clocks for a tile of
+// 128 x 128, whose products take 512), so a tile is as large as the shape of the product lets it be, and the sums stay in
+// registers (256 for 256 x 256: one wavefront a SIMD).  And with the whole chip at it, power: the clock falls to 1.6 GHz (2.1 on
+// operands of zeros), and what counts is the energy of an operation.  v_mfma_f32_16x16x32_bf16 reads and writes its sums half as
+// often as the 32 x 32 x 16 form: 4,096 x 4,096 x 14,336 rows 353 to 321 us (1.5 PFLOP/s), the same bits.
+//
+// Steps of 64 elements of K (128 bytes of a row, a whole cache line: steps of 32 elements in twice the buffers took 10 to 30 %
+// longer) go straight from memory to local memory; of W, which comes from memory, a step more is on its way than of A, which the
+// L2 holds (256 x 256: two steps of A and three of W are all of the 160 KB; with two of each a step waits for its loads, 148
+// against 132 us for 2,048 x 2,048 x 8,192).  A wavefront is alone on its SIMD, so the order within a step is written down: between a
+// block's products (32 elements of K) come the reads of the next block's operands and the loads of the steps ahead, a few at a
+// time (all at once behind the barrier: 2 to 8 % slower); one barrier a step, in front of its second block, when all of the step's
+// operands are in registers or on their way there.  Tiles of up to 128 x 256 ask for two wavefronts a SIMD (launch bounds) only
+// so that their sums are kept in the ordinary registers, where the compiler does not move them between the products.
 #pragma once
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 tile_bf16x8_t;
-typedef __attribute__((ext_vector_type(16))) float tile_f32x16_t;
+typedef __attribute__((ext_vector_type(4))) float tile_f32x4_t;
 
 #define TILE_K 64  // elements of K a step
 
@@ -39,15 +43,16 @@ __device__ __forceinline__ void tile_load(const void* base, unsigned off, unsign
 template <class S, bool GLU>
 struct TileLoop {
   static constexpr int TM = S::TM, TN = S::TN;
-  static constexpr int UNITS = TM * TN, READS = TM + TN;
+  static constexpr int XB = 2 * TM, WB = 2 * TN;  // blocks of 16 rows of A and of W that a wavefront owns
+  static constexpr int UNITS = XB * WB, READS = XB + WB;
   const char *a, *w;       // first bytes, in the rows of A and W, of the steps that are asked for next (uniform)
   unsigned off[S::LOADS];  // bytes from there to this lane's piece of every load: rows of A, then of W
   unsigned lds;
   int wave;
-  tile_f32x16_t acc[TN][TM];
-  const char *xl[4], *wl[4];  // a lane's first row in the first step's place, per 16 elements of K
+  tile_f32x4_t acc[WB][XB];
+  const char *xl[2], *wl[2];  // a lane's first row in the first step's place, per 32 elements of K
   struct Frag {
-    tile_bf16x8_t x[TM], w[TN];
+    tile_bf16x8_t x[XB], w[WB];
   };
   Frag f[2];
 
@@ -59,29 +64,29 @@ struct TileLoop {
       loads<N + 1, TO>(place);
     }
   }
-  // reads N .. of a block of 16 elements: w0, x0 .. , w1 ..
+  // reads N .. of a block of 32 elements: w0, x0 .. , w1 ..
   template <int N, int TO>
   __device__ __forceinline__ void reads(Frag& q, const char* xp, const char* wp) {
     if constexpr (N < TO) {
-      if constexpr (N >= 1 && N <= TM) {
-        q.x[N - 1] = *(const tile_bf16x8_t*)(xp + (N - 1) * 32 * S::ROW);
+      if constexpr (N >= 1 && N <= XB) {
+        q.x[N - 1] = *(const tile_bf16x8_t*)(xp + (N - 1) * 16 * S::ROW);
       } else {
-        constexpr int T = N == 0 ? 0 : N - TM;
-        constexpr int row = GLU ? (T < TN / 2 ? T * 32 : S::BN / 2 + (T - TN / 2) * 32) : T * 32;
+        constexpr int T = N == 0 ? 0 : N - XB;
+        constexpr int row = GLU && T >= TN ? S::BN / 2 + (T - TN) * 16 : T * 16;
         q.w[T] = *(const tile_bf16x8_t*)(wp + row * S::ROW);
       }
       reads<N + 1, TO>(q, xp, wp);
     }
   }
   static constexpr int reads_to(int u) {
-    const int n = u * READS * (UNITS < 16 ? 2 : 1) / UNITS;
+    const int n = u * READS * (UNITS < 64 ? 2 : 1) / UNITS;
     return n < READS ? n : READS;
   }
   // the products of a block; between them the reads of the next block and the loads FROM .. TO
   template <int U, bool READ, int FROM, int TO>
   __device__ __forceinline__ void units(const Frag& c, Frag& q, const char* xp, const char* wp, int place) {
     if constexpr (U < UNITS) {
-      acc[U / TM][U % TM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c.w[U / TM], c.x[U % TM], acc[U / TM][U % TM], 0, 0, 0);
+      acc[U / XB][U % XB] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c.w[U / XB], c.x[U % XB], acc[U / XB][U % XB], 0, 0, 0);
       if constexpr (READ) reads<reads_to(U), reads_to(U + 1)>(q, xp, wp);
       loads<FROM + U * (TO - FROM) / UNITS, FROM + (U + 1) * (TO - FROM) / UNITS>(place);
       __builtin_amdgcn_sched_barrier(0);
@@ -89,17 +94,11 @@ struct TileLoop {
     }
   }
   int a_here, a_next, w_last, w_here, w_next;  // places of a step, the next and the one before, in bytes
-  // loads that have been asked for before block b of a step: the rows of A behind the barrier, those of W in the blocks behind
-  // that (in one where they are needed at the next barrier)
-  static constexpr int W_BLOCKS = S::SA == 2 && S::SW == 2 ? 1 : 3;
-  static constexpr int wl_to(int b) { return b >= W_BLOCKS ? S::LOADS : S::LA + S::LW * b / W_BLOCKS; }
   // FW: the rest of the loads of the step whose rows of A were asked for last (W's), FA: the rows of A of the next such step
   template <bool FW, bool FA, bool LAST>
   __device__ __forceinline__ void step() {
     __builtin_amdgcn_sched_barrier(0);
-    units<0, true, FW ? wl_to(0) : 0, FW ? wl_to(1) : 0>(f[0], f[1], xl[1] + a_here, wl[1] + w_here, w_last);
-    units<0, true, FW ? wl_to(1) : 0, FW ? wl_to(2) : 0>(f[1], f[0], xl[2] + a_here, wl[2] + w_here, w_last);
-    units<0, true, FW ? wl_to(2) : 0, FW ? wl_to(3) : 0>(f[0], f[1], xl[3] + a_here, wl[3] + w_here, w_last);
+    units<0, true, FW ? S::LA : 0, FW ? S::LOADS : 0>(f[0], f[1], xl[1] + a_here, wl[1] + w_here, w_last);
     if constexpr (!LAST) {
       w += S::ROW;
       if constexpr (FW) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S::SA - 2) * S::LOADS + (S::SW - S::SA) * S::LW) : "memory");
@@ -114,19 +113,17 @@ struct TileLoop {
     w_next = w_next == (S::SW - 1) * S::W_STEP ? 0 : w_next + S::W_STEP;
   }
   __device__ __forceinline__ void run(char* smem, int steps, int wm, int wn, int lane) {
-    const int r = lane & 31, h = lane >> 5;
+    const int r = lane & 15, q = lane >> 4;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int place = ((2 * k + h) ^ tile_swizzle(r)) * 16;
+    for (int k = 0; k < 2; ++k) {
+      const int place = ((4 * k + q) ^ tile_swizzle(r)) * 16;
       xl[k] = smem + (wm * (32 * TM) + r) * S::ROW + place;
       wl[k] = smem + S::W_AT + (wn * (GLU ? 16 * TN : 32 * TN) + r) * S::ROW + place;
     }
 #pragma unroll
-    for (int t = 0; t < TN; ++t)
+    for (int t = 0; t < WB; ++t)
 #pragma unroll
-      for (int m = 0; m < TM; ++m)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) acc[t][m][j] = 0.f;
+      for (int m = 0; m < XB; ++m) acc[t][m] = tile_f32x4_t{0.f, 0.f, 0.f, 0.f};
     // asked for in front of the loop: SA steps of A and SW - 1 of W
 #pragma unroll
     for (int st = 0; st < S::SA; ++st) {
@@ -164,24 +161,21 @@ struct TileLoop {
   __device__ __forceinline__ void deliver(char* smem, int wm, int wn, int lane, int n0, int N, Value value, Dst dst) {
     constexpr int OUT = GLU ? S::BN / 2 : S::BN, PIECES = OUT / 8, MASK = PIECES % 16 == 0 ? 15 : 7;
     bf16_t* rows = (bf16_t*)smem;
-    const int r = lane & 31, h = lane >> 5;
+    const int r = lane & 15, q = lane >> 4;
     __syncthreads();
 #pragma unroll
-    for (int m = 0; m < TM; ++m) {
-      const int row = wm * (32 * TM) + m * 32 + r;
+    for (int m = 0; m < XB; ++m) {
+      const int row = wm * (32 * TM) + m * 16 + r;
 #pragma unroll
-      for (int t = 0; t < (GLU ? TN / 2 : TN); ++t) {
+      for (int t = 0; t < (GLU ? TN : WB); ++t) {
+        union { bf16_t v[4]; uint2 raw; } o;
 #pragma unroll
-        for (int j4 = 0; j4 < 4; ++j4) {  // a lane holds the outputs 8 j4 + 4 h + 0 .. 3 of a block of 32
-          union { bf16_t v[4]; uint2 raw; } o;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float y = GLU ? value(acc[t][m][4 * j4 + j], acc[t + (GLU ? TN / 2 : 0)][m][4 * j4 + j], m) : acc[t][m][4 * j4 + j];
-            o.v[j] = __float2bfloat16(y);
-          }
-          const int u = (wn * (GLU ? 16 * TN : 32 * TN) + t * 32) / 4 + 2 * j4 + h;  // of 4 outputs
-          *(uint2*)(rows + row * OUT + ((u >> 1) ^ (row & MASK)) * 8 + (u & 1) * 4) = o.raw;
+        for (int j = 0; j < 4; ++j) {  // a lane holds the outputs 4 q + 0 .. 3 of a block of 16
+          const float y = GLU ? value(acc[t][m][j], acc[t + (GLU ? TN : 0)][m][j], m) : acc[t][m][j];
+          o.v[j] = __float2bfloat16(y);
         }
+        const int u = (wn * (GLU ? 16 * TN : 32 * TN) + t * 16) / 4 + q;  // of 4 outputs
+        *(uint2*)(rows + row * OUT + ((u >> 1) ^ (row & MASK)) * 8 + (u & 1) * 4) = o.raw;
       }
     }
     __syncthreads();

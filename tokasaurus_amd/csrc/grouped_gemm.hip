@@ -12,7 +12,7 @@
 // first operand of the matrix core, read straight from memory 16 bytes a lane, the rows of A the second; a lane ends up with
 // 4 neighbouring outputs of one row.  The next step's operands are asked for before the current step's products.
 // Experts (grouped_gemm_staged_kernel): tiles of GS_M = 128 slots x 128 weight rows through local memory, however few slots a
-// tile holds (see there); experts of many rows take two such tiles as one of 256 x 256 (grouped_gemm_wide_kernel).  Sums are 32-bit and run over k in ascending steps for every output: a row's result does not
+// tile holds (see there); experts of many rows take two such tiles as one of 256 x 256 (grouped_gemm_pairs_kernel).  Sums are 32-bit and run over k in ascending steps for every output: a row's result does not
 // depend on which other rows share its tile.
 #include <math.h>
 
@@ -334,10 +334,11 @@ __global__ __launch_bounds__(256, 3) void grouped_gemm_staged_kernel(GroupedArgs
 // Experts of many rows: two neighbouring tiles of a group as one of 256 slots x 256 weight rows (in the gated form 128 of gate and
 // 128 of up), the odd last tile of a group 128 x 128 (gemm_tile.h).  The path from the L2 to a compute unit bounds these products,
 // and a tile of 256 x 256 asks for half as many bytes a product; pairs keep an expert's rows filled up to 128 and not to 256.
-// All pairs come before the first single tile, so that the short work fills what the last round of pairs leaves free.
-// 32 experts of 2,048 x 1,024, 2,048 tokens x 8: gate and up 206 to 182 us, down 114 to 93 (with 512 rows for every expert 158
-// and 79: the single tiles cost the rest); 64 x (1,024 x 512) 8,192 tokens x 4: 130 and 66.  With single tiles of 128 x 256 190 and
-// 96; every tile 128 x 256, without pairs, 185 and 105.
+// The single tiles have a launch of their own, whose sums fit the ordinary registers.
+// 32 experts of 2,048 x 1,024, 2,048 tokens x 8: gate and up 206 to 157 us for the pairs and 25 for the singles, down 114 to 78 and
+// 14 (with 512 rows for every expert 157 and 4.6, 78 and 4.6); 64 experts of 1,024 x 512, 8,192 tokens x 4: 107 and 30, 56 and 16.
+// Every tile 128 x 256, without pairs, took 185 and 105.  What is left is the weights' way from memory: the pairs' products of one
+// weight of 16,384 x 2,048 for 2,048 rows, as many of them, take 120 us.
 template <class S, bool GLU>
 __device__ __forceinline__ void wide_tile(const GroupedArgs& a, char* smem, int g, int first, int n0) {
   constexpr int OUT = GLU ? S::BN / 2 : S::BN;
@@ -351,7 +352,7 @@ __device__ __forceinline__ void wide_tile(const GroupedArgs& a, char* smem, int 
   t.w = (const char*)(a.W + (size_t)g * a.w_stride + (size_t)n0 * a.K);
   // (all numbers of rows are asked for before the first is used)
   const int lr = lane >> 3;
-  int from[S::LA], frow[S::TM], to = -1;
+  int from[S::LA], frow[2 * S::TM], to = -1;
 #pragma unroll
   for (int i = 0; i < S::LA; ++i) {
     const int slot = min(first + wave * (16 * S::TM) + i * 8 + lr, top);
@@ -362,14 +363,14 @@ __device__ __forceinline__ void wide_tile(const GroupedArgs& a, char* smem, int 
     to = a.c_row ? a.c_row[own] : own;
     if (a.a_row && a.a_row[own] < 0) to = -1;
   }
-  float factor[S::TM];
+  float factor[2 * S::TM];
 #pragma unroll
-  for (int m = 0; m < S::TM; ++m) factor[m] = 1.f;
+  for (int m = 0; m < 2 * S::TM; ++m) factor[m] = 1.f;
   if (GLU && a.row_scale) {
 #pragma unroll
-    for (int m = 0; m < S::TM; ++m) frow[m] = a.scale_row[min(first + wm * (32 * S::TM) + m * 32 + (lane & 31), top)];  // (< 0: an empty slot)
+    for (int m = 0; m < 2 * S::TM; ++m) frow[m] = a.scale_row[min(first + wm * (32 * S::TM) + m * 16 + (lane & 15), top)];  // (< 0: an empty slot)
 #pragma unroll
-    for (int m = 0; m < S::TM; ++m) factor[m] = a.row_scale[max(frow[m], 0)];
+    for (int m = 0; m < 2 * S::TM; ++m) factor[m] = a.row_scale[max(frow[m], 0)];
   }
 #pragma unroll
   for (int i = 0; i < S::LA; ++i)
@@ -400,28 +401,27 @@ struct TileRun {
 };
 // runs: the numbers of pairs and of single tiles (as TileRun's first two), the pairs, the single tiles
 template <bool GLU>
-__global__ __launch_bounds__(256, 1) void grouped_gemm_wide_kernel(GroupedArgs a, const TileRun* __restrict__ runs, int max_pairs, int n_blocks,
-                                                                   int single_blocks) {
+__global__ __launch_bounds__(256, 1) void grouped_gemm_pairs_kernel(GroupedArgs a, const TileRun* __restrict__ runs, int n_blocks) {
   extern __shared__ __align__(16) char smem[];
-  const int pairs = runs->tile, singles = runs->group;
-  int seq = blockIdx.x / GS_DIES;
-  const int per = (pairs * n_blocks + GS_DIES - 1) / GS_DIES;
-  if (seq < per) {
-    const int item = blockIdx.x % GS_DIES * per + seq;
-    if (item >= pairs * n_blocks) return;
-    const int some = item / n_blocks;
-    const TileRun r = runs[1 + some];
-    // the chunk of up to WIDE_PAIRS pairs of the group that the item lies in
-    const int chunk = r.first + (some - r.first) / WIDE_PAIRS * WIDE_PAIRS, len = min(WIDE_PAIRS, r.first + r.count - chunk);
-    const int off = item - chunk * n_blocks, pair = chunk + off % len;
-    wide_tile<PairShape, GLU>(a, smem, r.group, (r.tile + 2 * (pair - r.first)) * GS_M, off / len * WIDE_OUT(GLU));
-    return;
-  }
-  seq -= per;
-  const int per1 = (singles * single_blocks + GS_DIES - 1) / GS_DIES, item = blockIdx.x % GS_DIES * per1 + seq;
-  if (seq >= per1 || item >= singles * single_blocks) return;
-  const TileRun r = runs[1 + max_pairs + item / single_blocks];
-  wide_tile<SingleShape, GLU>(a, smem, r.group, r.tile * GS_M, item % single_blocks * (WIDE_OUT(GLU) / 2));
+  const int items = runs->tile * n_blocks, per = (items + GS_DIES - 1) / GS_DIES;
+  const int seq = blockIdx.x / GS_DIES, item = blockIdx.x % GS_DIES * per + seq;
+  if (seq >= per || item >= items) return;
+  const int some = item / n_blocks;
+  const TileRun r = runs[1 + some];
+  // the chunk of up to WIDE_PAIRS pairs of the group that the item lies in
+  const int chunk = r.first + (some - r.first) / WIDE_PAIRS * WIDE_PAIRS, len = min(WIDE_PAIRS, r.first + r.count - chunk);
+  const int off = item - chunk * n_blocks, pair = chunk + off % len;
+  wide_tile<PairShape, GLU>(a, smem, r.group, (r.tile + 2 * (pair - r.first)) * GS_M, off / len * WIDE_OUT(GLU));
+}
+
+template <bool GLU>
+__global__ __launch_bounds__(256, 2) void grouped_gemm_singles_kernel(GroupedArgs a, const TileRun* __restrict__ runs, int max_pairs, int n_blocks) {
+  extern __shared__ __align__(16) char smem[];
+  const int items = runs->group * n_blocks, per = (items + GS_DIES - 1) / GS_DIES;
+  const int seq = blockIdx.x / GS_DIES, item = blockIdx.x % GS_DIES * per + seq;
+  if (seq >= per || item >= items) return;
+  const TileRun r = runs[1 + max_pairs + item / n_blocks];
+  wide_tile<SingleShape, GLU>(a, smem, r.group, r.tile * GS_M, item % n_blocks * (WIDE_OUT(GLU) / 2));
 }
 
 template <bool GLU>
@@ -430,12 +430,16 @@ static bool launch_by_tile(const GroupedArgs& a, int tiles, const TileRun* runs,
   const int outs = GLU ? 64 : 128, n_blocks = (a.N + outs - 1) / outs;
   if (runs) {
     const int max_pairs = tiles / 2, wide_blocks = (a.N + WIDE_OUT(GLU) - 1) / WIDE_OUT(GLU);
-    const long grid = groups((long)max_pairs * wide_blocks) + groups((long)max_singles * n_blocks);
-    constexpr int lds = PairShape::LDS;
-    static_assert(lds >= SingleShape::LDS && SingleShape::BM == GS_M && PairShape::BM == 2 * GS_M, "");
-    auto kernel = grouped_gemm_wide_kernel<GLU>;
-    if (grid >= (1l << 31) || hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return false;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), lds, stream, a, runs, max_pairs, wide_blocks, n_blocks);
+    const long pairs = groups((long)max_pairs * wide_blocks), singles = groups((long)max_singles * n_blocks);
+    static_assert(SingleShape::BM == GS_M && PairShape::BM == 2 * GS_M, "");
+    auto pair_kernel = grouped_gemm_pairs_kernel<GLU>;
+    auto single_kernel = grouped_gemm_singles_kernel<GLU>;
+    if (pairs + singles >= (1l << 31)
+        || hipFuncSetAttribute((const void*)pair_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PairShape::LDS) != hipSuccess
+        || hipFuncSetAttribute((const void*)single_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, SingleShape::LDS) != hipSuccess)
+      return false;
+    if (pairs > 0) hipLaunchKernelGGL(pair_kernel, dim3((unsigned)pairs), dim3(256), PairShape::LDS, stream, a, runs, wide_blocks);
+    hipLaunchKernelGGL(single_kernel, dim3((unsigned)singles), dim3(256), SingleShape::LDS, stream, a, runs, max_pairs, n_blocks);
     return true;
   }
   const long grid = groups((long)tiles * n_blocks);
@@ -489,7 +493,7 @@ TK_API int tk_grouped_gemm_bf16(const void* A, int lda, const int* a_row, const 
 struct SortJob {
   const int* ids;
   int *slot_pair, *slot_token, *tile_group;
-  TileRun* runs;  // (grouped_gemm_wide_kernel: room for the numbers, max_tiles / 2 pairs and max_singles single tiles)
+  TileRun* runs;  // (grouped_gemm_pairs_kernel: room for the numbers, max_tiles / 2 pairs and max_singles single tiles)
   int pairs, top, experts, max_tiles, max_singles;
 };
 #define SORT_JOBS 48

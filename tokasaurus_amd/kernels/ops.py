@@ -1246,6 +1246,60 @@ def gemm_library_bf16(x: torch.Tensor, w: torch.Tensor, out_f32: bool = False, o
     return out
 
 
+# The tiles of gemm_tiles.hip: rows of A, rows of W, and the us that a step of 64 elements of K takes and that a tile's beginning and end
+# add (fitted to 234 products of 13 weights at 129 to 8,192 rows, weights from memory; the tile that comes out fastest by them is the
+# fastest measured one in 218)
+TILE_SHAPES = ((128, 128, 0.47, 4.3), (192, 128, 0.54, 6.5), (128, 256, 0.79, 5.5), (192, 256, 0.96, 11.2), (256, 256, 1.19, 15.5))
+GLU_TILES_FROM_ROWS = 65  # (up to 64 rows gate and up stream through local memory)
+# two rounds of tiles of 256 x 256: with more the chip's power bounds the step, and the library's kernel needs less of it (a prompt of
+# 2,048 tokens of the 1B shape 5,027 to 4,984 us with the tiles, four of 1,024 of the 8B shape 43.3 to 44.6 ms)
+GLU_TILES_MOST_SUMS = 2 * 256 * 256 * 256
+
+
+@functools.lru_cache(maxsize=4096)
+def tiles_choice(m: int, n: int, k: int, glu: bool = False) -> int:
+    """Which tile (of ``TILE_SHAPES``) a product of ``m`` rows and ``n`` outputs takes, or with ``glu`` of ``n`` of gate and as many of up;
+    -1: the library's product is faster.
+
+    In the gated form the tiles save the pass behind the library's product; they pay where they fill four fifths of the compute
+    units' rounds, up to ``GLU_TILES_MOST_SUMS``.  us library and pass / tiles, weights from memory: 16,384 x 2,048 33.5 / 26.4 at 256 rows, 41.7 / 37.7 at 512, 70.1 /
+    61.3 at 1,024, 98.7 / 94.9 at 1,500, 117 / 120 at 2,048; 16,384 x 3,072 45.1 / 37.8 at 256, 92.0 / 81.6 at 1,024, 172 / 165 at 2,048;
+    28,672 x 4,096 105 / 102 at 512, 204 / 194 at 1,024 (fill 0.73: 262 / 279 at 1,280).
+    A plain product in tiles is ahead of the library's where one round of tiles of 128 outputs fills the chip and the library's
+    larger tiles do not: 3,072 x 8,192 71.8 / 65.0 at 1,280 rows, 90.4 / 78.9 at 1,792; 5,120 x 3,072 40.1 / 35.2 at 1,024; 4,096 x 4,096
+    47.4 / 43.9 at 1,280; not where a tile of 128 x 128 leaves more than a sixth of it idle (2,048 x 8,192 55.6 / 62.0 at 1,500
+    rows, fill 0.75; 4,096 x 4,096 33.3 / 38.5 at 768), tiles of 192 rows a quarter (3,072 x 8,192 85.3 / 76.8 at 1,500, fill 0.75); tiles of
+    128 x 256 only pay over a long inner size (4,096 x 14,336 203 / 187 at 2,048 rows, 4,096 x 4,096 58.3 / 58.6), larger ones
+    not (2,048 x 8,192 171 / 184 at 8,192 rows)."""
+    if k % 64 or n % 8 or (256 + 2 * n if glu else 256) * k >= 2 ** 31:
+        return -1
+    best, shape, fill, rounds = math.inf, 0, 0.0, 0
+    for i, (rows, cols, step, ends) in enumerate(TILE_SHAPES):
+        tiles = -(-m // rows) * -(-(2 * n if glu else n) // cols)
+        turns = -(-tiles // 256)
+        cost = turns * (step * (k // 64) + ends)
+        if cost < best:
+            best, shape, fill, rounds = cost, i, tiles / (256 * turns), turns
+    if glu:
+        return shape if m >= GLU_TILES_FROM_ROWS and (fill >= 0.8 or m <= 128 and fill >= 0.5) and m * 2 * n <= GLU_TILES_MOST_SUMS else -1
+    least = (0.84, 0.75, 0.84 if k >= 8192 else 2.0, 2.0, 2.0)[shape]
+    return shape if rounds == 1 and fill >= least else -1
+
+
+def gemm_tiles_bf16(x: torch.Tensor, w: torch.Tensor, shape: int, glu: bool = False) -> torch.Tensor:
+    """x [M, K] . w [N, K]^T in bfloat16 in tiles of ``TILE_SHAPES[shape]``; ``glu``: w is [gate | up], silu(gate) * up.  Rows of x and w
+    start at multiples of 16 bytes."""
+    _gpu(x, w)
+    if not (x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.dtype == w.dtype == torch.bfloat16 and x.stride(1) == 1
+            and w.is_contiguous() and (not glu or w.shape[0] % 2 == 0)):
+        raise KernelError(f"gemm_tiles: x {tuple(x.shape)} {x.dtype} and w {tuple(w.shape)} {w.dtype} must be bfloat16 [M, K] and [N, K] of contiguous rows")
+    m, k = x.shape
+    n = w.shape[0] // 2 if glu else w.shape[0]
+    out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    call("tk_gemm_tiles_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), n, m, n, k, 1 if glu else 0, shape, _stream())
+    return out
+
+
 # --------------------------------------------------------------------------
 # a recorded step's traffic with the host
 # --------------------------------------------------------------------------

@@ -11,7 +11,8 @@ Which kernel runs is decided by the storage type and the number of rows:
     up): the hand-written matrix-core kernels that stream the weight once and fuses the epilogue; it can also fold in the
     norm in front (``Normed`` input), leave what the norm behind it needs
     (``emit_norm``), and rotate and append q, k and v (``rope_append``);
-  * bfloat16, more rows (large decode batches, prefill): the library's matrix product,
+  * bfloat16, more rows (large decode batches, prefill): tiles of up to 256 x 256 where they are ahead
+    (``ops.tiles_choice``; gate and up with the activation in the same kernel), else the library's matrix product,
     as in the reference (its projections are library calls), followed by the epilogue
     kernel; a bfloat16 weight whose inner size is no multiple of 8 takes the plain
     kernel for few rows.
@@ -141,9 +142,15 @@ class Linear:
                                             prenorm=prenorm, norm_eps=eps, out=out, bias=bias, glu=glu if swiglu else None,
                                             out_scale=out_scale,
                                             staged=2 if swiglu and ops.glu_streams(m, self.total_out // 2, self.in_features) else -1)
+            # many rows: in tiles where these are ahead of the library's product (the gated form with silu in one kernel)
+            direct = ops.gemm_library_direct(x, w)
+            if direct and bias is None and not out_f32 and (glu is None or not swiglu):
+                shape = ops.tiles_choice(m, w.shape[0] // 2 if swiglu else w.shape[0], self.in_features, swiglu)
+                if shape >= 0:
+                    prod = ops.gemm_tiles_bf16(x, w, shape, swiglu)
+                    return ops.add(prod, residual.contiguous()) if residual is not None else prod
             # library matrix product (hipBLASLt), 32-bit accumulation; with a bias through the tensor
             # library, whose call adds it to the 32-bit sums in the product's own epilogue (addmm)
-            direct = ops.gemm_library_direct(x, w)
             if out_f32:
                 if direct:
                     prod = ops.gemm_library_bf16(x, w, out_f32=True, out=out)
