@@ -37,6 +37,18 @@ def test_sizes(m, nk):
     check(ops.gemm_generic(a, w, residual=residual, bias=bias), a, w, bias, residual)
 
 
+@pytest.mark.parametrize("m", [1, 7, 8, 9])
+@pytest.mark.parametrize("nk", [(1, 256), (8, 288), (20, 4096), (2047, 320), (2048, 2080), (2049, 256)])
+def test_few_rows_by_halves_of_k(m, nk):
+    """Weights of few enough rows for 8 a workgroup: K's second half beside the first, with blocks left over in each, and the sizes around."""
+    n, k = nk
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, w = torch.randn((m, k + 4), generator=g, device="cuda")[:, 4:], torch.randn((n, k), generator=g, device="cuda")
+    bias, residual = torch.randn((n,), generator=g, device="cuda"), torch.randn((m, n + 3), generator=g, device="cuda")[:, 1 : n + 1]
+    check(ops.gemm_generic(a, w), a, w)
+    check(ops.gemm_generic(a, w, residual=residual, bias=bias), a, w, bias, residual)
+
+
 def test_large_tiles():
     g = torch.Generator(device="cuda").manual_seed(5)
     a = torch.randn((2100, 100), generator=g, device="cuda")

@@ -19,8 +19,8 @@
 //     themselves need 32 and reach half of the matrix cores' rate (2 048 x 16 384 x 2 048: 76 TFLOP/s, straight from
 //     memory or through local memory of their own); a shared tile of 64 x 64 needs 16, of 128 x 128 8.  Where the tiles are
 //     too few to fill the chip K is cut among workgroups, whose sums a second kernel adds in the order of K.
-// Measured against the plain kernels that this replaces (us; floors at 5.05 TB/s and 153 TFLOP/s): 4 tokens 2 048 x 2 048 8.4
-// (floor 3.3), 2 048 x 8 192 28 (13), 16 384 x 2 048 29.5 (27); before 36 for the first two in the mean, and 33.  301
+// Measured against the plain kernels that this replaces (us; floors at 5.05 TB/s and 153 TFLOP/s): 4 tokens 2 048 x 2 048 6.9
+// (floor 3.3), 2 048 x 8 192 17.5 (13), 16 384 x 2 048 29.5 (27); before 36 for the first two in the mean, and 33.  301
 // tokens 2 048 x 2 048 38 (17), 2 048 x 8 192 116 (66), 3 072 x 2 048 53 (25), 16 384 x 2 048 207 (132); before 746 for
 // the first two in the mean, 301 and 643.  2 048 tokens 16 384 x 2 048 1 115 (898, 123 TFLOP/s).  Errors against 64-bit
 // sums: up to 32 tokens those of the plain kernel (1.2e-7 of the norm at 2 048 elements), beyond at most the plain kernel's.
@@ -62,18 +62,27 @@ __device__ __forceinline__ void gf_store(const GemmF32Args& a, f4 v, int token, 
   }
 }
 
+#define GF_HALVES_ROWS 2048  // weight rows up to which the few-row kernel takes 8 a workgroup: one for each of 256 compute units
 #define GF_UNROLL 4  // blocks of 16 elements a set of loads
 
+// HALVES (up to 8 tokens, K a multiple of 32): a workgroup has 8 weight rows, and the unused half of the matrix core's rows and of its
+// columns takes the second half of K (the blocks of results off the diagonal are not used), so that a weight of few rows gives
+// every compute unit a workgroup.  4 tokens, us by rows of 16 / of 8, weights from memory: 2,048 x 2,048 8.6 / 6.9, 2,048 x 8,192 26.4 / 17.5
+// (3.8 TB/s), 3,072 x 2,048 8.8 / 9.6, 16,384 x 2,048 26.8 / 31.2.  Each chain of sums is half as long: error 1.2e-7 / 1.0e-7 of the norm
+// over 2,048 elements, 1.6e-7 / 1.3e-7 over 8,192.
+template <bool HALVES>
 __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a) {
   extern __shared__ __align__(16) f4 sums[];  // [wavefronts - 1][64]
   // (the wavefront's number as one value for all its lanes, so that its loop counts in scalar registers)
   const int lane = threadIdx.x & 63, kw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), KS = blockDim.x >> 6;
   const int r = lane & 15, q = lane >> 4;
-  const int n0 = blockIdx.x * 16;
-  const int blocks = (a.K + 15) >> 4;
+  constexpr int ROWS = HALVES ? 8 : 16;
+  const int n0 = blockIdx.x * ROWS, own = HALVES ? r & 7 : r;
+  const size_t from = HALVES ? (size_t)(r >> 3) * (a.K / 2) : 0;  // of K
+  const int blocks = HALVES ? a.K >> 5 : (a.K + 15) >> 4;
   const int b0 = (int)((long)blocks * kw / KS), b1 = (int)((long)blocks * (kw + 1) / KS);
-  const float* wp = a.W + (size_t)min(n0 + r, a.N - 1) * a.K + 4 * q;
-  const float* ap = a.A + (size_t)min(r, a.M - 1) * a.lda + 4 * q;
+  const float* wp = a.W + (size_t)min(n0 + own, a.N - 1) * a.K + from + 4 * q;
+  const float* ap = a.A + (size_t)min(own, a.M - 1) * a.lda + from + 4 * q;
   f4 acc[GF_UNROLL][4];
 #pragma unroll
   for (int u = 0; u < GF_UNROLL; ++u)
@@ -92,7 +101,7 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a) {
 #define GF_MULTIPLY(set)                                                                            \
   _Pragma("unroll") for (int u = 0; u < GF_UNROLL; ++u) _Pragma("unroll") for (int s = 0; s < 4; ++s) \
       acc[u][s] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[set][u][s], x[set][u][s], acc[u][s], 0, 0, 0)
-  const int exact = (a.K & 15) == 0 ? b1 : min(b1, blocks - 1);  // blocks up to here lie inside K whole
+  const int exact = HALVES || (a.K & 15) == 0 ? b1 : min(b1, blocks - 1);  // blocks up to here lie inside K whole
   const int sets = max(exact - b0, 0) / GF_UNROLL;
   int b = b0;
   if (sets > 0) {
@@ -119,7 +128,7 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a) {
 #undef GF_MULTIPLY
 #pragma unroll 1
   for (; b < b1; ++b) {  // what is left, the last block perhaps cut by K: zeros behind it
-    const bool in = b * 16 + 4 * q < a.K;
+    const bool in = HALVES || b * 16 + 4 * q < a.K;
     const long off = in ? (long)b * 16 : -4L * q;
     f4 wv = *(const f4*)(wp + off), xv = *(const f4*)(ap + off);
     if (!in) wv = xv = (f4){0.f, 0.f, 0.f, 0.f};
@@ -136,7 +145,11 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a) {
     if (kw > 0) return;
     for (int k = 0; k < KS - 1; ++k) sum += sums[k * 64 + lane];
   }
-  if (r < a.M && n0 + 4 * q < a.N) gf_store(a, sum, r, n0 + 4 * q);
+  if (HALVES) {  // the second half's sums of token r lie in the lanes of token r + 8 and of rows 8 more
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sum[j] += __shfl(sum[j], (lane + 40) & 63, 64);
+  }
+  if (r < min(a.M, ROWS) && 4 * q < ROWS && n0 + 4 * q < a.N) gf_store(a, sum, r, n0 + 4 * q);
 }
 
 #define GS_ROW 36  // floats a row of 32 takes in local memory: 16 lanes that read 16 rows at one place meet 64 different banks
@@ -307,7 +320,11 @@ TK_API int tk_gemm_f32(const void* A, int lda, const void* W, void* C, int ldc, 
   if (M <= 16) {
     // (2, 4, 8 wavefronts at 4 tokens, 2 048 x 2 048: 9.0, 8.2, 9.0 us, 2 048 x 8 192: 34, 25, 26, 16 384 x 2 048: 33, 30, 30)
     const int KS = K < 64 ? 1 : (K < 4096 ? 4 : 8);
-    hipLaunchKernelGGL(gemm_f32_few_kernel, dim3((N + 15) / 16), dim3(64 * KS), (KS - 1) * 64 * sizeof(f4), stream, a);
+    // rows of 8 where rows of 16 leave compute units without a workgroup
+    if (M <= 8 && K % 32 == 0 && K >= 256 && N <= GF_HALVES_ROWS)
+      hipLaunchKernelGGL(gemm_f32_few_kernel<true>, dim3((N + 7) / 8), dim3(64 * KS), (KS - 1) * 64 * sizeof(f4), stream, a);
+    else
+      hipLaunchKernelGGL(gemm_f32_few_kernel<false>, dim3((N + 15) / 16), dim3(64 * KS), (KS - 1) * 64 * sizeof(f4), stream, a);
     TK_CHECK_LAUNCH("gemm_f32");
     return 0;
   }
