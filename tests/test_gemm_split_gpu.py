@@ -73,6 +73,27 @@ def test_rotation_and_append(nq, nkv, d, page, tables):
     assert pages[0][0].count_nonzero() > 0
 
 
+def test_product_and_pass_in_one_call():
+    """The bits of the two calls, and what they refuse is refused."""
+    x, w, gen = _case(33, 256, 192, 5)
+    residual, weight = torch.randn((33, 256), generator=gen, device="cuda").bfloat16(), torch.randn((256,), generator=gen, device="cuda")
+    for got, want in zip(ops.split_linear_add_rmsnorm(x, w, residual, weight, 1e-5), ops.split_add_rmsnorm(ops.gemm_split(x, w), residual, weight, 1e-5)):
+        assert torch.equal(got, want)
+    positions, table = torch.arange(33, device="cuda", dtype=torch.int32), torch.randperm(3, generator=gen, device="cuda").to(torch.int32).view(1, 3)
+    cos, sin = ops.rope_table(1.0 / 10000 ** (torch.arange(0, 32, 2, device="cuda").float() / 32), 48)
+    pages = [[torch.zeros(shape(3, 2, 16, 32), dtype=torch.bfloat16, device="cuda") for shape in (ops.key_pages_shape, ops.value_pages_shape)] for _ in range(2)]
+    rope = [ops.RopeAppend(positions, torch.zeros_like(positions), table, cos, sin, *p, 4, 2, 32, 16) for p in pages]
+    assert torch.equal(ops.split_linear_rope_append(x, w, rope[0]), ops.split_rope_append(ops.gemm_split(x, w), rope[1]))
+    assert torch.equal(pages[0][0], pages[1][0]) and torch.equal(pages[0][1], pages[1][1])
+    for bad in ((x[:, :96], w[:, :96].contiguous(), residual, weight), (x, w[:60], residual, weight), (x, w, residual[:30], weight),
+                (x, w, residual, weight[:100]), (x, w, residual.float(), weight), (x[:, 1:65], w[:, :64].contiguous(), residual, weight)):
+        with pytest.raises(ops.KernelError):
+            ops.split_linear_add_rmsnorm(*bad, 1e-5)
+    rope[0].positions = positions[:30]
+    with pytest.raises(ops.KernelError):
+        ops.split_linear_rope_append(x, w, rope[0])
+
+
 def test_what_is_refused():
     x, w, _ = _case(4, 64, 128, 1)
     for bad in ((x[:, :96], w[:, :96].contiguous()), (x, w[:60]), (torch.cat([x] * 33), w), (x.float(), w.float()), (x[:, 1:65], w[:, :64].contiguous())):

@@ -308,3 +308,23 @@ TK_API int tk_split_rope_append(const float* part, int cuts, void* q, const int*
   TK_CHECK_LAUNCH("split_rope_append");
   return 0;
 }
+
+// ---------------------------------------------------------------------------------
+// A product and the pass behind it in one call of the host, which in steps of few tokens is what bounds them: a call from Python
+// with its checks and its launch takes 8 us or more, a launch from here 2.
+// ---------------------------------------------------------------------------------
+
+TK_API int tk_split_linear_add_rmsnorm(const void* A, int lda, const void* W, float* part, int M, int N, int K, int cuts, const void* residual,
+                                       const void* w, int w_f32, void* stream_out, void* out, float eps, hipStream_t stream) {
+  const int rc = tk_gemm_split_bf16(A, lda, W, part, M, N, K, cuts, stream);
+  return rc ? rc : tk_split_add_rmsnorm(part, cuts, residual, w, w_f32, stream_out, out, M, N, eps, stream);
+}
+
+TK_API int tk_split_linear_rope_append(const void* A, int lda, const void* W, float* part, int M, int K, int cuts, void* q, const int* positions,
+                                       const int* token_req, const int* block_table, int table_stride, const float* cos_t,
+                                       const float* sin_t, void* kcache, void* vcache, int nq, int nkv, int d, int P, hipStream_t stream) {
+  const int rc = tk_gemm_split_bf16(A, lda, W, part, M, (nq + 2 * nkv) * d, K, cuts, stream);
+  return rc ? rc
+            : tk_split_rope_append(part, cuts, q, positions, token_req, block_table, table_stride, cos_t, sin_t, kcache, vcache, M, nq, nkv, d, P,
+                                   stream);
+}

@@ -1192,6 +1192,55 @@ def split_rope_append(part: torch.Tensor, r: RopeAppend) -> torch.Tensor:
     return q
 
 
+# The same, a product and the pass behind it in one call: in steps of few tokens the host's calls are what takes the time (a prompt of
+# 101 tokens of the 1B shape, 45 such pairs among its 130 launches: 1,800 us with two calls each, 1,683 with one).
+
+
+def split_linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float) -> tuple[torch.Tensor, torch.Tensor]:
+    """``split_add_rmsnorm(gemm_split(x, w), residual, weight, eps)``."""
+    m, k = x.shape
+    n = w.shape[0]
+    dtype = weight.dtype
+    if not (x.is_cuda and residual.is_cuda and weight.is_cuda and w.is_contiguous() and w.shape[1] == k and split_takes(x, w)
+            and residual.shape == (m, n) and residual.dtype == torch.bfloat16 and residual.is_contiguous()
+            and weight.shape == (n,) and weight.is_contiguous() and (dtype == torch.bfloat16 or dtype == torch.float32)):
+        raise KernelError(f"split_linear_add_rmsnorm: x {tuple(x.shape)} {x.dtype}, w {tuple(w.shape)} {w.dtype}, residual {tuple(residual.shape)} "
+                          f"{residual.dtype} and norm weight {tuple(weight.shape)} {dtype} do not go together, or not on the GPU")
+    cuts = split_cuts(n, k)
+    part = torch.empty((cuts, m, n), dtype=torch.float32, device=x.device)
+    stream_out, out = torch.empty_like(residual), torch.empty_like(residual)
+    call("tk_split_linear_add_rmsnorm", x.data_ptr(), x.stride(0), w.data_ptr(), part.data_ptr(), m, n, k, cuts, residual.data_ptr(),
+         weight.data_ptr(), 1 if dtype == torch.float32 else 0, stream_out.data_ptr(), out.data_ptr(), eps, _stream())
+    return stream_out, out
+
+
+def split_linear_rope_append(x: torch.Tensor, w: torch.Tensor, r: RopeAppend) -> torch.Tensor:
+    """``split_rope_append(gemm_split(x, w), r)``."""
+    m, k = x.shape
+    n, half = w.shape[0], r.head_dim // 2
+    i32 = torch.int32
+    if not (x.is_cuda and w.is_contiguous() and w.shape[1] == k and split_takes(x, w) and n == (r.nq + 2 * r.nkv) * r.head_dim
+            and (r.rotary_dim is None or r.rotary_dim == r.head_dim)
+            and r.positions.dtype == r.token_req.dtype == r.block_table.dtype == i32 and r.positions.numel() == r.token_req.numel() == m
+            and r.positions.is_contiguous() and r.token_req.is_contiguous() and r.block_table.is_contiguous() and r.block_table.dim() == 2
+            and r.positions.is_cuda and r.token_req.is_cuda and r.block_table.is_cuda and r.kcache.is_cuda and r.vcache.is_cuda):
+        raise KernelError(f"split_linear_rope_append: x {tuple(x.shape)} {x.dtype}, w {tuple(w.shape)} {w.dtype} and the tokens' arrays "
+                          f"(contiguous int32, one entry a row) do not go together, or not on the GPU")
+    _check_pages(r.kcache, r.vcache, r.nkv, r.page_size, r.head_dim, torch.bfloat16, "split_linear_rope_append")
+    cos, sin = r.cos, r.sin
+    if cos is not None and not (sin is not None and cos.is_cuda and sin.is_cuda and cos.dtype == sin.dtype == torch.float32
+                                and cos.shape == sin.shape and cos.shape[1] == half and cos.is_contiguous() and sin.is_contiguous()):
+        raise KernelError("split_linear_rope_append: cos/sin tables must be contiguous float32 [positions, d/2]")
+    cuts = split_cuts(n, k)
+    part = torch.empty((cuts, m, n), dtype=torch.float32, device=x.device)
+    q = torch.empty((m, r.nq * r.head_dim), dtype=torch.bfloat16, device=x.device)
+    call("tk_split_linear_rope_append", x.data_ptr(), x.stride(0), w.data_ptr(), part.data_ptr(), m, k, cuts, q.data_ptr(),
+         r.positions.data_ptr(), r.token_req.data_ptr(), r.block_table.data_ptr(), r.block_table.stride(0),
+         cos.data_ptr() if cos is not None else None, sin.data_ptr() if cos is not None else None, r.kcache.data_ptr(), r.vcache.data_ptr(),
+         r.nq, r.nkv, r.head_dim, r.page_size, _stream())
+    return q
+
+
 def add(x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
     """x + y, each rounded operand added in 32-bit and rounded once."""
     _gpu(x, y)
