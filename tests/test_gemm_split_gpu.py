@@ -18,7 +18,7 @@ def _case(m, n, k, seed):
     return wide[:, 32 : k + 32], (torch.randn((n, k), generator=gen, device="cuda") / k ** 0.5).bfloat16(), gen
 
 
-@pytest.mark.parametrize("m", [1, 15, 16, 17, 32, 33, 64, 65, 96, 97, 128])
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 32, 33, 64, 65, 96, 97, 128, 129, 200, 256])
 @pytest.mark.parametrize("n,k", [(8, 64), (72, 192), (64, 256), (200, 1088), (2048, 2048), (3000, 960)])
 def test_cuts_against_64_bit_sums(m, n, k):
     """Every cut is 32-bit sums of at most k products, and their sum has as many terms as there are cuts: (k + 16) 2^-24 of the
@@ -26,7 +26,7 @@ def test_cuts_against_64_bit_sums(m, n, k):
     x, w, _ = _case(m, n, k, m + n + k)
     want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
     part = ops.gemm_split(x, w)
-    assert part.shape == (ops.split_cuts(n, k), m, n)
+    assert part.shape == (ops.split_cuts(n, k, m), m, n)
     for cuts in {1, 2, 3, k // 64}:
         if cuts > k // 64:
             continue
@@ -96,7 +96,7 @@ def test_product_and_pass_in_one_call():
 
 def test_what_is_refused():
     x, w, _ = _case(4, 64, 128, 1)
-    for bad in ((x[:, :96], w[:, :96].contiguous()), (x, w[:60]), (torch.cat([x] * 33), w), (x.float(), w.float()), (x[:, 1:65], w[:, :64].contiguous())):
+    for bad in ((x[:, :96], w[:, :96].contiguous()), (x, w[:60]), (torch.cat([x] * 65), w), (x.float(), w.float()), (x[:, 1:65], w[:, :64].contiguous())):
         with pytest.raises(ops.KernelError):
             ops.gemm_split(*bad)
 

@@ -1,4 +1,4 @@
-// bfloat16 matrix products for 17 to 128 rows (9 and more over a long inner size) whose outputs are too narrow to give every
+// bfloat16 matrix products for 17 to 256 rows (9 and more over a long inner size) whose outputs are too narrow to give every
 // compute unit weights of its own:  C[M,N] = A[M,K] * W[N,K]^T with K cut among workgroups, and the passes that add the cuts.
 //
 // The product is bound by reading W once; at these rows the output and down projections and the stacked q, k, v product have
@@ -11,6 +11,10 @@
 // 13.4 / 8.5 at 16 rows, 22.8 / 9.5 at 64 (33.5 MB: 3.5 TB/s, a launch's floor included), 21.2 / 12.3 at 128; 2,048 x 2,048 9.0 / 4.9
 // at 64; 3,072 x 2,048 11.1 / 5.5 at 64; 4,096 x 14,336 27.2 / 21.9 at 16 (5.4 TB/s), 38.5 / 25.0 at 64, 75.3 / 33.0 at 128.  Four steps
 // in local memory measured best: with 8 or 9 (144 KB) 2,048 x 8,192 takes 9.7 at 16 rows, with 3 9.1.
+// From 129 rows on there are two blocks of rows, which read W twice, the second time from the caches.  With the passes, library /
+// this one: 2,048 x 8,192 29.4 / 22.9 at 129 rows, 30.7 / 25.9 at 256; 2,048 x 2,048 12.6 / 12.7, 13.6 / 15.6; 4,096 x 4,096 26.3 / 23.7, 27.1 /
+// 25.6; 3,072 x 2,048 with the rotation 14.7 / 16.4, 16.5 / 18.9; 5,120 x 3,072 24.9 / 24.8, 40.5 / 28.5; and a call of the host less, which
+// bounds such steps.  With three blocks it is behind (2,048 x 2,048 14.8 / 18.1 at 300 rows, 4,096 x 14,336 75 / 91).
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
@@ -26,6 +30,7 @@ struct SplitArgs {
 
 #define GS_K 64      // elements of K a step
 #define GS_STAGES 4  // steps that local memory holds
+#define GS_ROWS 256   // rows of A (in blocks of 128, a workgroup one)
 
 // A workgroup of 4 wavefronts owns 64 weight rows and the steps of its cut.  W and A (16 * MB rows, the last one again behind M)
 // go straight from memory to local memory STAGES - 1 steps ahead, the 16-byte piece c of row r at place c ^ (r % 8): a load
@@ -40,7 +45,7 @@ __global__ __launch_bounds__(256) void gemm_split_kernel(SplitArgs a) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, q = lane >> 4;
   // (the cut runs fastest: with 8 cuts a die reads one eighth of A)
-  const int cut = blockIdx.x % a.cuts, first = blockIdx.x / a.cuts * 64;
+  const int cut = blockIdx.x % a.cuts, first = blockIdx.x / a.cuts * 64, row0 = blockIdx.y * 128;
   const int all = a.K / GS_K, s0 = (int)((long)all * cut / a.cuts), steps = (int)((long)all * (cut + 1) / a.cuts) - s0;
   bf16_t* rows = (bf16_t*)smem;
   const unsigned lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) bf16_t*)rows;
@@ -50,7 +55,7 @@ __global__ __launch_bounds__(256) void gemm_split_kernel(SplitArgs a) {
   for (int i = 0; i < 2; ++i) src[i] = a.W + (size_t)min(first + wave * 16 + i * 8 + lr, a.N - 1) * a.K + (size_t)s0 * GS_K + piece;
 #pragma unroll
   for (int i = 0; i < MB / 2; ++i)
-    src[2 + i] = a.A + (size_t)min((wave * (MB / 2) + i) * 8 + lr, a.M - 1) * a.lda + (size_t)s0 * GS_K + piece;
+    src[2 + i] = a.A + (size_t)min(row0 + (wave * (MB / 2) + i) * 8 + lr, a.M - 1) * a.lda + (size_t)s0 * GS_K + piece;
   auto ask = [&](int step, int place) {
     const unsigned base = lds + (unsigned)(place * ROWS * GS_K * (int)sizeof(bf16_t));
     const size_t k = (size_t)step * GS_K;
@@ -94,7 +99,7 @@ __global__ __launch_bounds__(256) void gemm_split_kernel(SplitArgs a) {
   float* out = a.part + (size_t)cut * a.M * a.N;
 #pragma unroll
   for (int mb = 0; mb < NW; ++mb) {
-    const int token = 16 * (wm * NW + mb) + r;
+    const int token = row0 + 16 * (wm * NW + mb) + r;
     if (token >= a.M) continue;
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
@@ -109,14 +114,14 @@ static bool launch_split(const SplitArgs& a, hipStream_t stream) {
   constexpr int lds = GS_STAGES * (64 + 16 * MB) * GS_K * (int)sizeof(bf16_t);
   auto kernel = gemm_split_kernel<MB, NB, GS_STAGES>;
   if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return false;
-  hipLaunchKernelGGL(kernel, dim3((a.N + 63) / 64 * a.cuts), dim3(256), lds, stream, a);
+  hipLaunchKernelGGL(kernel, dim3((a.N + 63) / 64 * a.cuts, (a.M + 127) / 128), dim3(256), lds, stream, a);
   return true;
 }
 
 // part [cuts][M][N] (32-bit) = A [M, K] (rows lda apart) . W [N, K]^T over each cut of K; the sum over the cuts in ascending
 // order is the product.
 TK_API int tk_gemm_split_bf16(const void* A, int lda, const void* W, float* part, int M, int N, int K, int cuts, hipStream_t stream) {
-  TK_REQUIRE(M >= 0 && M <= 128 && N > 0 && N % 4 == 0 && K > 0 && K % GS_K == 0, "gemm_split: bad sizes M=%d N=%d K=%d", M, N, K);
+  TK_REQUIRE(M >= 0 && M <= GS_ROWS && N > 0 && N % 4 == 0 && K > 0 && K % GS_K == 0, "gemm_split: bad sizes M=%d N=%d K=%d", M, N, K);
   TK_REQUIRE(cuts > 0 && cuts <= K / GS_K, "gemm_split: %d cuts of K=%d", cuts, K);
   TK_REQUIRE(lda >= K && lda % 8 == 0 && (((uintptr_t)A | (uintptr_t)W | (uintptr_t)part) & 15) == 0,
              "gemm_split: rows of A, W and the sums must be 16-byte aligned (lda=%d)", lda);

@@ -1097,7 +1097,7 @@ def gemm_skinny_bf16(
 # bfloat16 products with K cut among workgroups, and the passes that add the cuts
 # --------------------------------------------------------------------------
 
-SPLIT_ROWS = 128  # rows the split product takes
+SPLIT_ROWS = 256  # rows the split product takes (gemm_split.hip: beyond, the library's product is ahead)
 SPLIT_TILE, SPLIT_STEP = 64, 64  # weight rows a workgroup, elements of K a step
 # Elements of x (rows x inner size) from which the split product and the pass that adds its cuts are ahead of the
 # weight-streaming kernel, whose workgroups each read all of x.  Measured on an MI355X, weights from memory, us:
@@ -1118,10 +1118,10 @@ SPLIT_WEIGHT_ELEMENTS = 1 << 20
 
 
 @functools.lru_cache(maxsize=None)
-def split_cuts(n: int, k: int) -> int:
-    """Cuts of K for a weight [n, k]: the fewest for which the 256 compute units' rounds of workgroups are filled to nine tenths,
+def split_cuts(n: int, k: int, m: int = 1) -> int:
+    """Cuts of K for a weight [n, k] and ``m`` rows: the fewest for which the 256 compute units' rounds of workgroups are filled to nine tenths,
     a workgroup keeping four steps of K."""
-    tiles = -(-n // SPLIT_TILE)
+    tiles = -(-n // SPLIT_TILE) * -(-m // 128)
     most = max(1, min(16, k // (4 * SPLIT_STEP)))
     filled = lambda c: tiles * c / (256 * -(-tiles * c // 256))  # noqa: E731
     return next((c for c in range(1, most + 1) if filled(c) >= 0.9), max(range(1, most + 1), key=filled))
@@ -1140,13 +1140,13 @@ def split_norm_takes(residual: torch.Tensor, weight: torch.Tensor) -> bool:
 
 
 def gemm_split(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """x [M <= 128, K] . w [N, K]^T in bfloat16 with K cut among workgroups: the cuts' 32-bit sums [cuts, M, N], which
+    """x [M <= 256, K] . w [N, K]^T in bfloat16 with K cut among workgroups: the cuts' 32-bit sums [cuts, M, N], which
     ``split_add_rmsnorm`` or ``split_rope_append`` adds in ascending order."""
     _gpu(x, w)
     _need(x.dim() == 2 and w.dim() == 2 and w.is_contiguous() and x.shape[1] == w.shape[1] and split_takes(x, w),
-          "gemm_split: x [M, K] (up to 128 rows at multiples of 16 bytes) and w [N, K] must be bfloat16, K a multiple of 64, N of 8")
+          "gemm_split: x [M, K] (up to 256 rows at multiples of 16 bytes) and w [N, K] must be bfloat16, K a multiple of 64, N of 8")
     m, (n, k) = x.shape[0], w.shape
-    cuts = split_cuts(n, k)
+    cuts = split_cuts(n, k, m)
     part = torch.empty((cuts, m, n), dtype=torch.float32, device=x.device)
     call("tk_gemm_split_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), part.data_ptr(), m, n, k, cuts, _stream())
     return part
@@ -1206,7 +1206,7 @@ def split_linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.T
             and weight.shape == (n,) and weight.is_contiguous() and (dtype == torch.bfloat16 or dtype == torch.float32)):
         raise KernelError(f"split_linear_add_rmsnorm: x {tuple(x.shape)} {x.dtype}, w {tuple(w.shape)} {w.dtype}, residual {tuple(residual.shape)} "
                           f"{residual.dtype} and norm weight {tuple(weight.shape)} {dtype} do not go together, or not on the GPU")
-    cuts = split_cuts(n, k)
+    cuts = split_cuts(n, k, m)
     part = torch.empty((cuts, m, n), dtype=torch.float32, device=x.device)
     stream_out, out = torch.empty_like(residual), torch.empty_like(residual)
     call("tk_split_linear_add_rmsnorm", x.data_ptr(), x.stride(0), w.data_ptr(), part.data_ptr(), m, n, k, cuts, residual.data_ptr(),
@@ -1231,7 +1231,7 @@ def split_linear_rope_append(x: torch.Tensor, w: torch.Tensor, r: RopeAppend) ->
     if cos is not None and not (sin is not None and cos.is_cuda and sin.is_cuda and cos.dtype == sin.dtype == torch.float32
                                 and cos.shape == sin.shape and cos.shape[1] == half and cos.is_contiguous() and sin.is_contiguous()):
         raise KernelError("split_linear_rope_append: cos/sin tables must be contiguous float32 [positions, d/2]")
-    cuts = split_cuts(n, k)
+    cuts = split_cuts(n, k, m)
     part = torch.empty((cuts, m, n), dtype=torch.float32, device=x.device)
     q = torch.empty((m, r.nq * r.head_dim), dtype=torch.bfloat16, device=x.device)
     call("tk_split_linear_rope_append", x.data_ptr(), x.stride(0), w.data_ptr(), part.data_ptr(), m, k, cuts, q.data_ptr(),
