@@ -1299,6 +1299,7 @@ def gemm_library_bf16(x: torch.Tensor, w: torch.Tensor, out_f32: bool = False, o
 # add (fitted to 234 products of 13 weights at 129 to 8,192 rows, weights from memory; the tile that comes out fastest by them is the
 # fastest measured one in 218)
 TILE_SHAPES = ((128, 128, 0.47, 4.3), (192, 128, 0.54, 6.5), (128, 256, 0.79, 5.5), (192, 256, 0.96, 11.2), (256, 256, 1.19, 15.5))
+TILES_LONGEST_STRIDE = 1 << 22  # elements between rows of x (a tile's rows lie within 32-bit bytes of its first)
 GLU_TILES_FROM_ROWS = 65  # (up to 64 rows gate and up stream through local memory)
 # two rounds of tiles of 256 x 256: with more the chip's power bounds the step, and the library's kernel needs less of it (a prompt of
 # 2,048 tokens of the 1B shape 5,027 to 4,984 us with the tiles, four of 1,024 of the 8B shape 43.3 to 44.6 ms)

@@ -144,7 +144,7 @@ class Linear:
                                             staged=2 if swiglu and ops.glu_streams(m, self.total_out // 2, self.in_features) else -1)
             # many rows: in tiles where these are ahead of the library's product (the gated form with silu in one kernel)
             direct = ops.gemm_library_direct(x, w)
-            if direct and bias is None and not out_f32 and (glu is None or not swiglu):
+            if direct and bias is None and not out_f32 and (glu is None or not swiglu) and x.stride(0) <= ops.TILES_LONGEST_STRIDE:
                 shape = ops.tiles_choice(m, w.shape[0] // 2 if swiglu else w.shape[0], self.in_features, swiglu)
                 if shape >= 0:
                     prod = ops.gemm_tiles_bf16(x, w, shape, swiglu)
