@@ -1,0 +1,48 @@
+"""Which product a linear map takes and what the products' wrappers refuse, without a GPU: tensors that say they lie on one, and
+recorders in the place of the kernels."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from tokasaurus_amd.kernels import ops
+
+
+class OnGpu(torch.Tensor):
+    is_cuda = True
+
+
+def on_gpu(*shape, dtype=torch.bfloat16, device="cpu"):
+    return torch.empty(shape, dtype=dtype, device=device).as_subclass(OnGpu)
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    """Names of the kernels that are called; none is."""
+    made = []
+    monkeypatch.setattr(ops, "call", lambda name, *a: made.append(name))
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    return made
+
+
+def _rope(rows, nq=4, nkv=2, d=32, page=16):
+    i32 = dict(dtype=torch.int32)
+    return ops.RopeAppend(on_gpu(rows, **i32), on_gpu(rows, **i32), on_gpu(1, 4, **i32), on_gpu(64, d // 2, dtype=torch.float32),
+                          on_gpu(64, d // 2, dtype=torch.float32), on_gpu(*ops.key_pages_shape(4, nkv, page, d)),
+                          on_gpu(*ops.value_pages_shape(4, nkv, page, d)), nq, nkv, d, page)
+
+
+@pytest.mark.parametrize("where", ["host", "another device"])
+def test_a_weight_that_is_not_where_the_rows_are_is_refused(calls, where):
+    x, residual, norm = on_gpu(33, 192), on_gpu(33, 256), on_gpu(256)
+    ops.split_linear_add_rmsnorm(x, on_gpu(256, 192), residual, norm, 1e-5)
+    ops.split_linear_rope_append(x, on_gpu(256, 192), _rope(33))
+    ops.gemm_tiles_bf16(x, on_gpu(256, 192), 0)
+    assert calls == ["tk_split_linear_add_rmsnorm", "tk_split_linear_rope_append", "tk_gemm_tiles_bf16"]
+    w = torch.empty((256, 192), dtype=torch.bfloat16) if where == "host" else on_gpu(256, 192, device="meta")
+    for refused in (lambda: ops.split_linear_add_rmsnorm(x, w, residual, norm, 1e-5), lambda: ops.split_linear_rope_append(x, w, _rope(33)),
+                    lambda: ops.gemm_split(x, w), lambda: ops.gemm_tiles_bf16(x, w, 0)):
+        with pytest.raises(ops.KernelError):
+            refused()
+    assert len(calls) == 3

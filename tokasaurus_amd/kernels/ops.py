@@ -1143,8 +1143,8 @@ def gemm_split(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x [M <= 256, K] . w [N, K]^T in bfloat16 with K cut among workgroups: the cuts' 32-bit sums [cuts, M, N], which
     ``split_add_rmsnorm`` or ``split_rope_append`` adds in ascending order."""
     _gpu(x, w)
-    _need(x.dim() == 2 and w.dim() == 2 and w.is_contiguous() and x.shape[1] == w.shape[1] and split_takes(x, w),
-          "gemm_split: x [M, K] (up to 256 rows at multiples of 16 bytes) and w [N, K] must be bfloat16, K a multiple of 64, N of 8")
+    _need(x.dim() == 2 and w.dim() == 2 and w.is_contiguous() and x.shape[1] == w.shape[1] and x.device == w.device and split_takes(x, w),
+          "gemm_split: x [M, K] (up to 256 rows at multiples of 16 bytes) and w [N, K] must be bfloat16 on one device, K a multiple of 64, N of 8")
     m, (n, k) = x.shape[0], w.shape
     cuts = split_cuts(n, k, m)
     part = torch.empty((cuts, m, n), dtype=torch.float32, device=x.device)
@@ -1201,8 +1201,8 @@ def split_linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.T
     m, k = x.shape
     n = w.shape[0]
     dtype = weight.dtype
-    if not (x.is_cuda and residual.is_cuda and weight.is_cuda and w.is_contiguous() and w.shape[1] == k and split_takes(x, w)
-            and residual.shape == (m, n) and residual.dtype == torch.bfloat16 and residual.is_contiguous()
+    if not (x.is_cuda and w.is_cuda and residual.is_cuda and weight.is_cuda and x.device == w.device and w.is_contiguous()
+            and w.shape[1] == k and split_takes(x, w) and residual.shape == (m, n) and residual.dtype == torch.bfloat16 and residual.is_contiguous()
             and weight.shape == (n,) and weight.is_contiguous() and (dtype == torch.bfloat16 or dtype == torch.float32)):
         raise KernelError(f"split_linear_add_rmsnorm: x {tuple(x.shape)} {x.dtype}, w {tuple(w.shape)} {w.dtype}, residual {tuple(residual.shape)} "
                           f"{residual.dtype} and norm weight {tuple(weight.shape)} {dtype} do not go together, or not on the GPU")
@@ -1219,7 +1219,8 @@ def split_linear_rope_append(x: torch.Tensor, w: torch.Tensor, r: RopeAppend) ->
     m, k = x.shape
     n, half = w.shape[0], r.head_dim // 2
     i32 = torch.int32
-    if not (x.is_cuda and w.is_contiguous() and w.shape[1] == k and split_takes(x, w) and n == (r.nq + 2 * r.nkv) * r.head_dim
+    if not (x.is_cuda and w.is_cuda and x.device == w.device and w.is_contiguous() and w.shape[1] == k and split_takes(x, w)
+            and n == (r.nq + 2 * r.nkv) * r.head_dim
             and (r.rotary_dim is None or r.rotary_dim == r.head_dim)
             and r.positions.dtype == r.token_req.dtype == r.block_table.dtype == i32 and r.positions.numel() == r.token_req.numel() == m
             and r.positions.is_contiguous() and r.token_req.is_contiguous() and r.block_table.is_contiguous() and r.block_table.dim() == 2
@@ -1341,8 +1342,8 @@ def gemm_tiles_bf16(x: torch.Tensor, w: torch.Tensor, shape: int, glu: bool = Fa
     start at multiples of 16 bytes."""
     _gpu(x, w)
     if not (x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.dtype == w.dtype == torch.bfloat16 and x.stride(1) == 1
-            and w.is_contiguous() and (not glu or w.shape[0] % 2 == 0)):
-        raise KernelError(f"gemm_tiles: x {tuple(x.shape)} {x.dtype} and w {tuple(w.shape)} {w.dtype} must be bfloat16 [M, K] and [N, K] of contiguous rows")
+            and w.is_contiguous() and x.device == w.device and (not glu or w.shape[0] % 2 == 0)):
+        raise KernelError(f"gemm_tiles: x {tuple(x.shape)} {x.dtype} and w {tuple(w.shape)} {w.dtype} must be bfloat16 [M, K] and [N, K] of contiguous rows, on one device")
     m, k = x.shape
     n = w.shape[0] // 2 if glu else w.shape[0]
     out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
