@@ -91,6 +91,14 @@ def test_tiles_hold_every_choice(tokens, top, experts, spread):
         assert (t < used) == (mine.numel() > 0) and (ids.flatten()[mine] == group[t]).all()
 
 
+@pytest.mark.parametrize("spread", ["one expert", "all", "each its own"])
+def test_as_many_experts_as_local_memory_holds(spread):
+    """4,096 experts, three numbers each: 48 KB, which a kernel has without asking for more; one expert more is refused."""
+    test_tiles_hold_every_choice(700, 8, 4096, spread)
+    with pytest.raises(ops.KernelError, match="too many experts"):
+        ops.expert_sort([(torch.zeros((2, 2), dtype=torch.int32, device="cuda"), 4097)])
+
+
 def test_room_for_the_experts_is_that_of_the_pairs():
     """256 experts of inner size 2,048, 64 pairs: rows between the two products are the pairs', not those of tiles an expert."""
     g = torch.Generator(device="cuda").manual_seed(1)

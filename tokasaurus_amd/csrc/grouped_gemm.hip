@@ -507,15 +507,13 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(SortJobs jobs) {
   int* __restrict__ slot_pair = jb.slot_pair;
   int* __restrict__ slot_token = jb.slot_token;
   int* __restrict__ tile_group = jb.tile_group;
-  extern __shared__ int sh[];  // [experts] each: counts, first slots, cursors, first pairs of tiles, first single tiles
+  extern __shared__ int sh[];  // [experts] each: counts (then the slots that are left), first slots, first single tiles
   int* count = sh;
   int* first = sh + experts;
-  int* cursor = sh + 2 * experts;
-  int* first_pair = sh + 3 * experts;
-  int* first_single = sh + 4 * experts;
+  int* first_single = sh + 2 * experts;
   TileRun* run_of_pair = jb.runs + 1;
   TileRun* run_of_single = run_of_pair + max_tiles / 2;
-  for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = cursor[e] = 0;
+  for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = 0;
   for (int s = threadIdx.x; s < max_tiles * tm; s += blockDim.x) slot_pair[s] = slot_token[s] = -1;
   for (int t = threadIdx.x; t < max_tiles; t += blockDim.x) tile_group[t] = -1;
   __syncthreads();
@@ -529,7 +527,6 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(SortJobs jobs) {
     for (int e = 0; e < experts; ++e) {
       const int n = (count[e] + tm - 1) / tm;
       first[e] = at;
-      first_pair[e] = twos;
       first_single[e] = ones;
       at += n * tm;
       twos += n / 2;
@@ -541,14 +538,16 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(SortJobs jobs) {
   __syncthreads();
   for (int e = threadIdx.x; e < experts; e += blockDim.x) {
     const int t0 = first[e] / tm, n = (count[e] + tm - 1) / tm;
+    const int first_pair = (t0 - first_single[e]) / 2;  // (the tiles in front are pairs of two and singles)
     for (int t = 0; t < n; ++t) tile_group[t0 + t] = e;
-    for (int p = 0; p < n / 2; ++p) run_of_pair[first_pair[e] + p] = {t0, e, first_pair[e], n / 2};
+    for (int p = 0; p < n / 2; ++p) run_of_pair[first_pair + p] = {t0, e, first_pair, n / 2};
     if (n & 1) run_of_single[first_single[e]] = {t0 + n - 1, e, first_single[e], 1};
   }
+  __syncthreads();
   for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
     const int e = ids[p];
     if (e >= 0 && e < experts) {
-      const int s = first[e] + atomicAdd(&cursor[e], 1);
+      const int s = first[e] + atomicSub(&count[e], 1) - 1;
       slot_pair[s] = p;
       slot_token[s] = p / top;
     }
@@ -568,10 +567,10 @@ TK_API int tk_expert_sort(const SortJob* jobs, int n_jobs, hipStream_t stream) {
       TK_REQUIRE(j.max_tiles >= (j.pairs + (long)(GS_M - 1) * min(j.experts, j.pairs)) / GS_M, "expert_sort: %d tiles cannot hold %d pairs of %d experts", j.max_tiles,
                  j.pairs, j.experts);
       TK_REQUIRE(j.max_singles >= min(j.experts, j.max_tiles), "expert_sort: %d single tiles cannot hold those of %d experts", j.max_singles, j.experts);
-      TK_REQUIRE(5 * j.experts * sizeof(int) <= 80 * 1024, "expert_sort: too many experts");
+      TK_REQUIRE(3 * j.experts * sizeof(int) <= 48 * 1024, "expert_sort: too many experts");
       most = max(most, j.experts);
     }
-    hipLaunchKernelGGL(expert_sort_kernel, dim3(n), dim3(1024), 5 * most * sizeof(int), stream, all);
+    hipLaunchKernelGGL(expert_sort_kernel, dim3(n), dim3(1024), 3 * most * sizeof(int), stream, all);
     TK_CHECK_LAUNCH("expert_sort");
   }
   return 0;
