@@ -52,6 +52,38 @@ def test_residual_sum_and_norm(rows, hidden, cuts, w32):
         assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("rows,hidden,cuts", [(1, 8, 1), (3, 72, 5), (17, 2048, 8), (2, 9000, 2)])
+@pytest.mark.parametrize("w32", [False, True])
+def test_normed_rows_rounded_once(rows, hidden, cuts, w32):
+    """The rows that go on are as without it; the normed ones are their 64-bit norm rounded once (8 significant bits: 2^-8 of the value at
+    most, twice rounded up to 2^-7; the sum of squares, its root and the product are 32-bit: well under 2^-15)."""
+    gen = torch.Generator(device="cuda").manual_seed(hidden + cuts + 1)
+    part, residual = torch.randn((cuts, rows, hidden), generator=gen, device="cuda"), torch.randn((rows, hidden), generator=gen, device="cuda").bfloat16()
+    weight = torch.randn((hidden,), generator=gen, device="cuda")
+    weight = weight if w32 else weight.bfloat16()
+    stream, normed = ops.split_add_rmsnorm(part, residual, weight, 1e-5, once=True)
+    assert torch.equal(stream, ops.split_add_rmsnorm(part, residual, weight, 1e-5)[0])
+    x = stream.double()
+    want = x / torch.sqrt((x * x).mean(1, keepdim=True) + 1e-5) * weight.double()
+    assert ((normed.double() - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -15)).all()
+
+
+@pytest.mark.parametrize("rows,n,k", [(6, 2048, 8192), (24, 2048, 2048), (4, 4096, 14336)])
+def test_few_rows_are_rounded_once_behind_a_linear_map(rows, n, k):
+    """As many rows as the weight-streaming product would have taken, in the split form: what stands behind the norm is rounded once."""
+    from tokasaurus_amd.parts.linear import Linear
+    from tokasaurus_amd.parts.norm import RMSNorm
+
+    x, w, gen = _case(rows, n, k, rows + n)
+    lin, norm = Linear(k, ["w"], [n]), RMSNorm(n, 1e-5, "n")
+    lin.weight, norm.weight = w, (1 + 0.1 * torch.randn((n,), generator=gen, device="cuda")).bfloat16()
+    assert rows <= ops.skinny_rows(k) and lin._splits(x, ops.SPLIT_NORM_ELEMENTS)
+    stream, prepared = lin.with_residual(x, torch.randn((rows, n), generator=gen, device="cuda").bfloat16(), norm)
+    s = stream.double()
+    want = s / torch.sqrt((s * s).mean(1, keepdim=True) + 1e-5) * norm.weight.double()
+    assert ((prepared.normed.double() - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -15)).all()
+
+
 @pytest.mark.parametrize("nq,nkv,d,page", [(4, 2, 16, 16), (32, 8, 64, 16), (5, 5, 80, 4), (16, 2, 128, 32)])
 @pytest.mark.parametrize("tables", [True, False])
 def test_rotation_and_append(nq, nkv, d, page, tables):

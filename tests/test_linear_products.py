@@ -7,6 +7,9 @@ import pytest
 import torch
 
 from tokasaurus_amd.kernels import ops
+from tokasaurus_amd.parts.base import Normed, Prepared
+from tokasaurus_amd.parts.linear import Linear
+from tokasaurus_amd.parts.norm import RMSNorm
 
 
 class OnGpu(torch.Tensor):
@@ -46,3 +49,27 @@ def test_a_weight_that_is_not_where_the_rows_are_is_refused(calls, where):
         with pytest.raises(ops.KernelError):
             refused()
     assert len(calls) == 3
+
+
+def linear(outputs, inner):
+    lin = Linear(inner, ["w"], [outputs])
+    lin.weight = on_gpu(outputs, inner)
+    return lin
+
+
+def norm(size):
+    n = RMSNorm(size, 1e-5, "n")
+    n.weight = on_gpu(size)
+    return n
+
+
+def test_a_prepared_norm_is_folded_into_the_product_with_the_rotation(calls):
+    """Rows that the weight-streaming product in front left for this norm: no pass of a norm's own, no second rounding."""
+    lin, n = linear(3072, 2048), norm(2048)
+    data = ops.Prenorm(on_gpu(16, 2048), on_gpu(16, 128, dtype=torch.float32))
+    rope = _rope(16, 32, 8, 64)
+    assert lin.rope_append(Normed(on_gpu(16, 2048), n, Prepared(data, n)), rope) is not None
+    assert calls == ["tk_gemm_skinny_bf16"]
+    calls.clear()
+    assert lin.rope_append(Normed(on_gpu(16, 2048), n, Prepared(None, n, on_gpu(16, 2048))), rope) is not None
+    assert calls == ["tk_split_linear_rope_append"]

@@ -155,11 +155,14 @@ __device__ __forceinline__ void product8(const float* part, size_t apart, int cu
 }
 
 // stream_out = product + residual (rounded); out = RMSNorm(stream_out) * w: a workgroup a row, the arithmetic of
-// rmsnorm_packed_kernel.  A thread keeps the first SN_HELD pieces of 8 that it takes in registers.
+// rmsnorm_packed_kernel.  A thread keeps the first SN_HELD pieces of 8 that it takes in registers.  once: the normed value is not
+// rounded in front of the weight.  Rows that few go through the weight-streaming kernel round an operand of the next product
+// once (x w, the row's factor on the 32-bit sums), and keep that where the split form takes its place: 8 rows of 2,048 against
+// 64 bits 1.7e-3 of the norm, rounded twice 2.4e-3.
 #define SN_HELD 4
 __global__ __launch_bounds__(256) void split_add_rmsnorm_kernel(const float* __restrict__ part, int cuts, const bf16_t* __restrict__ residual,
                                                                 const void* __restrict__ w, int w_f32, bf16_t* __restrict__ stream_out,
-                                                                bf16_t* __restrict__ out, int rows, int hidden, float eps) {
+                                                                bf16_t* __restrict__ out, int rows, int hidden, float eps, int once) {
   __shared__ float red[16];
   const size_t base = (size_t)blockIdx.x * hidden, apart = (size_t)rows * hidden;
   const int pieces = hidden / 8;
@@ -204,7 +207,7 @@ __global__ __launch_bounds__(256) void split_add_rmsnorm_kernel(const float* __r
     float wf[8];
     weights(piece, wf);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o.v[j] = from_f32<bf16_t>(wf[j] * round_to<bf16_t>(v[j] * rstd));
+    for (int j = 0; j < 8; ++j) o.v[j] = from_f32<bf16_t>(wf[j] * (once ? v[j] * rstd : round_to<bf16_t>(v[j] * rstd)));
     o.store(out + base + (size_t)piece * 8);
   };
 #pragma unroll
@@ -223,7 +226,7 @@ __global__ __launch_bounds__(256) void split_add_rmsnorm_kernel(const float* __r
 }
 
 TK_API int tk_split_add_rmsnorm(const float* part, int cuts, const void* residual, const void* w, int w_f32, void* stream_out, void* out,
-                                int rows, int hidden, float eps, hipStream_t stream) {
+                                int rows, int hidden, float eps, int once, hipStream_t stream) {
   TK_REQUIRE(rows >= 0 && hidden > 0 && hidden % 8 == 0 && cuts > 0, "split_add_rmsnorm: bad sizes %d %d, %d cuts", rows, hidden, cuts);
   TK_REQUIRE(part && residual && w && stream_out && out, "split_add_rmsnorm: an operand is missing");
   TK_REQUIRE((((uintptr_t)part | (uintptr_t)residual | (uintptr_t)w | (uintptr_t)stream_out | (uintptr_t)out) & 15) == 0,
@@ -231,7 +234,7 @@ TK_API int tk_split_add_rmsnorm(const float* part, int cuts, const void* residua
   TK_REQUIRE(out != residual && out != stream_out && stream_out != residual, "split_add_rmsnorm: inputs and outputs must not share a buffer");
   if (rows == 0) return 0;
   hipLaunchKernelGGL(split_add_rmsnorm_kernel, dim3(rows), dim3(256), 0, stream, part, cuts, (const bf16_t*)residual, w, w_f32,
-                     (bf16_t*)stream_out, (bf16_t*)out, rows, hidden, eps);
+                     (bf16_t*)stream_out, (bf16_t*)out, rows, hidden, eps, once);
   TK_CHECK_LAUNCH("split_add_rmsnorm");
   return 0;
 }
@@ -320,9 +323,9 @@ TK_API int tk_split_rope_append(const float* part, int cuts, void* q, const int*
 // ---------------------------------------------------------------------------------
 
 TK_API int tk_split_linear_add_rmsnorm(const void* A, int lda, const void* W, float* part, int M, int N, int K, int cuts, const void* residual,
-                                       const void* w, int w_f32, void* stream_out, void* out, float eps, hipStream_t stream) {
+                                       const void* w, int w_f32, void* stream_out, void* out, float eps, int once, hipStream_t stream) {
   const int rc = tk_gemm_split_bf16(A, lda, W, part, M, N, K, cuts, stream);
-  return rc ? rc : tk_split_add_rmsnorm(part, cuts, residual, w, w_f32, stream_out, out, M, N, eps, stream);
+  return rc ? rc : tk_split_add_rmsnorm(part, cuts, residual, w, w_f32, stream_out, out, M, N, eps, once, stream);
 }
 
 TK_API int tk_split_linear_rope_append(const void* A, int lda, const void* W, float* part, int M, int K, int cuts, void* q, const int* positions,

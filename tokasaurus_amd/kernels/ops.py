@@ -1152,8 +1152,10 @@ def gemm_split(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return part
 
 
-def split_add_rmsnorm(part: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float) -> tuple[torch.Tensor, torch.Tensor]:
-    """``add_rmsnorm`` of a split product: (product rounded, + residual, rounded; its RMSNorm times ``weight``) in one pass."""
+def split_add_rmsnorm(part: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float,
+                      once: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
+    """``add_rmsnorm`` of a split product: (product rounded, + residual, rounded; its RMSNorm times ``weight``) in one pass.
+    ``once``: the normed value is rounded with the weight on it only, not in front of it too."""
     _gpu(part, residual, weight)
     _need(part.dim() == 3 and part.dtype == torch.float32 and part.is_contiguous() and residual.shape == part.shape[1:]
           and residual.is_contiguous() and residual.dtype == torch.bfloat16,
@@ -1163,7 +1165,7 @@ def split_add_rmsnorm(part: torch.Tensor, residual: torch.Tensor, weight: torch.
         raise KernelError("split_add_rmsnorm: the weight must be [H] of bfloat16 or float32")
     stream_out, out = torch.empty_like(residual), torch.empty_like(residual)
     call("tk_split_add_rmsnorm", part.data_ptr(), cuts, residual.data_ptr(), weight.data_ptr(), 1 if weight.dtype == torch.float32 else 0,
-         stream_out.data_ptr(), out.data_ptr(), rows, hidden, float(eps), _stream())
+         stream_out.data_ptr(), out.data_ptr(), rows, hidden, float(eps), 1 if once else 0, _stream())
     return stream_out, out
 
 
@@ -1196,8 +1198,9 @@ def split_rope_append(part: torch.Tensor, r: RopeAppend) -> torch.Tensor:
 # 101 tokens of the 1B shape, 45 such pairs among its 130 launches: 1,800 us with two calls each, 1,683 with one).
 
 
-def split_linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float) -> tuple[torch.Tensor, torch.Tensor]:
-    """``split_add_rmsnorm(gemm_split(x, w), residual, weight, eps)``."""
+def split_linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float,
+                             once: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
+    """``split_add_rmsnorm(gemm_split(x, w), residual, weight, eps, once)``."""
     m, k = x.shape
     n = w.shape[0]
     dtype = weight.dtype
@@ -1210,7 +1213,7 @@ def split_linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.T
     part = torch.empty((cuts, m, n), dtype=torch.float32, device=x.device)
     stream_out, out = torch.empty_like(residual), torch.empty_like(residual)
     call("tk_split_linear_add_rmsnorm", x.data_ptr(), x.stride(0), w.data_ptr(), part.data_ptr(), m, n, k, cuts, residual.data_ptr(),
-         weight.data_ptr(), 1 if dtype == torch.float32 else 0, stream_out.data_ptr(), out.data_ptr(), eps, _stream())
+         weight.data_ptr(), 1 if dtype == torch.float32 else 0, stream_out.data_ptr(), out.data_ptr(), eps, 1 if once else 0, _stream())
     return stream_out, out
 
 

@@ -184,7 +184,8 @@ class Linear:
         that will be applied to the result) needs so that it costs no kernel of its own."""
         fusable = emit_norm is not None and getattr(emit_norm, "fusable_rms", False)
         if fusable and residual.is_contiguous() and self._splits(x, ops.SPLIT_NORM_ELEMENTS) and ops.split_norm_takes(residual, emit_norm.weight):
-            out, normed = ops.split_linear_add_rmsnorm(x, self.weight, residual, emit_norm.weight, emit_norm.eps)
+            # (few rows: the next product's operand is rounded once, as where the weight-streaming product emits it)
+            out, normed = ops.split_linear_add_rmsnorm(x, self.weight, residual, emit_norm.weight, emit_norm.eps, self._fast(x.shape[0]))
             return out, Prepared(None, emit_norm, normed)
         if fusable and self._fast(x.shape[0]):
             out, data = ops.gemm_skinny_bf16(x, self.weight, residual=residual, emit_weight=emit_norm.weight, bias=self.bias)
@@ -202,17 +203,19 @@ class Linear:
         m = (x.x if isinstance(x, Normed) else x).shape[0]
         whole = rope.head_dim % 8 == 0 and (rope.rotary_dim is None or rope.rotary_dim == rope.head_dim)
         stream = x.x if isinstance(x, Normed) else x
-        if whole and self._splits(stream, ops.SPLIT_ROPE_ELEMENTS):
+        # (a norm that the product in front prepared is folded in below: its rows are not made for the split form)
+        prepared = x.usable() if isinstance(x, Normed) else None
+        if whole and prepared is None and self._splits(stream, ops.SPLIT_ROPE_ELEMENTS):
             rows = x.materialize() if isinstance(x, Normed) else x  # (a norm's rows lie as their stream does, or from their own start)
             if ops.split_takes(rows, self.weight):
                 return ops.split_linear_rope_append(rows, self.weight, rope)
+            x = rows
         most = min(ops.SKINNY_ROPE_ROWS, 2 * ops.skinny_rows(self.in_features, paired=True))
         fits = self.weight.dtype == torch.bfloat16 and 0 < m <= most and self._aligned()
         if not fits or rope.head_dim % 2 or (rope.rotary_dim is not None and rope.rotary_dim != rope.head_dim):
             return None
         prenorm, eps = None, 0.0
         if isinstance(x, Normed):
-            prepared = x.usable()
             if prepared is not None:
                 prenorm, eps, x = prepared.data, x.norm.eps, prepared.data.scaled
             else:
