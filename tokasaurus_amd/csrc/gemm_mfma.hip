@@ -600,7 +600,7 @@ __global__ __launch_bounds__(1024) void gemm_staged_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------------
-// Gate and up projections for up to 64 rows (SwiGLU epilogue; glu_streams says when): a workgroup of 4 wavefronts owns 32 pairs of weight rows
+// Gate and up projections for up to 64 rows (SwiGLU epilogue; ops.glu_streams says when): a workgroup of 4 wavefronts owns 32 pairs of weight rows
 // and all of K.  In steps of 64 elements the 64 rows of W and the rows of A (16 * MB, the last one again behind M) go
 // straight from memory to local memory, gl_stages - 1 steps ahead, so that a compute unit has 40 KB and more of W on the
 // way whatever the wavefronts do; two workgroups share a unit.  Wavefront w takes 8 gate rows and their 8 up rows as one
@@ -728,18 +728,6 @@ static bool launch_staged_one(const GemmArgs& a, int groups, int WK, hipStream_t
   return true;
 }
 
-// Where gate and up are streamed through local memory instead of into the wavefronts' registers.  Measured on an MI355X
-// (us, weights from memory; skinny / streamed): N = 14,336, K = 4,096: 50.5 / 47.0 at 2 rows, 55.6 / 47.1 at 8, 63.5 / 47.5 at
-// 16; 8,192 x 3,072: 24.2 / 21.1 at 2, 30.2 / 19.9 at 16; 8,192 x 2,048: 17.1 / 18.2 at 4, 18.4 / 17.0 at 16 (at 8 alone 18.1 /
-// 17.5, but a whole 1B step, with the norm in front, 1,318 / 1,347); 8,192 x 2,304: 20.2 / 17.4 at 2, 22.5 / 16.3 at 16; 8,192 x
-// 2,560: 23.1 / 19.1 at 2; 8,192 x 2,816: 23.6 / 20.7 at 2;
-// with fewer workgroups than compute units 4,096 x 2,048: 10.3 / 10.3 at 16, 11.9 / 11.7 at 20, 13.6 / 11.6 at 32; 1,000 x 1,024:
-// 6.6 / 7.0 at 32, 9.4 / 9.1 at 48.
-static bool glu_streams(int M, int N, int K) {
-  if (N >= 32 * 256) return M >= (K >= 2304 ? 2 : 16);
-  return (long)M * K >= 40000;
-}
-
 template <int MB, int NB>
 static bool launch_glu_stream(const GemmArgs& a, bool norm, hipStream_t stream) {
   const size_t lds = (size_t)gl_stages<MB>() * (64 + 16 * MB) * GL_K * sizeof(bf16_t) + (norm ? 16 * MB * sizeof(float) : 0);
@@ -847,7 +835,7 @@ TK_API int tk_gemm_skinny_parts(int M, int N, int tile_rows) {
 // norm in front, the outputs for a following norm and the rotation's operands.
 // waves_k: wavefronts (skinny) or wavefront rows (staged) that split K inside a workgroup
 // (0 = choose); tiles: weight tiles per wavefront, 1 or 2 (0 = choose; SwiGLU and the rotation
-// always pair); staged: -1 = choose, 0 = skinny, 1 = staged, 2 = streamed gate and up; tile_rows: weight rows of a
+// always pair); staged: -1 = choose of the first two, 0 = skinny, 1 = staged, 2 = streamed gate and up; tile_rows: weight rows of a
 // tile that the skinny kernel uses, 16 or 8 (0 = choose; tk_gemm_skinny_parts tells the
 // choice to whoever sizes emit_sumsq); fold: 0 = never fold K into the unused half of the matrix
 // core, else where it can be done (tiles of 8 weight rows, up to 8 rows of A: gemm_skinny_kernel).
@@ -909,9 +897,8 @@ TK_API int tk_gemm_skinny_bf16(const void* A, int lda, const void* W, void* C, i
   int NT = paired ? 2 : (tiles > 0 ? tiles : 1);
   TK_REQUIRE(NT == 1 || NT == 2, "gemm_skinny: tiles=%d outside 1..2", NT);
   bool ok;
-  const bool stream_fits = epi == EPI_SWIGLU && M <= 64 && K % GL_K == 0;
-  TK_REQUIRE(staged != 2 || stream_fits, "gemm_skinny: the streamed gate and up product takes 64 rows and a K of a multiple of 64");
-  if (staged == 2 || (staged < 0 && stream_fits && glu_streams(M, N, K))) {
+  TK_REQUIRE(staged != 2 || (epi == EPI_SWIGLU && M <= 64 && K % GL_K == 0), "gemm_skinny: the streamed gate and up product takes 64 rows and a K of a multiple of 64");
+  if (staged == 2) {
     ok = M <= 16 ? launch_glu_stream<2, 1>(a, norm, stream)
                  : (M <= 32 ? launch_glu_stream<2, 2>(a, norm, stream) : launch_glu_stream<4, 4>(a, norm, stream));
   } else if (use_staged) {

@@ -902,11 +902,23 @@ def glu_rows(inner: int, outputs: int = 0) -> int:
     return GLU_STREAM_ROWS if inner <= 4096 and (rounds <= 1 or 8 * groups >= 7 * 256 * rounds) else GLU_STREAM_DEEP_ROWS
 
 
+@functools.lru_cache(maxsize=4096)
 def glu_streams(rows: int, outputs: int, inner: int) -> bool:
-    """Whether gate and up are asked for in their streamed form whatever the product itself would choose: where there is a workgroup
-    for every compute unit.  Weight-streaming / streamed on an MI355X since its workgroups begin their walks apart, us: 8,192 x 2,048
-    15.8 / 14.9 at one row, 16.8 / 14.1 at 8; 8,192 x 3,072 24.0 / 21.5 at one; 14,336 x 4,096 49.6 / 42.3 at one."""
-    return outputs >= 32 * 256 and inner % 64 == 0 and 0 < rows <= GLU_STREAM_ROWS
+    """Whether gate and up (``outputs`` of each) of up to 64 rows stream through local memory instead of into the wavefronts' registers.
+    Weight-streaming / streamed on an MI355X, us, weights from memory, at 1, 4, 8 and 16 rows: 8,192 x 2,048 16.1 / 14.8, 16.5 / 14.8, 17.3 /
+    14.3, 18.9 / 14.2; 8,192 x 3,072 24.1 / 21.4, 25.2 / 21.4, 25.0 / 20.1, 28.1 / 20.2; 14,336 x 4,096 49.0 / 45.1, 50.0 / 42.6, 53.8 / 42.3,
+    61.7 / 42.7; 9,216 x 2,048 21.4 / 20.9, 21.5 / 20.4, 22.6 / 20.6, 25.2 / 20.7; 10,240 x 2,560 33.3 / 27.2, 31.9 / 26.7, 31.1 / 27.0,
+    34.7 / 28.0; 13,824 x 5,120 63.2 / 53.5, 67.0 / 50.9, 73.0 / 51.5, 84.5 / 53.2; 18,944 x 3,584 55.4 / 55.0, 56.9 / 53.1, 61.7 / 53.2, 71.3 /
+    53.4; 28,672 x 8,192 187 / 173, 190 / 167, 202 / 167, 224 / 168: ahead wherever there is a workgroup for every compute unit, but
+    for one row of a long inner size where fewer than half of the units have a second one: 11,008 x 4,096 39.7 / 41.1 (40.3 / 39.4 at 4),
+    12,288 x 4,096 40.8 / 41.3.  With fewer workgroups it needs rows: 4,096 x 2,048 10.6 / 11.4, 10.7 / 11.5, 11.2 / 10.9, 11.9 / 11.0 and
+    14.1 / 12.1 at 24; 1,000 x 1,024 5.2 / 7.1, 5.4 / 7.3, 5.6 / 7.0, 6.0 / 6.7, 7.0 / 7.5 at 32 and 10.6 / 10.2 at 64."""
+    if inner % 64 != 0 or not 0 < rows <= GLU_STREAM_ROWS:
+        return False
+    groups = -(-outputs // 32)
+    if groups < 256:
+        return rows * inner >= 40_000
+    return rows > 1 or groups == 256 or groups > 384 or inner < 4096
 
 
 def rows_at_16_bytes(x: torch.Tensor) -> bool:
@@ -996,7 +1008,8 @@ def gemm_skinny_bf16(
     ``glu`` (with ``swiglu``): (limit, alpha); the gated epilogue is then min(gate, limit) *
     sigmoid(alpha * min(gate, limit)) * (clamp(up, -limit, limit) + 1).
     ``out_scale`` (with ``out_f32``): the 32-bit result is multiplied by it.
-    ``waves_k``, ``tiles``, ``staged``, ``tile_rows``, ``fold``: the kernel's own choices overridden (for measurements)."""
+    ``waves_k``, ``tiles``, ``staged``, ``tile_rows``, ``fold``: the kernel's own choices overridden (for measurements); 2 for ``staged``
+    is gate and up streamed, which ``glu_streams`` chooses."""
     _gpu(a, w, residual, emit_weight, bias)
     _check_bias(bias, w, "gemm_skinny")
     _need(a.dim() == 2 and a.stride(1) == 1 and a.dtype == torch.bfloat16, "gemm_skinny: A must be bfloat16 [M, K]")
@@ -1013,6 +1026,8 @@ def gemm_skinny_bf16(
         n //= 2
         n_out = n
         epi = EPI_SWIGLU
+        if staged < 0 and glu_streams(m, n, k):
+            staged = 2
         if glu == "gelu_tanh":  # gelu(gate) * up
             extra.glu_gelu = 1
             use_extra = True

@@ -140,8 +140,7 @@ class Linear:
             if self._fast(m, swiglu, out_f32) and (not swiglu or ops.rows_at_16_bytes(x) or m <= ops.skinny_rows(self.in_features, paired=True)):
                 return ops.gemm_skinny_bf16(x, w, residual=residual, out_f32=out_f32, swiglu=swiglu,
                                             prenorm=prenorm, norm_eps=eps, out=out, bias=bias, glu=glu if swiglu else None,
-                                            out_scale=out_scale,
-                                            staged=2 if swiglu and ops.glu_streams(m, self.total_out // 2, self.in_features) else -1)
+                                            out_scale=out_scale)
             # many rows: in tiles where these are ahead of the library's product (the gated form with silu in one kernel)
             direct = ops.gemm_library_direct(x, w)
             if direct and bias is None and not out_f32 and (glu is None or not swiglu) and x.stride(0) <= ops.TILES_LONGEST_STRIDE:
