@@ -105,6 +105,45 @@ def test_rotation_and_append(nq, nkv, d, page, tables):
     assert pages[0][0].count_nonzero() > 0
 
 
+@pytest.mark.parametrize("n,k", [(2048, 8192), (2048, 2048), (4096, 14336)])
+@pytest.mark.parametrize("m,size", [(3, 4), (5, 8), (9, 16), (11, 16), (17, 32), (33, 48), (39, 48), (65, 80), (113, 128)])
+def test_a_row_padded_to_a_recorded_size_keeps_its_bits(m, size, n, k):
+    """A decode step of m rows alone and padded to the size that it is recorded at: output or down projection with the norm behind
+    it, and the stacked q, k, v product, by one kernel, where both counts are few rows or split products."""
+    from tokasaurus_amd.parts.linear import Linear
+    from tokasaurus_amd.parts.norm import RMSNorm
+
+    x, w, gen = _case(size, n, k, size + n + k)
+    lin, norm = Linear(k, ["w"], [n]), RMSNorm(n, 1e-5, "n")
+    lin.weight, norm.weight = w, torch.ones((n,), dtype=torch.bfloat16, device="cuda")
+    residual = torch.randn((size, n), generator=gen, device="cuda").bfloat16()
+    (a, pa), (b, pb) = lin.with_residual(x[:m], residual[:m], norm), lin.with_residual(x, residual, norm)
+    assert torch.equal(a, b[:m])
+    assert (pa.data is None) == (pb.data is None)
+    for p, q in [(pa.normed, pb.normed)] if pa.data is None else [(pa.data.scaled, pb.data.scaled), (pa.data.sumsq, pb.data.sumsq)]:
+        assert torch.equal(p, q[:m])
+
+
+@pytest.mark.parametrize("m,size", [(3, 4), (5, 8), (9, 16), (11, 16), (17, 32), (33, 48), (113, 128)])
+def test_rotated_rows_padded_to_a_recorded_size_keep_their_bits(m, size):
+    from tokasaurus_amd.parts.linear import Linear
+
+    nq, nkv, d, page = 32, 8, 64, 16
+    x, w, gen = _case(size, (nq + 2 * nkv) * d, 2048, size)
+    lin = Linear(2048, ["w"], [(nq + 2 * nkv) * d])
+    lin.weight = w
+    cos, sin = ops.rope_table(1.0 / 10000 ** (torch.arange(0, d, 2, device="cuda").float() / d), 4 * page)
+    table = torch.randperm(size, generator=gen, device="cuda").to(torch.int32).view(size, 1)
+    out = []
+    for rows in (m, size):
+        positions = (torch.arange(rows, device="cuda") % page).to(torch.int32)
+        pages = [torch.zeros(shape(size, nkv, page, d), dtype=torch.bfloat16, device="cuda") for shape in (ops.key_pages_shape, ops.value_pages_shape)]
+        q = lin.rope_append(x[:rows], ops.RopeAppend(positions, torch.arange(rows, device="cuda", dtype=torch.int32), table, cos, sin, *pages, nq, nkv, d, page))
+        out.append((q, *(p[table[:m, 0].long()] for p in pages)))
+    assert torch.equal(out[0][0], out[1][0][:m])
+    assert torch.equal(out[0][1], out[1][1]) and torch.equal(out[0][2], out[1][2])
+
+
 def test_product_and_pass_in_one_call():
     """The bits of the two calls, and what they refuse is refused."""
     x, w, gen = _case(33, 256, 192, 5)

@@ -73,3 +73,25 @@ def test_a_prepared_norm_is_folded_into_the_product_with_the_rotation(calls):
     calls.clear()
     assert lin.rope_append(Normed(on_gpu(16, 2048), n, Prepared(None, n, on_gpu(16, 2048))), rope) is not None
     assert calls == ["tk_split_linear_rope_append"]
+
+
+def test_recorded_rows_are_those_that_decode_steps_are_padded_to():
+    from tokasaurus_amd.engine.runner import graph_buckets
+
+    sizes = graph_buckets(128, 16)
+    assert [ops.recorded_rows(m) for m in range(1, 129)] == [min(s for s in sizes if s >= m) for m in range(1, 129)]
+
+
+@pytest.mark.parametrize("outputs,inner", [(2048, 2048), (2048, 8192), (3072, 3072), (4096, 4096), (4096, 14336), (3072, 8192)])
+def test_a_decode_step_takes_the_same_products_alone_and_padded(calls, monkeypatch, outputs, inner):
+    """Among the engine's own products: where a count or the size it is padded to is the library's, nothing is asked."""
+    def made(m):
+        calls.clear()
+        linear(outputs, inner).with_residual(on_gpu(m, inner), on_gpu(m, outputs), norm(outputs))
+        linear(outputs, inner).rope_append(on_gpu(m, inner), _rope(m, outputs // 64 - 16, 8, 64))
+        return list(calls)
+
+    monkeypatch.setattr(ops, "load", lambda name: type("Lib", (), {"tk_gemm_skinny_parts": lambda self, *a: 4})())
+    for m in range(1, 129):
+        assert made(m) == made(ops.recorded_rows(m))
+    assert made(2)[0] == "tk_gemm_skinny_bf16" and made(128) == ["tk_split_linear_add_rmsnorm", "tk_split_linear_rope_append"]

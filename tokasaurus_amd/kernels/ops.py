@@ -902,6 +902,13 @@ def glu_rows(inner: int, outputs: int = 0) -> int:
     return GLU_STREAM_ROWS if inner <= 4096 and (rounds <= 1 or 8 * groups >= 7 * 256 * rounds) else GLU_STREAM_DEEP_ROWS
 
 
+def recorded_rows(rows: int) -> int:
+    """Rows that a decode step of ``rows`` rows has once it is padded to a recorded size (up to 128; ``engine.runner.graph_buckets`` with
+    its default step).  Few-row products choose by it between kernels that sum in different orders, so that a token's bits do
+    not depend on whether its step was replayed or run as it is."""
+    return 1 << (rows - 1).bit_length() if rows < 16 else -(-rows // 16) * 16
+
+
 @functools.lru_cache(maxsize=4096)
 def glu_streams(rows: int, outputs: int, inner: int) -> bool:
     """Whether gate and up (``outputs`` of each) of up to 64 rows stream through local memory instead of into the wavefronts' registers.
@@ -917,7 +924,7 @@ def glu_streams(rows: int, outputs: int, inner: int) -> bool:
         return False
     groups = -(-outputs // 32)
     if groups < 256:
-        return rows * inner >= 40_000
+        return recorded_rows(rows) * inner >= 40_000
     return rows > 1 or groups == 256 or groups > 384 or inner < 4096
 
 
@@ -1127,8 +1134,8 @@ SPLIT_TILE, SPLIT_STEP = 64, 64  # weight rows a workgroup, elements of K a step
 #   and 33.6 / 25.7 for the last)
 SPLIT_NORM_ELEMENTS = 48_000
 SPLIT_ROPE_ELEMENTS = 24_000
-# Elements of w from which: it pays below too (1,024 x 1,024 8.8 / 7.4 at 48 rows, 512 x 512 7.3 / 6.5 at 64), but little, and there a
-# step keeps one kernel, hence its bits, whether it is padded to a recorded size or not.
+# (the rows counted are those of the recorded size: recorded_rows).  Elements of w from which: it pays below too (1,024 x 1,024 8.8 /
+# 7.4 at 48 rows, 512 x 512 7.3 / 6.5 at 64), but little.
 SPLIT_WEIGHT_ELEMENTS = 1 << 20
 
 

@@ -172,8 +172,8 @@ class Linear:
 
     def _splits(self, x: torch.Tensor, least: int) -> bool:
         """Whether the product takes the form with K cut among workgroups (``ops.gemm_split``), for a pass behind it that adds
-        the cuts: from ``least`` elements of x on, where the weight-streaming kernel's reads of x show."""
-        return (self.bias is None and x.shape[0] * self.in_features >= least
+        the cuts: from ``least`` elements of x (padded to a recorded size) on, where the weight-streaming kernel's reads of x show."""
+        return (self.bias is None and ops.recorded_rows(x.shape[0]) * self.in_features >= least
                 and self.in_features * self.total_out >= ops.SPLIT_WEIGHT_ELEMENTS and ops.split_takes(x, self.weight))
 
     def with_residual(
@@ -183,8 +183,10 @@ class Linear:
         that will be applied to the result) needs so that it costs no kernel of its own."""
         fusable = emit_norm is not None and getattr(emit_norm, "fusable_rms", False)
         if fusable and residual.is_contiguous() and self._splits(x, ops.SPLIT_NORM_ELEMENTS) and ops.split_norm_takes(residual, emit_norm.weight):
-            # (few rows: the next product's operand is rounded once, as where the weight-streaming product emits it)
-            out, normed = ops.split_linear_add_rmsnorm(x, self.weight, residual, emit_norm.weight, emit_norm.eps, self._fast(x.shape[0]))
+            # (few rows, or as many as they are padded to: the next product's operand is rounded once, as where the weight-streaming
+            # product emits it)
+            few = ops.recorded_rows(ops.skinny_rows(self.in_features))
+            out, normed = ops.split_linear_add_rmsnorm(x, self.weight, residual, emit_norm.weight, emit_norm.eps, x.shape[0] <= few)
             return out, Prepared(None, emit_norm, normed)
         if fusable and self._fast(x.shape[0]):
             out, data = ops.gemm_skinny_bf16(x, self.weight, residual=residual, emit_weight=emit_norm.weight, bias=self.bias)
