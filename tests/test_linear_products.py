@@ -95,3 +95,18 @@ def test_a_decode_step_takes_the_same_products_alone_and_padded(calls, monkeypat
     for m in range(1, 129):
         assert made(m) == made(ops.recorded_rows(m))
     assert made(2)[0] == "tk_gemm_skinny_bf16" and made(128) == ["tk_split_linear_add_rmsnorm", "tk_split_linear_rope_append"]
+
+
+@pytest.mark.parametrize("field", ["cos", "sin", "kcache", "vcache"])
+def test_tables_and_pages_that_start_anywhere_are_not_refused(calls, field):
+    """16 rows go to the product that reads them one by one, 33 back to the caller, who rotates them one by one."""
+    lin = linear(3072, 2048)
+    for rows, aligned, moved in ((16, ["tk_split_linear_rope_append"], ["tk_gemm_skinny_bf16"]), (33, ["tk_split_linear_rope_append"], [])):
+        for want in (aligned, moved):
+            rope = _rope(rows, 32, 8, 64)
+            if want is moved:
+                old = getattr(rope, field)
+                setattr(rope, field, on_gpu(old.numel() + 4, dtype=old.dtype)[1 : old.numel() + 1].view(old.shape))
+            calls.clear()
+            assert (lin.rope_append(on_gpu(rows, 2048), rope) is None) == (not want)
+            assert calls == want

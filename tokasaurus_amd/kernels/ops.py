@@ -1161,6 +1161,17 @@ def split_norm_takes(residual: torch.Tensor, weight: torch.Tensor) -> bool:
     return residual.dtype == torch.bfloat16 and residual.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and residual.shape[1] % 8 == 0
 
 
+def split_rope_takes(r: RopeAppend) -> bool:
+    """Whether ``split_rope_append`` rotates and stores these: whole heads of a multiple of 8, tables and pages that start at multiples of
+    16 bytes."""
+    if r.head_dim % 8 or not (r.rotary_dim is None or r.rotary_dim == r.head_dim):
+        return False
+    starts = r.kcache.data_ptr() | r.vcache.data_ptr()
+    if r.cos is not None and r.sin is not None:
+        starts |= r.cos.data_ptr() | r.sin.data_ptr()
+    return starts % 16 == 0
+
+
 def gemm_split(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x [M <= 256, K] . w [N, K]^T in bfloat16 with K cut among workgroups: the cuts' 32-bit sums [cuts, M, N], which
     ``split_add_rmsnorm`` or ``split_rope_append`` adds in ascending order."""

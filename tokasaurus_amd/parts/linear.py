@@ -202,11 +202,10 @@ class Linear:
         append of k and v to the pages in its epilogue; returns q [M, nq*d], or None when
         that kernel does not take this case (the caller then does the steps one by one)."""
         m = (x.x if isinstance(x, Normed) else x).shape[0]
-        whole = rope.head_dim % 8 == 0 and (rope.rotary_dim is None or rope.rotary_dim == rope.head_dim)
         stream = x.x if isinstance(x, Normed) else x
         # (a norm that the product in front prepared is folded in below: its rows are not made for the split form)
         prepared = x.usable() if isinstance(x, Normed) else None
-        if whole and prepared is None and self._splits(stream, ops.SPLIT_ROPE_ELEMENTS):
+        if prepared is None and self._splits(stream, ops.SPLIT_ROPE_ELEMENTS) and ops.split_rope_takes(rope):
             rows = x.materialize() if isinstance(x, Normed) else x  # (a norm's rows lie as their stream does, or from their own start)
             if ops.split_takes(rows, self.weight):
                 return ops.split_linear_rope_append(rows, self.weight, rope)
