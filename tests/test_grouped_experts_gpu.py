@@ -59,9 +59,18 @@ def test_experts_in_tiles(tokens, experts, top, width, ff, form):
 @pytest.mark.parametrize("form", ["silu", "clamps", "on input"])
 def test_experts_in_pairs_of_tiles(monkeypatch, tokens, experts, top, width, ff, form):
     """One step of K, fewer than local memory holds, and more; outputs that end inside a block; no, one and several pairs."""
-    monkeypatch.setattr(ops, "EXPERT_PAIRS_FROM_ROWS", 1)
+    for least in ("ROWS", "WIDTH", "INNER", "WALK"):
+        monkeypatch.setattr(ops, f"EXPERT_PAIRS_FROM_{least}", 0)
     assert ops.experts_go_in_pairs_of_tiles(tokens * top, experts, width + 8, width, ff)
     test_experts_in_tiles(tokens, experts, top, width, ff, form)
+
+
+@pytest.mark.parametrize("pairs,experts,width,ff,wanted", [
+    (16384, 32, 2048, 1024, True), (15000, 32, 2048, 1024, False), (8000, 16, 2048, 2048, True), (6700, 16, 2048, 2048, False), (51200, 128, 2048, 768, True),
+    (38400, 128, 2048, 768, False), (67840, 64, 1024, 512, False), (3040, 8, 4096, 14336, True), (3680, 8, 4096, 1792, False), (5280, 8, 4096, 1792, True),
+    (51200, 128, 2048, 760, False), (51200, 128, 2056, 768, False)])
+def test_which_experts_go_in_pairs_of_tiles(pairs, experts, width, ff, wanted):
+    assert ops.experts_go_in_pairs_of_tiles(pairs, experts, width, width, ff) == wanted
 
 
 @pytest.mark.parametrize("tokens,top,experts", [(1, 1, 300), (13, 8, 256), (130, 1, 2), (129, 1, 1), (400, 3, 5), (64, 2, 64)])
@@ -82,10 +91,9 @@ def test_tiles_hold_every_choice(tokens, top, experts, spread):
     assert used == int((-(-count // ops.EXPERT_TILE)).sum()) <= s.max_tiles
     slot_pair, group = s.slot_pair.cpu().view(-1, ops.EXPERT_TILE), s.tile_group.cpu()
     assert sorted(slot_pair[slot_pair >= 0].tolist()) == list(range(pairs))
-    runs = s.runs.cpu().view(-1, 4).tolist()  # every used tile in one pair of its expert or alone
-    twos, ones = runs[1 : 1 + runs[0][0]], runs[1 + s.max_tiles // 2 :][: runs[0][1]]
-    mine = [(t + 2 * (i - first) + j, e) for i, (t, e, first, _) in enumerate(twos) for j in range(2)] + [(t, e) for t, e, _, _ in ones]
-    assert sorted(mine) == list(enumerate(group[:used].tolist()))
+    runs = s.runs.cpu().view(-1, 4).tolist()  # every used tile in one pair of its expert, the last one perhaps alone in it
+    mine = [(t + 2 * (i - first) + j, e) for i, (t, e, first, tiles) in enumerate(runs[1 : 1 + runs[0][0]]) for j in range(2) if 2 * (i - first) + j < tiles]
+    assert mine == list(enumerate(group[:used].tolist())) and runs[0][0] <= s.max_pairs
     for t in range(s.max_tiles):
         mine = slot_pair[t][slot_pair[t] >= 0].long()
         assert (t < used) == (mine.numel() > 0) and (ids.flatten()[mine] == group[t]).all()

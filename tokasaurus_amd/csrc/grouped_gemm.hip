@@ -332,19 +332,18 @@ __global__ __launch_bounds__(256, 3) void grouped_gemm_staged_kernel(GroupedArgs
 }
 
 // Experts of many rows: two neighbouring tiles of a group as one of 256 slots x 256 weight rows (in the gated form 128 of gate and
-// 128 of up), the odd last tile of a group 128 x 128 (gemm_tile.h).  The path from the L2 to a compute unit bounds these products,
-// and a tile of 256 x 256 asks for half as many bytes a product; pairs keep an expert's rows filled up to 128 and not to 256.
-// The single tiles have a launch of their own, whose sums fit the ordinary registers.
-// 32 experts of 2,048 x 1,024, 2,048 tokens x 8: gate and up 206 to 157 us for the pairs and 25 for the singles, down 114 to 78 and
-// 14 (with 512 rows for every expert 157 and 4.6, 78 and 4.6); 64 experts of 1,024 x 512, 8,192 tokens x 4: 107 and 30, 56 and 16.
-// Every tile 128 x 256, without pairs, took 185 and 105.  What is left is the weights' way from memory: the pairs' products of one
-// weight of 16,384 x 2,048 for 2,048 rows, as many of them, take 120 us.
+// 128 of up; gemm_tile.h), the odd last tile of a group as half of one.  The path from the L2 to a compute unit bounds these
+// products, and a tile of 256 x 256 asks for half as many bytes a product.
+// us by tiles of 128 x 128 / in pairs, gate and up and down, every expert 3, 4, 5 and 6 tiles: 32 experts of 2,048 x 1,024 147 / 140 and
+// 85 / 70, 184 / 142 and 110 / 73, 222 / 199 and 131 / 100, 260 / 203 and 155 / 105; 32 of 2,880 x 2,880 546 / 479 and 299 / 217 to
+// 1,048 / 717 and 546 / 347.  Odd tiles of 128 x 128 in a launch of their own read the experts' weights a second time: with 3 tiles 172
+// and 87 us for the first, with 5 234 and 118.
 template <class S, bool GLU>
-__device__ __forceinline__ void wide_tile(const GroupedArgs& a, char* smem, int g, int first, int n0) {
+__device__ __forceinline__ void wide_tile(const GroupedArgs& a, char* smem, int g, int first, int n0, int top) {  // top: the last slot
   constexpr int OUT = GLU ? S::BN / 2 : S::BN;
   static_assert(S::BM <= 256 && S::BM * S::BN * 2 + S::BM * 4 <= S::LDS, "");
   const int lane = threadIdx.x & (TK_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TK_WAVE);
-  const int wm = wave & 1, wn = wave >> 1, top = a.slots - 1;
+  const int wm = wave & 1, wn = wave >> 1;
   TileLoop<S, GLU> t;
   t.wave = wave;
   t.lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
@@ -393,13 +392,11 @@ __device__ __forceinline__ void wide_tile(const GroupedArgs& a, char* smem, int 
 #define WIDE_OUT(glu) ((glu) ? 128 : 256)
 #define WIDE_PAIRS (GS_TILES / 2)
 using PairShape = TileShape<4, 4, 2, 3>;
-using SingleShape = TileShape<2, 2, 5, 5>;
-// A pair of tiles or a single one, as a workgroup reads it: the group's first tile (a single: its own), the group, the number of the
-// group's first pair and how many it has.
+// A pair, as a workgroup reads it: the group's first tile, the group, the number of the group's first pair and how many tiles it has.
 struct TileRun {
-  int tile, group, first, count;
+  int tile, group, first, tiles;
 };
-// runs: the numbers of pairs and of single tiles (as TileRun's first two), the pairs, the single tiles
+// runs: the number of pairs (as the first's tile), then the pairs
 template <bool GLU>
 __global__ __launch_bounds__(256, 1) void grouped_gemm_pairs_kernel(GroupedArgs a, const TileRun* __restrict__ runs, int n_blocks) {
   extern __shared__ __align__(16) char smem[];
@@ -409,37 +406,23 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_pairs_kernel(GroupedArgs 
   const int some = item / n_blocks;
   const TileRun r = runs[1 + some];
   // the chunk of up to WIDE_PAIRS pairs of the group that the item lies in
-  const int chunk = r.first + (some - r.first) / WIDE_PAIRS * WIDE_PAIRS, len = min(WIDE_PAIRS, r.first + r.count - chunk);
+  const int chunk = r.first + (some - r.first) / WIDE_PAIRS * WIDE_PAIRS, len = min(WIDE_PAIRS, r.first + (r.tiles + 1) / 2 - chunk);
   const int off = item - chunk * n_blocks, pair = chunk + off % len;
-  wide_tile<PairShape, GLU>(a, smem, r.group, (r.tile + 2 * (pair - r.first)) * GS_M, off / len * WIDE_OUT(GLU));
+  wide_tile<PairShape, GLU>(a, smem, r.group, (r.tile + 2 * (pair - r.first)) * GS_M, off / len * WIDE_OUT(GLU), (r.tile + r.tiles) * GS_M - 1);
 }
 
 template <bool GLU>
-__global__ __launch_bounds__(256, 2) void grouped_gemm_singles_kernel(GroupedArgs a, const TileRun* __restrict__ runs, int max_pairs, int n_blocks) {
-  extern __shared__ __align__(16) char smem[];
-  const int items = runs->group * n_blocks, per = (items + GS_DIES - 1) / GS_DIES;
-  const int seq = blockIdx.x / GS_DIES, item = blockIdx.x % GS_DIES * per + seq;
-  if (seq >= per || item >= items) return;
-  const TileRun r = runs[1 + max_pairs + item / n_blocks];
-  wide_tile<SingleShape, GLU>(a, smem, r.group, r.tile * GS_M, item % n_blocks * (WIDE_OUT(GLU) / 2));
-}
-
-template <bool GLU>
-static bool launch_by_tile(const GroupedArgs& a, int tiles, const TileRun* runs, int max_singles, hipStream_t stream) {
+static bool launch_by_tile(const GroupedArgs& a, int tiles, const TileRun* runs, int max_pairs, hipStream_t stream) {
   const auto groups = [](long n) { return (n + GS_DIES - 1) / GS_DIES * GS_DIES; };
   const int outs = GLU ? 64 : 128, n_blocks = (a.N + outs - 1) / outs;
   if (runs) {
-    const int max_pairs = tiles / 2, wide_blocks = (a.N + WIDE_OUT(GLU) - 1) / WIDE_OUT(GLU);
-    const long pairs = groups((long)max_pairs * wide_blocks), singles = groups((long)max_singles * n_blocks);
-    static_assert(SingleShape::BM == GS_M && PairShape::BM == 2 * GS_M, "");
-    auto pair_kernel = grouped_gemm_pairs_kernel<GLU>;
-    auto single_kernel = grouped_gemm_singles_kernel<GLU>;
-    if (pairs + singles >= (1l << 31)
-        || hipFuncSetAttribute((const void*)pair_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PairShape::LDS) != hipSuccess
-        || hipFuncSetAttribute((const void*)single_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, SingleShape::LDS) != hipSuccess)
+    const int wide_blocks = (a.N + WIDE_OUT(GLU) - 1) / WIDE_OUT(GLU);
+    const long pairs = groups((long)max_pairs * wide_blocks);
+    static_assert(PairShape::BM == 2 * GS_M, "");
+    auto kernel = grouped_gemm_pairs_kernel<GLU>;
+    if (pairs >= (1l << 31) || hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PairShape::LDS) != hipSuccess)
       return false;
-    if (pairs > 0) hipLaunchKernelGGL(pair_kernel, dim3((unsigned)pairs), dim3(256), PairShape::LDS, stream, a, runs, wide_blocks);
-    hipLaunchKernelGGL(single_kernel, dim3((unsigned)singles), dim3(256), SingleShape::LDS, stream, a, runs, max_pairs, n_blocks);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)pairs), dim3(256), PairShape::LDS, stream, a, runs, wide_blocks);
     return true;
   }
   const long grid = groups((long)tiles * n_blocks);
@@ -451,7 +434,7 @@ static bool launch_by_tile(const GroupedArgs& a, int tiles, const TileRun* runs,
 
 TK_API int tk_grouped_gemm_bf16(const void* A, int lda, const int* a_row, const int* c_row, const int* tile_group, int tiles,
                                 int groups_z, int a_cols, int c_cols, const void* W, size_t w_stride, void* C, int ldc,
-                                int N, int K, int slots, const TileRun* runs, int max_singles, long a_rows, int glu, int out_f32, const float* row_scale, const int* scale_row,
+                                int N, int K, int slots, const TileRun* runs, int max_pairs, long a_rows, int glu, int out_f32, const float* row_scale, const int* scale_row,
                                 float limit, float alpha, hipStream_t stream) {
   TK_REQUIRE(A && W && C && N > 0 && K > 0 && slots >= 0 && tiles >= 0, "grouped_gemm: bad arguments");
   TK_REQUIRE(K % 8 == 0 && lda % 8 == 0 && a_cols % 8 == 0 && w_stride % 8 == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0,
@@ -464,9 +447,9 @@ TK_API int tk_grouped_gemm_bf16(const void* A, int lda, const int* a_row, const 
                 row_scale, scale_row, limit, alpha};
   if (tile_group) {
     TK_REQUIRE(!out_f32 && a_cols == 0 && c_cols == 0, "grouped_gemm: groups by tile write the storage type and have no columns of their own");
-    TK_REQUIRE(!runs || (((uintptr_t)runs & 15) == 0 && K % TILE_K == 0 && a_rows * lda * 2 < (1l << 32) && (glu ? 2l : 1l) * N * K * 2 < (1l << 32) && max_singles > 0),
+    TK_REQUIRE(!runs || (((uintptr_t)runs & 15) == 0 && K % TILE_K == 0 && a_rows * lda * 2 < (1l << 32) && (glu ? 2l : 1l) * N * K * 2 < (1l << 32) && max_pairs > 0),
                "grouped_gemm: pairs of tiles take whole steps of %d of K, and rows that 32-bit offsets reach", TILE_K);
-    TK_REQUIRE(glu ? launch_by_tile<true>(a, tiles, runs, max_singles, stream) : launch_by_tile<false>(a, tiles, runs, max_singles, stream), "grouped_gemm: too many outputs");
+    TK_REQUIRE(glu ? launch_by_tile<true>(a, tiles, runs, max_pairs, stream) : launch_by_tile<false>(a, tiles, runs, max_pairs, stream), "grouped_gemm: too many outputs");
     TK_CHECK_LAUNCH("grouped_gemm");
     return 0;
   }
@@ -493,8 +476,8 @@ TK_API int tk_grouped_gemm_bf16(const void* A, int lda, const int* a_row, const 
 struct SortJob {
   const int* ids;
   int *slot_pair, *slot_token, *tile_group;
-  TileRun* runs;  // (grouped_gemm_pairs_kernel: room for the numbers, max_tiles / 2 pairs and max_singles single tiles)
-  int pairs, top, experts, max_tiles, max_singles;
+  TileRun* runs;  // (grouped_gemm_pairs_kernel: room for the number and max_pairs pairs)
+  int pairs, top, experts, max_tiles, max_pairs;
 };
 #define SORT_JOBS 48
 struct SortJobs {
@@ -507,12 +490,10 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(SortJobs jobs) {
   int* __restrict__ slot_pair = jb.slot_pair;
   int* __restrict__ slot_token = jb.slot_token;
   int* __restrict__ tile_group = jb.tile_group;
-  extern __shared__ int sh[];  // [experts] each: counts (then the slots that are left), first slots, first single tiles
+  extern __shared__ int sh[];  // [experts] each: counts (then the slots that are left), first slots, first pairs of tiles
   int* count = sh;
   int* first = sh + experts;
-  int* first_single = sh + 2 * experts;
-  TileRun* run_of_pair = jb.runs + 1;
-  TileRun* run_of_single = run_of_pair + max_tiles / 2;
+  int* first_pair = sh + 2 * experts;
   for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = 0;
   for (int s = threadIdx.x; s < max_tiles * tm; s += blockDim.x) slot_pair[s] = slot_token[s] = -1;
   for (int t = threadIdx.x; t < max_tiles; t += blockDim.x) tile_group[t] = -1;
@@ -523,25 +504,22 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(SortJobs jobs) {
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    int at = 0, twos = 0, ones = 0;
+    int at = 0, twos = 0;
     for (int e = 0; e < experts; ++e) {
       const int n = (count[e] + tm - 1) / tm;
       first[e] = at;
-      first_single[e] = ones;
+      first_pair[e] = twos;
       at += n * tm;
-      twos += n / 2;
-      ones += n & 1;
+      twos += (n + 1) / 2;
     }
     tile_group[max_tiles] = at / tm;
-    jb.runs[0] = {twos, ones, 0, 0};
+    jb.runs[0] = {twos, 0, 0, 0};
   }
   __syncthreads();
   for (int e = threadIdx.x; e < experts; e += blockDim.x) {
     const int t0 = first[e] / tm, n = (count[e] + tm - 1) / tm;
-    const int first_pair = (t0 - first_single[e]) / 2;  // (the tiles in front are pairs of two and singles)
     for (int t = 0; t < n; ++t) tile_group[t0 + t] = e;
-    for (int p = 0; p < n / 2; ++p) run_of_pair[first_pair + p] = {t0, e, first_pair, n / 2};
-    if (n & 1) run_of_single[first_single[e]] = {t0 + n - 1, e, first_single[e], 1};
+    for (int p = 0; p < (n + 1) / 2; ++p) jb.runs[1 + first_pair[e] + p] = {t0, e, first_pair[e], n};
   }
   __syncthreads();
   for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
@@ -566,7 +544,7 @@ TK_API int tk_expert_sort(const SortJob* jobs, int n_jobs, hipStream_t stream) {
       // (each expert that has pairs leaves at most one tile partly empty)
       TK_REQUIRE(j.max_tiles >= (j.pairs + (long)(GS_M - 1) * min(j.experts, j.pairs)) / GS_M, "expert_sort: %d tiles cannot hold %d pairs of %d experts", j.max_tiles,
                  j.pairs, j.experts);
-      TK_REQUIRE(j.max_singles >= min(j.experts, j.max_tiles), "expert_sort: %d single tiles cannot hold those of %d experts", j.max_singles, j.experts);
+      TK_REQUIRE(j.max_pairs >= (j.max_tiles + min(j.experts, j.max_tiles)) / 2, "expert_sort: %d pairs cannot hold those of %d tiles", j.max_pairs, j.max_tiles);
       TK_REQUIRE(3 * j.experts * sizeof(int) <= 48 * 1024, "expert_sort: too many experts");
       most = max(most, j.experts);
     }

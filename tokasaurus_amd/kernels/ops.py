@@ -2631,7 +2631,7 @@ class _SortJob(ctypes.Structure):
 
     _fields_ = [("ids", ctypes.c_void_p), ("slot_pair", ctypes.c_void_p), ("slot_token", ctypes.c_void_p), ("tile_group", ctypes.c_void_p),
                 ("runs", ctypes.c_void_p), ("pairs", ctypes.c_int), ("top", ctypes.c_int), ("experts", ctypes.c_int), ("max_tiles", ctypes.c_int),
-                ("max_singles", ctypes.c_int)]
+                ("max_pairs", ctypes.c_int)]
 
 
 @dataclass
@@ -2641,9 +2641,9 @@ class SortedPairs:
     slot_pair: torch.Tensor
     slot_token: torch.Tensor
     tile_group: torch.Tensor
-    runs: torch.Tensor  # two neighbouring tiles of an expert each, and the odd last ones
+    runs: torch.Tensor  # how many pairs of neighbouring tiles there are, the odd last one of an expert alone, and the pairs
     max_tiles: int
-    max_singles: int
+    max_pairs: int
     shape: tuple  # of the ids
 
 
@@ -2661,12 +2661,12 @@ def expert_sort(choices: "list[tuple[torch.Tensor, int]]") -> "list[SortedPairs]
         n, top = ids.shape
         max_tiles = expert_tiles(n * top, int(experts))
         slots = max_tiles * EXPERT_TILE
-        singles, end = min(int(experts), max_tiles), 2 * slots + max_tiles + 1
+        max_pairs, end = (max_tiles + min(int(experts), max_tiles)) // 2, 2 * slots + max_tiles + 1
         at = -(-end // 4) * 4  # (a run is 16 bytes)
-        book = torch.empty((at + 4 * (1 + max_tiles // 2 + singles),), dtype=torch.int32, device=ids.device)
-        s = SortedPairs(book[:slots], book[slots : 2 * slots], book[2 * slots : end], book[at:], max_tiles, singles, (n, top))
+        book = torch.empty((at + 4 * (1 + max_pairs),), dtype=torch.int32, device=ids.device)
+        s = SortedPairs(book[:slots], book[slots : 2 * slots], book[2 * slots : end], book[at:], max_tiles, max_pairs, (n, top))
         job.ids, job.slot_pair, job.slot_token, job.tile_group, job.runs = (t.data_ptr() for t in (ids, s.slot_pair, s.slot_token, s.tile_group, s.runs))
-        job.pairs, job.top, job.experts, job.max_tiles, job.max_singles = n * top, top, int(experts), max_tiles, singles
+        job.pairs, job.top, job.experts, job.max_tiles, job.max_pairs = n * top, top, int(experts), max_tiles, max_pairs
         out.append(s)
     call("tk_expert_sort", ctypes.addressof(jobs), len(choices), _stream())
     return out
@@ -2680,18 +2680,28 @@ def experts_go_in_tiles(rows: int, top: int, dtype: torch.dtype, width: int, ff:
     return rows > GROUPED_FROM_ROWS and many and dtype == torch.bfloat16 and width % 8 == 0 and ff % 8 == 0
 
 
-# Rows an expert, on average, from which two neighbouring tiles of an expert are multiplied as one of 256 x 256: with fewer, too
-# many of the tiles are odd ones or nearly empty.  In us by single tiles / in pairs, both products and the sum: 32 experts of
-# 2,048 x 1,024, 256 rows an expert 227 / 201, 375 rows 268 / 260, 512 rows 360 / 298, 1,024 rows 659 / 517; 16 of 2,048 x 2,048, 256 rows
-# 211 / 215, 375 rows 274 / 233, 512 rows 360 / 273; 64 of 1,024 x 512, 256 rows 125 / 137, 512 rows 211 / 209; 128 of 2,048 x 768,
-# 187 rows 489 / 436, 256 rows 616 / 602, 512 rows 1,074 / 910.
+# Where two neighbouring tiles of an expert's rows are multiplied as one of 256 x 256 (grouped_gemm.hip): from so many rows an expert on
+# average, widths and inner sizes whose steps outweigh a tile's beginning and end, and so many elements of K that a compute unit walks in
+# gate and up: a round of pairs takes all units for one pair each, and a last round that is nearly empty costs as much as a full one.
+# In us by single tiles / in pairs, both products and the sum, experts' rows even, uneven (weights e^(0.5 N(0, 1))) and an eighth of the
+# experts 4.5 times as likely: 32 experts of 2,048 x 1,024, 420 rows an expert (4,380 elements) 276 / 221, 274 / 299, 276 / 296; 500
+# (5,020) 318 / 306, 316 / 304, 327 / 305; 700 425 / 329, 421 / 409, 445 / 405; 1,020 618 / 519, 610 / 518, 612 / 515.  16 of 2,048 x 2,048,
+# 420 rows 271 / 209, 267 / 295, 270 / 295; 500 308 / 302, 314 / 303, 309 / 303.  128 of 2,048 x 768, 220 rows 503 / 490, 527 / 532, 543 / 466;
+# 400 830 / 677, 808 / 738, 848 / 821.  8 of 4,096 x 1,792, 460 rows (4,110) 260 / 179, 263 / 214, 263 / 300; 660 381 / 307, 370 / 306, 342 /
+# 308.  8 of 4,096 x 14,336, 380 rows 1,668 / 1,130, 1,740 / 1,134, 1,696 / 1,439.  64 of 1,024 x 512, 500 rows 186 / 218, 1,060 372 / 374.
 EXPERT_PAIRS_FROM_ROWS = 320
+EXPERT_PAIRS_FROM_WIDTH = 2048
+EXPERT_PAIRS_FROM_INNER = 768
+EXPERT_PAIRS_FROM_WALK = 5_000
 
 
 def experts_go_in_pairs_of_tiles(pairs: int, experts: int, stride: int, width: int, ff: int) -> bool:
     """Whether two neighbouring tiles of an expert's rows are multiplied as one."""
+    if pairs < EXPERT_PAIRS_FROM_ROWS * experts or width < EXPERT_PAIRS_FROM_WIDTH or ff < EXPERT_PAIRS_FROM_INNER or width % 64 or ff % 64:
+        return False
     reach = 2 * max(pairs * max(stride, ff), 2 * ff * width) < 2 ** 32  # (the kernel's offsets are 32-bit bytes)
-    return pairs >= EXPERT_PAIRS_FROM_ROWS * experts and width % 64 == 0 and ff % 64 == 0 and reach
+    wide = pairs / (2 * EXPERT_TILE) + experts / 2  # pairs of tiles, half of the experts with an odd one
+    return reach and wide * -(-ff // 128) * width >= 256 * EXPERT_PAIRS_FROM_WALK
 
 
 def expert_mix(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor | None,
@@ -2733,15 +2743,15 @@ def expert_mix(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, i
             pairs = expert_sort([(ids, experts)])[0]
         _need(pairs.shape == (n, top), "expert_mix: pairs of another choice")
         slot_pair, slot_token, tile_group, max_tiles = pairs.slot_pair, pairs.slot_token, pairs.tile_group, pairs.max_tiles
-        slots, singles = max_tiles * EXPERT_TILE, pairs.max_singles
+        slots, wide_pairs = max_tiles * EXPERT_TILE, pairs.max_pairs
         wide = pairs.runs.data_ptr() if experts_go_in_pairs_of_tiles(n * top, experts, h.stride(0), width, ff) else None
         inter = torch.empty((n * top, ff), dtype=h.dtype, device=h.device)  # a row a pair: slots are many more where experts have few
         call("tk_grouped_gemm_bf16", h.data_ptr(), h.stride(0), slot_token.data_ptr(), slot_pair.data_ptr(), tile_group.data_ptr(), max_tiles, 0,
-             0, 0, w_gate_up.data_ptr(), 2 * ff * width, inter.data_ptr(), ff, ff, width, slots, wide, singles, n, 1, 0, on_input,
+             0, 0, w_gate_up.data_ptr(), 2 * ff * width, inter.data_ptr(), ff, ff, width, slots, wide, wide_pairs, n, 1, 0, on_input,
              slot_pair.data_ptr() if weights_on_input else None, limit, alpha, _stream())
         y = torch.empty((n * top, width), dtype=h.dtype, device=h.device)
         call("tk_grouped_gemm_bf16", inter.data_ptr(), ff, slot_pair.data_ptr(), slot_pair.data_ptr(), tile_group.data_ptr(), max_tiles, 0,
-             0, 0, w_down.data_ptr(), width * ff, y.data_ptr(), width, width, ff, slots, wide, singles, n * top, 0, 0, None, None, 0.0, 0.0, _stream())
+             0, 0, w_down.data_ptr(), width * ff, y.data_ptr(), width, width, ff, slots, wide, wide_pairs, n * top, 0, 0, None, None, 0.0, 0.0, _stream())
         call("tk_expert_sum", h.data_ptr(), h.stride(0), y.data_ptr(), ids.data_ptr(), weight_ptr,
              shared.data_ptr() if shared is not None else None, shared_gate.data_ptr() if shared is not None else None,
              out.data_ptr(), n, width, experts, top, unit, _stream())
