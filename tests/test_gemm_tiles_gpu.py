@@ -28,6 +28,18 @@ def test_against_64_bit_sums(shape, m, n, k):
     assert ((plain.cpu().double() - want).abs() <= want.abs() * 2.0 ** -8 + size * (k + 8) * 2.0 ** -23).all()
 
 
+@pytest.mark.parametrize("m", [1, 65, 127, 128, 129, 300])
+@pytest.mark.parametrize("n,k", [(8, 64), (32, 128), (72, 320), (520, 384), (1000, 448), (264, 1024)])
+def test_gated_tiles_of_64_weight_rows(m, n, k):
+    """Fewer steps of K than local memory holds, as many and more; outputs that end inside a tile of 32."""
+    from tokasaurus_amd.kernels import ops
+
+    x, w, _ = _case(m, n, k, 3 * m + n + k)
+    wide = torch.zeros((m, k + 8), dtype=torch.bfloat16)  # rows apart
+    wide[:, :k] = x
+    _check(ops.gemm_tiles_bf16(wide.cuda()[:, :k], w.cuda(), 5, glu=True), x.double(), w, _silu, k)
+
+
 @pytest.mark.parametrize("m,n,k,glu", [(65, 8192, 2048, True), (101, 8192, 2048, True), (1000, 2048, 1024, True), (1270, 3072, 512, False), (1800, 2048, 192, False)])
 def test_linear_takes_them(m, n, k, glu):
     """The rule's tiles through the linear map, and its other products."""

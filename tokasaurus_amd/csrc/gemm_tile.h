@@ -159,7 +159,7 @@ struct TileLoop {
   // (null: none), columns n0 .. of N; value(gate's sum, up's sum, m) in the gated form.
   template <class Value, class Dst>
   __device__ __forceinline__ void deliver(char* smem, int wm, int wn, int lane, int n0, int N, Value value, Dst dst) {
-    constexpr int OUT = GLU ? S::BN / 2 : S::BN, PIECES = OUT / 8, MASK = PIECES % 16 == 0 ? 15 : 7;
+    constexpr int OUT = GLU ? S::BN / 2 : S::BN, PIECES = OUT / 8, MASK = PIECES % 16 == 0 ? 15 : (PIECES % 8 == 0 ? 7 : 3);
     bf16_t* rows = (bf16_t*)smem;
     const int r = lane & 15, q = lane >> 4;
     __syncthreads();

@@ -1334,8 +1334,8 @@ def gemm_library_bf16(x: torch.Tensor, w: torch.Tensor, out_f32: bool = False, o
 
 # The tiles of gemm_tiles.hip: rows of A, rows of W, and the us that a step of 64 elements of K takes and that a tile's beginning and end
 # add (fitted to 234 products of 13 weights at 129 to 8,192 rows, weights from memory; the tile that comes out fastest by them is the
-# fastest measured one in 218)
-TILE_SHAPES = ((128, 128, 0.47, 4.3), (192, 128, 0.54, 6.5), (128, 256, 0.79, 5.5), (192, 256, 0.96, 11.2), (256, 256, 1.19, 15.5))
+# fastest measured one in 218); the last is for gate and up of up to 128 rows
+TILE_SHAPES = ((128, 128, 0.47, 4.3), (192, 128, 0.54, 6.5), (128, 256, 0.79, 5.5), (192, 256, 0.96, 11.2), (256, 256, 1.19, 15.5), (128, 64, 0.38, 4.0))
 TILES_LONGEST_STRIDE = 1 << 22  # elements between rows of x (a tile's rows lie within 32-bit bytes of its first)
 GLU_TILES_FROM_ROWS = 65  # (up to 64 rows gate and up stream through local memory)
 # two rounds of tiles of 256 x 256: with more the chip's power bounds the step, and the library's kernel needs less of it (a prompt of
@@ -1352,6 +1352,11 @@ def tiles_choice(m: int, n: int, k: int, glu: bool = False) -> int:
     units' rounds, up to ``GLU_TILES_MOST_SUMS``.  us library and pass / tiles, weights from memory: 16,384 x 2,048 33.5 / 26.4 at 256 rows, 41.7 / 37.7 at 512, 70.1 /
     61.3 at 1,024, 98.7 / 94.9 at 1,500, 117 / 120 at 2,048; 16,384 x 3,072 45.1 / 37.8 at 256, 92.0 / 81.6 at 1,024, 172 / 165 at 2,048;
     28,672 x 4,096 105 / 102 at 512, 204 / 194 at 1,024 (fill 0.73: 262 / 279 at 1,280).
+    Up to 128 rows, at 65 and 128: tiles of 64 weight rows where one round holds them, 16,384 x 2,048 21.7 / 19.1 and 23.9 / 20.9 (of 128
+    weight rows, half of the units, 23.1 and 26.7), 16,384 x 3,072 29.0 / 25.9 and 30.5 / 29.3, 16,384 x 8,192 66.7 / 62.8 and 68.7 / 66.1; wider
+    weights tiles of 128, which there pay from two thirds of the units on, 22,016 x 2,048 27.5 / 24.9 and 29.9 / 28.0, 22,016 x 4,096 46.9 / 44.9
+    and 47.1 / 48.0, 24,576 x 4,096 51.9 / 45.7 and 50.6 / 48.8, 28,672 x 4,096 58.6 / 55.2 and 57.6 / 56.2 (20,480 x 2,560, fill 0.63, 36.4 / 36.1
+    and 34.6 / 37.5).
     A plain product in tiles is ahead of the library's where one round of tiles of 128 outputs fills the chip and the library's
     larger tiles do not: 3,072 x 8,192 71.8 / 65.0 at 1,280 rows, 90.4 / 78.9 at 1,792; 5,120 x 3,072 40.1 / 35.2 at 1,024; 4,096 x 4,096
     47.4 / 43.9 at 1,280; not where a tile of 128 x 128 leaves more than a sixth of it idle (2,048 x 8,192 55.6 / 62.0 at 1,500
@@ -1361,14 +1366,14 @@ def tiles_choice(m: int, n: int, k: int, glu: bool = False) -> int:
     if k % 64 or n % 8 or (256 + 2 * n if glu else 256) * k >= 2 ** 31:
         return -1
     best, shape, fill, rounds = math.inf, 0, 0.0, 0
-    for i, (rows, cols, step, ends) in enumerate(TILE_SHAPES):
+    for i, (rows, cols, step, ends) in enumerate(TILE_SHAPES if glu and m <= 128 else TILE_SHAPES[:5]):
         tiles = -(-m // rows) * -(-(2 * n if glu else n) // cols)
         turns = -(-tiles // 256)
         cost = turns * (step * (k // 64) + ends)
         if cost < best:
             best, shape, fill, rounds = cost, i, tiles / (256 * turns), turns
     if glu:
-        return shape if m >= GLU_TILES_FROM_ROWS and (fill >= 0.8 or m <= 128 and fill >= 0.5) and m * 2 * n <= GLU_TILES_MOST_SUMS else -1
+        return shape if m >= GLU_TILES_FROM_ROWS and fill >= (0.65 if m <= 128 else 0.8) and m * 2 * n <= GLU_TILES_MOST_SUMS else -1
     least = (0.84, 0.75, 0.84 if k >= 8192 else 2.0, 2.0, 2.0)[shape]
     return shape if rounds == 1 and fill >= least else -1
 
