@@ -110,3 +110,15 @@ def test_tables_and_pages_that_start_anywhere_are_not_refused(calls, field):
             calls.clear()
             assert (lin.rope_append(on_gpu(rows, 2048), rope) is None) == (not want)
             assert calls == want
+
+
+@pytest.mark.parametrize("m,n,k,shape", [
+    (64, 8192, 2048, -1), (65, 8192, 2048, 5), (128, 8192, 2048, 5), (129, 8192, 2048, 0), (256, 8192, 2048, 0), (257, 8192, 2048, 1), (1024, 8192, 2048, 4),
+    # more than one round: only whole ones, up to two of 192 x 256
+    (1280, 8192, 2048, -1), (1408, 8192, 2048, 3), (1536, 8192, 2048, 3), (1664, 8192, 2048, -1), (2048, 8192, 2048, -1), (512, 14336, 4096, 4),
+    (640, 14336, 4096, -1), (1024, 14336, 4096, -1),
+    # up to 128 rows: two thirds of the units
+    (128, 11008, 4096, 0), (128, 10240, 2560, -1), (129, 11008, 4096, -1), (128, 4096, 2048, -1), (200, 4096, 2048, -1)])
+def test_which_tile_gate_and_up_take(m, n, k, shape):
+    assert ops.tiles_choice(m, n, k, True) == shape
+    assert ops.tiles_choice(m, n, k - 8, True) == -1

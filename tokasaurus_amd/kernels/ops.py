@@ -1338,9 +1338,9 @@ def gemm_library_bf16(x: torch.Tensor, w: torch.Tensor, out_f32: bool = False, o
 TILE_SHAPES = ((128, 128, 0.47, 4.3), (192, 128, 0.54, 6.5), (128, 256, 0.79, 5.5), (192, 256, 0.96, 11.2), (256, 256, 1.19, 15.5), (128, 64, 0.38, 4.0))
 TILES_LONGEST_STRIDE = 1 << 22  # elements between rows of x (a tile's rows lie within 32-bit bytes of its first)
 GLU_TILES_FROM_ROWS = 65  # (up to 64 rows gate and up stream through local memory)
-# two rounds of tiles of 256 x 256: with more the chip's power bounds the step, and the library's kernel needs less of it (a prompt of
-# 2,048 tokens of the 1B shape 5,027 to 4,984 us with the tiles, four of 1,024 of the 8B shape 43.3 to 44.6 ms)
-GLU_TILES_MOST_SUMS = 2 * 256 * 256 * 256
+# two rounds of tiles of 192 x 256: with more the chip's power bounds the step, and the library's kernel needs less of it
+GLU_TILES_MOST_SUMS = 2 * 256 * 192 * 256
+GLU_TILES_LATER_FILL = 0.95  # how much of its rounds a product fills that takes more than one
 
 
 @functools.lru_cache(maxsize=4096)
@@ -1348,10 +1348,13 @@ def tiles_choice(m: int, n: int, k: int, glu: bool = False) -> int:
     """Which tile (of ``TILE_SHAPES``) a product of ``m`` rows and ``n`` outputs takes, or with ``glu`` of ``n`` of gate and as many of up;
     -1: the library's product is faster.
 
-    In the gated form the tiles save the pass behind the library's product; they pay where they fill four fifths of the compute
-    units' rounds, up to ``GLU_TILES_MOST_SUMS``.  us library and pass / tiles, weights from memory: 16,384 x 2,048 33.5 / 26.4 at 256 rows, 41.7 / 37.7 at 512, 70.1 /
+    In the gated form the tiles save the pass behind the library's product; they pay where they fill four fifths of one round of
+    the compute units, or further rounds whole, up to ``GLU_TILES_MOST_SUMS``.  us library and pass / tiles, weights from memory: 16,384 x 2,048 33.5 / 26.4 at 256 rows, 41.7 / 37.7 at 512, 70.1 /
     61.3 at 1,024, 98.7 / 94.9 at 1,500, 117 / 120 at 2,048; 16,384 x 3,072 45.1 / 37.8 at 256, 92.0 / 81.6 at 1,024, 172 / 165 at 2,048;
-    28,672 x 4,096 105 / 102 at 512, 204 / 194 at 1,024 (fill 0.73: 262 / 279 at 1,280).
+    28,672 x 4,096 105 / 102 at 512, 204 / 194 at 1,024 (fill 0.73: 262 / 279 at 1,280).  In whole steps, where power counts, us a layer that
+    tiles save on two machines: one round, 16,384 x 2,048 15 and 16 at 512 rows, 16,384 x 3,072 9 and 5 at 1,024, 28,672 x 4,096 9 and 3 at 512;
+    two rounds filled whole, 16,384 x 2,048 -0.4 and 1.0 at 1,408, -1.2 and 2.9 at 1,536 (in another model 7 and 7), but -1.7 and -5.6 at
+    2,048; filled to 0.88, 16,384 x 2,048 -6.2 and -8.9 at 1,280, -5.9 and -9.4 at 1,664, 28,672 x 4,096 -13 and -18 at 640, -4.4 and -9.2 at 896.
     Up to 128 rows, at 65 and 128: tiles of 64 weight rows where one round holds them, 16,384 x 2,048 21.7 / 19.1 and 23.9 / 20.9 (of 128
     weight rows, half of the units, 23.1 and 26.7), 16,384 x 3,072 29.0 / 25.9 and 30.5 / 29.3, 16,384 x 8,192 66.7 / 62.8 and 68.7 / 66.1; wider
     weights tiles of 128, which there pay from two thirds of the units on, 22,016 x 2,048 27.5 / 24.9 and 29.9 / 28.0, 22,016 x 4,096 46.9 / 44.9
@@ -1373,7 +1376,8 @@ def tiles_choice(m: int, n: int, k: int, glu: bool = False) -> int:
         if cost < best:
             best, shape, fill, rounds = cost, i, tiles / (256 * turns), turns
     if glu:
-        return shape if m >= GLU_TILES_FROM_ROWS and fill >= (0.65 if m <= 128 else 0.8) and m * 2 * n <= GLU_TILES_MOST_SUMS else -1
+        least = GLU_TILES_LATER_FILL if rounds > 1 else (0.65 if m <= 128 else 0.8)
+        return shape if m >= GLU_TILES_FROM_ROWS and fill >= least and m * 2 * n <= GLU_TILES_MOST_SUMS else -1
     least = (0.84, 0.75, 0.84 if k >= 8192 else 2.0, 2.0, 2.0)[shape]
     return shape if rounds == 1 and fill >= least else -1
 
