@@ -122,3 +122,9 @@ def test_tables_and_pages_that_start_anywhere_are_not_refused(calls, field):
 def test_which_tile_gate_and_up_take(m, n, k, shape):
     assert ops.tiles_choice(m, n, k, True) == shape
     assert ops.tiles_choice(m, n, k - 8, True) == -1
+
+
+@pytest.mark.parametrize("m,n,k,shape", [(20, 28672, 4096, -1), (128, 32768, 1024, -1), (129, 32768, 1024, 1), (1280, 3072, 8192, 0), (1800, 2048, 192, 0),
+                                         (1500, 2048, 8192, -1), (2048, 4096, 14336, 2), (2048, 4096, 4096, -1), (8192, 2048, 8192, -1)])
+def test_which_tile_a_plain_product_takes(m, n, k, shape):
+    assert ops.tiles_choice(m, n, k) == shape

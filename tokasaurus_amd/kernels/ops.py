@@ -1337,6 +1337,7 @@ def gemm_library_bf16(x: torch.Tensor, w: torch.Tensor, out_f32: bool = False, o
 # fastest measured one in 218); the last is for gate and up of up to 128 rows
 TILE_SHAPES = ((128, 128, 0.47, 4.3), (192, 128, 0.54, 6.5), (128, 256, 0.79, 5.5), (192, 256, 0.96, 11.2), (256, 256, 1.19, 15.5), (128, 64, 0.38, 4.0))
 TILES_LONGEST_STRIDE = 1 << 22  # elements between rows of x (a tile's rows lie within 32-bit bytes of its first)
+PLAIN_TILES_FROM_ROWS = 129  # (where the fit begins)
 GLU_TILES_FROM_ROWS = 65  # (up to 64 rows gate and up stream through local memory)
 # two rounds of tiles of 192 x 256: with more the chip's power bounds the step, and the library's kernel needs less of it
 GLU_TILES_MOST_SUMS = 2 * 256 * 192 * 256
@@ -1361,9 +1362,10 @@ def tiles_choice(m: int, n: int, k: int, glu: bool = False) -> int:
     and 47.1 / 48.0, 24,576 x 4,096 51.9 / 45.7 and 50.6 / 48.8, 28,672 x 4,096 58.6 / 55.2 and 57.6 / 56.2 (20,480 x 2,560, fill 0.63, 36.4 / 36.1
     and 34.6 / 37.5).
     A plain product in tiles is ahead of the library's where one round of tiles of 128 outputs fills the chip and the library's
-    larger tiles do not: 3,072 x 8,192 71.8 / 65.0 at 1,280 rows, 90.4 / 78.9 at 1,792; 5,120 x 3,072 40.1 / 35.2 at 1,024; 4,096 x 4,096
-    47.4 / 43.9 at 1,280; not where a tile of 128 x 128 leaves more than a sixth of it idle (2,048 x 8,192 55.6 / 62.0 at 1,500
-    rows, fill 0.75; 4,096 x 4,096 33.3 / 38.5 at 768), tiles of 192 rows a quarter (3,072 x 8,192 85.3 / 76.8 at 1,500, fill 0.75); tiles of
+    larger tiles do not, from 129 rows on (below the two are even, 32,000 x 2,048 31.6 / 32.6 at 96 rows, 28,672 x 4,096 54.3 / 55.2 and 27,648
+    x 1,024 17.8 / 16.9 at 128, and steps are the library's): 3,072 x 8,192 71.8 / 65.0 at 1,280 rows, 90.4 / 78.9 at 1,792; 5,120 x 3,072 40.1 / 35.2 at 1,024; 4,096 x 4,096
+    47.4 / 43.9 at 1,280; not where tiles of 128 x 128 fill less than 0.84 of it (2,048 x 8,192 55.6 / 62.0 at 1,500
+    rows, fill 0.75; 4,096 x 4,096 33.3 / 38.5 at 768; between 0.75 and 0.84 nothing was measured), tiles of 192 rows less than 0.75 (3,072 x 8,192 85.3 / 76.8 at 1,500, fill 0.75); tiles of
     128 x 256 only pay over a long inner size (4,096 x 14,336 203 / 187 at 2,048 rows, 4,096 x 4,096 58.3 / 58.6), larger ones
     not (2,048 x 8,192 171 / 184 at 8,192 rows)."""
     if k % 64 or n % 8 or (256 + 2 * n if glu else 256) * k >= 2 ** 31:
@@ -1379,7 +1381,7 @@ def tiles_choice(m: int, n: int, k: int, glu: bool = False) -> int:
         least = GLU_TILES_LATER_FILL if rounds > 1 else (0.65 if m <= 128 else 0.8)
         return shape if m >= GLU_TILES_FROM_ROWS and fill >= least and m * 2 * n <= GLU_TILES_MOST_SUMS else -1
     least = (0.84, 0.75, 0.84 if k >= 8192 else 2.0, 2.0, 2.0)[shape]
-    return shape if rounds == 1 and fill >= least else -1
+    return shape if m >= PLAIN_TILES_FROM_ROWS and rounds == 1 and fill >= least else -1
 
 
 def gemm_tiles_bf16(x: torch.Tensor, w: torch.Tensor, shape: int, glu: bool = False) -> torch.Tensor:
