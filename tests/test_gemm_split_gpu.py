@@ -77,7 +77,7 @@ def test_few_rows_are_rounded_once_behind_a_linear_map(rows, n, k):
     x, w, gen = _case(rows, n, k, rows + n)
     lin, norm = Linear(k, ["w"], [n]), RMSNorm(n, 1e-5, "n")
     lin.weight, norm.weight = w, (1 + 0.1 * torch.randn((n,), generator=gen, device="cuda")).bfloat16()
-    assert rows <= ops.skinny_rows(k) and lin._splits(x, ops.SPLIT_NORM_ELEMENTS)
+    assert lin.split_norm_from <= rows <= ops.skinny_rows(k)
     stream, prepared = lin.with_residual(x, torch.randn((rows, n), generator=gen, device="cuda").bfloat16(), norm)
     s = stream.double()
     want = s / torch.sqrt((s * s).mean(1, keepdim=True) + 1e-5) * norm.weight.double()

@@ -1139,6 +1139,14 @@ SPLIT_ROPE_ELEMENTS = 24_000
 SPLIT_WEIGHT_ELEMENTS = 1 << 20
 
 
+def split_from_rows(inner: int, outputs: int, elements: int) -> int:
+    """Rows from which a weight of these sizes takes the split product for a pass behind it that adds the cuts: those that have
+    ``elements`` elements once they are padded to a recorded size (more than ``SPLIT_ROWS``: never)."""
+    if inner * outputs < SPLIT_WEIGHT_ELEMENTS:
+        return SPLIT_ROWS + 1
+    return next((m for m in range(1, SPLIT_ROWS + 1) if recorded_rows(m) * inner >= elements), SPLIT_ROWS + 1)
+
+
 @functools.lru_cache(maxsize=None)
 def split_cuts(n: int, k: int, m: int = 1) -> int:
     """Cuts of K for a weight [n, k] and ``m`` rows: the fewest for which the 256 compute units' rounds of workgroups are filled to nine tenths,
@@ -2652,10 +2660,16 @@ class SortedPairs:
     slot_pair: torch.Tensor
     slot_token: torch.Tensor
     tile_group: torch.Tensor
-    runs: torch.Tensor  # how many pairs of neighbouring tiles there are, the odd last one of an expert alone, and the pairs
+    book: torch.Tensor  # all of it, from `runs_at` on
+    runs_at: int
     max_tiles: int
     max_pairs: int
     shape: tuple  # of the ids
+
+    @property
+    def runs(self) -> torch.Tensor:
+        """How many pairs of neighbouring tiles there are, the odd last tile of an expert alone in one, and the pairs."""
+        return self.book[self.runs_at :]
 
 
 def expert_tiles(pairs: int, experts: int) -> int:
@@ -2675,8 +2689,9 @@ def expert_sort(choices: "list[tuple[torch.Tensor, int]]") -> "list[SortedPairs]
         max_pairs, end = (max_tiles + min(int(experts), max_tiles)) // 2, 2 * slots + max_tiles + 1
         at = -(-end // 4) * 4  # (a run is 16 bytes)
         book = torch.empty((at + 4 * (1 + max_pairs),), dtype=torch.int32, device=ids.device)
-        s = SortedPairs(book[:slots], book[slots : 2 * slots], book[2 * slots : end], book[at:], max_tiles, max_pairs, (n, top))
-        job.ids, job.slot_pair, job.slot_token, job.tile_group, job.runs = (t.data_ptr() for t in (ids, s.slot_pair, s.slot_token, s.tile_group, s.runs))
+        s = SortedPairs(book[:slots], book[slots : 2 * slots], book[2 * slots : end], book, at, max_tiles, max_pairs, (n, top))
+        start = book.data_ptr()  # (4 bytes a number)
+        job.ids, job.slot_pair, job.slot_token, job.tile_group, job.runs = ids.data_ptr(), start, start + 4 * slots, start + 8 * slots, start + 4 * at
         job.pairs, job.top, job.experts, job.max_tiles, job.max_pairs = n * top, top, int(experts), max_tiles, max_pairs
         out.append(s)
     call("tk_expert_sort", ctypes.addressof(jobs), len(choices), _stream())

@@ -57,6 +57,9 @@ class Linear:
         self.bias_names = list(bias_names) if bias_names and any(bias_names) else None
         assert self.bias_names is None or len(self.bias_names) == len(names)
         self.bias: torch.Tensor | None = None
+        # rows from which the split product is taken (counted once: few calls of a step reach them)
+        self.split_norm_from = ops.split_from_rows(in_features, self.total_out, ops.SPLIT_NORM_ELEMENTS)
+        self.split_rope_from = ops.split_from_rows(in_features, self.total_out, ops.SPLIT_ROPE_ELEMENTS)
 
     def tensor_specs(self) -> list[TensorSpec]:
         specs = [TensorSpec(n, (o, self.in_features), MATRIX) for n, o in zip(self.names, self.out_features)]
@@ -143,9 +146,10 @@ class Linear:
                                             out_scale=out_scale)
             # many rows: in tiles where these are ahead of the library's product (the gated form with silu in one kernel)
             direct = ops.gemm_library_direct(x, w)
-            if direct and bias is None and not out_f32 and (glu is None or not swiglu) and x.stride(0) <= ops.TILES_LONGEST_STRIDE:
+            if (m >= (ops.GLU_TILES_FROM_ROWS if swiglu else ops.PLAIN_TILES_FROM_ROWS) and not out_f32 and bias is None and direct
+                    and (glu is None or not swiglu)):
                 shape = ops.tiles_choice(m, w.shape[0] // 2 if swiglu else w.shape[0], self.in_features, swiglu)
-                if shape >= 0:
+                if shape >= 0 and x.stride(0) <= ops.TILES_LONGEST_STRIDE:
                     prod = ops.gemm_tiles_bf16(x, w, shape, swiglu)
                     return ops.add(prod, residual.contiguous()) if residual is not None else prod
             # library matrix product (hipBLASLt), 32-bit accumulation; with a bias through the tensor
@@ -170,28 +174,24 @@ class Linear:
         prod = ops.gemm_generic(x, w, residual=residual, out_f32=out_f32, out=out, bias=bias)
         return gated(prod) if swiglu else scaled(prod)
 
-    def _splits(self, x: torch.Tensor, least: int) -> bool:
-        """Whether the product takes the form with K cut among workgroups (``ops.gemm_split``), for a pass behind it that adds
-        the cuts: from ``least`` elements of x (padded to a recorded size) on, where the weight-streaming kernel's reads of x show."""
-        return (self.bias is None and ops.recorded_rows(x.shape[0]) * self.in_features >= least
-                and self.in_features * self.total_out >= ops.SPLIT_WEIGHT_ELEMENTS and ops.split_takes(x, self.weight))
-
     def with_residual(
         self, x: torch.Tensor, residual: torch.Tensor, emit_norm: Norm | None
     ) -> tuple[torch.Tensor, Prepared | None]:
         """residual + product and, where the kernel can, what ``emit_norm`` (the norm
         that will be applied to the result) needs so that it costs no kernel of its own."""
+        m = x.shape[0]
         fusable = emit_norm is not None and getattr(emit_norm, "fusable_rms", False)
-        if fusable and residual.is_contiguous() and self._splits(x, ops.SPLIT_NORM_ELEMENTS) and ops.split_norm_takes(residual, emit_norm.weight):
+        if (fusable and self.split_norm_from <= m <= ops.SPLIT_ROWS and self.bias is None and ops.split_takes(x, self.weight)
+                and residual.is_contiguous() and ops.split_norm_takes(residual, emit_norm.weight)):
             # (few rows, or as many as they are padded to: the next product's operand is rounded once, as where the weight-streaming
             # product emits it)
             few = ops.recorded_rows(ops.skinny_rows(self.in_features))
-            out, normed = ops.split_linear_add_rmsnorm(x, self.weight, residual, emit_norm.weight, emit_norm.eps, x.shape[0] <= few)
+            out, normed = ops.split_linear_add_rmsnorm(x, self.weight, residual, emit_norm.weight, emit_norm.eps, m <= few)
             return out, Prepared(None, emit_norm, normed)
-        if fusable and self._fast(x.shape[0]):
+        if fusable and self._fast(m):
             out, data = ops.gemm_skinny_bf16(x, self.weight, residual=residual, emit_weight=emit_norm.weight, bias=self.bias)
             return out, Prepared(data, emit_norm)
-        if fusable and x.shape[0] > 0:
+        if fusable and m > 0:
             # one pass adds the residual and norms the sum
             out, normed = ops.add_rmsnorm(self(x), residual.contiguous(), emit_norm.weight, emit_norm.eps)
             return out, Prepared(None, emit_norm, normed)
@@ -201,11 +201,11 @@ class Linear:
         """For a stacked [q | k | v] weight: the product with the rotation of q and k and the
         append of k and v to the pages in its epilogue; returns q [M, nq*d], or None when
         that kernel does not take this case (the caller then does the steps one by one)."""
-        m = (x.x if isinstance(x, Normed) else x).shape[0]
         stream = x.x if isinstance(x, Normed) else x
+        m = stream.shape[0]
         # (a norm that the product in front prepared is folded in below: its rows are not made for the split form)
-        prepared = x.usable() if isinstance(x, Normed) else None
-        if prepared is None and self._splits(stream, ops.SPLIT_ROPE_ELEMENTS) and ops.split_rope_takes(rope):
+        if (self.split_rope_from <= m <= ops.SPLIT_ROWS and self.bias is None and ops.split_takes(stream, self.weight)
+                and not (isinstance(x, Normed) and x.usable()) and ops.split_rope_takes(rope)):
             rows = x.materialize() if isinstance(x, Normed) else x  # (a norm's rows lie as their stream does, or from their own start)
             if ops.split_takes(rows, self.weight):
                 return ops.split_linear_rope_append(rows, self.weight, rope)
@@ -216,6 +216,7 @@ class Linear:
             return None
         prenorm, eps = None, 0.0
         if isinstance(x, Normed):
+            prepared = x.usable()
             if prepared is not None:
                 prenorm, eps, x = prepared.data, x.norm.eps, prepared.data.scaled
             else:
