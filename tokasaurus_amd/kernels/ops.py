@@ -1142,7 +1142,7 @@ SPLIT_WEIGHT_ELEMENTS = 1 << 20
 def split_from_rows(inner: int, outputs: int, elements: int) -> int:
     """Rows from which a weight of these sizes takes the split product for a pass behind it that adds the cuts: those that have
     ``elements`` elements once they are padded to a recorded size (more than ``SPLIT_ROWS``: never)."""
-    if inner * outputs < SPLIT_WEIGHT_ELEMENTS:
+    if inner * outputs < SPLIT_WEIGHT_ELEMENTS or inner % SPLIT_STEP or outputs % 8:
         return SPLIT_ROWS + 1
     return next((m for m in range(1, SPLIT_ROWS + 1) if recorded_rows(m) * inner >= elements), SPLIT_ROWS + 1)
 
@@ -1167,17 +1167,6 @@ def split_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
 def split_norm_takes(residual: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether ``split_add_rmsnorm`` reads these: rows and a weight that start at multiples of 16 bytes."""
     return residual.dtype == torch.bfloat16 and residual.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and residual.shape[1] % 8 == 0
-
-
-def split_rope_takes(r: RopeAppend) -> bool:
-    """Whether ``split_rope_append`` rotates and stores these: whole heads of a multiple of 8, tables and pages that start at multiples of
-    16 bytes."""
-    if r.head_dim % 8 or not (r.rotary_dim is None or r.rotary_dim == r.head_dim):
-        return False
-    starts = r.kcache.data_ptr() | r.vcache.data_ptr()
-    if r.cos is not None and r.sin is not None:
-        starts |= r.cos.data_ptr() | r.sin.data_ptr()
-    return starts % 16 == 0
 
 
 def gemm_split(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -1258,13 +1247,13 @@ def split_linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.T
     return stream_out, out
 
 
-def split_linear_rope_append(x: torch.Tensor, w: torch.Tensor, r: RopeAppend) -> torch.Tensor:
-    """``split_rope_append(gemm_split(x, w), r)``."""
+def split_linear_rope_append(x: torch.Tensor, w: torch.Tensor, r: RopeAppend) -> torch.Tensor | None:
+    """``split_rope_append(gemm_split(x, w), r)``; None, and nothing done, where tables or pages do not start at multiples of 16 bytes."""
     m, k = x.shape
     n, half = w.shape[0], r.head_dim // 2
     i32 = torch.int32
     if not (x.is_cuda and w.is_cuda and x.device == w.device and w.is_contiguous() and w.shape[1] == k and split_takes(x, w)
-            and n == (r.nq + 2 * r.nkv) * r.head_dim
+            and n == (r.nq + 2 * r.nkv) * r.head_dim and r.head_dim % 8 == 0
             and (r.rotary_dim is None or r.rotary_dim == r.head_dim)
             and r.positions.dtype == r.token_req.dtype == r.block_table.dtype == i32 and r.positions.numel() == r.token_req.numel() == m
             and r.positions.is_contiguous() and r.token_req.is_contiguous() and r.block_table.is_contiguous() and r.block_table.dim() == 2
@@ -1273,15 +1262,21 @@ def split_linear_rope_append(x: torch.Tensor, w: torch.Tensor, r: RopeAppend) ->
                           f"(contiguous int32, one entry a row) do not go together, or not on the GPU")
     _check_pages(r.kcache, r.vcache, r.nkv, r.page_size, r.head_dim, torch.bfloat16, "split_linear_rope_append")
     cos, sin = r.cos, r.sin
-    if cos is not None and not (sin is not None and cos.is_cuda and sin.is_cuda and cos.dtype == sin.dtype == torch.float32
-                                and cos.shape == sin.shape and cos.shape[1] == half and cos.is_contiguous() and sin.is_contiguous()):
-        raise KernelError("split_linear_rope_append: cos/sin tables must be contiguous float32 [positions, d/2]")
+    keys, values, cos_at, sin_at = r.kcache.data_ptr(), r.vcache.data_ptr(), None, None
+    starts = keys | values
+    if cos is not None:
+        if not (sin is not None and cos.is_cuda and sin.is_cuda and cos.dtype == sin.dtype == torch.float32
+                and cos.shape == sin.shape and cos.shape[1] == half and cos.is_contiguous() and sin.is_contiguous()):
+            raise KernelError("split_linear_rope_append: cos/sin tables must be contiguous float32 [positions, d/2]")
+        cos_at, sin_at = cos.data_ptr(), sin.data_ptr()
+        starts |= cos_at | sin_at
+    if starts % 16:
+        return None
     cuts = split_cuts(n, k, m)
     part = torch.empty((cuts, m, n), dtype=torch.float32, device=x.device)
     q = torch.empty((m, r.nq * r.head_dim), dtype=torch.bfloat16, device=x.device)
     call("tk_split_linear_rope_append", x.data_ptr(), x.stride(0), w.data_ptr(), part.data_ptr(), m, k, cuts, q.data_ptr(),
-         r.positions.data_ptr(), r.token_req.data_ptr(), r.block_table.data_ptr(), r.block_table.stride(0),
-         cos.data_ptr() if cos is not None else None, sin.data_ptr() if cos is not None else None, r.kcache.data_ptr(), r.vcache.data_ptr(),
+         r.positions.data_ptr(), r.token_req.data_ptr(), r.block_table.data_ptr(), r.block_table.stride(0), cos_at, sin_at, keys, values,
          r.nq, r.nkv, r.head_dim, r.page_size, _stream())
     return q
 

@@ -60,6 +60,8 @@ class Linear:
         # rows from which the split product is taken (counted once: few calls of a step reach them)
         self.split_norm_from = ops.split_from_rows(in_features, self.total_out, ops.SPLIT_NORM_ELEMENTS)
         self.split_rope_from = ops.split_from_rows(in_features, self.total_out, ops.SPLIT_ROPE_ELEMENTS)
+        # rows, or as many as they are padded to, that the weight-streaming product would take: rounded once where they are split
+        self.split_once_to = ops.recorded_rows(ops.skinny_rows(in_features))
 
     def tensor_specs(self) -> list[TensorSpec]:
         specs = [TensorSpec(n, (o, self.in_features), MATRIX) for n, o in zip(self.names, self.out_features)]
@@ -183,10 +185,8 @@ class Linear:
         fusable = emit_norm is not None and getattr(emit_norm, "fusable_rms", False)
         if (fusable and self.split_norm_from <= m <= ops.SPLIT_ROWS and self.bias is None and ops.split_takes(x, self.weight)
                 and residual.is_contiguous() and ops.split_norm_takes(residual, emit_norm.weight)):
-            # (few rows, or as many as they are padded to: the next product's operand is rounded once, as where the weight-streaming
-            # product emits it)
-            few = ops.recorded_rows(ops.skinny_rows(self.in_features))
-            out, normed = ops.split_linear_add_rmsnorm(x, self.weight, residual, emit_norm.weight, emit_norm.eps, m <= few)
+            # (few rows: the next product's operand is rounded once, as where the weight-streaming product emits it)
+            out, normed = ops.split_linear_add_rmsnorm(x, self.weight, residual, emit_norm.weight, emit_norm.eps, m <= self.split_once_to)
             return out, Prepared(None, emit_norm, normed)
         if fusable and self._fast(m):
             out, data = ops.gemm_skinny_bf16(x, self.weight, residual=residual, emit_weight=emit_norm.weight, bias=self.bias)
@@ -204,11 +204,12 @@ class Linear:
         stream = x.x if isinstance(x, Normed) else x
         m = stream.shape[0]
         # (a norm that the product in front prepared is folded in below: its rows are not made for the split form)
-        if (self.split_rope_from <= m <= ops.SPLIT_ROWS and self.bias is None and ops.split_takes(stream, self.weight)
-                and not (isinstance(x, Normed) and x.usable()) and ops.split_rope_takes(rope)):
-            rows = x.materialize() if isinstance(x, Normed) else x  # (a norm's rows lie as their stream does, or from their own start)
-            if ops.split_takes(rows, self.weight):
-                return ops.split_linear_rope_append(rows, self.weight, rope)
+        if (self.split_rope_from <= m <= ops.SPLIT_ROWS and self.bias is None and stream.dtype == torch.bfloat16 and rope.head_dim % 8 == 0
+                and (rope.rotary_dim is None or rope.rotary_dim == rope.head_dim) and not (isinstance(x, Normed) and x.usable())):
+            rows = x.materialize() if isinstance(x, Normed) else x
+            q = ops.split_linear_rope_append(rows, self.weight, rope) if ops.split_takes(rows, self.weight) else None
+            if q is not None:
+                return q
             x = rows
         most = min(ops.SKINNY_ROPE_ROWS, 2 * ops.skinny_rows(self.in_features, paired=True))
         fits = self.weight.dtype == torch.bfloat16 and 0 < m <= most and self._aligned()
