@@ -610,7 +610,6 @@ __global__ __launch_bounds__(1024) void gemm_staged_kernel(GemmArgs a) {
 // Bound by reading W.  Measured against the library's product and the pass behind it (us): N = 14,336, K = 4,096 (235 MB)
 // 62.3 / 42.3 at 16 rows (5.6 TB/s), 60.5 / 45.5 at 32, 64.2 / 49.0 at 48, 55.9 / 52.9 at 64; 8,192 x 3,072 24.0 / 20.4 at 16, 25.9 /
 // 25.0 at 64; 8,192 x 2,048 19.2 / 14.2 at 16, 20.0 / 17.1 at 64 (ops.glu_rows has more, and where the library is ahead).
-// With all workgroups at the same step of K: 46.3, 48.6, 52.0 and 54.8; 20.1 and 24.9; 17.2 and 19.4.
 // ---------------------------------------------------------------------------------
 #define GL_K 64
 
@@ -636,9 +635,12 @@ __global__ __launch_bounds__(256, 2) void gemm_glu_stream_kernel(GemmArgs a) {
 #pragma unroll
   for (int i = 0; i < MB / 2; ++i) src[2 + i] = a.A + (size_t)min((wave * (MB / 2) + i) * 8 + lr, a.M - 1) * a.lda + piece;
   const int steps = a.K / GL_K;
-  // a workgroup begins its walk over K 7 steps behind its neighbour's beginning and comes round: in step, 256 workgroups would
-  // read the same columns of rows that lie 2 K bytes apart, which for a K of a power of two are few of the memory's channels
-  const int turn = (int)(blockIdx.x * 7u % (unsigned)steps);
+  // a workgroup begins its walk over K 7 steps behind its neighbour's beginning and comes round, for a K of a power of two: in step,
+  // the workgroups would read the same columns of rows that lie 2 K bytes apart, which then are few of the memory's channels.  In step /
+  // apart, 8 rows: 8,192 x 2,048 18.3 / 14.9 us, 8,192 x 4,096 30.8 / 26.8, 28,672 x 8,192 179 / 164, 5,632 x 2,048 12.6 / 11.4; but 8,192 x
+  // 2,304 16.5 / 17.3, 8,192 x 3,072 20.3 / 20.6, 13,824 x 5,120 52.4 / 53.6, and with half of the compute units 4,096 x 2,048 11.6 / 12.6.
+  const bool apart = (a.K & (a.K - 1)) == 0 && gridDim.x > 128;
+  const int turn = apart ? (int)(blockIdx.x * 7u % (unsigned)steps) : 0;
   auto ask = [&](int step) {
     const unsigned base = lds + (unsigned)(step % S * ROWS * GL_K * sizeof(bf16_t));
     const size_t k = (size_t)(step + turn < steps ? step + turn : step + turn - steps) * GL_K;
