@@ -1169,13 +1169,46 @@ def split_norm_takes(residual: torch.Tensor, weight: torch.Tensor) -> bool:
     return residual.dtype == torch.bfloat16 and residual.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0 and residual.shape[1] % 8 == 0
 
 
+def _check_split(x: torch.Tensor, w: torch.Tensor, who: str) -> tuple[int, int, int]:
+    """(rows, outputs, inner size); ``split_takes`` and what it leaves to the caller."""
+    if x.dim() == 2 and w.dim() == 2:
+        (m, k), (n, inner) = x.shape, w.shape
+        if (k == inner and 0 < m <= SPLIT_ROWS and k % SPLIT_STEP == 0 and n % 8 == 0 and x.is_cuda and w.is_cuda and x.device == w.device
+                and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and rows_at_16_bytes(x) and w.data_ptr() % 16 == 0):
+            return m, n, k
+    raise KernelError(f"{who}: x {tuple(x.shape)} {x.dtype} (up to {SPLIT_ROWS} rows at multiples of 16 bytes) and w {tuple(w.shape)} {w.dtype} must "
+                      "be bfloat16 [M, K] and [N, K] on one GPU, K a multiple of 64, N of 8")
+
+
+def _check_split_norm(residual: torch.Tensor, weight: torch.Tensor, rows: int, hidden: int, who: str) -> None:
+    if not (residual.is_cuda and weight.is_cuda and residual.shape == (rows, hidden) and residual.dtype == torch.bfloat16 and residual.is_contiguous()
+            and weight.shape == (hidden,) and weight.is_contiguous() and (weight.dtype == torch.bfloat16 or weight.dtype == torch.float32)):
+        raise KernelError(f"{who}: residual {tuple(residual.shape)} {residual.dtype} must be contiguous bfloat16 [{rows}, {hidden}] and the norm's weight "
+                          f"{tuple(weight.shape)} {weight.dtype} [{hidden}] of bfloat16 or float32, on the GPU")
+
+
+def _check_split_rope(r: RopeAppend, rows: int, width: int, who: str) -> tuple:
+    """Addresses of the tables (or None) and of the pages."""
+    if not (r.head_dim % 8 == 0 and (r.rotary_dim is None or r.rotary_dim == r.head_dim) and width == (r.nq + 2 * r.nkv) * r.head_dim):
+        raise KernelError(f"{who} takes [q | k | v] of whole heads that are rotated whole, their size a multiple of 8")
+    positions, req, table, cos, sin = r.positions, r.token_req, r.block_table, r.cos, r.sin
+    if not (positions.dtype == req.dtype == table.dtype == torch.int32 and positions.numel() == req.numel() == rows and table.dim() == 2
+            and positions.is_contiguous() and req.is_contiguous() and table.is_contiguous()
+            and positions.is_cuda and req.is_cuda and table.is_cuda and r.kcache.is_cuda and r.vcache.is_cuda):
+        raise KernelError(f"{who}: positions and token_req need one entry a row, block_table [requests, width], contiguous int32 on the GPU like the pages")
+    _check_pages(r.kcache, r.vcache, r.nkv, r.page_size, r.head_dim, torch.bfloat16, who)
+    if cos is None:
+        return None, None, r.kcache.data_ptr(), r.vcache.data_ptr()
+    if not (sin is not None and cos.is_cuda and sin.is_cuda and cos.dtype == sin.dtype == torch.float32
+            and cos.shape == sin.shape and cos.shape[1] == r.head_dim // 2 and cos.is_contiguous() and sin.is_contiguous()):
+        raise KernelError(f"{who}: cos/sin tables must be contiguous float32 [positions, d/2]")
+    return cos.data_ptr(), sin.data_ptr(), r.kcache.data_ptr(), r.vcache.data_ptr()
+
+
 def gemm_split(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x [M <= 256, K] . w [N, K]^T in bfloat16 with K cut among workgroups: the cuts' 32-bit sums [cuts, M, N], which
     ``split_add_rmsnorm`` or ``split_rope_append`` adds in ascending order."""
-    _gpu(x, w)
-    _need(x.dim() == 2 and w.dim() == 2 and w.is_contiguous() and x.shape[1] == w.shape[1] and x.device == w.device and split_takes(x, w),
-          "gemm_split: x [M, K] (up to 256 rows at multiples of 16 bytes) and w [N, K] must be bfloat16 on one device, K a multiple of 64, N of 8")
-    m, (n, k) = x.shape[0], w.shape
+    m, n, k = _check_split(x, w, "gemm_split")
     cuts = split_cuts(n, k, m)
     part = torch.empty((cuts, m, n), dtype=torch.float32, device=x.device)
     call("tk_gemm_split_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), part.data_ptr(), m, n, k, cuts, _stream())
@@ -1186,13 +1219,10 @@ def split_add_rmsnorm(part: torch.Tensor, residual: torch.Tensor, weight: torch.
                       once: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
     """``add_rmsnorm`` of a split product: (product rounded, + residual, rounded; its RMSNorm times ``weight``) in one pass.
     ``once``: the normed value is rounded with the weight on it only, not in front of it too."""
-    _gpu(part, residual, weight)
-    _need(part.dim() == 3 and part.dtype == torch.float32 and part.is_contiguous() and residual.shape == part.shape[1:]
-          and residual.is_contiguous() and residual.dtype == torch.bfloat16,
-          "split_add_rmsnorm: the sums must be float32 [cuts, rows, H], the residual contiguous bfloat16 [rows, H]")
+    _gpu(part)
+    _need(part.dim() == 3 and part.dtype == torch.float32 and part.is_contiguous(), "split_add_rmsnorm: the sums must be float32 [cuts, rows, H]")
     cuts, rows, hidden = part.shape
-    if weight.shape != (hidden,) or not weight.is_contiguous() or weight.dtype not in (torch.bfloat16, torch.float32):
-        raise KernelError("split_add_rmsnorm: the weight must be [H] of bfloat16 or float32")
+    _check_split_norm(residual, weight, rows, hidden, "split_add_rmsnorm")
     stream_out, out = torch.empty_like(residual), torch.empty_like(residual)
     call("tk_split_add_rmsnorm", part.data_ptr(), cuts, residual.data_ptr(), weight.data_ptr(), 1 if weight.dtype == torch.float32 else 0,
          stream_out.data_ptr(), out.data_ptr(), rows, hidden, float(eps), 1 if once else 0, _stream())
@@ -1202,25 +1232,13 @@ def split_add_rmsnorm(part: torch.Tensor, residual: torch.Tensor, weight: torch.
 def split_rope_append(part: torch.Tensor, r: RopeAppend) -> torch.Tensor:
     """``rope_append`` of a split [q | k | v] product (whole heads rotated): the cuts added and rounded, q and k rotated, k and v
     stored in the tokens' pages; returns q [rows, nq * d]."""
-    _gpu(part, r.positions, r.token_req, r.block_table, r.cos, r.sin, r.kcache, r.vcache)
-    _need(part.dim() == 3 and part.dtype == torch.float32 and part.is_contiguous() and part.shape[2] == (r.nq + 2 * r.nkv) * r.head_dim,
-          "split_rope_append: the sums must be float32 [cuts, rows, (nq + 2 nkv) d]")
-    _need(r.rotary_dim is None or r.rotary_dim == r.head_dim, "split_rope_append rotates whole heads")
-    cuts, rows, _ = part.shape
-    for t, name in ((r.positions, "positions"), (r.token_req, "token_req"), (r.block_table, "block_table")):
-        _i32(t, name)
-    _need(r.positions.numel() == rows and r.token_req.numel() == rows and r.block_table.dim() == 2,
-          "split_rope_append: positions/token_req need one entry a row, block_table [requests, width]")
-    _check_pages(r.kcache, r.vcache, r.nkv, r.page_size, r.head_dim, torch.bfloat16, "split_rope_append")
-    if r.cos is not None:
-        _need(r.sin is not None and r.cos.dtype == r.sin.dtype == torch.float32 and r.cos.shape == r.sin.shape
-              and r.cos.shape[1] == r.head_dim // 2 and r.cos.is_contiguous() and r.sin.is_contiguous(),
-              "split_rope_append: cos/sin tables must be contiguous float32 [positions, d/2]")
+    _gpu(part)
+    _need(part.dim() == 3 and part.dtype == torch.float32 and part.is_contiguous(), "split_rope_append: the sums must be float32 [cuts, rows, (nq + 2 nkv) d]")
+    cuts, rows, width = part.shape
+    cos, sin, keys, values = _check_split_rope(r, rows, width, "split_rope_append")
     q = torch.empty((rows, r.nq * r.head_dim), dtype=torch.bfloat16, device=part.device)
     call("tk_split_rope_append", part.data_ptr(), cuts, q.data_ptr(), r.positions.data_ptr(), r.token_req.data_ptr(),
-         r.block_table.data_ptr(), r.block_table.stride(0), r.cos.data_ptr() if r.cos is not None else None,
-         r.sin.data_ptr() if r.sin is not None else None, r.kcache.data_ptr(), r.vcache.data_ptr(), rows, r.nq, r.nkv, r.head_dim,
-         r.page_size, _stream())
+         r.block_table.data_ptr(), r.block_table.stride(0), cos, sin, keys, values, rows, r.nq, r.nkv, r.head_dim, r.page_size, _stream())
     return q
 
 
@@ -1231,52 +1249,27 @@ def split_rope_append(part: torch.Tensor, r: RopeAppend) -> torch.Tensor:
 def split_linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float,
                              once: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
     """``split_add_rmsnorm(gemm_split(x, w), residual, weight, eps, once)``."""
-    m, k = x.shape
-    n = w.shape[0]
-    dtype = weight.dtype
-    if not (x.is_cuda and w.is_cuda and residual.is_cuda and weight.is_cuda and x.device == w.device and w.is_contiguous()
-            and w.shape[1] == k and split_takes(x, w) and residual.shape == (m, n) and residual.dtype == torch.bfloat16 and residual.is_contiguous()
-            and weight.shape == (n,) and weight.is_contiguous() and (dtype == torch.bfloat16 or dtype == torch.float32)):
-        raise KernelError(f"split_linear_add_rmsnorm: x {tuple(x.shape)} {x.dtype}, w {tuple(w.shape)} {w.dtype}, residual {tuple(residual.shape)} "
-                          f"{residual.dtype} and norm weight {tuple(weight.shape)} {dtype} do not go together, or not on the GPU")
+    m, n, k = _check_split(x, w, "split_linear_add_rmsnorm")
+    _check_split_norm(residual, weight, m, n, "split_linear_add_rmsnorm")
     cuts = split_cuts(n, k, m)
     part = torch.empty((cuts, m, n), dtype=torch.float32, device=x.device)
     stream_out, out = torch.empty_like(residual), torch.empty_like(residual)
     call("tk_split_linear_add_rmsnorm", x.data_ptr(), x.stride(0), w.data_ptr(), part.data_ptr(), m, n, k, cuts, residual.data_ptr(),
-         weight.data_ptr(), 1 if dtype == torch.float32 else 0, stream_out.data_ptr(), out.data_ptr(), eps, 1 if once else 0, _stream())
+         weight.data_ptr(), 1 if weight.dtype == torch.float32 else 0, stream_out.data_ptr(), out.data_ptr(), eps, 1 if once else 0, _stream())
     return stream_out, out
 
 
 def split_linear_rope_append(x: torch.Tensor, w: torch.Tensor, r: RopeAppend) -> torch.Tensor | None:
     """``split_rope_append(gemm_split(x, w), r)``; None, and nothing done, where tables or pages do not start at multiples of 16 bytes."""
-    m, k = x.shape
-    n, half = w.shape[0], r.head_dim // 2
-    i32 = torch.int32
-    if not (x.is_cuda and w.is_cuda and x.device == w.device and w.is_contiguous() and w.shape[1] == k and split_takes(x, w)
-            and n == (r.nq + 2 * r.nkv) * r.head_dim and r.head_dim % 8 == 0
-            and (r.rotary_dim is None or r.rotary_dim == r.head_dim)
-            and r.positions.dtype == r.token_req.dtype == r.block_table.dtype == i32 and r.positions.numel() == r.token_req.numel() == m
-            and r.positions.is_contiguous() and r.token_req.is_contiguous() and r.block_table.is_contiguous() and r.block_table.dim() == 2
-            and r.positions.is_cuda and r.token_req.is_cuda and r.block_table.is_cuda and r.kcache.is_cuda and r.vcache.is_cuda):
-        raise KernelError(f"split_linear_rope_append: x {tuple(x.shape)} {x.dtype}, w {tuple(w.shape)} {w.dtype} and the tokens' arrays "
-                          f"(contiguous int32, one entry a row) do not go together, or not on the GPU")
-    _check_pages(r.kcache, r.vcache, r.nkv, r.page_size, r.head_dim, torch.bfloat16, "split_linear_rope_append")
-    cos, sin = r.cos, r.sin
-    keys, values, cos_at, sin_at = r.kcache.data_ptr(), r.vcache.data_ptr(), None, None
-    starts = keys | values
-    if cos is not None:
-        if not (sin is not None and cos.is_cuda and sin.is_cuda and cos.dtype == sin.dtype == torch.float32
-                and cos.shape == sin.shape and cos.shape[1] == half and cos.is_contiguous() and sin.is_contiguous()):
-            raise KernelError("split_linear_rope_append: cos/sin tables must be contiguous float32 [positions, d/2]")
-        cos_at, sin_at = cos.data_ptr(), sin.data_ptr()
-        starts |= cos_at | sin_at
-    if starts % 16:
+    m, n, k = _check_split(x, w, "split_linear_rope_append")
+    cos, sin, keys, values = _check_split_rope(r, m, n, "split_linear_rope_append")
+    if (keys | values | (cos or 0) | (sin or 0)) % 16:
         return None
     cuts = split_cuts(n, k, m)
     part = torch.empty((cuts, m, n), dtype=torch.float32, device=x.device)
     q = torch.empty((m, r.nq * r.head_dim), dtype=torch.bfloat16, device=x.device)
     call("tk_split_linear_rope_append", x.data_ptr(), x.stride(0), w.data_ptr(), part.data_ptr(), m, k, cuts, q.data_ptr(),
-         r.positions.data_ptr(), r.token_req.data_ptr(), r.block_table.data_ptr(), r.block_table.stride(0), cos_at, sin_at, keys, values,
+         r.positions.data_ptr(), r.token_req.data_ptr(), r.block_table.data_ptr(), r.block_table.stride(0), cos, sin, keys, values,
          r.nq, r.nkv, r.head_dim, r.page_size, _stream())
     return q
 
