@@ -170,10 +170,3 @@ def test_what_is_refused():
     for bad in ((x[:, :96], w[:, :96].contiguous()), (x, w[:60]), (torch.cat([x] * 65), w), (x.float(), w.float()), (x[:, 1:65], w[:, :64].contiguous())):
         with pytest.raises(ops.KernelError):
             ops.gemm_split(*bad)
-
-
-def test_cuts_fill_the_compute_units():
-    for n in range(64, 16384, 192):
-        for k in (64, 512, 2048, 8192):
-            cuts = ops.split_cuts(n, k)
-            assert 1 <= cuts <= max(1, min(16, k // 256))

@@ -128,3 +128,44 @@ def test_which_tile_gate_and_up_take(m, n, k, shape):
                                          (1500, 2048, 8192, -1), (2048, 4096, 14336, 2), (2048, 4096, 4096, -1), (8192, 2048, 8192, -1)])
 def test_which_tile_a_plain_product_takes(m, n, k, shape):
     assert ops.tiles_choice(m, n, k) == shape
+
+
+@pytest.mark.parametrize("m", [1, 128, 129, 256])
+def test_cuts_fill_the_compute_units(m):
+    """The fewest cuts whose workgroups fill nine tenths of the 256 units' rounds, four steps of K each; else those that fill most."""
+    for n in range(64, 16384, 192):
+        for k in (64, 512, 2048, 8192, 14336):
+            most = max(1, min(16, k // 256))
+            groups = [-(-n // 64) * (2 if m > 128 else 1) * c for c in range(1, most + 1)]
+            filled = [g / (-(-g // 256) * 256) for g in groups]
+            enough = [c for c, f in enumerate(filled, 1) if f >= 0.9]
+            assert ops.split_cuts(n, k, m) == (enough[0] if enough else 1 + filled.index(max(filled)))
+
+
+def _taken(calls, lin, x, residual, n, rope):
+    calls.clear()
+    lin.with_residual(x, residual, n)
+    lin.rope_append(x, rope)
+    return list(calls)
+
+
+def test_what_the_split_products_take(calls, monkeypatch):
+    """Both sides of the thresholds of a weight of 2,048 x 2,048 (48,000 and 24,000 elements of x, counted at the recorded size), and
+    calls that they do not take: with a bias, of rows that start anywhere, of weights below 2^20 elements, in 32-bit."""
+    monkeypatch.setattr(ops, "load", lambda name: type("Lib", (), {"tk_gemm_skinny_parts": lambda self, *a: 4})())
+    monkeypatch.setattr(ops, "library_workspace", lambda: on_gpu(16))
+    monkeypatch.setattr(ops, "_gpu", lambda *tensors: None)  # (what a product leaves here does not say that it lies on one)
+    n, skinny, split = norm(2048), "tk_gemm_skinny_bf16", ["tk_split_linear_add_rmsnorm", "tk_split_linear_rope_append"]
+    library = ["tk_gemm_library_bf16", "tk_add_rmsnorm"]
+    for m, want in ((8, [skinny, skinny]), (9, [skinny, split[1]]), (16, [skinny, split[1]]), (17, split), (64, split), (256, split), (257, library)):
+        assert _taken(calls, linear(2048, 2048), on_gpu(m, 2048), on_gpu(m, 2048), n, _rope(m, 16, 8, 64)) == want, m
+    biased = linear(2048, 2048)
+    biased.bias = on_gpu(2048)
+    assert _taken(calls, biased, on_gpu(24, 2048), on_gpu(24, 2048), n, _rope(24, 16, 8, 64)) == [skinny, skinny]
+    small = linear(512, 2040)
+    assert _taken(calls, small, on_gpu(36, 2040), on_gpu(36, 512), norm(512), _rope(36, 4, 2, 64)) == [skinny]
+    shifted = on_gpu(200, 2056)[:, 4:2052]  # (the library's product is asked through the tensor library)
+    monkeypatch.setattr(torch, "mm", lambda x, w: calls.append("mm") or on_gpu(x.shape[0], w.shape[1]))
+    assert _taken(calls, linear(2048, 2048), shifted, on_gpu(200, 2048), n, _rope(200, 16, 8, 64)) == ["mm", "tk_add_rmsnorm"]
+    wide = on_gpu(33, 2049)[:, 1:]  # a residual whose rows do not follow each other
+    assert _taken(calls, linear(2048, 2048), on_gpu(33, 2048), wide, n, _rope(33, 16, 8, 64)) == [skinny, split[1]]

@@ -134,9 +134,10 @@ def test_the_bfloat16_measure_finds_a_wrong_page_and_a_wrong_position(model, fau
             check_against_plain_bfloat16(got, plain, plain16, largest_too=False)
 
 
-def test_recorded_steps_with_library_products_agree_with_eager_ones(model):
-    """At these sizes the library picks other kernels than for the tiny models: every recorded
-    size up to 128 rows, replayed with eager steps between, against an eager run."""
+def test_recorded_steps_of_many_rows_agree_with_eager_ones(model):
+    """At these sizes a step takes other products than the tiny models' (split ones, gate and up streamed and in
+    tiles, the library's for the head): every recorded size up to 128 rows, replayed with eager steps between, against an
+    eager run."""
     from test_engine_gpu import recorded_against_eager
 
     folder = model[0]

@@ -74,16 +74,19 @@ static bool launch_shape(const TilesArgs& a, int shape, hipStream_t stream) {
     case 0: return launch_tiles<TileShape<2, 2, 5, 5>, GLU>(a, stream);
     case 1: return launch_tiles<TileShape<3, 2, 4, 4>, GLU>(a, stream);
     case 2: return launch_tiles<TileShape<2, 4, 3, 3>, GLU>(a, stream);
-    case 3: return launch_tiles<TileShape<3, 4, 2, 3>, GLU>(a, stream);
-    case 4: return launch_tiles<TileShape<4, 4, 2, 3>, GLU>(a, stream);
-    case 5:
-      if constexpr (GLU) return launch_tiles<TileShape<2, 1, 6, 6>, GLU>(a, stream);
-    default: return false;
   }
+  if constexpr (GLU) {
+    switch (shape) {
+      case 3: return launch_tiles<TileShape<3, 4, 2, 3>, GLU>(a, stream);
+      case 4: return launch_tiles<TileShape<4, 4, 2, 3>, GLU>(a, stream);
+      case 5: return launch_tiles<TileShape<2, 1, 6, 6>, GLU>(a, stream);
+    }
+  }
+  return false;
 }
 
-// glu: W is [gate | up], [2 N, K]; else [N, K].  shape: 0 .. 4, tiles of 128 x 128, 192 x 128, 128 x 256, 192 x 256 and 256 x 256 rows of
-// A and of W; 5, gated only: 128 x 64.
+// glu: W is [gate | up], [2 N, K]; else [N, K].  shape: tiles of 128 x 128 (0), 192 x 128 and 128 x 256 rows of A and of W, and gated of
+// 192 x 256 (3), 256 x 256 and 128 x 64; plain products of such tiles were behind the library's.
 TK_API int tk_gemm_tiles_bf16(const void* A, int lda, const void* W, void* C, int ldc, int M, int N, int K, int glu, int shape,
                               hipStream_t stream) {
   TK_REQUIRE(A && W && C && M >= 0 && N > 0 && K > 0 && K % TILE_K == 0, "gemm_tiles: bad sizes M=%d N=%d K=%d", M, N, K);
@@ -95,7 +98,7 @@ TK_API int tk_gemm_tiles_bf16(const void* A, int lda, const void* W, void* C, in
   if (M == 0) return 0;
   const TilesArgs a{(const bf16_t*)A, lda, (const bf16_t*)W, (bf16_t*)C, ldc, M, N, K, 0, 0};
   const bool ok = glu ? launch_shape<true>(a, shape, stream) : launch_shape<false>(a, shape, stream);
-  TK_REQUIRE(ok, "gemm_tiles: tile %d (0 .. 4, gated 5 too) cannot be launched", shape);
+  TK_REQUIRE(ok, "gemm_tiles: tile %d (0 .. 2, gated up to 5) cannot be launched", shape);
   TK_CHECK_LAUNCH("gemm_tiles");
   return 0;
 }

@@ -1376,7 +1376,7 @@ def tiles_choice(m: int, n: int, k: int, glu: bool = False) -> int:
     if glu:
         least = GLU_TILES_LATER_FILL if rounds > 1 else (0.65 if m <= 128 else 0.8)
         return shape if m >= GLU_TILES_FROM_ROWS and fill >= least and m * 2 * n <= GLU_TILES_MOST_SUMS else -1
-    least = (0.84, 0.75, 0.84 if k >= 8192 else 2.0, 2.0, 2.0)[shape]
+    least = (0.84, 0.75, 0.84 if k >= 8192 else 2.0)[shape] if shape < 3 else 2.0  # (2: the library's is ahead however full)
     return shape if m >= PLAIN_TILES_FROM_ROWS and rounds == 1 and fill >= least else -1
 
 
