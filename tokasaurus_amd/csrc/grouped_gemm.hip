@@ -12,8 +12,8 @@
 // first operand of the matrix core, read straight from memory 16 bytes a lane, the rows of A the second; a lane ends up with
 // 4 neighbouring outputs of one row.  The next step's operands are asked for before the current step's products.
 // Experts (grouped_gemm_staged_kernel): tiles of GS_M = 128 slots x 128 weight rows through local memory, however few slots a
-// tile holds (see there); experts of many rows take two such tiles as one of 256 x 256 (grouped_gemm_pairs_kernel).  Sums are 32-bit and run over k in ascending steps for every output: a row's result does not
-// depend on which other rows share its tile.
+// tile holds (see there); experts of many rows take two such tiles as one of 256 x 256 (grouped_gemm_pairs_kernel).  Sums are 32-bit
+// and run over k in ascending steps for every output: a row's result does not depend on which other rows share its tile.
 #include <math.h>
 
 #include "gemm_tile.h"
@@ -332,18 +332,18 @@ __global__ __launch_bounds__(256, 3) void grouped_gemm_staged_kernel(GroupedArgs
 }
 
 // Experts of many rows: two neighbouring tiles of a group as one of 256 slots x 256 weight rows (in the gated form 128 of gate and
-// 128 of up; gemm_tile.h), the odd last tile of a group as half of one.  The path from the L2 to a compute unit bounds these
-// products, and a tile of 256 x 256 asks for half as many bytes a product.
-// us by tiles of 128 x 128 / in pairs, gate and up and down, every expert 3, 4, 5 and 6 tiles: 32 experts of 2,048 x 1,024 147 / 140 and
-// 85 / 70, 184 / 142 and 110 / 73, 222 / 199 and 131 / 100, 260 / 203 and 155 / 105; 32 of 2,880 x 2,880 546 / 479 and 299 / 217 to
-// 1,048 / 717 and 546 / 347.  Odd tiles of 128 x 128 in a launch of their own read the experts' weights a second time: with 3 tiles 172
-// and 87 us for the first, with 5 234 and 118.
+// 128 of up; gemm_tile.h), the odd last tile of a group as one of 128 x 256 in the same launch.  The path from the L2 to a compute
+// unit bounds these products, and a tile of 256 x 256 asks for half as many bytes a product.
+// us by tiles of 128 x 128 / in pairs, gate and up and down, every expert 3, 4, 5 and 6 tiles: 32 experts of 2,048 x 1,024 147 / 136 and
+// 86 / 69, 185 / 141 and 109 / 75, 224 / 190 and 132 / 97, 265 / 202 and 155 / 107; 32 of 2,880 x 2,880 547 / 461 and 300 / 213 to
+// 1,060 / 726 and 554 / 355.  Odd tiles as halves of a pair: 140 and 70, 199 and 100 for the first with 3 and 5.  In a launch of
+// their own, which reads the experts' weights a second time: 172 and 87, 234 and 118.
 template <class S, bool GLU>
-__device__ __forceinline__ void wide_tile(const GroupedArgs& a, char* smem, int g, int first, int n0, int top) {  // top: the last slot
+__device__ __forceinline__ void wide_tile(const GroupedArgs& a, char* smem, int g, int first, int n0) {
   constexpr int OUT = GLU ? S::BN / 2 : S::BN;
   static_assert(S::BM <= 256 && S::BM * S::BN * 2 + S::BM * 4 <= S::LDS, "");
   const int lane = threadIdx.x & (TK_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TK_WAVE);
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave & 1, wn = wave >> 1, top = a.slots - 1;
   TileLoop<S, GLU> t;
   t.wave = wave;
   t.lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
@@ -392,6 +392,7 @@ __device__ __forceinline__ void wide_tile(const GroupedArgs& a, char* smem, int 
 #define WIDE_OUT(glu) ((glu) ? 128 : 256)
 #define WIDE_PAIRS (GS_TILES / 2)
 using PairShape = TileShape<4, 4, 2, 3>;
+using HalfShape = TileShape<2, 4, 3, 3>;
 // A pair, as a workgroup reads it: the group's first tile, the group, the number of the group's first pair and how many tiles it has.
 struct TileRun {
   int tile, group, first, tiles;
@@ -408,7 +409,9 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_pairs_kernel(GroupedArgs 
   // the chunk of up to WIDE_PAIRS pairs of the group that the item lies in
   const int chunk = r.first + (some - r.first) / WIDE_PAIRS * WIDE_PAIRS, len = min(WIDE_PAIRS, r.first + (r.tiles + 1) / 2 - chunk);
   const int off = item - chunk * n_blocks, pair = chunk + off % len;
-  wide_tile<PairShape, GLU>(a, smem, r.group, (r.tile + 2 * (pair - r.first)) * GS_M, off / len * WIDE_OUT(GLU), (r.tile + r.tiles) * GS_M - 1);
+  const int tile = r.tile + 2 * (pair - r.first), n0 = off / len * WIDE_OUT(GLU);
+  if (tile + 1 < r.tile + r.tiles) wide_tile<PairShape, GLU>(a, smem, r.group, tile * GS_M, n0);
+  else wide_tile<HalfShape, GLU>(a, smem, r.group, tile * GS_M, n0);
 }
 
 template <bool GLU>
@@ -418,7 +421,7 @@ static bool launch_by_tile(const GroupedArgs& a, int tiles, const TileRun* runs,
   if (runs) {
     const int wide_blocks = (a.N + WIDE_OUT(GLU) - 1) / WIDE_OUT(GLU);
     const long pairs = groups((long)max_pairs * wide_blocks);
-    static_assert(PairShape::BM == 2 * GS_M, "");
+    static_assert(PairShape::BM == 2 * GS_M && HalfShape::BM == GS_M && HalfShape::LDS <= PairShape::LDS, "");
     auto kernel = grouped_gemm_pairs_kernel<GLU>;
     if (pairs >= (1l << 31) || hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PairShape::LDS) != hipSuccess)
       return false;

@@ -2698,11 +2698,11 @@ def experts_go_in_tiles(rows: int, top: int, dtype: torch.dtype, width: int, ff:
 # average, widths and inner sizes whose steps outweigh a tile's beginning and end, and so many elements of K that a compute unit walks in
 # gate and up: a round of pairs takes all units for one pair each, and a last round that is nearly empty costs as much as a full one.
 # In us by single tiles / in pairs, both products and the sum, experts' rows even, uneven (weights e^(0.5 N(0, 1))) and an eighth of the
-# experts 4.5 times as likely: 32 experts of 2,048 x 1,024, 420 rows an expert (4,380 elements) 276 / 221, 274 / 299, 276 / 296; 500
-# (5,020) 318 / 306, 316 / 304, 327 / 305; 700 425 / 329, 421 / 409, 445 / 405; 1,020 618 / 519, 610 / 518, 612 / 515.  16 of 2,048 x 2,048,
-# 420 rows 271 / 209, 267 / 295, 270 / 295; 500 308 / 302, 314 / 303, 309 / 303.  128 of 2,048 x 768, 220 rows 503 / 490, 527 / 532, 543 / 466;
-# 400 830 / 677, 808 / 738, 848 / 821.  8 of 4,096 x 1,792, 460 rows (4,110) 260 / 179, 263 / 214, 263 / 300; 660 381 / 307, 370 / 306, 342 /
-# 308.  8 of 4,096 x 14,336, 380 rows 1,668 / 1,130, 1,740 / 1,134, 1,696 / 1,439.  64 of 1,024 x 512, 500 rows 186 / 218, 1,060 372 / 374.
+# experts 4.5 times as likely: 32 experts of 2,048 x 1,024, 420 rows an expert (4,380 elements) 338 / 242, 299 / 304, 294 / 303; 500
+# (5,020) 334 / 304, 337 / 307, 338 / 312; 700 444 / 336, 446 / 411, 452 / 410; 1,020 633 / 517, 630 / 524, 641 / 524.  16 of 2,048 x 2,048,
+# 420 rows 277 / 217, 290 / 304, 293 / 301; 500 329 / 310, 334 / 303, 327 / 309.  128 of 2,048 x 768, 400 rows 849 / 699, 835 / 738, 868 / 825.
+# 8 of 4,096 x 1,792, 460 rows (4,110) 262 / 185, 269 / 221, 281 / 305; 660 401 / 313, 363 / 319, 362 / 317.  8 of 4,096 x 14,336, 380 rows
+# 1,681 / 1,135, 1,702 / 1,149, 1,746 / 1,437.  64 of 1,024 x 512, 500 rows 191 / 222, 193 / 220, 193 / 220, 1,060 392 / 374, 379 / 381, 369 / 387.
 EXPERT_PAIRS_FROM_ROWS = 320
 EXPERT_PAIRS_FROM_WIDTH = 2048
 EXPERT_PAIRS_FROM_INNER = 768
