@@ -81,6 +81,7 @@ struct GemmArgs {
   float out_scale;  // the 32-bit epilogue multiplies its result by this (1: as it is)
   int M, N, K;  // N: outputs (for SwiGLU the intermediate size; W then has 2N rows, gate first)
   int TH;       // weight rows of a tile that are used (16, or 8 to make twice the workgroups of a narrow output)
+  int turn;  // streamed gate and up: mask of the step of K that a workgroup begins at (0: all begin with the first)
 };
 
 // the bias of output `i` (a row of W), 0 without one; `i` is clamped to the rows there are
@@ -635,12 +636,11 @@ __global__ __launch_bounds__(256, 2) void gemm_glu_stream_kernel(GemmArgs a) {
 #pragma unroll
   for (int i = 0; i < MB / 2; ++i) src[2 + i] = a.A + (size_t)min((wave * (MB / 2) + i) * 8 + lr, a.M - 1) * a.lda + piece;
   const int steps = a.K / GL_K;
-  // a workgroup begins its walk over K 7 steps behind its neighbour's beginning and comes round, for a K of a power of two: in step,
+  // a workgroup begins its walk over K 7 steps behind its neighbour's beginning and comes round, for a K of a power of two (a.turn): in step,
   // the workgroups would read the same columns of rows that lie 2 K bytes apart, which then are few of the memory's channels.  In step /
   // apart, 8 rows: 8,192 x 2,048 18.3 / 14.9 us, 8,192 x 4,096 30.8 / 26.8, 28,672 x 8,192 179 / 164, 5,632 x 2,048 12.6 / 11.4; but 8,192 x
   // 2,304 16.5 / 17.3, 8,192 x 3,072 20.3 / 20.6, 13,824 x 5,120 52.4 / 53.6, and with half of the compute units 4,096 x 2,048 11.6 / 12.6.
-  const bool apart = (a.K & (a.K - 1)) == 0 && gridDim.x > 128;
-  const int turn = apart ? (int)(blockIdx.x * 7u % (unsigned)steps) : 0;
+  const int turn = (int)(blockIdx.x * 7u) & a.turn;
   auto ask = [&](int step) {
     const unsigned base = lds + (unsigned)(step % S * ROWS * GL_K * sizeof(bf16_t));
     const size_t k = (size_t)(step + turn < steps ? step + turn : step + turn - steps) * GL_K;
@@ -731,7 +731,8 @@ static bool launch_staged_one(const GemmArgs& a, int groups, int WK, hipStream_t
 }
 
 template <int MB, int NB>
-static bool launch_glu_stream(const GemmArgs& a, bool norm, hipStream_t stream) {
+static bool launch_glu_stream(GemmArgs a, bool norm, hipStream_t stream) {
+  a.turn = (a.K & (a.K - 1)) == 0 && a.N > 128 * 32 ? a.K / GL_K - 1 : 0;  // (K / GL_K is a power of two then)
   const size_t lds = (size_t)gl_stages<MB>() * (64 + 16 * MB) * GL_K * sizeof(bf16_t) + (norm ? 16 * MB * sizeof(float) : 0);
   auto kernel = norm ? gemm_glu_stream_kernel<MB, NB, true> : gemm_glu_stream_kernel<MB, NB, false>;
   if (!allow_lds(kernel, lds)) return false;
