@@ -1,5 +1,5 @@
-// bfloat16 matrix products for 17 to 256 rows (9 and more over a long inner size) whose outputs are too narrow to give every
-// compute unit weights of its own:  C[M,N] = A[M,K] * W[N,K]^T with K cut among workgroups, and the passes that add the cuts.
+// bfloat16 matrix products for few to 256 rows (from 17 on over 2,048 inputs, 9 with the rotation behind, 5 over 8,192, 3 over 14,336:
+// ops.split_from_rows) whose outputs are too narrow to give every compute unit weights of its own:  C[M,N] = A[M,K] * W[N,K]^T with K cut among workgroups, and the passes that add the cuts.
 //
 // The product is bound by reading W once; at these rows the output and down projections and the stacked q, k, v product have
 // 32 to 64 tiles of 64 weight rows for 256 compute units, so K is cut until there is a workgroup a unit.  What a workgroup
@@ -13,8 +13,10 @@
 // in local memory measured best: with 8 or 9 (144 KB) 2,048 x 8,192 takes 9.7 at 16 rows, with 3 9.1.
 // From 129 rows on there are two blocks of rows, which read W twice, the second time from the caches.  With the passes, library /
 // this one: 2,048 x 8,192 29.4 / 22.9 at 129 rows, 30.7 / 25.9 at 256; 2,048 x 2,048 12.6 / 12.7, 13.6 / 15.6; 4,096 x 4,096 26.3 / 23.7, 27.1 /
-// 25.6; 3,072 x 2,048 with the rotation 14.7 / 16.4, 16.5 / 18.9; 5,120 x 3,072 24.9 / 24.8, 40.5 / 28.5; and a call of the host less, which
-// bounds such steps.  With three blocks it is behind (2,048 x 2,048 14.8 / 18.1 at 300 rows, 4,096 x 14,336 75 / 91).
+// 25.6; 3,072 x 2,048 with the rotation 14.7 / 16.4, 16.5 / 18.9; 5,120 x 3,072 24.9 / 24.8, 40.5 / 28.5.  In whole recorded steps, where the
+// weights come from memory between other products, the short ones are ahead too: 1B decode of 192 and 256 with the output projection
+// the library's / split 1,968 / 1,854 and 2,194 / 2,062 us, with q, k, v 2,081 / 1,854 and 2,172 / 2,062; 3B 5,309 / 4,761 and 5,718 / 5,358.
+// With three blocks it is behind (2,048 x 2,048 14.8 / 18.1 at 300 rows, 4,096 x 14,336 75 / 91).
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;

@@ -1119,7 +1119,7 @@ def gemm_skinny_bf16(
 # bfloat16 products with K cut among workgroups, and the passes that add the cuts
 # --------------------------------------------------------------------------
 
-SPLIT_ROWS = 256  # rows the split product takes (gemm_split.hip: beyond, the library's product is ahead)
+SPLIT_ROWS = 256  # rows the split product takes, two blocks of them (gemm_split.hip: with three it is behind the library's)
 SPLIT_TILE, SPLIT_STEP = 64, 64  # weight rows a workgroup, elements of K a step
 # Elements of x (rows x inner size) from which the split product and the pass that adds its cuts are ahead of the
 # weight-streaming kernel, whose workgroups each read all of x.  Measured on an MI355X, weights from memory, us:
@@ -1134,7 +1134,7 @@ SPLIT_TILE, SPLIT_STEP = 64, 64  # weight rows a workgroup, elements of K a step
 #   and 33.6 / 25.7 for the last)
 SPLIT_NORM_ELEMENTS = 48_000
 SPLIT_ROPE_ELEMENTS = 24_000
-# (the rows counted are those of the recorded size: recorded_rows).  Elements of w from which: it pays below too (1,024 x 1,024 8.8 /
+# (the rows counted are those of the recorded size: recorded_rows.)  Elements of w from which: it pays below too (1,024 x 1,024 8.8 /
 # 7.4 at 48 rows, 512 x 512 7.3 / 6.5 at 64), but little.
 SPLIT_WEIGHT_ELEMENTS = 1 << 20
 

@@ -11,6 +11,8 @@ Which kernel runs is decided by the storage type and the number of rows:
     up): the hand-written matrix-core kernels that stream the weight once and fuses the epilogue; it can also fold in the
     norm in front (``Normed`` input), leave what the norm behind it needs
     (``emit_norm``), and rotate and append q, k and v (``rope_append``);
+  * bfloat16, up to 256 rows with the residual sum and norm or the rotation behind (from ``ops.split_from_rows`` on): K cut
+    among workgroups, the cuts added by that pass (``ops.split_linear_add_rmsnorm``, ``ops.split_linear_rope_append``);
   * bfloat16, more rows (large decode batches, prefill): tiles of up to 256 x 256 where they are ahead
     (``ops.tiles_choice``; gate and up with the activation in the same kernel), else the library's matrix product,
     as in the reference (its projections are library calls), followed by the epilogue
