@@ -117,16 +117,27 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// Every lane's value meets its partners' 32, 16, 8, 4, 2 and 1 lanes away, in this order, through the lanes' own data paths: a step
+// takes a few clocks, through local memory (a shuffle) fifty, and these chains stand between two trips to memory.  After the
+// step of 8 a row of 16 lanes holds its 8 values twice, so that a turn by 4 is an exchange.
+template <typename Op>
+__device__ __forceinline__ float wave_reduce(float v, Op op) {
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+  v = op(__int_as_float(h[0]), __int_as_float(h[1]));
+  const auto q = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+  v = op(__int_as_float(q[0]), __int_as_float(q[1]));
+  v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, true)));  // row_ror:8
+  v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xF, 0xF, true)));  // row_ror:4
+  v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, true)));   // quad_perm:[2,3,0,1]
+  return op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true)));  // quad_perm:[1,0,3,2]
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = TK_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, TK_WAVE);
-  return v;
+  return wave_reduce(v, [](float a, float b) { return a + b; });
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = TK_WAVE / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, TK_WAVE));
-  return v;
+  return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Sum over a workgroup of up to 1024 threads; every thread gets the result.

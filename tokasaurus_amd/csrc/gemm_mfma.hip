@@ -43,10 +43,14 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 enum { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_F32 = 3, EPI_ROPE = 4 };
 
+// (What the first loads of a kernel need comes first: the compiler asks for neighbouring arguments together.)
 struct GemmArgs {
   const bf16_t* A;
-  int lda;
   const bf16_t* W;
+  int lda, M, N, K;  // N: outputs (for SwiGLU the intermediate size; W then has 2N rows, gate first)
+  int TH;            // weight rows of a tile that are used (16, or 8 to make twice the workgroups of a narrow output)
+  int waves, share, spare;  // skinny kernel: wavefronts that split K, steps of each, wavefronts that take one more
+  int turn;  // streamed gate and up: mask of the step of K that a workgroup begins at (0: all begin with the first)
   void* C;
   int ldc;
   const bf16_t* residual;
@@ -79,14 +83,26 @@ struct GemmArgs {
   float glu_limit, glu_alpha;
   int glu_gelu;  // the gated epilogue's third form: gelu(gate) * up with the tanh form of gelu
   float out_scale;  // the 32-bit epilogue multiplies its result by this (1: as it is)
-  int M, N, K;  // N: outputs (for SwiGLU the intermediate size; W then has 2N rows, gate first)
-  int TH;       // weight rows of a tile that are used (16, or 8 to make twice the workgroups of a narrow output)
-  int turn;  // streamed gate and up: mask of the step of K that a workgroup begins at (0: all begin with the first)
 };
 
 // the bias of output `i` (a row of W), 0 without one; `i` is clamped to the rows there are
 __device__ __forceinline__ float bias_at(const GemmArgs& a, int i, int rows) {
   return a.bias != nullptr ? __bfloat162float(a.bias[min(i, rows - 1)]) : 0.f;
+}
+
+// outputs n .. n + 3 of a token, rounded to bfloat16
+__device__ __forceinline__ void store_rounded(const GemmArgs& a, const float (&o)[4], int token, int n) {
+  bf16_t* c = (bf16_t*)a.C + (size_t)token * a.ldc + n;
+  if (n + 3 < a.N && (a.ldc & 3) == 0) {
+    union { bf16_t h[4]; uint2 u; } pk;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) pk.h[j] = __float2bfloat16(o[j]);
+    *(uint2*)c = pk.u;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (n + j < a.N) c[j] = __float2bfloat16(o[j]);
+  }
 }
 
 template <int EPI>
@@ -107,8 +123,6 @@ __device__ __forceinline__ void store4(const GemmArgs& a, f32x4_t v, f32x4_t up,
         o[j] = silu_mul_bf16(g, u);
       }
     }
-    if (EPI == EPI_RESIDUAL && n + j < a.N)
-      o[j] = round_to<bf16_t>(o[j]) + __bfloat162float(a.residual[(size_t)token * a.ldr + n + j]);
   }
   if (EPI == EPI_F32) {
 #pragma unroll
@@ -122,17 +136,7 @@ __device__ __forceinline__ void store4(const GemmArgs& a, f32x4_t v, f32x4_t up,
         if (n + j < a.N) c[j] = o[j];
     }
   } else {
-    bf16_t* c = (bf16_t*)a.C + (size_t)token * a.ldc + n;
-    if (n + 3 < a.N && (a.ldc & 3) == 0) {
-      union { bf16_t h[4]; uint2 u; } pk;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) pk.h[j] = __float2bfloat16(o[j]);
-      *(uint2*)c = pk.u;
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (n + j < a.N) c[j] = __float2bfloat16(o[j]);
-    }
+    store_rounded(a, o, token, n);
   }
 }
 
@@ -146,10 +150,17 @@ __device__ __forceinline__ bf16x8_t zero8() {
 // 1 / rms of every row of A from the partial sums its producer left, into LDS `scale`
 // (16 * MB floats).  A wavefront takes a row at a time: every lane adds 4 parts (one
 // 16-byte load), then the lanes' sums are added by a butterfly, so the order is fixed.
+// What the first row's first 256 parts are is asked for at a kernel's beginning (row_parts) and
+// used at its end: only the epilogue needs the factors, and a wait for them in front of the
+// weights' loads is a trip to memory that nothing else fills.
+__device__ __forceinline__ f32x4_t row_parts(const GemmArgs& a, int wave, int lane) {
+  f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+  if ((a.parts_in & 3) == 0 && lane * 4 < a.parts_in) v = *(const f32x4_t*)(a.sumsq_in + (size_t)min(wave, a.M - 1) * a.parts_in + lane * 4);
+  return v;
+}
+
 template <int MB>
-__device__ __forceinline__ void row_scales(const GemmArgs& a, float* scale) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int nwaves = blockDim.x >> 6;
+__device__ __forceinline__ void row_scales(const GemmArgs& a, float* scale, f32x4_t first, int wave, int lane, int nwaves) {
   const int rows = min(a.M, 16 * MB);
   const bool vec = (a.parts_in & 3) == 0;
   for (int token = wave; token < rows; token += nwaves) {
@@ -157,7 +168,7 @@ __device__ __forceinline__ void row_scales(const GemmArgs& a, float* scale) {
     float ss = 0.f;
     for (int p = lane * 4; p < a.parts_in; p += 256) {
       if (vec) {
-        const f32x4_t v = *(const f32x4_t*)(part + p);
+        const f32x4_t v = token == wave && p < 256 ? first : *(const f32x4_t*)(part + p);
         ss += (v[0] + v[1]) + (v[2] + v[3]);
       } else {
         for (int j = 0; j < 4 && p + j < a.parts_in; ++j) ss += part[p + j];
@@ -193,31 +204,32 @@ __device__ __forceinline__ void emit_for_norm(const GemmArgs& a, const float (&x
   if (live && (lane >> 4) == 0) a.emit_sumsq[(size_t)token * a.parts_out + part] = total;
 }
 
-// Rotation with append for 4 columns c .. c+3 of head h (and their partners c + d/2): x1, x2
-// are the products rounded to bfloat16 as a plain store would leave them.
-// What the rotation of one unit (token, head h, columns c .. c+3) reads besides the products;
-// asked for before the main loop so that the epilogue does not wait for it.
+// What the rotation of one unit (token, head h, columns c .. c+3) reads besides the products.  The
+// first step's loads go out before the weights', the second's, which need the first's, behind
+// them: nothing waits for either until the weights are there.
+typedef float f32x4_any_t __attribute__((ext_vector_type(4), aligned(4)));  // wherever a float can lie
+
 struct RopeOperands {
-  int pos, page;
-  float cs[4], sn[4];
+  int pos, req, page;
+  f32x4_any_t cs, sn;
 };
 
-__device__ __forceinline__ RopeOperands rope_operands(const GemmArgs& a, int token, int h, int c) {
-  RopeOperands r;
-  const int half = a.d >> 1;
+__device__ __forceinline__ void rope_ask(const GemmArgs& a, int token, RopeOperands& r) {
   const int t = min(token, a.M - 1);
   r.pos = a.positions[t];
-  r.page = h >= a.nq ? a.block_table[(size_t)a.token_req[t] * a.table_stride + r.pos / a.P] : 0;
-  const bool rotate = h < a.nq + a.nkv && a.cos_t != nullptr;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const bool on = rotate && c + j < half;
-    r.cs[j] = on ? a.cos_t[(size_t)r.pos * half + c + j] : 1.f;
-    r.sn[j] = on ? a.sin_t[(size_t)r.pos * half + c + j] : 0.f;
-  }
-  return r;
+  r.req = a.token_req[t];
 }
 
+__device__ __forceinline__ void rope_ask_further(const GemmArgs& a, int h, int c, RopeOperands& r) {
+  const int half = a.d >> 1;
+  r.page = h >= a.nq ? a.block_table[(size_t)r.req * a.table_stride + r.pos / a.P] : 0;
+  const bool on = h < a.nq + a.nkv && a.cos_t != nullptr && c < half;  // (half and c are multiples of 4)
+  r.cs = on ? *(const f32x4_any_t*)(a.cos_t + (size_t)r.pos * half + c) : f32x4_any_t{1.f, 1.f, 1.f, 1.f};
+  r.sn = on ? *(const f32x4_any_t*)(a.sin_t + (size_t)r.pos * half + c) : f32x4_any_t{0.f, 0.f, 0.f, 0.f};
+}
+
+// Rotation with append for 4 columns c .. c+3 of head h (and their partners c + d/2): x1, x2
+// are the products rounded to bfloat16 as a plain store would leave them.
 __device__ __forceinline__ void rope_store(const GemmArgs& a, f32x4_t s0, f32x4_t s1, int token, int h, int c,
                                            const RopeOperands& r) {
   if (token >= a.M) return;
@@ -268,7 +280,8 @@ __device__ __forceinline__ void rope_store(const GemmArgs& a, f32x4_t s0, f32x4_
   }
 }
 
-#define SK_MAX_WAVES 16
+// wavefronts of a workgroup at most: with two tiles 8, so that a wavefront has the registers for its loads in flight
+__host__ __device__ constexpr int sk_max_waves(int NT) { return NT == 2 ? 8 : 16; }
 
 // LDS of the skinny kernel: [scales: 16 * MB floats when NORM][sums: waves * NT * MB * 64 f32x4]
 // FOLD (up to 8 rows of A, tiles of 8 weight rows, K a multiple of 64): a tile of 8 rows leaves
@@ -278,42 +291,38 @@ __device__ __forceinline__ void rope_store(const GemmArgs& a, f32x4_t s0, f32x4_
 // columns 0..7: the first half of K, 8..15: the second; the other two quarters mix the halves and
 // are not used), and the quarters are added when the wavefronts' sums are.  Every lane loads
 // weights, and a wavefront issues half as many loads for the same bytes.
+//
+// A product of a few megabytes is bound by its chain of waits, not by the bytes: a launch takes 1.6 us of 4.8 (8 MB).
+// So the weights' first loads go out as soon as the addresses are there (the arguments they need lie together, every
+// division is the host's), and whatever the epilogue needs is asked for beside them.
 template <int MB, int NT, int EPI, bool NORM, bool FOLD = false>
-__global__ __launch_bounds__(SK_MAX_WAVES * 64) void gemm_skinny_kernel(GemmArgs a) {
+__global__ __launch_bounds__(sk_max_waves(NT) * 64) void gemm_skinny_kernel(GemmArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int U = (NT + MB <= 3) ? 8 : ((NT + MB <= 6) ? 4 : 2);  // steps whose loads are in flight together
   constexpr bool PAIRED = EPI == EPI_SWIGLU || EPI == EPI_ROPE;     // two tiles that meet in the epilogue
   static_assert(!FOLD || (MB == 1 && NT == 1 && !PAIRED), "folding K takes one tile of 8 weight rows and up to 8 rows of A");
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int WK = blockDim.x >> 6;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int WK = a.waves;
   const int r = FOLD ? (lane & 7) : (lane & 15), q = lane >> 4;
   const int g = blockIdx.x;
-  const int K32 = FOLD ? a.K >> 6 : (a.K + 31) >> 5;  // steps a lane walks (with FOLD: of its half of K)
-  const size_t fold = FOLD ? (size_t)((lane >> 3) & 1) * (size_t)K32 * 32 : 0;  // where this lane's half of K begins
-  const int ks0 = (int)((long)K32 * wave / WK), ks1 = (int)((long)K32 * (wave + 1) / WK);
-  const bool k_exact = (a.K & 31) == 0;
-  float* scales = (float*)smem;
-  f32x4_t* red = (f32x4_t*)(smem + (NORM ? 16 * MB * sizeof(float) : 0));
-  if (NORM) row_scales<MB>(a, scales);
+  // steps of 32 that a lane walks (with FOLD: of its half of K)
+  const int ks0 = wave * a.share + min(wave, a.spare), ks1 = ks0 + a.share + (wave < a.spare ? 1 : 0);
+  const size_t fold = FOLD ? (size_t)((lane >> 3) & 1) * (size_t)(a.K >> 1) : 0;  // where this lane's half of K begins
 
-  // rows of W this lane streams (clamped: rows past the end are masked at the store);
-  // with tiles of 8 rows the upper lanes have no row and hold zeros
-  const int TH = a.TH;
-  const bool has_row = r < TH;  // (with FOLD: TH is 8 and r below it)
-  int rope_head = 0, rope_col = 0;  // EPI_ROPE: the head and the first column of this workgroup's pair of tiles
+  // rows of W this lane streams (clamped: rows past the end are masked at the store); with tiles of 8 or 12 rows the upper
+  // lanes repeat the last one, at no cost to memory and into outputs that are not stored
+  const int TH = a.TH, rw = FOLD ? r : min(r, TH - 1);
+  const int rope_head = EPI == EPI_ROPE ? (int)blockIdx.y : 0, rope_col = g * TH;  // EPI_ROPE: the head and the first column of this workgroup's pair of tiles
   const bf16_t* wp[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     int row;
     if (EPI == EPI_SWIGLU) {
-      row = min(g * TH + r, a.N - 1) + t * a.N;  // t = 0 gate, t = 1 up
+      row = min(g * TH + rw, a.N - 1) + t * a.N;  // t = 0 gate, t = 1 up
     } else if (EPI == EPI_ROPE) {
-      const int pairs = (a.d / 2 + TH - 1) / TH;  // pairs of tiles a head
-      rope_head = g / pairs;
-      rope_col = (g - rope_head * pairs) * TH;
-      row = rope_head * a.d + min(rope_col + r, a.d / 2 - 1) + t * (a.d / 2);
+      row = rope_head * a.d + min(rope_col + rw, a.d / 2 - 1) + t * (a.d / 2);
     } else {
-      row = min((g * NT + t) * TH + r, a.N - 1);
+      row = min((g * NT + t) * TH + rw, a.N - 1);
     }
     wp[t] = a.W + (size_t)row * a.K + q * 8 + fold;
   }
@@ -321,66 +330,80 @@ __global__ __launch_bounds__(SK_MAX_WAVES * 64) void gemm_skinny_kernel(GemmArgs
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) ap[mb] = a.A + (size_t)min(mb * 16 + r, a.M - 1) * a.lda + q * 8 + fold;
 
-  // what the rotation of this thread's first unit reads besides the sums (position, page,
-  // cos and sin) is asked for now, so that it has arrived when the main loop is through
+  // what the epilogue's first unit of this thread needs besides the sums: asked for in front of the weights, used behind them
   constexpr int UNITS = (PAIRED ? 1 : NT) * MB * 64;
+  const bool has_unit = wave < UNITS / 64;
+  const int l0 = tid & 63, mb0 = wave % MB, t0 = wave / MB;
   RopeOperands rope_pre = {};
-  if (EPI == EPI_ROPE && tid < UNITS) {
-    const int l0 = tid & 63, mb0 = (tid >> 6) % MB;
-    rope_pre = rope_operands(a, mb0 * 16 + (l0 & 15), rope_head, rope_col + (l0 >> 4) * 4);
+  bf16_t res_pre[4] = {};
+  f32x4_t parts_pre = {0.f, 0.f, 0.f, 0.f};
+  if (NORM) parts_pre = row_parts(a, wave, lane);
+  if (EPI == EPI_ROPE && has_unit) rope_ask(a, mb0 * 16 + (l0 & 15), rope_pre);
+  if (EPI == EPI_RESIDUAL && has_unit) {
+    const bf16_t* from = a.residual + (size_t)min(mb0 * 16 + (l0 & 15), a.M - 1) * a.ldr;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) res_pre[j] = from[min((g * NT + t0) * TH + (l0 >> 4) * 4 + j, a.N - 1)];
   }
-
   f32x4_t acc[NT][MB];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) acc[t][mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
   int ks = ks0;
-  if (k_exact) {
-    for (; ks + U <= ks1; ks += U) {
-      bf16x8_t w[U][NT], av[U][MB];
+  if ((a.K & 31) == 0) {
+    bf16x8_t w[U][NT], av[U][MB];
+    auto load = [&](int u, int step) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
+      for (int t = 0; t < NT; ++t) w[u][t] = *(const bf16x8_t*)(wp[t] + (size_t)step * 32);
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          if (has_row) {
-            w[u][t] = *(const bf16x8_t*)(wp[t] + (size_t)(ks + u) * 32);
-          } else {
-            w[u][t] = zero8();
-          }
-        }
+      for (int mb = 0; mb < MB; ++mb) av[u][mb] = *(const bf16x8_t*)(ap[mb] + (size_t)step * 32);
+    };
+    auto multiply = [&](int u) {
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) av[u][mb] = *(const bf16x8_t*)(ap[mb] + (size_t)(ks + u) * 32);
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+          acc[t][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][t], av[u][mb], acc[t][mb], 0, 0, 0);
+    };
+    // first as many steps as leave whole groups of U; the loads of the steps that are not there repeat the last one, so that
+    // no branch stands between the loads
+    const int some = (ks1 - ks0 + U - 1) % U + 1;
+#pragma unroll
+    for (int u = 0; u < U; ++u) load(u, ks0 + min(u, some - 1));
+    if (EPI == EPI_ROPE && has_unit) rope_ask_further(a, rope_head, rope_col + (l0 >> 4) * 4, rope_pre);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (u < some) multiply(u);
+    for (ks += some; ks < ks1; ks += U) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) load(u, ks + u);
+#pragma unroll
+      for (int u = 0; u < U; ++u) multiply(u);
+    }
+  } else {
+    if (EPI == EPI_ROPE && has_unit) rope_ask_further(a, rope_head, rope_col + (l0 >> 4) * 4, rope_pre);
+    for (; ks < ks1; ++ks) {
+      // a step may reach past K (K is a multiple of 8): read a valid chunk and zero the weight
+      const bool k_ok = ks * 32 + q * 8 < a.K;
+      const long off = k_ok ? (long)ks * 32 : -(long)(q * 8);
+      bf16x8_t w[NT], av[MB];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        w[t] = *(const bf16x8_t*)(wp[t] + off);
+        if (!k_ok) w[t] = zero8();
       }
 #pragma unroll
-      for (int u = 0; u < U; ++u)
+      for (int mb = 0; mb < MB; ++mb) av[mb] = *(const bf16x8_t*)(ap[mb] + off);
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int mb = 0; mb < MB; ++mb)
-            acc[t][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][t], av[u][mb], acc[t][mb], 0, 0, 0);
+        for (int mb = 0; mb < MB; ++mb)
+          acc[t][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], av[mb], acc[t][mb], 0, 0, 0);
     }
-  }
-  for (; ks < ks1; ++ks) {
-    // a step may reach past K (K is a multiple of 8): read a valid chunk and zero the weight
-    const bool k_ok = ks * 32 + q * 8 < a.K;
-    const long off = k_ok ? (long)ks * 32 : -(long)(q * 8);
-    bf16x8_t w[NT], av[MB];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      w[t] = *(const bf16x8_t*)(wp[t] + off);
-      if (!k_ok || !has_row) w[t] = zero8();
-    }
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) av[mb] = *(const bf16x8_t*)(ap[mb] + off);
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-        acc[t][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], av[mb], acc[t][mb], 0, 0, 0);
   }
 
+  float* scales = (float*)smem;
+  f32x4_t* red = (f32x4_t*)(smem + (NORM ? 16 * MB * sizeof(float) : 0));
   // add the wavefronts' partial sums in wavefront order (with FOLD: the first half of K, then the second)
   if (WK > 1 || FOLD) {
 #pragma unroll
@@ -388,22 +411,33 @@ __global__ __launch_bounds__(SK_MAX_WAVES * 64) void gemm_skinny_kernel(GemmArgs
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) red[(wave * NT * MB + t * MB + mb) * 64 + lane] = acc[t][mb];
   }
+  if (NORM) row_scales<MB>(a, scales, parts_pre, wave, lane, WK);
   if (WK > 1 || NORM || FOLD) __syncthreads();
-  for (int u = tid; u < UNITS; u += blockDim.x) {
+  // the sum of `WK` values that lie `apart` from each other, in order; four are on their way together
+  auto add_up = [&](f32x4_t& s, const f32x4_t* at, int apart) {
+    int w = 0;
+    for (; w + 4 <= WK; w += 4) {
+      const f32x4_t v0 = at[w * apart], v1 = at[(w + 1) * apart], v2 = at[(w + 2) * apart], v3 = at[(w + 3) * apart];
+      s += v0;
+      s += v1;
+      s += v2;
+      s += v3;
+    }
+    for (; w < WK; ++w) s += at[w * apart];
+  };
+  for (int u = tid; u < UNITS; u += WK * 64) {
     const int l = u & 63, mb = (u >> 6) % MB, t = (u >> 6) / MB;
     const int token = mb * 16 + (l & 15), qq = l >> 4;
     f32x4_t s0 = f32x4_t{0.f, 0.f, 0.f, 0.f}, s1 = s0;
     if (FOLD) {
       // the second half's sums of (token, rows 4 qq ..) lie 8 tokens and 8 rows on: 8 + 2 * 16 lanes
       if (token < 8 && qq < 2) {
-        for (int w = 0; w < WK; ++w) s0 += red[w * 64 + l];
-        for (int w = 0; w < WK; ++w) s0 += red[w * 64 + l + 40];
+        add_up(s0, red + l, 64);
+        add_up(s0, red + l + 40, 64);
       }
     } else if (WK > 1) {
-      for (int w = 0; w < WK; ++w) {
-        s0 += red[(w * NT * MB + t * MB + mb) * 64 + l];
-        if (PAIRED) s1 += red[(w * NT * MB + MB + mb) * 64 + l];
-      }
+      add_up(s0, red + (t * MB + mb) * 64 + l, NT * MB * 64);
+      if (PAIRED) add_up(s1, red + (MB + mb) * 64 + l, NT * MB * 64);
     } else {
       // one wavefront: unit u is this very lane's accumulator (u < 64 * NT * MB, tid == lane)
 #pragma unroll
@@ -417,23 +451,26 @@ __global__ __launch_bounds__(SK_MAX_WAVES * 64) void gemm_skinny_kernel(GemmArgs
     const float scale = NORM ? scales[token] : 1.0f;
     const bool live = qq * 4 < TH && token < a.M;  // (with FOLD: M is 8 at most)
     if (EPI == EPI_ROPE) {
-      if (live)
-        rope_store(a, s0 * scale, s1 * scale, token, rope_head, rope_col + qq * 4,
-                   u == tid ? rope_pre : rope_operands(a, token, rope_head, rope_col + qq * 4));
+      if (u != tid) {
+        rope_ask(a, token, rope_pre);
+        rope_ask_further(a, rope_head, rope_col + qq * 4, rope_pre);
+      }
+      if (live) rope_store(a, s0 * scale, s1 * scale, token, rope_head, rope_col + qq * 4, rope_pre);
     } else {
       const int tile = PAIRED ? g : g * NT + t;
       const int n = tile * TH + qq * 4;
-      if (EPI == EPI_RESIDUAL && a.emit_w != nullptr) {
+      if (EPI == EPI_RESIDUAL) {
         float x[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          x[j] = (live && n + j < a.N)
-                     ? round_to<bf16_t>(s0[j] * scale + bias_at(a, n + j, a.N)) +
-                           __bfloat162float(a.residual[(size_t)token * a.ldr + n + j])
-                     : 0.f;
-        emit_for_norm(a, x, live && n < a.N, token, n, tile, l);
+        for (int j = 0; j < 4; ++j) {
+          const float res = __bfloat162float(u == tid ? res_pre[j] : a.residual[(size_t)min(token, a.M - 1) * a.ldr + min(n + j, a.N - 1)]);
+          x[j] = live && n + j < a.N ? round_to<bf16_t>(s0[j] * scale + bias_at(a, n + j, a.N)) + res : 0.f;
+        }
+        if (a.emit_w != nullptr) emit_for_norm(a, x, live && n < a.N, token, n, tile, l);
+        if (live) store_rounded(a, x, token, n);
+      } else if (live) {
+        store4<EPI>(a, s0, s1, scale, token, n);
       }
-      if (live) store4<EPI>(a, s0, s1, scale, token, n);
     }
   }
 }
@@ -466,7 +503,6 @@ __global__ __launch_bounds__(1024) void gemm_staged_kernel(GemmArgs a) {
   unsigned char* stage = smem + (NORM ? 16 * MB * sizeof(float) : 0);
   bf16x8_t* stage_v = (bf16x8_t*)stage;  // [buffer][wk][step][mb][lane]
   f32x4_t* red = (f32x4_t*)stage;         // [wk][wn][NT * MB][lane], after the last round
-  if (NORM) row_scales<MB>(a, scales);
 
   const int unit = blockIdx.x * ST_WN + wn;  // SwiGLU: a pair of tiles; else NT tiles
   const bf16_t* wp[NT];
@@ -527,6 +563,7 @@ __global__ __launch_bounds__(1024) void gemm_staged_kernel(GemmArgs a) {
   bf16x8_t w_cur[ST_SC][NT], piece[MB];
   load_w(0, w_cur);
   load_a(0, piece);
+  if (NORM) row_scales<MB>(a, scales, row_parts(a, wave, lane), wave, lane, nwaves);
   store_a(0, piece);
   __syncthreads();
   int buf = 0;
@@ -650,8 +687,9 @@ __global__ __launch_bounds__(256, 2) void gemm_glu_stream_kernel(GemmArgs a) {
       load_to_lds(src[i] + k, base + (unsigned)(row * GL_K * sizeof(bf16_t)));
     }
   };
+  f32x4_t parts = {0.f, 0.f, 0.f, 0.f};
+  if (NORM) parts = row_parts(a, wave, lane);  // (asked for first, used behind the last step: nothing waits for them in between)
   for (int s = 0; s < S - 1 && s < steps; ++s) ask(s);
-  if (NORM) row_scales<MB>(a, scales);
   f32x4_t acc[NB];
 #pragma unroll
   for (int mb = 0; mb < NB; ++mb) acc[mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -672,6 +710,10 @@ __global__ __launch_bounds__(256, 2) void gemm_glu_stream_kernel(GemmArgs a) {
         acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, av, acc[mb], 0, 0, 0);
       }
     }
+  }
+  if (NORM) {
+    row_scales<MB>(a, scales, parts, wave, lane, 4);
+    __syncthreads();
   }
   // lanes of q < 2 hold gate rows 4 q + j, those of q + 2 the same rows of up
 #pragma unroll
@@ -694,12 +736,18 @@ static bool allow_lds(Kernel kernel, size_t lds) {
 }
 
 template <int MB, int NT, int EPI, bool NORM, bool FOLD = false>
-static bool launch_skinny_one(const GemmArgs& a, int groups, int WK, hipStream_t stream) {
+static bool launch_skinny_one(const GemmArgs& given, int groups, int WK, hipStream_t stream) {
+  GemmArgs a = given;
+  const int steps = FOLD ? a.K / 64 : (a.K + 31) / 32;
+  a.waves = WK;
+  a.share = steps / WK;
+  a.spare = steps % WK;
+  const dim3 grid = EPI == EPI_ROPE ? dim3(groups / (a.nq + 2 * a.nkv), a.nq + 2 * a.nkv) : dim3(groups);  // (a head's pairs of tiles, the heads)
   size_t lds = (WK > 1 || FOLD) ? (size_t)WK * NT * MB * 64 * sizeof(f32x4_t) : 0;
   if (NORM) lds += (size_t)16 * MB * sizeof(float);
   auto kernel = gemm_skinny_kernel<MB, NT, EPI, NORM, FOLD>;
   if (!allow_lds(kernel, lds)) return false;
-  hipLaunchKernelGGL(kernel, dim3(groups), dim3(WK * 64), lds, stream, a);
+  hipLaunchKernelGGL(kernel, grid, dim3(WK * 64), lds, stream, a);
   return true;
 }
 
@@ -946,7 +994,7 @@ TK_API int tk_gemm_skinny_bf16(const void* A, int lda, const void* W, void* C, i
     }
     const int lds_cap = 65536 / (NT * MB * 64 * (int)sizeof(f32x4_t));
     if (WK > lds_cap) WK = lds_cap;
-    if (WK > SK_MAX_WAVES) WK = SK_MAX_WAVES;
+    if (WK > sk_max_waves(NT)) WK = sk_max_waves(NT);
     if (WK > steps) WK = steps;
     if (WK < 1) WK = 1;
     if (folded) {

@@ -141,89 +141,117 @@ TK_API int tk_gemm_split_bf16(const void* A, int lda, const void* W, float* part
 // The passes that add the cuts
 // ---------------------------------------------------------------------------------
 
-// the sum over the cuts of 8 outputs from `at` on, rounded to bfloat16 as a product that is stored is
-__device__ __forceinline__ void product8(const float* part, size_t apart, int cuts, size_t at, float (&v)[8]) {
-  f32x4_t lo = *(const f32x4_t*)(part + at), hi = *(const f32x4_t*)(part + at + 4);
-#pragma unroll 4
-  for (int c = 1; c < cuts; ++c) {
-    lo += *(const f32x4_t*)(part + c * apart + at);
-    hi += *(const f32x4_t*)(part + c * apart + at + 4);
-  }
+// Both passes are bound by their chain of waits: the bytes are few, a launch takes 1.6 us, and every trip to sums that other dies
+// have just written 0.8 or more.  So all that a thread reads is asked for at once: the first G cuts (of cuts that are not there
+// the last one again: no branch stands between the loads) beside the residual row and the norm's weight.
+
+// the cuts' values at `at`, 4 outputs each: the first G cuts asked for together, all added in ascending order
+template <int G>
+struct CutSums {
+  f32x4_t v[G];
+  __device__ __forceinline__ void ask(const float* part, size_t apart, int cuts, size_t at) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    v[j] = round_to<bf16_t>(lo[j]);
-    v[4 + j] = round_to<bf16_t>(hi[j]);
+    for (int c = 0; c < G; ++c) v[c] = *(const f32x4_t*)(part + min(c, cuts - 1) * apart + at);
   }
-}
+  __device__ __forceinline__ f32x4_t sum(const float* part, size_t apart, int cuts, size_t at) const {
+    f32x4_t s = v[0];
+#pragma unroll
+    for (int c = 1; c < G; ++c)
+      if (c < cuts) s += v[c];
+#pragma unroll 4
+    for (int c = G; c < cuts; ++c) s += *(const f32x4_t*)(part + c * apart + at);
+    return s;
+  }
+};
 
 // stream_out = product + residual (rounded); out = RMSNorm(stream_out) * w: a workgroup a row, the arithmetic of
-// rmsnorm_packed_kernel.  A thread keeps the first SN_HELD pieces of 8 that it takes in registers.  once: the normed value is not
+// rmsnorm_packed_kernel.  A thread keeps the first HELD pieces of 8 that it takes in registers.  once: the normed value is not
 // rounded in front of the weight.  Rows that few go through the weight-streaming kernel round an operand of the next product
 // once (x w, the row's factor on the 32-bit sums), and keep that where the split form takes its place: 8 rows of 2,048 against
 // 64 bits 1.7e-3 of the norm, rounded twice 2.4e-3.
-#define SN_HELD 4
+template <int HELD, int G>
 __global__ __launch_bounds__(256) void split_add_rmsnorm_kernel(const float* __restrict__ part, int cuts, const bf16_t* __restrict__ residual,
                                                                 const void* __restrict__ w, int w_f32, bf16_t* __restrict__ stream_out,
                                                                 bf16_t* __restrict__ out, int rows, int hidden, float eps, int once) {
-  __shared__ float red[16];
+  __shared__ float red[4];
   const size_t base = (size_t)blockIdx.x * hidden, apart = (size_t)rows * hidden;
   const int pieces = hidden / 8;
-  float held[SN_HELD][8];
+  CutSums<G> lo[HELD], hi[HELD];
+  Pack<bf16_t> res[HELD];
+  struct Weights { f32x4_t a, b; } wp[HELD];  // 8 floats, or 8 of 16 bits in `a`
+  auto weights = [&](int piece) {
+    const char* from = (const char*)w + (size_t)piece * (w_f32 ? 32 : 16);
+    Weights v;
+    v.a = *(const f32x4_t*)from;
+    v.b = *(const f32x4_t*)(w_f32 ? from + 16 : from);
+    return v;
+  };
+  auto weight = [&](const Weights& v, int j) {
+    const unsigned two = __float_as_uint(v.a[j / 2]);
+    const float narrow = __uint_as_float(j & 1 ? two & 0xffff0000u : two << 16);
+    return w_f32 ? (j < 4 ? v.a[j & 3] : v.b[j & 3]) : narrow;
+  };
+#pragma unroll
+  for (int c = 0; c < HELD; ++c) {
+    const int piece = min((int)threadIdx.x + c * 256, pieces - 1);
+    const size_t at = base + (size_t)piece * 8;
+    lo[c].ask(part, apart, cuts, at);
+    hi[c].ask(part, apart, cuts, at + 4);
+    res[c].load(residual + at);
+  }
+#pragma unroll
+  for (int c = 0; c < HELD; ++c) wp[c] = weights(min((int)threadIdx.x + c * 256, pieces - 1));
+  float held[HELD][8];
   float ss = 0.f;
-  auto take = [&](int piece, float (&v)[8]) {
-    Pack<bf16_t> r, s;
-    r.load(residual + base + (size_t)piece * 8);
-    product8(part, apart, cuts, base + (size_t)piece * 8, v);
+  // the product rounded as one that is stored is, + the residual, rounded
+  auto take = [&](int piece, f32x4_t a, f32x4_t b, const Pack<bf16_t>& r, float (&v)[8]) {
+    Pack<bf16_t> s;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      v[j] = round_to<bf16_t>(v[j] + to_f32<bf16_t>(r.v[j]));
+      v[j] = round_to<bf16_t>(round_to<bf16_t>(j < 4 ? a[j & 3] : b[j & 3]) + to_f32<bf16_t>(r.v[j]));
       s.v[j] = from_f32<bf16_t>(v[j]);
       ss += v[j] * v[j];
     }
     s.store(stream_out + base + (size_t)piece * 8);
   };
-  auto weights = [&](int piece, float (&wf)[8]) {
-    if (w_f32) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) wf[j] = ((const float*)w)[(size_t)piece * 8 + j];
-    } else {
-      Pack<bf16_t> wp;
-      wp.load((const bf16_t*)w + (size_t)piece * 8);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) wf[j] = to_f32<bf16_t>(wp.v[j]);
-    }
-  };
-#pragma unroll
-  for (int c = 0; c < SN_HELD; ++c) {
+  for (int c = 0; c < HELD; ++c) {
     const int piece = threadIdx.x + c * 256;
-    if (piece < pieces) take(piece, held[c]);
+    const size_t at = base + (size_t)piece * 8;
+    if (piece < pieces) take(piece, lo[c].sum(part, apart, cuts, at), hi[c].sum(part, apart, cuts, at + 4), res[c], held[c]);
   }
-  for (int piece = threadIdx.x + SN_HELD * 256; piece < pieces; piece += 256) {
+  for (int piece = threadIdx.x + HELD * 256; piece < pieces; piece += 256) {
+    const size_t at = base + (size_t)piece * 8;
+    Pack<bf16_t> r;
     float v[8];
-    take(piece, v);
+    r.load(residual + at);
+    lo[0].ask(part, apart, cuts, at);
+    hi[0].ask(part, apart, cuts, at + 4);
+    take(piece, lo[0].sum(part, apart, cuts, at), hi[0].sum(part, apart, cuts, at + 4), r, v);
   }
-  ss = block_sum(ss, red);
-  const float rstd = 1.0f / sqrtf(ss / (float)hidden + eps);
-  auto give = [&](int piece, const float (&v)[8]) {
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  const float rstd = 1.0f / sqrtf((((0.f + red[0]) + red[1]) + red[2] + red[3]) / (float)hidden + eps);
+  auto give = [&](int piece, const Weights& wv, const float (&v)[8]) {
     Pack<bf16_t> o;
-    float wf[8];
-    weights(piece, wf);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o.v[j] = from_f32<bf16_t>(wf[j] * (once ? v[j] * rstd : round_to<bf16_t>(v[j] * rstd)));
+    for (int j = 0; j < 8; ++j)
+      o.v[j] = from_f32<bf16_t>(weight(wv, j) * (once ? v[j] * rstd : round_to<bf16_t>(v[j] * rstd)));
     o.store(out + base + (size_t)piece * 8);
   };
 #pragma unroll
-  for (int c = 0; c < SN_HELD; ++c) {
+  for (int c = 0; c < HELD; ++c) {
     const int piece = threadIdx.x + c * 256;
-    if (piece < pieces) give(piece, held[c]);
+    if (piece < pieces) give(piece, wp[c], held[c]);
   }
-  for (int piece = threadIdx.x + SN_HELD * 256; piece < pieces; piece += 256) {
+  for (int piece = threadIdx.x + HELD * 256; piece < pieces; piece += 256) {
     Pack<bf16_t> a;
     a.load(stream_out + base + (size_t)piece * 8);  // a thread reads back what it wrote
     float v[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = to_f32<bf16_t>(a.v[j]);
-    give(piece, v);
+    give(piece, weights(piece), v);
   }
 }
 
@@ -235,7 +263,11 @@ TK_API int tk_split_add_rmsnorm(const float* part, int cuts, const void* residua
              "split_add_rmsnorm: operands must be 16-byte aligned");
   TK_REQUIRE(out != residual && out != stream_out && stream_out != residual, "split_add_rmsnorm: inputs and outputs must not share a buffer");
   if (rows == 0) return 0;
-  hipLaunchKernelGGL(split_add_rmsnorm_kernel, dim3(rows), dim3(256), 0, stream, part, cuts, (const bf16_t*)residual, w, w_f32,
+  const int held = hidden <= 2048 ? 1 : (hidden <= 4096 ? 2 : 4);  // (a row in registers as far as 8,192)
+  auto kernel = held == 4 ? split_add_rmsnorm_kernel<4, 4>
+                          : (cuts <= 4 ? (held == 1 ? split_add_rmsnorm_kernel<1, 4> : split_add_rmsnorm_kernel<2, 4>)
+                                       : (held == 1 ? split_add_rmsnorm_kernel<1, 8> : split_add_rmsnorm_kernel<2, 8>));
+  hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, stream, part, cuts, (const bf16_t*)residual, w, w_f32,
                      (bf16_t*)stream_out, (bf16_t*)out, rows, hidden, eps, once);
   TK_CHECK_LAUNCH("split_add_rmsnorm");
   return 0;
@@ -244,6 +276,7 @@ TK_API int tk_split_add_rmsnorm(const float* part, int cuts, const void* residua
 // The stacked q, k, v product's cuts added, q and k rotated (element j of a head with element j + d / 2; without tables they
 // pass as they are), q to `q` [rows, nq * d], k and v to the token's page.  A workgroup a token and `share` of its units, a
 // unit 4 neighbouring columns of one half of a head and the same 4 of the other.
+template <int G>
 __global__ __launch_bounds__(256) void split_rope_append_kernel(const float* __restrict__ part, int cuts, bf16_t* __restrict__ q,
                                                                 const int* __restrict__ positions, const int* __restrict__ token_req,
                                                                 const int* __restrict__ block_table, int table_stride,
@@ -256,20 +289,19 @@ __global__ __launch_bounds__(256) void split_rope_append_kernel(const float* __r
   const int h = u / each, c = (u - h * each) * 4;
   const int width = (nq + 2 * nkv) * d;
   const size_t apart = (size_t)rows * width, at = (size_t)t * width + h * d + c;
-  const int pos = positions[t];
-  f32x4_t lo = *(const f32x4_t*)(part + at), hi = *(const f32x4_t*)(part + at + half);
+  // (positions and requests first: what they lead to is asked for while the sums are on their way)
+  const int pos = positions[t], req = token_req[t];
+  CutSums<G> slo, shi;
+  slo.ask(part, apart, cuts, at);
+  shi.ask(part, apart, cuts, at + half);
   f32x4_t cs = {1.f, 1.f, 1.f, 1.f}, sn = {0.f, 0.f, 0.f, 0.f};
   const bool rotate = h < nq + nkv && cos_t != nullptr;
   if (rotate) {
     cs = *(const f32x4_t*)(cos_t + (size_t)pos * half + c);
     sn = *(const f32x4_t*)(sin_t + (size_t)pos * half + c);
   }
-  const int page = h >= nq ? block_table[(size_t)token_req[t] * table_stride + pos / P] : 0;
-#pragma unroll 4
-  for (int i = 1; i < cuts; ++i) {
-    lo += *(const f32x4_t*)(part + i * apart + at);
-    hi += *(const f32x4_t*)(part + i * apart + at + half);
-  }
+  const int page = h >= nq ? block_table[(size_t)req * table_stride + pos / P] : 0;
+  const f32x4_t lo = slo.sum(part, apart, cuts, at), hi = shi.sum(part, apart, cuts, at + half);
   union { bf16_t h[4]; uint2 u; } o1, o2;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -313,7 +345,8 @@ TK_API int tk_split_rope_append(const float* part, int cuts, void* q, const int*
              "split_rope_append: operands must be 16-byte aligned");
   if (rows == 0) return 0;
   const int units = (nq + 2 * nkv) * (d / 8);
-  hipLaunchKernelGGL(split_rope_append_kernel, dim3(rows, (units + 255) / 256), dim3(256), 0, stream, part, cuts, (bf16_t*)q, positions,
+  auto kernel = cuts <= 4 ? split_rope_append_kernel<4> : split_rope_append_kernel<8>;
+  hipLaunchKernelGGL(kernel, dim3(rows, (units + 255) / 256), dim3(256), 0, stream, part, cuts, (bf16_t*)q, positions,
                      token_req, block_table, table_stride, cos_t, sin_t, (bf16_t*)kcache, (bf16_t*)vcache, rows, nq, nkv, d, P);
   TK_CHECK_LAUNCH("split_rope_append");
   return 0;
