@@ -1,0 +1,64 @@
+"""The weight-streaming and the streamed gate and up products with a norm in front, at the edges of what is asked for early: rows
+beyond a wavefront's first, partial sums that are as many as the lanes take, more, and no multiple of 4; and a rotation
+behind a folded K."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from tokasaurus_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _norm(m, k, parts, gen):
+    x = torch.randn((m, k), generator=gen, device="cuda").bfloat16()
+    sumsq = torch.rand((m, parts), generator=gen, device="cuda") * 2 * k / parts
+    return ops.Prenorm(x, sumsq), x.double() / torch.sqrt(sumsq.double().sum(1, keepdim=True) / k + 1e-5)
+
+
+@pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("parts", [4, 252, 256, 260, 6])
+def test_norm_in_front(m, parts):
+    """32-bit sums of k products and of the partial sums, the factor's root and division: (k + parts + 8) 2^-24 of the sum of the
+    magnitudes; the activation behind gate and up rounds three times to 8 bits."""
+    gen = torch.Generator(device="cuda").manual_seed(m + parts)
+    n, k = 264, 448
+    pre, rows = _norm(m, k, parts, gen)
+    w = (torch.randn((2 * n, k), generator=gen, device="cuda") / k ** 0.5).bfloat16()
+    want, size = rows @ w.double().T, rows.abs() @ w.double().abs().T
+    for kw in ({}, {"tile_rows": 8}, {"staged": 1}):
+        got = ops.gemm_skinny_bf16(pre.scaled, w, prenorm=pre, norm_eps=1e-5, out_f32=True, **kw)
+        assert ((got.double() - want).abs() <= (k + parts + 8) * 2.0 ** -24 * size).all(), kw
+    got = ops.gemm_skinny_bf16(pre.scaled, w, prenorm=pre, norm_eps=1e-5, swiglu=True, staged=2)
+    gate, up = want[:, :n], want[:, n:]
+    # a rounding to 8 significant bits is off by 2^-8 of the value at most: gate (silu's slope is at most 1.1), up, silu, the product
+    s = torch.nn.functional.silu(gate)
+    bound = 2.0 ** -8 * (1.1 * gate.abs() * up.abs() + 3 * (s * up).abs()) * 1.1 + 1e-6
+    assert ((got.double() - s * up).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("m", [1, 3, 8, 9])
+@pytest.mark.parametrize("k", [64, 448, 576, 2048])
+def test_rotation_behind_a_folded_inner_size(m, k):
+    """Queries and pages as the plain product and the rotation kernel leave them, up to the order of the product's 32-bit sums: a rounding
+    of 8 bits falls the other way at most, which is 2^-8 of a pair's length."""
+    gen = torch.Generator(device="cuda").manual_seed(m + k)
+    nq, nkv, d, page = 4, 2, 48, 16
+    width = (nq + 2 * nkv) * d
+    pre, rows = _norm(m, k, 64, gen)
+    w = (torch.randn((width, k), generator=gen, device="cuda") / k ** 0.5).bfloat16()
+    positions = torch.randint(0, 90, (m,), generator=gen, device="cuda").to(torch.int32)
+    req = torch.arange(m, device="cuda", dtype=torch.int32)
+    table = torch.randperm(m * 6, generator=gen, device="cuda").to(torch.int32).view(m, 6)
+    cos, sin = ops.rope_table(1.0 / 10000 ** (torch.arange(0, d, 2, device="cuda").float() / d), 96)
+    pages = [(torch.zeros(ops.key_pages_shape(6 * m, nkv, page, d), device="cuda", dtype=torch.bfloat16),
+              torch.zeros(ops.value_pages_shape(6 * m, nkv, page, d), device="cuda", dtype=torch.bfloat16)) for _ in range(2)]
+    ropes = [ops.RopeAppend(positions, req, table, cos, sin, *p, nq, nkv, d, page) for p in pages]
+    stacked = (rows @ w.double().T).bfloat16()
+    ops.rope_append(stacked, positions, req, table, cos, sin, *pages[0], nq, nkv, d, page)
+    q = ops.gemm_skinny_bf16(pre.scaled, w, rope=ropes[1], tile_rows=8, prenorm=pre, norm_eps=1e-5)
+    largest = float(stacked.double().abs().max())
+    for got, want in ((q, stacked[:, : nq * d]), (pages[1][0], pages[0][0]), (pages[1][1], pages[0][1])):
+        assert float((got.double() - want.double()).abs().max()) <= 2.0 ** -7 * largest

@@ -50,7 +50,14 @@ struct GemmArgs {
   int lda, M, N, K;  // N: outputs (for SwiGLU the intermediate size; W then has 2N rows, gate first)
   int TH;            // weight rows of a tile that are used (16, or 8 to make twice the workgroups of a narrow output)
   int waves, share, spare;  // skinny kernel: wavefronts that split K, steps of each, wavefronts that take one more
+  int each_die;  // workgroups whose tiles are neighbours on a die (0: tiles in the order of the workgroups)
   int turn;  // streamed gate and up: mask of the step of K that a workgroup begins at (0: all begin with the first)
+  // norm in front: where a row's partial sums can be asked for without a look at how many there are (row_parts)
+  const float* early;
+  int early_apart, early_lanes;
+  // rotation with append
+  const int* positions;
+  const int* token_req;
   void* C;
   int ldc;
   const bf16_t* residual;
@@ -68,8 +75,6 @@ struct GemmArgs {
   float* emit_sumsq;
   int parts_out;
   // rotation with append
-  const int* positions;
-  const int* token_req;
   const int* block_table;
   int table_stride;
   const float* cos_t;  // [positions][d / 2], null: no rotation
@@ -150,51 +155,75 @@ __device__ __forceinline__ bf16x8_t zero8() {
 // 1 / rms of every row of A from the partial sums its producer left, into LDS `scale`
 // (16 * MB floats).  A wavefront takes a row at a time: every lane adds 4 parts (one
 // 16-byte load), then the lanes' sums are added by a butterfly, so the order is fixed.
-// What the first row's first 256 parts are is asked for at a kernel's beginning (row_parts) and
-// used at its end: only the epilogue needs the factors, and a wait for them in front of the
-// weights' loads is a trip to memory that nothing else fills.
-__device__ __forceinline__ f32x4_t row_parts(const GemmArgs& a, int wave, int lane) {
-  f32x4_t v = {0.f, 0.f, 0.f, 0.f};
-  if ((a.parts_in & 3) == 0 && lane * 4 < a.parts_in) v = *(const f32x4_t*)(a.sumsq_in + (size_t)min(wave, a.M - 1) * a.parts_in + lane * 4);
-  return v;
+// A wavefront's first row is asked for at a kernel's beginning (row_parts), with no branch in front of the weights' loads, and
+// added up while those are on their way; that takes rows of up to 256 partial sums, a multiple of 4 (early_lanes > 0).
+__device__ __forceinline__ const f32x4_t* row_parts(const GemmArgs& a, int row, int lane) {
+  return (const f32x4_t*)(a.early + (size_t)min(row, a.M - 1) * a.early_apart + (lane < a.early_lanes ? lane * 4 : 0));
 }
 
+__device__ __forceinline__ float row_scale(const GemmArgs& a, float ss) { return 1.0f / sqrtf(wave_sum(ss) / (float)a.K + a.eps); }
+
+__device__ __forceinline__ void early_row_scale(const GemmArgs& a, float* scale, f32x4_t v, int row, int lane) {
+  if (a.early_lanes == 0 || row >= a.M) return;
+  const float f = row_scale(a, lane < a.early_lanes ? (v[0] + v[1]) + (v[2] + v[3]) : 0.f);
+  if (lane == 0) scale[row] = f;
+}
+
+// the rows that are left behind `early` of the wavefront's, every `nwaves`-th
 template <int MB>
-__device__ __forceinline__ void row_scales(const GemmArgs& a, float* scale, f32x4_t first, int wave, int lane, int nwaves) {
+__device__ __forceinline__ void row_scales(const GemmArgs& a, float* scale, int wave, int lane, int nwaves, int early = 1) {
   const int rows = min(a.M, 16 * MB);
   const bool vec = (a.parts_in & 3) == 0;
-  for (int token = wave; token < rows; token += nwaves) {
+  for (int token = a.early_lanes > 0 ? wave + early * nwaves : wave; token < rows; token += nwaves) {
     const float* part = a.sumsq_in + (size_t)token * a.parts_in;
     float ss = 0.f;
     for (int p = lane * 4; p < a.parts_in; p += 256) {
       if (vec) {
-        const f32x4_t v = token == wave && p < 256 ? first : *(const f32x4_t*)(part + p);
+        const f32x4_t v = *(const f32x4_t*)(part + p);
         ss += (v[0] + v[1]) + (v[2] + v[3]);
       } else {
         for (int j = 0; j < 4 && p + j < a.parts_in; ++j) ss += part[p + j];
       }
     }
-    ss = wave_sum(ss);
-    if (lane == 0) scale[token] = 1.0f / sqrtf(ss / (float)a.K + a.eps);
+    const float f = row_scale(a, ss);
+    if (lane == 0) scale[token] = f;
   }
 }
 
 // The residual epilogue's extra outputs for the norm that follows: x * w rounded once,
 // and the sum of x^2 over this tile's columns.  All 64 lanes of a wavefront call this
 // together; lanes (token, qq = 0..3) share a token.
-__device__ __forceinline__ void emit_for_norm(const GemmArgs& a, const float (&x)[4], bool live, int token,
+// Its weights of outputs n .. n + 3, asked for without a branch on their type: the 4 bytes that hold a weight, and the weight.
+__device__ __forceinline__ void emit_ask(const GemmArgs& a, int n, unsigned (&w)[4]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const char* at = (const char*)a.emit_w + (size_t)min(n + j, a.N - 1) * (a.emit_w_f32 ? 4 : 2);
+    w[j] = *(const unsigned*)(at - ((uintptr_t)at & 3));
+  }
+}
+__device__ __forceinline__ float emit_weight(const GemmArgs& a, int n, int j, unsigned w) {
+  const bool upper = (((uintptr_t)a.emit_w + (size_t)min(n + j, a.N - 1) * 2) & 2) != 0;
+  return __uint_as_float(a.emit_w_f32 ? w : (upper ? w & 0xffff0000u : w << 16));
+}
+
+__device__ __forceinline__ void emit_for_norm(const GemmArgs& a, const float (&x)[4], const unsigned (&w)[4], bool live, int token,
                                               int n, int part, int lane) {
   float ss = 0.f;
   if (live) {
     bf16_t* dst = a.emit_scaled + (size_t)token * a.ld_emit + n;
+    union { bf16_t h[4]; uint2 u; } pk;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if (n + j < a.N) {
-        const float xr = round_to<bf16_t>(x[j]);
-        const float w = a.emit_w_f32 ? ((const float*)a.emit_w)[n + j] : __bfloat162float(((const bf16_t*)a.emit_w)[n + j]);
-        ss = fmaf(xr, xr, ss);
-        dst[j] = __float2bfloat16(w * xr);
-      }
+      const float xr = n + j < a.N ? round_to<bf16_t>(x[j]) : 0.f;
+      ss = fmaf(xr, xr, ss);
+      pk.h[j] = __float2bfloat16(emit_weight(a, n, j, w[j]) * xr);
+    }
+    if (n + 3 < a.N && (a.ld_emit & 3) == 0) {
+      *(uint2*)dst = pk.u;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (n + j < a.N) dst[j] = pk.h[j];
     }
   }
   const float s1 = __shfl_xor(ss, 16, 64);
@@ -222,7 +251,7 @@ __device__ __forceinline__ void rope_ask(const GemmArgs& a, int token, RopeOpera
 
 __device__ __forceinline__ void rope_ask_further(const GemmArgs& a, int h, int c, RopeOperands& r) {
   const int half = a.d >> 1;
-  r.page = h >= a.nq ? a.block_table[(size_t)r.req * a.table_stride + r.pos / a.P] : 0;
+  r.page = a.block_table[(size_t)r.req * a.table_stride + r.pos / a.P];  // (for the query heads too: no branch)
   const bool on = h < a.nq + a.nkv && a.cos_t != nullptr && c < half;  // (half and c are multiples of 4)
   r.cs = on ? *(const f32x4_any_t*)(a.cos_t + (size_t)r.pos * half + c) : f32x4_any_t{1.f, 1.f, 1.f, 1.f};
   r.sn = on ? *(const f32x4_any_t*)(a.sin_t + (size_t)r.pos * half + c) : f32x4_any_t{0.f, 0.f, 0.f, 0.f};
@@ -286,11 +315,12 @@ __host__ __device__ constexpr int sk_max_waves(int NT) { return NT == 2 ? 8 : 16
 // LDS of the skinny kernel: [scales: 16 * MB floats when NORM][sums: waves * NT * MB * 64 f32x4]
 // FOLD (up to 8 rows of A, tiles of 8 weight rows, K a multiple of 64): a tile of 8 rows leaves
 // half of the matrix core's 16 rows, and up to 8 rows of A half of its 16 columns, unused.  The
-// upper 8 lanes of every 16 then take the same weight rows and the same rows of A over the second
-// half of K: one product adds both halves' terms, into different quarters of the result (rows and
-// columns 0..7: the first half of K, 8..15: the second; the other two quarters mix the halves and
-// are not used), and the quarters are added when the wavefronts' sums are.  Every lane loads
-// weights, and a wavefront issues half as many loads for the same bytes.
+// upper 8 lanes of every 16 then take the same weight rows and the same rows of A 32 elements
+// further on: one product adds the terms of 64 elements, into different quarters of the result
+// (rows and columns 0..7: the even blocks of 32, 8..15: the odd ones; the other two quarters mix
+// them and are not used), and the quarters are added when the wavefronts' sums are.  Every lane
+// loads weights, and a load instruction takes whole lines of 128 bytes of 8 rows: with the upper
+// lanes in the other half of K it took 64 bytes of 16 places, and a line came twice.
 //
 // A product of a few megabytes is bound by its chain of waits, not by the bytes: a launch takes 1.6 us of 4.8 (8 MB).
 // So the weights' first loads go out as soon as the addresses are there (the arguments they need lie together, every
@@ -300,14 +330,23 @@ __global__ __launch_bounds__(sk_max_waves(NT) * 64) void gemm_skinny_kernel(Gemm
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int U = (NT + MB <= 3) ? 8 : ((NT + MB <= 6) ? 4 : 2);  // steps whose loads are in flight together
   constexpr bool PAIRED = EPI == EPI_SWIGLU || EPI == EPI_ROPE;     // two tiles that meet in the epilogue
-  static_assert(!FOLD || (MB == 1 && NT == 1 && !PAIRED), "folding K takes one tile of 8 weight rows and up to 8 rows of A");
+  static_assert(!FOLD || (MB == 1 && (NT == 1 || EPI == EPI_ROPE)), "folding K takes one tile of 8 weight rows, or a pair, and up to 8 rows of A");
+  // every argument that a first load needs, in one trip
+  asm volatile("" ::"s"(a.A), "s"(a.W), "s"(a.lda), "s"(a.M), "s"(a.N), "s"(a.K), "s"(a.TH), "s"(a.waves), "s"(a.share), "s"(a.spare));
+  if (NORM) asm volatile("" ::"s"(a.early), "s"(a.early_apart), "s"(a.early_lanes));
+  if (EPI == EPI_ROPE) asm volatile("" ::"s"(a.positions), "s"(a.token_req), "s"(a.d));
+  if (EPI == EPI_RESIDUAL) asm volatile("" ::"s"(a.residual), "s"(a.ldr), "s"(a.emit_w), "s"(a.emit_w_f32), "s"(a.each_die));
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int WK = a.waves;
+  float* scales = (float*)smem;
+  f32x4_t* red = (f32x4_t*)(smem + (NORM ? 16 * MB * sizeof(float) : 0));
   const int r = FOLD ? (lane & 7) : (lane & 15), q = lane >> 4;
-  const int g = blockIdx.x;
-  // steps of 32 that a lane walks (with FOLD: of its half of K)
+  // Workgroups go to the chip's eight dies in turn.  With a norm behind, a die takes neighbouring tiles, so that a line of the three
+  // outputs is one die's: lines that several dies write go to memory in pieces (2,048 x 2,048 at one row 5.6 / 5.2 us).
+  const int g = EPI == EPI_RESIDUAL && a.each_die > 0 ? (int)((blockIdx.x & 7) * a.each_die + (blockIdx.x >> 3)) : (int)blockIdx.x;
+  constexpr int STEP = FOLD ? 64 : 32;  // elements of K a step
   const int ks0 = wave * a.share + min(wave, a.spare), ks1 = ks0 + a.share + (wave < a.spare ? 1 : 0);
-  const size_t fold = FOLD ? (size_t)((lane >> 3) & 1) * (size_t)(a.K >> 1) : 0;  // where this lane's half of K begins
+  const int begin = (FOLD ? (lane & 8) * 4 : 0) + q * 8;  // this lane's place in a step
 
   // rows of W this lane streams (clamped: rows past the end are masked at the store); with tiles of 8 or 12 rows the upper
   // lanes repeat the last one, at no cost to memory and into outputs that are not stored
@@ -324,11 +363,11 @@ __global__ __launch_bounds__(sk_max_waves(NT) * 64) void gemm_skinny_kernel(Gemm
     } else {
       row = min((g * NT + t) * TH + rw, a.N - 1);
     }
-    wp[t] = a.W + (size_t)row * a.K + q * 8 + fold;
+    wp[t] = a.W + (size_t)row * a.K + begin;
   }
   const bf16_t* ap[MB];
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) ap[mb] = a.A + (size_t)min(mb * 16 + r, a.M - 1) * a.lda + q * 8 + fold;
+  for (int mb = 0; mb < MB; ++mb) ap[mb] = a.A + (size_t)min(mb * 16 + r, a.M - 1) * a.lda + begin;
 
   // what the epilogue's first unit of this thread needs besides the sums: asked for in front of the weights, used behind them
   constexpr int UNITS = (PAIRED ? 1 : NT) * MB * 64;
@@ -336,13 +375,15 @@ __global__ __launch_bounds__(sk_max_waves(NT) * 64) void gemm_skinny_kernel(Gemm
   const int l0 = tid & 63, mb0 = wave % MB, t0 = wave / MB;
   RopeOperands rope_pre = {};
   bf16_t res_pre[4] = {};
+  unsigned emit_pre[4] = {};
   f32x4_t parts_pre = {0.f, 0.f, 0.f, 0.f};
-  if (NORM) parts_pre = row_parts(a, wave, lane);
-  if (EPI == EPI_ROPE && has_unit) rope_ask(a, mb0 * 16 + (l0 & 15), rope_pre);
+  if (NORM) parts_pre = *row_parts(a, wave, lane);
+  if (EPI == EPI_ROPE) rope_ask(a, mb0 * 16 + (l0 & 15), rope_pre);
   if (EPI == EPI_RESIDUAL && has_unit) {
     const bf16_t* from = a.residual + (size_t)min(mb0 * 16 + (l0 & 15), a.M - 1) * a.ldr;
 #pragma unroll
     for (int j = 0; j < 4; ++j) res_pre[j] = from[min((g * NT + t0) * TH + (l0 >> 4) * 4 + j, a.N - 1)];
+    if (a.emit_w != nullptr) emit_ask(a, (g * NT + t0) * TH + (l0 >> 4) * 4, emit_pre);
   }
   f32x4_t acc[NT][MB];
 #pragma unroll
@@ -350,13 +391,13 @@ __global__ __launch_bounds__(sk_max_waves(NT) * 64) void gemm_skinny_kernel(Gemm
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) acc[t][mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   int ks = ks0;
-  if ((a.K & 31) == 0) {
+  if (FOLD || (a.K & 31) == 0) {
     bf16x8_t w[U][NT], av[U][MB];
     auto load = [&](int u, int step) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) w[u][t] = *(const bf16x8_t*)(wp[t] + (size_t)step * 32);
+      for (int t = 0; t < NT; ++t) w[u][t] = *(const bf16x8_t*)(wp[t] + (size_t)step * STEP);
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) av[u][mb] = *(const bf16x8_t*)(ap[mb] + (size_t)step * 32);
+      for (int mb = 0; mb < MB; ++mb) av[u][mb] = *(const bf16x8_t*)(ap[mb] + (size_t)step * STEP);
     };
     auto multiply = [&](int u) {
 #pragma unroll
@@ -368,9 +409,12 @@ __global__ __launch_bounds__(sk_max_waves(NT) * 64) void gemm_skinny_kernel(Gemm
     // first as many steps as leave whole groups of U; the loads of the steps that are not there repeat the last one, so that
     // no branch stands between the loads
     const int some = (ks1 - ks0 + U - 1) % U + 1;
+    __builtin_amdgcn_sched_barrier(0);  // (loads return in order: what is waited for first goes out first)
 #pragma unroll
     for (int u = 0; u < U; ++u) load(u, ks0 + min(u, some - 1));
+    __builtin_amdgcn_sched_barrier(0);
     if (EPI == EPI_ROPE && has_unit) rope_ask_further(a, rope_head, rope_col + (l0 >> 4) * 4, rope_pre);
+    if (NORM) early_row_scale(a, scales, parts_pre, wave, lane);
 #pragma unroll
     for (int u = 0; u < U; ++u)
       if (u < some) multiply(u);
@@ -382,6 +426,7 @@ __global__ __launch_bounds__(sk_max_waves(NT) * 64) void gemm_skinny_kernel(Gemm
     }
   } else {
     if (EPI == EPI_ROPE && has_unit) rope_ask_further(a, rope_head, rope_col + (l0 >> 4) * 4, rope_pre);
+    if (NORM) early_row_scale(a, scales, parts_pre, wave, lane);
     for (; ks < ks1; ++ks) {
       // a step may reach past K (K is a multiple of 8): read a valid chunk and zero the weight
       const bool k_ok = ks * 32 + q * 8 < a.K;
@@ -402,16 +447,14 @@ __global__ __launch_bounds__(sk_max_waves(NT) * 64) void gemm_skinny_kernel(Gemm
     }
   }
 
-  float* scales = (float*)smem;
-  f32x4_t* red = (f32x4_t*)(smem + (NORM ? 16 * MB * sizeof(float) : 0));
-  // add the wavefronts' partial sums in wavefront order (with FOLD: the first half of K, then the second)
+  // add the wavefronts' partial sums in wavefront order (with FOLD: the even blocks', then the odd ones')
   if (WK > 1 || FOLD) {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) red[(wave * NT * MB + t * MB + mb) * 64 + lane] = acc[t][mb];
   }
-  if (NORM) row_scales<MB>(a, scales, parts_pre, wave, lane, WK);
+  if (NORM) row_scales<MB>(a, scales, wave, lane, WK);
   if (WK > 1 || NORM || FOLD) __syncthreads();
   // the sum of `WK` values that lie `apart` from each other, in order; four are on their way together
   auto add_up = [&](f32x4_t& s, const f32x4_t* at, int apart) {
@@ -430,10 +473,14 @@ __global__ __launch_bounds__(sk_max_waves(NT) * 64) void gemm_skinny_kernel(Gemm
     const int token = mb * 16 + (l & 15), qq = l >> 4;
     f32x4_t s0 = f32x4_t{0.f, 0.f, 0.f, 0.f}, s1 = s0;
     if (FOLD) {
-      // the second half's sums of (token, rows 4 qq ..) lie 8 tokens and 8 rows on: 8 + 2 * 16 lanes
+      // the odd blocks' sums of (token, rows 4 qq ..) lie 8 tokens and 8 rows on: 8 + 2 * 16 lanes
       if (token < 8 && qq < 2) {
-        add_up(s0, red + l, 64);
-        add_up(s0, red + l + 40, 64);
+        add_up(s0, red + l, NT * 64);
+        add_up(s0, red + l + 40, NT * 64);
+        if (PAIRED) {
+          add_up(s1, red + 64 + l, NT * 64);
+          add_up(s1, red + 64 + l + 40, NT * 64);
+        }
       }
     } else if (WK > 1) {
       add_up(s0, red + (t * MB + mb) * 64 + l, NT * MB * 64);
@@ -466,7 +513,10 @@ __global__ __launch_bounds__(sk_max_waves(NT) * 64) void gemm_skinny_kernel(Gemm
           const float res = __bfloat162float(u == tid ? res_pre[j] : a.residual[(size_t)min(token, a.M - 1) * a.ldr + min(n + j, a.N - 1)]);
           x[j] = live && n + j < a.N ? round_to<bf16_t>(s0[j] * scale + bias_at(a, n + j, a.N)) + res : 0.f;
         }
-        if (a.emit_w != nullptr) emit_for_norm(a, x, live && n < a.N, token, n, tile, l);
+        if (a.emit_w != nullptr) {
+          if (u != tid) emit_ask(a, n, emit_pre);
+          emit_for_norm(a, x, emit_pre, live && n < a.N, token, n, tile, l);
+        }
         if (live) store_rounded(a, x, token, n);
       } else if (live) {
         store4<EPI>(a, s0, s1, scale, token, n);
@@ -561,9 +611,14 @@ __global__ __launch_bounds__(1024) void gemm_staged_kernel(GemmArgs a) {
     for (int mb = 0; mb < MB; ++mb) acc[t][mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   bf16x8_t w_cur[ST_SC][NT], piece[MB];
+  f32x4_t parts = {0.f, 0.f, 0.f, 0.f};
+  if (NORM) parts = *row_parts(a, wave, lane);
   load_w(0, w_cur);
   load_a(0, piece);
-  if (NORM) row_scales<MB>(a, scales, row_parts(a, wave, lane), wave, lane, nwaves);
+  if (NORM) {
+    early_row_scale(a, scales, parts, wave, lane);
+    row_scales<MB>(a, scales, wave, lane, nwaves);
+  }
   store_a(0, piece);
   __syncthreads();
   int buf = 0;
@@ -687,9 +742,22 @@ __global__ __launch_bounds__(256, 2) void gemm_glu_stream_kernel(GemmArgs a) {
       load_to_lds(src[i] + k, base + (unsigned)(row * GL_K * sizeof(bf16_t)));
     }
   };
-  f32x4_t parts = {0.f, 0.f, 0.f, 0.f};
-  if (NORM) parts = row_parts(a, wave, lane);  // (asked for first, used behind the last step: nothing waits for them in between)
+  // With a norm in front: the partial sums of a wavefront's first rows come into the place of the step that is asked for last,
+  // and are added up while the weights are on their way (added behind the last step 0.5 us at one row, 0.8 at 8).
+  constexpr int EARLY = MB == 2 ? 2 : 4;
+  static_assert(4 * EARLY * 1024 <= ROWS * GL_K * (int)sizeof(bf16_t), "the partial sums fit a step's place");
+  const unsigned parts = (unsigned)((S - 1) * ROWS * GL_K * sizeof(bf16_t)) + wave * (EARLY * 1024);
+  if (NORM && a.early_lanes > 0) {
+#pragma unroll
+    for (int i = 0; i < EARLY; ++i) load_to_lds((const bf16_t*)row_parts(a, wave + 4 * i, lane), lds + parts + i * 1024);
+  }
   for (int s = 0; s < S - 1 && s < steps; ++s) ask(s);
+  if (NORM && a.early_lanes > 0) {
+    if (steps >= S - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < EARLY; ++i) early_row_scale(a, scales, *(const f32x4_t*)(smem + parts + i * 1024 + lane * 16), wave + 4 * i, lane);
+  }
   f32x4_t acc[NB];
 #pragma unroll
   for (int mb = 0; mb < NB; ++mb) acc[mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -711,8 +779,8 @@ __global__ __launch_bounds__(256, 2) void gemm_glu_stream_kernel(GemmArgs a) {
       }
     }
   }
-  if (NORM) {
-    row_scales<MB>(a, scales, parts, wave, lane, 4);
+  if (NORM && (a.early_lanes == 0 || a.M > 4 * EARLY)) {
+    row_scales<MB>(a, scales, wave, lane, 4, EARLY);
     __syncthreads();
   }
   // lanes of q < 2 hold gate rows 4 q + j, those of q + 2 the same rows of up
@@ -742,6 +810,7 @@ static bool launch_skinny_one(const GemmArgs& given, int groups, int WK, hipStre
   a.waves = WK;
   a.share = steps / WK;
   a.spare = steps % WK;
+  a.each_die = a.emit_w != nullptr && groups % 8 == 0 ? groups / 8 : 0;
   const dim3 grid = EPI == EPI_ROPE ? dim3(groups / (a.nq + 2 * a.nkv), a.nq + 2 * a.nkv) : dim3(groups);  // (a head's pairs of tiles, the heads)
   size_t lds = (WK > 1 || FOLD) ? (size_t)WK * NT * MB * 64 * sizeof(f32x4_t) : 0;
   if (NORM) lds += (size_t)16 * MB * sizeof(float);
@@ -752,7 +821,7 @@ static bool launch_skinny_one(const GemmArgs& given, int groups, int WK, hipStre
 }
 
 // the skinny kernel with K folded into the unused half of the matrix core (one tile of 8 weight
-// rows a workgroup, up to 8 rows of A)
+// rows a workgroup, or a pair that rotates, up to 8 rows of A)
 static bool launch_folded(const GemmArgs& a, int epi, bool norm, int groups, int WK, hipStream_t stream) {
   switch (epi) {
     case EPI_RESIDUAL: return norm ? false : launch_skinny_one<1, 1, EPI_RESIDUAL, false, true>(a, groups, WK, stream);
@@ -762,6 +831,9 @@ static bool launch_folded(const GemmArgs& a, int epi, bool norm, int groups, int
     case EPI_F32:
       return norm ? launch_skinny_one<1, 1, EPI_F32, true, true>(a, groups, WK, stream)
                   : launch_skinny_one<1, 1, EPI_F32, false, true>(a, groups, WK, stream);
+    case EPI_ROPE:
+      return norm ? launch_skinny_one<1, 2, EPI_ROPE, true, true>(a, groups, WK, stream)
+                  : launch_skinny_one<1, 2, EPI_ROPE, false, true>(a, groups, WK, stream);
     default: return false;
   }
 }
@@ -860,7 +932,10 @@ static int compute_units() {
 // Weight rows of a tile that the skinny kernel uses for up to 32 rows of A: 16 fill the matrix
 // core, fewer make more workgroups.  A workgroup streams its rows over all of K, so the time is
 // that of the rounds of workgroups the compute units take, times the rows of each: the fewest
-// win, and among equals the larger tile (A is read once a workgroup).  With two rounds or more
+// win, and among equals the larger tile (A is read once a workgroup); for one and two rows of A
+// tiles of 8, which are folded and load whole lines (16 / 8 at one row: 4,096 x 4,096 10.5 / 9.8 us,
+// 4,096 x 14,336 25.9 / 24.7, 6,144 x 4,096 with the rotation 14.9 / 14.2; at 4 rows 10.8 / 10.8, 27.9 /
+// 28.1, 15.6 / 15.1; at 8 11.3 / 13.1, 31.5 / 34.0, 16.2 / 16.3).  With two rounds or more
 // of full tiles the rounds overlap and even out: 16 rows then (measured: smaller tiles lose).
 // With the rotation epilogue (heads > 0) a workgroup takes `th` columns of one half of a head.
 static int choose_tile_rows(int M, int N, int heads = 0, int half = 0) {
@@ -871,7 +946,7 @@ static int choose_tile_rows(int M, int N, int heads = 0, int half = 0) {
     const int groups = heads > 0 ? heads * ((half + th - 1) / th) : (N + th - 1) / th;
     if (th == 16 && groups >= 2 * units) return 16;
     const int cost = ((groups + units - 1) / units) * th;
-    if (th == 16 || cost < best_cost) { best = th; best_cost = cost; }
+    if (th == 16 || cost < best_cost || (cost == best_cost && th == 8 && M <= 2)) { best = th; best_cost = cost; }
   }
   return best;
 }
@@ -921,10 +996,14 @@ TK_API int tk_gemm_skinny_bf16(const void* A, int lda, const void* W, void* C, i
     a.glu_limit = extra->glu_limit; a.glu_alpha = extra->glu_alpha; a.glu_gelu = extra->glu_gelu;
     if (extra->out_scale != 0.f) a.out_scale = extra->out_scale;
     norm = a.sumsq_in != nullptr;
+    const bool early = norm && a.parts_in > 0 && a.parts_in <= 256 && a.parts_in % 4 == 0 && ((uintptr_t)a.sumsq_in & 15) == 0;
+    a.early = early ? a.sumsq_in : (const float*)A;  // (else 16 bytes that are there in any case)
+    a.early_apart = early ? a.parts_in : 0;
+    a.early_lanes = early ? a.parts_in / 4 : 0;
   }
   TK_REQUIRE(!norm || a.parts_in > 0, "gemm_skinny: a norm in front needs its partial sums");
   TK_REQUIRE(!(norm && epi == EPI_RESIDUAL), "gemm_skinny: a norm in front cannot be combined with a residual behind");
-  TK_REQUIRE(a.emit_w == nullptr || (epi == EPI_RESIDUAL && a.emit_scaled && a.emit_sumsq && a.ld_emit >= N),
+  TK_REQUIRE(a.emit_w == nullptr || (epi == EPI_RESIDUAL && a.emit_scaled && a.emit_sumsq && a.ld_emit >= N && ((uintptr_t)a.emit_scaled & 7) == 0),
              "gemm_skinny: outputs for a following norm go with the residual epilogue and need their buffers");
   if (epi == EPI_ROPE) {
     TK_REQUIRE(extra && a.positions && a.token_req && a.block_table && a.kcache && a.vcache,
@@ -983,18 +1062,19 @@ TK_API int tk_gemm_skinny_bf16(const void* A, int lda, const void* W, void* C, i
     }
     TK_REQUIRE(a.emit_w == nullptr || a.parts_out == th_units, "gemm_skinny: %d partial sums a row, the caller sized for %d", th_units, a.parts_out);
     // tiles of 8 weight rows for up to 8 rows of A: both halves of K in one product
-    const bool folded = fold != 0 && a.TH == 8 && M <= 8 && NT == 1 && !paired && K % 64 == 0 && !(norm && epi == EPI_RESIDUAL);
-    const int steps = folded ? K32 / 2 : K32;  // steps of 32 that a lane walks
+    const bool folded = fold != 0 && a.TH == 8 && M <= 8 && (NT == 1 || epi == EPI_ROPE) && epi != EPI_SWIGLU && K % 64 == 0 && !(norm && epi == EPI_RESIDUAL);
+    const int steps = folded ? K / 64 : K32;
     int WK = waves_k;
     if (WK <= 0) {
       // a wavefront issues the loads of U steps together: best when that is all it has to do,
       // so that the whole matrix is asked for at once and the hardware queues the workgroups
       const int U = (NT + MB <= 3) ? 8 : ((NT + MB <= 6) ? 4 : 2);
-      WK = steps / (U * NT);
+      WK = folded ? steps / U : steps / (U * NT);
     }
     const int lds_cap = 65536 / (NT * MB * 64 * (int)sizeof(f32x4_t));
     if (WK > lds_cap) WK = lds_cap;
-    if (WK > sk_max_waves(NT)) WK = sk_max_waves(NT);
+    // (folded, two groups of U in 8 wavefronts are ahead of one in 16: 2,048 x 8,192 10.3 / 9.8 us at one row, 13.6 / 12.9 at 8)
+    if (WK > sk_max_waves(folded ? 2 : NT)) WK = sk_max_waves(folded ? 2 : NT);
     if (WK > steps) WK = steps;
     if (WK < 1) WK = 1;
     if (folded) {
