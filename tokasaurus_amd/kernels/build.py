@@ -29,7 +29,7 @@ IN_TREE_DIR = Path(__file__).resolve().parent / "_build"
 GROUPS = {
     "core": ["errors.hip", "elementwise.hip", "attention_generic.hip", "gemm_generic.hip", "gemm_f32.hip", "sample.hip", "step_io.hip",
              "stream_f32.hip", "attention_prepare.hip", "attention_tile_f32.hip", "attention_tile_bf16.hip", "delta_rule.hip", "delta_rule_chunks.hip", "routed_experts.hip", "gated_recurrence.hip", "linear_attention.hip", "linear_attention_chunks.hip", "state_space.hip"],
-    "mfma": ["errors.hip", "attention_mfma.hip", "gemm_mfma.hip", "gemm_split.hip", "gemm_tiles.hip", "grouped_gemm.hip"],
+    "mfma": ["errors.hip", "attention_mfma.hip", "gemm_mfma.hip", "gemm_split.hip", "gemm_tiles.hip", "grouped_gemm.hip", "block_calls.hip"],
     "library": ["errors.hip", "gemm_library.hip"],
 }
 # what a group's library is linked with beside the HIP runtime

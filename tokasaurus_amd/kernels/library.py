@@ -107,6 +107,7 @@ _SIGNATURES: dict[str, dict[str, list]] = {
         "tk_split_linear_add_rmsnorm": [_P, c_int, _P, _P] + [c_int] * 4 + [_P, _P, c_int, _P, _P, c_float, c_int, _P],
         "tk_split_linear_rope_append": [_P, c_int, _P, _P] + [c_int] * 3 + [_P, _P, _P, _P, c_int, _P, _P, _P, _P] + [c_int] * 4 + [_P],
         "tk_gemm_tiles_bf16": [_P, c_int, _P, _P] + [c_int] * 6 + [_P],
+        "tk_block_calls": [_P, _P],
         "tk_grouped_gemm_bf16": [_P, c_int, _P, _P, _P, c_int, c_int, c_int, c_int, _P, c_size_t, _P, c_int, c_int, c_int, c_int, _P, c_int, c_long,
                                  c_int, c_int, _P, _P, c_float, c_float, _P],
         "tk_expert_sort": [_P, c_int, _P],

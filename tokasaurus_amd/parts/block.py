@@ -31,7 +31,11 @@ from tokasaurus_amd.parts.base import (
     TensorSpec,
 )
 from tokasaurus_amd.parts.base import AVERAGE_WEIGHT, MATRIX
+from tokasaurus_amd.kernels.block_calls import LAUNCHES, MOST_ROWS, BlockPlan
+from tokasaurus_amd.parts.attention import PagedAttention, attention_plan
+from tokasaurus_amd.parts.feedforward import SwiGLU
 from tokasaurus_amd.parts.linear import Linear, Placer
+from tokasaurus_amd.parts.norm import RMSNorm
 from tokasaurus_amd.parts.short_conv import ShortConvResidual
 
 
@@ -96,6 +100,10 @@ class PreNormBlock(Block):
         prepared: Prepared | None = None,
         next_norm=None,
     ):
+        if rows is None and x.dtype == torch.bfloat16 and x.shape[0] <= MOST_ROWS:
+            done = self._in_one_call(x, ctx, cache, prepared, next_norm)
+            if done is not None:
+                return done
         residual = x if rows is None else ops.gather_rows(x, rows)
         if self.mixer.fuses_norm:
             out = self.mixer.forward(Normed(x, self.mixer_norm, prepared), residual, ctx, cache, state, rows,
@@ -106,6 +114,50 @@ class PreNormBlock(Block):
         if self.feed_forward.fuses_norm:
             return self.feed_forward.forward(Normed(x, self.ff_norm, prepared), x, emit_norm=next_norm)
         return self.feed_forward.forward(Normed(x, self.ff_norm, prepared).materialize(), x)
+
+
+    def _in_one_call(self, x: torch.Tensor, ctx: StepContext, cache: CacheView | None, prepared: Prepared | None, next_norm):
+        """The whole block for a few hundred rows of bfloat16 by one call of the host (``kernels.block_calls``), with the kernels that
+        the parts would launch one by one; None where the block, the step or a tensor is not of that kind."""
+        mixer, ff = self.mixer, self.feed_forward
+        if (type(mixer) is not PagedAttention or type(ff) is not SwiGLU or ff.glu is not None or mixer.head_norm or mixer.rotary_dim is not None
+                or cache is None or not cache.writable or ctx.extras.get("static")
+                or not (type(self.mixer_norm) is type(self.ff_norm) is type(next_norm) is RMSNorm)
+                or any(lin.bias is not None for lin in (mixer.qkv, mixer.out, ff.gate_up, ff.down))
+                or (prepared is not None and prepared.data is not None)):
+            return None
+        m, hidden = x.shape
+        key = ("block_calls", m, hidden, ff.intermediate_size, mixer.num_heads, mixer.num_kv_heads, mixer.head_dim, mixer.window, mixer.scale, cache.page_size)
+        plan = ctx.extras.get(key)
+        if plan is None:
+            plan = ctx.extras[key] = self._plan_one_call(x, ctx, cache) or False  # (made once a step, shared by its layers)
+        # (layers of one size may still differ in their position encoding)
+        if plan is False or plan.position is not mixer.position:
+            return None
+        done = plan.run(x, Normed(x, self.mixer_norm, prepared).materialize(),
+                        {"w_qkv": mixer.qkv.weight, "w_out": mixer.out.weight, "w_gate_up": ff.gate_up.weight, "w_down": ff.down.weight},
+                        self.ff_norm.weight, self.ff_norm.eps, next_norm.weight, next_norm.eps, cache.keys, cache.values, cache.block_table)
+        return None if done is None else (done[0], Prepared(None, next_norm, done[1]))
+
+    def _plan_one_call(self, x: torch.Tensor, ctx: StepContext, cache: CacheView) -> BlockPlan | None:
+        mixer, ff, m = self.mixer, self.feed_forward, x.shape[0]
+        nq, nkv, d, page = mixer.num_heads, mixer.num_kv_heads, mixer.head_dim, cache.page_size
+        cos, sin = (mixer.position.cos, mixer.position.sin) if mixer.position is not None else (None, None)
+        routes = {"qkv": mixer.qkv.many_rows_route(m, mixer.qkv.split_rope_from), "out": mixer.out.many_rows_route(m, mixer.out.split_norm_from),
+                  "gate": ff.gate_up.gate_up_route(m), "down": ff.down.many_rows_route(m, ff.down.split_norm_from)}
+        tables = (ctx.positions, ctx.token_req, ctx.q_start, ctx.kv_len)
+        fits = (None not in routes.values() and ops.attention_mfma_supports(x.dtype, d, page) and d % 8 == 0
+                and (routes["qkv"][0] > 0 or m > min(ops.SKINNY_ROPE_ROWS, 2 * ops.skinny_rows(mixer.hidden_size, paired=True)))
+                and all(t.is_cuda and t.dtype == torch.int32 and t.is_contiguous() for t in tables)
+                and ctx.positions.numel() == ctx.token_req.numel() == m and ctx.kv_len.numel() == ctx.num_requests == ctx.q_start.numel() - 1
+                and (cos is None or (cos.is_cuda and cos.dtype == sin.dtype == torch.float32 and cos.shape == sin.shape and cos.shape[1] == d // 2
+                                     and cos.is_contiguous() and sin.is_contiguous())))
+        launches = attention_plan(ctx, nq // nkv, nkv, d, page).launches if fits else []
+        if not fits or len(launches) > LAUNCHES:
+            return None
+        plan = BlockPlan(ctx, m, x.shape[1], ff.intermediate_size, nq, nkv, d, page, mixer.window, mixer.scale, cos, sin, routes, launches)
+        plan.position = mixer.position
+        return plan
 
 
 class NormPair(Part):

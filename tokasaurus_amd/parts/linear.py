@@ -103,6 +103,27 @@ class Linear:
         return (m <= ops.skinny_rows(self.in_features, paired)
                 or (paired and m <= ops.GLU_STREAM_ROWS and m <= ops.glu_rows(self.in_features, self.total_out // 2)))
 
+    def many_rows_route(self, m: int, split_from: int) -> "tuple[int, int, bool] | None":
+        """How ``m`` rows go through this product with a pass behind it: (cuts of K, or 0 for a whole product; its tile, or -1 for the
+        library's; whether the rows that the pass norms are rounded once); None where a kernel for few rows takes them, or another
+        path.  ``split_from``: the rows from which that pass has the product split."""
+        if self.weight.dtype != torch.bfloat16 or self.bias is not None or self.in_features % 8 or self.total_out % 8:
+            return None
+        if split_from <= m <= ops.SPLIT_ROWS:
+            return ops.split_cuts(self.total_out, self.in_features, m), -1, m <= self.split_once_to
+        if self._fast(m):
+            return None
+        return 0, ops.tiles_choice(m, self.total_out, self.in_features) if m >= ops.PLAIN_TILES_FROM_ROWS else -1, False
+
+    def gate_up_route(self, m: int) -> "int | None":
+        """The same for gate and up with silu behind: a tile, -1 for the library's product, -2 for the streamed form."""
+        inner = self.total_out // 2
+        if self.weight.dtype != torch.bfloat16 or self.bias is not None or self.in_features % 8 or inner % 8:
+            return None
+        if self._fast(m, paired=True):
+            return -2 if ops.glu_streams(m, inner, self.in_features) else None
+        return ops.tiles_choice(m, inner, self.in_features, True) if m >= ops.GLU_TILES_FROM_ROWS else -1
+
     def __call__(
         self,
         x: torch.Tensor | Normed,
