@@ -75,3 +75,22 @@ def test_what_does_not_lie_as_the_kernels_read_it_goes_part_by_part(monkeypatch)
     assert made[0] is None and made[1] is not None
     for g, w in zip(got, want):
         assert float((g - w).norm() / w.norm()) < 0.02  # (other kernels for one projection: the order of 32-bit sums in front of 8-bit roundings)
+
+
+def test_a_steps_memory_goes_back_with_the_step():
+    """The plan and its memory end with the step, with the collector off."""
+    import gc
+
+    runner = ModelRunner.from_random(CONFIGS["1b"], 3, "bfloat16", 16, 100, 4, use_graphs=False)
+    runner.run([StepEntry("a", list(range(100)), [])])
+    gc.collect()
+    gc.disable()
+    try:
+        held = []
+        for i in range(6):
+            runner.release("a")
+            runner.run([StepEntry("a", list(range(100)), [])])
+            held.append(torch.cuda.memory_allocated())
+    finally:
+        gc.enable()
+    assert held[-1] == held[1]

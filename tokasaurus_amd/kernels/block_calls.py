@@ -64,7 +64,8 @@ class BlockPlan:
         b.library = _address("library", "tk_gemm_library_bf16")
         workspace = ops.library_workspace()
         b.workspace, b.workspace_bytes = workspace.data_ptr(), workspace.numel()
-        b.positions, b.token_req, b.q_start, b.kv_len = (t.data_ptr() for t in (ctx.positions, ctx.token_req, ctx.q_start, ctx.kv_len))
+        tables = (ctx.positions, ctx.token_req, ctx.q_start, ctx.kv_len)
+        b.positions, b.token_req, b.q_start, b.kv_len = (t.data_ptr() for t in tables)
         b.cos_t, b.sin_t = (cos.data_ptr(), sin.data_ptr()) if cos is not None else (None, None)
         for name in ("qkv", "out", "down"):
             cuts, route, once = routes[name]
@@ -74,7 +75,9 @@ class BlockPlan:
                 setattr(b, name + "_once", 1 if once else 0)
         b.gate_route = routes["gate"]
         b.launches = len(launches)
-        self.kept = [ctx, cos, sin, workspace]  # (whose addresses the struct holds)
+        # what the struct holds the addresses of (not the step itself, which holds this plan: a circle of references would keep the memory
+        # until the collector comes by)
+        self.kept = [*tables, cos, sin, workspace]
         for a, l in zip(b.attention, launches):
             n_tiles, splits = l.tile_req.numel(), max(1, -(-l.max_kv_len // l.split))
             a.tile_req, a.tile_row0 = l.tile_req.data_ptr(), l.tile_row0.data_ptr()
