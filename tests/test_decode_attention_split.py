@@ -1,0 +1,25 @@
+"""How decoded tokens' keys are cut: whole steps of 32 keys a wavefront, no split below 128 keys, and what a mixed step cuts evenly."""
+
+import pytest
+
+from tokasaurus_amd.kernels import ops
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("bound", [1, 100, 128, 129, 1024, 2048, 4096, 100000])
+@pytest.mark.parametrize("tiles", [1, 2, 5, 45, 512])
+def test_splits_are_worth_handing_over(head_dim, bound, tiles):
+    split, waves = ops.attention_split(bound, tiles, 8, head_dim)
+    assert split % (32 * waves) == 0 and waves <= (16 if head_dim == 64 else 4)
+    assert split >= min(bound, 128) and -(-bound // split) <= max(16, bound // 2048 + 1)
+    if tiles == 1 and 1024 <= bound <= 4096:
+        assert waves == 4 and -(-bound // split) in (8, 16)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("lengths", [[1], [2000] * 45, [250 + 39 * i for i in range(45)], [8192] + [40] * 63, [100, 131072]])
+def test_even_splits(head_dim, lengths):
+    split, waves = ops.attention_even_split(lengths, 8, head_dim)
+    whole = ops.attention_split(max(lengths), len(lengths), 8, head_dim)
+    assert split % (32 * waves) == 0 and 1 <= waves <= ops.attention_max_waves(head_dim, 1)
+    assert (split, waves) == whole or (512 <= split < whole[0] and waves == 4)

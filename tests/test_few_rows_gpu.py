@@ -62,3 +62,32 @@ def test_rotation_behind_a_folded_inner_size(m, k):
     largest = float(stacked.double().abs().max())
     for got, want in ((q, stacked[:, : nq * d]), (pages[1][0], pages[0][0]), (pages[1][1], pages[0][1])):
         assert float((got.double() - want.double()).abs().max()) <= 2.0 ** -7 * largest
+
+
+@pytest.mark.parametrize("d,split,waves", [(64, 128, 4), (64, 96, 3), (64, 2048, 16), (128, 256, 4), (128, 160, 5), (128, 4096, 8)])
+@pytest.mark.parametrize("window", [0, 70])
+def test_wavefronts_share_the_keys_that_a_split_has(d, split, waves, window):
+    """Requests that end anywhere in a split (or whose window begins there), against 64-bit attention: keys, values and weights have 8
+    significant bits, and the sums are 32-bit: 2^-7 of the weighted magnitudes."""
+    nq, nkv, page = 8, 2, 16
+    lens = [1, 31, 32, 33, 95, 127, 128, 129, 200, 400]
+    gen = torch.Generator(device="cuda").manual_seed(d + split)
+    rand = lambda *s: torch.randn(s, generator=gen, device="cuda").bfloat16()  # noqa: E731
+    pages = [-(-n // page) for n in lens]
+    kc, vc = rand(*ops.key_pages_shape(sum(pages), nkv, page, d)), rand(*ops.value_pages_shape(sum(pages), nkv, page, d))
+    table, at = torch.zeros((len(lens), 32), dtype=torch.int32), 0
+    for i, n in enumerate(pages):
+        table[i, :n] = torch.arange(at, at + n)
+        at += n
+    q = rand(len(lens), nq * d)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    got = ops.paged_attention_mfma(q, kc, vc, table.cuda(), i32(range(len(lens) + 1)), i32(lens), i32(range(len(lens))), i32([0] * len(lens)), 1,
+                                   nq, nkv, d, page, 512, split, waves=waves, window=window)
+    for i, n in enumerate(lens):
+        mine = table[i, : pages[i]].long().cuda()
+        k = kc[mine].double().permute(1, 0, 3, 2, 4).reshape(nkv, -1, d)[:, max(0, n - window) if window else 0 : n]
+        v = vc[mine].double().permute(1, 0, 2, 4, 3).reshape(nkv, -1, d)[:, max(0, n - window) if window else 0 : n]
+        k, v = k.repeat_interleave(nq // nkv, 0), v.repeat_interleave(nq // nkv, 0)
+        p = torch.softmax((k @ q[i].double().view(nq, d, 1))[..., 0] * d ** -0.5, -1)
+        want, size = (p[:, None] @ v)[:, 0], (p[:, None] @ v.abs())[:, 0]
+        assert ((got[i].double().view(nq, d) - want).abs() <= 2.0 ** -7 * size + 1e-6).all(), n

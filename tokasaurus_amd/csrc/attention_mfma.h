@@ -103,8 +103,9 @@ __device__ __forceinline__ TileRange tile_range(const AttnArgs& a, int tile, int
     t.rt_lo[rt] = t.full_lo[rt] = 0x7fffffff;
     t.rt_hi[rt] = t.full_hi[rt] = -1;
     if (t.row0[rt] < 0) continue;
-    const int first_tok = t.row0[rt] / a.group;
-    const int last_tok = min(t.row0[rt] + 15, t.n_rows - 1) / a.group;
+    // (a request of one token, decoded: no divisions in front of its first loads)
+    const int first_tok = t.qlen == 1 ? 0 : t.row0[rt] / a.group;
+    const int last_tok = t.qlen == 1 ? 0 : min(t.row0[rt] + 15, t.n_rows - 1) / a.group;
     const int pos_first = t.kvl - t.qlen + first_tok, pos_last = t.kvl - t.qlen + last_tok;
     t.rt_hi[rt] = pos_last;
     t.rt_lo[rt] = a.window > 0 ? max(0, pos_first - a.window + 1) : 0;
@@ -113,8 +114,8 @@ __device__ __forceinline__ TileRange tile_range(const AttnArgs& a, int tile, int
     t.lo = min(t.lo, t.rt_lo[rt]);
     t.hi = max(t.hi, t.rt_hi[rt]);
   }
-  t.s_first = t.lo / a.split;
-  t.s_last = t.hi / a.split;
+  t.s_first = a.max_splits == 1 || t.lo == 0 ? 0 : t.lo / a.split;
+  t.s_last = a.max_splits == 1 ? 0 : t.hi / a.split;
   return t;
 }
 
@@ -320,10 +321,13 @@ __device__ __forceinline__ void attention_item(const AttnArgs& a, const int tile
   const int s = GROUPED ? 0 : t.s_first + split_index;
   if (!GROUPED && s > t.s_last) return;
   const int nsp = GROUPED ? 1 : t.s_last - t.s_first + 1;
-  // this wavefront's part of the split: `sub` keys, a multiple of 32
-  const int sub = a.split / NW;
-  const int k_begin = max((t.lo >> 5) << 5, s * a.split + wave * sub);
-  const int k_end = min(t.hi + 1, s * a.split + (wave + 1) * sub);
+  // this wavefront's part of the keys that the split has: `sub` of them, a multiple of 32.  (Of a request that ends, or whose
+  // window begins, inside the split every wavefront still takes as many as the others: cut by the split's size instead, 64
+  // requests of 375 to 3,000 keys planned for 4,096 waited for wavefronts of 512 keys.)
+  const int k_first = max((t.lo >> 5) << 5, s * a.split), k_last = min(t.hi + 1, (s + 1) * a.split);
+  const int sub = NW == 1 ? a.split : (((k_last - k_first + NW - 1) / NW + 31) >> 5) << 5;
+  const int k_begin = k_first + wave * sub;
+  const int k_end = min(k_last, k_begin + sub);
   const int* table = a.block_table + (size_t)t.req * a.table_stride;
 
   // the steps (by their first key) in which a row tile has a row that sees a key, in which all
@@ -346,7 +350,7 @@ __device__ __forceinline__ void attention_item(const AttnArgs& a, const int tile
     const int flat = t.row0[rt] >= 0 ? t.row0[rt] + r : t.n_rows;
     const bool valid = flat < t.n_rows;
     const int fl = valid ? flat : t.n_rows - 1;
-    const int tok = fl / a.group, g = fl - tok * a.group;
+    const int tok = t.qlen == 1 ? 0 : fl / a.group, g = fl - tok * a.group;
     const int pos = t.kvl - t.qlen + tok;
     pos_r[rt] = valid ? pos : -1;
     const bf16_t* qp = a.q + (size_t)(t.qs + tok) * a.q_stride + (size_t)(kvh * a.group + g) * D;
@@ -605,20 +609,36 @@ __device__ __forceinline__ void attention_item(const AttnArgs& a, const int tile
     __syncthreads();
     if (wave != 0 && !hand_over) return;
     if (wave == 0) {
+      // (rows of several wavefronts are on their way together; behind the last one it is asked for again and not used)
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
+      const float* mine = wg_part + (size_t)(rt * 16 + r) * ROW;
+      constexpr int NEXT = 16 * RT * ROW;  // to the next wavefront's row
       float m = -INFINITY;
-      for (int w = 0; w < NW; ++w) m = fmaxf(m, wg_part[((size_t)w * 16 * RT + rt * 16 + r) * ROW]);
+      for (int w = 0; w < NW; w += 4)
+        m = fmaxf(m, fmaxf(fmaxf(mine[w * NEXT], mine[min(w + 1, NW - 1) * NEXT]), fmaxf(mine[min(w + 2, NW - 1) * NEXT], mine[min(w + 3, NW - 1) * NEXT])));
       float l = 0.f;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) acc[rt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      for (int w = 0; w < NW; ++w) {
-        const float* row = wg_part + ((size_t)w * 16 * RT + rt * 16 + r) * ROW;
-        const float mw = row[0];
+      auto add = [&](const float mw, const float lw, const f32x4_t (&v)[DT]) {
         const float f = (mw == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(mw - m);
-        l += f * row[1];
+        l += f * lw;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) acc[rt][dt] += f * *(const f32x4_t*)(row + 4 + dt * 16 + q * 4);
+        for (int dt = 0; dt < DT; ++dt) acc[rt][dt] += f * v[dt];
+      };
+      for (int w = 0; w < NW; w += 2) {
+        float mw[2], lw[2];
+        f32x4_t v[2][DT];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const float* row = mine + min(w + i, NW - 1) * NEXT;
+          mw[i] = row[0];
+          lw[i] = row[1];
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt) v[i][dt] = *(const f32x4_t*)(row + 4 + dt * 16 + q * 4);
+        }
+        add(mw[0], lw[0], v[0]);
+        if (w + 1 < NW) add(mw[1], lw[1], v[1]);
       }
       m_run[rt] = m;
       l_run[rt] = l;

@@ -607,21 +607,36 @@ def attention_split(max_kv_len: int, n_tiles: int, nkv: int, head_dim: int = 64)
     or more.
     Measured best on an MI355X at 8192 keys, with the cache read from memory:
     64 keys x 8 wavefronts x 16 splits at batch 1, 256 x 8 x 4 at batch 8,
-    512 x 16 x 1 at batch 64."""
+    512 x 16 x 1 at batch 64.  Handing a split over costs 3 us and more, so a split has 128 keys or more, four wavefronts of 32
+    of them, and beyond eight splits 256 (us a layer of 8 kv heads at one request, planned for 1,024: splits of 64 keys for one
+    wavefront / of 128 for four, head size 64 9.4 / 6.3 at 500 keys, 10.5 / 6.8 at 1,000, head size 128 16.4 / 9.0; planned for 2,048: 128
+    for two / 256 for four 8.1 / 7.2 at 1,100, 9.3 / 7.7 at 2,000; two requests of 1,000 keys 12.8 / 8.1).  At head sizes above 64 a
+    compute unit has room for eight wavefronts: two workgroups of four hide each other's ends (eight / four wavefronts,
+    16 requests of 1,500 keys 26.2 / 25.3, 64 of 47 to 380 19.7 / 17.0)."""
     base = max(n_tiles * nkv, 1)
     kv = max(max_kv_len, 1)
-    splits = max(1, min(16, -(-256 // base)))
+    splits = max(1, min(16, -(-256 // base), -(-kv // 128), max(8, kv // 256)))
     # at most 8 192 keys a split (2 048 with a thousand tiles and more), however many tiles there are: the bound
     # is that of the longest request, and one long request among short ones must still spread over the chip
     # (63 requests of 2 048 keys beside one of 131 072: 881 us a layer with one split a tile, 168 us with splits of
     # 8 192 keys; 255 of 512 beside one of 32 768: 401 / 114 us; requests of one length lose nothing)
     raw = min(-(-kv // splits), 8192 if base < 1024 else 2048)
-    per_wave = min(512, max(64, kv * base // 2048))
+    per_wave = min(512, max(32 if raw <= 128 else 64, kv * base // 2048))
     waves = 1
-    while waves * 2 <= min(attention_max_waves(head_dim, 1), raw // per_wave):
+    while waves * 2 <= min(attention_max_waves(head_dim, 1), raw // per_wave, 16 if head_dim <= 64 else 4):
         waves *= 2
     step = 32 * waves
     return -(-raw // step) * step, waves
+
+
+def attention_even_split(lengths: list[int], nkv: int, head_dim: int) -> tuple[int, int]:
+    """The same for decoded tokens beside prompts, in a step that is not recorded: their lengths are known, and where they differ the keys
+    are cut so that the workgroups (two a compute unit) get as many each.  3B shape, 45 requests of 250 to 2,000 keys, us a layer:
+    a split of 2,048 keys 52.7, of 1,024 49.4, of 512 48.0, of 256 51.8; 1B shape 29.1, 30.1, 26.8, -."""
+    split, waves = attention_split(max(lengths), len(lengths), nkv, head_dim)
+    even = -(-sum(lengths) * nkv // 512)
+    even = max(512, -(-even // 128) * 128)
+    return (even, 4) if even < split else (split, waves)
 
 
 # Whether the splits of decoded tokens' tiles are added inside the attention kernel, by the

@@ -78,8 +78,13 @@ def attention_plan(ctx: StepContext, group: int, nkv: int, head_dim: int, page_s
         lists: list[tuple[list[int], list[int], list[int] | None, int, int, int, int, int]] = []
         if small:
             req, row0, _ = ops.attention_tiles(q_lens, group, 1, small)
-            split, waves = ops.attention_split(bound, len(req), nkv, head_dim)
-            lists.append((req, row0, None, 1, split, waves, 0, bound))
+            if large and not static:
+                lengths = [ctx.host_kv_len[r] for r in small]
+                split, waves = ops.attention_even_split(lengths, nkv, head_dim)
+                lists.append((req, row0, None, 1, split, waves, 0, max(lengths)))
+            else:
+                split, waves = ops.attention_split(bound, len(req), nkv, head_dim)
+                lists.append((req, row0, None, 1, split, waves, 0, bound))
         # Portions that come after a past several times their own length walk far more keys a row than
         # whole prompts do: they are planned apart, or one of them among whole prompts would take a
         # form chosen for the many short walks and walk its long past on a few wavefronts.
