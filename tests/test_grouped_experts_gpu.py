@@ -120,3 +120,32 @@ def test_room_for_the_experts_is_that_of_the_pairs():
     before = torch.cuda.memory_allocated()
     out = ops.expert_mix(h, gu, dn, ids, weights, pairs=pairs)
     assert torch.isfinite(out).all() and torch.cuda.max_memory_allocated() - before < 4 << 20
+
+
+@pytest.mark.parametrize("tokens,experts,top,width,ff", [(257, 3, 2, 64, 4224), (700, 90, 3, 1600, 64), (385, 1, 1, 320, 192), (320, 1, 1, 192, 320),
+                                                         (321, 1, 1, 64, 64), (65, 1, 1, 64, 128), (900, 40, 3, 320, 192)])
+@pytest.mark.parametrize("form", ["silu", "on input"])
+def test_odd_tiles_apart_and_beside_their_pairs(monkeypatch, tokens, experts, top, width, ff, form):
+    """An inner size beyond which odd tiles stay beside their pairs, experts enough that they do, and odd tiles of 1, 64 and 65 rows and of
+    more apart."""
+    test_experts_in_pairs_of_tiles(monkeypatch, tokens, experts, top, width, ff, form)
+
+
+@pytest.mark.parametrize("tokens,top,experts", [(130, 1, 2), (400, 3, 5), (64, 2, 64), (1000, 4, 3)])
+def test_whole_pairs_and_odd_tiles_are_listed_apart(tokens, top, experts):
+    """Every tile that is used once, in a whole pair or as an odd one with the rows that it holds."""
+    ids = torch.randint(0, experts, (tokens, top), dtype=torch.int32, generator=torch.Generator().manual_seed(tokens))
+    s = ops.expert_sort([(ids.cuda(), experts)])[0]
+    runs, group = s.runs.cpu().view(-1, 4).tolist(), s.tile_group.cpu().tolist()
+    pairs, whole, odd, _ = runs[0]
+    order = runs[1 + s.max_pairs : 1 + 2 * s.max_pairs]
+    assert pairs == whole + odd
+    tiles = []
+    for i, (tile, e, first, count) in enumerate(order[:whole]):
+        assert first <= i < first + count
+        tiles += [(tile + 2 * (i - first) + j, e) for j in range(2)]
+    counts = torch.bincount(ids.flatten().long(), minlength=experts).tolist()
+    for tile, e, rows, _ in order[len(order) - odd :]:
+        assert rows == (counts[e] - 1) % ops.EXPERT_TILE + 1
+        tiles.append((tile, e))
+    assert sorted(tiles) == list(enumerate(group[: group[-1]]))

@@ -332,7 +332,7 @@ __global__ __launch_bounds__(256, 3) void grouped_gemm_staged_kernel(GroupedArgs
 }
 
 // Experts of many rows: two neighbouring tiles of a group as one of 256 slots x 256 weight rows (in the gated form 128 of gate and
-// 128 of up; gemm_tile.h), the odd last tile of a group as one of 128 x 256 in the same launch.  The path from the L2 to a compute
+// 128 of up; gemm_tile.h), the odd last tile of a group in smaller ones in the same launch.  The path from the L2 to a compute
 // unit bounds these products, and a tile of 256 x 256 asks for half as many bytes a product.
 // us by tiles of 128 x 128 / in pairs, gate and up and down, every expert 3, 4, 5 and 6 tiles: 32 experts of 2,048 x 1,024 147 / 136 and
 // 86 / 69, 185 / 141 and 109 / 75, 224 / 190 and 132 / 97, 265 / 202 and 155 / 107; 32 of 2,880 x 2,880 547 / 461 and 300 / 213 to
@@ -390,29 +390,61 @@ __device__ __forceinline__ void wide_tile(const GroupedArgs& a, char* smem, int 
 }
 
 #define WIDE_OUT(glu) ((glu) ? 128 : 256)
+#define ODD_OUT(glu) ((glu) ? 64 : 128)
 #define WIDE_PAIRS (GS_TILES / 2)
 using PairShape = TileShape<4, 4, 2, 3>;
-using HalfShape = TileShape<2, 4, 3, 3>;
-// A pair, as a workgroup reads it: the group's first tile, the group, the number of the group's first pair and how many tiles it has.
+using HalfShape = TileShape<2, 4, 3, 3>;   // an odd tile beside its group's pairs
+using OddShape = TileShape<2, 2, 5, 5>;    // an odd tile apart: half as many outputs a workgroup, so that the last round is short
+using ShortShape = TileShape<1, 2, 6, 6>;  // of up to 64 rows
+// A pair of neighbouring tiles of a group or an odd last tile alone: the group's first tile, the group, the number of the group's
+// first pair and how many tiles it has.
 struct TileRun {
   int tile, group, first, tiles;
 };
-// runs: the number of pairs (as the first's tile), then the pairs
-template <bool GLU>
-__global__ __launch_bounds__(256, 1) void grouped_gemm_pairs_kernel(GroupedArgs a, const TileRun* __restrict__ runs, int n_blocks) {
+// runs: the number of pairs, the odd ones with them (as the first's tile), of whole pairs (as its group) and of odd tiles (as its first);
+// then room for max_pairs pairs in the order of the tiles, then the order in which they are multiplied: whole pairs from the front (tile,
+// group, the group's first whole pair, how many it has), odd tiles from the back (tile, group, rows that it holds).
+//
+// A compute unit holds one workgroup, and a round of pairs takes all of them for one pair each.  APART: the whole pairs come first and the
+// odd tiles, cut so that one takes a third of a pair's time and less, behind them.  An expert's last tile often holds few rows: 2,048
+// tokens, 8 of 32 experts, are 512 rows an expert give or take 20, so that half of the experts have a fifth tile of some 16.  Not
+// APART they are tiles of 128 x 256 among their group's pairs, which read the same weights.
+template <bool GLU, bool APART>
+__global__ __launch_bounds__(256, 1) void grouped_gemm_pairs_kernel(GroupedArgs a, const TileRun* __restrict__ runs, int max_pairs, int n_blocks, int odd_blocks) {
   extern __shared__ __align__(16) char smem[];
-  const int items = runs->tile * n_blocks, per = (items + GS_DIES - 1) / GS_DIES;
-  const int seq = blockIdx.x / GS_DIES, item = blockIdx.x % GS_DIES * per + seq;
-  if (seq >= per || item >= items) return;
-  const int some = item / n_blocks;
-  const TileRun r = runs[1 + some];
-  // the chunk of up to WIDE_PAIRS pairs of the group that the item lies in
-  const int chunk = r.first + (some - r.first) / WIDE_PAIRS * WIDE_PAIRS, len = min(WIDE_PAIRS, r.first + (r.tiles + 1) / 2 - chunk);
-  const int off = item - chunk * n_blocks, pair = chunk + off % len;
-  const int tile = r.tile + 2 * (pair - r.first), n0 = off / len * WIDE_OUT(GLU);
-  if (tile + 1 < r.tile + r.tiles) wide_tile<PairShape, GLU>(a, smem, r.group, tile * GS_M, n0);
-  else wide_tile<HalfShape, GLU>(a, smem, r.group, tile * GS_M, n0);
+  const TileRun head = runs[0];
+  const TileRun* __restrict__ order = runs + 1 + (APART ? max_pairs : 0);
+  const int items = (APART ? head.group : head.tile) * n_blocks, per = (items + GS_DIES - 1) / GS_DIES;
+  const int seq = blockIdx.x / GS_DIES, die = blockIdx.x % GS_DIES;
+  if (seq < per) {
+    const int item = die * per + seq;
+    if (item >= items) return;
+    const int some = item / n_blocks;
+    const TileRun r = order[some];
+    // the chunk of up to WIDE_PAIRS pairs of the group that the item lies in
+    const int pairs = APART ? r.tiles : (r.tiles + 1) / 2;
+    const int chunk = r.first + (some - r.first) / WIDE_PAIRS * WIDE_PAIRS, len = min(WIDE_PAIRS, r.first + pairs - chunk);
+    const int off = item - chunk * n_blocks, pair = chunk + off % len;
+    const int tile = r.tile + 2 * (pair - r.first), n0 = off / len * WIDE_OUT(GLU);
+    if (APART || tile + 1 < r.tile + r.tiles) wide_tile<PairShape, GLU>(a, smem, r.group, tile * GS_M, n0);
+    else if constexpr (!APART) wide_tile<HalfShape, GLU>(a, smem, r.group, tile * GS_M, n0);
+  } else if constexpr (APART) {
+    const int odd = head.first * odd_blocks, odd_per = (odd + GS_DIES - 1) / GS_DIES, item = die * odd_per + seq - per;
+    if (seq - per >= odd_per || item >= odd) return;
+    const int some = item / odd_blocks;
+    const TileRun r = order[max_pairs - 1 - some];
+    const int n0 = (item - some * odd_blocks) * ODD_OUT(GLU);
+    if (r.first <= ShortShape::BM) wide_tile<ShortShape, GLU>(a, smem, r.group, r.tile * GS_M, n0);
+    else wide_tile<OddShape, GLU>(a, smem, r.group, r.tile * GS_M, n0);
+  }
 }
+
+// Whether odd tiles go apart: where they are at most about one round of workgroups (`odd` of them at the most, half of that as a rule), and
+// reading their experts' weights once more costs little beside.  Both products and the sum, us, with their pairs / apart, experts'
+// rows even and uneven: 32 experts of 2,048 x 1,024 234 / 234 and 302 / 265 at 420 rows an expert, 301 / 270 and 311 / 280 at 500, 336 /
+// 334 and 408 / 369 at 700; 16 of 2,048 x 2,048 307 / 247 and 300 / 263 at 500; 8 of 4,096 x 1,792 183 / 184 and 219 / 197 at 460; but 128 of 2,048 x
+// 768 682 / 710 and 722 / 725 at 400, 8 of 4,096 x 14,336 1,109 / 1,251 and 1,123 / 1,302 at 380.
+static bool odd_apart(int odd, int n_blocks, int K) { return (long)odd * n_blocks < 512 && K <= 4096; }
 
 template <bool GLU>
 static bool launch_by_tile(const GroupedArgs& a, int tiles, const TileRun* runs, int max_pairs, hipStream_t stream) {
@@ -420,12 +452,16 @@ static bool launch_by_tile(const GroupedArgs& a, int tiles, const TileRun* runs,
   const int outs = GLU ? 64 : 128, n_blocks = (a.N + outs - 1) / outs;
   if (runs) {
     const int wide_blocks = (a.N + WIDE_OUT(GLU) - 1) / WIDE_OUT(GLU);
-    const long pairs = groups((long)max_pairs * wide_blocks);
-    static_assert(PairShape::BM == 2 * GS_M && HalfShape::BM == GS_M && HalfShape::LDS <= PairShape::LDS, "");
-    auto kernel = grouped_gemm_pairs_kernel<GLU>;
+    const int odd_blocks = (a.N + ODD_OUT(GLU) - 1) / ODD_OUT(GLU);
+    // whole pairs W and odd tiles O are 2 W + O tiles at most, and W + O pairs: W + 2 O <= 3 max_pairs - tiles + 1 (an odd tile is two items;
+    // each die's stretch is rounded up)
+    const long pairs = groups((3l * max_pairs - tiles + 1) * wide_blocks) + 2 * GS_DIES;
+    static_assert(PairShape::BM == 2 * GS_M && OddShape::BM == GS_M && HalfShape::BM == GS_M && HalfShape::LDS <= PairShape::LDS && OddShape::LDS <= PairShape::LDS && ShortShape::LDS <= PairShape::LDS &&
+                      WIDE_OUT(GLU) == 2 * ODD_OUT(GLU), "");
+    auto kernel = odd_apart(2 * max_pairs - tiles + 1, wide_blocks, a.K) ? grouped_gemm_pairs_kernel<GLU, true> : grouped_gemm_pairs_kernel<GLU, false>;
     if (pairs >= (1l << 31) || hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PairShape::LDS) != hipSuccess)
       return false;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)pairs), dim3(256), PairShape::LDS, stream, a, runs, wide_blocks);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)pairs), dim3(256), PairShape::LDS, stream, a, runs, max_pairs, wide_blocks, odd_blocks);
     return true;
   }
   const long grid = groups((long)tiles * n_blocks);
@@ -479,7 +515,7 @@ TK_API int tk_grouped_gemm_bf16(const void* A, int lda, const int* a_row, const 
 struct SortJob {
   const int* ids;
   int *slot_pair, *slot_token, *tile_group;
-  TileRun* runs;  // (grouped_gemm_pairs_kernel: room for the number and max_pairs pairs)
+  TileRun* runs;  // (grouped_gemm_pairs_kernel: room for the numbers and twice max_pairs pairs)
   int pairs, top, experts, max_tiles, max_pairs;
 };
 #define SORT_JOBS 48
@@ -516,13 +552,18 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(SortJobs jobs) {
       twos += (n + 1) / 2;
     }
     tile_group[max_tiles] = at / tm;
-    jb.runs[0] = {twos, 0, 0, 0};
+    jb.runs[0] = {twos, at / tm - twos, 2 * twos - at / tm, 0};
   }
   __syncthreads();
   for (int e = threadIdx.x; e < experts; e += blockDim.x) {
     const int t0 = first[e] / tm, n = (count[e] + tm - 1) / tm;
     for (int t = 0; t < n; ++t) tile_group[t0 + t] = e;
     for (int p = 0; p < (n + 1) / 2; ++p) jb.runs[1 + first_pair[e] + p] = {t0, e, first_pair[e], n};
+    // of the t0 tiles in front, in first_pair[e] pairs: whole pairs t0 - first_pair[e], odd tiles the rest of the pairs
+    TileRun* order = jb.runs + 1 + jb.max_pairs;
+    const int whole = t0 - first_pair[e];
+    for (int p = 0; p < n / 2; ++p) order[whole + p] = {t0, e, whole, n / 2};
+    if (n & 1) order[jb.max_pairs - 1 - (first_pair[e] - whole)] = {t0 + n - 1, e, count[e] - (n - 1) * tm, 1};
   }
   __syncthreads();
   for (int p = threadIdx.x; p < pairs; p += blockDim.x) {

@@ -2691,7 +2691,7 @@ def expert_sort(choices: "list[tuple[torch.Tensor, int]]") -> "list[SortedPairs]
         slots = max_tiles * EXPERT_TILE
         max_pairs, end = (max_tiles + min(int(experts), max_tiles)) // 2, 2 * slots + max_tiles + 1
         at = -(-end // 4) * 4  # (a run is 16 bytes)
-        book = torch.empty((at + 4 * (1 + max_pairs),), dtype=torch.int32, device=ids.device)
+        book = torch.empty((at + 4 * (1 + 2 * max_pairs),), dtype=torch.int32, device=ids.device)
         s = SortedPairs(book[:slots], book[slots : 2 * slots], book[2 * slots : end], book, at, max_tiles, max_pairs, (n, top))
         start = book.data_ptr()  # (4 bytes a number)
         job.ids, job.slot_pair, job.slot_token, job.tile_group, job.runs = ids.data_ptr(), start, start + 4 * slots, start + 8 * slots, start + 4 * at
