@@ -76,3 +76,16 @@ def test_infinities_and_nan_stay_in_their_rows(m):
     a[0, 3], a[1, 5] = float("inf"), float("nan")
     got = ops.gemm_generic(a, w)
     assert torch.isinf(got[0]).all() and torch.isnan(got[1]).all() and torch.isfinite(got[2:]).all()
+
+
+@pytest.mark.parametrize("m", [17, 32, 33, 64, 65, 129, 300])
+@pytest.mark.parametrize("nk", [(1, 32), (63, 64), (64, 96), (260, 128), (1000, 160), (1133, 1024), (2052, 992)])
+def test_steps_straight_to_local_memory(m, nk):
+    """Inner sizes of whole steps: fewer than local memory holds, as many, and more; every one in one and in several parts."""
+    test_sizes(m, nk)
+
+
+def test_largest_tiles_straight_to_local_memory():
+    """128 x 128, which take as many tiles as fill the chip twice; rows and columns that end inside one."""
+    for m, n, k in ((2100, 4100, 64), (2048, 4160, 96), (2049, 4096, 32)):
+        test_sizes(m, (n, k))

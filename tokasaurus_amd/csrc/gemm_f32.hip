@@ -9,12 +9,12 @@
 // every lane, so it sums the elements 4 q + s, q < 4, which is a permutation of K that both operands share.  Weights as
 // the first operand: acc[j] of lane (r, q) = C[token r][weight row 4 q + j], a 16-byte store.
 //
-// Two kernels:
+// Two kinds of kernels:
 //   gemm_f32_few_kernel (up to 16 tokens, bound by reading W once): a workgroup's wavefronts cut K between them and add up
 //     in the order of K; operands straight from memory to registers, two sets of them, so that one set's loads are in
 //     flight while the other is multiplied.  Sixteen sums a result (one an instruction of a set) keep every chain of
 //     additions at 32 to 64 elements: with one chain a wavefront the error is three times as large, at no gain.
-//   gemm_f32_kernel (more tokens, bound by the matrix cores): four wavefronts share a tile's rows through local memory.
+//   gemm_f32_stream_kernel and, for a K that is no multiple of 32, gemm_f32_kernel (more tokens, bound by the matrix cores): four wavefronts share a tile's rows through local memory.
 //     A compute unit's caches bring about 18 bytes a cycle: wavefronts that each load the operands of 32 x 32 results for
 //     themselves need 32 and reach half of the matrix cores' rate (2 048 x 16 384 x 2 048: 76 TFLOP/s, straight from
 //     memory or through local memory of their own); a shared tile of 64 x 64 needs 16, of 128 x 128 8.  Where the tiles are
@@ -22,7 +22,7 @@
 // Measured against the plain kernels that this replaces (us; floors at 5.05 TB/s and 153 TFLOP/s): 4 tokens 2 048 x 2 048 6.9
 // (floor 3.3), 2 048 x 8 192 17.5 (13), 16 384 x 2 048 29.5 (27); before 36 for the first two in the mean, and 33.  301
 // tokens 2 048 x 2 048 38 (17), 2 048 x 8 192 116 (66), 3 072 x 2 048 53 (25), 16 384 x 2 048 207 (132); before 746 for
-// the first two in the mean, 301 and 643.  2 048 tokens 16 384 x 2 048 1 115 (898, 123 TFLOP/s).  Errors against 64-bit
+// the first two in the mean, 301 and 643 (gemm_f32_stream_kernel has the figures for K of a multiple of 32).  Errors against 64-bit
 // sums: up to 32 tokens those of the plain kernel (1.2e-7 of the norm at 2 048 elements), beyond at most the plain kernel's.
 #include "common.h"
 
@@ -152,6 +152,34 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a) {
   if (r < min(a.M, ROWS) && 4 * q < ROWS && n0 + 4 * q < a.N) gf_store(a, sum, r, n0 + 4 * q);
 }
 
+// The chains of a tile's sums added, and the results stored, or the part of K among the other parts' sums.
+template <int TM, int TN, int CHAINS>
+__device__ __forceinline__ void gf_finish(const GemmF32Args& a, f4 (&acc)[CHAINS][TN][TM], int m0, int n0, int wave, int r, int q) {
+#pragma unroll
+  for (int half = CHAINS / 2; half > 0; half /= 2)
+#pragma unroll
+    for (int c = 0; c < half; ++c)
+#pragma unroll
+      for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int u = 0; u < TM; ++u) acc[c][t][u] += acc[c + half][t][u];
+#pragma unroll
+  for (int u = 0; u < TM; ++u) {
+    const int token = m0 + (wave >> 1) * 16 * TM + 16 * u + r;
+    if (token >= a.M) continue;
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+      const int n = n0 + (wave & 1) * 16 * TN + 16 * t + 4 * q;
+      if (n >= a.N) continue;
+      if (a.part) {  // (N is a multiple of 4 then)
+        *(f4*)(a.part + ((size_t)blockIdx.y * a.M + token) * a.N + n) = acc[0][t][u];
+      } else {
+        gf_store(a, acc[0][t][u], token, n);
+      }
+    }
+  }
+}
+
 #define GS_ROW 36  // floats a row of 32 takes in local memory: 16 lanes that read 16 rows at one place meet 64 different banks
 
 // A workgroup: a tile of 32 TM tokens x 32 TN weight rows, its four wavefronts a quarter each, over the steps of 32 elements
@@ -237,29 +265,83 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmF32Args a) {
           }
     __syncthreads();
   }
+  gf_finish<TM, TN, CHAINS>(a, acc, m0, n0, wave, r, q);
+}
+
+// The same for a K of a multiple of 32, with the same bits: rows of A and W go straight from memory to local memory, STAGES - 1 steps
+// ahead, with no registers between, the 16-byte piece c of a row at place c ^ gs_swizzle(row), which 16 lanes that read 16
+// rows at one place find in 64 different banks.  Through registers a compute unit gets about 18 bytes a cycle, and a tile of 64 x 64 needs
+// 16 at the matrix cores' full rate.  us through registers / straight, weights from memory: 301 tokens 16,384 x 2,048 192 / 177, 2,048 x
+// 8,192 105 / 97, 3,072 x 2,048 48.3 / 44.6; 100 tokens 90 / 81, 50 / 46, 24.1 / 22.5; 17 tokens 44.6 / 40.0, 27.8 / 24.8, 13.9 / 12.4; 2,048 tokens
+// 1,117 / 1,018 (135 TFLOP/s), 604 / 559, 229 / 213.
+__device__ __forceinline__ int gs_swizzle(int row) { return (row ^ (row >> 3 & 1)) & 7; }
+
+template <int TM, int TN, int CHAINS, int STAGES>
+__global__ __launch_bounds__(256) void gemm_f32_stream_kernel(GemmF32Args a) {
+  extern __shared__ __align__(16) float tile[];  // [STAGES][32 * (TN + TM)][32], weight rows first
+  constexpr int ROWS = 32 * (TN + TM), LOADS = ROWS / 32;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int mt = (a.M + 32 * TM - 1) / (32 * TM);  // (workgroups on the dies as in gemm_f32_kernel)
+  const int g = blockIdx.x / 8;
+  const int n0 = ((g / mt) * 8 + blockIdx.x % 8) * 32 * TN, m0 = (g % mt) * 32 * TM;
+  if (n0 >= a.N) return;  // the same for the whole workgroup
+  const int all = a.K >> 5;
+  const int s0 = (int)((long)all * blockIdx.y / gridDim.y), steps = (int)((long)all * (blockIdx.y + 1) / gridDim.y) - s0;
+  const int lr = 8 * wave + (lane >> 3);  // load i brings row 32 i + lr
+  const int lc = ((lane & 7) ^ gs_swizzle(lr)) * 4;
+  const float* src[LOADS];
 #pragma unroll
-  for (int half = CHAINS / 2; half > 0; half /= 2)
+  for (int i = 0; i < LOADS; ++i)
+    src[i] = (i < TN ? a.W + (size_t)min(n0 + 32 * i + lr, a.N - 1) * a.K : a.A + (size_t)min(m0 + 32 * (i - TN) + lr, a.M - 1) * a.lda) + lc + (size_t)s0 * 32;
+  const unsigned lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)tile;
+  auto ask = [&](int step, int place) {
 #pragma unroll
-    for (int c = 0; c < half; ++c)
+    for (int i = 0; i < LOADS; ++i)
+      load_to_lds((const bf16_t*)(src[i] + (size_t)step * 32), lds + (unsigned)((place * ROWS + 32 * i + 8 * wave) * 32 * (int)sizeof(float)));
+  };
+  for (int s = 0; s < STAGES - 1 && s < steps; ++s) ask(s, s);
+  f4 acc[CHAINS][TN][TM];
 #pragma unroll
-      for (int t = 0; t < TN; ++t)
+  for (int c = 0; c < CHAINS; ++c)
 #pragma unroll
-        for (int u = 0; u < TM; ++u) acc[c][t][u] += acc[c + half][t][u];
+    for (int t = 0; t < TN; ++t)
 #pragma unroll
-  for (int u = 0; u < TM; ++u) {
-    const int token = m0 + (wave >> 1) * 16 * TM + 16 * u + r;
-    if (token >= a.M) continue;
+      for (int u = 0; u < TM; ++u) acc[c][t][u] = (f4){0.f, 0.f, 0.f, 0.f};
+  const int piece[2] = {(q ^ gs_swizzle(r)) * 4, ((4 + q) ^ gs_swizzle(r)) * 4};
+  const float* wrow = tile + ((wave & 1) * 16 * TN + r) * 32;
+  const float* xrow = tile + (32 * TN + (wave >> 1) * 16 * TM + r) * 32;
+  int here = 0, next = STAGES - 1;
+#pragma unroll 1
+  for (int s = 0; s < steps; ++s) {
+    // the step is there when only the loads of the STAGES - 2 behind it are left; behind the barrier every wavefront's are,
+    // and every wavefront is through with the step before, whose place is filled again
+    if (s + STAGES - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 2) * LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (s + STAGES - 1 < steps) ask(s + STAGES - 1, next);
+    f4 w[2][TN], x[2][TM];
 #pragma unroll
-    for (int t = 0; t < TN; ++t) {
-      const int n = n0 + (wave & 1) * 16 * TN + 16 * t + 4 * q;
-      if (n >= a.N) continue;
-      if (a.part) {  // (N is a multiple of 4 then)
-        *(f4*)(a.part + ((size_t)blockIdx.y * a.M + token) * a.N + n) = acc[0][t][u];
-      } else {
-        gf_store(a, acc[0][t][u], token, n);
-      }
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+      for (int t = 0; t < TN; ++t) w[b][t] = *(const f4*)(wrow + (here * ROWS + 16 * t) * 32 + piece[b]);
+#pragma unroll
+      for (int t = 0; t < TM; ++t) x[b][t] = *(const f4*)(xrow + (here * ROWS + 16 * t) * 32 + piece[b]);
     }
+    here = here + 1 == STAGES ? 0 : here + 1;
+    next = next + 1 == STAGES ? 0 : next + 1;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t = 0; t < TN; ++t)
+#pragma unroll
+          for (int u = 0; u < TM; ++u) {
+            const int c = (4 * b + e) % CHAINS;
+            acc[c][t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[b][t][e], x[b][u][e], acc[c][t][u], 0, 0, 0);
+          }
   }
+  gf_finish<TM, TN, CHAINS>(a, acc, m0, n0, wave, r, q);
 }
 
 // The sums of K's parts added in the order of K: a thread four neighbouring outputs.
@@ -300,8 +382,12 @@ template <int TM, int TN, int CHAINS>
 static bool gf_launch(const GemmF32Args& a, int cuts, hipStream_t stream) {
   const long grid = gf_tiles(a.M, a.N, TM, TN);
   if (grid > 0x7fffffffL) return false;
-  const size_t lds = (size_t)2 * 32 * (TM + TN) * GS_ROW * sizeof(float);
-  auto kernel = gemm_f32_kernel<TM, TN, CHAINS>;
+  // steps in local memory: 2 of the largest tile, so that two workgroups share a compute unit (3: 1,117 us for 2,048 tokens and 16,384 x 2,048
+  // as before, 2: 1,018), else 3 (2: 301 tokens 189 / 177, 102 / 97 us)
+  constexpr int STAGES = TM * TN == 16 ? 2 : 3;
+  const bool stream_in = a.K % 32 == 0;
+  const size_t lds = stream_in ? (size_t)STAGES * 32 * (TM + TN) * 32 * sizeof(float) : (size_t)2 * 32 * (TM + TN) * GS_ROW * sizeof(float);
+  auto kernel = stream_in ? gemm_f32_stream_kernel<TM, TN, CHAINS, STAGES> : gemm_f32_kernel<TM, TN, CHAINS>;
   if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return false;
   hipLaunchKernelGGL(kernel, dim3((unsigned)grid, cuts), dim3(256), lds, stream, a);
   return true;
