@@ -38,6 +38,8 @@
 // by the token's position, writes q to the output and k and v into the token's page.
 #include "common.h"
 
+#include <type_traits>
+
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
@@ -733,52 +735,60 @@ __global__ __launch_bounds__(256, 2) void gemm_glu_stream_kernel(GemmArgs a) {
   // apart, 8 rows: 8,192 x 2,048 18.3 / 14.9 us, 8,192 x 4,096 30.8 / 26.8, 28,672 x 8,192 179 / 164, 5,632 x 2,048 12.6 / 11.4; but 8,192 x
   // 2,304 16.5 / 17.3, 8,192 x 3,072 20.3 / 20.6, 13,824 x 5,120 52.4 / 53.6, and with half of the compute units 4,096 x 2,048 11.6 / 12.6.
   const int turn = (int)(blockIdx.x * 7u) & a.turn;
-  auto ask = [&](int step) {
-    const unsigned base = lds + (unsigned)(step % S * ROWS * GL_K * sizeof(bf16_t));
-    const size_t k = (size_t)(step + turn < steps ? step + turn : step + turn - steps) * GL_K;
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const int row = i < 2 ? wave * 16 + i * 8 : 64 + (wave * (MB / 2) + i - 2) * 8;
-      load_to_lds(src[i] + k, base + (unsigned)(row * GL_K * sizeof(bf16_t)));
-    }
-  };
   // With a norm in front: the partial sums of a wavefront's first rows come into the place of the step that is asked for last,
   // and are added up while the weights are on their way (added behind the last step 0.5 us at one row, 0.8 at 8).
   constexpr int EARLY = MB == 2 ? 2 : 4;
   static_assert(4 * EARLY * 1024 <= ROWS * GL_K * (int)sizeof(bf16_t), "the partial sums fit a step's place");
   const unsigned parts = (unsigned)((S - 1) * ROWS * GL_K * sizeof(bf16_t)) + wave * (EARLY * 1024);
-  if (NORM && a.early_lanes > 0) {
-#pragma unroll
-    for (int i = 0; i < EARLY; ++i) load_to_lds((const bf16_t*)row_parts(a, wave + 4 * i, lane), lds + parts + i * 1024);
-  }
-  for (int s = 0; s < S - 1 && s < steps; ++s) ask(s);
-  if (NORM && a.early_lanes > 0) {
-    if (steps >= S - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * LOADS) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < EARLY; ++i) early_row_scale(a, scales, *(const f32x4_t*)(smem + parts + i * 1024 + lane * 16), wave + 4 * i, lane);
-  }
   f32x4_t acc[NB];
 #pragma unroll
   for (int mb = 0; mb < NB; ++mb) acc[mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < steps; ++s) {
-    // the step is there when only the loads of the S - 2 behind it are left; behind the barrier every wavefront's are, and
-    // every wavefront is through with the step before, whose place is filled again
-    if (s + S - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * LOADS) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (s + S - 1 < steps) ask(s + S - 1);
-    const bf16_t* at = rows + (size_t)(s % S) * ROWS * GL_K;
+  // LOADS: of W's rows alone for a wavefront whose rows of A are all behind the last (what lies in their place is read into results
+  // that nobody stores); the last row again in their place / nothing, us: 8,192 x 2,048 14.6 / 14.4 at one row, 14.1 / 13.8 at 8,
+  // 14,336 x 4,096 44.7 / 44.1, 42.2 / 41.6, 1,024 x 2,048 10.2 / 9.8
+  auto walk = [&](auto loads_a_step) {
+    constexpr int LOADS = decltype(loads_a_step)::value;
+    auto ask = [&](int step) {
+      const unsigned base = lds + (unsigned)(step % S * ROWS * GL_K * sizeof(bf16_t));
+      const size_t k = (size_t)(step + turn < steps ? step + turn : step + turn - steps) * GL_K;
 #pragma unroll
-    for (int kk = 0; kk < GL_K / 32; ++kk) {
-      const int place = ((4 * kk + q) ^ (r & 7)) * 8;
-      const bf16x8_t wv = *(const bf16x8_t*)(at + (wave * 16 + r) * GL_K + place);
+      for (int i = 0; i < LOADS; ++i) {
+        const int row = i < 2 ? wave * 16 + i * 8 : 64 + (wave * (MB / 2) + i - 2) * 8;
+        load_to_lds(src[i] + k, base + (unsigned)(row * GL_K * sizeof(bf16_t)));
+      }
+    };
+    if (NORM && a.early_lanes > 0) {
 #pragma unroll
-      for (int mb = 0; mb < NB; ++mb) {
-        const bf16x8_t av = *(const bf16x8_t*)(at + (64 + 16 * mb + r) * GL_K + place);
-        acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, av, acc[mb], 0, 0, 0);
+      for (int i = 0; i < EARLY; ++i) load_to_lds((const bf16_t*)row_parts(a, wave + 4 * i, lane), lds + parts + i * 1024);
+    }
+    for (int s = 0; s < S - 1 && s < steps; ++s) ask(s);
+    if (NORM && a.early_lanes > 0) {
+      if (steps >= S - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * LOADS) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < EARLY; ++i) early_row_scale(a, scales, *(const f32x4_t*)(smem + parts + i * 1024 + lane * 16), wave + 4 * i, lane);
+    }
+    for (int s = 0; s < steps; ++s) {
+      // the step is there when only the loads of the S - 2 behind it are left; behind the barrier every wavefront's are, and
+      // every wavefront is through with the step before, whose place is filled again
+      if (s + S - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * LOADS) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (s + S - 1 < steps) ask(s + S - 1);
+      const bf16_t* at = rows + (size_t)(s % S) * ROWS * GL_K;
+#pragma unroll
+      for (int kk = 0; kk < GL_K / 32; ++kk) {
+        const int place = ((4 * kk + q) ^ (r & 7)) * 8;
+        const bf16x8_t wv = *(const bf16x8_t*)(at + (wave * 16 + r) * GL_K + place);
+#pragma unroll
+        for (int mb = 0; mb < NB; ++mb) {
+          const bf16x8_t av = *(const bf16x8_t*)(at + (64 + 16 * mb + r) * GL_K + place);
+          acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, av, acc[mb], 0, 0, 0);
+        }
       }
     }
-  }
+  };
+  if (wave * (MB / 2) * 8 < a.M) walk(std::integral_constant<int, 2 + MB / 2>());
+  else walk(std::integral_constant<int, 2>());
   if (NORM && (a.early_lanes == 0 || a.M > 4 * EARLY)) {
     row_scales<MB>(a, scales, wave, lane, 4, EARLY);
     __syncthreads();

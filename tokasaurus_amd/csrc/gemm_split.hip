@@ -19,6 +19,8 @@
 // With three blocks it is behind (2,048 x 2,048 14.8 / 18.1 at 300 rows, 4,096 x 14,336 75 / 91).
 #include "common.h"
 
+#include <type_traits>
+
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
@@ -58,46 +60,53 @@ __global__ __launch_bounds__(256) void gemm_split_kernel(SplitArgs a) {
 #pragma unroll
   for (int i = 0; i < MB / 2; ++i)
     src[2 + i] = a.A + (size_t)min(row0 + (wave * (MB / 2) + i) * 8 + lr, a.M - 1) * a.lda + (size_t)s0 * GS_K + piece;
-  auto ask = [&](int step, int place) {
-    const unsigned base = lds + (unsigned)(place * ROWS * GS_K * (int)sizeof(bf16_t));
-    const size_t k = (size_t)step * GS_K;
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const int row = i < 2 ? wave * 16 + i * 8 : 64 + (wave * (MB / 2) + i - 2) * 8;
-      load_to_lds(src[i] + k, base + (unsigned)(row * GS_K * (int)sizeof(bf16_t)));
-    }
-  };
-  for (int s = 0; s < STAGES - 1 && s < steps; ++s) ask(s, s);
   f32x4_t acc[TW][NW];
 #pragma unroll
   for (int t = 0; t < TW; ++t)
 #pragma unroll
     for (int mb = 0; mb < NW; ++mb) acc[t][mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int wn = WM == 2 ? wave >> 1 : wave, wm = WM == 2 ? wave & 1 : 0;
-  int at_stage = 0, next_stage = STAGES - 1;
-  for (int s = 0; s < steps; ++s) {
-    // the step is there when only the loads of the STAGES - 2 behind it are left; behind the barrier every wavefront's are,
-    // and every wavefront is through with the step before, whose place is filled again
-    if (s + STAGES - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 2) * LOADS) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (s + STAGES - 1 < steps) ask(s + STAGES - 1, next_stage);
-    const bf16_t* at = rows + (size_t)at_stage * ROWS * GS_K;
-    at_stage = at_stage + 1 == STAGES ? 0 : at_stage + 1;
-    next_stage = next_stage + 1 == STAGES ? 0 : next_stage + 1;
+  // LOADS: of W's rows alone for a wavefront whose rows of A are all behind the last (what lies in their place is read into results
+  // that nobody stores)
+  auto walk = [&](auto loads_a_step) {
+    constexpr int LOADS = decltype(loads_a_step)::value;
+    auto ask = [&](int step, int place) {
+      const unsigned base = lds + (unsigned)(place * ROWS * GS_K * (int)sizeof(bf16_t));
+      const size_t k = (size_t)step * GS_K;
 #pragma unroll
-    for (int kk = 0; kk < GS_K / 32; ++kk) {
-      const int place = ((4 * kk + q) ^ (r & 7)) * 8;
-      bf16x8_t wv[TW];
+      for (int i = 0; i < LOADS; ++i) {
+        const int row = i < 2 ? wave * 16 + i * 8 : 64 + (wave * (MB / 2) + i - 2) * 8;
+        load_to_lds(src[i] + k, base + (unsigned)(row * GS_K * (int)sizeof(bf16_t)));
+      }
+    };
+    for (int s = 0; s < STAGES - 1 && s < steps; ++s) ask(s, s);
+    int at_stage = 0, next_stage = STAGES - 1;
+    for (int s = 0; s < steps; ++s) {
+      // the step is there when only the loads of the STAGES - 2 behind it are left; behind the barrier every wavefront's are,
+      // and every wavefront is through with the step before, whose place is filled again
+      if (s + STAGES - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 2) * LOADS) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (s + STAGES - 1 < steps) ask(s + STAGES - 1, next_stage);
+      const bf16_t* at = rows + (size_t)at_stage * ROWS * GS_K;
+      at_stage = at_stage + 1 == STAGES ? 0 : at_stage + 1;
+      next_stage = next_stage + 1 == STAGES ? 0 : next_stage + 1;
 #pragma unroll
-      for (int t = 0; t < TW; ++t) wv[t] = *(const bf16x8_t*)(at + ((wn * TW + t) * 16 + r) * GS_K + place);
+      for (int kk = 0; kk < GS_K / 32; ++kk) {
+        const int place = ((4 * kk + q) ^ (r & 7)) * 8;
+        bf16x8_t wv[TW];
 #pragma unroll
-      for (int mb = 0; mb < NW; ++mb) {
-        const bf16x8_t av = *(const bf16x8_t*)(at + (64 + 16 * (wm * NW + mb) + r) * GS_K + place);
+        for (int t = 0; t < TW; ++t) wv[t] = *(const bf16x8_t*)(at + ((wn * TW + t) * 16 + r) * GS_K + place);
 #pragma unroll
-        for (int t = 0; t < TW; ++t) acc[t][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[t], av, acc[t][mb], 0, 0, 0);
+        for (int mb = 0; mb < NW; ++mb) {
+          const bf16x8_t av = *(const bf16x8_t*)(at + (64 + 16 * (wm * NW + mb) + r) * GS_K + place);
+#pragma unroll
+          for (int t = 0; t < TW; ++t) acc[t][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[t], av, acc[t][mb], 0, 0, 0);
+        }
       }
     }
-  }
+  };
+  if (MB > 2 || wave * (MB / 2) * 8 < a.M - row0) walk(std::integral_constant<int, 2 + MB / 2>());
+  else walk(std::integral_constant<int, 2>());
   float* out = a.part + (size_t)cut * a.M * a.N;
 #pragma unroll
   for (int mb = 0; mb < NW; ++mb) {
