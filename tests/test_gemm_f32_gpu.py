@@ -89,3 +89,10 @@ def test_largest_tiles_straight_to_local_memory():
     """128 x 128, which take as many tiles as fill the chip twice; rows and columns that end inside one."""
     for m, n, k in ((2100, 4100, 64), (2048, 4160, 96), (2049, 4096, 32)):
         test_sizes(m, (n, k))
+
+
+@pytest.mark.parametrize("m", [1, 3, 4, 8])
+@pytest.mark.parametrize("nk", [(20, 8192), (9, 8224), (2050, 8192), (24, 16384)])
+def test_few_rows_over_long_inner_sizes(m, nk):
+    """Where the second half of K, or the next elements, take the matrix core's unused half."""
+    test_sizes(m, nk)

@@ -66,21 +66,26 @@ __device__ __forceinline__ void gf_store(const GemmF32Args& a, f4 v, int token, 
 #define GF_UNROLL 4  // blocks of 16 elements a set of loads
 
 // HALVES (up to 8 tokens, K a multiple of 32): a workgroup has 8 weight rows, and the unused half of the matrix core's rows and of its
-// columns takes the second half of K (the blocks of results off the diagonal are not used), so that a weight of few rows gives
-// every compute unit a workgroup.  4 tokens, us by rows of 16 / of 8, weights from memory: 2,048 x 2,048 8.6 / 6.9, 2,048 x 8,192 26.4 / 17.5
+// columns takes other elements of K (the blocks of results off the diagonal are not used), so that a weight of few rows gives
+// every compute unit a workgroup.  NEXT: the next 16 elements, so that a load takes whole lines of 128 bytes; else the second half
+// of K, for up to 3 tokens and long rows.  us second half / next: 4 tokens 2,048 x 2,048 6.4 / 5.9, 2,048 x 8,192 20.3 / 20.3, 8 tokens 7.4 / 6.5,
+// 23.4 / 22.1, 1 token 5.8 / 5.4, 16.5 / 19.4 (rows 32 KB apart begin in one of the memory's channels).  4 tokens, us by rows of 16 / of 8, weights from memory: 2,048 x 2,048 8.6 / 6.9, 2,048 x 8,192 26.4 / 17.5
 // (3.8 TB/s), 3,072 x 2,048 8.8 / 9.6, 16,384 x 2,048 26.8 / 31.2.  Each chain of sums is half as long: error 1.2e-7 / 1.0e-7 of the norm
 // over 2,048 elements, 1.6e-7 / 1.3e-7 over 8,192.
-template <bool HALVES>
-__global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a) {
+template <bool HALVES, bool NEXT>
+__global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a, int KS, int share, int spare) {
   extern __shared__ __align__(16) f4 sums[];  // [wavefronts - 1][64]
+  // every argument that a first load needs, in one trip
+  asm volatile("" ::"s"(a.A), "s"(a.W), "s"(a.lda), "s"(a.M), "s"(a.N), "s"(a.K), "s"(KS), "s"(share), "s"(spare));
   // (the wavefront's number as one value for all its lanes, so that its loop counts in scalar registers)
-  const int lane = threadIdx.x & 63, kw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), KS = blockDim.x >> 6;
+  const int lane = threadIdx.x & 63, kw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, q = lane >> 4;
   constexpr int ROWS = HALVES ? 8 : 16;
   const int n0 = blockIdx.x * ROWS, own = HALVES ? r & 7 : r;
-  const size_t from = HALVES ? (size_t)(r >> 3) * (a.K / 2) : 0;  // of K
+  const int from = HALVES ? (r >> 3) * (NEXT ? 16 : a.K / 2) : 0;
+  constexpr int STEP = HALVES && NEXT ? 32 : 16;  // elements of K a block and its partner are on
   const int blocks = HALVES ? a.K >> 5 : (a.K + 15) >> 4;
-  const int b0 = (int)((long)blocks * kw / KS), b1 = (int)((long)blocks * (kw + 1) / KS);
+  const int b0 = kw * share + min(kw, spare), b1 = b0 + share + (kw < spare ? 1 : 0);
   const float* wp = a.W + (size_t)min(n0 + own, a.N - 1) * a.K + from + 4 * q;
   const float* ap = a.A + (size_t)min(own, a.M - 1) * a.lda + from + 4 * q;
   f4 acc[GF_UNROLL][4];
@@ -93,8 +98,8 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a) {
 #define GF_LOAD(set, b)                                                                             \
   do {                                                                                              \
     _Pragma("unroll") for (int u = 0; u < GF_UNROLL; ++u) {                                         \
-      w[set][u] = *(const f4*)(wp + (size_t)((b) + u) * 16);                                        \
-      x[set][u] = *(const f4*)(ap + (size_t)((b) + u) * 16);                                        \
+      w[set][u] = *(const f4*)(wp + (size_t)((b) + u) * STEP);                                      \
+      x[set][u] = *(const f4*)(ap + (size_t)((b) + u) * STEP);                                      \
     }                                                                                               \
     __builtin_amdgcn_sched_barrier(0);                                                              \
   } while (0)
@@ -129,7 +134,7 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a) {
 #pragma unroll 1
   for (; b < b1; ++b) {  // what is left, the last block perhaps cut by K: zeros behind it
     const bool in = HALVES || b * 16 + 4 * q < a.K;
-    const long off = in ? (long)b * 16 : -4L * q;
+    const long off = in ? (long)b * STEP : -4L * q;
     f4 wv = *(const f4*)(wp + off), xv = *(const f4*)(ap + off);
     if (!in) wv = xv = (f4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -143,9 +148,10 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a) {
     if (kw > 0) sums[(kw - 1) * 64 + lane] = sum;
     __syncthreads();
     if (kw > 0) return;
+#pragma unroll 4
     for (int k = 0; k < KS - 1; ++k) sum += sums[k * 64 + lane];
   }
-  if (HALVES) {  // the second half's sums of token r lie in the lanes of token r + 8 and of rows 8 more
+  if (HALVES) {  // the partners' sums of token r lie in the lanes of token r + 8 and of rows 8 more
 #pragma unroll
     for (int j = 0; j < 4; ++j) sum[j] += __shfl(sum[j], (lane + 40) & 63, 64);
   }
@@ -407,10 +413,11 @@ TK_API int tk_gemm_f32(const void* A, int lda, const void* W, void* C, int ldc, 
     // (2, 4, 8 wavefronts at 4 tokens, 2 048 x 2 048: 9.0, 8.2, 9.0 us, 2 048 x 8 192: 34, 25, 26, 16 384 x 2 048: 33, 30, 30)
     const int KS = K < 64 ? 1 : (K < 4096 ? 4 : 8);
     // rows of 8 where rows of 16 leave compute units without a workgroup
-    if (M <= 8 && K % 32 == 0 && K >= 256 && N <= GF_HALVES_ROWS)
-      hipLaunchKernelGGL(gemm_f32_few_kernel<true>, dim3((N + 7) / 8), dim3(64 * KS), (KS - 1) * 64 * sizeof(f4), stream, a);
-    else
-      hipLaunchKernelGGL(gemm_f32_few_kernel<false>, dim3((N + 15) / 16), dim3(64 * KS), (KS - 1) * 64 * sizeof(f4), stream, a);
+    const bool halves = M <= 8 && K % 32 == 0 && K >= 256 && N <= GF_HALVES_ROWS;
+    const int blocks = halves ? K / 32 : (K + 15) / 16;
+    auto few = !halves ? gemm_f32_few_kernel<false, false> : (M >= 4 || K < 8192 ? gemm_f32_few_kernel<true, true> : gemm_f32_few_kernel<true, false>);
+    const int rows = halves ? 8 : 16;
+    hipLaunchKernelGGL(few, dim3((N + rows - 1) / rows), dim3(64 * KS), (KS - 1) * 64 * sizeof(f4), stream, a, KS, blocks / KS, blocks % KS);
     TK_CHECK_LAUNCH("gemm_f32");
     return 0;
   }
