@@ -1,6 +1,6 @@
 """The weight-streaming and the streamed gate and up products with a norm in front, at the edges of what is asked for early: rows
-beyond a wavefront's first, partial sums that are as many as the lanes take, more, and no multiple of 4; and a rotation
-behind a folded K."""
+beyond a wavefront's first, partial sums that are as many as the lanes take, more, and no multiple of 4; a rotation
+behind a folded K; and the norm by itself where the pieces of a row that a thread holds change in number."""
 
 from __future__ import annotations
 
@@ -91,3 +91,22 @@ def test_wavefronts_share_the_keys_that_a_split_has(d, split, waves, window):
         p = torch.softmax((k @ q[i].double().view(nq, d, 1))[..., 0] * d ** -0.5, -1)
         want, size = (p[:, None] @ v)[:, 0], (p[:, None] @ v.abs())[:, 0]
         assert ((got[i].double().view(nq, d) - want).abs() <= 2.0 ** -7 * size + 1e-6).all(), n
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("pieces", [1, 255, 256, 257, 511, 512, 513, 1024, 1025])
+def test_rows_held_in_registers_by_the_norm(dtype, pieces):
+    """Where a thread's pieces of 16 bytes go from one to two to four and to a loop, and where its last one lies behind the row's end."""
+    hidden = pieces * 16 // dtype.itemsize
+    gen = torch.Generator().manual_seed(pieces)
+    x, r = (torch.randn((3, hidden), generator=gen).to(dtype) for _ in range(2))
+    for weight_dtype in {dtype, torch.float32}:
+        w = (1 + 0.1 * torch.randn((hidden,), generator=gen)).to(weight_dtype)
+        stream, normed = (t.cpu() for t in ops.add_rmsnorm(x.cuda(), r.cuda(), w.cuda(), 1e-5))
+        assert torch.equal(stream, x + r)
+        rows = stream.double()
+        want = w.double() * rows / torch.sqrt(rows.pow(2).mean(1, keepdim=True) + 1e-5)
+        # a row's sum of squares is good to (hidden / 256 + 16) roundings; the normed value and its product with the weight are rounded (half an eps each)
+        limit = want.abs() * (1.02 * torch.finfo(dtype).eps + (hidden / 256 + 24) * 2.0 ** -23)
+        assert ((normed.double() - want).abs() <= limit).all()
+        assert torch.equal(ops.rmsnorm(stream.cuda(), w.cuda(), 1e-5).cpu(), normed)

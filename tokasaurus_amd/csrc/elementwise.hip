@@ -72,9 +72,12 @@ __global__ void rmsnorm_kernel(const T* __restrict__ x, const T* __restrict__ re
   }
 }
 
-// The same with 16-byte accesses; a thread keeps its first RN_HELD pieces of the row in registers.
-#define RN_HELD 4
-template <typename T, bool ADD>
+// The same with 16-byte accesses; a thread keeps its first HELD pieces of the row in registers.  For few rows the kernel is its chain
+// of waits: all of a thread's pieces, the residual's and the weight's are asked for at once, before each piece was waited for by itself and
+// the weight behind the sum (before / now, alone and with the residual: 4 rows of 2,048 in 32-bit 2.72 and 2.82 us / 2.29 and 2.36, 4
+// of 4,096 in bfloat16 2.98 and 3.24 / 2.59 and 2.70).  Many rows are bound by memory (4,096 of 4,096 13.4 and 20.3 / 11.9 and 20.4; 134 MB
+// with the residual, 6.6 TB/s with its share in the caches).
+template <typename T, bool ADD, int HELD>
 __global__ __launch_bounds__(256) void rmsnorm_packed_kernel(
     const T* __restrict__ x, const T* __restrict__ residual, const void* __restrict__ w, int w_f32,
     T* __restrict__ stream_out, T* __restrict__ out, int hidden, float eps) {
@@ -82,14 +85,34 @@ __global__ __launch_bounds__(256) void rmsnorm_packed_kernel(
   __shared__ float red[16];
   const size_t base = (size_t)blockIdx.x * hidden;
   const int pieces = hidden / N;
-  float held[RN_HELD][N];
+  struct Weights { unsigned word[8]; };  // N weights of the storage type in the first four, or N floats
+  auto weights = [&](int piece) {
+    const char* from = (const char*)w + (size_t)piece * (w_f32 ? N * 4 : 16);
+    const uint4 a = *(const uint4*)from;
+    uint4 b = {};  // (a copy of `a` here would be waited for)
+    if (N == 8 && w_f32) b = *(const uint4*)(from + 16);
+    return Weights{{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}};
+  };
+  auto weight = [&](const Weights& v, int j) {
+    if (N == 4) return __uint_as_float(v.word[j]);
+    const unsigned two = v.word[j / 2];
+    return __uint_as_float(w_f32 ? v.word[j] : (j & 1 ? two & 0xffff0000u : two << 16));
+  };
+  Pack<T> xp[HELD], rp[HELD];
+  Weights wp[HELD];
+#pragma unroll
+  for (int c = 0; c < HELD; ++c) {  // (behind the row's end: its last piece again, so that no branch stands between the loads)
+    const size_t at = base + (size_t)min((int)threadIdx.x + c * 256, pieces - 1) * N;
+    xp[c].load(x + at);
+    if (ADD) rp[c].load(residual + at);
+  }
+#pragma unroll
+  for (int c = 0; c < HELD; ++c) wp[c] = weights(min((int)threadIdx.x + c * 256, pieces - 1));
+  float held[HELD][N];
   float ss = 0.f;
-  auto take = [&](int piece, float (&v)[N]) {
-    Pack<T> a;
-    a.load(x + base + (size_t)piece * N);
+  auto take = [&](int piece, const Pack<T>& a, const Pack<T>& r, float (&v)[N]) {
     if (ADD) {
-      Pack<T> r, s;
-      r.load(residual + base + (size_t)piece * N);
+      Pack<T> s;
 #pragma unroll
       for (int j = 0; j < N; ++j) {
         v[j] = round_to<T>(to_f32<T>(a.v[j]) + to_f32<T>(r.v[j]));
@@ -104,58 +127,55 @@ __global__ __launch_bounds__(256) void rmsnorm_packed_kernel(
     for (int j = 0; j < N; ++j) ss += v[j] * v[j];
   };
 #pragma unroll
-  for (int c = 0; c < RN_HELD; ++c) {
+  for (int c = 0; c < HELD; ++c) {
     const int piece = threadIdx.x + c * 256;
-    if (piece < pieces) take(piece, held[c]);
+    if (piece < pieces) take(piece, xp[c], rp[c], held[c]);
   }
-  for (int piece = threadIdx.x + RN_HELD * 256; piece < pieces; piece += 256) {
+  for (int piece = threadIdx.x + HELD * 256; piece < pieces; piece += 256) {
+    Pack<T> a, r;
     float v[N];
-    take(piece, v);
+    a.load(x + base + (size_t)piece * N);
+    if (ADD) r.load(residual + base + (size_t)piece * N);
+    take(piece, a, r, v);
   }
   ss = block_sum(ss, red);
   const float rstd = 1.0f / sqrtf(ss / (float)hidden + eps);
-  auto give = [&](int piece, const float (&v)[N]) {
+  auto give = [&](int piece, const Weights& wv, const float (&v)[N]) {
     Pack<T> o;
-    float wf[N];
-    if (w_f32) {
 #pragma unroll
-      for (int j = 0; j < N; ++j) wf[j] = ((const float*)w)[(size_t)piece * N + j];
-    } else {
-      Pack<T> wp;
-      wp.load((const T*)w + (size_t)piece * N);
-#pragma unroll
-      for (int j = 0; j < N; ++j) wf[j] = to_f32<T>(wp.v[j]);
-    }
-#pragma unroll
-    for (int j = 0; j < N; ++j) o.v[j] = from_f32<T>(wf[j] * round_to<T>(v[j] * rstd));
+    for (int j = 0; j < N; ++j) o.v[j] = from_f32<T>(weight(wv, j) * round_to<T>(v[j] * rstd));
     o.store(out + base + (size_t)piece * N);
   };
 #pragma unroll
-  for (int c = 0; c < RN_HELD; ++c) {
+  for (int c = 0; c < HELD; ++c) {
     const int piece = threadIdx.x + c * 256;
-    if (piece < pieces) give(piece, held[c]);
+    if (piece < pieces) give(piece, wp[c], held[c]);
   }
-  for (int piece = threadIdx.x + RN_HELD * 256; piece < pieces; piece += 256) {
+  for (int piece = threadIdx.x + HELD * 256; piece < pieces; piece += 256) {
     Pack<T> a;
     a.load((ADD ? stream_out : x) + base + (size_t)piece * N);  // a thread reads back what it wrote
     float v[N];
 #pragma unroll
     for (int j = 0; j < N; ++j) v[j] = to_f32<T>(a.v[j]);
-    give(piece, v);
+    give(piece, weights(piece), v);
   }
 }
 
 template <typename T, bool ADD>
 static void launch_rmsnorm(const void* x, const void* residual, const void* w, int w_f32, void* stream_out,
                            void* out, int rows, int hidden, float eps, hipStream_t stream) {
-  const bool packed = hidden % Pack<T>::N == 0 && aligned16(x) && aligned16(out) && aligned16(w) &&
+  constexpr int N = Pack<T>::N;
+  const bool packed = hidden % N == 0 && aligned16(x) && aligned16(out) && aligned16(w) &&
                       (!ADD || (aligned16(residual) && aligned16(stream_out)));
-  if (packed)
-    hipLaunchKernelGGL((rmsnorm_packed_kernel<T, ADD>), dim3(rows), dim3(256), 0, stream, (const T*)x,
-                       (const T*)residual, w, w_f32, (T*)stream_out, (T*)out, hidden, eps);
-  else
+  if (packed) {
+    // as many pieces as a row has: pieces that are held but not there would be asked for all the same
+    auto kernel = hidden <= 256 * N ? rmsnorm_packed_kernel<T, ADD, 1> : (hidden <= 512 * N ? rmsnorm_packed_kernel<T, ADD, 2> : rmsnorm_packed_kernel<T, ADD, 4>);
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, stream, (const T*)x, (const T*)residual, w, sizeof(T) == 4 ? 1 : w_f32, (T*)stream_out,
+                       (T*)out, hidden, eps);
+  } else {
     hipLaunchKernelGGL((rmsnorm_kernel<T, ADD>), dim3(rows), dim3(256), 0, stream, (const T*)x,
                        (const T*)residual, w, w_f32, (T*)stream_out, (T*)out, hidden, eps);
+  }
 }
 
 TK_API int tk_rmsnorm(int dt, const void* x, const void* w, int w_f32, void* out, int rows,
