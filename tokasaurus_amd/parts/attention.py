@@ -73,7 +73,8 @@ def attention_plan(ctx: StepContext, group: int, nkv: int, head_dim: int, page_s
         small = [r for r, n in enumerate(q_lens) if 0 < n * group <= 16]
         large = [r for r, n in enumerate(q_lens) if n * group > 16]
         static = bool(ctx.extras.get("static"))
-        # launches are chosen for the bound the step was planned for, not for the lengths in it
+        # launches are chosen for the bound the step was planned for, not for the lengths in it (but for decoded rows beside prompts,
+        # which no recorded step holds: they are cut by their own lengths)
         bound = max(int(ctx.extras.get("kv_bound", 0)), ctx.max_kv_len)
         lists: list[tuple[list[int], list[int], list[int] | None, int, int, int, int, int]] = []
         if small:
