@@ -40,7 +40,7 @@ def test_sizes(m, nk):
 @pytest.mark.parametrize("m", [1, 7, 8, 9])
 @pytest.mark.parametrize("nk", [(1, 256), (8, 288), (20, 4096), (2047, 320), (2048, 2080), (2049, 256)])
 def test_few_rows_by_halves_of_k(m, nk):
-    """Weights of few enough rows for 8 a workgroup: K's second half beside the first, with blocks left over in each, and the sizes around."""
+    """Weights of few enough rows for 8 a workgroup: neighbouring blocks of K beside each other, with blocks left over, and the sizes around."""
     n, k = nk
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
     a, w = torch.randn((m, k + 4), generator=g, device="cuda")[:, 4:], torch.randn((n, k), generator=g, device="cuda")
@@ -94,5 +94,16 @@ def test_largest_tiles_straight_to_local_memory():
 @pytest.mark.parametrize("m", [1, 3, 4, 8])
 @pytest.mark.parametrize("nk", [(20, 8192), (9, 8224), (2050, 8192), (24, 16384)])
 def test_few_rows_over_long_inner_sizes(m, nk):
-    """Where the second half of K, or the next elements, take the matrix core's unused half."""
+    """Where a wavefront has several sets of loads, and workgroups begin at different ones."""
     test_sizes(m, nk)
+
+
+@pytest.mark.parametrize("nk", [(2048, 8192), (1031, 8192), (77, 16384), (300, 9248), (2048, 2048), (70, 256)])
+def test_a_rows_bits_do_not_depend_on_how_many_rows_there_are(nk):
+    """Steps of up to 8 rows are recorded with 1, 2, 4 or 8: a row alone, among 3 and among the recorded sizes is the same sums in one order."""
+    n, k = nk
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    a, w = torch.randn((8, k), generator=g, device="cuda"), torch.randn((n, k), generator=g, device="cuda")
+    all_rows = ops.gemm_generic(a, w)
+    for m in range(1, 8):
+        assert torch.equal(ops.gemm_generic(a[:m], w), all_rows[:m]), m

@@ -66,13 +66,16 @@ __device__ __forceinline__ void gf_store(const GemmF32Args& a, f4 v, int token, 
 #define GF_UNROLL 4  // blocks of 16 elements a set of loads
 
 // HALVES (up to 8 tokens, K a multiple of 32): a workgroup has 8 weight rows, and the unused half of the matrix core's rows and of its
-// columns takes other elements of K (the blocks of results off the diagonal are not used), so that a weight of few rows gives
-// every compute unit a workgroup.  NEXT: the next 16 elements, so that a load takes whole lines of 128 bytes; else the second half
-// of K, for up to 3 tokens and long rows.  us second half / next: 4 tokens 2,048 x 2,048 6.4 / 5.9, 2,048 x 8,192 20.3 / 20.3, 8 tokens 7.4 / 6.5,
-// 23.4 / 22.1, 1 token 5.8 / 5.4, 16.5 / 19.4 (rows 32 KB apart begin in one of the memory's channels).  4 tokens, us by rows of 16 / of 8, weights from memory: 2,048 x 2,048 8.6 / 6.9, 2,048 x 8,192 26.4 / 17.5
-// (3.8 TB/s), 3,072 x 2,048 8.8 / 9.6, 16,384 x 2,048 26.8 / 31.2.  Each chain of sums is half as long: error 1.2e-7 / 1.0e-7 of the norm
-// over 2,048 elements, 1.6e-7 / 1.3e-7 over 8,192.
-template <bool HALVES, bool NEXT>
+// columns takes the next 16 elements of K (the blocks of results off the diagonal are not used), so that a weight of few rows gives
+// every compute unit a workgroup and a load takes whole lines of 128 bytes.  4 tokens, us by rows of 16 / of 8, weights from memory: 2,048 x
+// 2,048 8.6 / 6.9, 2,048 x 8,192 26.4 / 17.5, 3,072 x 2,048 8.8 / 9.6, 16,384 x 2,048 26.8 / 31.2 (these of 8 with the other half's elements
+// a half of K on, 1 to 8 tokens at 2,048 x 4,096 9.8 to 12.4, now 8.4 to 10.3).  Each chain of sums is half as long: error 1.2e-7 / 1.0e-7 of
+// the norm over 2,048 elements, 1.6e-7 / 1.3e-7 over 8,192.
+// A wavefront's walk begins at a set that the workgroup's number gives, those of one die at different ones: begun at the first by
+// all, rows of 32 and 64 KB keep to few of the memory's channels (us together / apart: 2,048 x 8,192 19.4 / 15.0 at 1 token, 19.4 / 15.4 at 4,
+// 2,048 x 16,384 29.9 / 24.0 and 30.2 / 26.5, 2,048 x 11,008 21.4 / 19.9 and 22.0 / 20.6, else within 2 %).  One order for all rows up to 8, whatever
+// their number: a step of 3 rows is recorded with 4.
+template <bool HALVES>
 __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a, int KS, int share, int spare) {
   extern __shared__ __align__(16) f4 sums[];  // [wavefronts - 1][64]
   // every argument that a first load needs, in one trip
@@ -82,8 +85,8 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a, int KS
   const int r = lane & 15, q = lane >> 4;
   constexpr int ROWS = HALVES ? 8 : 16;
   const int n0 = blockIdx.x * ROWS, own = HALVES ? r & 7 : r;
-  const int from = HALVES ? (r >> 3) * (NEXT ? 16 : a.K / 2) : 0;
-  constexpr int STEP = HALVES && NEXT ? 32 : 16;  // elements of K a block and its partner are on
+  const int from = HALVES ? (r >> 3) * 16 : 0;
+  constexpr int STEP = HALVES ? 32 : 16;  // elements of K a block and its partner are on
   const int blocks = HALVES ? a.K >> 5 : (a.K + 15) >> 4;
   const int b0 = kw * share + min(kw, spare), b1 = b0 + share + (kw < spare ? 1 : 0);
   const float* wp = a.W + (size_t)min(n0 + own, a.N - 1) * a.K + from + 4 * q;
@@ -98,8 +101,8 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a, int KS
 #define GF_LOAD(set, b)                                                                             \
   do {                                                                                              \
     _Pragma("unroll") for (int u = 0; u < GF_UNROLL; ++u) {                                         \
-      w[set][u] = *(const f4*)(wp + (size_t)((b) + u) * STEP);                                      \
-      x[set][u] = *(const f4*)(ap + (size_t)((b) + u) * STEP);                                      \
+      w[set][u] = *(const f4*)(wp + (size_t)(place(b) + u) * STEP);                                 \
+      x[set][u] = *(const f4*)(ap + (size_t)(place(b) + u) * STEP);                                 \
     }                                                                                               \
     __builtin_amdgcn_sched_barrier(0);                                                              \
   } while (0)
@@ -108,6 +111,8 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a, int KS
       acc[u][s] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[set][u][s], x[set][u][s], acc[u][s], 0, 0, 0)
   const int exact = HALVES || (a.K & 15) == 0 ? b1 : min(b1, blocks - 1);  // blocks up to here lie inside K whole
   const int sets = max(exact - b0, 0) / GF_UNROLL;
+  const int turn = HALVES && sets > 0 ? (int)((blockIdx.x >> 3) % (unsigned)sets) * GF_UNROLL : 0;
+  auto place = [&](int at) { return !HALVES ? at : (at + turn < b0 + sets * GF_UNROLL ? at + turn : at + turn - sets * GF_UNROLL); };
   int b = b0;
   if (sets > 0) {
     GF_LOAD(0, b);
@@ -415,7 +420,7 @@ TK_API int tk_gemm_f32(const void* A, int lda, const void* W, void* C, int ldc, 
     // rows of 8 where rows of 16 leave compute units without a workgroup
     const bool halves = M <= 8 && K % 32 == 0 && K >= 256 && N <= GF_HALVES_ROWS;
     const int blocks = halves ? K / 32 : (K + 15) / 16;
-    auto few = !halves ? gemm_f32_few_kernel<false, false> : (M >= 4 || K < 8192 ? gemm_f32_few_kernel<true, true> : gemm_f32_few_kernel<true, false>);
+    auto few = halves ? gemm_f32_few_kernel<true> : gemm_f32_few_kernel<false>;
     const int rows = halves ? 8 : 16;
     hipLaunchKernelGGL(few, dim3((N + rows - 1) / rows), dim3(64 * KS), (KS - 1) * 64 * sizeof(f4), stream, a, KS, blocks / KS, blocks % KS);
     TK_CHECK_LAUNCH("gemm_f32");
