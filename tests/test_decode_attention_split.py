@@ -23,3 +23,26 @@ def test_even_splits(head_dim, lengths):
     whole = ops.attention_split(max(lengths), len(lengths), 8, head_dim)
     assert split % (32 * waves) == 0 and 1 <= waves <= ops.attention_max_waves(head_dim, 1)
     assert (split, waves) == whole or (512 <= split < whole[0] and waves == 4)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("nkv", [1, 8])
+@pytest.mark.parametrize("lengths", [[40] * 63 + [28000], [64] * 127 + [24000], [64] * 255 + [16000], [1] * 999 + [262143], [1] * 999 + [31000], [500] * 63 + [8000],
+                                     [100] * 3 + [16000], [300] * 100 + [3000], [100, 131072]])
+def test_even_splits_have_a_bounded_grid(head_dim, nkv, lengths):
+    """A launch has a workgroup and partial results for every split of the longest request, times the requests: no more than a bound, or
+    than the planned cut has."""
+    count = lambda split: len(lengths) * nkv * -(-max(lengths) // split)  # noqa: E731
+    split, _ = ops.attention_even_split(lengths, nkv, head_dim)
+    planned, _ = ops.attention_split(max(lengths), len(lengths), nkv, head_dim)
+    assert split <= planned and count(split) <= max(count(planned), ops.ATTENTION_EVEN_WORKGROUPS)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_even_splits_where_they_are_ahead(head_dim):
+    """Not where planned workgroups of rising lengths fill one round or several, nor where they are few."""
+    even = lambda lengths: ops.attention_even_split(lengths, 8, head_dim) != ops.attention_split(max(lengths), len(lengths), 8, head_dim)  # noqa: E731
+    for lengths in ([1000 + 466 * i for i in range(16)], [200 + 122 * i for i in range(32)], [100 + 9 * i for i in range(100)], [100] * 3 + [16000], [2000] * 60):
+        assert not even(lengths)
+    for lengths in ([250 + 39 * i for i in range(45)], [1500] * 20 + [6000] * 4, [500] * 63 + [8000], [300] * 10 + [4000] * 2):
+        assert even(lengths)
