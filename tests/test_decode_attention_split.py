@@ -46,3 +46,11 @@ def test_even_splits_where_they_are_ahead(head_dim):
         assert not even(lengths)
     for lengths in ([250 + 39 * i for i in range(45)], [1500] * 20 + [6000] * 4, [500] * 63 + [8000], [300] * 10 + [4000] * 2):
         assert even(lengths)
+
+
+@pytest.mark.parametrize("group,nkv,requests,keys,waves", [(8, 8, 1, 8192, 8), (5, 8, 4, 32768, 8), (7, 4, 1, 32768, 8), (8, 1, 16, 8192, 8), (4, 8, 1, 8192, 4), (4, 8, 16, 8192, 4),
+                                                           (3, 8, 45, 2000, 4), (4, 8, 64, 8192, 8), (4, 8, 2, 131072, 8), (8, 8, 1, 1024, 4)])
+def test_wavefronts_at_head_sizes_above_64(group, nkv, requests, keys, waves):
+    """Eight a workgroup for many query heads a kv head and for long splits, four for few heads."""
+    split, got = ops.attention_split(keys, requests, nkv, 128, group)
+    assert got == waves and split % (32 * waves) == 0

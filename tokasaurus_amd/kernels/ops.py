@@ -599,20 +599,25 @@ def attention_max_waves(head_dim: int, row_tiles: int) -> int:
     return 4 if row_tiles == 2 else (16 if head_dim <= 64 else 8)
 
 
-def attention_split(max_kv_len: int, n_tiles: int, nkv: int, head_dim: int = 64) -> tuple[int, int]:
-    """(keys per split, wavefronts per workgroup) for tiles of one row tile (decode).
+def attention_split(max_kv_len: int, n_tiles: int, nkv: int, head_dim: int = 64, group: int | None = None) -> tuple[int, int]:
+    """(keys per split, wavefronts per workgroup) for tiles of one row tile (decode) of ``group`` query heads a kv head (None: not known,
+    four wavefronts at most at head sizes above 64).
     The keys of a tile are cut so that there are about 256 workgroups (one a compute
     unit) or more, into splits of 8 192 keys at most; the wavefronts of a workgroup, which
-    adds their results itself, take 64 to 512 keys each, about two thousand wavefronts in all
+    adds their results itself, take 64 to 512 keys each, at head size 64 about two thousand wavefronts in all
     or more.
     Measured best on an MI355X at 8192 keys, with the cache read from memory:
     64 keys x 8 wavefronts x 16 splits at batch 1, 256 x 8 x 4 at batch 8,
     512 x 16 x 1 at batch 64.  Handing a split over costs 3 us and more, so a split has 128 keys or more, four wavefronts of 32
     of them, and beyond eight splits 256 (us a layer of 8 kv heads at one request, planned for 1,024: splits of 64 keys for one
     wavefront / of 128 for four, head size 64 9.4 / 6.3 at 500 keys, 10.5 / 6.8 at 1,000, head size 128 16.4 / 9.0; planned for 2,048: 128
-    for two / 256 for four 8.1 / 7.2 at 1,100, 9.3 / 7.7 at 2,000; two requests of 1,000 keys 12.8 / 8.1).  At head sizes above 64 a
-    compute unit has room for eight wavefronts: two workgroups of four hide each other's ends (eight / four wavefronts,
-    16 requests of 1,500 keys 26.2 / 25.3, 64 of 47 to 380 19.7 / 17.0)."""
+    for two / 256 for four 8.1 / 7.2 at 1,100, 9.3 / 7.7 at 2,000; two requests of 1,000 keys 12.8 / 8.1).  At head sizes above 64
+    a compute unit has room for eight wavefronts.  Eight of a workgroup are ahead of four where a kv head has more than four query heads (us at head
+    size 128, four / eight: 40 on 8 at one request of 8,192 keys 18.4 / 16.2, at 4 of 32,768 98 / 95, at 16 of 1,500 25.6 / 25.0, of 8,192 94 / 101; 28 on 4 14.5 / 12.6 and 55 / 55; 8
+    on 1 14.2 / 12.3 and 32.7 / 32.0; head size 80, 32 on 4, 12.9 / 10.7 and 39.4 / 36.7), four where it has up to four (32 on 8 16.4 / 16.5 at one request of
+    8,192, 33.3 / 34.7 of 32,768, 20.5 / 21.1 and 52 / 56 at two, 93 / 100 at 16 of 8,192, 24.6 / 25.2 of 1,500, 178 / 195 at 64 of 4,096; 16 on 4 12.1 / 12.3 and 31.0 / 32.1 at one, 22.0 /
+    24.3 at two of 16,384), but for splits of 8,192 keys, where eight are again (32 on 8 8 requests of 32,768 192 / 180, 64 of 8,192 400 / 361, 2 of 131,072 196 /
+    189, 4 of 131,072 388 / 441)."""
     base = max(n_tiles * nkv, 1)
     kv = max(max_kv_len, 1)
     splits = max(1, min(16, -(-256 // base), -(-kv // 128), max(8, kv // 256)))
@@ -622,8 +627,9 @@ def attention_split(max_kv_len: int, n_tiles: int, nkv: int, head_dim: int = 64)
     # 8 192 keys; 255 of 512 beside one of 32 768: 401 / 114 us; requests of one length lose nothing)
     raw = min(-(-kv // splits), 8192 if base < 1024 else 2048)
     per_wave = min(512, max(32 if raw <= 128 else 64, kv * base // 2048))
+    most = 4 if head_dim > 64 and (group is None or (group <= 4 and raw < 8192)) else attention_max_waves(head_dim, 1)
     waves = 1
-    while waves * 2 <= min(attention_max_waves(head_dim, 1), raw // per_wave, 16 if head_dim <= 64 else 4):
+    while waves * 2 <= min(most, raw // per_wave):
         waves *= 2
     step = 32 * waves
     return -(-raw // step) * step, waves
@@ -633,7 +639,7 @@ def attention_split(max_kv_len: int, n_tiles: int, nkv: int, head_dim: int = 64)
 ATTENTION_EVEN_WORKGROUPS = 4096
 
 
-def attention_even_split(lengths: list[int], nkv: int, head_dim: int) -> tuple[int, int]:
+def attention_even_split(lengths: list[int], nkv: int, head_dim: int, group: int | None = None) -> tuple[int, int]:
     """The same for decoded tokens beside prompts, in a step that is not recorded: their lengths are known, and where a workgroup's
     longest walk is over a compute unit's share of the keys by a fifth the keys are cut shorter, so that the workgroups (two a unit) get as many
     each.  That pays where some units have two of the planned workgroups and others one, or where few requests are long.  us a layer
@@ -644,7 +650,7 @@ def attention_even_split(lengths: list[int], nkv: int, head_dim: int) -> tuple[i
     fill several (100 of 100 to 1,000 28.4 / 29.3 and 49 / 53), or are fewer than half the units (3 of 100 and one of 16,000 19.3 / 22.9 and 30.9 / 30.4).
     The grid and the partial results are as many as the longest request has splits, for every request: they are bounded (63 of 40 and one of 28,000, by
     512 keys 28,160 workgroups of which 944 have keys; 127 of 64 and one of 24,000 planned / by 512 keys 55 / 75 and 76 / 117)."""
-    split, waves = attention_split(max(lengths), len(lengths), nkv, head_dim)
+    split, waves = attention_split(max(lengths), len(lengths), nkv, head_dim, group)
     longest, total = max(lengths), sum(lengths)
     planned = sum(-(-n // split) for n in lengths) * nkv
     if not (min(split, longest) * 256 * 5 >= total * nkv * 6 and planned >= 128 and (planned > 256 or longest * len(lengths) * 5 > total * 11)):

@@ -81,10 +81,10 @@ def attention_plan(ctx: StepContext, group: int, nkv: int, head_dim: int, page_s
             req, row0, _ = ops.attention_tiles(q_lens, group, 1, small)
             if large and not static:
                 lengths = [ctx.host_kv_len[r] for r in small]
-                split, waves = ops.attention_even_split(lengths, nkv, head_dim)
+                split, waves = ops.attention_even_split(lengths, nkv, head_dim, group)
                 lists.append((req, row0, None, 1, split, waves, 0, max(lengths)))
             else:
-                split, waves = ops.attention_split(bound, len(req), nkv, head_dim)
+                split, waves = ops.attention_split(bound, len(req), nkv, head_dim, group)
                 lists.append((req, row0, None, 1, split, waves, 0, bound))
         # Portions that come after a past several times their own length walk far more keys a row than
         # whole prompts do: they are planned apart, or one of them among whole prompts would take a
