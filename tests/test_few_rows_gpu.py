@@ -39,6 +39,21 @@ def test_norm_in_front(m, parts):
     assert ((got.double() - s * up).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("weight_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [1, 3, 9, 200, 201])
+@pytest.mark.parametrize("begin", [0, 1, 2])
+def test_weights_of_the_norm_behind_that_begin_and_end_anywhere(weight_dtype, n, begin):
+    """Weights that start 0, 1 and 2 elements behind a multiple of 16 bytes and are no whole words: the emitted rows are x w, rounded once,
+    and the partial sums those of the rounded rows (16 squares of one sign: 16 roundings of 2^-24)."""
+    gen = torch.Generator(device="cuda").manual_seed(n + begin)
+    m, k = 3, 96
+    a, w, res = (torch.randn(s, generator=gen, device="cuda").bfloat16() for s in ((m, k), (n, k), (m, n)))
+    weight = (1 + torch.randn((n + begin,), generator=gen, device="cuda")).to(weight_dtype)[begin:]
+    x, pre = ops.gemm_skinny_bf16(a, w, residual=res, emit_weight=weight)
+    assert torch.equal(pre.scaled, (weight.float() * x.float()).bfloat16())
+    assert torch.allclose(pre.sumsq.sum(1), x.float().pow(2).sum(1), rtol=16 * 2.0 ** -24 + n * 2.0 ** -24, atol=0)
+
+
 @pytest.mark.parametrize("m", [1, 3, 8, 9])
 @pytest.mark.parametrize("k", [64, 448, 576, 2048])
 def test_rotation_behind_a_folded_inner_size(m, k):

@@ -195,20 +195,24 @@ __device__ __forceinline__ void row_scales(const GemmArgs& a, float* scale, int 
 // The residual epilogue's extra outputs for the norm that follows: x * w rounded once,
 // and the sum of x^2 over this tile's columns.  All 64 lanes of a wavefront call this
 // together; lanes (token, qq = 0..3) share a token.
-// Its weights of outputs n .. n + 3, asked for without a branch on their type: the 4 bytes that hold a weight, and the weight.
-__device__ __forceinline__ void emit_ask(const GemmArgs& a, int n, unsigned (&w)[4]) {
+// Its weights of outputs n .. n + 3, asked for without a branch on their type and no byte beside them: the lower and the upper two
+// bytes of a 32-bit one, or one of 16 bits twice.
+struct EmitWeights {
+  unsigned lower[4], upper[4];
+};
+__device__ __forceinline__ void emit_ask(const GemmArgs& a, int n, EmitWeights& w) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const char* at = (const char*)a.emit_w + (size_t)min(n + j, a.N - 1) * (a.emit_w_f32 ? 4 : 2);
-    w[j] = *(const unsigned*)(at - ((uintptr_t)at & 3));
+    const unsigned short* at = (const unsigned short*)((const char*)a.emit_w + (size_t)min(n + j, a.N - 1) * (a.emit_w_f32 ? 4 : 2));
+    w.lower[j] = at[0];
+    w.upper[j] = at[a.emit_w_f32 ? 1 : 0];
   }
 }
-__device__ __forceinline__ float emit_weight(const GemmArgs& a, int n, int j, unsigned w) {
-  const bool upper = (((uintptr_t)a.emit_w + (size_t)min(n + j, a.N - 1) * 2) & 2) != 0;
-  return __uint_as_float(a.emit_w_f32 ? w : (upper ? w & 0xffff0000u : w << 16));
+__device__ __forceinline__ float emit_weight(const GemmArgs& a, const EmitWeights& w, int j) {
+  return __uint_as_float(w.upper[j] << 16 | (a.emit_w_f32 ? w.lower[j] : 0u));
 }
 
-__device__ __forceinline__ void emit_for_norm(const GemmArgs& a, const float (&x)[4], const unsigned (&w)[4], bool live, int token,
+__device__ __forceinline__ void emit_for_norm(const GemmArgs& a, const float (&x)[4], const EmitWeights& w, bool live, int token,
                                               int n, int part, int lane) {
   float ss = 0.f;
   if (live) {
@@ -218,7 +222,7 @@ __device__ __forceinline__ void emit_for_norm(const GemmArgs& a, const float (&x
     for (int j = 0; j < 4; ++j) {
       const float xr = n + j < a.N ? round_to<bf16_t>(x[j]) : 0.f;
       ss = fmaf(xr, xr, ss);
-      pk.h[j] = __float2bfloat16(emit_weight(a, n, j, w[j]) * xr);
+      pk.h[j] = __float2bfloat16(emit_weight(a, w, j) * xr);
     }
     if (n + 3 < a.N && (a.ld_emit & 3) == 0) {
       *(uint2*)dst = pk.u;
@@ -377,7 +381,7 @@ __global__ __launch_bounds__(sk_max_waves(NT) * 64) void gemm_skinny_kernel(Gemm
   const int l0 = tid & 63, mb0 = wave % MB, t0 = wave / MB;
   RopeOperands rope_pre = {};
   bf16_t res_pre[4] = {};
-  unsigned emit_pre[4] = {};
+  EmitWeights emit_pre = {};
   f32x4_t parts_pre = {0.f, 0.f, 0.f, 0.f};
   if (NORM) parts_pre = *row_parts(a, wave, lane);
   if (EPI == EPI_ROPE) rope_ask(a, mb0 * 16 + (l0 & 15), rope_pre);
