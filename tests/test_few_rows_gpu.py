@@ -54,6 +54,19 @@ def test_weights_of_the_norm_behind_that_begin_and_end_anywhere(weight_dtype, n,
     assert torch.allclose(pre.sumsq.sum(1), x.float().pow(2).sum(1), rtol=16 * 2.0 ** -24 + n * 2.0 ** -24, atol=0)
 
 
+@pytest.mark.parametrize("begin", [1, 2, 3])
+def test_rows_for_the_norm_behind_that_begin_anywhere(begin, monkeypatch):
+    """Memory for x w that starts 2, 4 and 6 bytes behind a multiple of 8: the same values."""
+    gen = torch.Generator(device="cuda").manual_seed(begin)
+    a, w, res, weight = (torch.randn(s, generator=gen, device="cuda").bfloat16() for s in ((3, 96), (200, 96), (3, 200), (200,)))
+    want = ops.gemm_skinny_bf16(a, w, residual=res, emit_weight=weight)
+    made = ops.Prenorm
+    monkeypatch.setattr(ops, "Prenorm", lambda scaled, sumsq: made(torch.empty((603,), dtype=scaled.dtype, device="cuda")[begin:][:600].view(3, 200), sumsq))
+    got = ops.gemm_skinny_bf16(a, w, residual=res, emit_weight=weight)
+    assert got[1].scaled.data_ptr() % 8 == 2 * begin
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1].scaled, want[1].scaled) and torch.equal(got[1].sumsq, want[1].sumsq)
+
+
 @pytest.mark.parametrize("m", [1, 3, 8, 9])
 @pytest.mark.parametrize("k", [64, 448, 576, 2048])
 def test_rotation_behind_a_folded_inner_size(m, k):

@@ -224,7 +224,7 @@ __device__ __forceinline__ void emit_for_norm(const GemmArgs& a, const float (&x
       ss = fmaf(xr, xr, ss);
       pk.h[j] = __float2bfloat16(emit_weight(a, w, j) * xr);
     }
-    if (n + 3 < a.N && (a.ld_emit & 3) == 0) {
+    if (n + 3 < a.N && ((a.ld_emit & 3) | ((uintptr_t)a.emit_scaled & 7)) == 0) {
       *(uint2*)dst = pk.u;
     } else {
 #pragma unroll
@@ -1017,7 +1017,7 @@ TK_API int tk_gemm_skinny_bf16(const void* A, int lda, const void* W, void* C, i
   }
   TK_REQUIRE(!norm || a.parts_in > 0, "gemm_skinny: a norm in front needs its partial sums");
   TK_REQUIRE(!(norm && epi == EPI_RESIDUAL), "gemm_skinny: a norm in front cannot be combined with a residual behind");
-  TK_REQUIRE(a.emit_w == nullptr || (epi == EPI_RESIDUAL && a.emit_scaled && a.emit_sumsq && a.ld_emit >= N && ((uintptr_t)a.emit_scaled & 7) == 0),
+  TK_REQUIRE(a.emit_w == nullptr || (epi == EPI_RESIDUAL && a.emit_scaled && a.emit_sumsq && a.ld_emit >= N),
              "gemm_skinny: outputs for a following norm go with the residual epilogue and need their buffers");
   if (epi == EPI_ROPE) {
     TK_REQUIRE(extra && a.positions && a.token_req && a.block_table && a.kcache && a.vcache,
