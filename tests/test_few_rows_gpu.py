@@ -54,6 +54,26 @@ def test_weights_of_the_norm_behind_that_begin_and_end_anywhere(weight_dtype, n,
     assert torch.allclose(pre.sumsq.sum(1), x.float().pow(2).sum(1), rtol=16 * 2.0 ** -24 + n * 2.0 ** -24, atol=0)
 
 
+@pytest.mark.parametrize("m", [1, 2])
+def test_tiles_of_8_for_one_and_two_rows_where_they_are_folded(m):
+    """4,096 outputs fill the compute units with tiles of 16 as well: an inner size of no multiple of 64, two tiles a wavefront, and a product that
+    is asked not to fold K take those; and the partial sums are as many as the caller is told."""
+    from tokasaurus_amd.kernels.library import load
+
+    parts = load("mfma").tk_gemm_skinny_parts
+    assert parts(m, 4096, 2048, 0, 0, 1) == 512
+    assert parts(m, 4096, 2080, 0, 0, 1) == parts(m, 4096, 2048, 2, 0, 1) == parts(m, 4096, 2048, 0, 0, 0) == 256
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    for k in (64, 96):
+        a, w, res, weight = (torch.randn(s, generator=gen, device="cuda").bfloat16() for s in ((m, k), (4096, k), (m, 4096), (4096,)))
+        for kw in ({}, {"tiles": 2}, {"fold": False}):
+            x, pre = ops.gemm_skinny_bf16(a, w, residual=res, emit_weight=weight, **kw)
+            want = (a.double() @ w.double().T).bfloat16().double() + res.double()
+            assert ((x.double() - want).abs() <= 2.0 ** -7 * (want.abs() + (a.double().abs() @ w.double().abs().T))).all()
+            assert torch.equal(pre.scaled, (weight.float() * x.float()).bfloat16())
+            assert torch.allclose(pre.sumsq.sum(1), x.float().pow(2).sum(1), rtol=4096 * 2.0 ** -24, atol=0)
+
+
 @pytest.mark.parametrize("begin", [1, 2, 3])
 def test_rows_for_the_norm_behind_that_begin_anywhere(begin, monkeypatch):
     """Memory for x w that starts 2, 4 and 6 bytes behind a multiple of 8: the same values."""

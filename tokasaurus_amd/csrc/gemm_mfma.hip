@@ -947,12 +947,13 @@ static int compute_units() {
 // core, fewer make more workgroups.  A workgroup streams its rows over all of K, so the time is
 // that of the rounds of workgroups the compute units take, times the rows of each: the fewest
 // win, and among equals the larger tile (A is read once a workgroup); for one and two rows of A
-// tiles of 8, which are folded and load whole lines (16 / 8 at one row: 4,096 x 4,096 10.5 / 9.8 us,
+// tiles of 8 where they are folded and load whole lines (16 / 8 at one row: 4,096 x 4,096 10.5 / 9.8 us,
 // 4,096 x 14,336 25.9 / 24.7, 6,144 x 4,096 with the rotation 14.9 / 14.2; at 4 rows 10.8 / 10.8, 27.9 /
-// 28.1, 15.6 / 15.1; at 8 11.3 / 13.1, 31.5 / 34.0, 16.2 / 16.3).  With two rounds or more
+// 28.1, 15.6 / 15.1; at 8 11.3 / 13.1, 31.5 / 34.0, 16.2 / 16.3).  Not where they are not (at one row 4,096 x 4,128 9.8 / 11.5,
+// 4,096 x 2,080 6.2 / 7.7; gate and up 3,584 x 2,048 10.1 / 10.5, 3,073 x 1,024 6.9 / 7.4, 4,096 x 1,056 7.7 / 8.3).  With two rounds or more
 // of full tiles the rounds overlap and even out: 16 rows then (measured: smaller tiles lose).
 // With the rotation epilogue (heads > 0) a workgroup takes `th` columns of one half of a head.
-static int choose_tile_rows(int M, int N, int heads = 0, int half = 0) {
+static int choose_tile_rows(int M, int N, bool folds, int heads = 0, int half = 0) {
   if (M > 32) return 16;
   const int units = compute_units();
   int best = 16, best_cost = 0;
@@ -960,13 +961,16 @@ static int choose_tile_rows(int M, int N, int heads = 0, int half = 0) {
     const int groups = heads > 0 ? heads * ((half + th - 1) / th) : (N + th - 1) / th;
     if (th == 16 && groups >= 2 * units) return 16;
     const int cost = ((groups + units - 1) / units) * th;
-    if (th == 16 || cost < best_cost || (cost == best_cost && th == 8 && M <= 2)) { best = th; best_cost = cost; }
+    if (th == 16 || cost < best_cost || (cost == best_cost && th == 8 && M <= 2 && folds)) { best = th; best_cost = cost; }
   }
   return best;
 }
 
-TK_API int tk_gemm_skinny_parts(int M, int N, int tile_rows) {
-  const int th = tile_rows > 0 ? tile_rows : choose_tile_rows(M, N);
+// whether tiles of 8 weight rows for up to 8 rows of A have K folded (launch_folded)
+static bool folds(int K, int epi, int NT, int fold) { return fold != 0 && K % 64 == 0 && epi != EPI_SWIGLU && (NT == 1 || epi == EPI_ROPE); }
+
+TK_API int tk_gemm_skinny_parts(int M, int N, int K, int tiles, int tile_rows, int fold) {
+  const int th = tile_rows > 0 ? tile_rows : choose_tile_rows(M, N, folds(K, EPI_RESIDUAL, tiles > 0 ? tiles : 1, fold));
   return (N + th - 1) / th;
 }
 
@@ -1066,7 +1070,7 @@ TK_API int tk_gemm_skinny_bf16(const void* A, int lda, const void* W, void* C, i
     }
   } else {
     a.TH = tile_rows > 0 ? tile_rows
-                         : (epi == EPI_ROPE ? choose_tile_rows(M, N, a.nq + 2 * a.nkv, a.d / 2) : choose_tile_rows(M, N));
+                         : choose_tile_rows(M, N, folds(K, epi, NT, fold), epi == EPI_ROPE ? a.nq + 2 * a.nkv : 0, a.d / 2);
     const int th_units = (N + a.TH - 1) / a.TH;
     int groups;
     if (epi == EPI_ROPE) {
@@ -1075,8 +1079,8 @@ TK_API int tk_gemm_skinny_bf16(const void* A, int lda, const void* W, void* C, i
       groups = paired ? th_units : (th_units + NT - 1) / NT;
     }
     TK_REQUIRE(a.emit_w == nullptr || a.parts_out == th_units, "gemm_skinny: %d partial sums a row, the caller sized for %d", th_units, a.parts_out);
-    // tiles of 8 weight rows for up to 8 rows of A: both halves of K in one product
-    const bool folded = fold != 0 && a.TH == 8 && M <= 8 && (NT == 1 || epi == EPI_ROPE) && epi != EPI_SWIGLU && K % 64 == 0 && !(norm && epi == EPI_RESIDUAL);
+    // tiles of 8 weight rows for up to 8 rows of A: even and odd blocks of 32 of K in one product (a norm in front goes with no residual)
+    const bool folded = a.TH == 8 && M <= 8 && folds(K, epi, NT, fold);
     const int steps = folded ? K / 64 : K32;
     int WK = waves_k;
     if (WK <= 0) {

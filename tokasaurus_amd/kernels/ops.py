@@ -1133,7 +1133,7 @@ def gemm_skinny_bf16(
         _need(epi == EPI_RESIDUAL, "gemm_skinny: outputs for a following norm go with the residual epilogue")
         _need(emit_weight.shape == (n,) and emit_weight.is_contiguous() and emit_weight.dtype in (torch.bfloat16, torch.float32),
               "gemm_skinny: the following norm's weight must be contiguous [N], bfloat16 or float32")
-        parts = load("mfma").tk_gemm_skinny_parts(m, n, tile_rows)
+        parts = load("mfma").tk_gemm_skinny_parts(m, n, k, tiles, tile_rows, 1 if fold else 0)
         emitted = Prenorm(torch.empty((m, n), dtype=torch.bfloat16, device=a.device),
                           torch.empty((m, parts), dtype=torch.float32, device=a.device))
         extra.emit_w, extra.emit_w_f32 = emit_weight.data_ptr(), 1 if emit_weight.dtype == torch.float32 else 0
