@@ -149,3 +149,27 @@ def test_whole_pairs_and_odd_tiles_are_listed_apart(tokens, top, experts):
         assert rows == (counts[e] - 1) % ops.EXPERT_TILE + 1
         tiles.append((tile, e))
     assert sorted(tiles) == list(enumerate(group[: group[-1]]))
+
+
+def test_room_that_is_no_list_of_the_tiles_pairs_is_refused(monkeypatch):
+    """The grid of the pairs comes from how many tiles and pairs there can be: fewer pairs than half the tiles would leave tiles out."""
+    import dataclasses
+
+    for least in ("ROWS", "WIDTH", "INNER", "WALK"):
+        monkeypatch.setattr(ops, f"EXPERT_PAIRS_FROM_{least}", 0)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    tokens, experts, width, ff = 771, 3, 64, 64
+    h = torch.randn((tokens, width), generator=g, device="cuda").bfloat16()
+    gu, dn = (torch.randn(s, generator=g, device="cuda").bfloat16() for s in ((experts, 2 * ff, width), (experts, width, ff)))
+    ids = (torch.arange(tokens, dtype=torch.int32) % experts).view(tokens, 1).cuda()  # 257 rows an expert: a whole pair and an odd tile each
+    pairs = ops.expert_sort([(ids, experts)])[0]
+    assert pairs.max_tiles == 9 and pairs.runs[:3].tolist() == [6, 3, 3]
+    got = ops.expert_mix(h, gu, dn, ids, None, pairs=pairs)
+    for e in range(experts):
+        y = h[e::experts].double() @ gu[e].double().T
+        act = (torch.nn.functional.silu(y[:, :ff]) * y[:, ff:]).bfloat16().double()
+        want, size = act @ dn[e].double().T, act.abs() @ dn[e].double().abs().T
+        # gate, up, silu and their product are rounded to 8 bits in front of the sums, a row behind them
+        assert ((got[e::experts].double() - want).abs() <= 2.0 ** -6 * (size + want.abs())).all()
+    with pytest.raises(ops.KernelError, match="pairs of 9 tiles"):
+        ops.expert_mix(h, gu, dn, ids, None, pairs=dataclasses.replace(pairs, max_pairs=4))

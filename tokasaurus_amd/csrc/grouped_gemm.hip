@@ -453,12 +453,13 @@ static bool launch_by_tile(const GroupedArgs& a, int tiles, const TileRun* runs,
   if (runs) {
     const int wide_blocks = (a.N + WIDE_OUT(GLU) - 1) / WIDE_OUT(GLU);
     const int odd_blocks = (a.N + ODD_OUT(GLU) - 1) / ODD_OUT(GLU);
-    // whole pairs W and odd tiles O are 2 W + O tiles at most, and W + O pairs: W + 2 O <= 3 max_pairs - tiles + 1 (an odd tile is two items;
-    // each die's stretch is rounded up)
-    const long pairs = groups((3l * max_pairs - tiles + 1) * wide_blocks) + 2 * GS_DIES;
+    // Whole pairs W and odd tiles O: 2 W + O = `tiles` at the most, and O = `odd`, what room for (tiles + O) / 2 pairs in all was made for.
+    // An odd tile apart is two items, so there are W + 2 O = (2 W + O) / 2 + 3 O / 2 <= (tiles + 3 odd) / 2 (each die's stretch is rounded up).
+    const int odd = min(2 * max_pairs - tiles + 1, tiles);
+    const long pairs = groups((tiles + 3l * odd) / 2 * wide_blocks) + 2 * GS_DIES;
     static_assert(PairShape::BM == 2 * GS_M && OddShape::BM == GS_M && HalfShape::BM == GS_M && HalfShape::LDS <= PairShape::LDS && OddShape::LDS <= PairShape::LDS && ShortShape::LDS <= PairShape::LDS &&
                       WIDE_OUT(GLU) == 2 * ODD_OUT(GLU), "");
-    auto kernel = odd_apart(2 * max_pairs - tiles + 1, wide_blocks, a.K) ? grouped_gemm_pairs_kernel<GLU, true> : grouped_gemm_pairs_kernel<GLU, false>;
+    auto kernel = odd_apart(odd, wide_blocks, a.K) ? grouped_gemm_pairs_kernel<GLU, true> : grouped_gemm_pairs_kernel<GLU, false>;
     if (pairs >= (1l << 31) || hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PairShape::LDS) != hipSuccess)
       return false;
     hipLaunchKernelGGL(kernel, dim3((unsigned)pairs), dim3(256), PairShape::LDS, stream, a, runs, max_pairs, wide_blocks, odd_blocks);
@@ -488,6 +489,7 @@ TK_API int tk_grouped_gemm_bf16(const void* A, int lda, const int* a_row, const 
     TK_REQUIRE(!out_f32 && a_cols == 0 && c_cols == 0, "grouped_gemm: groups by tile write the storage type and have no columns of their own");
     TK_REQUIRE(!runs || (((uintptr_t)runs & 15) == 0 && K % TILE_K == 0 && a_rows * lda * 2 < (1l << 32) && (glu ? 2l : 1l) * N * K * 2 < (1l << 32) && max_pairs > 0),
                "grouped_gemm: pairs of tiles take whole steps of %d of K, and rows that 32-bit offsets reach", TILE_K);
+    TK_REQUIRE(!runs || (2l * max_pairs >= tiles), "grouped_gemm: %d pairs are no list of the pairs of %d tiles", max_pairs, tiles);
     TK_REQUIRE(glu ? launch_by_tile<true>(a, tiles, runs, max_pairs, stream) : launch_by_tile<false>(a, tiles, runs, max_pairs, stream), "grouped_gemm: too many outputs");
     TK_CHECK_LAUNCH("grouped_gemm");
     return 0;
