@@ -30,6 +30,7 @@
 // partial (max, sum, weighted values) go to scratch and a second kernel adds them
 // in split order.  With few tiles (decode) many wavefronts with two or three steps
 // each keep enough loads in flight; with many tiles (prompts) NW is 1.
+#include "calls.h"
 #include "attention_mfma.h"
 
 template <int DT, int RT, bool BIG, bool SHARED>

@@ -7,23 +7,7 @@
 // 2 to 3 us and the layers of a step share the memory for what lies between two products.  Whole steps, us, part by part / in one call:
 // 1B shape 17 tokens 1,695 / 1,012, 101 1,685 / 1,242, 300 2,219 / 1,908, 500 2,247 / 2,158, 800 3,004 / 2,990; 3B shape 100 tokens 2,777 /
 // 2,716, 8B shape 100 tokens 4,870 / 4,782.
-#include "common.h"
-
-extern "C" {
-int tk_gemm_skinny_bf16(const void* A, int lda, const void* W, void* C, int ldc, const void* residual, int ldr, const void* extra, int M, int N,
-                        int K, int epi, int waves_k, int tiles, int staged, int tile_rows, int fold, hipStream_t stream);
-int tk_split_linear_add_rmsnorm(const void* A, int lda, const void* W, float* part, int M, int N, int K, int cuts, const void* residual,
-                                const void* w, int w_f32, void* stream_out, void* out, float eps, int once, hipStream_t stream);
-int tk_split_linear_rope_append(const void* A, int lda, const void* W, float* part, int M, int K, int cuts, void* q, const int* positions,
-                                const int* token_req, const int* block_table, int table_stride, const float* cos_t, const float* sin_t,
-                                void* kcache, void* vcache, int nq, int nkv, int d, int P, hipStream_t stream);
-int tk_gemm_tiles_bf16(const void* A, int lda, const void* W, void* C, int ldc, int M, int N, int K, int glu, int shape, hipStream_t stream);
-int tk_paged_attention_mfma(const void* q, int q_stride, void* out, int out_stride, const void* kcache, const void* vcache,
-                            const int* block_table, int table_stride, const int* q_start, const int* kv_len, const int* tile_req,
-                            const int* tile_row0, const int* tile_row1, int n_tiles, int row_tiles, int nq, int nkv, int d, int P, int window,
-                            float scale, int split, int waves, int grid_splits, int max_splits, float* part_o, float* part_ml, unsigned* tickets,
-                            int grouped, hipStream_t stream);
-}
+#include "calls.h"
 
 #define BLOCK_LAUNCHES 4
 enum { ROUTE_LIBRARY = -1, ROUTE_STREAMED = -2 };  // else the tile of tk_gemm_tiles_bf16
@@ -44,11 +28,10 @@ struct BlockCalls {
   int M, hidden, nq, nkv, d, P, window, inner;
   float scale;
   // entry points of the other libraries: rotation with append, residual sum with norm, the gated activation, the library's product
-  int (*rope_append)(int, void*, int, const int*, const int*, const int*, int, const float*, const float*, void*, void*, int, int, int, int, int,
-                     int, int, hipStream_t);
-  int (*add_rmsnorm)(int, const void*, const void*, const void*, int, void*, void*, int, int, float, hipStream_t);
-  int (*swiglu)(int, const void*, void*, int, int, hipStream_t);
-  int (*library)(const void*, int, const void*, int, void*, int, int, int, int, int, void*, size_t, hipStream_t);
+  decltype(&tk_rope_append) rope_append;
+  decltype(&tk_add_rmsnorm) add_rmsnorm;
+  decltype(&tk_swiglu) swiglu;
+  decltype(&tk_gemm_library_bf16) library;
   void* workspace;
   size_t workspace_bytes;
   // what every layer of the step reads

@@ -2,7 +2,7 @@
 // gather, the rotary tables, and rotation fused with the append to the paged cache.
 // Every kernel is a template over the storage type (float or bfloat16) and
 // computes in 32-bit.
-#include "common.h"
+#include "calls.h"
 
 // --------------------------------------------------------------------------
 // embedding: out[t, :] = table[id_t, :]; id_t < 0 names slot -id_t-1 of `last_token`

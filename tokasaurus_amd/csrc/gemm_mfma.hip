@@ -36,7 +36,7 @@
 // 32-bit store, and rotation with append: the output rows are [q heads | k heads |
 // v heads]; a workgroup takes the rows (c, c + d/2) of a head together, rotates q and k
 // by the token's position, writes q to the output and k and v into the token's page.
-#include "common.h"
+#include "calls.h"
 
 #include <type_traits>
 

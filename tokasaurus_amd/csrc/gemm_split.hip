@@ -17,7 +17,7 @@
 // weights come from memory between other products, the short ones are ahead too: 1B decode of 192 and 256 with the output projection
 // the library's / split 1,968 / 1,854 and 2,194 / 2,062 us, with q, k, v 2,081 / 1,854 and 2,172 / 2,062; 3B 5,309 / 4,761 and 5,718 / 5,358.
 // With three blocks it is behind (2,048 x 2,048 14.8 / 18.1 at 300 rows, 4,096 x 14,336 75 / 91).
-#include "common.h"
+#include "calls.h"
 
 #include <type_traits>
 

@@ -6,6 +6,7 @@
 // measurements.  Tiles come in bands of BAND tiles of rows through all outputs, each of the chip's eight dies a stretch of that order
 // (the hardware deals workgroups to the dies in turn), so that the tiles a die works on at a time share rows of A and of W in its
 // L2 (bands of 4 or 8: the same within 3 %; tiles of rows without bands 119 to 138 us for 2,048 rows of gate and up, 16,384 x 2,048).
+#include "calls.h"
 #include "gemm_tile.h"
 
 #define TILE_DIES 8
