@@ -169,3 +169,12 @@ def test_what_the_split_products_take(calls, monkeypatch):
     assert _taken(calls, linear(2048, 2048), shifted, on_gpu(200, 2048), n, _rope(200, 16, 8, 64)) == ["mm", "tk_add_rmsnorm"]
     wide = on_gpu(33, 2049)[:, 1:]  # a residual whose rows do not follow each other
     assert _taken(calls, linear(2048, 2048), on_gpu(33, 2048), wide, n, _rope(33, 16, 8, 64)) == [skinny, split[1]]
+
+
+def test_rows_that_lie_too_far_apart_for_tiles_are_the_librarys_in_a_blocks_call_too():
+    """The longest row that a tile's offsets reach, and the next size: as the product called by itself."""
+    for inner, want in ((ops.TILES_LONGEST_STRIDE, 0), (ops.TILES_LONGEST_STRIDE + 64, -1)):
+        assert ops.tiles_choice(1024, 4096, inner) == 0
+        lin = Linear(inner, ["w"], [4096])
+        lin.weight = torch.empty((4096, inner), dtype=torch.bfloat16, device="meta")
+        assert lin.many_rows_route(1024, 1 << 30) == (0, want, False)

@@ -113,7 +113,8 @@ class Linear:
             return ops.split_cuts(self.total_out, self.in_features, m), -1, m <= self.split_once_to
         if self._fast(m):
             return None
-        return 0, ops.tiles_choice(m, self.total_out, self.in_features) if m >= ops.PLAIN_TILES_FROM_ROWS else -1, False
+        tiles = m >= ops.PLAIN_TILES_FROM_ROWS and self.in_features <= ops.TILES_LONGEST_STRIDE
+        return 0, ops.tiles_choice(m, self.total_out, self.in_features) if tiles else -1, False
 
     def gate_up_route(self, m: int) -> "int | None":
         """The same for gate and up with silu behind: a tile, -1 for the library's product, -2 for the streamed form."""
@@ -122,7 +123,8 @@ class Linear:
             return None
         if self._fast(m, paired=True):
             return -2 if ops.glu_streams(m, inner, self.in_features) else None
-        return ops.tiles_choice(m, inner, self.in_features, True) if m >= ops.GLU_TILES_FROM_ROWS else -1
+        tiles = m >= ops.GLU_TILES_FROM_ROWS and self.in_features <= ops.TILES_LONGEST_STRIDE
+        return ops.tiles_choice(m, inner, self.in_features, True) if tiles else -1
 
     def __call__(
         self,
