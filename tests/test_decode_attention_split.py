@@ -49,8 +49,14 @@ def test_even_splits_where_they_are_ahead(head_dim):
 
 
 @pytest.mark.parametrize("group,nkv,requests,keys,waves", [(8, 8, 1, 8192, 8), (5, 8, 4, 32768, 8), (7, 4, 1, 32768, 8), (8, 1, 16, 8192, 8), (4, 8, 1, 8192, 4), (4, 8, 16, 8192, 4),
-                                                           (3, 8, 45, 2000, 4), (4, 8, 64, 8192, 8), (4, 8, 2, 131072, 8), (8, 8, 1, 1024, 4)])
+                                                           (3, 8, 45, 2000, 4), (4, 8, 32, 4096, 8), (2, 4, 48, 8192, 8), (2, 4, 12, 32768, 8), (4, 8, 4, 16000, 8), (4, 8, 64, 8192, 8), (4, 8, 2, 131072, 8), (8, 8, 1, 1024, 4)])
 def test_wavefronts_at_head_sizes_above_64(group, nkv, requests, keys, waves):
-    """Eight a workgroup for many query heads a kv head and for long splits, four for few heads."""
+    """Eight a workgroup, but for few query heads a kv head where every workgroup has a compute unit to itself and short walks."""
     split, got = ops.attention_split(keys, requests, nkv, 128, group)
     assert got == waves and split % (32 * waves) == 0
+
+
+@pytest.mark.parametrize("head_dim,tiles,nkv,waves,even", [(64, 64, 8, 8, True), (64, 32, 16, 8, True), (64, 63, 8, 8, False), (64, 64, 8, 4, False), (64, 64, 8, 16, False),
+                                                           (128, 64, 8, 8, False)])
+def test_even_parts_where_two_workgroups_of_eight_fill_a_unit(head_dim, tiles, nkv, waves, even):
+    assert ops.attention_even_parts(tiles, nkv, head_dim, waves) == even

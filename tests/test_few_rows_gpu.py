@@ -141,6 +141,15 @@ def test_wavefronts_share_the_keys_that_a_split_has(d, split, waves, window):
         assert ((got[i].double().view(nq, d) - want).abs() <= 2.0 ** -7 * size + 1e-6).all(), n
 
 
+@pytest.mark.parametrize("d,split,waves", [(64, 128, 4), (64, 96, 3), (64, 4096, 8), (128, 256, 4), (128, 160, 5), (128, 4096, 8)])
+@pytest.mark.parametrize("window", [0, 70])
+def test_wavefronts_share_the_keys_that_are_there(d, split, waves, window, monkeypatch):
+    """The same where a request's keys, not the split, are shared evenly."""
+    attention = ops.paged_attention_mfma
+    monkeypatch.setattr(ops, "paged_attention_mfma", lambda *a, **kw: attention(*a, **kw, even=True))
+    test_wavefronts_share_the_keys_that_a_split_has(d, split, waves, window)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("pieces", [1, 255, 256, 257, 511, 512, 513, 1024, 1025])
 def test_rows_held_in_registers_by_the_norm(dtype, pieces):

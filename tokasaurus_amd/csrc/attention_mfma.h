@@ -61,6 +61,7 @@ struct AttnArgs {
   int nq, nkv, group, P, p_shift, window;
   float scale_log2;  // scale * log2(e) > 0
   int split;         // keys per split, a multiple of 32
+  int even;          // whether the wavefronts of a workgroup share the keys that are there evenly
   int max_splits;    // splits a tile may have (size of the scratch)
   float* part_o;     // [tiles][nkv][max_splits][16 * RT][D]
   float* part_ml;    // [tiles][nkv][max_splits][16 * RT][2]
@@ -321,13 +322,15 @@ __device__ __forceinline__ void attention_item(const AttnArgs& a, const int tile
   const int s = GROUPED ? 0 : t.s_first + split_index;
   if (!GROUPED && s > t.s_last) return;
   const int nsp = GROUPED ? 1 : t.s_last - t.s_first + 1;
-  // this wavefront's part of the keys that the split has: `sub` of them, a multiple of 32.  (Of a request that ends, or whose
-  // window begins, inside the split every wavefront still takes as many as the others: cut by the split's size instead, 64
-  // requests of 375 to 3,000 keys planned for 4,096 waited for wavefronts of 512 keys.)
+  // this wavefront's part of the split: `sub` keys, a multiple of 32.  Fixed parts of the split, or (`even`) of the keys that are there:
+  // of a request that ends, or whose window begins, inside the split every wavefront then takes as many as the others.  Fixed
+  // parts give a workgroup as many wavefronts as it has keys to read, so that requests of all lengths end at one time, and are the
+  // rule; the host asks for even ones where they were ahead.
   const int k_first = max((t.lo >> 5) << 5, s * a.split), k_last = min(t.hi + 1, (s + 1) * a.split);
-  const int sub = NW == 1 ? a.split : (((k_last - k_first + NW - 1) / NW + 31) >> 5) << 5;
-  const int k_begin = k_first + wave * sub;
-  const int k_end = min(k_last, k_begin + sub);
+  const bool even = RT == 1 && a.even;
+  const int sub = even ? (((k_last - k_first + NW - 1) / NW + 31) >> 5) << 5 : a.split / NW;
+  const int part = (even ? k_first : s * a.split) + wave * sub;
+  const int k_begin = max(k_first, part), k_end = min(k_last, part + sub);
   const int* table = a.block_table + (size_t)t.req * a.table_stride;
 
   // the steps (by their first key) in which a row tile has a row that sees a key, in which all

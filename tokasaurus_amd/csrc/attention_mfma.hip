@@ -243,7 +243,7 @@ TK_API int tk_paged_attention_mfma(const void* q, int q_stride, void* out, int o
                                        const int* tile_req, const int* tile_row0, const int* tile_row1,
                                        int n_tiles, int row_tiles, int nq, int nkv, int d, int P, int window,
                                        float scale, int split, int waves, int grid_splits, int max_splits,
-                                       float* part_o, float* part_ml, unsigned* tickets, int grouped, hipStream_t stream) {
+                                       float* part_o, float* part_ml, unsigned* tickets, int grouped, int even, hipStream_t stream) {
   TK_REQUIRE(n_tiles >= 0 && nq > 0 && nkv > 0 && nq % nkv == 0, "attention_mfma: bad sizes tiles=%d nq=%d nkv=%d", n_tiles, nq, nkv);
   TK_REQUIRE(d % 16 == 0 && d >= 16 && d <= 128, "attention_mfma: head size %d is not a multiple of 16 up to 128", d);
   TK_REQUIRE(P >= 4 && (P & (P - 1)) == 0, "attention_mfma: page size %d is not a power of two from 4", P);
@@ -278,7 +278,7 @@ TK_API int tk_paged_attention_mfma(const void* q, int q_stride, void* out, int o
   a.p_shift = 0;
   while ((1 << a.p_shift) < P) ++a.p_shift;
   a.scale_log2 = scale * 1.4426950408889634f;
-  a.split = split; a.max_splits = max_splits; a.part_o = part_o; a.part_ml = part_ml;
+  a.split = split; a.even = even; a.max_splits = max_splits; a.part_o = part_o; a.part_ml = part_ml;
   a.tickets = (max_splits > 1 && row_tiles == 1) ? tickets : nullptr;
   const bool ok = grouped ? launch_group_d(a, d / 16, grouped, stream)
                           : (row_tiles == 1 ? launch_attn_d<1>(a, d / 16, grid_splits, waves, stream)

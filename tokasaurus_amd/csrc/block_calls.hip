@@ -19,7 +19,7 @@ struct BlockAttention {  // one launch of the attention: its tiles, and how keys
   float* part_o;
   float* part_ml;
   unsigned* tickets;
-  int n_tiles, row_tiles, split, waves, max_splits, grouped;
+  int n_tiles, row_tiles, split, waves, max_splits, grouped, even;
 };
 
 struct BlockCalls {
@@ -118,7 +118,7 @@ TK_API int tk_block_calls(BlockCalls* given, hipStream_t stream) {
     const BlockAttention& l = b.attention[i];
     rc = tk_paged_attention_mfma(b.qkv, b.qkv_cuts > 0 ? heads : width, b.attended, heads, b.kcache, b.vcache, b.block_table, b.table_stride, b.q_start,
                                  b.kv_len, l.tile_req, l.tile_row0, l.tile_row1, l.n_tiles, l.row_tiles, b.nq, b.nkv, b.d, b.P, b.window, b.scale,
-                                 l.split, l.waves, l.max_splits, l.max_splits, l.part_o, l.part_ml, l.tickets, l.grouped, stream);
+                                 l.split, l.waves, l.max_splits, l.max_splits, l.part_o, l.part_ml, l.tickets, l.grouped, l.even, stream);
     if (rc) return rc;
   }
   rc = project(b, b.attended, heads, b.w_out, b.out_cuts, b.out_route, b.out_once, b.x, b.mid_w, b.mid_w_f32, b.mid_eps, b.stream, b.normed, stream);

@@ -19,7 +19,7 @@ TK_API int tk_paged_attention_mfma(const void* q, int q_stride, void* out, int o
                                    const int* block_table, int table_stride, const int* q_start, const int* kv_len, const int* tile_req,
                                    const int* tile_row0, const int* tile_row1, int n_tiles, int row_tiles, int nq, int nkv, int d, int P,
                                    int window, float scale, int split, int waves, int grid_splits, int max_splits, float* part_o, float* part_ml,
-                                   unsigned* tickets, int grouped, hipStream_t stream);
+                                   unsigned* tickets, int grouped, int even, hipStream_t stream);
 
 // of the other libraries, called by their addresses
 TK_API int tk_rope_append(int dt, void* qkv, int row_stride, const int* positions, const int* token_req, const int* block_table, int table_stride,

@@ -24,7 +24,7 @@ MOST_ROWS = 1024
 
 class _Attention(ctypes.Structure):
     _fields_ = [(n, c_void_p) for n in ("tile_req", "tile_row0", "tile_row1", "part_o", "part_ml", "tickets")] + [
-        (n, c_int) for n in ("n_tiles", "row_tiles", "split", "waves", "max_splits", "grouped")]
+        (n, c_int) for n in ("n_tiles", "row_tiles", "split", "waves", "max_splits", "grouped", "even")]
 
 
 class _BlockCalls(ctypes.Structure):
@@ -82,7 +82,7 @@ class BlockPlan:
             n_tiles, splits = l.tile_req.numel(), max(1, -(-l.max_kv_len // l.split))
             a.tile_req, a.tile_row0 = l.tile_req.data_ptr(), l.tile_row0.data_ptr()
             a.tile_row1 = l.tile_row1.data_ptr() if l.tile_row1 is not None else None
-            a.n_tiles, a.row_tiles, a.split, a.waves, a.max_splits, a.grouped = n_tiles, l.row_tiles, l.split, l.waves, splits, int(l.grouped)
+            a.n_tiles, a.row_tiles, a.split, a.waves, a.max_splits, a.grouped, a.even = n_tiles, l.row_tiles, l.split, l.waves, splits, int(l.grouped), int(l.even)
             if splits > 1:
                 in_kernel = l.row_tiles == 1 and ops.ATTENTION_MERGE_IN_KERNEL
                 items = n_tiles * nkv * splits * 16 * l.row_tiles

@@ -98,7 +98,7 @@ _SIGNATURES: dict[str, dict[str, list]] = {
     "mfma": {
         "tk_paged_attention_mfma": [_P, c_int, _P, c_int, _P, _P, _P, c_int, _P, _P, _P, _P, _P]
         + [c_int] * 7
-        + [c_float, c_int, c_int, c_int, c_int, _P, _P, _P, c_int, _P],
+        + [c_float, c_int, c_int, c_int, c_int, _P, _P, _P, c_int, c_int, _P],
         "tk_gemm_skinny_bf16": [_P, c_int, _P, _P, c_int, _P, c_int, _P] + [c_int] * 9 + [_P],
         "tk_gemm_skinny_parts": [c_int] * 6,
         "tk_gemm_split_bf16": [_P, c_int, _P, _P] + [c_int] * 4 + [_P],

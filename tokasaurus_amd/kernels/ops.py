@@ -612,12 +612,12 @@ def attention_split(max_kv_len: int, n_tiles: int, nkv: int, head_dim: int = 64,
     of them, and beyond eight splits 256 (us a layer of 8 kv heads at one request, planned for 1,024: splits of 64 keys for one
     wavefront / of 128 for four, head size 64 9.4 / 6.3 at 500 keys, 10.5 / 6.8 at 1,000, head size 128 16.4 / 9.0; planned for 2,048: 128
     for two / 256 for four 8.1 / 7.2 at 1,100, 9.3 / 7.7 at 2,000; two requests of 1,000 keys 12.8 / 8.1).  At head sizes above 64
-    a compute unit has room for eight wavefronts.  Eight of a workgroup are ahead of four where a kv head has more than four query heads (us at head
-    size 128, four / eight: 40 on 8 at one request of 8,192 keys 18.4 / 16.2, at 4 of 32,768 98 / 95, at 16 of 1,500 25.6 / 25.0, of 8,192 94 / 101; 28 on 4 14.5 / 12.6 and 55 / 55; 8
-    on 1 14.2 / 12.3 and 32.7 / 32.0; head size 80, 32 on 4, 12.9 / 10.7 and 39.4 / 36.7), four where it has up to four (32 on 8 16.4 / 16.5 at one request of
-    8,192, 33.3 / 34.7 of 32,768, 20.5 / 21.1 and 52 / 56 at two, 93 / 100 at 16 of 8,192, 24.6 / 25.2 of 1,500, 178 / 195 at 64 of 4,096; 16 on 4 12.1 / 12.3 and 31.0 / 32.1 at one, 22.0 /
-    24.3 at two of 16,384), but for splits of 8,192 keys, where eight are again (32 on 8 8 requests of 32,768 192 / 180, 64 of 8,192 400 / 361, 2 of 131,072 196 /
-    189, 4 of 131,072 388 / 441)."""
+    a compute unit has room for eight wavefronts, and a workgroup has them, or four at head sizes above 96 with up to four query heads a kv head
+    where every workgroup has a unit to itself and the keys are in two to four splits or the splits are short (us at head size 128, eight / four: 32
+    heads on 8, 16 requests of 4,080 52.2 / 51.5, of 510 to 4,080 37.0 / 35.5, 16 of 190 to 1,520 18.2 / 17.2; in the mean of 100 mixes 2 to 3 %, at the
+    worst 2 % behind).  Not elsewhere: 32 requests of 280 to 2,236 planned for 4,096 35.7 / 43.4 (a wavefront walks 1,024 keys), 48 of 766 to 6,128 on 4
+    kv heads 71.2 / 84.3 and 12 of 4,094 to 32,752 89 / 134 (two workgroups of four on one unit, none on others), one request of 16,000 beside
+    three of 100 21.6 / 22.8, 40 heads on 8 at 8,192 keys 16.2 / 18.4, head size 96 8 of 560 to 4,489 20.7 / 21.8."""
     base = max(n_tiles * nkv, 1)
     kv = max(max_kv_len, 1)
     splits = max(1, min(16, -(-256 // base), -(-kv // 128), max(8, kv // 256)))
@@ -627,12 +627,23 @@ def attention_split(max_kv_len: int, n_tiles: int, nkv: int, head_dim: int = 64,
     # 8 192 keys; 255 of 512 beside one of 32 768: 401 / 114 us; requests of one length lose nothing)
     raw = min(-(-kv // splits), 8192 if base < 1024 else 2048)
     per_wave = min(512, max(32 if raw <= 128 else 64, kv * base // 2048))
-    most = 4 if head_dim > 64 and (group is None or (group <= 4 and raw < 8192)) else attention_max_waves(head_dim, 1)
+    four = head_dim > 96 and group is not None and group <= 4 and 1 < splits <= 256 // base and (raw < 1024 or (splits <= 4 and base * splits > 128))
+    most = 4 if head_dim > 64 and (group is None or four) else attention_max_waves(head_dim, 1)
     waves = 1
     while waves * 2 <= min(most, raw // per_wave):
         waves *= 2
     step = 32 * waves
     return -(-raw // step) * step, waves
+
+
+def attention_even_parts(n_tiles: int, nkv: int, head_dim: int, waves: int) -> bool:
+    """Whether the wavefronts of a decoding workgroup share the keys that a request has in its split evenly; else each has a fixed part of the split,
+    so that a request keeps as many wavefronts busy as it has keys and requests of all lengths end at one time.
+    Where two workgroups of eight fill a compute unit even parts are ahead: 396 mixes of 32 to 125 requests planned for 4,096 to 6,000 keys,
+    head size 64, in the mean 3.3 %, 197 by 2 % and more (to 25 %), 19 behind by as much (at the worst 5 %, few long requests among short ones);
+    64 of 380 to 3,000 keys fixed / even 53.5 / 49.8 us.  Of 246 mixes of all sizes, head sizes 64 and 128, 49 were ahead and 92 behind: 32 of 500 to
+    4,000 planned for 4,096 58.7 / 62.7 at head size 128, 32 of 380 to 3,000 24.8 / 26.8, 48 of 280 to 2,236 29.4 / 32.3, 64 of 190 to 1,500 25.0 / 26.6 at 64."""
+    return head_dim <= 64 and waves == 8 and n_tiles * nkv >= 512
 
 
 # workgroups with and without keys that even cuts may take, where the planned ones take fewer: partial results of 33 MB at head size 128
@@ -725,6 +736,7 @@ def paged_attention_mfma(
     longest: int | None = None,
     grouped: bool | int = False,
     merge_kernel: bool = False,
+    even: bool = False,
 ) -> torch.Tensor:
     """Attention of every token of the batch over its request's pages on the
     matrix cores (bfloat16).  ``q`` is 2-d and its first nq*d columns are the
@@ -742,7 +754,8 @@ def paged_attention_mfma(
 
     The splits of a tile of one row tile (decoded tokens) are added inside the kernel by the
     workgroup that arrives last; ``merge_kernel`` has a second kernel add them instead, as for
-    tiles of two row tiles."""
+    tiles of two row tiles.  ``even`` (one row tile): the wavefronts of a workgroup share the keys that a request has
+    in the split evenly, instead of the split (see ``attention_even_parts``)."""
     _gpu(q, kcache, vcache, block_table, q_start, kv_len, tile_req, tile_row0)
     _need(q.dim() == 2 and q.stride(1) == 1 and q.shape[1] >= nq * head_dim and q.dtype == torch.bfloat16,
           "attention_mfma: q must be bfloat16, 2-d with unit inner stride and nq*d leading columns")
@@ -800,6 +813,7 @@ def paged_attention_mfma(
         part_ml.data_ptr() if part_ml is not None else None,
         tickets.data_ptr() if tickets is not None else None,
         int(grouped),
+        int(even),
         _stream(),
     )
     return out

@@ -46,6 +46,7 @@ class AttentionLaunch:
     max_kv_len: int  # bounds the keys of the launch's requests: sizes its grid and scratch
     scratch: ops.AttentionScratch | None = None  # a replayed step keeps its own
     grouped: int = 0  # 1, 2: tiles in groups of one request that share their loads, with so many sets of wavefronts (long prompts)
+    even: bool = False  # decoded tokens: the wavefronts of a workgroup share the keys that are there, not the split
 
 
 @dataclass
@@ -77,15 +78,18 @@ def attention_plan(ctx: StepContext, group: int, nkv: int, head_dim: int, page_s
         # which no recorded step holds: they are cut by their own lengths)
         bound = max(int(ctx.extras.get("kv_bound", 0)), ctx.max_kv_len)
         lists: list[tuple[list[int], list[int], list[int] | None, int, int, int, int, int]] = []
+        even = False
         if small:
             req, row0, _ = ops.attention_tiles(q_lens, group, 1, small)
             if large and not static:
                 lengths = [ctx.host_kv_len[r] for r in small]
                 split, waves = ops.attention_even_split(lengths, nkv, head_dim, group)
+                even = (split, waves) != ops.attention_split(max(lengths), len(req), nkv, head_dim, group)
                 lists.append((req, row0, None, 1, split, waves, 0, max(lengths)))
             else:
                 split, waves = ops.attention_split(bound, len(req), nkv, head_dim, group)
                 lists.append((req, row0, None, 1, split, waves, 0, bound))
+            even = even or ops.attention_even_parts(len(req), nkv, head_dim, waves)
         # Portions that come after a past several times their own length walk far more keys a row than
         # whole prompts do: they are planned apart, or one of them among whole prompts would take a
         # form chosen for the many short walks and walk its long past on a few wavefronts.
@@ -120,7 +124,7 @@ def attention_plan(ctx: StepContext, group: int, nkv: int, head_dim: int, page_s
             t_row1 = dev[at + 2 * n : at + 3 * n] if row1 is not None else None
             at += (3 if row1 is not None else 2) * n
             launches.append(AttentionLaunch(t_req, t_row0, t_row1, row_tiles, split, waves, max_kv_len,
-                                            ops.AttentionScratch(ctx.device) if static else None, grouped))
+                                            ops.AttentionScratch(ctx.device) if static else None, grouped, even and row_tiles == 1))
         plan = AttentionPlan(launches, bound)
         ctx.extras[key] = plan
     return plan
@@ -245,7 +249,7 @@ class PagedAttention(Mixer):
                     launch.tile_req, launch.tile_row0, launch.row_tiles, nq, nkv, d, cache.page_size,
                     launch.max_kv_len, launch.split, window=self.window, scale=self.scale, waves=launch.waves,
                     out=attn, scratch=launch.scratch, tile_row1=launch.tile_row1, longest=min(ctx.max_kv_len, launch.max_kv_len),
-                    grouped=launch.grouped,
+                    grouped=launch.grouped, even=launch.even,
                 )
         elif q.dtype == torch.float32 and ops.attention_tile_f32_fits(nq, nkv, d, d, cache.page_size):
             # the true 32-bit path: 32-bit products on the matrix cores, prompt portions in tiles of 16 tokens, single
