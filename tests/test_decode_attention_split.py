@@ -44,8 +44,12 @@ def test_even_splits_where_they_are_ahead(head_dim):
     even = lambda lengths: ops.attention_even_split(lengths, 8, head_dim) != ops.attention_split(max(lengths), len(lengths), 8, head_dim)  # noqa: E731
     for lengths in ([1000 + 466 * i for i in range(16)], [200 + 122 * i for i in range(32)], [100 + 9 * i for i in range(100)], [100] * 3 + [16000], [2000] * 60):
         assert not even(lengths)
-    for lengths in ([250 + 39 * i for i in range(45)], [1500] * 20 + [6000] * 4, [500] * 63 + [8000], [300] * 10 + [4000] * 2):
+    for lengths in ([1000] * 30 + [3000] * 2, [1500] * 20 + [6000] * 4, [90 + 17 * i for i in range(41)]):
+        assert not even(lengths)
+    for lengths in ([500] * 63 + [8000], [300] * 10 + [4000] * 2):
         assert even(lengths)
+    for lengths in ([250 + 39 * i for i in range(45)], [1000 + 159 * i for i in range(45)], [500 + 64 * i for i in range(40)]):
+        assert even(lengths) == (head_dim > 64)
 
 
 @pytest.mark.parametrize("group,nkv,requests,keys,waves", [(8, 8, 1, 8192, 8), (5, 8, 4, 32768, 8), (7, 4, 1, 32768, 8), (8, 1, 16, 8192, 8), (4, 8, 1, 8192, 4), (4, 8, 16, 8192, 4),

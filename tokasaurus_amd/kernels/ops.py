@@ -652,25 +652,26 @@ ATTENTION_EVEN_WORKGROUPS = 4096
 
 def attention_even_split(lengths: list[int], nkv: int, head_dim: int, group: int | None = None) -> tuple[int, int]:
     """The same for decoded tokens beside prompts, in a step that is not recorded: their lengths are known, and where a workgroup's
-    longest walk is over a compute unit's share of the keys by a fifth the keys are cut shorter, so that the workgroups (two a unit) get as many
-    each.  That pays where some units have two of the planned workgroups and others one, or where few requests are long.  us a layer
-    of 8 kv heads, planned / even, head sizes 64 and 128: 45 requests of 250 to 2,000 keys 28.0 / 28.7 and 49.8 / 47.9, 45 of 1,000 to 8,000
-    103 / 88 and 184 / 164, 50 of any length to 4,000 50.6 / 54.1 and 96 / 93, 20 of 1,500 and 4 of 6,000 38.2 / 31.1 and 62 / 56, 63 of 500 and one of 8,000 92 /
-    29 and 158 / 53, 10 of 300 and 2 of 4,000 16.2 / 12.6 and 23.9 / 20.7, 30 of 1,000 and 2 of 3,000 25.9 / 24.0 and 43.5 / 46.0.  It does not where the planned
-    workgroups fill one round and their lengths rise evenly (16 of 1,000 to 8,000 37.5 / 39.7 and 61 / 70, 32 of 200 to 4,000 32.4 / 34.8 and 59 / 64),
-    fill several (100 of 100 to 1,000 28.4 / 29.3 and 49 / 53), or are fewer than half the units (3 of 100 and one of 16,000 19.3 / 22.9 and 30.9 / 30.4).
+    longest walk is over a compute unit's share of the keys by a fifth the keys may be cut shorter, so that the workgroups (two a unit) get as many
+    each, their wavefronts even parts.  That pays where few requests are four times as long as the mean, and at head sizes above 64 also where some units
+    have two of the planned workgroups.  us a layer of 8 kv heads, planned / even, head sizes 64 and 128: 63 requests of 500 keys and one of 8,000
+    79 / 26 and 153 / 52, 10 of 300 and 2 of 4,000 13.8 / 11.2 and 17.9 / 16.4, 45 of 250 to 2,000 25.8 / 28.4 and 50.3 / 47.6, 45 of 1,000 to 8,000 104 / 88
+    and 172 / 164, 50 of any length to 4,000 49.2 / 52.8 and 98 / 92, 40 of 500 to 3,000 34.6 / 35.7 and 69.3 / 63.7.  It does not, or seldom, where the planned workgroups
+    fill one round (16 of 1,000 to 8,000 34.2 / 38.6 and 59.3 / 70.8, 32 of 200 to 4,000 31.7 / 35.2 and 60.5 / 63.5, 30 of 1,000 and 2 of 3,000 20.7 / 21.4 and
+    43.5 / 45.2, 20 of 1,500 and 4 of 6,000 33.6 / 31.3 and 59.1 / 55.5) or several (100 of 100 to 1,000 25.5 / 29.1 and 48.3 / 52.9), are fewer than half the units (3 of 100
+    and one of 16,000 13.6 / 17.7 and 22.8 / 26.5), or where no request has two whole cuts (41 of any length to 770 18.3 / 19.5 at 128).
     The grid and the partial results are as many as the longest request has splits, for every request: they are bounded (63 of 40 and one of 28,000, by
     512 keys 28,160 workgroups of which 944 have keys; 127 of 64 and one of 24,000 planned / by 512 keys 55 / 75 and 76 / 117)."""
     split, waves = attention_split(max(lengths), len(lengths), nkv, head_dim, group)
     longest, total = max(lengths), sum(lengths)
     planned = sum(-(-n // split) for n in lengths) * nkv
-    if not (min(split, longest) * 256 * 5 >= total * nkv * 6 and planned >= 128 and (planned > 256 or longest * len(lengths) * 5 > total * 11)):
+    if not (min(split, longest) * 256 * 5 >= total * nkv * 6 and planned >= 128 and ((head_dim > 64 and planned > 256) or longest * len(lengths) > total * 4)):
         return split, waves
     even = max(512, -(-(-(-total * nkv // 512)) // 128) * 128)
     # (in as many cuts of the longest request as there is room for)
     cuts = max(1, ATTENTION_EVEN_WORKGROUPS // (len(lengths) * nkv))
     even = max(even, -(-(-(-longest // cuts)) // 128) * 128)
-    return (even, 4) if even < split else (split, waves)
+    return (even, 4) if even < split and longest >= 2 * even else (split, waves)
 
 
 # Whether the splits of decoded tokens' tiles are added inside the attention kernel, by the
