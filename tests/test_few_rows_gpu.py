@@ -74,6 +74,29 @@ def test_tiles_of_8_for_one_and_two_rows_where_they_are_folded(m):
             assert torch.allclose(pre.sumsq.sum(1), x.float().pow(2).sum(1), rtol=4096 * 2.0 ** -24, atol=0)
 
 
+@pytest.mark.parametrize("m", [1, 9, 17, 40])
+@pytest.mark.parametrize("steps", [1, 2, 3, 5, 7, 8, 9, 10, 15, 16, 17])
+def test_steps_that_are_left_behind_whole_groups(m, steps):
+    """Walks of one wavefront, and of two of uneven length, over fewer steps than a group of loads, whole groups and some more: sums of k products
+    in 32-bit, k 2^-24 of the sum of the magnitudes; behind gate and up three roundings to 8 bits more."""
+    gen = torch.Generator(device="cuda").manual_seed(m + steps)
+    k, n = 32 * steps, 72
+    pre, rows = _norm(m, k, 8, gen)
+    w = torch.randn((2 * n, k), generator=gen, device="cuda").bfloat16()
+    want, size = rows @ w.double().T, rows.abs() @ w.double().abs().T
+    for waves in (1, 2):
+        got = ops.gemm_skinny_bf16(pre.scaled, w, out_f32=True, waves_k=waves, fold=steps % 2 == 0)
+        plain, plain_size = pre.scaled.double() @ w.double().T, pre.scaled.double().abs() @ w.double().abs().T
+        assert ((got.double() - plain).abs() <= (k + 8) * 2.0 ** -24 * plain_size).all()
+        got = ops.gemm_skinny_bf16(pre.scaled, w, prenorm=pre, norm_eps=1e-5, out_f32=True, waves_k=waves)
+        assert ((got.double() - want).abs() <= (k + 16) * 2.0 ** -24 * size).all()
+        got = ops.gemm_skinny_bf16(pre.scaled, w, prenorm=pre, norm_eps=1e-5, swiglu=True, staged=0, waves_k=waves)
+        gate, up, slack = want[:, :n], want[:, n:], (k + 16) * 2.0 ** -24
+        s = torch.nn.functional.silu(gate)
+        bound = 2.0 ** -8 * (1.1 * gate.abs() * up.abs() + 3 * (s * up).abs()) * 1.1 + 2 * slack * (size[:, :n] * up.abs() + s.abs() * size[:, n:]) + 1e-6
+        assert ((got.double() - s * up).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("begin", [1, 2, 3])
 def test_rows_for_the_norm_behind_that_begin_anywhere(begin, monkeypatch):
     """Memory for x w that starts 2, 4 and 6 bytes behind a multiple of 8: the same values."""

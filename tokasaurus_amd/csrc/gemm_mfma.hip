@@ -412,23 +412,33 @@ __global__ __launch_bounds__(sk_max_waves(NT) * 64) void gemm_skinny_kernel(Gemm
         for (int mb = 0; mb < MB; ++mb)
           acc[t][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][t], av[u][mb], acc[t][mb], 0, 0, 0);
     };
-    // first as many steps as leave whole groups of U; the loads of the steps that are not there repeat the last one, so that
-    // no branch stands between the loads
-    const int some = (ks1 - ks0 + U - 1) % U + 1;
-    __builtin_amdgcn_sched_barrier(0);  // (loads return in order: what is waited for first goes out first)
-#pragma unroll
-    for (int u = 0; u < U; ++u) load(u, ks0 + min(u, some - 1));
-    __builtin_amdgcn_sched_barrier(0);
-    if (EPI == EPI_ROPE && has_unit) rope_ask_further(a, rope_head, rope_col + (l0 >> 4) * 4, rope_pre);
-    if (NORM) early_row_scale(a, scales, parts_pre, wave, lane);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (u < some) multiply(u);
-    for (ks += some; ks < ks1; ks += U) {
+    // Whole groups of U steps, then what is left as one group more, behind branches that are the same for the whole wavefront.  (Its missing
+    // loads may not repeat one that is there instead: 16 loads for 10 steps took 16 rows of 264 x 5,120 14.1 us, so 9.9, 8 rows of
+    // 5,120 x 5,120 25.2 and 18.6, 1 of 7,168 x 5,120 with the rotation 22.8 and 16.6.)
+    bool first = true;
+    auto meanwhile = [&]() {  // behind a wavefront's first loads
+      if (first && EPI == EPI_ROPE && has_unit) rope_ask_further(a, rope_head, rope_col + (l0 >> 4) * 4, rope_pre);
+      if (first && NORM) early_row_scale(a, scales, parts_pre, wave, lane);
+      first = false;
+    };
+    for (; ks + U <= ks1; ks += U) {
+      __builtin_amdgcn_sched_barrier(0);  // (loads return in order: what is waited for first goes out first)
 #pragma unroll
       for (int u = 0; u < U; ++u) load(u, ks + u);
+      __builtin_amdgcn_sched_barrier(0);
+      meanwhile();
 #pragma unroll
       for (int u = 0; u < U; ++u) multiply(u);
+    }
+    if (ks < ks1) {
+      const int some = ks1 - ks;
+#pragma unroll
+      for (int u = 0; u < U - 1; ++u)
+        if (u < some) load(u, ks + u);
+      meanwhile();
+#pragma unroll
+      for (int u = 0; u < U - 1; ++u)
+        if (u < some) multiply(u);
     }
   } else {
     if (EPI == EPI_ROPE && has_unit) rope_ask_further(a, rope_head, rope_col + (l0 >> 4) * 4, rope_pre);
