@@ -173,3 +173,33 @@ def test_room_that_is_no_list_of_the_tiles_pairs_is_refused(monkeypatch):
         assert ((got[e::experts].double() - want).abs() <= 2.0 ** -6 * (size + want.abs())).all()
     with pytest.raises(ops.KernelError, match="pairs of 9 tiles"):
         ops.expert_mix(h, gu, dn, ids, None, pairs=dataclasses.replace(pairs, max_pairs=4))
+
+
+@pytest.mark.parametrize("counts", [[0, 1, 64, 65, 128, 129, 256, 257, 320, 321], [640, 192, 448, 511], [64] * 70])
+def test_odd_tiles_of_few_rows_are_counted(counts):
+    """Experts whose odd last tile has up to 64 rows, beside whole pairs and odd tiles."""
+    ids = torch.cat([torch.full((n,), e, dtype=torch.int32) for e, n in enumerate(counts)])
+    s = ops.expert_sort([(ids[torch.randperm(len(ids), generator=torch.Generator().manual_seed(1))].view(-1, 1).cuda(), len(counts))])[0]
+    tiles = [-(-n // 128) for n in counts]
+    assert s.runs[:4].tolist() == [sum((t + 1) // 2 for t in tiles), sum(t // 2 for t in tiles), sum(t % 2 for t in tiles),
+                                   sum(t % 2 == 1 and n - 128 * (t - 1) <= 64 for n, t in zip(counts, tiles))]
+
+
+@pytest.mark.parametrize("counts", [[520, 640, 300, 129], [270] * 4, [512, 768, 256, 1024]])
+def test_odd_tiles_apart_and_beside(counts, monkeypatch):
+    """Where odd tiles behind the pairs save a round (many outputs) and where they do not, or there are none: the same bits, those of tiles by themselves."""
+    for least in ("ROWS", "WIDTH", "INNER", "WALK"):
+        monkeypatch.setattr(ops, f"EXPERT_PAIRS_FROM_{least}", 0)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    ids = torch.cat([torch.full((n,), e, dtype=torch.int32) for e, n in enumerate(counts)]).view(-1, 1).cuda()
+    for width, ff in ((64, 64), (128, 12288)):  # (96 blocks of gate and up: several rounds of workgroups)
+        h = torch.randn((len(ids), width), generator=g, device="cuda").bfloat16()
+        gu, dn = ((torch.randn(s, generator=g, device="cuda") * 0.1).bfloat16() for s in ((len(counts), 2 * ff, width), (len(counts), width, ff)))
+        got = ops.expert_mix(h, gu, dn, ids, None)
+        monkeypatch.setattr(ops, "experts_go_in_pairs_of_tiles", lambda *a: False)
+        want = ops.expert_mix(h, gu, dn, ids, None)
+        monkeypatch.undo()
+        for least in ("ROWS", "WIDTH", "INNER", "WALK"):
+            monkeypatch.setattr(ops, f"EXPERT_PAIRS_FROM_{least}", 0)
+        # the activations' 8 bits (off by one rounding where the orders of 32-bit sums differ) and the sums behind them
+        assert float((got.double() - want.double()).norm()) <= 2.0 ** -7 * float(want.double().norm())

@@ -401,20 +401,33 @@ using ShortShape = TileShape<1, 2, 6, 6>;  // of up to 64 rows
 struct TileRun {
   int tile, group, first, tiles;
 };
-// runs: the number of pairs, the odd ones with them (as the first's tile), of whole pairs (as its group) and of odd tiles (as its first);
+// runs: the number of pairs, the odd ones with them (as the first's tile), of whole pairs (as its group), of odd tiles (as its first) and of those with up
+// to ShortShape::BM rows (as its tiles);
 // then room for max_pairs pairs in the order of the tiles, then the order in which they are multiplied: whole pairs from the front (tile,
 // group, the group's first whole pair, how many it has), odd tiles from the back (tile, group, rows that it holds).
 //
-// A compute unit holds one workgroup, and a round of pairs takes all of them for one pair each.  APART: the whole pairs come first and the
-// odd tiles, cut so that one takes a third of a pair's time and less, behind them.  An expert's last tile often holds few rows: 2,048
-// tokens, 8 of 32 experts, are 512 rows an expert give or take 20, so that half of the experts have a fifth tile of some 16.  Not
-// APART they are tiles of 128 x 256 among their group's pairs, which read the same weights.
+// A compute unit holds one workgroup, and a round of pairs takes all of them for one pair each.  Odd tiles are tiles of 128 x 256 among their
+// group's pairs, which read the same weights; or (APART, and where the numbers of pairs and odd tiles make it pay) the whole pairs come first and the
+// odd tiles, cut in two, behind them.  An expert's last tile often holds few rows: 2,048 tokens, 8 of 32 experts, are 512 rows an
+// expert give or take 20, so that half of the experts have a fifth tile of some 16.
+// It pays where it saves a round: a half of an odd tile takes some 0.65 of a pair's time, of up to 64 rows 0.35, and units that the last
+// round of pairs leaves idle take them beside it.  Both products, beside / apart: 32 experts of 2,048 x 1,024 with 95 pairs and one odd tile (3.0
+// rounds with it, 3.0 without) 370 / 403 us, 66 and 13 (2.5, 2.1) 338 / 353, 87 and 18 (3.3, 2.7) 438 / 411, 128 and 8 (4.3, 4.0) 562 / 525; 16 of 2,048 x
+// 2,048 with 33 and 7 (2.5, 2.1) 321 / 341, 64 and 3 (4.2, 4.0) 530 / 470; 8 of 2,048 x 5,632 with 8 and 8 (2.8, 1.4) 318 / 355, 32 and 3 (6.0, 5.5) 726 / 695.
+__device__ __forceinline__ bool odd_tiles_apart(const TileRun& head, int n_blocks, int odd_blocks) {
+  const int pairs = head.group * n_blocks, rounds = (pairs + 255) / 256;
+  const int odd = (13 * (head.first - head.tiles) + 7 * head.tiles) * odd_blocks;  // in twentieths of a pair
+  const int behind = max(odd - 20 * (256 * rounds - pairs), 0), beside = (head.tile * n_blocks + 255) / 256;
+  return rounds * 5120 + behind + 2880 < beside * 5120;  // (a round is 256 pairs; more than half of one is to be saved)
+}
+
 template <bool GLU, bool APART>
 __global__ __launch_bounds__(256, 1) void grouped_gemm_pairs_kernel(GroupedArgs a, const TileRun* __restrict__ runs, int max_pairs, int n_blocks, int odd_blocks) {
   extern __shared__ __align__(16) char smem[];
   const TileRun head = runs[0];
-  const TileRun* __restrict__ order = runs + 1 + (APART ? max_pairs : 0);
-  const int items = (APART ? head.group : head.tile) * n_blocks, per = (items + GS_DIES - 1) / GS_DIES;
+  const bool apart = APART && odd_tiles_apart(head, n_blocks, odd_blocks);
+  const TileRun* __restrict__ order = runs + 1 + (apart ? max_pairs : 0);
+  const int items = (apart ? head.group : head.tile) * n_blocks, per = (items + GS_DIES - 1) / GS_DIES;
   const int seq = blockIdx.x / GS_DIES, die = blockIdx.x % GS_DIES;
   if (seq < per) {
     const int item = die * per + seq;
@@ -422,13 +435,14 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_pairs_kernel(GroupedArgs 
     const int some = item / n_blocks;
     const TileRun r = order[some];
     // the chunk of up to WIDE_PAIRS pairs of the group that the item lies in
-    const int pairs = APART ? r.tiles : (r.tiles + 1) / 2;
+    const int pairs = apart ? r.tiles : (r.tiles + 1) / 2;
     const int chunk = r.first + (some - r.first) / WIDE_PAIRS * WIDE_PAIRS, len = min(WIDE_PAIRS, r.first + pairs - chunk);
     const int off = item - chunk * n_blocks, pair = chunk + off % len;
     const int tile = r.tile + 2 * (pair - r.first), n0 = off / len * WIDE_OUT(GLU);
-    if (APART || tile + 1 < r.tile + r.tiles) wide_tile<PairShape, GLU>(a, smem, r.group, tile * GS_M, n0);
-    else if constexpr (!APART) wide_tile<HalfShape, GLU>(a, smem, r.group, tile * GS_M, n0);
+    if (apart || tile + 1 < r.tile + r.tiles) wide_tile<PairShape, GLU>(a, smem, r.group, tile * GS_M, n0);
+    else wide_tile<HalfShape, GLU>(a, smem, r.group, tile * GS_M, n0);
   } else if constexpr (APART) {
+    if (!apart) return;
     const int odd = head.first * odd_blocks, odd_per = (odd + GS_DIES - 1) / GS_DIES, item = die * odd_per + seq - per;
     if (seq - per >= odd_per || item >= odd) return;
     const int some = item / odd_blocks;
@@ -439,12 +453,11 @@ __global__ __launch_bounds__(256, 1) void grouped_gemm_pairs_kernel(GroupedArgs 
   }
 }
 
-// Whether odd tiles go apart: where they are at most about one round of workgroups (`odd` of them at the most, half of that as a rule), and
-// reading their experts' weights once more costs little beside.  Both products and the sum, us, with their pairs / apart, experts'
-// rows even and uneven: 32 experts of 2,048 x 1,024 234 / 234 and 302 / 265 at 420 rows an expert, 301 / 270 and 311 / 280 at 500, 336 /
-// 334 and 408 / 369 at 700; 16 of 2,048 x 2,048 307 / 247 and 300 / 263 at 500; 8 of 4,096 x 1,792 183 / 184 and 219 / 197 at 460; but 128 of 2,048 x
-// 768 682 / 710 and 722 / 725 at 400, 8 of 4,096 x 14,336 1,109 / 1,251 and 1,123 / 1,302 at 380.
-static bool odd_apart(int odd, int n_blocks, int K) { return (long)odd * n_blocks < 512 && K <= 4096; }
+// Whether odd tiles may go apart at all (the kernel knows how many there are): where they are at most about one round of workgroups (`odd` of
+// them at the most, half of that as a rule), and reading their experts' weights once more costs little beside.  Both products and the
+// sum, us, with their pairs / all apart: 128 experts of 2,048 x 768 682 / 710 and 722 / 725 at 400 rows an expert, 8 of 4,096 x 14,336 1,109 / 1,251 and
+// 1,123 / 1,302 at 380.
+static bool odd_may_go_apart(int odd, int n_blocks, int K) { return (long)odd * n_blocks < 512 && K <= 4096; }
 
 template <bool GLU>
 static bool launch_by_tile(const GroupedArgs& a, int tiles, const TileRun* runs, int max_pairs, hipStream_t stream) {
@@ -459,7 +472,7 @@ static bool launch_by_tile(const GroupedArgs& a, int tiles, const TileRun* runs,
     const long pairs = groups((tiles + 3l * odd) / 2 * wide_blocks) + 2 * GS_DIES;
     static_assert(PairShape::BM == 2 * GS_M && OddShape::BM == GS_M && HalfShape::BM == GS_M && HalfShape::LDS <= PairShape::LDS && OddShape::LDS <= PairShape::LDS && ShortShape::LDS <= PairShape::LDS &&
                       WIDE_OUT(GLU) == 2 * ODD_OUT(GLU), "");
-    auto kernel = odd_apart(odd, wide_blocks, a.K) ? grouped_gemm_pairs_kernel<GLU, true> : grouped_gemm_pairs_kernel<GLU, false>;
+    auto kernel = odd_may_go_apart(odd, wide_blocks, a.K) ? grouped_gemm_pairs_kernel<GLU, true> : grouped_gemm_pairs_kernel<GLU, false>;
     if (pairs >= (1l << 31) || hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PairShape::LDS) != hipSuccess)
       return false;
     hipLaunchKernelGGL(kernel, dim3((unsigned)pairs), dim3(256), PairShape::LDS, stream, a, runs, max_pairs, wide_blocks, odd_blocks);
@@ -535,6 +548,8 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(SortJobs jobs) {
   int* count = sh;
   int* first = sh + experts;
   int* first_pair = sh + 2 * experts;
+  __shared__ int shorts;
+  if (threadIdx.x == 0) shorts = 0;
   for (int e = threadIdx.x; e < experts; e += blockDim.x) count[e] = 0;
   for (int s = threadIdx.x; s < max_tiles * tm; s += blockDim.x) slot_pair[s] = slot_token[s] = -1;
   for (int t = threadIdx.x; t < max_tiles; t += blockDim.x) tile_group[t] = -1;
@@ -544,8 +559,8 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(SortJobs jobs) {
     if (e >= 0 && e < experts) atomicAdd(&count[e], 1);
   }
   __syncthreads();
+  int at = 0, twos = 0;
   if (threadIdx.x == 0) {
-    int at = 0, twos = 0;
     for (int e = 0; e < experts; ++e) {
       const int n = (count[e] + tm - 1) / tm;
       first[e] = at;
@@ -554,9 +569,14 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(SortJobs jobs) {
       twos += (n + 1) / 2;
     }
     tile_group[max_tiles] = at / tm;
-    jb.runs[0] = {twos, at / tm - twos, 2 * twos - at / tm, 0};
+  } else if (threadIdx.x >= TK_WAVE) {  // beside that: odd last tiles of few rows
+    for (int e = threadIdx.x - TK_WAVE; e < experts; e += blockDim.x - TK_WAVE) {
+      const int over = count[e] % (2 * tm);
+      if (over > 0 && over <= ShortShape::BM) atomicAdd(&shorts, 1);
+    }
   }
   __syncthreads();
+  if (threadIdx.x == 0) jb.runs[0] = {twos, at / tm - twos, 2 * twos - at / tm, shorts};
   for (int e = threadIdx.x; e < experts; e += blockDim.x) {
     const int t0 = first[e] / tm, n = (count[e] + tm - 1) / tm;
     for (int t = 0; t < n; ++t) tile_group[t0 + t] = e;
