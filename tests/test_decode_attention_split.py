@@ -60,7 +60,20 @@ def test_wavefronts_at_head_sizes_above_64(group, nkv, requests, keys, waves):
     assert got == waves and split % (32 * waves) == 0
 
 
-@pytest.mark.parametrize("head_dim,tiles,nkv,waves,even", [(64, 64, 8, 8, True), (64, 32, 16, 8, True), (64, 63, 8, 8, False), (64, 64, 8, 4, False), (64, 64, 8, 16, False),
+@pytest.mark.parametrize("head_dim,tiles,nkv,waves,even", [(64, 64, 8, 8, True), (64, 32, 16, 8, True), (64, 48, 8, 8, False), (64, 61, 8, 8, True), (64, 64, 8, 4, False), (64, 64, 8, 16, False),
                                                            (128, 64, 8, 8, False)])
 def test_even_parts_where_two_workgroups_of_eight_fill_a_unit(head_dim, tiles, nkv, waves, even):
-    assert ops.attention_even_parts(tiles, nkv, head_dim, waves) == even
+    assert ops.attention_even_parts(4096, tiles, nkv, head_dim, waves) == even
+
+
+@pytest.mark.parametrize("head_dim,nkv", [(32, 2), (64, 1), (64, 8), (128, 2), (128, 8)])
+@pytest.mark.parametrize("bound", [1024, 1100, 2048, 4096, 8192])
+def test_short_requests_are_summed_in_one_order(head_dim, nkv, bound):
+    """Of a step of some requests and of the recorded step that they are padded to: those of up to 64 keys in parts of 32, or in one part."""
+    def parts(n):
+        split, waves = ops.attention_split(bound, n, nkv, head_dim, 4)
+        even = ops.attention_even_parts(bound, n, nkv, head_dim, waves)
+        assert not even or waves >= 2  # (64 keys among two and more: 32 each)
+        return 32 if even else min(split // waves, 64)
+    for n in range(1, 129):
+        assert parts(n) == parts(ops.recorded_rows(n)), n

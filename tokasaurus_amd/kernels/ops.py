@@ -636,14 +636,16 @@ def attention_split(max_kv_len: int, n_tiles: int, nkv: int, head_dim: int = 64,
     return -(-raw // step) * step, waves
 
 
-def attention_even_parts(n_tiles: int, nkv: int, head_dim: int, waves: int) -> bool:
+def attention_even_parts(max_kv_len: int, n_tiles: int, nkv: int, head_dim: int, waves: int) -> bool:
     """Whether the wavefronts of a decoding workgroup share the keys that a request has in its split evenly; else each has a fixed part of the split,
     so that a request keeps as many wavefronts busy as it has keys and requests of all lengths end at one time.
+    Plans for up to 1,024 keys have parts of 32 for few requests and of 64 and more for others; even ones are 32 for a short request however many
+    there are, so that it is summed in one order in a step of 5 and in its recording, which has 8 (18 mixes at head size 64 in the mean as fast).
     Where two workgroups of eight fill a compute unit even parts are ahead: 396 mixes of 32 to 125 requests planned for 4,096 to 6,000 keys,
     head size 64, in the mean 3.3 %, 197 by 2 % and more (to 25 %), 19 behind by as much (at the worst 5 %, few long requests among short ones);
     64 of 380 to 3,000 keys fixed / even 53.5 / 49.8 us.  Of 246 mixes of all sizes, head sizes 64 and 128, 49 were ahead and 92 behind: 32 of 500 to
     4,000 planned for 4,096 58.7 / 62.7 at head size 128, 32 of 380 to 3,000 24.8 / 26.8, 48 of 280 to 2,236 29.4 / 32.3, 64 of 190 to 1,500 25.0 / 26.6 at 64."""
-    return head_dim <= 64 and waves == 8 and n_tiles * nkv >= 512
+    return max_kv_len <= 1024 or (head_dim <= 64 and waves == 8 and 512 <= recorded_rows(n_tiles) * nkv < 1024)
 
 
 # workgroups with and without keys that even cuts may take, where the planned ones take fewer: partial results of 33 MB at head size 128

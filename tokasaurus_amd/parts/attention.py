@@ -88,8 +88,8 @@ def attention_plan(ctx: StepContext, group: int, nkv: int, head_dim: int, page_s
                 lists.append((req, row0, None, 1, split, waves, 0, max(lengths)))
             else:
                 split, waves = ops.attention_split(bound, len(req), nkv, head_dim, group)
+                even = ops.attention_even_parts(bound, len(req), nkv, head_dim, waves)
                 lists.append((req, row0, None, 1, split, waves, 0, bound))
-            even = even or ops.attention_even_parts(len(req), nkv, head_dim, waves)
         # Portions that come after a past several times their own length walk far more keys a row than
         # whole prompts do: they are planned apart, or one of them among whole prompts would take a
         # form chosen for the many short walks and walk its long past on a few wavefronts.
