@@ -410,15 +410,15 @@ struct TileRun {
 // group's pairs, which read the same weights; or (APART, and where the numbers of pairs and odd tiles make it pay) the whole pairs come first and the
 // odd tiles, cut in two, behind them.  An expert's last tile often holds few rows: 2,048 tokens, 8 of 32 experts, are 512 rows an
 // expert give or take 20, so that half of the experts have a fifth tile of some 16.
-// It pays where it saves a round: a half of an odd tile takes some 0.65 of a pair's time, of up to 64 rows 0.35, and units that the last
+// It pays where it saves a round: a half of an odd tile counts 0.8 of a pair, of up to 64 rows 0.35, and units that the last
 // round of pairs leaves idle take them beside it.  Both products, beside / apart: 32 experts of 2,048 x 1,024 with 95 pairs and one odd tile (3.0
 // rounds with it, 3.0 without) 370 / 403 us, 66 and 13 (2.5, 2.1) 338 / 353, 87 and 18 (3.3, 2.7) 438 / 411, 128 and 8 (4.3, 4.0) 562 / 525; 16 of 2,048 x
 // 2,048 with 33 and 7 (2.5, 2.1) 321 / 341, 64 and 3 (4.2, 4.0) 530 / 470; 8 of 2,048 x 5,632 with 8 and 8 (2.8, 1.4) 318 / 355, 32 and 3 (6.0, 5.5) 726 / 695.
 __device__ __forceinline__ bool odd_tiles_apart(const TileRun& head, int n_blocks, int odd_blocks) {
   const int pairs = head.group * n_blocks, rounds = (pairs + 255) / 256;
-  const int odd = (13 * (head.first - head.tiles) + 7 * head.tiles) * odd_blocks;  // in twentieths of a pair
+  const int odd = (16 * (head.first - head.tiles) + 7 * head.tiles) * odd_blocks;  // in twentieths of a pair
   const int behind = max(odd - 20 * (256 * rounds - pairs), 0), beside = (head.tile * n_blocks + 255) / 256;
-  return rounds * 5120 + behind + 2880 < beside * 5120;  // (a round is 256 pairs; more than half of one is to be saved)
+  return rounds * 5120 + behind + 2560 < beside * 5120;  // (a round is 256 pairs; more than half of one is to be saved)
 }
 
 template <bool GLU, bool APART>

@@ -2753,11 +2753,12 @@ def experts_go_in_tiles(rows: int, top: int, dtype: torch.dtype, width: int, ff:
 # average, widths and inner sizes whose steps outweigh a tile's beginning and end, and so many elements of K that a compute unit walks in
 # gate and up: a round of pairs takes all units for one pair each, and a last round that is nearly empty costs as much as a full one.
 # In us by single tiles / in pairs, both products and the sum, experts' rows even, uneven (weights e^(0.5 N(0, 1))) and an eighth of the
-# experts 4.5 times as likely: 32 experts of 2,048 x 1,024, 420 rows an expert (4,380 elements) 338 / 242, 299 / 304, 294 / 303; 500
-# (5,020) 334 / 304, 337 / 307, 338 / 312; 700 444 / 336, 446 / 411, 452 / 410; 1,020 633 / 517, 630 / 524, 641 / 524.  16 of 2,048 x 2,048,
-# 420 rows 277 / 217, 290 / 304, 293 / 301; 500 329 / 310, 334 / 303, 327 / 309.  128 of 2,048 x 768, 400 rows 849 / 699, 835 / 738, 868 / 825.
-# 8 of 4,096 x 1,792, 460 rows (4,110) 262 / 185, 269 / 221, 281 / 305; 660 401 / 313, 363 / 319, 362 / 317.  8 of 4,096 x 14,336, 380 rows
-# 1,681 / 1,135, 1,702 / 1,149, 1,746 / 1,437.  64 of 1,024 x 512, 500 rows 191 / 222, 193 / 220, 193 / 220, 1,060 392 / 374, 379 / 381, 369 / 387.
+# experts 4.5 times as likely: 32 experts of 2,048 x 1,024, 320 rows an expert (3,580 elements) 254 / 236, 247 / 233, 262 / 233; 420 (4,380) 315 /
+# 256, 308 / 287, 317 / 302; 500 (5,020) 358 / 294, 343 / 322, 358 / 336; 700 460 / 370, 477 / 407, 479 / 412; 1,020 654 / 531, 657 / 566, 664 / 555.  16 of
+# 2,048 x 2,048, 420 rows 293 / 224, 289 / 273, 290 / 287; 500 334 / 269, 336 / 307, 343 / 306.  128 of 2,048 x 768, 400 rows 897 / 777, 887 / 820, 922 / 905.
+# 8 of 4,096 x 1,792, 460 rows (4,110) 275 / 195, 293 / 200, 279 / 251; 660 392 / 322, 377 / 319, 351 / 324.  8 of 4,096 x 14,336, 380 rows
+# 1,707 / 1,139, 1,753 / 1,425, 1,759 / 1,420.  64 of 1,024 x 512, 500 rows 239 / 236, 233 / 260, 235 / 261, 1,060 446 / 455, 437 / 464, 442 / 468.  (The line at 5,000
+# elements is from when odd tiles were always beside their pairs, 420 rows uneven 299 / 304; now that they go apart where it pays pairs are ahead below it.)
 EXPERT_PAIRS_FROM_ROWS = 320
 EXPERT_PAIRS_FROM_WIDTH = 2048
 EXPERT_PAIRS_FROM_INNER = 768
