@@ -318,6 +318,191 @@ __global__ __launch_bounds__(256) void gated_head_norm_kernel(const float* __res
     out[(size_t)unit * dv + i] = from_f32<T>(x[i] * rstd * w[i] * sigmoid_f32(g[i]));
 }
 
+// --------------------------------------------------------------------------
+// A step of single tokens (every request one, as many kv heads as heads): all of the above for a (head, request) in one workgroup, with
+// the bits of the three kernels, every sum in their order.  A column of the state is owned by DR_LANES lanes as above, a thread has
+// NC of them, DS_GROUPS apart; they are asked for in front of all else, so that the convolutions, norms and decays (a
+// channel a thread, through local memory) are made while the state is on its way.  What bounds it: two trips to memory, the convolution's
+// inputs and the state beside each other and the slot's number in front, and the state's bytes (128 KB read and
+// written a head of 128 x 128).  us a layer, 16 heads of 128 x 128, three kernels / this one, states from memory: 1 request 11.1 / 5.0, 8 requests
+// 21.6 / 7.2, 64 requests 67.5 / 35.2 (3.8 TB/s); 16 heads of 256 x 256, 8 requests 56.4 / 20.2; a decode step of 8 requests, eight layers, 735 / 635.
+// --------------------------------------------------------------------------
+#define DS_THREADS 1024
+#define DS_GROUPS (DS_THREADS / DR_LANES)
+#define DS_MAX 256  // dk, dv
+
+struct DeltaSingleArgs {
+  const void* proj;
+  int ld, col_b;
+  const float* a_pre;
+  int ld_a;
+  const float* conv_w;
+  int taps;
+  const float *a_log, *dt_bias;
+  float* state;
+  size_t state_stride, tail_off;
+  const int *q_start, *slots;
+  const float* gate;
+  int ld_gate;
+  const float* norm_w;
+  float eps;
+  void* out;
+  int H, dk, dv;
+};
+
+template <typename T, int NQ, int NC>
+__global__ __launch_bounds__(DS_THREADS) void delta_single_kernel(DeltaSingleArgs a) {
+  constexpr int DKP = NQ * DR_LANES * 4;
+  __shared__ __align__(16) float qs[DKP], ks[DKP], gs[DKP], vs[DS_MAX], os[DS_MAX], mul[2], beta;
+  const int h = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, dk = a.dk, dv = a.dv;
+  const int t = a.q_start[r];
+  if (a.q_start[r + 1] <= t) return;
+  const int lane = tid % DR_LANES, grp = tid / DR_LANES;
+  float* row = a.state + (size_t)a.slots[r] * a.state_stride;
+  float* s_at = row + (size_t)h * dv * dk;
+  float4 s[NC][NQ];
+#pragma unroll
+  for (int j = 0; j < NC; ++j)
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+      const int col = grp + j * DS_GROUPS, i = 4 * (lane + DR_LANES * n);
+      s[j][n] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (col < dv && i < dk) s[j][n] = *(const float4*)(s_at + (size_t)col * dk + i);
+    }
+  const T* x_row = (const T*)a.proj + (size_t)t * a.ld;
+  const int conv = 2 * dk + dv, C = a.H * conv;
+  for (int c = tid; c < conv + dk + 1; c += DS_THREADS) {
+    if (c < conv) {  // a channel of q, k or v through the convolution and silu, its tail moved on
+      const int which = c < dk ? 0 : (c < 2 * dk ? 1 : 2), x = c - which * dk;
+      const int ch = (which == 2 ? 2 * a.H * dk + h * dv : (which * a.H + h) * dk) + x;
+      float* tail = row + a.tail_off + ch;
+      const float* w = a.conv_w + (size_t)ch * a.taps;
+      const float own = to_f32<T>(x_row[ch]);
+      float acc = 0.f;
+      if (a.taps == 4) {  // (all of them asked for before the first is moved)
+        const float x0 = tail[0], x1 = tail[C], x2 = tail[2 * (size_t)C];
+        acc = fmaf(w[0], x0, acc);
+        acc = fmaf(w[1], x1, acc);
+        acc = fmaf(w[2], x2, acc);
+        acc = fmaf(w[3], own, acc);
+        tail[0] = x1;
+        tail[C] = x2;
+        tail[2 * (size_t)C] = own;
+      } else {
+        for (int j = 0; j < a.taps; ++j) {
+          const float in = j < a.taps - 1 ? tail[(size_t)j * C] : own;
+          acc = fmaf(w[j], in, acc);
+          if (j >= 1) tail[(size_t)(j - 1) * C] = in;
+        }
+      }
+      (which == 0 ? qs : (which == 1 ? ks : vs))[x] = silu_f32(acc);
+    } else if (c < conv + dk) {
+      const int x = c - conv;
+      const float rate = expf(a.a_log[h]);
+      gs[x] = expf(-rate * softplus_f32(a.a_pre[(size_t)t * a.ld_a + h * dk + x] + a.dt_bias[h * dk + x]));
+    } else {
+      beta = sigmoid_f32(to_f32<T>(x_row[a.col_b + h]));
+    }
+  }
+  if (tid < DKP - dk) qs[dk + tid] = ks[dk + tid] = gs[dk + tid] = 0.f;  // (lanes beyond the head's channels)
+  __syncthreads();
+  const int wave = tid / TK_WAVE, wl = tid % TK_WAVE;
+  if (wave < 2) {  // unit vectors; the queries also times dk^-1/2
+    const float* y = wave == 0 ? qs : ks;
+    float ss = 0.f;
+    for (int i = wl; i < dk; i += TK_WAVE) ss = fmaf(y[i], y[i], ss);
+    float m = 1.0f / sqrtf(wave_sum(ss) + 1e-6f);
+    if (wave == 0) m *= 1.0f / sqrtf((float)dk);
+    if (wl == 0) mul[wave] = m;
+  }
+  __syncthreads();
+  const float mq = mul[0], mk = mul[1], b = beta;
+  float4 q[NQ], k[NQ], g[NQ];
+#pragma unroll
+  for (int n = 0; n < NQ; ++n) {
+    const int i = lane + DR_LANES * n;
+    q[n] = ((const float4*)qs)[i];
+    k[n] = ((const float4*)ks)[i];
+    g[n] = ((const float4*)gs)[i];
+    q[n].x *= mq; q[n].y *= mq; q[n].z *= mq; q[n].w *= mq;
+    k[n].x *= mk; k[n].y *= mk; k[n].z *= mk; k[n].w *= mk;
+  }
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    const int col = grp + j * DS_GROUPS;
+    float dot[2] = {0.f, 0.f}, qd[2] = {0.f, 0.f}, kq[2] = {0.f, 0.f};
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+      float4& z = s[j][n];
+      z.x *= g[n].x; z.y *= g[n].y; z.z *= g[n].z; z.w *= g[n].w;
+      dot[0] = fmaf(k[n].x, z.x, dot[0]); dot[1] = fmaf(k[n].y, z.y, dot[1]);
+      dot[0] = fmaf(k[n].z, z.z, dot[0]); dot[1] = fmaf(k[n].w, z.w, dot[1]);
+      qd[0] = fmaf(q[n].x, z.x, qd[0]); qd[1] = fmaf(q[n].y, z.y, qd[1]);
+      qd[0] = fmaf(q[n].z, z.z, qd[0]); qd[1] = fmaf(q[n].w, z.w, qd[1]);
+      kq[0] = fmaf(q[n].x, k[n].x, kq[0]); kq[1] = fmaf(q[n].y, k[n].y, kq[1]);
+      kq[0] = fmaf(q[n].z, k[n].z, kq[0]); kq[1] = fmaf(q[n].w, k[n].w, kq[1]);
+    }
+    const float d = row_sum16(dot[0] + dot[1]), qsum = row_sum16(qd[0] + qd[1]), kqsum = row_sum16(kq[0] + kq[1]);
+    const float u = b * ((col < dv ? vs[col] : 0.f) - d);
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+      float4& z = s[j][n];
+      z.x = fmaf(k[n].x, u, z.x); z.y = fmaf(k[n].y, u, z.y); z.z = fmaf(k[n].z, u, z.z); z.w = fmaf(k[n].w, u, z.w);
+      const int i = 4 * (lane + DR_LANES * n);
+      if (col < dv && i < dk) *(float4*)(s_at + (size_t)col * dk + i) = z;
+    }
+    if (col < dv && lane == 0) os[col] = fmaf(u, kqsum, qsum);
+  }
+  __syncthreads();
+  if (wave > 0) return;
+  const float* gate = a.gate + (size_t)t * a.ld_gate + (size_t)h * dv;
+  float ss = 0.f;
+  for (int i = wl; i < dv; i += TK_WAVE) ss = fmaf(os[i], os[i], ss);
+  const float rstd = 1.0f / sqrtf(wave_sum(ss) / (float)dv + a.eps);
+  T* out = (T*)a.out + ((size_t)t * a.H + h) * dv;
+  for (int i = wl; i < dv; i += TK_WAVE) out[i] = from_f32<T>(os[i] * rstd * a.norm_w[i] * sigmoid_f32(gate[i]));
+}
+
+template <typename T, int NQ>
+static void launch_delta_single(const DeltaSingleArgs& a, int n_requests, hipStream_t stream) {
+  const dim3 grid(a.H, n_requests);
+  if (a.dv <= DS_GROUPS) hipLaunchKernelGGL((delta_single_kernel<T, NQ, 1>), grid, dim3(DS_THREADS), 0, stream, a);
+  else if (a.dv <= 2 * DS_GROUPS) hipLaunchKernelGGL((delta_single_kernel<T, NQ, 2>), grid, dim3(DS_THREADS), 0, stream, a);
+  else hipLaunchKernelGGL((delta_single_kernel<T, NQ, 4>), grid, dim3(DS_THREADS), 0, stream, a);
+}
+
+// Whether tk_delta_single takes these heads and this state: pieces of 16 bytes.
+TK_API int tk_delta_single_takes(int H, int G, int dk, int dv, const float* state, size_t state_stride) {
+  return H == G && dk > 0 && dk <= DS_MAX && dk % 4 == 0 && dv > 0 && dv <= DS_MAX && state_stride % 4 == 0 && ((uintptr_t)state & 15) == 0 ? 1 : 0;
+}
+
+// A step of one token a request: tk_delta_prepare, tk_delta_rule and tk_gated_head_norm in one launch (their arguments; out [tokens][H * dv]).
+TK_API int tk_delta_single(int dt, const void* proj, int ld, int col_b, const float* a_pre, int ld_a, const float* conv_w, int taps,
+                           const float* a_log, const float* dt_bias, float* state, size_t state_stride, size_t tail_off, const int* q_start,
+                           const int* slots, const float* gate, int ld_gate, const float* norm_w, float eps, void* out, int n_requests, int H,
+                           int dk, int dv, hipStream_t stream) {
+  TK_REQUIRE(n_requests >= 0 && n_requests < 65536 && H > 0 && tk_delta_single_takes(H, H, dk, dv, state, state_stride),
+             "delta_single: bad sizes requests=%d heads=%d dk=%d dv=%d", n_requests, H, dk, dv);
+  TK_REQUIRE(taps >= 1 && taps <= DR_MAX_TAPS, "delta_single: %d taps (1..%d)", taps, DR_MAX_TAPS);
+  const int C = H * (2 * dk + dv);
+  TK_REQUIRE(ld >= C && col_b >= 0 && col_b + H <= ld && ld_a >= H * dk && ld_gate >= H * dv, "delta_single: row strides %d, %d, %d too short", ld, ld_a, ld_gate);
+  TK_REQUIRE((size_t)H * dv * dk <= tail_off && tail_off + (size_t)(taps - 1) * C <= state_stride, "delta_single: the state row is too short");
+  if (n_requests == 0) return 0;
+  const DeltaSingleArgs a = {proj, ld, col_b, a_pre, ld_a, conv_w, taps, a_log, dt_bias, state, state_stride, tail_off, q_start, slots,
+                             gate, ld_gate, norm_w, eps, out, H, dk, dv};
+#define DS_CASE(T)                                                       \
+  do {                                                                   \
+    if (dk <= 64) launch_delta_single<T, 1>(a, n_requests, stream);      \
+    else if (dk <= 128) launch_delta_single<T, 2>(a, n_requests, stream); \
+    else launch_delta_single<T, 4>(a, n_requests, stream);               \
+  } while (0)
+  if (dt == TK_F32) DS_CASE(float);
+  else DS_CASE(bf16_t);
+#undef DS_CASE
+  TK_CHECK_LAUNCH("delta_single");
+  return 0;
+}
+
 // The tails of `C` channels moved on by the step's rows (after whoever reads the old ones).
 TK_API int tk_delta_tail(int dt, const void* proj, int ld, int taps, float* state, size_t state_stride, size_t tail_off,
                          const int* q_start, const int* slots, int n_requests, int C, hipStream_t stream) {

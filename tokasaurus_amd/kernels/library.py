@@ -85,6 +85,9 @@ _SIGNATURES: dict[str, dict[str, list]] = {
         "tk_delta_tail": [c_int, _P, c_int, c_int, _P, c_size_t, c_size_t, _P, _P, c_int, c_int, _P],
         "tk_delta_chunks": [c_int, _P, c_int, c_int, _P, c_int, _P, c_int, _P, _P, _P, c_size_t, c_size_t, _P, _P, _P, _P, _P, _P, _P]
         + [c_int] * 6 + [_P],
+        "tk_delta_single_takes": [c_int] * 4 + [_P, c_size_t],
+        "tk_delta_single": [c_int, _P, c_int, c_int, _P, c_int, _P, c_int, _P, _P, _P, c_size_t, c_size_t, _P, _P, _P, c_int, _P, c_float, _P]
+        + [c_int] * 4 + [_P],
         "tk_delta_chunk_tokens": [],
         "tk_delta_chunk_words": [c_int, c_int],
         "tk_gated_head_norm": [c_int, _P, _P, c_int, _P, c_float, _P, c_int, c_int, c_int, _P],

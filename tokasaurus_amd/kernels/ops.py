@@ -2480,6 +2480,33 @@ def delta_rule(rec: torch.Tensor, state: torch.Tensor, q_start: torch.Tensor, sl
     return o
 
 
+def delta_single_takes(tokens: int, slots: torch.Tensor, heads: int, kv_heads: int, key_dim: int, value_dim: int, state: torch.Tensor) -> bool:
+    """Whether ``delta_single`` takes a step: one token a request, as many kv heads as heads, state rows in pieces of 16 bytes."""
+    return tokens == slots.numel() and bool(load("core").tk_delta_single_takes(heads, kv_heads, key_dim, value_dim, state.data_ptr(), state.stride(0)))
+
+
+def delta_single(proj: torch.Tensor, col_b: int, a_pre: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor,
+                 state: torch.Tensor, q_start: torch.Tensor, slots: torch.Tensor, gate: torch.Tensor, weight: torch.Tensor, eps: float,
+                 heads: int, key_dim: int, value_dim: int, out_dtype: torch.dtype) -> torch.Tensor:
+    """A step of one token a request: ``gated_head_norm(delta_rule(delta_prepare(..)), gate, ..)`` in one kernel, with its bits.
+    [tokens, heads * value_dim] of ``out_dtype``, the rows' own type."""
+    _gpu(proj, a_pre, conv_w, a_log, dt_bias, state, q_start, slots, gate, weight)
+    n, taps = _check_delta(proj, a_pre, conv_w, a_log, dt_bias, state, q_start, slots, heads, heads, key_dim, value_dim)
+    _need(n == slots.numel() and out_dtype == proj.dtype, "delta_single: one token a request, the result of the rows' type")
+    _need(gate.shape == (n, heads * value_dim) and gate.dtype == torch.float32 and gate.stride(1) == 1,
+          "delta_single: the gate must be float32 [tokens, heads * value_dim] with unit inner stride")
+    _f32_vector(weight, value_dim, "delta_single: the norm's weight")
+    _need(0 <= col_b and col_b + heads <= proj.shape[1], "delta_single: the write strengths lie outside the rows")
+    out = torch.empty((n, heads * value_dim), dtype=out_dtype, device=proj.device)
+    if n:
+        one = n == 1  # (a single row's stride says nothing)
+        call("tk_delta_single", dtype_code(proj.dtype), proj.data_ptr(), max(proj.stride(0), proj.shape[1]) if one else proj.stride(0), int(col_b),
+             a_pre.data_ptr(), heads * key_dim if one else a_pre.stride(0), conv_w.data_ptr(), taps, a_log.data_ptr(), dt_bias.data_ptr(),
+             state.data_ptr(), state.stride(0), heads * key_dim * value_dim, q_start.data_ptr(), slots.data_ptr(), gate.data_ptr(),
+             heads * value_dim if one else gate.stride(0), weight.data_ptr(), float(eps), out.data_ptr(), n, heads, key_dim, value_dim, _stream())
+    return out
+
+
 def gated_head_norm(o: torch.Tensor, gate: torch.Tensor, weight: torch.Tensor, eps: float, heads: int, value_dim: int,
                     out_dtype: torch.dtype) -> torch.Tensor:
     """Every head's ``value_dim`` numbers divided by their root mean square, times ``weight``

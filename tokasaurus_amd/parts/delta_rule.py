@@ -124,6 +124,10 @@ class ChannelDeltaRule(Mixer):
         low = self.low(self._columns(proj, self.col_a1, self.decay_rank + self.gate_rank), out_f32=True)
         a_pre, gate = low[:, : H * dk], low[:, H * dk :]  # 32-bit, rows a stride apart
         size, few = self._chunks(ctx)
+        if ctx.max_q_len == 1 and h.dtype == proj.dtype and ops.delta_single_takes(proj.shape[0], ctx.slots, H, G, dk, dv, state):
+            y = ops.delta_single(proj, self.col_b, a_pre, self.conv_w, self.a_log, self.dt_bias, state, ctx.q_start, ctx.slots, gate,
+                                 self.norm_w, self.norm_eps, H, dk, dv, h.dtype)
+            return y if rows is None else ops.gather_rows(y, rows)
         if size:
             least = ops.DELTA_CHUNKS_FROM
             o = ops.delta_rule_chunks(proj, self.col_b, a_pre, self.conv_w, self.a_log, self.dt_bias, state, ctx.q_start,
