@@ -75,8 +75,27 @@ __device__ __forceinline__ void gf_store(const GemmF32Args& a, f4 v, int token, 
 // all, rows of 32 and 64 KB keep to few of the memory's channels (us together / apart: 2,048 x 8,192 19.4 / 15.0 at 1 token, 19.4 / 15.4 at 4,
 // 2,048 x 16,384 29.9 / 24.0 and 30.2 / 26.5, 2,048 x 11,008 21.4 / 19.9 and 22.0 / 20.6, else within 2 %).  One order for all rows up to 8, whatever
 // their number: a step of 3 rows is recorded with 4.
-template <bool HALVES>
-__global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a, int KS, int share, int spare) {
+//
+// What a step of few rows would launch a kernel for behind the product (4 rows of the 1B shape: rotation and append 4.9 us, activation 4.6,
+// each little more than a launch and a trip to memory) is done where the results pass anyway:
+// EPI = FEW_GLU: W is [gate | up], 8 rows of each a workgroup, so that a gate and its up lie 32 lanes apart: silu(gate) * up.
+// EPI = FEW_ROPE: W is [q | k | v] by heads, a workgroup's rows are 8 elements of a head and the 8 half a head on, which the
+//   rotation pairs: q turned to its rows, k turned and v as it is to their pages.
+// (The norm in front of a product does not pay here: its weight is a third load beside those of A and W, in every workgroup; gate and
+// up with the norm folded in 31.9 us for 26.2 and the norm's own 4.5, the head 209 for 182.)
+enum { FEW_STORE = 0, FEW_GLU = 1, FEW_ROPE = 2 };
+struct FewExtra {
+  // FEW_ROPE: positions and requests of the rows, the requests' pages, cosines and sines [positions][d / 2] (null: no rotation)
+  const int *positions, *token_req, *block_table;
+  int table_stride;
+  const float *cos, *sin;
+  float *kcache, *vcache;
+  int nq, nkv, d, P;
+};
+
+template <bool HALVES, int EPI>
+__global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a, FewExtra more, int KS, int share, int spare) {
+  static_assert(!HALVES || EPI == FEW_STORE, "");
   extern __shared__ __align__(16) f4 sums[];  // [wavefronts - 1][64]
   // every argument that a first load needs, in one trip
   asm volatile("" ::"s"(a.A), "s"(a.W), "s"(a.lda), "s"(a.M), "s"(a.N), "s"(a.K), "s"(KS), "s"(share), "s"(spare));
@@ -91,7 +110,19 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a, int KS
   // (the last wavefronts take one block more, so that a block that K cuts lies behind whole sets: 4 tokens, 2,048 x
   // 2,056 9.2 / 8.1 us, 1 token 8.6 / 7.5)
   const int b0 = kw * share + max(kw - (KS - spare), 0), b1 = b0 + share + (kw >= KS - spare ? 1 : 0);
-  const float* wp = a.W + (size_t)min(n0 + own, a.N - 1) * a.K + from + 4 * q;
+  // (FEW_GLU, FEW_ROPE: a.N outputs in pairs, of which a workgroup has 8)
+  int w_row = min(n0 + own, a.N - 1), first = 0, head = 0;
+  if (EPI == FEW_GLU) {
+    first = blockIdx.x * 8;
+    w_row = min(first + (r & 7), a.N / 2 - 1) + (r >> 3) * (a.N / 2);
+  }
+  if (EPI == FEW_ROPE) {
+    const int each = more.d >> 4;
+    head = blockIdx.x / each;
+    first = (blockIdx.x - head * each) * 8;
+    w_row = head * more.d + first + (r & 7) + (r >> 3) * (more.d >> 1);
+  }
+  const float* wp = a.W + (size_t)w_row * a.K + from + 4 * q;
   const float* ap = a.A + (size_t)min(own, a.M - 1) * a.lda + from + 4 * q;
   f4 acc[GF_UNROLL][4];
 #pragma unroll
@@ -162,7 +193,53 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a, int KS
 #pragma unroll
     for (int j = 0; j < 4; ++j) sum[j] += __shfl(sum[j], (lane + 40) & 63, 64);
   }
-  if (r < min(a.M, ROWS) && 4 * q < ROWS && n0 + 4 * q < a.N) gf_store(a, sum, r, n0 + 4 * q);
+  if (EPI == FEW_STORE) {
+    if (r < min(a.M, ROWS) && 4 * q < ROWS && n0 + 4 * q < a.N) gf_store(a, sum, r, n0 + 4 * q);
+    return;
+  }
+  f4 other;  // lanes of the first 8 rows: their partners
+  if (a.bias) {
+    const int n = EPI == FEW_GLU ? (q >> 1) * (a.N / 2) + first + 4 * (q & 1) : head * more.d + (q >> 1) * (more.d >> 1) + first + 4 * (q & 1);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (EPI == FEW_ROPE || first + 4 * (q & 1) + j < a.N / 2) sum[j] += a.bias[n + j];
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) other[j] = __shfl_xor(sum[j], 32, 64);
+  if (r >= a.M) return;
+  if (EPI == FEW_GLU) {
+    const int n = first + 4 * q;
+    if (q >= 2) return;
+    float* c = a.C + (size_t)r * a.ldc + n;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (n + j < a.N / 2) c[j] = sum[j] / (1.0f + expf(-sum[j])) * other[j];
+    return;
+  }
+  const int pos = more.positions[r], pair = first + 4 * (q & 1), e = pair + (q >> 1) * (more.d >> 1);
+  f4 o = sum;
+  if (head < more.nq + more.nkv && more.cos) {
+    const f4 cs = *(const f4*)(more.cos + (size_t)pos * (more.d >> 1) + pair), sn = *(const f4*)(more.sin + (size_t)pos * (more.d >> 1) + pair);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float u = q < 2 ? sum[j] : other[j], v = q < 2 ? other[j] : sum[j];
+      rotate_pair(u, v, cs[j], sn[j], u, v);
+      o[j] = q < 2 ? u : v;
+    }
+  }
+  if (head < more.nq) {
+    *(f4*)(a.C + (size_t)r * a.ldc + head * more.d + e) = o;
+    return;
+  }
+  const size_t page = more.block_table[(size_t)more.token_req[r] * more.table_stride + pos / more.P];
+  const int p = pos % more.P;
+  if (head < more.nq + more.nkv) {
+    *(f4*)(more.kcache + (page * more.nkv + head - more.nq) * key_page_elems(more.P, more.d) + key_offset(more.P, p, e)) = o;
+  } else {
+    float* v = more.vcache + (page * more.nkv + head - more.nq - more.nkv) * more.P * more.d;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[value_offset(more.d, p, e + j)] = o[j];
+  }
 }
 
 // The chains of a tile's sums added, and the results stored, or the part of K among the other parts' sums.
@@ -406,6 +483,25 @@ static bool gf_launch(const GemmF32Args& a, int cuts, hipStream_t stream) {
   return true;
 }
 
+template <int EPI>
+static void gf_launch_few(const GemmF32Args& a, const FewExtra& x, hipStream_t stream) {
+  // (2, 4, 8 wavefronts at 4 tokens, 2 048 x 2 048: 9.0, 8.2, 9.0 us, 2 048 x 8 192: 34, 25, 26, 16 384 x 2 048: 33, 30, 30)
+  const int KS = a.K < 64 ? 1 : (a.K < 4096 ? 4 : 8);
+  const size_t lds = (KS - 1) * 64 * sizeof(f4);
+  if constexpr (EPI == FEW_STORE) {
+    // rows of 8 where rows of 16 leave compute units without a workgroup
+    if (a.M <= 8 && a.K % 32 == 0 && a.K >= 256 && a.N <= GF_HALVES_ROWS) {
+      const int blocks = a.K / 32;
+      hipLaunchKernelGGL((gemm_f32_few_kernel<true, FEW_STORE>), dim3((a.N + 7) / 8), dim3(64 * KS), lds, stream, a, x, KS, blocks / KS, blocks % KS);
+      return;
+    }
+  }
+  const int blocks = (a.K + 15) / 16;
+  // (pairs of rows: 8 a workgroup, of a head or of gate and up)
+  const int groups = EPI == FEW_STORE ? (a.N + 15) / 16 : (EPI == FEW_GLU ? (a.N / 2 + 7) / 8 : a.N / 16);
+  hipLaunchKernelGGL((gemm_f32_few_kernel<false, EPI>), dim3(groups), dim3(64 * KS), lds, stream, a, x, KS, blocks / KS, blocks % KS);
+}
+
 TK_API int tk_gemm_f32(const void* A, int lda, const void* W, void* C, int ldc, const void* residual, int ldr,
                        const void* bias, int M, int N, int K, int cuts, void* part, hipStream_t stream) {
   TK_REQUIRE(M >= 0 && N > 0 && K > 0 && lda >= K && ldc >= N, "gemm_f32: bad sizes M=%d N=%d K=%d lda=%d ldc=%d", M, N, K, lda, ldc);
@@ -417,14 +513,7 @@ TK_API int tk_gemm_f32(const void* A, int lda, const void* W, void* C, int ldc, 
   GemmF32Args a = {(const float*)A, lda, (const float*)W, (float*)C, ldc, (const float*)residual, ldr, (const float*)bias, M, N, K,
                    cuts > 1 ? (float*)part : nullptr};
   if (M <= 16) {
-    // (2, 4, 8 wavefronts at 4 tokens, 2 048 x 2 048: 9.0, 8.2, 9.0 us, 2 048 x 8 192: 34, 25, 26, 16 384 x 2 048: 33, 30, 30)
-    const int KS = K < 64 ? 1 : (K < 4096 ? 4 : 8);
-    // rows of 8 where rows of 16 leave compute units without a workgroup
-    const bool halves = M <= 8 && K % 32 == 0 && K >= 256 && N <= GF_HALVES_ROWS;
-    const int blocks = halves ? K / 32 : (K + 15) / 16;
-    auto few = halves ? gemm_f32_few_kernel<true> : gemm_f32_few_kernel<false>;
-    const int rows = halves ? 8 : 16;
-    hipLaunchKernelGGL(few, dim3((N + rows - 1) / rows), dim3(64 * KS), (KS - 1) * 64 * sizeof(f4), stream, a, KS, blocks / KS, blocks % KS);
+    gf_launch_few<FEW_STORE>(a, FewExtra{}, stream);
     TK_CHECK_LAUNCH("gemm_f32");
     return 0;
   }
@@ -437,5 +526,26 @@ TK_API int tk_gemm_f32(const void* A, int lda, const void* W, void* C, int ldc, 
   TK_REQUIRE(ok, "gemm_f32: M=%d N=%d take too many workgroups, or their local memory could not be reserved", M, N);
   if (cuts > 1) hipLaunchKernelGGL(gemm_f32_sum_kernel, dim3((N / 4 + 255) / 256, M), dim3(256), 0, stream, a, cuts);
   TK_CHECK_LAUNCH("gemm_f32");
+  return 0;
+}
+
+// Few rows (up to 16) with what stands behind the product.  glu: W is [gate | up] and C takes silu(gate) * up, [M, N / 2].  Else W is
+// [q | k | v] by heads of d elements, C takes the turned queries [M, nq * d], keys and values go to the pages; cos and sin may be
+// null: no rotation.
+TK_API int tk_gemm_f32_few(const void* A, int lda, const void* W, void* C, int ldc, const void* bias, int M, int N, int K, int glu,
+                           const int* positions, const int* token_req, const int* block_table, int table_stride, const float* cos,
+                           const float* sin, float* kcache, float* vcache, int nq, int nkv, int d, int P, hipStream_t stream) {
+  TK_REQUIRE(M > 0 && M <= 16 && N > 0 && K > 0 && lda >= K, "gemm_f32_few: bad sizes M=%d N=%d K=%d lda=%d", M, N, K, lda);
+  TK_REQUIRE(tk_gemm_f32_takes(A, lda, W, K), "gemm_f32_few: rows of A and W must start at multiples of 16 bytes");
+  TK_REQUIRE(!glu || (N % 2 == 0 && ldc >= N / 2), "gemm_f32_few: gate and up of %d rows, result rows of %d", N, ldc);
+  TK_REQUIRE(glu || (positions && token_req && block_table && kcache && vcache && nq > 0 && nkv > 0 && d > 0 && d % 16 == 0 && P > 0 &&
+                     N == (nq + 2 * nkv) * d && ldc >= nq * d && ldc % 4 == 0 && !cos == !sin &&
+                     (((uintptr_t)C | (uintptr_t)cos | (uintptr_t)sin | (uintptr_t)kcache) & 15) == 0),
+             "gemm_f32_few: rotation and append of %d + 2 x %d heads of %d from %d outputs", nq, nkv, d, N);
+  const GemmF32Args a = {(const float*)A, lda, (const float*)W, (float*)C, ldc, nullptr, 0, (const float*)bias, M, N, K, nullptr};
+  const FewExtra x = {positions, token_req, block_table, table_stride, cos, sin, kcache, vcache, nq, nkv, d, P};
+  if (glu) gf_launch_few<FEW_GLU>(a, x, stream);
+  else gf_launch_few<FEW_ROPE>(a, x, stream);
+  TK_CHECK_LAUNCH("gemm_f32_few");
   return 0;
 }

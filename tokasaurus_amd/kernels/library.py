@@ -33,6 +33,7 @@ _SIGNATURES: dict[str, dict[str, list]] = {
         "tk_gemm_generic": [c_int, _P, c_int, _P, _P, c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, _P],
         "tk_gemm_f32": [_P, c_int, _P, _P, c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, _P, _P],
         "tk_gemm_f32_takes": [_P, c_int, _P, c_int],
+        "tk_gemm_f32_few": [_P, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, _P, _P, _P, c_int, _P, _P, _P, _P] + [c_int] * 4 + [_P],
         "tk_gemm_f32_cuts": [c_int, c_int, c_int],
         "tk_add_bias": [c_int, _P, _P, c_int, c_int, _P],
         "tk_head_rmsnorm": [c_int, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, c_float, _P],

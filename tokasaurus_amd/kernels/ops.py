@@ -1170,6 +1170,56 @@ def gemm_skinny_bf16(
     return (out, emitted) if emit_weight is not None else out
 
 
+FEW_F32_ROWS = 16  # rows of the 32-bit few-row product, which reads its weight once
+
+
+def few_f32_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``gemm_f32_few`` takes this product: up to ``FEW_F32_ROWS`` 32-bit rows that start at multiples of 16 bytes."""
+    return (x.dtype == w.dtype == torch.float32 and 0 < x.shape[0] <= FEW_F32_ROWS and x.stride(1) == 1 and x.shape[1] % 4 == 0
+            and x.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.is_contiguous())
+
+
+def few_f32_ropes(rope: RopeAppend) -> bool:
+    """Whether ``gemm_f32_few`` rotates and appends for these heads: whole heads of a multiple of 16, 32-bit pages and tables."""
+    tables = [t for t in (rope.cos, rope.sin) if t is not None]
+    return (rope.head_dim % 16 == 0 and (rope.rotary_dim is None or rope.rotary_dim == rope.head_dim) and rope.nkv > 0
+            and rope.kcache.dtype == rope.vcache.dtype == torch.float32 and rope.kcache.data_ptr() % 16 == 0 and len(tables) != 1
+            and all(t.dtype == torch.float32 and t.is_contiguous() and t.shape[1] == rope.head_dim // 2 and t.data_ptr() % 16 == 0 for t in tables))
+
+
+def gemm_f32_few(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, rope: RopeAppend | None = None) -> torch.Tensor:
+    """Few 32-bit rows x [M, K] . w [N, K]^T (+ bias), the sums of ``gemm_generic``, and what stands behind the product in its kernel:
+    with ``rope`` w is [q | k | v] by heads, q and k are turned, k and v appended to their pages, the result is q [M, nq * d];
+    without, w is [gate | up] and the result silu(gate) * up."""
+    _gpu(x, w, bias)
+    _check_bias(bias, w, "gemm_f32_few")
+    _need(x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and few_f32_takes(x, w),
+          f"gemm_f32_few: x {tuple(x.shape)} {x.dtype} and w {tuple(w.shape)} {w.dtype} must be up to {FEW_F32_ROWS} 32-bit rows and a contiguous "
+          "weight at multiples of 16 bytes")
+    (m, k), n = x.shape, w.shape[0]
+    _need(n % 2 == 0, "gemm_f32_few: gate and up are halves of the weight")
+    pointers: list = [None] * 3 + [0] + [None] * 4 + [0] * 4
+    width = n // 2
+    if rope is not None:
+        r = rope
+        _gpu(r.positions, r.token_req, r.block_table, r.cos, r.sin, r.kcache, r.vcache)
+        for t, name in ((r.positions, "positions"), (r.token_req, "token_req"), (r.block_table, "block_table")):
+            _i32(t, name)
+        _need(n == (r.nq + 2 * r.nkv) * r.head_dim and few_f32_ropes(r) and (r.cos is None or r.cos.shape == r.sin.shape),
+              "gemm_f32_few: W is not [q | k | v] of these heads, or tables and pages are not as the kernel reads them")
+        _need(r.positions.numel() == m and r.token_req.numel() == m and r.block_table.dim() == 2,
+              "gemm_f32_few: positions/token_req need one entry a row, block_table [requests, width]")
+        _check_pages(r.kcache, r.vcache, r.nkv, r.page_size, r.head_dim, torch.float32, "gemm_f32_few")
+        pointers = [r.positions.data_ptr(), r.token_req.data_ptr(), r.block_table.data_ptr(), r.block_table.stride(0),
+                    r.cos.data_ptr() if r.cos is not None else None, r.sin.data_ptr() if r.sin is not None else None,
+                    r.kcache.data_ptr(), r.vcache.data_ptr(), r.nq, r.nkv, r.head_dim, r.page_size]
+        width = r.nq * r.head_dim
+    out = torch.empty((m, width), dtype=torch.float32, device=x.device)
+    call("tk_gemm_f32_few", x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), width, bias.data_ptr() if bias is not None else None, m, n, k,
+         0 if rope is not None else 1, *pointers, _stream())
+    return out
+
+
 # --------------------------------------------------------------------------
 # bfloat16 products with K cut among workgroups, and the passes that add the cuts
 # --------------------------------------------------------------------------

@@ -6,7 +6,8 @@ may be stacked along the output rows into one product (q|k|v, gate|up).  The bia
 to the 32-bit sums, before the product is rounded.
 
 Which kernel runs is decided by the storage type and the number of rows:
-  * float32: 32-bit multiply-adds throughout (the true 32-bit path), on the matrix cores where the sizes fit them;
+  * float32: 32-bit multiply-adds throughout (the true 32-bit path), on the matrix cores where the sizes fit them; up to 16
+    rows (``ops.gemm_f32_few``) with the activation, or the rotation and append, in the same kernel;
   * bfloat16, few rows (decode; how many depends on the inner size, ``ops.skinny_rows``, and ``ops.glu_rows`` for gate and
     up): the hand-written matrix-core kernels that stream the weight once and fuses the epilogue; it can also fold in the
     norm in front (``Normed`` input), leave what the norm behind it needs
@@ -197,6 +198,8 @@ class Linear:
                 # few-row kernel and in the pass that adds and norms (and as the reference's separate add)
                 return ops.add(prod, residual.contiguous())
             return gated(prod) if swiglu else prod
+        if swiglu and glu is None and residual is None and not out_f32 and w.shape[0] % 2 == 0 and ops.few_f32_takes(x, w):
+            return ops.gemm_f32_few(x, w, bias)  # few 32-bit rows: the activation is part of the product's kernel
         # the 32-bit path, and few bfloat16 rows of a width the matrix-core kernel does not take
         prod = ops.gemm_generic(x, w, residual=residual, out_f32=out_f32, out=out, bias=bias)
         return gated(prod) if swiglu else scaled(prod)
@@ -236,6 +239,11 @@ class Linear:
             if q is not None:
                 return q
             x = rows
+        if self.weight.dtype == torch.float32:
+            if not (0 < m <= ops.FEW_F32_ROWS and ops.few_f32_ropes(rope)):
+                return None
+            x = x.materialize() if isinstance(x, Normed) else x
+            return ops.gemm_f32_few(x, self.weight, self.bias, rope) if ops.few_f32_takes(x, self.weight) else None
         most = min(ops.SKINNY_ROPE_ROWS, 2 * ops.skinny_rows(self.in_features, paired=True))
         fits = self.weight.dtype == torch.bfloat16 and 0 < m <= most and self._aligned()
         if not fits or rope.head_dim % 2 or (rope.rotary_dim is not None and rope.rotary_dim != rope.head_dim):
