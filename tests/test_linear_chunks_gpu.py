@@ -1,0 +1,51 @@
+"""Linear attention in chunks against the recurrence: numbers of chunks around those whose operands are on their way at a time, blocks of
+columns shared out over several workgroups and over one, key heads of one slab to four."""
+
+import pytest
+import torch
+
+from tokasaurus_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def plan(lengths):
+    req, row0, first, at = [], [], [0], 0
+    for r, n in enumerate(lengths):
+        rows = range(at, at + n, ops.linear_attention_chunk_tokens())
+        req, row0, at = req + [r] * len(rows), row0 + list(rows), at + n
+        first.append(len(req))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    return ops.ChunkPlan(i32(req), i32(row0), i32(first))
+
+
+@pytest.mark.parametrize("heads,dk,dv,lengths", [(2, 128, 144, [64 * 4, 64 * 5 + 1, 64 * 6 - 1]), (1, 64, 16, [64 * 11]), (3, 200, 33, [33, 64 * 10]),
+                                                 (1, 256, 130, [64 * 5, 1, 40]), (16, 20, 128, [64 * 3 + 7] * 9)])
+@pytest.mark.parametrize("memory", [False, True])
+def test_chunks_follow_the_recurrence(heads, dk, dv, lengths, memory):
+    g = torch.Generator(device="cuda").manual_seed(dk + dv)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    n, R, off = sum(lengths), len(lengths), heads * (2 * dk + dv)
+    proj, before = rand(n, off + max(2 * heads, 16)), rand(R + 1, ops.linear_attention_state_words(heads, dk, dv, memory)) * 0.3
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    starts, slots = i32([sum(lengths[:i]) for i in range(R + 1)]), i32(range(R, 0, -1))
+    up, bias, i_bias, f_bias = rand(16, heads * dk) * 0.3, rand(heads * dk), rand(heads), rand(heads) + 2
+
+    def run(chunks):
+        state = before.clone()
+        if memory:
+            positions = torch.cat([torch.arange(m) for m in lengths]).int().cuda()
+            o, _ = ops.matrix_memory(proj, 0, heads * dk, 2 * heads * dk, off, off + heads, i_bias, f_bias, 15.0, dk ** -0.5, state, starts, slots,
+                                     positions, heads, dk, dv, max(lengths), chunks=chunks)
+            o = o.view(n, heads, -1)[..., : dv + 1]
+        else:
+            o = ops.gated_linear_attention(proj, 0, heads * dk, 2 * heads * dk, off, up, bias, 16.0, dk ** -0.5, state, starts, slots, heads, dk, dv,
+                                           max(lengths), chunks=chunks)
+        return o, state
+
+    (o, state), (want_o, want_state) = run(plan(lengths)), run(None)
+    rel = lambda x, y: float((x.double() - y.double()).norm() / y.double().norm())  # noqa: E731
+    # the same terms in two orders: a decay's exponent is a sum of up to 64 logarithms of about one each in one of them (64 roundings of
+    # 2^-24 of up to 64), a product of as many factors in the other
+    assert rel(o, want_o) <= 64 * 2.0 ** -24 and rel(state[1:], want_state[1:]) <= 64 * 2.0 ** -24
+    assert torch.equal(state[0], before[0])

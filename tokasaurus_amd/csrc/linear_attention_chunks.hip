@@ -11,10 +11,17 @@
 // diagonal the second exponent is positive; where it stays below LC_REACH in every channel (the decays of 16 tokens leave
 // more than 2^-LC_REACH) both factors and their product are numbers as good as any, else the block is summed pair by pair.
 //
-// Two kernels.  The first works on all (chunk, head) at once: decays, their sums, and the factors of the products above, in
-// `rec`.  The second walks a request's chunks for 16 columns of a head's state in a workgroup: per chunk two products on what
-// the first has left and one update of S, which stays in registers and goes round through LDS.
+// Three kernels.  The first works on all (chunk, head) at once: decays, their sums, and the factors of the products above, in
+// `rec`.  The second walks a request's chunks for a tile of 16 x 16 of a head's state in a wavefront, and leaves the state in front
+// of every chunk in `rec`.  The third makes the results from those, all (chunk, head) at once.
+// The walk is the only chain, and it is as short as it can be: 16 products a chunk.  Walked together with the results (one kernel, 16 columns of
+// a head a workgroup, the state handed round through local memory) a chunk took 2.3 us on as few workgroups as a prompt has heads and
+// blocks of columns.  us, all kernels of a layer, walked together / apart, heads of 128 x 128: LA_MEMORY, 8 heads: 2,048 tokens 95 / 52, 8,192 tokens
+// 329 / 165, 300 and 1,200 tokens 66 / 49, 100 tokens 20 / 19, six of 500 66 / 67; LA_CHANNEL, 16 heads: 114 / 75, 462 / 334, 87 / 73, 35 / 28, four
+// of 500 88 / 80; 4 heads of 256 x 256, 1,000 tokens 121 / 61.
 #include "linear_attention.h"
+#include <algorithm>
+#include <type_traits>
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
@@ -29,15 +36,22 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float lc_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// What a (chunk, head) leaves in `rec`: the factors of q and of k, P, and the decay of S over the chunk [dkp].  The first three
-// lie as the lanes of the second kernel read them, 64 lanes' four numbers side by side: lane 16 c + col of block
+// What a (chunk, head) leaves in `rec`: the factors of q and of k, P, the decay of S over the chunk [dkp], the state in front of the chunk
+// and the values (with ones in the column that sums the keys).  All but the decay lie as the lanes of the second and third kernel
+// read them, 64 lanes' four numbers side by side: lane 16 c + col of block
 //     q [w][m]   has token 16 w + col, channels 16 m + 4 c + e
 //     k [n][T]   has channel 16 n + col, tokens 16 T + 4 c + e
 //     P [w][T]   has token 16 w + col, tokens s = 16 T + 4 c + e
-__host__ __device__ __forceinline__ size_t lc_words(int dkp) { return (size_t)2 * LC_CHUNK * dkp + LC_CHUNK * LC_CHUNK + dkp; }
+//     S [z][m]   has column 16 z + col, rows 16 m + 4 c + e
+//     v [z][T]   has column 16 z + col, tokens 16 T + 4 c + e
 __host__ __device__ __forceinline__ size_t lc_k_at(int dkp) { return (size_t)LC_CHUNK * dkp; }
 __host__ __device__ __forceinline__ size_t lc_p_at(int dkp) { return (size_t)2 * LC_CHUNK * dkp; }
 __host__ __device__ __forceinline__ size_t lc_d_at(int dkp) { return lc_p_at(dkp) + LC_CHUNK * LC_CHUNK; }
+__host__ __device__ __forceinline__ size_t lc_s_at(int dkp) { return lc_d_at(dkp) + dkp; }
+__host__ __device__ __forceinline__ size_t lc_v_at(int dkp, int blocks) { return lc_s_at(dkp) + (size_t)dkp * 16 * blocks; }
+__host__ __device__ __forceinline__ size_t lc_words(int dkp, int blocks) { return lc_v_at(dkp, blocks) + (size_t)LC_CHUNK * 16 * blocks; }
+template <int MODE>
+__host__ __device__ __forceinline__ int lc_blocks(int dv) { return (la_columns<MODE>(dv) + 15) / 16; }
 
 bool la_chunks_take(int mode, int dk, int longest) {
   return (mode == LA_CHANNEL || mode == LA_MEMORY) && dk <= LC_SLAB * LC_MAX_SLABS && longest >= LC_FROM;
@@ -57,8 +71,24 @@ __global__ __launch_bounds__(256) void la_chunk_factors_kernel(LaArgs a, int dkp
   const int r = a.chunk_req[chunk], row0 = a.chunk_row0[chunk], last = a.q_start[r + 1];
   const int lane = threadIdx.x & (TK_WAVE - 1), g = __builtin_amdgcn_readfirstlane(threadIdx.x / TK_WAVE);
   const int col = lane & 15, c = lane >> 4;
-  float* out = rec + ((size_t)chunk * a.H + h) * lc_words(dkp);
+  const int blocks = lc_blocks<MODE>(a.dv);
+  float* out = rec + ((size_t)chunk * a.H + h) * lc_words(dkp, blocks);
   const int t0 = row0 + 16 * g;
+  // the values, as the products' operands lie (zeros behind the last token; 1 in the column that sums the keys)
+#pragma unroll 4
+  for (int zc = 0; zc < blocks; ++zc) {
+    const int j = zc * 16 + col;
+    const float* src = proj + a.v_off + h * a.dv + min(j, a.dv - 1);
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int t = t0 + 4 * c + e;
+      v[e] = src[(size_t)min(t, last - 1) * a.ld];
+      if (!CHANNEL && j == a.dv) v[e] = 1.f;
+      if (t >= last || j >= la_columns<MODE>(a.dv)) v[e] = 0.f;
+    }
+    ((float4*)(out + lc_v_at(dkp, blocks)))[(zc * 4 + g) * TK_WAVE + lane] = make_float4(v[0], v[1], v[2], v[3]);
+  }
   if (!CHANNEL && g == 0) {
     const int t = row0 + lane;
     const float2 e = t < last ? gates[(size_t)t * a.H + h] : make_float2(0.f, 0.f);
@@ -123,9 +153,15 @@ __global__ __launch_bounds__(256) void la_chunk_factors_kernel(LaArgs a, int dkp
       }
       const float bias = in ? a.low_bias[x] : 0.f;
       float sum = 0.f;
+      const float per_tau = LC_LOG2E / a.tau;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        sum += in && t0 + j < last ? la_log_sigmoid(A[j] + bias) / a.tau * LC_LOG2E : 0.f;
+        A[j] = la_log_sigmoid(A[j] + bias) * per_tau;
+        asm volatile("" : "+v"(A[j]));  // (all of them, side by side: no branch around each)
+      }
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        sum += in && t0 + j < last ? A[j] : 0.f;
         A[j] = sum;
       }
       sums[g * LC_SLAB + lane] = sum;
@@ -162,7 +198,7 @@ __global__ __launch_bounds__(256) void la_chunk_factors_kernel(LaArgs a, int dkp
         kv[j] *= ws[16 * g + j];
       }
     }
-    // the factors of the products that the second kernel makes (those of q below)
+    // the factors of the products that the other kernels make (those of q below)
     {
       float4* kt = (float4*)(out + lc_k_at(dkp)) + ((ch / 16) * 4 + g) * TK_WAVE + col;
 #pragma unroll
@@ -191,12 +227,19 @@ __global__ __launch_bounds__(256) void la_chunk_factors_kernel(LaArgs a, int dkp
         if (g > 0) ref = *(const float4*)(as + (16 * g - 1) * LC_LD + at);
         q4.x *= lc_exp2(a4.x - ref.x); q4.y *= lc_exp2(a4.y - ref.y); q4.z *= lc_exp2(a4.z - ref.z); q4.w *= lc_exp2(a4.w - ref.w);
       }
+      float4 kj[4], bj[4];  // (asked for together, those not used too)
+#pragma unroll
+      for (int J = 0; J < 4; ++J) {
+        kj[J] = *(const float4*)(ks + (16 * J + col) * LC_LD + at);
+        if (CHANNEL) bj[J] = *(const float4*)(as + (16 * J + col) * LC_LD + at);
+      }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int J = 0; J < 4; ++J) {
         if (J > g || (J == g && !near)) continue;  // (the same for all lanes)
-        float4 k4 = *(const float4*)(ks + (16 * J + col) * LC_LD + at);
+        float4 k4 = kj[J];
         if (CHANNEL) {
-          const float4 b4 = *(const float4*)(as + (16 * J + col) * LC_LD + at);
+          const float4 b4 = bj[J];
           k4.x *= lc_exp2(ref.x - b4.x); k4.y *= lc_exp2(ref.y - b4.y); k4.z *= lc_exp2(ref.z - b4.z); k4.w *= lc_exp2(ref.w - b4.w);
         }
         acc[J] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4.x, q4.x, acc[J], 0, 0, 0);
@@ -224,7 +267,7 @@ __global__ __launch_bounds__(256) void la_chunk_factors_kernel(LaArgs a, int dkp
     }
     __syncthreads();  // the slab is used up
   }
-  // P as far as the second kernel uses it: up to the diagonal block's end
+  // P as far as the third kernel uses it: up to the diagonal block's end
 #pragma unroll
   for (int J = 0; J < 4; ++J) {
     if (J > g) continue;
@@ -240,170 +283,191 @@ __global__ __launch_bounds__(256) void la_chunk_factors_kernel(LaArgs a, int dkp
 }
 
 // --------------------------------------------------------------------------
-// The second kernel.  A workgroup owns 16 columns of the state of one (head, request): wavefront w computes the results of
-// tokens 16 w .. of every chunk, and the rows 16 (w + 4 p) .. of S, whose tiles of 16 x 16 stay in its registers and are
-// handed to the others through LDS, [row / 4][column][4], in two buffers.  What a chunk needs is asked for while the chunk
-// before is computed, into one of two sets of registers in turn, and waited for once, in front of the chunk.  (P right of the
-// block of the diagonal is read with the rest and not used.)  The loads stand between the products: issued together in front of
-// them they would hold the products up.  NP: tiles of S of a wavefront (slabs of 64 rows).
+// The second kernel: the state in front of every chunk.  A wavefront owns 16 rows x 16 columns of a head's state of a request and
+// walks its chunks; nothing passes between wavefronts, so a chunk costs its 16 products, one chain.  What a chunk needs (its
+// factors of k, its decay, its values) is asked for LC_SETS - 1 chunks ahead, into sets of registers in turn.
 // --------------------------------------------------------------------------
-template <int NP>
-struct LcChunk {
-  float4 q[4 * NP], k[4 * NP], p[4], d[NP];
-  float v[4];  // of tokens 16 w + 4 c + e: a wavefront brings a quarter of a chunk's values, which go round through LDS
+#define LC_SETS 5
+
+struct LcStep {
+  float4 k[4], v[4], d;
 };
 
-template <int MODE, int NP>
-__global__ __launch_bounds__(256) void la_chunk_walk_kernel(LaArgs a, const float* __restrict__ proj, const float* __restrict__ rec,
-                                                            float* __restrict__ o) {
-  constexpr int DKP = LC_SLAB * NP;
-  __shared__ __align__(16) float s_lds[2][DKP * 16], v_lds[2][LC_CHUNK * 16];
+template <int MODE>
+__global__ __launch_bounds__(TK_WAVE) void la_chunk_states_kernel(LaArgs a, int dkp, float* __restrict__ rec) {
   const int h = blockIdx.x, r = blockIdx.y;
-  const int c0 = a.first_chunk[r], c1 = a.first_chunk[r + 1];
-  if (c0 >= c1) return;
-  const int first = a.q_start[r], last = a.q_start[r + 1];
+  const int c0 = a.first_chunk[r], chunks = a.first_chunk[r + 1] - c0;
+  if (chunks <= 0) return;
+  const int lane = threadIdx.x, col = lane & 15, c = lane >> 4;
+  const int zc = blockIdx.z / (dkp / 16), n = blockIdx.z % (dkp / 16);  // columns 16 zc .., rows 16 n ..
+  const int columns = la_columns<MODE>(a.dv), blocks = lc_blocks<MODE>(a.dv), j = zc * 16 + col;
+  const bool live = j < columns;
+  float* s_col = a.state + (size_t)a.slots[r] * a.state_stride + ((size_t)h * columns + (live ? j : 0)) * a.dk + 16 * n + 4 * c;
+  v4f s;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) s[i] = live && 16 * n + 4 * c + i < a.dk ? s_col[i] : 0.f;
+  const size_t words = lc_words(dkp, blocks), step = (size_t)a.H * words;
+  float* own = rec + ((size_t)c0 * a.H + h) * words;
+  const float* k_at = own + lc_k_at(dkp) + (n * 4 * TK_WAVE + lane) * 4;
+  const float* v_at = own + lc_v_at(dkp, blocks) + (zc * 4 * TK_WAVE + lane) * 4;
+  const float* d_at = own + lc_d_at(dkp) + 16 * n + 4 * c;
+  float* s_at = own + lc_s_at(dkp) + ((size_t)zc * dkp + 16 * n) * 16 + lane * 4;
+  // of the request's chunk i: T < 4 (factors of k and values, and with the first the decay)
+  auto ask = [&](LcStep& x, int i, int T) {
+    const size_t at = (size_t)i * step;
+    x.k[T] = *(const float4*)(k_at + at + T * TK_WAVE * 4);
+    x.v[T] = *(const float4*)(v_at + at + T * TK_WAVE * 4);
+    if (T == 0) x.d = *(const float4*)(d_at + at);
+    __builtin_amdgcn_sched_barrier(0);  // (asked for here, chunks ahead of their use)
+  };
+  // (the loads stand between the products, which wait for each other)
+  auto take = [&](const LcStep& x, int i, LcStep& next, auto more) {
+    const int ahead = min(i + LC_SETS - 1, chunks - 1);  // (behind the last chunk that one again)
+    *(float4*)(s_at + (size_t)i * step) = make_float4(s[0], s[1], s[2], s[3]);
+    s[0] *= x.d.x; s[1] *= x.d.y; s[2] *= x.d.z; s[3] *= x.d.w;
+#pragma unroll
+    for (int T = 0; T < 4; ++T) {
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[T].x, x.v[T].x, s, 0, 0, 0);
+      if constexpr (decltype(more)::value) ask(next, ahead, T);
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[T].y, x.v[T].y, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[T].z, x.v[T].z, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[T].w, x.v[T].w, s, 0, 0, 0);
+    }
+  };
+  LcStep x[LC_SETS];
+#pragma unroll
+  for (int i = 0; i < LC_SETS - 1; ++i)
+#pragma unroll
+    for (int T = 0; T < 4; ++T) ask(x[i], min(i, chunks - 1), T);
+  // (whole turns of the sets, and what is left behind them: with a way out of the middle of a turn the compiler moves what was asked for
+  // between registers at its end, and waits for all of it there)
+  int i = 0;
+#pragma unroll 1
+  for (; i + LC_SETS <= chunks; i += LC_SETS) {
+#pragma unroll
+    for (int u = 0; u < LC_SETS; ++u) take(x[u], i + u, x[(u + LC_SETS - 1) % LC_SETS], std::true_type{});
+  }
+#pragma unroll
+  for (int u = 0; u < LC_SETS - 1; ++u)
+    if (i + u < chunks) take(x[u], i + u, x[u], std::false_type{});
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (live && 16 * n + 4 * c + i < a.dk) s_col[i] = s[i];
+}
+
+// --------------------------------------------------------------------------
+// The third kernel: the results, all (chunk, head) at once.  Wavefront w has tokens 16 w .. of a chunk, whose factors of q and
+// rows of P stay in its registers while it goes through the workgroup's blocks of 16 columns: the state in front of the chunk times
+// the factors of q, and P times the chunk's values.  A block of the state and of the values goes straight to local memory, two
+// ahead, and is read there by all four wavefronts: the path from the L2 to a compute unit gives some 35 bytes a cycle.  NP: slabs of 64
+// rows of S.
+// --------------------------------------------------------------------------
+#define LC_PLACES 3
+
+template <int MODE, int NP>
+__global__ __launch_bounds__(256) void la_chunk_outputs_kernel(LaArgs a, int share, const float* __restrict__ rec, float* __restrict__ o) {
+  constexpr int DKP = LC_SLAB * NP, PIECES = 4 * NP + 4, LOADS = PIECES / 4;  // of 1 KB: a block of the state, then of the values
+  __shared__ __align__(16) float4 lds[LC_PLACES][PIECES * TK_WAVE];
+  const int chunk = blockIdx.x, h = blockIdx.y;
   const int lane = threadIdx.x & (TK_WAVE - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / TK_WAVE);
   const int col = lane & 15, c = lane >> 4;
-  const int columns = la_columns<MODE>(a.dv), j = blockIdx.z * 16 + col;
-  const bool live = j < columns;
-  const bool one = MODE == LA_MEMORY && j == a.dv;  // the column that sums the keys
-  const int v_at = a.v_off + h * a.dv + min(j, a.dv - 1);
-  float* s_col = a.state + (size_t)a.slots[r] * a.state_stride + ((size_t)h * columns + (live ? j : 0)) * a.dk;
-  v4f s[NP];
+  const int columns = la_columns<MODE>(a.dv), blocks = lc_blocks<MODE>(a.dv);
+  const int z0 = blockIdx.z * share, z1 = min(blocks, z0 + share);
+  const float* src = rec + ((size_t)chunk * a.H + h) * lc_words(DKP, blocks);
+  const unsigned base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float4*)lds;
+  auto ask = [&](int zc, int place) {
 #pragma unroll
-  for (int p = 0; p < NP; ++p)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int n = 16 * (w + 4 * p) + 4 * c + i;
-      s[p][i] = live && n < a.dk ? s_col[n] : 0.f;
-    }
-  // The loads of a chunk, piece by piece: m < 4 NP (q and k), T < 4 (P, and with the first all else)
-  auto ask_qk = [&](LcChunk<NP>& x, const float* src, int m) {
-    x.q[m] = ((const float4*)src)[(w * (DKP / 16) + m) * TK_WAVE + lane];
-    x.k[m] = ((const float4*)(src + lc_k_at(DKP)))[((w + 4 * (m / 4)) * 4 + m % 4) * TK_WAVE + lane];
-  };
-  auto ask_p = [&](LcChunk<NP>& x, const float* src, int chunk, int T) {
-    x.p[T] = ((const float4*)(src + lc_p_at(DKP)))[(w * 4 + T) * TK_WAVE + lane];
-    if (T == 0) {
-#pragma unroll
-      for (int p = 0; p < NP; ++p) x.d[p] = *(const float4*)(src + lc_d_at(DKP) + 16 * (w + 4 * p) + 4 * c);
-      const int t0 = first + (chunk - c0) * LC_CHUNK + 16 * w + 4 * c;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) x.v[e] = proj[(size_t)min(t0 + e, last - 1) * a.ld + v_at];
+    for (int i = 0; i < LOADS; ++i) {
+      const int piece = w * LOADS + i;
+      const float* from = piece < 4 * NP ? src + lc_s_at(DKP) + ((size_t)zc * 4 * NP + piece) * TK_WAVE * 4
+                                         : src + lc_v_at(DKP, blocks) + ((size_t)zc * 4 + piece - 4 * NP) * TK_WAVE * 4;
+      load_to_lds((const bf16_t*)(from + lane * 4), base + (unsigned)((place * PIECES + piece) * TK_WAVE * sizeof(float4)));
     }
   };
-  auto left_by = [&](int chunk) { return rec + ((size_t)chunk * a.H + h) * lc_words(DKP); };
-  // S, and the next chunk's values, to the other wavefronts
-  auto hand = [&](const LcChunk<NP>& x, int buf) {
-    *(float4*)(v_lds[buf] + (w * TK_WAVE + lane) * 4) = one ? make_float4(1.f, 1.f, 1.f, 1.f) : make_float4(x.v[0], x.v[1], x.v[2], x.v[3]);
+  ask(z0, 0);
+  if (z0 + 1 < z1) ask(z0 + 1, 1);
+  float4 q[4 * NP], p[4];
 #pragma unroll
-    for (int p = 0; p < NP; ++p)
-      *(float4*)(s_lds[buf] + ((4 * (w + 4 * p) + c) * 16 + col) * 4) = make_float4(s[p][0], s[p][1], s[p][2], s[p][3]);
-  };
-  // one chunk: the results of its tokens, the state behind it
-  auto take = [&](const LcChunk<NP>& x, LcChunk<NP>& next, int chunk, int buf) {
-    const int ahead = min(chunk + 1, c1 - 1);
-    const float* src = left_by(ahead);
-    // what the state in front of the chunk gives its tokens, and what the tokens give each other
-    v4f y0 = (v4f){0.f, 0.f, 0.f, 0.f}, y1 = y0;
-    float4 sm[4 * NP], vm[4];
+  for (int m = 0; m < 4 * NP; ++m) q[m] = ((const float4*)src)[(w * (DKP / 16) + m) * TK_WAVE + lane];
 #pragma unroll
-    for (int T = 0; T < 4; ++T) vm[T] = *(const float4*)(v_lds[buf] + (T * TK_WAVE + lane) * 4);
-#pragma unroll
-    for (int m = 0; m < 4 * NP; ++m) sm[m] = *(const float4*)(s_lds[buf] + ((4 * m + c) * 16 + col) * 4);
-    __builtin_amdgcn_sched_barrier(0);  // (all of them on their way before the first product)
-#pragma unroll
-    for (int m = 0; m < 4 * NP; ++m) {
-      y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[m].x, sm[m].x, y0, 0, 0, 0);
-      y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[m].y, sm[m].y, y1, 0, 0, 0);
-      y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[m].z, sm[m].z, y0, 0, 0, 0);
-      y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[m].w, sm[m].w, y1, 0, 0, 0);
-      ask_qk(next, src, m);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int T = 0; T < 4; ++T) ask_p(next, src, ahead, T);
-#pragma unroll
-    for (int T = 0; T < 4; ++T) {
-      if (T > w) continue;  // (the same for all lanes)
-      y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[T].x, vm[T].x, y0, 0, 0, 0);
-      y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[T].y, vm[T].y, y1, 0, 0, 0);
-      y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[T].z, vm[T].z, y0, 0, 0, 0);
-      y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[T].w, vm[T].w, y1, 0, 0, 0);
-    }
-    const int t0 = first + (chunk - c0) * LC_CHUNK + 16 * w + 4 * c;
-    float* dst = o + ((size_t)t0 * a.H + h) * a.o_head + j;
+  for (int T = 0; T < 4; ++T)
+    if (T <= w) p[T] = ((const float4*)(src + lc_p_at(DKP)))[(w * 4 + T) * TK_WAVE + lane];
+  const int row0 = a.chunk_row0[chunk], last = a.q_start[a.chunk_req[chunk] + 1];
+  const int t0 = row0 + 16 * w + 4 * c;
+  float* dst = o + ((size_t)t0 * a.H + h) * a.o_head + col;
+  v4f y0, y1;
+  auto deliver = [&](int zc) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (live && t0 + i < last) dst[(size_t)i * a.H * a.o_head] = y0[i] + y1[i];
-    // the state behind the chunk
+      if (zc * 16 + col < columns && t0 + i < last) dst[(size_t)i * a.H * a.o_head + zc * 16] = y0[i] + y1[i];
+  };
+  int place = 0;
+#pragma unroll 1
+  for (int zc = z0; zc < z1; ++zc) {
+    // the block is there when only the loads of the one behind it are left; behind the barrier every wavefront's are, and every
+    // wavefront is through with the block before, whose place is filled again
+    if (zc + 1 < z1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (zc > z0) deliver(zc - 1);
+    if (zc + 2 < z1) ask(zc + 2, place == 0 ? 2 : place - 1);
+    y0 = y1 = (v4f){0.f, 0.f, 0.f, 0.f};
+    const float4* x = lds[place] + lane;
+    float4 sm[4 * NP], vm[4];
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      s[p][0] *= x.d[p].x; s[p][1] *= x.d[p].y; s[p][2] *= x.d[p].z; s[p][3] *= x.d[p].w;
+    for (int m = 0; m < 4 * NP; ++m) sm[m] = x[m * TK_WAVE];
+#pragma unroll
+    for (int T = 0; T < 4; ++T)
+      if (T <= w) vm[T] = x[(4 * NP + T) * TK_WAVE];  // (the same for all lanes)
+#pragma unroll
+    for (int m = 0; m < 4 * NP; ++m) {
+      y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(q[m].x, sm[m].x, y0, 0, 0, 0);
+      y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(q[m].y, sm[m].y, y1, 0, 0, 0);
+      y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(q[m].z, sm[m].z, y0, 0, 0, 0);
+      y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(q[m].w, sm[m].w, y1, 0, 0, 0);
     }
 #pragma unroll
     for (int T = 0; T < 4; ++T) {
-#pragma unroll
-      for (int p = 0; p < NP; ++p) s[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[4 * p + T].x, vm[T].x, s[p], 0, 0, 0);
-#pragma unroll
-      for (int p = 0; p < NP; ++p) s[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[4 * p + T].y, vm[T].y, s[p], 0, 0, 0);
-#pragma unroll
-      for (int p = 0; p < NP; ++p) s[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[4 * p + T].z, vm[T].z, s[p], 0, 0, 0);
-#pragma unroll
-      for (int p = 0; p < NP; ++p) s[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[4 * p + T].w, vm[T].w, s[p], 0, 0, 0);
+      if (T > w) continue;
+      y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(p[T].x, vm[T].x, y0, 0, 0, 0);
+      y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(p[T].y, vm[T].y, y1, 0, 0, 0);
+      y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(p[T].z, vm[T].z, y0, 0, 0, 0);
+      y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(p[T].w, vm[T].w, y1, 0, 0, 0);
     }
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the next chunk's numbers are there
-    hand(next, buf ^ 1);
-    __syncthreads();
-  };
-  LcChunk<NP> xa, xb;
-#pragma unroll
-  for (int m = 0; m < 4 * NP; ++m) ask_qk(xa, left_by(c0), m);
-#pragma unroll
-  for (int T = 0; T < 4; ++T) ask_p(xa, left_by(c0), c0, T);
-  __builtin_amdgcn_s_waitcnt(0x0f70);
-  hand(xa, 0);
-  __syncthreads();
-#pragma unroll 1
-  for (int chunk = c0; chunk < c1; chunk += 2) {
-    take(xa, xb, chunk, 0);
-    if (chunk + 1 >= c1) break;
-    take(xb, xa, chunk + 1, 1);
+    place = place == LC_PLACES - 1 ? 0 : place + 1;
   }
-  if (!live) return;
-#pragma unroll
-  for (int p = 0; p < NP; ++p)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int n = 16 * (w + 4 * p) + 4 * c + i;
-      if (n < a.dk) s_col[n] = s[p][i];
-    }
+  deliver(z1 - 1);
 }
 
 // 32-bit words of working memory that a chunk of a step takes for all heads, and a token beside that (the gates).
-TK_API int tk_linear_attention_chunk_words(int mode, int H, int dk, int longest) {
+TK_API int tk_linear_attention_chunk_words(int mode, int H, int dk, int dv, int longest) {
   if (!la_chunks_take(mode, dk, longest)) return 0;
   const int dkp = (dk + LC_SLAB - 1) / LC_SLAB * LC_SLAB;
-  return (int)(H * lc_words(dkp));
+  return (int)(H * lc_words(dkp, mode == LA_MEMORY ? lc_blocks<LA_MEMORY>(dv) : lc_blocks<LA_CHANNEL>(dv)));
 }
 TK_API int tk_linear_attention_chunk_tokens() { return LC_CHUNK; }
 
 template <int MODE>
 static int lc_run(const LaArgs& a, hipStream_t stream) {
   const int slabs = (a.dk + LC_SLAB - 1) / LC_SLAB, dkp = slabs * LC_SLAB;
+  const int blocks = lc_blocks<MODE>(a.dv);
   float2* gates = nullptr;
   if (MODE == LA_MEMORY) {
-    gates = (float2*)(a.rec + (size_t)a.n_chunks * a.H * lc_words(dkp));
+    gates = (float2*)(a.rec + (size_t)a.n_chunks * a.H * lc_words(dkp, blocks));
     la_launch_gates(a, gates, 1, stream);
   }
   hipLaunchKernelGGL(la_chunk_factors_kernel<MODE>, dim3(a.n_chunks, a.H), dim3(256), 0, stream, a, dkp, a.proj, gates, a.rec);
-  const dim3 grid(a.H, a.n_requests, (la_columns<MODE>(a.dv) + 15) / 16);
-#define LC_WALK(NP) hipLaunchKernelGGL((la_chunk_walk_kernel<MODE, NP>), grid, dim3(256), 0, stream, a, a.proj, a.rec, a.o)
-  if (slabs == 1) LC_WALK(1);
-  else if (slabs == 2) LC_WALK(2);
-  else if (slabs == 3) LC_WALK(3);
-  else LC_WALK(4);
-#undef LC_WALK
+  hipLaunchKernelGGL(la_chunk_states_kernel<MODE>, dim3(a.H, a.n_requests, blocks * (dkp / 16)), dim3(TK_WAVE), 0, stream, a, dkp, a.rec);
+  // blocks of columns a workgroup: as many as leave two workgroups for each of 256 compute units, one of which reads its block while
+  // the other multiplies
+  const long parts = std::min<long>(blocks, std::max(1l, 512 / ((long)a.n_chunks * a.H)));
+  const int share = (int)((blocks + parts - 1) / parts);
+  const dim3 grid(a.n_chunks, a.H, (blocks + share - 1) / share);
+#define LC_OUTPUTS(NP) hipLaunchKernelGGL((la_chunk_outputs_kernel<MODE, NP>), grid, dim3(256), 0, stream, a, share, a.rec, a.o)
+  if (slabs == 1) LC_OUTPUTS(1);
+  else if (slabs == 2) LC_OUTPUTS(2);
+  else if (slabs == 3) LC_OUTPUTS(3);
+  else LC_OUTPUTS(4);
+#undef LC_OUTPUTS
   TK_CHECK_LAUNCH("linear_attention");
   return 0;
 }

@@ -58,7 +58,9 @@ HIPCC_FLAGS = [
 # them, and every difference of two infinities is guarded), so a maximum need not first make
 # its operands quiet numbers: an instruction less for every score, in a loop whose time goes
 # to such instructions.
-SOURCE_FLAGS = {"attention_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-fno-honor-nans"]}
+# The walks of linear attention and of the delta rule in chunks scale their sums in front of every chunk: ordinary registers there too.
+SOURCE_FLAGS = {"attention_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-fno-honor-nans"],
+                "linear_attention_chunks.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"], "delta_rule_chunks.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 # A developer's knob: extra flags for every hipcc call.  Part of the digest,

@@ -1676,7 +1676,7 @@ def linear_attention_chunk_tokens() -> int:
 
 def linear_attention_takes_chunks(memory: bool, key_dim: int, longest: int) -> bool:
     """Whether a step whose longest portion has this many tokens goes in chunks (and so needs a ``ChunkPlan``)."""
-    return load("core").tk_linear_attention_chunk_words(LA_MEMORY if memory else LA_CHANNEL, 1, int(key_dim), int(longest)) > 0
+    return load("core").tk_linear_attention_chunk_words(LA_MEMORY if memory else LA_CHANNEL, 1, int(key_dim), 1, int(longest)) > 0
 
 
 def _linear_attention(mode: int, proj: torch.Tensor, q_off: int, k_off: int, v_off: int, state: torch.Tensor, q_start: torch.Tensor,
@@ -1704,7 +1704,7 @@ def _linear_attention(mode: int, proj: torch.Tensor, q_off: int, k_off: int, v_o
         # tokens computes them in the recurrence's own kernel)
         n_chunks, chunk_words = 0, 0
         if chunks is not None:
-            chunk_words = load("core").tk_linear_attention_chunk_words(mode, H, dk, longest)
+            chunk_words = load("core").tk_linear_attention_chunk_words(mode, H, dk, dv, longest)
         if chunk_words:
             _gpu(chunks.req, chunks.row0, chunks.first)
             for t, name in ((chunks.req, "chunk requests"), (chunks.row0, "chunk rows"), (chunks.first, "first chunks")):
