@@ -20,7 +20,8 @@
 // request is cut into portions changes the order of the sums.
 // The recurrence token by token is one chain of 270 ns a token; here it is one of about 1 us a chunk of 16, and the first
 // kernel, bound by its vector instructions, has no chain.  Two prompts of 562 and 938 tokens, 16 heads of 128 x 128: 72 us of
-// delta_prepare and 256 us of delta_rule before, 99 and 58 us now.
+// delta_prepare and 256 us of delta_rule before, 80 and 53 us now (93 and 55 with sizes that the first kernel learned as it ran and walks that waited
+// for all of a chunk's operands, us of a layer with what surrounds it: these two prompts 142 / 121, one of 1,500 168 / 148, eight of 200 133 / 131).
 #include "delta_rule.h"
 
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -62,10 +63,11 @@ struct DeltaChunkArgs {
   int H, G, dk, dv, dkp, dvp;
 };
 
-template <typename T>
-__global__ __launch_bounds__(256) void delta_chunk_factors_kernel(DeltaChunkArgs a) {
+template <typename T, int DKP>
+__global__ __launch_bounds__(256, 4) void delta_chunk_factors_kernel(DeltaChunkArgs a) {
   extern __shared__ __align__(16) float sh[];
-  const int dkp = a.dkp, dvp = a.dvp, dk = a.dk, dv = a.dv;
+  constexpr int dkp = DKP;
+  const int dvp = a.dvp, dk = a.dk, dv = a.dv;
   float* qs = sh;                      // [16][dkp]
   float* ks = qs + DC_CHUNK * dkp;     // [16][dkp]
   float* gs = ks + DC_CHUNK * dkp;     // [16][dkp]
@@ -81,6 +83,15 @@ __global__ __launch_bounds__(256) void delta_chunk_factors_kernel(DeltaChunkArgs
   const int gk = h / (a.H / a.G), C = 2 * a.G * dk + a.H * dv;
   const float* tail = a.state + (size_t)a.slots[r] * a.state_stride + a.tail_off;
 
+  // what the decays are made from, asked for in front of all else
+  constexpr int DECAYS = DC_CHUNK * DKP / 256;
+  const float* pre = a.a_pre + (size_t)row0 * a.ld_a + h * dk;
+  float z[DECAYS];
+#pragma unroll
+  for (int u = 0; u < DECAYS; ++u) {
+    const int t = (u * 256 + tid) / DKP, x = (u * 256 + tid) % DKP;
+    z[u] = pre[(unsigned)(min(t, n - 1) * a.ld_a + min(x, dk - 1))] + a.dt_bias[(unsigned)(h * dk + min(x, dk - 1))];
+  }
   // a channel's 16 tokens through the convolution and silu, a thread a channel of q, k or v; zeros behind the last token
   for (int c = tid; c < 2 * dkp + dvp; c += 256) {
     const int which = c < dkp ? 0 : (c < 2 * dkp ? 1 : 2);
@@ -95,19 +106,20 @@ __global__ __launch_bounds__(256) void delta_chunk_factors_kernel(DeltaChunkArgs
       continue;
     }
     const float* w = a.conv_w + (size_t)ch * a.taps;
+    auto row_of = [&](int row) { return to_f32<T>((proj + (size_t)row * a.ld)[(unsigned)ch]); };
     auto input = [&](int src) {  // of place `src` among the step's tokens of the request, or from the tail before them
-      return src >= 0 ? to_f32<T>(proj[(size_t)(first + src) * a.ld + ch]) : tail[(size_t)(src + a.taps - 1) * C + ch];
+      return src >= 0 ? row_of(first + src) : tail[(size_t)(src + a.taps - 1) * C + ch];
     };
     if (a.taps <= 4) {
       float xs[DC_CHUNK + 3];  // the three inputs in front and the chunk's own
       if (local0 >= 3) {       // all of them this step's rows: asked for at once (rows behind the last token: that one's again)
 #pragma unroll
-        for (int u = 0; u < DC_CHUNK + 3; ++u) xs[u] = to_f32<T>(proj[(size_t)(row0 + min(u - 3, n - 1)) * a.ld + ch]);
+        for (int u = 0; u < DC_CHUNK + 3; ++u) xs[u] = row_of(row0 + min(u - 3, n - 1));
       } else {  // (places before the taps' reach are not read)
 #pragma unroll
         for (int u = 0; u < 3; ++u) xs[u] = u - 3 + a.taps - 1 >= 0 ? input(local0 + u - 3) : 0.f;
 #pragma unroll
-        for (int u = 3; u < DC_CHUNK + 3; ++u) xs[u] = to_f32<T>(proj[(size_t)(row0 + min(u - 3, n - 1)) * a.ld + ch]);
+        for (int u = 3; u < DC_CHUNK + 3; ++u) xs[u] = row_of(row0 + min(u - 3, n - 1));
       }
 #pragma unroll
       for (int t = 0; t < DC_CHUNK; ++t) {
@@ -127,10 +139,10 @@ __global__ __launch_bounds__(256) void delta_chunk_factors_kernel(DeltaChunkArgs
     }
   }
   const float rate = expf(a.a_log[h]);
-#pragma unroll 8
-  for (int i = tid; i < DC_CHUNK * dkp; i += 256) {
-    const int t = i / dkp, x = i % dkp;
-    gs[i] = t < n && x < dk ? expf(-rate * softplus_f32(a.a_pre[(size_t)(row0 + t) * a.ld_a + h * dk + x] + a.dt_bias[h * dk + x])) : 1.f;
+#pragma unroll
+  for (int u = 0; u < DECAYS; ++u) {
+    const int i = u * 256 + tid;
+    gs[i] = i / DKP < n && i % DKP < dk ? expf(-rate * softplus_f32(z[u])) : 1.f;
   }
   if (tid < DC_CHUNK) beta[tid] = tid < n ? sigmoid_f32(to_f32<T>(proj[(size_t)(row0 + tid) * a.ld + a.col_b + h])) : 0.f;
   __syncthreads();
@@ -141,10 +153,12 @@ __global__ __launch_bounds__(256) void delta_chunk_factors_kernel(DeltaChunkArgs
     for (int u = 0; u < 8; ++u) {
       float* row = (u < 4 ? qs : ks) + (wave * 4 + (u & 3)) * dkp;
       float ss = 0.f;
-      for (int i = lane; i < dk; i += TK_WAVE) ss = fmaf(row[i], row[i], ss);
+#pragma unroll
+      for (int i = lane; i < DKP; i += TK_WAVE) ss = fmaf(row[i], row[i], ss);  // (zeros behind dk)
       float mul = 1.0f / sqrtf(wave_sum(ss) + 1e-6f);
       if (u < 4) mul *= qmul;
-      for (int i = lane; i < dk; i += TK_WAVE) row[i] *= mul;
+#pragma unroll
+      for (int i = lane; i < DKP; i += TK_WAVE) row[i] *= mul;
     }
   }
   __syncthreads();
@@ -153,7 +167,10 @@ __global__ __launch_bounds__(256) void delta_chunk_factors_kernel(DeltaChunkArgs
     float M[DC_CHUNK], P[DC_CHUNK];
 #pragma unroll
     for (int t = 0; t < DC_CHUNK; ++t) M[t] = P[t] = 0.f;
-    for (int c = 4 * cg; c < dkp; c += 64) {
+    int end = DKP;
+    asm volatile("" : "+s"(end));  // (a loop also where it is one turn: its reads, all asked for at once, would fill the registers)
+#pragma unroll 1
+    for (int c = 4 * cg; c < end; c += 64) {
       const v4f k = *(const v4f*)(ks + s * dkp + c);
       v4f e = k;
 #pragma unroll
@@ -255,10 +272,13 @@ __global__ __launch_bounds__(256) void delta_chunk_factors_kernel(DeltaChunkArgs
   }
 }
 
-// RB: blocks of 16 rows of S a wavefront holds (dkp = 64 RB).
+// RB: blocks of 16 rows of S a wavefront holds (dkp = 64 RB).  Bound by a chunk's chain of products, sum and update (0.9 us): W S, which it
+// goes on from, comes first, Q S waits behind the barrier.  The sets of operands are taken in whole turns and the remainder by itself: left
+// out of the middle of a turn, the loop waits for all that is on its way and copies it.
 template <int RB>
 __global__ __launch_bounds__(256) void delta_chunk_walk_kernel(DeltaChunkArgs a) {
   __shared__ __align__(16) v4f part[2][2][4][TK_WAVE];  // [chunk's parity][W S, Q S][wavefront][lane]
+  constexpr int SETS = RB <= 2 ? 4 : (RB == 3 ? 3 : 2);  // chunks whose operands are there or on their way, as many as registers hold
   const int h = blockIdx.x, r = blockIdx.y, nb = blockIdx.z, tid = threadIdx.x;
   const int lane = tid & (TK_WAVE - 1), wave = tid / TK_WAVE;
   const int lr = lane & 15, q = lane >> 4;
@@ -299,42 +319,58 @@ __global__ __launch_bounds__(256) void delta_chunk_walk_kernel(DeltaChunkArgs a)
   };
   // the output this thread adds up: float tid of the products' [lane][4]
   const int token = 4 * (tid >> 6) + (tid & 3), ocol = nb * 16 + ((tid >> 2) & 15);
+  float o_before = 0.f;
+  auto deliver = [&](int c) {  // the outputs of chunk c, whose Q S the wavefronts left behind its barrier
+    const float* f = (const float*)part[c & 1][1];
+    const float sum = o_before + ((f[tid] + f[256 + tid]) + (f[512 + tid] + f[768 + tid]));
+    const int t = first + c * DC_CHUNK + token;
+    if (t < last && ocol < a.dv) a.o[(size_t)t * a.H * a.dv + (size_t)h * a.dv + ocol] = sum;
+  };
   auto walk = [&](int c, const Operands& x) {
     v4f ws = (v4f){0.f, 0.f, 0.f, 0.f}, qs = ws;
 #pragma unroll
     for (int b = 0; b < RB; ++b)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        ws = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w[b][e], S[b][e], ws, 0, 0, 0);
-        qs = __builtin_amdgcn_mfma_f32_16x16x4f32(x.qx[b][e], S[b][e], qs, 0, 0, 0);
-      }
+      for (int e = 0; e < 4; ++e) ws = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w[b][e], S[b][e], ws, 0, 0, 0);
     v4f(*p)[4][TK_WAVE] = part[c & 1];
     p[0][wave][lane] = ws;
-    p[1][wave][lane] = qs;
     __syncthreads();
-    const v4f u = x.v - ((p[0][0][lane] + p[0][1][lane]) + (p[0][2][lane] + p[0][3][lane]));
+    const v4f w0 = p[0][0][lane], w1 = p[0][1][lane], w2 = p[0][2][lane], w3 = p[0][3][lane];
+    __builtin_amdgcn_sched_barrier(0);  // (Q S while the quarters of W S come)
 #pragma unroll
-    for (int b = 0; b < RB; ++b) {
-      S[b] = S[b] * x.d[b];
+    for (int b = 0; b < RB; ++b)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[b][e], u[e], S[b], 0, 0, 0);
-    }
-    const int t = first + c * DC_CHUNK + token;
-    const float* f = (const float*)p[1];
-    const float sum = x.o + ((f[tid] + f[256 + tid]) + (f[512 + tid] + f[768 + tid]));
-    if (t < last && ocol < a.dv) a.o[(size_t)t * a.H * a.dv + (size_t)h * a.dv + ocol] = sum;
+      for (int e = 0; e < 4; ++e) qs = __builtin_amdgcn_mfma_f32_16x16x4f32(x.qx[b][e], S[b][e], qs, 0, 0, 0);
+    if (c > 0) deliver(c - 1);
+    o_before = x.o;
+    const v4f u = x.v - ((w0 + w1) + (w2 + w3));
+#pragma unroll
+    for (int b = 0; b < RB; ++b) S[b] = S[b] * x.d[b];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int b = 0; b < RB; ++b) S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[b][e], u[e], S[b], 0, 0, 0);
+    p[1][wave][lane] = qs;
   };
-  Operands x0, x1;
-  ask(0, x0);
+  Operands x[SETS];
+#pragma unroll
+  for (int i = 0; i < SETS - 1; ++i) ask(min(i, chunks - 1), x[i]);
+  // (whole turns of the sets, and what is left behind them: with a way out of the middle of a turn the compiler moves what was asked for
+  // between registers at its end, and waits for all of it there)
   int c = 0;
 #pragma unroll 1
-  for (; c + 1 < chunks; c += 2) {
-    ask(c + 1, x1);
-    walk(c, x0);
-    ask(min(c + 2, chunks - 1), x0);
-    walk(c + 1, x1);
+  for (; c + SETS <= chunks; c += SETS) {
+#pragma unroll
+    for (int i = 0; i < SETS; ++i) {
+      ask(min(c + i + SETS - 1, chunks - 1), x[(i + SETS - 1) % SETS]);  // (behind the last chunk that one again)
+      walk(c + i, x[i]);
+    }
   }
-  if (c < chunks) walk(c, x0);
+#pragma unroll
+  for (int i = 0; i < SETS - 1; ++i)
+    if (c + i < chunks) walk(c + i, x[i]);
+  __syncthreads();
+  deliver(chunks - 1);
   if (col < a.dv) {
 #pragma unroll
     for (int b = 0; b < RB; ++b)
@@ -343,6 +379,23 @@ __global__ __launch_bounds__(256) void delta_chunk_walk_kernel(DeltaChunkArgs a)
         const int row = 16 * (wave * RB + b) + 4 * q + j;
         if (row < a.dk) s_col[row] = S[b][j];
       }
+  }
+}
+
+template <typename T, int DKP>
+static bool launch_factors_of(const DeltaChunkArgs& a, int n_chunks, size_t lds, hipStream_t stream) {
+  auto kernel = delta_chunk_factors_kernel<T, DKP>;
+  if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return false;
+  hipLaunchKernelGGL(kernel, dim3(n_chunks, a.H), dim3(256), lds, stream, a);
+  return true;
+}
+template <typename T>
+static bool launch_factors(const DeltaChunkArgs& a, int n_chunks, size_t lds, hipStream_t stream) {
+  switch (a.dkp / 64) {
+    case 1: return launch_factors_of<T, 64>(a, n_chunks, lds, stream);
+    case 2: return launch_factors_of<T, 128>(a, n_chunks, lds, stream);
+    case 3: return launch_factors_of<T, 192>(a, n_chunks, lds, stream);
+    default: return launch_factors_of<T, 256>(a, n_chunks, lds, stream);
   }
 }
 
@@ -369,13 +422,8 @@ TK_API int tk_delta_chunks(int dt, const void* proj, int ld, int col_b, const fl
   DeltaChunkArgs a = {proj, ld, col_b, a_pre, ld_a, conv_w, taps, a_log, dt_bias, state, state_stride, tail_off, q_start, slots,
                       chunk_req, chunk_row0, chunk_first, rec, o, H, G, dk, dv, (dk + 63) / 64 * 64, (dv + 15) / 16 * 16};
   const size_t lds = sizeof(float) * ((size_t)DC_CHUNK * (3 * a.dkp + a.dvp) + 3 * DC_CHUNK * DC_LD + DC_CHUNK);
-  const void* kernel = dt == TK_F32 ? (const void*)delta_chunk_factors_kernel<float> : (const void*)delta_chunk_factors_kernel<bf16_t>;
-  TK_REQUIRE(lds <= 64 * 1024 || hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess,
-             "delta_chunks: %zu bytes of local memory could not be reserved", lds);
-  if (dt == TK_F32)
-    hipLaunchKernelGGL(delta_chunk_factors_kernel<float>, dim3(n_chunks, H), dim3(256), lds, stream, a);
-  else
-    hipLaunchKernelGGL(delta_chunk_factors_kernel<bf16_t>, dim3(n_chunks, H), dim3(256), lds, stream, a);
+  const bool ok = dt == TK_F32 ? launch_factors<float>(a, n_chunks, lds, stream) : launch_factors<bf16_t>(a, n_chunks, lds, stream);
+  TK_REQUIRE(ok, "delta_chunks: %zu bytes of local memory could not be reserved", lds);
   const dim3 grid(H, n_requests, a.dvp / 16);
   switch (a.dkp / 64) {
     case 1: hipLaunchKernelGGL(delta_chunk_walk_kernel<1>, grid, dim3(256), 0, stream, a); break;
