@@ -61,6 +61,26 @@ __device__ __forceinline__ void rotate_pair(float x1, float x2, float c, float s
   o2 = __fmaf_rn(x2, c, __fmul_rn(x1, s));
 }
 
+// log(1 + exp(-|x|)), the part of a softplus and of a logarithm of a sigmoid that is no straight line: with y = exp(-|x|) <= 1,
+// y + y^2 q(y) with q through the Chebyshev nodes of (log(1 + y) / y - 1) / y on [0, 1], 1e-8 of it in front of the roundings.  Some 35
+// instructions where log1pf(expf()) takes 150, in kernels bound by them.  Errors from 64 bits over |x| <= 12, root mean square (largest):
+// a softplus 1.28e-7 (4.8e-7) where log1pf(expf(x)) has 1.29e-7 (5.4e-7), decays exp(-softplus) 1.35e-8 (6.9e-8), before 1.36e-8 (6.5e-8); the
+// part by itself 5.6e-9 (6.9e-8), as log1pf(expf()) 5.2e-9 (5.1e-8), which a logarithm's other part, up to 12, hides.
+__device__ __forceinline__ float log1p_exp(float x) {
+  const float y = expf(-fabsf(x));
+  float q = 0.00287388382f;
+  q = fmaf(q, y, -0.0175122432f);
+  q = fmaf(q, y, 0.0499311797f);
+  q = fmaf(q, y, -0.0920296311f);
+  q = fmaf(q, y, 0.130713284f);
+  q = fmaf(q, y, -0.163785085f);
+  q = fmaf(q, y, 0.199593559f);
+  q = fmaf(q, y, -0.249970242f);
+  q = fmaf(q, y, 0.333332479f);
+  q = fmaf(q, y, -0.5f);
+  return fmaf(y * y, q, y);
+}
+
 template <typename T>
 __device__ __forceinline__ float to_f32(T v);
 template <>
