@@ -22,6 +22,7 @@
 //   row: [nq*dq | nkv*dk | nkv*dv]  (only the first part when !write_cache; no third part with v_from_k)
 //   K pages: [page][kv head][dk / 8][P][8]    V pages: [page][kv head][P / 4][dv][4]
 #include "common.h"
+#include "head_rows.h"
 
 // The work items of a head of size d of which the leading `rot` elements are rotated: item j names
 // one or two elements (e0, and e1 when `two`) and, when `turned`, the angle they are rotated by.
@@ -201,6 +202,25 @@ TK_API int tk_qk_prepare(int dt, void* qkv, int row_stride, const int* positions
              "qk_prepare: row stride %d is shorter than the heads it holds", row_stride);
   TK_REQUIRE(!write_cache || (kcache && vcache && block_table && nkv > 0), "qk_prepare: cache pointers missing");
   if (n_tokens == 0) return 0;
+  // (heads of one size, all of each rotated: as many bytes at a time as they allow)
+  if (dt != TK_F32 && rot > 0 && rot == dq && dq == dk && dk == dv && k_skip == 0 && !v_from_k && !vfreq && rotate_q && nkv > 0) {
+    const HeadRows rows = {(bf16_t*)qkv, row_stride, positions, token_req, block_table, table_stride, q_weight, k_weight, eps, freq,
+                           rot_scale, (bf16_t*)kcache, (bf16_t*)vcache, n_tokens, nq, nkv, dq, P, write_cache};
+    if (head_rows_take(rows)) {
+      const bool normed = q_weight || k_weight;
+      if (pair_half) {
+        if (!normed) launch_head_rows<HR_PLAIN, true>(rows, stream);
+        else if (per_head) launch_head_rows<HR_PER_HEAD, true>(rows, stream);
+        else launch_head_rows<HR_PER_ROW, true>(rows, stream);
+      } else {
+        if (!normed) launch_head_rows<HR_PLAIN, false>(rows, stream);
+        else if (per_head) launch_head_rows<HR_PER_HEAD, false>(rows, stream);
+        else launch_head_rows<HR_PER_ROW, false>(rows, stream);
+      }
+      TK_CHECK_LAUNCH("qk_prepare");
+      return 0;
+    }
+  }
   const size_t smem = sizeof(float) * (size_t)((rot > 0 ? rot : 2) + (vfreq ? dv : 0) + (per_head ? nq + nkv : 0));
   TK_REQUIRE(smem <= 48 * 1024, "qk_prepare: too many heads for one workgroup's local memory");
   if (dt == TK_F32)
