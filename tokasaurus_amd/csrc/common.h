@@ -100,11 +100,23 @@ __device__ __forceinline__ bf16_t from_f32<bf16_t>(float v) { return __float2bfl
 template <typename T>
 __device__ __forceinline__ float round_to(float v) { return to_f32<T>(from_f32<T>(v)); }
 
+// x / (1 + exp(-x)) of a bfloat16 number, to be rounded to one: the hardware's exponential and reciprocal, a correction of the quotient
+// and the hardware's repair of its special cases; both sides scaled, so that no reciprocal leaves the normal numbers.  Rounded, it is what
+// expf and the division give for every one of the 65,536 numbers, in 9 instructions where those take some 25, in epilogues that have nothing
+// beside them (a tile of 256 x 256 of gate and up: 128 a thread, one wavefront a SIMD).  us of gate and up in tiles, with those / with
+// this: 16,384 x 2,048 101 rows 19.2 / 18.8, 512 36.8 / 35.4, 1,045 78.6 / 75.0, 2,048 120 / 114; 16,384 x 3,072 1,045 rows 109 / 105; 28,672 x 4,096
+// 512 rows 99.1 / 96.6, 4,096 697 / 686.
+__device__ __forceinline__ float silu_of_bf16(float x) {
+  const float d = fmaf(__builtin_amdgcn_exp2f(x * -1.44269504f), 0.0625f, 0.0625f);
+  const float u = x * 0.0625f, r = __builtin_amdgcn_rcpf(d), q = u * r;
+  return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, u), r, q), d, u);
+}
+
 // silu(gate) * up as the engine's storage type sees it: both operands and the activation
 // rounded to bfloat16, the product left in 32-bit for the caller to round.
 __device__ __forceinline__ float silu_mul_bf16(float g, float u) {
   const float gr = round_to<bf16_t>(g), ur = round_to<bf16_t>(u);
-  const float s = round_to<bf16_t>(gr / (1.0f + expf(-gr)));
+  const float s = round_to<bf16_t>(silu_of_bf16(gr));
   return s * ur;
 }
 
