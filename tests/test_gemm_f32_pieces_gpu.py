@@ -1,0 +1,57 @@
+"""32-bit products of many rows by exact pieces of the numbers: against 64-bit sums and against the unsplit products (which an inner size of
+no whole steps goes to), at the edges of both tiles and of K's parts, with numbers at the ends of their range."""
+
+import pytest
+import torch
+
+from tokasaurus_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def unsplit(a, w, **more):
+    pad = lambda x: torch.nn.functional.pad(x, (0, 4))  # noqa: E731
+    return ops.gemm_generic(pad(a), pad(w), **more)
+
+
+def error(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+# (rows counted in tiles of 64) x columns x K at 7 * 2^27 and over; columns that no 16 bytes hold (K in one part), K of one step of parts and of many
+@pytest.mark.parametrize("m,n,k", [(33, 14336, 1024), (64, 14337, 1024), (65, 7170, 1056), (129, 4780, 1024), (300, 1233, 2400), (65, 820, 9088), (1000, 3588, 256),
+                                   (2049, 1604, 288), (512, 2400, 768), (1025, 4100, 512)])
+def test_errors_are_no_larger_than_unsplit(m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    wide = torch.randn((m, k + 8), generator=g, device="cuda")
+    a, w = wide[:, 4 : k + 4], torch.randn((n, k), generator=g, device="cuda")  # rows a stride apart
+    bias, residual = torch.randn((n,), generator=g, device="cuda"), torch.randn((m, n + 3), generator=g, device="cuda")[:, 1 : n + 1]
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    got = ops.gemm_generic(a, w)
+    # a sum of K products, each rounded, and what is left of each product (2^-20 at most)
+    assert bool(((got.double() - want).abs() <= ((k + 2) * 2.0 ** -24 + 2.0 ** -20) * size).all())
+    assert error(got, want) <= error(unsplit(a, w), want)
+    want = want + bias.double() + residual.double()
+    assert error(ops.gemm_generic(a, w, bias=bias, residual=residual), want) <= error(unsplit(a, w, bias=bias, residual=residual), want) * 1.01
+
+
+@pytest.mark.parametrize("m", [70, 300])
+def test_numbers_at_the_ends_of_their_range(m):
+    g = torch.Generator(device="cuda").manual_seed(m)
+    n, k = 7300, 1024
+    a, w = torch.randn((m, k), generator=g, device="cuda"), torch.randn((n, k), generator=g, device="cuda").abs() + 0.1
+    a[0, 3], a[1, 5], a[2, 7] = float("inf"), float("nan"), -float("inf")
+    a[3] *= 2.0 ** -130
+    a[4] = 0
+    a[5] *= 2.0 ** 112
+    a[6, 1:] = 0
+    a[6, 0] = 2.0 ** -140
+    got = ops.gemm_generic(a, w)
+    assert bool((got[0] == float("inf")).all() and torch.isnan(got[1]).all() and (got[2] == -float("inf")).all())
+    assert bool(torch.isfinite(got[3:]).all()) and bool((got[4] == 0).all())
+    want = a[3:].double() @ w.double().T
+    for i in (0, 2):
+        assert error(got[3 + i], want[i]) <= 2e-6, i
+    # one product of a number below the least normal one: rounded to a multiple of 2^-149
+    assert bool(((got[6].double() - want[3]).abs() <= 2.0 ** -149).all())
+    assert error(got[7:], want[4:]) <= 2e-6

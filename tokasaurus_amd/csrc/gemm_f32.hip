@@ -2,7 +2,8 @@
 //     C[M,N] = A[M,K] * W[N,K]^T (+ bias[N]) (+ residual[M,N])
 // for row-major operands whose rows start at multiples of 16 bytes (K and the stride of A
 // multiples of 4; gemm_generic.hip has the kernels for any others).  Products and sums are
-// 32-bit throughout: the instruction multiplies and adds 32-bit numbers, unsplit.
+// 32-bit throughout: the instruction multiplies and adds 32-bit numbers, unsplit (but for products so many that their time counts, which
+// gemm_f32_pieces_kernel makes of exact parts of the numbers, with smaller errors).
 //
 // A wavefront owns TM x TN blocks of 16 tokens x 16 weight rows.  In a block of 16 elements of K lane l holds elements
 // 4 * (l / 16) .. + 3 of weight row l % 16 and of token l % 16; instruction s of the block then multiplies element s of
@@ -25,6 +26,7 @@
 // the first two in the mean, 301 and 643 (gemm_f32_stream_kernel has the figures for K of a multiple of 32).  Errors against 64-bit
 // sums: up to 32 tokens those of the plain kernel (1.2e-7 of the norm at 2 048 elements), beyond at most the plain kernel's.
 #include "common.h"
+#include <type_traits>
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 
@@ -434,6 +436,137 @@ __global__ __launch_bounds__(256) void gemm_f32_stream_kernel(GemmF32Args a) {
   gf_finish<TM, TN, CHAINS>(a, acc, m0, n0, wave, r, q);
 }
 
+// Many products over a K of a multiple of 32: the numbers as exact sums of three bfloat16 numbers (their 24 bits, 8 at a time, by truncation)
+// on the matrix cores' bfloat16 multiply-adds, whose products are exact and whose sums are 32-bit.  Of the nine products of pieces the six
+// largest count; what is left out is under 2^-20 of a product and 2^-24 in the mean, and a step of 32 elements is added up inside one instruction, where the
+// 32-bit instruction rounds after every fourth: errors against 64 bits are smaller than the unsplit products' (below).
+// Six instructions of 16 x 16 x 32 take 102 cycles where eight of 16 x 16 x 4 take 272; the pieces, made by every wavefront for itself, cost as much as
+// the products, side by side with them where two workgroups share a compute unit.
+// LOW: the five smaller products in sums of their own, where registers allow it (a third of the error).
+// Pieces reach down to 2^-133, and an infinite number has pieces that are no numbers: a workgroup with a sum that is not finite, or not
+// zero and below 2^-60, does its products again, unsplit.  (Bits below 2^-133 that are lost are 2^-33 of a sum of 2^-60 with the other operand
+// at 2^40.)
+// us unsplit / split, and errors where both were taken (root of the squares' sums over that of the results):
+//   33 rows   16,384 x 2,048 50.3 / 41.3 (3.7e-7 / 1.5e-7), 2,048 x 8,192 33.8 / 28.5 (3.1e-7 / 1.5e-7), 128,256 x 2,048 522 / 270 (8.1e-7 / 2.8e-7)
+//   200       16,384 x 2,048 153 / 110 (8.1e-7 / 4.9e-7), 2,048 x 8,192 79.9 / 61.9 (5.2e-7 / 3.6e-7), 2,048 x 2,048 31.0 / 27.2 (2.9e-7 / 1.2e-7)
+//   301       16,384 x 2,048 177 / 148 (8.1e-7 / 2.0e-7), 2,048 x 8,192 98.3 / 79.7, 2,048 x 2,048 36.2 / 31.8, 3,072 x 2,048 49.9 / 39.4
+//   2,048     16,384 x 2,048 1,017 / 697 (8.1e-7 / 7.0e-7), 2,048 x 8,192 565 / 357 (1.6e-6 / 1.0e-6), 2,048 x 2,048 153 / 112 (8.1e-7 / 4.9e-7)
+typedef __attribute__((ext_vector_type(8))) __bf16 gf_bf16x8_t;
+
+__device__ __forceinline__ void gf_pieces(f4 lo, f4 hi, gf_bf16x8_t (&piece)[3]) {
+  float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+  for (int n = 0; n < 3; ++n) {
+    uint32_t packed[4];
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+      const uint32_t ua = __float_as_uint(v[i]), ub = __float_as_uint(v[i + 1]);
+      packed[i / 2] = __builtin_amdgcn_perm(ub, ua, 0x07060302);  // the upper halves, the first below
+      if (n < 2) {
+        v[i] -= __uint_as_float(ua & 0xffff0000u);
+        v[i + 1] -= __uint_as_float(ub & 0xffff0000u);
+      }
+    }
+    __builtin_memcpy(&piece[n], packed, sizeof(piece[n]));
+  }
+}
+
+#define GP_STAGES 2  // steps in local memory: two workgroups of the largest tile share a compute unit
+template <int TM, int TN, bool LOW>
+__global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) {
+  extern __shared__ __align__(16) float tile[];  // [GP_STAGES][32 * (TN + TM)][32], weight rows first, pieces in places as above
+  constexpr int ROWS = 32 * (TN + TM), LOADS = ROWS / 32, STAGES = GP_STAGES;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int mt = (a.M + 32 * TM - 1) / (32 * TM);  // (workgroups on the dies as in gemm_f32_kernel)
+  const int g = blockIdx.x / 8;
+  const int n0 = ((g / mt) * 8 + blockIdx.x % 8) * 32 * TN, m0 = (g % mt) * 32 * TM;
+  if (n0 >= a.N) return;  // the same for the whole workgroup
+  const int all = a.K >> 5;
+  const int s0 = (int)((long)all * blockIdx.y / gridDim.y), steps = (int)((long)all * (blockIdx.y + 1) / gridDim.y) - s0;
+  const int lr = 8 * wave + (lane >> 3);  // load i brings row 32 i + lr
+  const int lc = ((lane & 7) ^ gs_swizzle(lr)) * 4;
+  const float* src[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i)
+    src[i] = (i < TN ? a.W + (size_t)min(n0 + 32 * i + lr, a.N - 1) * a.K : a.A + (size_t)min(m0 + 32 * (i - TN) + lr, a.M - 1) * a.lda) + lc + (size_t)s0 * 32;
+  const unsigned lds = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)tile;
+  auto ask = [&](int step, int place) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+      load_to_lds((const bf16_t*)(src[i] + (size_t)step * 32), lds + (unsigned)((place * ROWS + 32 * i + 8 * wave) * 32 * (int)sizeof(float)));
+  };
+  f4 acc[1][TN][TM], small[LOW ? TN : 1][LOW ? TM : 1];
+  auto low = [&](int t, int u) -> f4& { return LOW ? small[LOW ? t : 0][LOW ? u : 0] : acc[0][t][u]; };
+  const int piece[2] = {(q ^ gs_swizzle(r)) * 4, ((4 + q) ^ gs_swizzle(r)) * 4};
+  const float* wrow = tile + ((wave & 1) * 16 * TN + r) * 32;
+  const float* xrow = tile + (32 * TN + (wave >> 1) * 16 * TM + r) * 32;
+  auto walk = [&](auto unsplit) {
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+      for (int u = 0; u < TM; ++u) acc[0][t][u] = low(t, u) = (f4){0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < STAGES - 1 && s < steps; ++s) ask(s, s);
+    int here = 0, next = STAGES - 1;
+#pragma unroll 1
+    for (int s = 0; s < steps; ++s) {
+      if (s + STAGES - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 2) * LOADS) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (s + STAGES - 1 < steps) ask(s + STAGES - 1, next);
+      const float *wr = wrow + here * ROWS * 32, *xr = xrow + here * ROWS * 32;
+      if constexpr (decltype(unsplit)::value) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int u = 0; u < TM; ++u) {
+            const f4 x = *(const f4*)(xr + 16 * u * 32 + piece[b]);
+#pragma unroll
+            for (int t = 0; t < TN; ++t) {
+              const f4 w = *(const f4*)(wr + 16 * t * 32 + piece[b]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[0][t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[e], x[e], acc[0][t][u], 0, 0, 0);
+            }
+          }
+      } else {
+        gf_bf16x8_t w[TN][3];
+#pragma unroll
+        for (int t = 0; t < TN; ++t) gf_pieces(*(const f4*)(wr + 16 * t * 32 + piece[0]), *(const f4*)(wr + 16 * t * 32 + piece[1]), w[t]);
+#pragma unroll
+        for (int u = 0; u < TM; ++u) {
+          gf_bf16x8_t x[3];
+          gf_pieces(*(const f4*)(xr + 16 * u * 32 + piece[0]), *(const f4*)(xr + 16 * u * 32 + piece[1]), x);
+#define GP_PRODUCTS(SUM, I, J) \
+  _Pragma("unroll") for (int t = 0; t < TN; ++t) SUM = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][I], x[J], SUM, 0, 0, 0)
+          GP_PRODUCTS(low(t, u), 2, 0);
+          GP_PRODUCTS(low(t, u), 0, 2);
+          GP_PRODUCTS(low(t, u), 1, 1);
+          GP_PRODUCTS(low(t, u), 1, 0);
+          GP_PRODUCTS(low(t, u), 0, 1);
+          GP_PRODUCTS(acc[0][t][u], 0, 0);
+#undef GP_PRODUCTS
+        }
+      }
+      here = here + 1 == STAGES ? 0 : here + 1;
+      next = next + 1 == STAGES ? 0 : next + 1;
+    }
+  };
+  walk(std::integral_constant<bool, false>{});
+  bool plain = true;
+#pragma unroll
+  for (int t = 0; t < TN; ++t)
+#pragma unroll
+    for (int u = 0; u < TM; ++u) {
+      if (LOW) acc[0][t][u] += low(t, u);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float size = fabsf(acc[0][t][u][j]);
+        plain = plain && (size == 0.f || (size >= 0x1p-60f && size < INFINITY));
+      }
+    }
+  if (__syncthreads_or(!plain)) walk(std::integral_constant<bool, true>{});
+  gf_finish<TM, TN, 1>(a, acc, m0, n0, wave, r, q);
+}
+
 // The sums of K's parts added in the order of K: a thread four neighbouring outputs.
 __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(GemmF32Args a, int cuts) {
   const int n = (blockIdx.x * blockDim.x + threadIdx.x) * 4, token = blockIdx.y;
@@ -455,11 +588,34 @@ static long gf_tiles(int M, int N, int tm, int tn) {
   return (((long)N + 32 * tn - 1) / (32 * tn) + 7) / 8 * 8 * (((long)M + 32 * tm - 1) / (32 * tm));
 }
 
+// Whether products go by bfloat16 pieces: the rows of a tile (64 or 128, 128 weight rows), 0 if not; and into how many parts they cut K, the same
+// for both ends of a call.  They pay from 7 * 2^27 multiply-adds on (rows counted in tiles of 64), where the steps' work outweighs a longer beginning:
+// 200 rows 2,816 x 1,024 25.3 / 25.4 us, 160 rows 2,048 x 2,048 25.8 / 27.7, 128 rows 3,072 x 2,048 26.6 / 27.0, 64 rows 19.7 / 21.5; 400 rows 8,192 x 256
+// 28.2 / 22.7 and 4,096 x 512 30.9 / 26.0, 200 rows 2,048 x 2,048 31.0 / 27.2.
+// Tile and parts are those of the least time by the steps of 32 elements of K that a compute unit takes one after the other (us a
+// step with one workgroup on it and with two, which fit: 1.05 and 1.58 for 64 rows, 1.6 and 2.75 for 128) and the parts' way through memory.
+static int gf_pieces_tile(int M, int N, int K, int* cuts) {
+  const long most = K / 256 < 32 ? K / 256 : 32, steps = K / 32;
+  if (M <= 32 || K % 32 != 0 || most < 1 || ((long)M + 63) / 64 * 64 * N * K < 7L << 27) return 0;
+  double best = 0;
+  int tile = 0;
+  for (int tm = 2; tm <= 4; tm += 2)
+    for (int c = 1; c <= ((N & 3) == 0 ? most : 1); ++c) {
+      const long groups = gf_tiles(M, N, tm, 4) * c, rest = groups % 512;
+      const double one = tm == 2 ? 1.05 : 1.6, two = tm == 2 ? 1.58 : 2.75;
+      const double us = (groups / 512 * two + (rest == 0 ? 0 : (rest <= 256 ? one : two))) * ((steps + c - 1) / c) + (c > 1 ? 2 + c * (4e-6 / 3) * M * N : 0);
+      if (tile == 0 || us < best) best = us, tile = 32 * tm, *cuts = c;
+    }
+  return tile;
+}
+
 // How many parts K is cut into among workgroups (the caller brings M * N floats for each where there is more than one):
 // so many that the tiles times the parts are about five workgroups a compute unit, of 256 elements of K at least.  In us at
 // 1 / 2 / 4 / 8 / 16 parts: 301 tokens 2 048 x 8 192 (160 tiles) 188 / 170 / 124 / 108 / 111; 600 tokens (320 tiles) 329 / 240 /
 // 199 / 199 / 207; 301 tokens 3 072 x 2 048 (240 tiles) 49 / 50 / 48 / 51 / 59; 16 384 x 2 048 (1 280 tiles) 203 / 202 / 216.
 TK_API int tk_gemm_f32_cuts(int M, int N, int K) {
+  int split_cuts;
+  if (gf_pieces_tile(M, N, K, &split_cuts)) return split_cuts;
   if (M <= 16 || (N & 3) != 0) return 1;
   long cuts = 1280 / gf_tiles(M, N, M <= 32 ? 1 : 2, 2);
   const long most = K / 256;
@@ -480,6 +636,15 @@ static bool gf_launch(const GemmF32Args& a, int cuts, hipStream_t stream) {
   auto kernel = stream_in ? gemm_f32_stream_kernel<TM, TN, CHAINS, STAGES> : gemm_f32_kernel<TM, TN, CHAINS>;
   if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return false;
   hipLaunchKernelGGL(kernel, dim3((unsigned)grid, cuts), dim3(256), lds, stream, a);
+  return true;
+}
+
+template <int TM, bool LOW>
+static bool gf_launch_pieces(const GemmF32Args& a, int cuts, hipStream_t stream) {
+  const long grid = gf_tiles(a.M, a.N, TM, 4);
+  if (grid > 0x7fffffffL) return false;
+  const size_t lds = (size_t)GP_STAGES * 32 * (TM + 4) * 32 * sizeof(float);  // (64 KB at most)
+  hipLaunchKernelGGL((gemm_f32_pieces_kernel<TM, 4, LOW>), dim3((unsigned)grid, cuts), dim3(256), lds, stream, a);
   return true;
 }
 
@@ -520,7 +685,11 @@ TK_API int tk_gemm_f32(const void* A, int lda, const void* W, void* C, int ldc, 
   // tiles of 128 x 128 read the operands half as often, where they still fill the chip twice over; up to 32 tokens leave half
   // of a 64-token tile empty
   bool ok;
-  if (M <= 32) ok = gf_launch<1, 2, 8>(a, cuts, stream);
+  int unused;
+  const int pieces = gf_pieces_tile(M, N, K, &unused);
+  if (pieces == 64) ok = gf_launch_pieces<2, true>(a, cuts, stream);
+  else if (pieces) ok = gf_launch_pieces<4, false>(a, cuts, stream);
+  else if (M <= 32) ok = gf_launch<1, 2, 8>(a, cuts, stream);
   else if (gf_tiles(M, N, 4, 4) >= 512) ok = gf_launch<4, 4, 1>(a, cuts, stream);
   else ok = gf_launch<2, 2, 1>(a, cuts, stream);
   TK_REQUIRE(ok, "gemm_f32: M=%d N=%d take too many workgroups, or their local memory could not be reserved", M, N);
