@@ -570,10 +570,27 @@ __device__ __forceinline__ void attention_item(const AttnArgs& a, const int tile
     load_step<DT, BIG>(regs, a, table, pages, kvh, k, t.lo, t.hi, r, q);
     if (AHEAD && k + 32 < k_end) pages = step_pages(a, table, k + 32, t.lo, t.hi);
   };
+  // Prompts' walks are whole turns of the ring, in which every load is asked for, then what is left: behind a load that may not have been
+  // asked for the compiler waits for all that were (us a layer: 24 heads of 128, 1,000 tokens by pairs 27.4 / 26.3, 32 heads 1,024 30.2 / 27.8).
+  // Decoded tokens' few steps are asked for together as it is (with turns of their own 64 uneven requests take 45.8 for 43.4).
+  int k_next = k_begin;
+  if (RT == 2 && k_end - k_begin > 32 * (2 * PF - 1)) {
 #pragma unroll
-  for (int i = 0; i < PF; ++i)
-    if (k_begin + 32 * i < k_end) issue(ring[i], k_begin + 32 * i);
-  for (int kb = k_begin; kb < k_end; kb += 32 * PF) {
+    for (int i = 0; i < PF; ++i) issue(ring[i], k_begin + 32 * i);
+    do {
+#pragma unroll
+      for (int i = 0; i < PF; ++i) {
+        compute_step(ring[i], k_next + 32 * i);
+        issue(ring[i], k_next + 32 * (i + PF));
+      }
+      k_next += 32 * PF;
+    } while (k_end - k_next > 32 * (2 * PF - 1));
+  } else {
+#pragma unroll
+    for (int i = 0; i < PF; ++i)
+      if (k_begin + 32 * i < k_end) issue(ring[i], k_begin + 32 * i);
+  }
+  for (int kb = k_next; kb < k_end; kb += 32 * PF) {
 #pragma unroll
     for (int i = 0; i < PF; ++i) {
       const int k = kb + 32 * i;
