@@ -100,6 +100,14 @@ def attention_plan(ctx: StepContext, group: int, nkv: int, head_dim: int, page_s
         tails = [r for r in large if long_past(r) and own(r) <= 512]
         after_past = [r for r in large if long_past(r) and own(r) > 512]
         whole = -(-max(bound, 1) // 128) * 128
+
+        def longest_first(req: list[int], row0: list[int], unit: int) -> tuple[list[int], list[int]]:
+            """The tiles by the keys they walk, ``unit`` of them together: what starts last is short, of whichever request.  us a layer, 8 kv
+            heads, request by request / so: 4 x 1,024 tokens of 32 heads of 128 74.3 / 61.0, of 64 53.1 / 45.9, 2 x 2,048 of 64 75.9 / 67.7."""
+            reach = lambda i: max(ctx.host_kv_len[req[j]] - q_lens[req[j]] + row0[j] // group for j in range(i, i + unit))  # noqa: E731
+            order = [j for i in sorted(range(0, len(req), unit), key=reach, reverse=True) for j in range(i, i + unit)]
+            return [req[j] for j in order], [row0[j] for j in order]
+
         for some in (fresh, after_past, tails):
             if not some:
                 continue
@@ -109,6 +117,7 @@ def attention_plan(ctx: StepContext, group: int, nkv: int, head_dim: int, page_s
             sets = 0 if split else ops.attention_group_sets(wavefronts, head_dim, page_size, longest)
             if sets:
                 req, row0, _ = ops.attention_tiles(q_lens, group, 2, some, fill=ops.ATTENTION_GROUP)
+                req, row0 = longest_first(req, row0, ops.ATTENTION_GROUP)
                 lists.append((req, row0, None, 2, whole, 1, sets, bound))
             else:
                 # (cut keys: the grid and the scratch are sized for these requests, not for a longer one that decodes beside them)
