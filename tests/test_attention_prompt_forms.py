@@ -1,4 +1,4 @@
-"""The order in which prompts' groups of tiles start."""
+"""Prompt portions whose keys the wavefronts of a workgroup share: single and neighbouring tiles against pairs in a wavefront, and when they are taken."""
 
 import pytest
 import torch
@@ -6,7 +6,14 @@ import torch
 from tokasaurus_amd.kernels import ops
 
 
-@pytest.mark.parametrize("q_lens,kv_lens,unit,form", [([1024, 1000, 1300], [1024, 1200, 1300], 4, 2), ([2048, 2048], [2048, 2100], 4, 2)])
+def test_which_form_prompt_portions_take():
+    form = ops.attention_prompt_form
+    assert form(608, 64, 5000) == form(448, 128, 100) == (1, 2)
+    assert form(609, 64, 699) == form(449, 128, 699) == (2, 1) and form(609, 64, 700) == form(3072, 128, 700) == (2, 2)
+    assert form(3073, 64, 4000) == (2, 1)
+
+
+@pytest.mark.parametrize("q_lens,kv_lens,unit,form", [([1024, 1000, 1300], [1024, 1200, 1300], 4, 2), ([90, 33, 60], [90, 500, 64], 1, 1), ([700, 720], [700, 720], 1, 2)])
 def test_longest_walks_start_first(monkeypatch, q_lens, kv_lens, unit, form):
     """The plan's tiles are those of every portion, each once, in the order of the keys they reach."""
     from types import SimpleNamespace
@@ -25,3 +32,34 @@ def test_longest_walks_start_first(monkeypatch, q_lens, kv_lens, unit, form):
     reach = [max(kv_lens[req[j]] - q_lens[req[j]] + row0[j] // 4 for j in range(i, i + unit)) for i in range(0, len(req), unit)]
     assert reach == sorted(reach, reverse=True)
     assert all(len(set(req[i : i + unit])) == 1 for i in range(0, len(req), unit))
+
+
+# portions whole, one token over a step, after a past; windows that end a walk inside a step; pages of fewer keys than a block has; every
+# wavefront with keys, and wavefronts without
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,portions,nq,nkv,d,page,window", [([97, 400], [97, 400], 8, 2, 64, 16, 0), ([33, 1, 640], [33, 1, 33], 4, 4, 128, 16, 0),
+                                                                ([300], [300], 6, 2, 112, 4, 0), ([500], [400], 4, 1, 16, 8, 70), ([900], [450], 3, 1, 128, 32, 333)])
+def test_shared_keys_give_the_same_as_pairs(lens, portions, nq, nkv, d, page, window):
+    g = torch.Generator(device="cuda").manual_seed(sum(lens) + d)
+    pages = -(-max(lens) // page)
+    rand = lambda shape: torch.randn(shape, generator=g, device="cuda").bfloat16()  # noqa: E731
+    keys, values = rand(ops.key_pages_shape(pages * len(lens), nkv, page, d)), rand(ops.value_pages_shape(pages * len(lens), nkv, page, d))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    table = torch.randperm(pages * len(lens), generator=torch.Generator().manual_seed(d)).int().cuda().view(len(lens), pages)
+    start = [sum(portions[:i]) for i in range(len(lens) + 1)]
+    q, bound = rand((start[-1], nq * d)), -(-max(lens) // 256) * 256
+
+    def run(row_tiles, waves, pair):
+        req, row0, row1 = ops.attention_tiles(portions, nq // nkv, row_tiles, pair=pair)
+        if not pair:
+            req, row0 = req[::-1], row0[::-1]
+        return ops.paged_attention_mfma(q, keys, values, table, i32(start), i32(lens), i32(req), i32(row0), row_tiles, nq, nkv, d, page, max(lens), bound,
+                                        window=window, waves=waves, tile_row1=None if row1 is None else i32(row1), even=waves > 1).double()
+
+    want = run(2, 1, True)
+    for row_tiles, waves in ((1, 2), (2, 2), (2, 4), (1, 8)):
+        # the weights of a softmax's terms rounded to bfloat16 under another maximum (2^-8 of each, values of up to five, in root mean square a
+        # tenth of that), and the result's own rounding
+        got = run(row_tiles, waves, False)
+        assert bool(((got - want).abs() <= 2.0 ** -7 * want.abs() + 5 * 2.0 ** -8).all()), (row_tiles, waves)
+        assert float((got - want).norm() / want.norm()) <= 2.0 ** -7, (row_tiles, waves)

@@ -323,11 +323,11 @@ __device__ __forceinline__ void attention_item(const AttnArgs& a, const int tile
   if (!GROUPED && s > t.s_last) return;
   const int nsp = GROUPED ? 1 : t.s_last - t.s_first + 1;
   // this wavefront's part of the split: `sub` keys, a multiple of 32.  Fixed parts of the split, or (`even`) of the keys that are there:
-  // of a request that ends, or whose window begins, inside the split every wavefront then takes as many as the others.  Fixed
+  // of a request (or a prompt's tile) that ends, or whose window begins, inside the split every wavefront then takes as many as the others.  Fixed
   // parts give a workgroup as many wavefronts as it has keys to read, so that requests of all lengths end at one time, and are the
   // rule; the host asks for even ones where they were ahead.
   const int k_first = max((t.lo >> 5) << 5, s * a.split), k_last = min(t.hi + 1, (s + 1) * a.split);
-  const bool even = RT == 1 && a.even;
+  const bool even = a.even != 0;
   const int sub = even ? (((k_last - k_first + NW - 1) / NW + 31) >> 5) << 5 : a.split / NW;
   const int part = (even ? k_first : s * a.split) + wave * sub;
   const int k_begin = max(k_first, part), k_end = min(k_last, part + sub);

@@ -562,6 +562,23 @@ def attention_prompt_split(wavefronts: int, head_dim: int, longest: int) -> int:
     return split if split < longest else 0
 
 
+def attention_prompt_form(wavefronts: int, head_dim: int, longest: int) -> tuple[int, int]:
+    """Row tiles of a wavefront and wavefronts of a workgroup for prompt portions whose keys are neither cut nor shared by groups, that
+    fill ``wavefronts`` wavefronts of two row tiles (over all kv heads): (2, 1) is an early tile beside a late one in a wavefront, which
+    evens the walks out but loads every key of the late one's for both; with two wavefronts a workgroup these share its keys evenly, and
+    (1, 2) takes single tiles, (2, 2) neighbouring ones, whose walks are one.
+    Few portions leave the chip idle with either, and then the shortest walk counts: single tiles.  us a layer, paired / single, 32 heads of
+    64 after 8 kv heads: 64 tokens 5.1 / 4.2, 101 5.8 / 4.6, 200 7.2 / 5.7, 400 10.0 / 7.9, 512 11.2 / 10.4, 8 x 64 5.5 / 5.1, 3 x 200 7.7 / 7.4, 2 x 300 9.1 / 8.9
+    (700, 704 wavefronts, 14.3 / 14.3); 24 heads of 128: 300 tokens 10.1 / 8.3, 500 14.3 / 12.1 (32 heads, 512 tokens, 512 wavefronts, 14.3 / 16.9).
+    More of them load more than the path from the L2 to the compute units gives (24 heads of 128, 1,000 tokens: 385 MB in 27 us, half of it by
+    neighbours), over walks long enough that it counts.  Paired / neighbours: 32 heads of 64, 700 tokens 14.3 / 13.4, 1,024 19.3 / 18.8, 1,500 30.1 /
+    27.0; 24 of 128, 700 tokens 18.6 / 17.2, 1,000 26.2 / 23.2, 1,400 49.7 / 35.8, 2 x 700 30.3 / 26.4 (4 x 400 of 64 14.6 / 17.4, 4 x 256 of 128 11.2 / 16.1;
+    4 x 1,024, 4,096 wavefronts, 94 / 99)."""
+    if wavefronts <= (608 if head_dim <= 64 else 448):
+        return 1, 2
+    return (2, 2) if longest >= 700 and wavefronts <= 3072 else (2, 1)
+
+
 def attention_tiles(
     q_lens: list[int], group: int, row_tiles: int, requests: list[int] | None = None, pair: bool = False, fill: int = 1
 ) -> tuple[list[int], list[int], list[int] | None]:
@@ -757,7 +774,7 @@ def paged_attention_mfma(
 
     The splits of a tile of one row tile (decoded tokens) are added inside the kernel by the
     workgroup that arrives last; ``merge_kernel`` has a second kernel add them instead, as for
-    tiles of two row tiles.  ``even`` (one row tile): the wavefronts of a workgroup share the keys that a request has
+    tiles of two row tiles.  ``even``: the wavefronts of a workgroup share the keys that a tile has
     in the split evenly, instead of the split (see ``attention_even_parts``)."""
     _gpu(q, kcache, vcache, block_table, q_start, kv_len, tile_req, tile_row0)
     _need(q.dim() == 2 and q.stride(1) == 1 and q.shape[1] >= nq * head_dim and q.dtype == torch.bfloat16,

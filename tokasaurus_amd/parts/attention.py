@@ -55,7 +55,8 @@ class AttentionPlan:
     a step for each group size and shared by the layers.  Requests that bring one
     row tile or less (decoded tokens) get wavefronts of one row tile and split keys;
     prompt portions get wavefronts of two row tiles and whole keys: an early tile paired with
-    a late one, or, when there are enough of them and a page holds 16 keys or more, neighbouring
+    a late one, or single or neighbouring tiles whose keys two wavefronts share (``ops.attention_prompt_form``),
+    or, when there are enough of them and a page holds 16 keys or more, neighbouring
     tiles in groups of four wavefronts that share every load of keys and values (with two such
     sets of wavefronts a group while the groups are too few to fill the chip several times
     over: ``ops.attention_group_sets``); portions that fill few wavefronts but walk many keys
@@ -77,19 +78,18 @@ def attention_plan(ctx: StepContext, group: int, nkv: int, head_dim: int, page_s
         # launches are chosen for the bound the step was planned for, not for the lengths in it (but for decoded rows beside prompts,
         # which no recorded step holds: they are cut by their own lengths)
         bound = max(int(ctx.extras.get("kv_bound", 0)), ctx.max_kv_len)
-        lists: list[tuple[list[int], list[int], list[int] | None, int, int, int, int, int]] = []
-        even = False
+        lists: list[tuple[list[int], list[int], list[int] | None, int, int, int, int, int, bool]] = []
         if small:
             req, row0, _ = ops.attention_tiles(q_lens, group, 1, small)
             if large and not static:
                 lengths = [ctx.host_kv_len[r] for r in small]
                 split, waves = ops.attention_even_split(lengths, nkv, head_dim, group)
                 even = (split, waves) != ops.attention_split(max(lengths), len(req), nkv, head_dim, group)
-                lists.append((req, row0, None, 1, split, waves, 0, max(lengths)))
+                lists.append((req, row0, None, 1, split, waves, 0, max(lengths), even))
             else:
                 split, waves = ops.attention_split(bound, len(req), nkv, head_dim, group)
                 even = ops.attention_even_parts(bound, len(req), nkv, head_dim, waves)
-                lists.append((req, row0, None, 1, split, waves, 0, bound))
+                lists.append((req, row0, None, 1, split, waves, 0, bound, even))
         # Portions that come after a past several times their own length walk far more keys a row than
         # whole prompts do: they are planned apart, or one of them among whole prompts would take a
         # form chosen for the many short walks and walk its long past on a few wavefronts.
@@ -118,22 +118,28 @@ def attention_plan(ctx: StepContext, group: int, nkv: int, head_dim: int, page_s
             if sets:
                 req, row0, _ = ops.attention_tiles(q_lens, group, 2, some, fill=ops.ATTENTION_GROUP)
                 req, row0 = longest_first(req, row0, ops.ATTENTION_GROUP)
-                lists.append((req, row0, None, 2, whole, 1, sets, bound))
+                lists.append((req, row0, None, 2, whole, 1, sets, bound, False))
+                continue
+            row_tiles, waves = (2, 1) if split else ops.attention_prompt_form(wavefronts, head_dim, longest)
+            if waves > 1:
+                req, row0, _ = ops.attention_tiles(q_lens, group, row_tiles, some)
+                req, row0 = longest_first(req, row0, 1)
+                lists.append((req, row0, None, row_tiles, whole, waves, 0, bound, True))
             else:
                 # (cut keys: the grid and the scratch are sized for these requests, not for a longer one that decodes beside them)
                 req, row0, row1 = ops.attention_tiles(q_lens, group, 2, some, pair=True)
-                lists.append((req, row0, row1, 2, split or whole, 1, 0, longest if split else bound))
+                lists.append((req, row0, row1, 2, split or whole, 1, 0, longest if split else bound, False))
         # one upload for all the tile lists of the step
         flat = [x for req, row0, row1, *_ in lists for x in (req + row0 + (row1 or []))]
         dev = upload(flat, torch.int32, ctx.device) if flat else None
         launches, at = [], 0
-        for req, row0, row1, row_tiles, split, waves, grouped, max_kv_len in lists:
+        for req, row0, row1, row_tiles, split, waves, grouped, max_kv_len, even in lists:
             n = len(req)
             t_req, t_row0 = dev[at : at + n], dev[at + n : at + 2 * n]
             t_row1 = dev[at + 2 * n : at + 3 * n] if row1 is not None else None
             at += (3 if row1 is not None else 2) * n
             launches.append(AttentionLaunch(t_req, t_row0, t_row1, row_tiles, split, waves, max_kv_len,
-                                            ops.AttentionScratch(ctx.device) if static else None, grouped, even and row_tiles == 1))
+                                            ops.AttentionScratch(ctx.device) if static else None, grouped, even))
         plan = AttentionPlan(launches, bound)
         ctx.extras[key] = plan
     return plan
