@@ -63,3 +63,40 @@ def test_shared_keys_give_the_same_as_pairs(lens, portions, nq, nkv, d, page, wi
         got = run(row_tiles, waves, False)
         assert bool(((got - want).abs() <= 2.0 ** -7 * want.abs() + 5 * 2.0 ** -8).all()), (row_tiles, waves)
         assert float((got - want).norm() / want.norm()) <= 2.0 ** -7, (row_tiles, waves)
+
+
+# products that climb by less than a row's reference allows, by just more, and far more a step of keys; that fall; and that stand still
+@pytest.mark.gpu
+@pytest.mark.parametrize("climb", [0.02, 0.2, 0.3, 3.0, -0.5, 0.0])
+@pytest.mark.parametrize("form", ["pairs", "single", "neighbours", "group", "sets", "decode"])
+def test_a_rows_reference_follows_its_products(climb, form):
+    """Against a softmax in 64 bits: key i has the product climb * i / log2(e) with every query, so the terms climb by 2^climb a key."""
+    nq, nkv, d, page, n = 4, 2, 64, 16, 700
+    g = torch.Generator(device="cuda").manual_seed(3)
+    pages = -(-n // page)
+    k = torch.zeros((n, nkv, d), device="cuda")
+    rows = climb * torch.arange(n, device="cuda").float()
+    k[:, :, 0] = (rows / 1.4427).bfloat16().float()[:, None]  # (two pieces of a bfloat16 number each: what is left of the first, by another element)
+    k[:, :, 1] = (rows / 1.4427 - k[:, 0, 0]).bfloat16().float()[:, None]
+    q = torch.zeros((n, nq, d), device="cuda")
+    q[..., 0] = q[..., 1] = 1
+    v = torch.randn((n, nkv, d), generator=g, device="cuda").bfloat16()
+    keys = torch.zeros(ops.key_pages_shape(pages, nkv, page, d), dtype=torch.bfloat16, device="cuda")
+    values = torch.zeros(ops.value_pages_shape(pages, nkv, page, d), dtype=torch.bfloat16, device="cuda")
+    pad = pages * page - n
+    kp, vp = (torch.nn.functional.pad(x, (0, 0, 0, 0, 0, pad)).view(pages, page, nkv, d) for x in (k.bfloat16(), v))
+    keys.view(pages, nkv, d // 8, page, 8).copy_(kp.view(pages, page, nkv, d // 8, 8).permute(0, 2, 3, 1, 4))
+    values.view(pages, nkv, page // 4, d, 4).copy_(vp.view(pages, page // 4, 4, nkv, d).permute(0, 3, 1, 4, 2))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    row_tiles, waves, grouped, tokens = {"pairs": (2, 1, 0, n), "single": (1, 2, 0, n), "neighbours": (2, 2, 0, n), "group": (2, 1, 1, n), "sets": (2, 1, 2, n),
+                                         "decode": (1, 2, 0, 1)}[form]
+    req, row0, row1 = ops.attention_tiles([tokens], nq // nkv, row_tiles, pair=form == "pairs", fill=ops.ATTENTION_GROUP if grouped else 1)
+    out = ops.paged_attention_mfma(q[-tokens:].reshape(tokens, -1).bfloat16(), keys, values, torch.arange(pages, device="cuda").int().view(1, -1), i32([0, tokens]),
+                                   i32([n]), i32(req), i32(row0), row_tiles, nq, nkv, d, page, n, 64 * waves if form == "decode" else 768, scale=1.0, waves=waves,
+                                   tile_row1=None if row1 is None else i32(row1), grouped=grouped, even=waves > 1 and form != "decode").view(tokens, nq, d)
+    scores = (k[:, 0, 0] + k[:, 0, 1]).double().expand(tokens, n).clone()
+    scores[torch.arange(n, device="cuda")[None] > torch.arange(n - tokens, n, device="cuda")[:, None]] = -float("inf")
+    want = torch.einsum("tk,khd->thd", scores.softmax(-1), v.double()).repeat_interleave(nq // nkv, 1)
+    # weights rounded to bfloat16 (2^-8 of each, of values of up to five) and the result's own rounding
+    assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 5 * 2.0 ** -8).all())
+    assert float((out.double() - want).norm() / want.norm()) <= 2.0 ** -8
