@@ -55,3 +55,18 @@ def test_numbers_at_the_ends_of_their_range(m):
     # one product of a number below the least normal one: rounded to a multiple of 2^-149
     assert bool(((got[6].double() - want[3]).abs() <= 2.0 ** -149).all())
     assert error(got[7:], want[4:]) <= 2e-6
+
+
+@pytest.mark.parametrize("m", [70, 300])
+@pytest.mark.parametrize("down,up", [(-118, 110), (110, -118), (-140, 127), (0, 40)])
+def test_numbers_whose_pieces_are_lost(m, down, up):
+    """Small numbers beside large ones: what their pieces leave out would be the whole of an ordinary sum."""
+    g = torch.Generator(device="cuda").manual_seed(m + up)
+    n, k = 7300, 1024
+    a, w = (torch.rand((r, k), generator=g, device="cuda") + 0.5 for r in (m, n))
+    a, w = (torch.ldexp(torch.ldexp(x, torch.tensor(e // 2, device="cuda")), torch.tensor(e - e // 2, device="cuda")) for x, e in ((a, down), (w, up)))
+    got, want = ops.gemm_generic(a, w), a.double() @ w.double().T
+    assert error(got, want) <= 2e-6
+    a[:, 1:] = 0  # one product a sum
+    got, want = ops.gemm_generic(a, w), a.double() @ w.double().T
+    assert bool(((got.double() - want).abs() <= 2.0 ** -22 * want.abs()).all())

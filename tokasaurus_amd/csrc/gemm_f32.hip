@@ -443,9 +443,11 @@ __global__ __launch_bounds__(256) void gemm_f32_stream_kernel(GemmF32Args a) {
 // Six instructions of 16 x 16 x 32 take 102 cycles where eight of 16 x 16 x 4 take 272; the pieces, made by every wavefront for itself, cost as much as
 // the products, side by side with them where two workgroups share a compute unit.
 // LOW: the five smaller products in sums of their own, where registers allow it (a third of the error).
-// Pieces reach down to 2^-133, and an infinite number has pieces that are no numbers: a workgroup with a sum that is not finite, or not
-// zero and below 2^-60, does its products again, unsplit.  (Bits below 2^-133 that are lost are 2^-33 of a sum of 2^-60 with the other operand
-// at 2^40.)
+// Pieces reach down to 2^-133, and an infinite number has pieces that are no numbers: a workgroup with a sum that is not finite, or below 2^-60
+// (zero too: numbers of less than 2^-133 have no pieces at all), or with an operand of 2^40 and more, does its products again, unsplit.  (Else the bits
+// below 2^-133 that are lost are at most 2^-33 of a sum, and a row of zeros costs its tiles their time twice.)
+// Two wavefronts make the pieces of the same rows: each looks at half a step's numbers, which the other has last (16 instructions of some 370 a
+// step; 301 rows 16,384 x 2,048 151.9 us without, 152.1 with, 2,048 rows 697 and 700).
 // us unsplit / split, and errors where both were taken (root of the squares' sums over that of the results):
 //   33 rows   16,384 x 2,048 50.3 / 41.3 (3.7e-7 / 1.5e-7), 2,048 x 8,192 33.8 / 28.5 (3.1e-7 / 1.5e-7), 128,256 x 2,048 522 / 270 (8.1e-7 / 2.8e-7)
 //   200       16,384 x 2,048 153 / 110 (8.1e-7 / 4.9e-7), 2,048 x 8,192 79.9 / 61.9 (5.2e-7 / 3.6e-7), 2,048 x 2,048 31.0 / 27.2 (2.9e-7 / 1.2e-7)
@@ -453,7 +455,11 @@ __global__ __launch_bounds__(256) void gemm_f32_stream_kernel(GemmF32Args a) {
 //   2,048     16,384 x 2,048 1,017 / 697 (8.1e-7 / 7.0e-7), 2,048 x 8,192 565 / 357 (1.6e-6 / 1.0e-6), 2,048 x 2,048 153 / 112 (8.1e-7 / 4.9e-7)
 typedef __attribute__((ext_vector_type(8))) __bf16 gf_bf16x8_t;
 
-__device__ __forceinline__ void gf_pieces(f4 lo, f4 hi, gf_bf16x8_t (&piece)[3]) {
+// (most: the greatest number of `lo` so far)
+__device__ __forceinline__ void gf_pieces(f4 lo, f4 hi, gf_bf16x8_t (&piece)[3], float& most) {
+  // (one instruction for two numbers; of the compiler's maximum each would first be made a quiet number)
+  asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(lo[0]), "v"(lo[1]));
+  asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(lo[2]), "v"(lo[3]));
   float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 #pragma unroll
   for (int n = 0; n < 3; ++n) {
@@ -498,9 +504,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) 
   };
   f4 acc[1][TN][TM], small[LOW ? TN : 1][LOW ? TM : 1];
   auto low = [&](int t, int u) -> f4& { return LOW ? small[LOW ? t : 0][LOW ? u : 0] : acc[0][t][u]; };
-  const int piece[2] = {(q ^ gs_swizzle(r)) * 4, ((4 + q) ^ gs_swizzle(r)) * 4};
+  const int last = 4 * ((wave ^ (wave >> 1)) & 1);  // the halves of a step change places between wavefronts that share rows
+  const int piece[2] = {((last + q) ^ gs_swizzle(r)) * 4, ((4 - last + q) ^ gs_swizzle(r)) * 4};
   const float* wrow = tile + ((wave & 1) * 16 * TN + r) * 32;
   const float* xrow = tile + (32 * TN + (wave >> 1) * 16 * TM + r) * 32;
+  float most = 0.f;
   auto walk = [&](auto unsplit) {
 #pragma unroll
     for (int t = 0; t < TN; ++t)
@@ -530,11 +538,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) 
       } else {
         gf_bf16x8_t w[TN][3];
 #pragma unroll
-        for (int t = 0; t < TN; ++t) gf_pieces(*(const f4*)(wr + 16 * t * 32 + piece[0]), *(const f4*)(wr + 16 * t * 32 + piece[1]), w[t]);
+        for (int t = 0; t < TN; ++t) gf_pieces(*(const f4*)(wr + 16 * t * 32 + piece[0]), *(const f4*)(wr + 16 * t * 32 + piece[1]), w[t], most);
 #pragma unroll
         for (int u = 0; u < TM; ++u) {
           gf_bf16x8_t x[3];
-          gf_pieces(*(const f4*)(xr + 16 * u * 32 + piece[0]), *(const f4*)(xr + 16 * u * 32 + piece[1]), x);
+          gf_pieces(*(const f4*)(xr + 16 * u * 32 + piece[0]), *(const f4*)(xr + 16 * u * 32 + piece[1]), x, most);
 #define GP_PRODUCTS(SUM, I, J) \
   _Pragma("unroll") for (int t = 0; t < TN; ++t) SUM = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][I], x[J], SUM, 0, 0, 0)
           GP_PRODUCTS(low(t, u), 2, 0);
@@ -551,7 +559,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) 
     }
   };
   walk(std::integral_constant<bool, false>{});
-  bool plain = true;
+  bool plain = most < 0x1p40f;
 #pragma unroll
   for (int t = 0; t < TN; ++t)
 #pragma unroll
@@ -560,7 +568,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) 
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float size = fabsf(acc[0][t][u][j]);
-        plain = plain && (size == 0.f || (size >= 0x1p-60f && size < INFINITY));
+        plain = plain && size >= 0x1p-60f && size < INFINITY;
       }
     }
   if (__syncthreads_or(!plain)) walk(std::integral_constant<bool, true>{});
