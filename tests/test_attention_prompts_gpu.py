@@ -158,3 +158,32 @@ def test_chunks_end_with_the_steps_own_longest_request(options):
     planned, _ = _run(*args, split=True, key_chunk=256, longest=8192, scale=0.125, **options)
     own, _ = _run(*args, split=True, key_chunk=256, longest=8192, step_longest=1100, scale=0.125, **options)
     assert torch.isfinite(own).all() and torch.equal(own, planned)
+
+
+@pytest.mark.parametrize("dk,dv", [(64, 64), (128, 128), (24, 176)])  # (176: heads of one block a step)
+@pytest.mark.parametrize("slope", [-0.4, 0.0, 0.01, 0.4, 4.0])
+@pytest.mark.parametrize("softcap", [0.0, 200.0, 30.0])
+def test_scores_that_rise_and_sinks(dk, dv, slope, softcap):
+    """Scores that rise with the keys by less than a reference allows, or by more (and fall), tanh on both sides of where its
+    polynomial ends, and sinks below, near and far above all of them."""
+    gen = torch.Generator().manual_seed(dk + int(100 * slope))
+    n, nq, nkv, page = 100, 4, 1, 16
+    keys, values, kc, vc, table = _paged([n], nkv, dk, dv, page, gen)
+    keys[0][:, :, 0] = (torch.arange(n) * slope).bfloat16()[:, None]
+    for i in range(-(-n // page)):
+        m = min(page, n - i * page)
+        kc[table[0, i], :, 0, :m, 0] = keys[0][i * page: i * page + m, :, 0].T
+    q = torch.randn((n, nq, dk), generator=gen).bfloat16()
+    q[:, :, 0] = dk ** 0.5
+    sink = torch.tensor([-1000.0, 0.0, 40.0, 1000.0])
+    options = {"softcap": softcap} if softcap else {}
+    out, _ = _run(q, kc, vc, table, [n], [n], nq, nkv, dk, dv, page, scale=dk ** -0.5, split=False, sink=sink.cuda(), **options)
+    s = torch.einsum("thd,kd->htk", q.double(), keys[0][:, 0].double()) * float(torch.tensor(dk ** -0.5, dtype=torch.float32))
+    if softcap:
+        s = softcap * torch.tanh(s / softcap)
+    s = s.masked_fill(torch.ones((n, n)).triu(1).bool(), -float("inf"))
+    p = torch.softmax(torch.cat([s, sink.double()[:, None, None].expand(nq, n, 1)], -1), -1)[:, :, :n]
+    want = torch.einsum("htk,kd->thd", p, values[0][:, 0].double())
+    # the result's rounding (half a unit of 8 bits: 2^-8 of it), and of every weight that of its score (2^-24 of up to 400, scaled and in units of log 2) and of its exponential
+    size = torch.einsum("htk,kd->thd", p, values[0][:, 0].double().abs())
+    assert bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + size * 8 * 400 * 2.0 ** -24 + 1e-30).all())

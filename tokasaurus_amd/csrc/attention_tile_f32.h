@@ -21,10 +21,12 @@
 // of its key (the page layout's unit) and of its query, piece lane / 16 + 4 m.
 //   K pages: [page][kv head][dk / 8][P][8]    V pages: [page][kv head][P / 4][dv][4]
 // With bfloat16 storage and a tile a wavefront (prompts) a step is 32 keys and the weighted values go through the bfloat16
-// matrix cores in three exact pieces (at_pieces).  Measured, one prompt of 2,048 tokens with 32 heads of 64: 339 us with
-// 32-bit products of the weights and tiles in launch order, 101 us now; with a window of 1,024 and a soft cap 228 / 101;
-// one of 8,192 tokens 2,899 / 1,035; 32 heads of 128 780 / 303.  Results that differ from the rounded 64-bit ones: 2.9e-4
-// (3.8e-4 before).  What is left is the softmax's vector arithmetic.
+// matrix cores in three exact pieces (at_pieces), and references move seldom (AT_SLACK).  Bound by the softmax's vector instructions: some
+// 250 a step, of which references that move with every maximum took 45, exp2f with its care for results below 2^-126 40, and tanhf
+// 200.  us, with these / now, 32 heads of 64 over 8 kv heads: 2,048 tokens 93.0 / 75.4, with a window of 1,024 and a soft cap 93.1 / 73.1, 8,192
+// 964 / 841, 562 and 938 with a window and sinks 63.5 / 49.4, 300 with a cap 29.0 / 19.9; 32 heads of 128, 2,048 tokens 153 / 122, with a cap 195 / 132; 16 of
+// 80, 4 x 1,024 105 / 80; of 256, one block a step, with a cap 559 / 511.  Results that differ from the rounded 64-bit ones: 2.84e-4 / 2.74e-4
+// at 2,048 tokens of 64, with the cap 2.99e-4 / 2.94e-4, keys eight times as large 3.49e-4 / 3.46e-4.
 // Needs dk % 8 == 0, dv % 16 == 0, P % 16 == 0 (a step of 16 keys lies inside one page).
 #pragma once
 
@@ -92,10 +94,33 @@ struct ScoreShape {
 };
 // `in_caps`: scale / softcap, so that the product of the stored numbers is rounded once on its way to the tanh (a
 // product and a division a score before, of which the division is ten instructions).
-__device__ __forceinline__ float shaped_score(const ScoreShape& sh, float product, float scale, float in_caps, int dist, int head, int nq) {
-  float s = sh.softcap > 0.f ? sh.softcap * tanhf(product * in_caps) : product * scale;
-  if (sh.rel) s += sh.rel[(size_t)sh.bucket_of[min(max(dist, 0), sh.far)] * nq + head];
-  return s;
+// tanh of all of a lane's scores together: up to AT_TANH_NEAR, which scores below five eighths of the cap are, x + x^3 q(x^2) with q through the
+// Chebyshev nodes of (tanh(x) / x - 1) / x^2, 4.5e-9 of the result in front of the roundings (root mean square of all errors 2.6e-8, largest 7.4e-8: what
+// the result's own rounding has is 2.5e-8 and 6e-8), in 8 instructions where tanhf takes some 30 and branches; tanhf where a wavefront has a greater one.
+#define AT_TANH_NEAR 0.625f
+template <int N>
+__device__ __forceinline__ void capped_scores(float (&sc)[N], float softcap) {
+  float most = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) most = fmaxf(most, fabsf(sc[i]));
+  if (__any(most > AT_TANH_NEAR)) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      sc[i] = softcap * tanhf(sc[i]);
+      asm volatile("" : "+v"(sc[i]));  // (one after the other: side by side they take registers from the walk)
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float z = sc[i] * sc[i];
+    float q = -0.00571021764f;
+    q = fmaf(q, z, 0.0206441283f);
+    q = fmaf(q, z, -0.0537413992f);
+    q = fmaf(q, z, 0.133314639f);
+    q = fmaf(q, z, -0.333332837f);
+    sc[i] = softcap * fmaf(sc[i] * z, q, sc[i]);
+  }
 }
 
 // Blocks of 16 keys that a wavefront takes a step: two where the weighted values go through the bfloat16 matrix cores
@@ -123,6 +148,15 @@ __device__ __forceinline__ void at_pieces(const float (&p)[8], bf16x8_t (&piece)
   }
 #pragma unroll
   for (int n = 0; n < 3; ++n) __builtin_memcpy(&piece[n], packed[n], sizeof(piece[n]));
+}
+
+// What a score may be above its column's reference, and the reference as the exponents take it (0 while no key was seen).
+#define AT_LOG2E 1.44269504088896341f
+#define AT_SLACK 5.5f
+__device__ __forceinline__ float at_reference(float m) {
+  float r = m == -INFINITY ? 0.f : m * AT_LOG2E;
+  asm("" : "+v"(r));  // (rounded wherever it is used: in a difference the compiler would leave the rounding out, 2e-6 of a weight at scores of 30)
+  return r;
 }
 
 // The result of matrix products moved to ordinary registers at this place, in front of any branch.  The compiler waits for a
@@ -154,9 +188,9 @@ __device__ __forceinline__ void at_place(int& tile, int& hy) {
 // unnormalised in `part`; attention_tile_merge_kernel adds the chunks in ascending order.  For single decoded
 // tokens after long contexts, where a tile's walk would else keep one workgroup busy and the chip idle.
 //
-// (Four wavefronts a SIMD for heads up to 64 elements: one hides the loads and the exponentials of another.)
+// (Four wavefronts a SIMD for heads up to 64 elements, two up to 128: one hides the loads and the exponentials of another.)
 template <typename T, int KM, int VT, bool SPLIT, int NW, bool PART = false>
-__global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 1) void attention_tile_f32_kernel(
+__global__ __launch_bounds__(NW * TK_WAVE, SPLIT ? 1 : (KM <= 2 && VT <= 4 ? 4 : (KM <= 4 && VT <= 8 ? 2 : 1))) void attention_tile_f32_kernel(
     const T* __restrict__ q, int q_stride, T* __restrict__ out, int out_stride, const T* __restrict__ kcache,
     const T* __restrict__ vcache, const int* __restrict__ block_table, int table_stride,
     const int* __restrict__ q_start, const int* __restrict__ kv_len, const int* __restrict__ tile_req,
@@ -220,7 +254,6 @@ __global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 
   v4f o[VT];
   const bool sig = score_bias != nullptr;
   const float in_caps = shape.softcap > 0.f ? scale / shape.softcap : 0.f;
-  const bool shaped = shape.softcap > 0.f || shape.rel != nullptr;
   const float pb = sig && live ? score_bias[head] : 0.f;
   // (sigmoid weights have no maximum to follow: it stays 0, so every merge below multiplies by exp(0))
   float m_run, l_run;  // l_run: this lane's share of the column's sum
@@ -316,20 +349,25 @@ __global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 
     for (int h = 0; h < H; ++h) at_settle(s[h]);
     // this lane now holds, for its column, keys k0 + 16 h + 4 c + i: number 4 h + i below
     float sc[4 * H];
+#pragma unroll
+    for (int i = 0; i < 4 * H; ++i) sc[i] = s[i / 4][i % 4] * (shape.softcap > 0.f ? in_caps : scale);
+    if (shape.softcap > 0.f) capped_scores(sc, shape.softcap);
+    if (shape.rel) {
+#pragma unroll
+      for (int i = 0; i < 4 * H; ++i) {
+        const int dist = pos - (k0 + 16 * (i / 4) + 4 * c + i % 4);
+        sc[i] += shape.rel[(size_t)shape.bucket_of[min(max(dist, 0), shape.far)] * nq + head];
+      }
+    }
     float tmax = -INFINITY;
     if (seen_whole(k0)) {
 #pragma unroll
-      for (int i = 0; i < 4 * H; ++i) {
-        const int kp = k0 + 16 * (i / 4) + 4 * c + i % 4;
-        sc[i] = shaped ? shaped_score(shape, s[i / 4][i % 4], scale, in_caps, pos - kp, head, nq) : s[i / 4][i % 4] * scale;
-        tmax = fmaxf(tmax, sc[i]);
-      }
+      for (int i = 0; i < 4 * H; ++i) tmax = fmaxf(tmax, sc[i]);
     } else {
 #pragma unroll
       for (int i = 0; i < 4 * H; ++i) {
         const int kp = k0 + 16 * (i / 4) + 4 * c + i % 4;
-        const float si = s[i / 4][i % 4];
-        sc[i] = sees(kp) ? (shaped ? shaped_score(shape, si, scale, in_caps, pos - kp, head, nq) : si * scale) : -INFINITY;
+        sc[i] = sees(kp) ? sc[i] : -INFINITY;
         tmax = fmaxf(tmax, sc[i]);
         // a key that no column sees may be anything (a page's places behind the request's last token, a page given back):
         // its weight is zero, and so must its values be, or a NaN there would reach the sums
@@ -364,6 +402,24 @@ __global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 
       // 1 / (1 + exp(-(score + bias))); a masked score gives 1 / (1 + inf) = 0
 #pragma unroll
       for (int i = 0; i < 4 * H; ++i) p[i] = 1.0f / (1.0f + exp2f(-(sc[i] + pb) * 1.44269504088896341f));
+    } else if constexpr (H == 2) {
+      // Any reference near the greatest score will do, so it moves only when a score is AT_SLACK above it (terms up to 256, whose roundings are
+      // relative as ever), and the four lanes of a column need to agree on nothing in between.  exp2 of (score - reference) log2(e), the reference's
+      // product rounded alike for all of a column: the hardware's own exponential (a masked score gives exp2(-inf) = 0)
+      if (__any(tmax > m_run + AT_SLACK)) {
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 16, TK_WAVE));
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, TK_WAVE));
+        const float m_new = tmax > m_run + AT_SLACK ? tmax : m_run;
+        const float back = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(at_reference(m_run) - at_reference(m_new));
+        l_run *= back;
+#pragma unroll
+        for (int t = 0; t < VT; ++t) o[t] = o[t] * back;
+        m_run = m_new;
+      }
+      const float reference = at_reference(m_run);
+#pragma unroll
+      for (int i = 0; i < 4 * H; ++i) p[i] = __builtin_amdgcn_exp2f(fmaf(sc[i], AT_LOG2E, -reference));
+      l_run += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
     } else {
       tmax = fmaxf(tmax, __shfl_xor(tmax, 16, TK_WAVE));
       tmax = fmaxf(tmax, __shfl_xor(tmax, 32, TK_WAVE));
@@ -379,12 +435,13 @@ __global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 
       }
       m_run = m_new;
       l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
-      if constexpr (H == 2) l_run += (p[4] + p[5]) + (p[6] + p[7]);
     }
     // O^T += V^T P^T
     // (for all VT blocks, also those behind dv, whose lanes hold some of the head's first values and are never stored)
+    if constexpr (H == 1) {
 #pragma unroll
-    for (int t = 0; t < VT; ++t) o[t] = o[t] * alpha;
+      for (int t = 0; t < VT; ++t) o[t] = o[t] * alpha;
+    }
     if constexpr (decltype(wide)::value) {
 #pragma unroll
       for (int t = 0; t < VT; ++t)
@@ -507,8 +564,14 @@ __global__ __launch_bounds__(NW * TK_WAVE, (!SPLIT && KM <= 2 && VT <= 4) ? 4 : 
   if (sink && live && !sig) {
     // the sink joins the softmax like one more score: the maximum may rise to it
     const float sk = sink[head], m_all = fmaxf(m_run, sk);
-    keep = (m_run == -INFINITY) ? 0.f : expf(m_run - m_all);
-    l = l * keep + expf(sk - m_all);
+    if (H == 2 && m_run > -INFINITY) {  // (from the reference that the terms have)
+      const float above = fmaf(sk, AT_LOG2E, -at_reference(m_run));
+      keep = above > 0.f ? exp2f(-above) : 1.f;
+      l = l * keep + (above > 0.f ? 1.f : exp2f(above));
+    } else {
+      keep = (m_run == -INFINITY) ? 0.f : expf(m_run - m_all);
+      l = l * keep + expf(sk - m_all);
+    }
   }
   if (!live) return;
   const float inv = sig ? 1.f : keep / l;
