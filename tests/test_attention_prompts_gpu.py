@@ -187,3 +187,24 @@ def test_scores_that_rise_and_sinks(dk, dv, slope, softcap):
     # the result's rounding (half a unit of 8 bits: 2^-8 of it), and of every weight that of its score (2^-24 of up to 400, scaled and in units of log 2) and of its exponential
     size = torch.einsum("htk,kd->thd", p, values[0][:, 0].double().abs())
     assert bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + size * 8 * 400 * 2.0 ** -24 + 1e-30).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("split", [False, True])
+def test_capped_scores_depend_on_no_key_that_is_not_seen(dtype, split):
+    """The places behind a request's end, and the page of no request, hold zeros, numbers far beyond the cap, or NaN: the same bits.
+    (Scores of three to six tenths of the cap, where the ways to a tanh differ in their last bits.)"""
+    gen = torch.Generator().manual_seed(12)
+    lens, nq, nkv, d, page = [23, 70, 130], 4, 2, 64, 16
+    _, _, kc, vc, table = _paged(lens, nkv, d, d, page, gen)
+    scores = torch.zeros_like(kc)
+    scores[:, :, 0, :, 0] = torch.rand(kc.shape[0], nkv, page, generator=gen) * 6 + 6
+    kc = torch.where(kc.isnan(), kc, scores)
+    q = torch.zeros((sum(lens), nq, d), dtype=dtype)
+    q[:, :, 0] = 8
+    got = []
+    for stale in (0.0, 1e4, -1e4, float("nan")):
+        k, v = (torch.where(x.isnan(), torch.tensor(stale, dtype=x.dtype), x).to(dtype) for x in (kc, vc))
+        out, _ = _run(q, k, v, table, lens, lens, nq, nkv, d, d, page, scale=d ** -0.5, split=split, softcap=20.0)
+        got.append(out)
+    assert torch.isfinite(got[0]).all() and all(torch.equal(x, got[0]) for x in got[1:])

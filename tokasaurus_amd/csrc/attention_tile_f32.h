@@ -96,31 +96,33 @@ struct ScoreShape {
 // product and a division a score before, of which the division is ten instructions).
 // tanh of all of a lane's scores together: up to AT_TANH_NEAR, which scores below five eighths of the cap are, x + x^3 q(x^2) with q through the
 // Chebyshev nodes of (tanh(x) / x - 1) / x^2, 4.5e-9 of the result in front of the roundings (root mean square of all errors 2.6e-8, largest 7.4e-8: what
-// the result's own rounding has is 2.5e-8 and 6e-8), in 8 instructions where tanhf takes some 30 and branches; tanhf where a wavefront has a greater one.
+// the result's own rounding has is 2.5e-8 and 6e-8), in 8 instructions where tanhf takes some 30 and branches; tanhf of a greater one, which a wavefront that has none of them does not compute.
 #define AT_TANH_NEAR 0.625f
+__device__ __forceinline__ float near_tanh(float x) {
+  const float z = x * x;
+  float q = -0.00571021764f;
+  q = fmaf(q, z, 0.0206441283f);
+  q = fmaf(q, z, -0.0537413992f);
+  q = fmaf(q, z, 0.133314639f);
+  q = fmaf(q, z, -0.333332837f);
+  return fmaf(x * z, q, x);
+}
 template <int N>
 __device__ __forceinline__ void capped_scores(float (&sc)[N], float softcap) {
   float most = 0.f;
 #pragma unroll
   for (int i = 0; i < N; ++i) most = fmaxf(most, fabsf(sc[i]));
   if (__any(most > AT_TANH_NEAR)) {
+    // (every score by its own size: the greatest may be of another row, or of a key that no row sees, whose page holds anything)
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-      sc[i] = softcap * tanhf(sc[i]);
+      sc[i] = softcap * (fabsf(sc[i]) > AT_TANH_NEAR ? tanhf(sc[i]) : near_tanh(sc[i]));
       asm volatile("" : "+v"(sc[i]));  // (one after the other: side by side they take registers from the walk)
     }
     return;
   }
 #pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const float z = sc[i] * sc[i];
-    float q = -0.00571021764f;
-    q = fmaf(q, z, 0.0206441283f);
-    q = fmaf(q, z, -0.0537413992f);
-    q = fmaf(q, z, 0.133314639f);
-    q = fmaf(q, z, -0.333332837f);
-    sc[i] = softcap * fmaf(sc[i] * z, q, sc[i]);
-  }
+  for (int i = 0; i < N; ++i) sc[i] = softcap * near_tanh(sc[i]);
 }
 
 // Blocks of 16 keys that a wavefront takes a step: two where the weighted values go through the bfloat16 matrix cores
