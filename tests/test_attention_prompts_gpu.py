@@ -208,3 +208,23 @@ def test_capped_scores_depend_on_no_key_that_is_not_seen(dtype, split):
         out, _ = _run(q, k, v, table, lens, lens, nq, nkv, d, d, page, scale=d ** -0.5, split=split, softcap=20.0)
         got.append(out)
     assert torch.isfinite(got[0]).all() and all(torch.equal(x, got[0]) for x in got[1:])
+
+
+@pytest.mark.parametrize("split", [False, True])
+def test_capped_scores_have_no_error_but_their_rounding(split):
+    """Tokens that see themselves alone beside a sink that is near their score, so that the weight shows a score's error: exact products over a cap of
+    32, tanh of a half to five eighths."""
+    gen = torch.Generator().manual_seed(13)
+    n, d, page, cap, sink = 16384, 16, 64, 32.0, 16.25
+    x = (torch.rand((n,), generator=gen) / 8 + 0.5) * cap
+    kc, vc = torch.zeros((n // page, 1, d // 8, page, 8)), torch.ones((n // page, 1, page // 4, d, 4))
+    kc[:, 0, 0, :, 0] = x.view(-1, page)
+    q = torch.zeros((n, 1, d))
+    q[:, :, 0] = 1
+    table = torch.arange(n // page, dtype=torch.int32)[None]
+    out, _ = _run(q, kc, vc, table, [n], [n], 1, 1, d, d, page, scale=1.0, softcap=cap, section=1, sink=torch.tensor([sink]).cuda(), split=split)
+    w, score = out[:, 0, 0].double(), cap * torch.tanh(x.double() / cap)
+    off = (torch.log(w / (1 - w)) + sink - score) / score
+    # the mean of the roundings (6e-8 at most each of the tanh, of the score and of the weight's terms, root mean square of all 4e-8) over 16,384, eight times as much
+    assert abs(float(off.mean())) <= 2.5e-9
+    assert float(off.pow(2).mean().sqrt()) <= 6e-8

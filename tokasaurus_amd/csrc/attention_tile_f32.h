@@ -94,17 +94,20 @@ struct ScoreShape {
 };
 // `in_caps`: scale / softcap, so that the product of the stored numbers is rounded once on its way to the tanh (a
 // product and a division a score before, of which the division is ten instructions).
-// tanh of all of a lane's scores together: up to AT_TANH_NEAR, which scores below five eighths of the cap are, x + x^3 q(x^2) with q through the
-// Chebyshev nodes of (tanh(x) / x - 1) / x^2, 4.5e-9 of the result in front of the roundings (root mean square of all errors 2.6e-8, largest 7.4e-8: what
-// the result's own rounding has is 2.5e-8 and 6e-8), in 8 instructions where tanhf takes some 30 and branches; tanhf of a greater one, which a wavefront that has none of them does not compute.
+// tanh of all of a lane's scores together: up to AT_TANH_NEAR, which scores below five eighths of the cap are, x + x^3 q(x^2) with q of the least
+// greatest error in (tanh(x) / x - 1) / x^2, 1.5e-10 of the result in front of the roundings, in 9 instructions where tanhf takes some 30 and
+// branches; tanhf of a greater one, which a wavefront that has none of them does not compute.  Relative errors from 64 bits, root mean square
+// (largest), tanhf / this: up to an eighth 2.46e-8 (6.14e-8) / 2.44e-8 (5.97e-8), to a quarter 2.47e-8 (6.44e-8) / 2.45e-8 (6.02e-8), to a half 2.53e-8
+// (6.43e-8) / 2.51e-8 (6.31e-8), to the end 2.84e-8 (7.46e-8) / 2.82e-8 (7.16e-8).
 #define AT_TANH_NEAR 0.625f
 __device__ __forceinline__ float near_tanh(float x) {
   const float z = x * x;
-  float q = -0.00571021764f;
-  q = fmaf(q, z, 0.0206441283f);
-  q = fmaf(q, z, -0.0537413992f);
-  q = fmaf(q, z, 0.133314639f);
-  q = fmaf(q, z, -0.333332837f);
+  float q = 0.002147537f;
+  q = fmaf(q, z, -0.008182674f);
+  q = fmaf(q, z, 0.021702968f);
+  q = fmaf(q, z, -0.053947203f);
+  q = fmaf(q, z, 0.1333321f);
+  q = fmaf(q, z, -0.3333333f);
   return fmaf(x * z, q, x);
 }
 template <int N>
