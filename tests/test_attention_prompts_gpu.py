@@ -228,3 +228,30 @@ def test_capped_scores_have_no_error_but_their_rounding(split):
     # the mean of the roundings (6e-8 at most each of the tanh, of the score and of the weight's terms, root mean square of all 4e-8) over 16,384, eight times as much
     assert abs(float(off.mean())) <= 2.5e-9
     assert float(off.pow(2).mean().sqrt()) <= 6e-8
+
+
+@pytest.mark.parametrize("product,value", [(5.0, 3e38), (2.5e38, 1.0), (-2.5e38, 1.0)])
+def test_sums_that_are_finite_by_weights_of_one_and_less(product, value):
+    """A key whose values are near the largest numbers and whose score is above the others' by less than a reference lags behind; scores whose
+    product with log2(e) is beyond 32 bits: against 64 bits, with and without a sink far below."""
+    gen = torch.Generator().manual_seed(14)
+    n, at, d, page = 40, 33, 64, 16
+    keys, values, kc, vc, table = _paged([n], 1, d, d, page, gen)
+    side = abs(product) ** 0.5
+    keys[0][:] = 0
+    keys[0][:, 0, 0] = -side if product < -9 else 0  # (all others are lowest where the one is greatest)
+    keys[0][at, 0, 0] = side if product > 0 else -side / 2
+    values[0][at] = (values[0][at].sign().float() * value).bfloat16()
+    for p in range(-(-n // page)):
+        m = min(page, n - p * page)
+        kc[table[0, p], 0, :, :m] = keys[0][p * page: p * page + m, 0].view(m, d // 8, 8).permute(1, 0, 2)
+    vc[table[0, at // page], 0, at % page // 4, :, at % 4] = values[0][at, 0]
+    q = torch.zeros((n, 2, d), dtype=torch.bfloat16)
+    q[:, :, 0] = side
+    s = torch.einsum("thd,kd->htk", q.double(), keys[0][:, 0].double()).masked_fill(torch.ones((n, n)).triu(1).bool(), -float("inf"))
+    w = torch.softmax(s, -1)
+    want = torch.einsum("htk,kd->thd", w, values[0][:, 0].double())
+    size = torch.einsum("htk,kd->thd", w, values[0][:, 0].double().abs())
+    for sink in (None, torch.full((2,), -3.3e38).cuda()):
+        out, _ = _run(q, kc, vc, table, [n], [n], 2, 1, d, d, page, scale=1.0, split=False, sink=sink)
+        assert bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + size * n * 2.0 ** -22).all()), sink

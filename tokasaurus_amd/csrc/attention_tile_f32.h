@@ -407,7 +407,7 @@ __global__ __launch_bounds__(NW * TK_WAVE, SPLIT ? 1 : (KM <= 2 && VT <= 4 ? 4 :
       // 1 / (1 + exp(-(score + bias))); a masked score gives 1 / (1 + inf) = 0
 #pragma unroll
       for (int i = 0; i < 4 * H; ++i) p[i] = 1.0f / (1.0f + exp2f(-(sc[i] + pb) * 1.44269504088896341f));
-    } else if constexpr (H == 2) {
+    } else if constexpr (!decltype(wide)::value) {
       // Any reference near the greatest score will do, so it moves only when a score is AT_SLACK above it (terms up to 256, whose roundings are
       // relative as ever), and the four lanes of a column need to agree on nothing in between.  exp2 of (score - reference) log2(e), the reference's
       // product rounded alike for all of a column: the hardware's own exponential (a masked score gives exp2(-inf) = 0)
@@ -440,10 +440,11 @@ __global__ __launch_bounds__(NW * TK_WAVE, SPLIT ? 1 : (KM <= 2 && VT <= 4 ? 4 :
       }
       m_run = m_new;
       l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
+      if constexpr (H == 2) l_run += (p[4] + p[5]) + (p[6] + p[7]);
     }
     // O^T += V^T P^T
     // (for all VT blocks, also those behind dv, whose lanes hold some of the head's first values and are never stored)
-    if constexpr (H == 1) {
+    if constexpr (decltype(wide)::value) {
 #pragma unroll
       for (int t = 0; t < VT; ++t) o[t] = o[t] * alpha;
     }
@@ -480,13 +481,19 @@ __global__ __launch_bounds__(NW * TK_WAVE, SPLIT ? 1 : (KM <= 2 && VT <= 4 ? 4 :
   }
   };
   walk(std::integral_constant<bool, H == 1>{});
+  bool late = H == 2;  // whether the terms' reference is at_reference's, which may be behind the greatest score
   if constexpr (H == 2) {
-    bool finite = true;
+    // again, with the greatest score as reference and 32-bit products, where that cannot be: an infinite value, values whose sum is finite only with
+    // weights of one and less, a score whose reference is beyond 32 bits
+    bool finite = fabsf(at_reference(m_run)) < INFINITY;
 #pragma unroll
     for (int t = 0; t < VT; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) finite = finite && fabsf(o[t][i]) < INFINITY;
-    if (!__all(finite)) walk(std::integral_constant<bool, true>{});
+    if (!__all(finite)) {
+      walk(std::integral_constant<bool, true>{});
+      late = false;
+    }
   }
 #undef AT_PAGES
   if (__builtin_expect(odd, 0)) {
@@ -569,7 +576,7 @@ __global__ __launch_bounds__(NW * TK_WAVE, SPLIT ? 1 : (KM <= 2 && VT <= 4 ? 4 :
   if (sink && live && !sig) {
     // the sink joins the softmax like one more score: the maximum may rise to it
     const float sk = sink[head], m_all = fmaxf(m_run, sk);
-    if (H == 2 && m_run > -INFINITY) {  // (from the reference that the terms have)
+    if (late && m_run > -INFINITY) {  // (from the reference that the terms have)
       const float above = fmaf(sk, AT_LOG2E, -at_reference(m_run));
       keep = above > 0.f ? exp2f(-above) : 1.f;
       l = l * keep + (above > 0.f ? 1.f : exp2f(above));
