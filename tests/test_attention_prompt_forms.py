@@ -65,17 +65,16 @@ def test_shared_keys_give_the_same_as_pairs(lens, portions, nq, nkv, d, page, wi
         assert float((got - want).norm() / want.norm()) <= 2.0 ** -7, (row_tiles, waves)
 
 
-# products that climb by less than a row's reference allows, by just more, and far more a step of keys; that fall; and that stand still
-@pytest.mark.gpu
-@pytest.mark.parametrize("climb", [0.02, 0.2, 0.3, 3.0, -0.5, 0.0])
-@pytest.mark.parametrize("form", ["pairs", "single", "neighbours", "group", "sets", "decode"])
-def test_a_rows_reference_follows_its_products(climb, form):
-    """Against a softmax in 64 bits: key i has the product climb * i / log2(e) with every query, so the terms climb by 2^climb a key."""
-    nq, nkv, d, page, n = 4, 2, 64, 16, 700
+FORMS = {"pairs": (2, 1, 0), "single": (1, 2, 0), "neighbours": (2, 2, 0), "group": (2, 1, 1), "sets": (2, 1, 2), "decode": (1, 2, 0)}
+
+
+def of_products(rows, form):
+    """One request of n keys, of which key i has the product rows[i] / log2(e) with every query: what the kernel gives for all its
+    tokens (``decode``: for the last), and what a softmax in 64 bits does."""
+    nq, nkv, d, page, n = 4, 2, 64, 16, rows.numel()
     g = torch.Generator(device="cuda").manual_seed(3)
     pages = -(-n // page)
     k = torch.zeros((n, nkv, d), device="cuda")
-    rows = climb * torch.arange(n, device="cuda").float()
     k[:, :, 0] = (rows / 1.4427).bfloat16().float()[:, None]  # (two pieces of a bfloat16 number each: what is left of the first, by another element)
     k[:, :, 1] = (rows / 1.4427 - k[:, 0, 0]).bfloat16().float()[:, None]
     q = torch.zeros((n, nq, d), device="cuda")
@@ -88,8 +87,8 @@ def test_a_rows_reference_follows_its_products(climb, form):
     keys.view(pages, nkv, d // 8, page, 8).copy_(kp.view(pages, page, nkv, d // 8, 8).permute(0, 2, 3, 1, 4))
     values.view(pages, nkv, page // 4, d, 4).copy_(vp.view(pages, page // 4, 4, nkv, d).permute(0, 3, 1, 4, 2))
     i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
-    row_tiles, waves, grouped, tokens = {"pairs": (2, 1, 0, n), "single": (1, 2, 0, n), "neighbours": (2, 2, 0, n), "group": (2, 1, 1, n), "sets": (2, 1, 2, n),
-                                         "decode": (1, 2, 0, 1)}[form]
+    row_tiles, waves, grouped = FORMS[form]
+    tokens = 1 if form == "decode" else n
     req, row0, row1 = ops.attention_tiles([tokens], nq // nkv, row_tiles, pair=form == "pairs", fill=ops.ATTENTION_GROUP if grouped else 1)
     out = ops.paged_attention_mfma(q[-tokens:].reshape(tokens, -1).bfloat16(), keys, values, torch.arange(pages, device="cuda").int().view(1, -1), i32([0, tokens]),
                                    i32([n]), i32(req), i32(row0), row_tiles, nq, nkv, d, page, n, 64 * waves if form == "decode" else 768, scale=1.0, waves=waves,
@@ -97,6 +96,32 @@ def test_a_rows_reference_follows_its_products(climb, form):
     scores = (k[:, 0, 0] + k[:, 0, 1]).double().expand(tokens, n).clone()
     scores[torch.arange(n, device="cuda")[None] > torch.arange(n - tokens, n, device="cuda")[:, None]] = -float("inf")
     want = torch.einsum("tk,khd->thd", scores.softmax(-1), v.double()).repeat_interleave(nq // nkv, 1)
+    return out.double(), want
+
+
+# products that climb slowly, quickly and far a step of keys; that fall; and that stand still
+@pytest.mark.gpu
+@pytest.mark.parametrize("climb", [0.02, 0.2, 0.3, 3.0, -0.5, 0.0])
+@pytest.mark.parametrize("form", list(FORMS))
+def test_a_rows_reference_follows_its_products(climb, form):
+    """Key i has the product climb * i / log2(e) with every query, so the terms climb by 2^climb a key."""
+    out, want = of_products(climb * torch.arange(700, device="cuda").float(), form)
     # weights rounded to bfloat16 (2^-8 of each, of values of up to five) and the result's own rounding
-    assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 5 * 2.0 ** -8).all())
-    assert float((out.double() - want).norm() / want.norm()) <= 2.0 ** -8
+    assert bool(((out - want).abs() <= 2.0 ** -8 * want.abs() + 5 * 2.0 ** -8).all())
+    assert float((out - want).norm() / want.norm()) <= 2.0 ** -8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("after", [40, 300])
+def test_the_greatest_weight_is_not_rounded(form, after):
+    """A key that outweighs all others, met behind one that is below it by a little or a lot: its weight is the reference's own, exactly one, so
+    that the result has the rounding of bfloat16 and no other."""
+    rows = torch.full((448,), -30.0, device="cuda")
+    rows[3] = 0
+    for above in torch.linspace(5.0, 9.0, 33).tolist():
+        rows[after] = above
+        out, want = of_products(rows, form)
+        out, want = out[-1], want[-1]
+        # the result's rounding; the other key's weight, 2^-above of the sum, rounded by 2^-8 of it (values of up to five); 32-bit sums
+        assert bool(((out - want).abs() <= 2.0 ** -8 * want.abs() + 5 * 2.0 ** (-above - 8) + 5 * 2.0 ** -20).all()), above

@@ -43,8 +43,6 @@ __device__ __forceinline__ void store_f32x2(float* p, float a, float b) {
   }
 }
 
-#define ATTN_SLACK 8.f
-
 struct AttnArgs {
   const bf16_t* q;
   int q_stride;
@@ -62,7 +60,6 @@ struct AttnArgs {
   int n_tiles;
   int nq, nkv, group, P, p_shift, window;
   float scale_log2;  // scale * log2(e) > 0
-  float slack;       // what a product may be above a row's reference: ATTN_SLACK / scale_log2
   int split;         // keys per split, a multiple of 32
   int even;          // whether the wavefronts of a workgroup share the keys that are there evenly
   int max_splits;    // splits a tile may have (size of the scratch)
@@ -372,18 +369,15 @@ __device__ __forceinline__ void attention_item(const AttnArgs& a, const int tile
     }
   }
 
-  // The row's reference, in units of log 2 (0 while nothing was seen), up to which product it holds, and the sum of this lane's keys.  A term is
-  // exp2(product - reference): any reference near the greatest product will do, so it moves only when a product is ATTN_SLACK above it (terms
-  // up to 256, whose roundings are relative as ever), not with every greater one, and the four lanes of a row need to agree on nothing in
-  // between: 12 of some 53 vector instructions a step and row tile less.  us a layer of 8 kv heads, with every maximum / so: 32 heads of 64, 1,024
-  // tokens by neighbours 19.6 / 17.7, 2,048 by sets 45.3 / 39.6, 8,192 by groups 358 / 329; of 128, 4 x 1,024 by groups 73.5 / 67.9; 24 of 128, 1,000
-  // 23.3 / 22.1; decoded tokens the same.
-  float m_run[RT], m_most[RT], l_run[RT];
+  // Running maximum of the row's products and sum of this lane's keys.  The maximum itself is the terms' reference, in every step: so the greatest
+  // weight is exactly 1 in bfloat16 too.  A reference that may be behind it moves seldom (us a layer of 8 kv heads: 32 heads of 64, 2,048 tokens
+  // 47.1 / 42.0, 8,192 370 / 343), but rounds the greatest weight, 2^-8 of a result that is that key's values.  (The same reference with lanes that agree
+  // only in steps where one has a greater product gives these bits and is slower, 51.7 and 406.)
+  float m_run[RT], l_run[RT];
   f32x4_t acc[RT][DT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
-    m_run[rt] = 0.f;
-    m_most[rt] = -INFINITY;
+    m_run[rt] = -INFINITY;
     l_run[rt] = 0.f;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) acc[rt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -431,24 +425,23 @@ __device__ __forceinline__ void attention_item(const AttnArgs& a, const int tile
         }
       }
       float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
-      if (__any(mx > m_most[rt])) {
-        // some row went past what its reference allows: the greatest product so far becomes the reference of those that did, and what
-        // was summed is weighed (the others by one)
-        mx = max_over_quarters(mx);
-        const bool moves = mx > m_most[rt];
-        const float m_new = moves ? mx * a.scale_log2 : m_run[rt];
-        const float alpha = m_most[rt] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[rt] - m_new);
+      mx = max_over_quarters(mx);
+      const float m_new = fmaxf(m_run[rt], mx);
+      const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+      const float mc = m_use * a.scale_log2;
+      if (__any(m_new > m_run[rt])) {
+        // some row's maximum moved: weigh what was summed so far
+        const float alpha = __builtin_amdgcn_exp2f(fmaf(m_run[rt], a.scale_log2, -mc));  // 0 while nothing was seen
         l_run[rt] *= alpha;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) acc[rt][dt] *= alpha;
         m_run[rt] = m_new;
-        m_most[rt] = moves ? mx + a.slack : m_most[rt];
       }
       float p[8];
       bf16x8_t pb;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        p[e] = __builtin_amdgcn_exp2f(fmaf(sc[e], a.scale_log2, -m_run[rt]));
+        p[e] = __builtin_amdgcn_exp2f(fmaf(sc[e], a.scale_log2, -mc));
         pb[e] = (__bf16)p[e];
       }
       l_run[rt] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
@@ -621,7 +614,7 @@ __device__ __forceinline__ void attention_item(const AttnArgs& a, const int tile
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
     l_run[rt] = l;
-    if (m_most[rt] == -INFINITY) m_run[rt] = -INFINITY;  // (nothing seen: as the merges take it)
+    m_run[rt] *= a.scale_log2;  // from here on in units of log 2, as the merges take it
   }
   const bool hand_over = SHARED && nsp > 1;  // the same for every wavefront of the workgroup
   if (!GROUPED && NW > 1) {

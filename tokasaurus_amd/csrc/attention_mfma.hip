@@ -278,7 +278,6 @@ TK_API int tk_paged_attention_mfma(const void* q, int q_stride, void* out, int o
   a.p_shift = 0;
   while ((1 << a.p_shift) < P) ++a.p_shift;
   a.scale_log2 = scale * 1.4426950408889634f;
-  a.slack = ATTN_SLACK / a.scale_log2;
   a.split = split; a.even = even; a.max_splits = max_splits; a.part_o = part_o; a.part_ml = part_ml;
   a.tickets = (max_splits > 1 && row_tiles == 1) ? tickets : nullptr;
   const bool ok = grouped ? launch_group_d(a, d / 16, grouped, stream)
