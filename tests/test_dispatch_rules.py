@@ -123,3 +123,15 @@ def test_rows_that_gate_and_up_take_in_the_hand_written_product():
     assert ops.glu_rows(4096, 14336) == 64 and ops.glu_rows(4096, 11008) == 16
     assert ops.glu_rows(5120, 13824) == ops.glu_rows(8192, 28672) == 16
     assert ops.glu_rows(2080, 8192) == ops.skinny_rows(2080, paired=True)
+
+
+def test_32_bit_products_of_more_rows_than_a_grid_has_are_not_cut():
+    # (the sums of K's parts are added by a grid with a row of workgroups a token; whole tiles of either kind take any number of rows)
+    from tokasaurus_amd.kernels.library import load
+
+    cuts = load("core").tk_gemm_f32_cuts
+    for m in (65536, 65568, 65600, 67264, 71168, 76736, 131072, 1 << 20):
+        for n in (16, 64, 128, 256, 1024, 1028, 4096):
+            for k in (1024, 2048, 8192, 14336):
+                assert cuts(m, n, k) == 1, (m, n, k)
+    assert cuts(301, 2048, 8192) > 1 and cuts(301, 2050, 8192) == 1

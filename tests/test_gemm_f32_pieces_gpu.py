@@ -70,3 +70,11 @@ def test_numbers_whose_pieces_are_lost(m, down, up):
     a[:, 1:] = 0  # one product a sum
     got, want = ops.gemm_generic(a, w), a.double() @ w.double().T
     assert bool(((got.double() - want).abs() <= 2.0 ** -22 * want.abs()).all())
+
+
+def test_more_rows_than_a_grid_has():
+    g = torch.Generator(device="cuda").manual_seed(2)
+    m, n, k = 65568, 16, 1024
+    a, w = torch.randn((m, k), generator=g, device="cuda"), torch.randn((n, k), generator=g, device="cuda")
+    residual = torch.randn((m, n), generator=g, device="cuda")
+    assert error(ops.gemm_generic(a, w, residual=residual), a.double() @ w.double().T + residual.double()) <= 1e-6

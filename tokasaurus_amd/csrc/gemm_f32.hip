@@ -596,6 +596,9 @@ static long gf_tiles(int M, int N, int tm, int tn) {
   return (((long)N + 32 * tn - 1) / (32 * tn) + 7) / 8 * 8 * (((long)M + 32 * tm - 1) / (32 * tm));
 }
 
+// Whether gemm_f32_sum_kernel takes parts of these results: four columns a thread, a row of workgroups a token.
+static bool gf_cuts_add(int M, int N) { return (N & 3) == 0 && M < 65536; }
+
 // Whether products go by bfloat16 pieces: the rows of a tile (64 or 128, 128 weight rows), 0 if not; and into how many parts they cut K, the same
 // for both ends of a call.  They pay from 7 * 2^27 multiply-adds on (rows counted in tiles of 64), where the steps' work outweighs a longer beginning:
 // 200 rows 2,816 x 1,024 25.3 / 25.4 us, 160 rows 2,048 x 2,048 25.8 / 27.7, 128 rows 3,072 x 2,048 26.6 / 27.0, 64 rows 19.7 / 21.5; 400 rows 8,192 x 256
@@ -608,7 +611,7 @@ static int gf_pieces_tile(int M, int N, int K, int* cuts) {
   double best = 0;
   int tile = 0;
   for (int tm = 2; tm <= 4; tm += 2)
-    for (int c = 1; c <= ((N & 3) == 0 ? most : 1); ++c) {
+    for (int c = 1; c <= (gf_cuts_add(M, N) ? most : 1); ++c) {
       const long groups = gf_tiles(M, N, tm, 4) * c, rest = groups % 512;
       const double one = tm == 2 ? 1.05 : 1.6, two = tm == 2 ? 1.58 : 2.75;
       const double us = (groups / 512 * two + (rest == 0 ? 0 : (rest <= 256 ? one : two))) * ((steps + c - 1) / c) + (c > 1 ? 2 + c * (4e-6 / 3) * M * N : 0);
@@ -624,7 +627,7 @@ static int gf_pieces_tile(int M, int N, int K, int* cuts) {
 TK_API int tk_gemm_f32_cuts(int M, int N, int K) {
   int split_cuts;
   if (gf_pieces_tile(M, N, K, &split_cuts)) return split_cuts;
-  if (M <= 16 || (N & 3) != 0) return 1;
+  if (M <= 16 || !gf_cuts_add(M, N)) return 1;
   long cuts = 1280 / gf_tiles(M, N, M <= 32 ? 1 : 2, 2);
   const long most = K / 256;
   if (cuts > most || M <= 32) cuts = most;  // (few tokens: chains of 32 elements in every part)
@@ -680,7 +683,7 @@ TK_API int tk_gemm_f32(const void* A, int lda, const void* W, void* C, int ldc, 
   TK_REQUIRE(M >= 0 && N > 0 && K > 0 && lda >= K && ldc >= N, "gemm_f32: bad sizes M=%d N=%d K=%d lda=%d ldc=%d", M, N, K, lda, ldc);
   TK_REQUIRE(!residual || ldr >= N, "gemm_f32: residual stride %d < N %d", ldr, N);
   TK_REQUIRE(tk_gemm_f32_takes(A, lda, W, K), "gemm_f32: rows of A and W must start at multiples of 16 bytes");
-  TK_REQUIRE(cuts >= 1 && cuts <= (K + 31) / 32 && cuts < 65536 && (cuts == 1 || (part && (N & 3) == 0 && M > 16 && M < 65536)),
+  TK_REQUIRE(cuts >= 1 && cuts <= (K + 31) / 32 && cuts < 65536 && (cuts == 1 || (part && gf_cuts_add(M, N) && M > 16)),
              "gemm_f32: K=%d in %d parts", K, cuts);
   if (M == 0) return 0;
   GemmF32Args a = {(const float*)A, lda, (const float*)W, (float*)C, ldc, (const float*)residual, ldr, (const float*)bias, M, N, K,
