@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from tokasaurus_amd.kernels import ops
+from tokasaurus_amd.kernels.library import load
 
 pytestmark = pytest.mark.gpu
 
@@ -28,11 +29,31 @@ def test_errors_are_no_larger_than_unsplit(m, n, k):
     bias, residual = torch.randn((n,), generator=g, device="cuda"), torch.randn((m, n + 3), generator=g, device="cuda")[:, 1 : n + 1]
     want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
     got = ops.gemm_generic(a, w)
-    # a sum of K products, each rounded, and what is left of each product (2^-20 at most)
-    assert bool(((got.double() - want).abs() <= ((k + 2) * 2.0 ** -24 + 2.0 ** -20) * size).all())
+    # a sum of K products, each rounded, and what is left of each product (2^-30 at most)
+    assert bool(((got.double() - want).abs() <= ((k + 2) * 2.0 ** -24 + 2.0 ** -30) * size).all())
     assert error(got, want) <= error(unsplit(a, w), want)
     want = want + bias.double() + residual.double()
     assert error(ops.gemm_generic(a, w, bias=bias, residual=residual), want) <= error(unsplit(a, w, bias=bias, residual=residual), want) * 1.01
+
+
+# a tile of 64 rows and one of 128, K in one part each (a part of a row without terms is a sum of zero, and made unsplit)
+@pytest.mark.parametrize("m,n,k", [(33, 28672, 512), (2048, 2048, 2048)])
+@pytest.mark.parametrize("terms", [1, 2, 3, 5, 8, 16, 40])
+def test_few_terms_a_row(m, n, k, terms):
+    """Ordinary numbers, the row with all bits of its numbers set among them, element by element."""
+    assert load("core").tk_gemm_f32_cuts(m, n, k) == 1
+    g = torch.Generator(device="cuda").manual_seed(m + terms)
+    a, w = torch.zeros((m, k), device="cuda"), torch.randn((n, k), generator=g, device="cuda")
+    at = torch.rand((m, k), generator=g, device="cuda").topk(terms, -1).indices
+    a.scatter_(1, at, torch.randn((m, terms), generator=g, device="cuda"))
+    a[0] = a[0].sign() * (1 + 2.0 ** -7 - 2.0 ** -23)
+    w[:100] = w[:100].sign() * (1 + 2.0 ** -7 - 2.0 ** -23)
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    got = ops.gemm_generic(a, w)
+    # the greatest pieces' product is exact; each further one is added with a rounding (by truncation at worst), the others once, at the end;
+    # what is left of a product is under 2^-30
+    assert bool(((got.double() - want).abs() <= ((2 * terms - 1) * 2.0 ** -24 + 2.0 ** -29) * size).all())
+    assert error(got, want) <= error(unsplit(a, w), want) * (1.01 if terms == 1 else 1)
 
 
 @pytest.mark.parametrize("m", [70, 300])
@@ -69,7 +90,7 @@ def test_numbers_whose_pieces_are_lost(m, down, up):
     assert error(got, want) <= 2e-6
     a[:, 1:] = 0  # one product a sum
     got, want = ops.gemm_generic(a, w), a.double() @ w.double().T
-    assert bool(((got.double() - want).abs() <= 2.0 ** -22 * want.abs()).all())
+    assert bool(((got.double() - want).abs() <= 2.0 ** -24 * want.abs()).all())
 
 
 def test_more_rows_than_a_grid_has():

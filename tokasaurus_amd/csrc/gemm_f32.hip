@@ -437,22 +437,26 @@ __global__ __launch_bounds__(256) void gemm_f32_stream_kernel(GemmF32Args a) {
 }
 
 // Many products over a K of a multiple of 32: the numbers as exact sums of three bfloat16 numbers (their 24 bits, 8 at a time, by truncation)
-// on the matrix cores' bfloat16 multiply-adds, whose products are exact and whose sums are 32-bit.  Of the nine products of pieces the six
-// largest count; what is left out is under 2^-20 of a product and 2^-24 in the mean, and a step of 32 elements is added up inside one instruction, where the
-// 32-bit instruction rounds after every fourth: errors against 64 bits are smaller than the unsplit products' (below).
-// Six instructions of 16 x 16 x 32 take 102 cycles where eight of 16 x 16 x 4 take 272; the pieces, made by every wavefront for itself, cost as much as
-// the products, side by side with them where two workgroups share a compute unit.
-// LOW: the five smaller products in sums of their own, where registers allow it (a third of the error).
+// on the matrix cores' bfloat16 multiply-adds, whose products are exact and whose sums are 32-bit.  Of the nine products of pieces all count but that
+// of the two smallest, under 2^-30 of the whole (without the next two, (1, 2) and (2, 1), up to 2^-21 would be left out, always towards zero: a
+// product by itself would be off by 6.5e-8 root mean square and 4.5e-7 at most, where a rounding is 2.5e-8 and 6.0e-8).  The largest are summed by
+// themselves, one rounding for 32 elements where the 32-bit instruction rounds after every fourth, the others beside them: errors against 64 bits
+// are not larger than the unsplit products', from one term a row to dense rows (below).
+// Eight instructions of 16 x 16 x 32 take 136 cycles where eight of 16 x 16 x 4 take 272; the pieces, made by every wavefront for itself, cost nearly as
+// much as the products, side by side with them where two workgroups share a compute unit.
 // Pieces reach down to 2^-133, and an infinite number has pieces that are no numbers: a workgroup with a sum that is not finite, or below 2^-60
 // (zero too: numbers of less than 2^-133 have no pieces at all), or with an operand of 2^40 and more, does its products again, unsplit.  (Else the bits
 // below 2^-133 that are lost are at most 2^-33 of a sum, and a row of zeros costs its tiles their time twice.)
 // Two wavefronts make the pieces of the same rows: each looks at half a step's numbers, which the other has last (16 instructions of some 370 a
 // step; 301 rows 16,384 x 2,048 151.9 us without, 152.1 with, 2,048 rows 697 and 700).
-// us unsplit / split, and errors where both were taken (root of the squares' sums over that of the results):
-//   33 rows   16,384 x 2,048 50.3 / 41.3 (3.7e-7 / 1.5e-7), 2,048 x 8,192 33.8 / 28.5 (3.1e-7 / 1.5e-7), 128,256 x 2,048 522 / 270 (8.1e-7 / 2.8e-7)
-//   200       16,384 x 2,048 153 / 110 (8.1e-7 / 4.9e-7), 2,048 x 8,192 79.9 / 61.9 (5.2e-7 / 3.6e-7), 2,048 x 2,048 31.0 / 27.2 (2.9e-7 / 1.2e-7)
-//   301       16,384 x 2,048 177 / 148 (8.1e-7 / 2.0e-7), 2,048 x 8,192 98.3 / 79.7, 2,048 x 2,048 36.2 / 31.8, 3,072 x 2,048 49.9 / 39.4
-//   2,048     16,384 x 2,048 1,017 / 697 (8.1e-7 / 7.0e-7), 2,048 x 8,192 565 / 357 (1.6e-6 / 1.0e-6), 2,048 x 2,048 153 / 112 (8.1e-7 / 4.9e-7)
+// us unsplit / split, weights from memory:
+//   33 rows   16,384 x 2,048 50.1 / 46.2, 2,048 x 8,192 32.5 / 29.6, 128,256 x 2,048 512 / 288
+//   200       16,384 x 2,048 146 / 121, 2,048 x 8,192 79.2 / 65.1, 2,048 x 2,048 28.5 / 25.4
+//   301       16,384 x 2,048 177 / 168, 2,048 x 8,192 96.6 / 89.8, 2,048 x 2,048 32.7 / 30.2, 3,072 x 2,048 44.6 / 39.2
+//   2,048     16,384 x 2,048 1,020 / 840, 2,048 x 8,192 565 / 423, 2,048 x 2,048 145 / 127
+// Errors, root of the squares' sums over that of the results, unsplit / split: 70 rows 7,300 x 1,024 2.9e-7 / 9.8e-8, of numbers in [1, 2) 1.27e-7 / 4.5e-8,
+// of 2, 8 and 32 terms a row 3.5e-8 / 3.5e-8, 5.2e-8 / 5.2e-8 and 6.8e-8 / 5.0e-8; 2,048 rows 2,048 x 2,048 8.1e-7 / 2.7e-7, in [1, 2) 6.8e-7 / 2.5e-7, of 1, 2,
+// 8 and 32 terms 2.53e-8 / 2.53e-8, 3.1e-8 / 2.6e-8, 5.4e-8 / 2.8e-8 and 1.0e-7 / 4.3e-8.
 typedef __attribute__((ext_vector_type(8))) __bf16 gf_bf16x8_t;
 
 // (most: the greatest number of `lo` so far)
@@ -478,7 +482,7 @@ __device__ __forceinline__ void gf_pieces(f4 lo, f4 hi, gf_bf16x8_t (&piece)[3],
 }
 
 #define GP_STAGES 2  // steps in local memory: two workgroups of the largest tile share a compute unit
-template <int TM, int TN, bool LOW>
+template <int TM, int TN>
 __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) {
   extern __shared__ __align__(16) float tile[];  // [GP_STAGES][32 * (TN + TM)][32], weight rows first, pieces in places as above
   constexpr int ROWS = 32 * (TN + TM), LOADS = ROWS / 32, STAGES = GP_STAGES;
@@ -502,8 +506,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) 
     for (int i = 0; i < LOADS; ++i)
       load_to_lds((const bf16_t*)(src[i] + (size_t)step * 32), lds + (unsigned)((place * ROWS + 32 * i + 8 * wave) * 32 * (int)sizeof(float)));
   };
-  f4 acc[1][TN][TM], small[LOW ? TN : 1][LOW ? TM : 1];
-  auto low = [&](int t, int u) -> f4& { return LOW ? small[LOW ? t : 0][LOW ? u : 0] : acc[0][t][u]; };
+  f4 acc[1][TN][TM], small[TN][TM];
   const int last = 4 * ((wave ^ (wave >> 1)) & 1);  // the halves of a step change places between wavefronts that share rows
   const int piece[2] = {((last + q) ^ gs_swizzle(r)) * 4, ((4 - last + q) ^ gs_swizzle(r)) * 4};
   const float* wrow = tile + ((wave & 1) * 16 * TN + r) * 32;
@@ -513,7 +516,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) 
 #pragma unroll
     for (int t = 0; t < TN; ++t)
 #pragma unroll
-      for (int u = 0; u < TM; ++u) acc[0][t][u] = low(t, u) = (f4){0.f, 0.f, 0.f, 0.f};
+      for (int u = 0; u < TM; ++u) acc[0][t][u] = small[t][u] = (f4){0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < STAGES - 1 && s < steps; ++s) ask(s, s);
     int here = 0, next = STAGES - 1;
 #pragma unroll 1
@@ -545,11 +548,13 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) 
           gf_pieces(*(const f4*)(xr + 16 * u * 32 + piece[0]), *(const f4*)(xr + 16 * u * 32 + piece[1]), x, most);
 #define GP_PRODUCTS(SUM, I, J) \
   _Pragma("unroll") for (int t = 0; t < TN; ++t) SUM = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][I], x[J], SUM, 0, 0, 0)
-          GP_PRODUCTS(low(t, u), 2, 0);
-          GP_PRODUCTS(low(t, u), 0, 2);
-          GP_PRODUCTS(low(t, u), 1, 1);
-          GP_PRODUCTS(low(t, u), 1, 0);
-          GP_PRODUCTS(low(t, u), 0, 1);
+          GP_PRODUCTS(small[t][u], 2, 1);
+          GP_PRODUCTS(small[t][u], 1, 2);
+          GP_PRODUCTS(small[t][u], 2, 0);
+          GP_PRODUCTS(small[t][u], 0, 2);
+          GP_PRODUCTS(small[t][u], 1, 1);
+          GP_PRODUCTS(small[t][u], 1, 0);
+          GP_PRODUCTS(small[t][u], 0, 1);
           GP_PRODUCTS(acc[0][t][u], 0, 0);
 #undef GP_PRODUCTS
         }
@@ -564,7 +569,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) 
   for (int t = 0; t < TN; ++t)
 #pragma unroll
     for (int u = 0; u < TM; ++u) {
-      if (LOW) acc[0][t][u] += low(t, u);
+      acc[0][t][u] += small[t][u];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float size = fabsf(acc[0][t][u][j]);
@@ -601,10 +606,11 @@ static bool gf_cuts_add(int M, int N) { return (N & 3) == 0 && M < 65536; }
 
 // Whether products go by bfloat16 pieces: the rows of a tile (64 or 128, 128 weight rows), 0 if not; and into how many parts they cut K, the same
 // for both ends of a call.  They pay from 7 * 2^27 multiply-adds on (rows counted in tiles of 64), where the steps' work outweighs a longer beginning:
-// 200 rows 2,816 x 1,024 25.3 / 25.4 us, 160 rows 2,048 x 2,048 25.8 / 27.7, 128 rows 3,072 x 2,048 26.6 / 27.0, 64 rows 19.7 / 21.5; 400 rows 8,192 x 256
-// 28.2 / 22.7 and 4,096 x 512 30.9 / 26.0, 200 rows 2,048 x 2,048 31.0 / 27.2.
-// Tile and parts are those of the least time by the steps of 32 elements of K that a compute unit takes one after the other (us a
-// step with one workgroup on it and with two, which fit: 1.05 and 1.58 for 64 rows, 1.6 and 2.75 for 128) and the parts' way through memory.
+// 200 rows 2,816 x 1,024 25.3 / 25.4 us, 160 rows 2,048 x 2,048 25.8 / 27.7, 128 rows 3,072 x 2,048 26.6 / 27.0, 64 rows 19.7 / 21.5 (with six of
+// the eight products); 400 rows 8,192 x 256 26.5 / 20.8 and 4,096 x 512 29.6 / 25.7, 200 rows 2,048 x 2,048 28.5 / 25.4.
+// Tile and parts are those of the least time by the steps of 32 elements of K that a compute unit takes one after the other (in proportion to
+// a step's time with one workgroup on it and with two, which fit: 1.25 and 1.9 us for 64 rows, 1.95 and 3.4 for 128) and the parts' way through memory.
+// What it takes was the best of 1 to 4 parts and its own, or within 1 % of it, at twenty sizes of 64 to 4,096 rows.
 static int gf_pieces_tile(int M, int N, int K, int* cuts) {
   const long most = K / 256 < 32 ? K / 256 : 32, steps = K / 32;
   if (M <= 32 || K % 32 != 0 || most < 1 || ((long)M + 63) / 64 * 64 * N * K < 7L << 27) return 0;
@@ -650,12 +656,12 @@ static bool gf_launch(const GemmF32Args& a, int cuts, hipStream_t stream) {
   return true;
 }
 
-template <int TM, bool LOW>
+template <int TM>
 static bool gf_launch_pieces(const GemmF32Args& a, int cuts, hipStream_t stream) {
   const long grid = gf_tiles(a.M, a.N, TM, 4);
   if (grid > 0x7fffffffL) return false;
   const size_t lds = (size_t)GP_STAGES * 32 * (TM + 4) * 32 * sizeof(float);  // (64 KB at most)
-  hipLaunchKernelGGL((gemm_f32_pieces_kernel<TM, 4, LOW>), dim3((unsigned)grid, cuts), dim3(256), lds, stream, a);
+  hipLaunchKernelGGL((gemm_f32_pieces_kernel<TM, 4>), dim3((unsigned)grid, cuts), dim3(256), lds, stream, a);
   return true;
 }
 
@@ -698,8 +704,8 @@ TK_API int tk_gemm_f32(const void* A, int lda, const void* W, void* C, int ldc, 
   bool ok;
   int unused;
   const int pieces = gf_pieces_tile(M, N, K, &unused);
-  if (pieces == 64) ok = gf_launch_pieces<2, true>(a, cuts, stream);
-  else if (pieces) ok = gf_launch_pieces<4, false>(a, cuts, stream);
+  if (pieces == 64) ok = gf_launch_pieces<2>(a, cuts, stream);
+  else if (pieces) ok = gf_launch_pieces<4>(a, cuts, stream);
   else if (M <= 32) ok = gf_launch<1, 2, 8>(a, cuts, stream);
   else if (gf_tiles(M, N, 4, 4) >= 512) ok = gf_launch<4, 4, 1>(a, cuts, stream);
   else ok = gf_launch<2, 2, 1>(a, cuts, stream);
