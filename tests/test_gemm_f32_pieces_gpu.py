@@ -99,3 +99,16 @@ def test_more_rows_than_a_grid_has():
     a, w = torch.randn((m, k), generator=g, device="cuda"), torch.randn((n, k), generator=g, device="cuda")
     residual = torch.randn((m, n), generator=g, device="cuda")
     assert error(ops.gemm_generic(a, w, residual=residual), a.double() @ w.double().T + residual.double()) <= 1e-6
+
+
+def test_many_products_whose_pieces_lose_a_little():
+    """65,536 numbers of 2^-125 beside some of up to 2^39 and one product of 2^-59 behind them: what their pieces lose is little of a product and 2^-20 of the sum."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    m, n, k = 64, 901, 65536
+    assert load("core").tk_gemm_f32_cuts(m, n, k) == 1
+    a = (torch.rand((m, k), generator=g, device="cuda") + 1) * 2.0 ** -125
+    w = (torch.rand((n, k), generator=g, device="cuda") + 1) * 2.0 ** 38
+    a[:, -1], w[:, -1] = 2.0 ** -60, 2.0
+    got, want = ops.gemm_generic(a, w), a.double() @ w.double().T
+    # one rounding, and up to 31 of the small products added behind the great one, each below half a place of it
+    assert bool(((got.double() - want).abs() <= (2.0 ** -24 + 31 * 2.0 ** (-86 + 1.2 + 59)) * want).all())

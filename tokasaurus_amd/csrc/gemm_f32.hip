@@ -444,9 +444,9 @@ __global__ __launch_bounds__(256) void gemm_f32_stream_kernel(GemmF32Args a) {
 // are not larger than the unsplit products', from one term a row to dense rows (below).
 // Eight instructions of 16 x 16 x 32 take 136 cycles where eight of 16 x 16 x 4 take 272; the pieces, made by every wavefront for itself, cost nearly as
 // much as the products, side by side with them where two workgroups share a compute unit.
-// Pieces reach down to 2^-133, and an infinite number has pieces that are no numbers: a workgroup with a sum that is not finite, or below 2^-60
-// (zero too: numbers of less than 2^-133 have no pieces at all), or with an operand of 2^40 and more, does its products again, unsplit.  (Else the bits
-// below 2^-133 that are lost are at most 2^-33 of a sum, and a row of zeros costs its tiles their time twice.)
+// Pieces reach down to 2^-133, and an infinite number has pieces that are no numbers: a workgroup with a sum that is not finite, or below GP_LEAST
+// (zero too: numbers of less than 2^-133 have no pieces at all), or with an operand of GP_MOST and more, does its products again, unsplit.  (Else the
+// bits below 2^-133 that are lost are at most 2^-102 of each of the K products, K 2^-52 of a sum, and a row of zeros costs its tiles their time twice.)
 // Two wavefronts make the pieces of the same rows: each looks at half a step's numbers, which the other has last (16 instructions of some 370 a
 // step; 301 rows 16,384 x 2,048 151.9 us without, 152.1 with, 2,048 rows 697 and 700).
 // us unsplit / split, weights from memory:
@@ -481,6 +481,8 @@ __device__ __forceinline__ void gf_pieces(f4 lo, f4 hi, gf_bf16x8_t (&piece)[3],
   }
 }
 
+#define GP_LEAST 0x1p-50f
+#define GP_MOST 0x1p30f
 #define GP_STAGES 2  // steps in local memory: two workgroups of the largest tile share a compute unit
 template <int TM, int TN>
 __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) {
@@ -564,7 +566,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) 
     }
   };
   walk(std::integral_constant<bool, false>{});
-  bool plain = most < 0x1p40f;
+  bool plain = most < GP_MOST;
 #pragma unroll
   for (int t = 0; t < TN; ++t)
 #pragma unroll
@@ -573,7 +575,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) 
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float size = fabsf(acc[0][t][u][j]);
-        plain = plain && size >= 0x1p-60f && size < INFINITY;
+        plain = plain && size >= GP_LEAST && size < INFINITY;
       }
     }
   if (__syncthreads_or(!plain)) walk(std::integral_constant<bool, true>{});
