@@ -101,6 +101,34 @@ def test_more_rows_than_a_grid_has():
     assert error(ops.gemm_generic(a, w, residual=residual), a.double() @ w.double().T + residual.double()) <= 1e-6
 
 
+# tiles of 64 and of 128 rows, K in one part and in several, columns that no 16 bytes hold
+@pytest.mark.parametrize("m,n,k,cuts", [(33, 28672, 512, False), (70, 7300, 1024, True), (2048, 2048, 2048, False), (300, 7300, 1024, True), (65, 7170, 1056, False)])
+def test_a_row_changes_no_other_row(m, n, k, cuts):
+    """Zeros, numbers without pieces, very large ones, infinity and NaN in a row of either operand: the bits of all results that are not made of it
+    stay, and its own are right."""
+    assert (load("core").tk_gemm_f32_cuts(m, n, k) > 1) == cuts
+    g = torch.Generator(device="cuda").manual_seed(m)
+    a, w = torch.randn((m, k), generator=g, device="cuda"), torch.randn((n, k), generator=g, device="cuda")
+    residual = torch.randn((m, n), generator=g, device="cuda")
+    before = ops.gemm_generic(a, w, residual=residual)
+    odd = [torch.zeros(k), torch.randn(k) * 2.0 ** -118, torch.randn(k) * 2.0 ** 31, torch.randn(k) * 2.0 ** 60, torch.full((k,), float("nan")),
+           torch.randn(k).scatter(0, torch.tensor([k - 1]), float("inf")), torch.randn(k).scatter(0, torch.tensor([3]), 2.0 ** 40)]
+    for row in odd:
+        for side, at in (("a", m // 2), ("w", n - 3)):
+            x, y = a.clone(), w.clone()
+            (x if side == "a" else y)[at] = row.cuda()
+            got = ops.gemm_generic(x, y, residual=residual)
+            rest = lambda t: torch.cat([t[:at], t[at + 1:]]) if side == "a" else torch.cat([t[:, :at], t[:, at + 1:]], 1)  # noqa: E731
+            assert torch.equal(rest(got), rest(before))
+            own = got[at].double() if side == "a" else got[:, at].double()
+            other, beside = (w, residual[at]) if side == "a" else (a, residual[:, at])
+            want = other.double() @ row.cuda().double() + beside.double()
+            if bool(torch.isfinite(row).all()):
+                assert bool(((own - want).abs() <= (k + 2) * 2.0 ** -24 * (other.double().abs() @ row.cuda().double().abs() + beside.double().abs())).all())
+            else:
+                assert torch.equal(own.isnan(), want.isnan()) and torch.equal(own[~own.isnan()], want[~want.isnan()])
+
+
 def test_many_products_whose_pieces_lose_a_little():
     """65,536 numbers of 2^-125 beside some of up to 2^39 and one product of 2^-59 behind them: what their pieces lose is little of a product and 2^-20 of the sum."""
     g = torch.Generator(device="cuda").manual_seed(4)

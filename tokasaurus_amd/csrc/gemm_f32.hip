@@ -43,8 +43,8 @@ struct GemmF32Args {
   float* part;  // [cuts][M][N] sums of K's parts, or null: one part, finished here
 };
 
-// bias and residual, and the store of four neighbouring outputs of a token
-__device__ __forceinline__ void gf_store(const GemmF32Args& a, f4 v, int token, int n) {
+// bias and residual, and the store of four neighbouring outputs of a token (of those whose bit in `only` is set)
+__device__ __forceinline__ void gf_store(const GemmF32Args& a, f4 v, int token, int n, int only = 15) {
   float* c = a.C + (size_t)token * a.ldc + n;
   float o[4];
 #pragma unroll
@@ -55,12 +55,12 @@ __device__ __forceinline__ void gf_store(const GemmF32Args& a, f4 v, int token, 
       if (a.residual) o[j] += a.residual[(size_t)token * a.ldr + n + j];
     }
   }
-  if (n + 3 < a.N && ((uintptr_t)c & 15) == 0) {
+  if (only == 15 && n + 3 < a.N && ((uintptr_t)c & 15) == 0) {
     *(f4*)c = (f4){o[0], o[1], o[2], o[3]};
   } else {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (n + j < a.N) c[j] = o[j];
+      if (n + j < a.N && (only >> j & 1)) c[j] = o[j];
   }
 }
 
@@ -244,9 +244,10 @@ __global__ __launch_bounds__(512) void gemm_f32_few_kernel(GemmF32Args a, FewExt
   }
 }
 
-// The chains of a tile's sums added, and the results stored, or the part of K among the other parts' sums.
-template <int TM, int TN, int CHAINS>
-__device__ __forceinline__ void gf_finish(const GemmF32Args& a, f4 (&acc)[CHAINS][TN][TM], int m0, int n0, int wave, int r, int q) {
+// The chains of a tile's sums added, and the results stored, or the part of K among the other parts' sums.  MASKED: of this lane's 4 TN TM
+// results only those whose bit (t, u, j) in `only` is set.
+template <int TM, int TN, int CHAINS, bool MASKED = false>
+__device__ __forceinline__ void gf_finish(const GemmF32Args& a, f4 (&acc)[CHAINS][TN][TM], int m0, int n0, int wave, int r, int q, uint64_t only = 0) {
 #pragma unroll
   for (int half = CHAINS / 2; half > 0; half /= 2)
 #pragma unroll
@@ -263,10 +264,19 @@ __device__ __forceinline__ void gf_finish(const GemmF32Args& a, f4 (&acc)[CHAINS
     for (int t = 0; t < TN; ++t) {
       const int n = n0 + (wave & 1) * 16 * TN + 16 * t + 4 * q;
       if (n >= a.N) continue;
+      const int some = MASKED ? (int)(only >> (4 * (t * TM + u))) & 15 : 15;
+      if (MASKED && some == 0) continue;
       if (a.part) {  // (N is a multiple of 4 then)
-        *(f4*)(a.part + ((size_t)blockIdx.y * a.M + token) * a.N + n) = acc[0][t][u];
+        float* part = a.part + ((size_t)blockIdx.y * a.M + token) * a.N + n;
+        if (!MASKED) {
+          *(f4*)part = acc[0][t][u];
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (some >> j & 1) part[j] = acc[0][t][u][j];
+        }
       } else {
-        gf_store(a, acc[0][t][u], token, n);
+        gf_store(a, acc[0][t][u], token, n, some);
       }
     }
   }
@@ -444,9 +454,11 @@ __global__ __launch_bounds__(256) void gemm_f32_stream_kernel(GemmF32Args a) {
 // are not larger than the unsplit products', from one term a row to dense rows (below).
 // Eight instructions of 16 x 16 x 32 take 136 cycles where eight of 16 x 16 x 4 take 272; the pieces, made by every wavefront for itself, cost nearly as
 // much as the products, side by side with them where two workgroups share a compute unit.
-// Pieces reach down to 2^-133, and an infinite number has pieces that are no numbers: a workgroup with a sum that is not finite, or below GP_LEAST
-// (zero too: numbers of less than 2^-133 have no pieces at all), or with an operand of GP_MOST and more, does its products again, unsplit.  (Else the
-// bits below 2^-133 that are lost are at most 2^-102 of each of the K products, K 2^-52 of a sum, and a row of zeros costs its tiles their time twice.)
+// Pieces reach down to 2^-133, and an infinite number has pieces that are no numbers: results that are not finite, or below GP_LEAST (zero too:
+// numbers of less than 2^-133 have no pieces at all), or of a row of A or W with an operand of GP_MOST and more, are made again, unsplit, by the
+// workgroup that has them.  Else the bits below 2^-133 that are lost are at most 2^-102 of each of the K products, K 2^-52 of a result.  Which
+// way a result is made depends on its own two rows alone, not on what else is in its tile (so a row of zeros costs its tiles their time
+// twice, and changes no other row).
 // Two wavefronts make the pieces of the same rows: each looks at half a step's numbers, which the other has last (16 instructions of some 370 a
 // step; 301 rows 16,384 x 2,048 151.9 us without, 152.1 with, 2,048 rows 697 and 700).
 // us unsplit / split, weights from memory:
@@ -566,7 +578,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) 
     }
   };
   walk(std::integral_constant<bool, false>{});
-  bool plain = most < GP_MOST;
+  // which results go unsplit: a bit each
+  uint64_t again = 0;
 #pragma unroll
   for (int t = 0; t < TN; ++t)
 #pragma unroll
@@ -575,11 +588,40 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_pieces_kernel(GemmF32Args a) 
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float size = fabsf(acc[0][t][u][j]);
-        plain = plain && size >= GP_LEAST && size < INFINITY;
+        again |= (uint64_t)!(size >= GP_LEAST && size < INFINITY) << (4 * (t * TM + u) + j);
       }
     }
-  if (__syncthreads_or(!plain)) walk(std::integral_constant<bool, true>{});
-  gf_finish<TM, TN, 1>(a, acc, m0, n0, wave, r, q);
+  const bool large = !(most < GP_MOST);
+  if (!__syncthreads_or(large || again != 0)) {
+    gf_finish<TM, TN, 1>(a, acc, m0, n0, wave, r, q);
+    return;
+  }
+  if (__syncthreads_or(large)) {
+    // the rows with such operands, a thread a row (none is read behind its cut of K)
+    if (tid < ROWS) {
+      const float* row = tid < 32 * TN ? a.W + (size_t)min(n0 + tid, a.N - 1) * a.K : a.A + (size_t)min(m0 + tid - 32 * TN, a.M - 1) * a.lda;
+      float top = 0.f;
+      for (int k = s0 * 32; k < (s0 + steps) * 32; k += 4) {
+        const f4 v = *(const f4*)(row + k);
+        top = fmaxf(fmaxf(fmaxf(top, fabsf(v[0])), fmaxf(fabsf(v[1]), fabsf(v[2]))), fabsf(v[3]));
+      }
+      tile[tid] = top;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+      for (int u = 0; u < TM; ++u)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float top = fmaxf(tile[(wave & 1) * 16 * TN + 16 * t + 4 * q + j], tile[32 * TN + (wave >> 1) * 16 * TM + 16 * u + r]);
+          again |= (uint64_t)!(top < GP_MOST) << (4 * (t * TM + u) + j);
+        }
+    __syncthreads();
+  }
+  gf_finish<TM, TN, 1, true>(a, acc, m0, n0, wave, r, q, ~again);
+  walk(std::integral_constant<bool, true>{});
+  gf_finish<TM, TN, 1, true>(a, acc, m0, n0, wave, r, q, again);
 }
 
 // The sums of K's parts added in the order of K: a thread four neighbouring outputs.
