@@ -7,4 +7,3 @@
 
 __device__ __forceinline__ float silu_f32(float x) { return x / (1.0f + expf(-x)); }
 __device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + expf(-x)); }
-__device__ __forceinline__ float softplus_f32(float x) { return fmaxf(x, 0.f) + log1p_exp(x); }

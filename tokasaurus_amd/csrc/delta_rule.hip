@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(
     const float rate = expf(a_log[h]);
     for (int i = lane; i < dk; i += TK_WAVE) {
       const int x = h * dk + i;
-      out[decay_off + x] = expf(-rate * softplus_f32(a_pre[(size_t)t * ld_a + x] + dt_bias[x]));
+      out[decay_off + x] = expf(-rate * softplus(a_pre[(size_t)t * ld_a + x] + dt_bias[x]));
     }
   } else {
     for (int i = lane; i < H; i += TK_WAVE)
@@ -399,7 +399,7 @@ __global__ __launch_bounds__(DS_THREADS) void delta_single_kernel(DeltaSingleArg
     } else if (c < conv + dk) {
       const int x = c - conv;
       const float rate = expf(a.a_log[h]);
-      gs[x] = expf(-rate * softplus_f32(a.a_pre[(size_t)t * a.ld_a + h * dk + x] + a.dt_bias[h * dk + x]));
+      gs[x] = expf(-rate * softplus(a.a_pre[(size_t)t * a.ld_a + h * dk + x] + a.dt_bias[h * dk + x]));
     } else {
       beta = sigmoid_f32(to_f32<T>(x_row[a.col_b + h]));
     }

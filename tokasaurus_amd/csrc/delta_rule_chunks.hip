@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256, 4) void delta_chunk_factors_kernel(DeltaChunkA
 #pragma unroll
   for (int u = 0; u < DECAYS; ++u) {
     const int i = u * 256 + tid;
-    gs[i] = i / DKP < n && i % DKP < dk ? expf(-rate * softplus_f32(z[u])) : 1.f;
+    gs[i] = i / DKP < n && i % DKP < dk ? expf(-rate * softplus(z[u])) : 1.f;
   }
   if (tid < DC_CHUNK) beta[tid] = tid < n ? sigmoid_f32(to_f32<T>(proj[(size_t)(row0 + tid) * a.ld + a.col_b + h])) : 0.f;
   __syncthreads();

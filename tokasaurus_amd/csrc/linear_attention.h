@@ -36,7 +36,7 @@ __device__ __forceinline__ float la_silu(float x) { return x / (1.0f + expf(-x))
 __device__ __forceinline__ float la_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 // the forget gate, written out in one multiply-add so that every kernel that computes it gets the same bits
 __device__ __forceinline__ float la_forget(float x, float bias, float lo) { return fmaf(1.0f - lo, la_sigmoid(x + bias), lo); }
-__device__ __forceinline__ float la_log_sigmoid(float x) { return fminf(x, 0.f) - log1p_exp(x); }
+__device__ __forceinline__ float la_log_sigmoid(float x) { return -softplus(-x); }
 __device__ __forceinline__ float la_channel_decay(float z, float tau) { return expf(la_log_sigmoid(z) / tau); }
 __device__ __forceinline__ float la_soft_cap(float x, float cap) { return cap * tanhf(x / cap); }
 
