@@ -63,12 +63,12 @@ __device__ __forceinline__ void rotate_pair(float x1, float x2, float c, float s
 
 // log(1 + exp(x)), also -(logarithm of a sigmoid) of -x: max(x, 0) + log(1 + y) with y = exp(-|x|) <= 1.  log(1 + y) is log 2 (or 0, y below a half) and
 // f - f^2 / 2 + f^3 q(f) of f = (y - 1) / 2 (or y), with q of the least greatest error on [-1/4, 1/2], 9e-10 of the result.  The greater terms are
-// added with what each sum leaves, so that one rounding remains.  Some 55 instructions where log1pf(expf()) takes 150, in kernels bound by
+// added with what each sum leaves, so that one rounding remains.  Some 50 instructions where log1pf(expf()) takes 150, in kernels bound by
 // them: the first kernel of the delta rule in chunks took 80 us for prompts of 562 and 938 tokens with 35 of them, their parts added plainly, and 87 with log1pf; the call of
-// those prompts takes the same with 55 as with 35 (2,983 us).  Errors from 64 bits, root mean square (largest), with
-// log1pf(expf(x)) / so: |x| <= 12 1.291e-7 (5.54e-7) / 1.279e-7 (4.77e-7), |x| <= 2 2.93e-8 (1.67e-7) / 2.67e-8 (1.30e-7), in [-1, 0] 1.610e-8 (5.78e-8) / 1.616e-8
-// (5.75e-8), the rest there being expf's; of a logarithm of a sigmoid over |x| <= 2 2.94e-8 (1.36e-7) / 2.67e-8 (1.30e-7); of decays exp(-softplus) 1.356e-8 / 1.349e-8
-// over |x| <= 12, 1.638e-8 / 1.608e-8 over |x| <= 2.
+// those prompts takes the same with 50 as with 35 (2,983 us).  Errors from 64 bits, root mean square (largest), with
+// log1pf(expf(x)) / so: |x| <= 12 1.291e-7 (5.54e-7) / 1.279e-7 (4.77e-7), |x| <= 2 2.93e-8 (1.67e-7) / 2.66e-8 (1.29e-7), in [-1, 0] 1.610e-8 (5.78e-8) / 1.610e-8
+// (5.75e-8), the rest there being expf's; of a logarithm of a sigmoid over |x| <= 2 2.94e-8 (1.36e-7) / 2.66e-8 (1.29e-7); of decays exp(-softplus) 1.356e-8 / 1.349e-8
+// over |x| <= 12, 1.638e-8 / 1.607e-8 over |x| <= 2.
 __device__ __forceinline__ float softplus(float x) {
   const float y = expf(-fabsf(x));
   const bool upper = y >= 0.5f;
@@ -83,10 +83,9 @@ __device__ __forceinline__ float softplus(float x) {
   q = fmaf(q, f, 0.19999605f);
   q = fmaf(q, f, -0.25000164f);
   q = fmaf(q, f, 0.3333334f);
-  const float h = -0.5f * f, p = h * f, p_left = fmaf(h, f, -p);
-  const float s = log2_hi + f, s_left = f - (s - log2_hi);
-  const float l = s + p, l_left = p - (l - s);
-  const float left = fmaf(f * f, f * q, (s_left + l_left) + (p_left + log2_lo));
+  const float h = -0.5f * f, s = log2_hi + f, s_left = f - (s - log2_hi);
+  const float l = fmaf(h, f, s), l_left = fmaf(h, f, s - l);
+  const float left = fmaf(f * f, f * q, (s_left + l_left) + log2_lo);
   const float line = fmaxf(x, 0.f), hi = fmaxf(line, l), lo = fminf(line, l), t = hi + lo;
   return t + ((hi < 64.f ? lo - (t - hi) : 0.f) + left);  // (no difference of infinities)
 }
