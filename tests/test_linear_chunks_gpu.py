@@ -49,3 +49,23 @@ def test_chunks_follow_the_recurrence(heads, dk, dv, lengths, memory):
     # 2^-24 of up to 64), a product of as many factors in the other
     assert rel(o, want_o) <= 64 * 2.0 ** -24 and rel(state[1:], want_state[1:]) <= 64 * 2.0 ** -24
     assert torch.equal(state[0], before[0])
+
+
+@pytest.mark.parametrize("tau", [5.0, 15.0, 16.0])
+def test_a_quotient_by_tau_is_not_off_to_one_side(tau):
+    """One token's key and value behind 63 decays of a channel: the state is exp(63 log(sigmoid(bias)) / tau)."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    heads, dk, dv, n = 8, 256, 16, 64
+    off = heads * (2 * dk + dv)
+    proj = torch.zeros((n, off + 16), device="cuda")
+    proj[0, heads * dk: off] = 1
+    bias = torch.rand((heads * dk,), generator=g, device="cuda") * 2 - 1
+    state = torch.zeros((2, ops.linear_attention_state_words(heads, dk, dv, False)), device="cuda")
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    ops.gated_linear_attention(proj, 0, heads * dk, 2 * heads * dk, off, torch.zeros((16, heads * dk), device="cuda"), bias, tau, 1.0, state, i32([0, n]), i32([1]),
+                               heads, dk, dv, n, chunks=plan([n]))
+    got, log_a = state[1].view(heads, dv, dk)[:, 0].double(), 63 * torch.nn.functional.logsigmoid(bias.double()).view(heads, dk) / tau
+    off_by = (torch.log(got) - log_a) / log_a
+    # the mean of 2,048 channels' errors, each a sum's of 64 terms and an exponential's (a few 2^-24 of the logarithm): a third of a rounding, where the
+    # quotient rounded once is off by up to 2^-24
+    assert abs(float(off_by.mean())) <= 2.0 ** -24 / 3

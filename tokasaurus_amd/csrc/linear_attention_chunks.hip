@@ -153,10 +153,12 @@ __global__ __launch_bounds__(256) void la_chunk_factors_kernel(LaArgs a, int dkp
       }
       const float bias = in ? a.low_bias[x] : 0.f;
       float sum = 0.f;
-      const float per_tau = LC_LOG2E / a.tau;
+      const float per_tau = 1.f / a.tau;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        A[j] = la_log_sigmoid(A[j] + bias) * per_tau;
+        // the quotient by tau, corrected as a division does it (a product alone would be off to one side, 64 times over in a chunk's sum), then in units of log 2
+        const float x = la_log_sigmoid(A[j] + bias), y = x * per_tau;
+        A[j] = __builtin_amdgcn_div_fixupf(fmaf(fmaf(-y, a.tau, x), per_tau, y), a.tau, x) * LC_LOG2E;
         asm volatile("" : "+v"(A[j]));  // (all of them, side by side: no branch around each)
       }
 #pragma unroll
