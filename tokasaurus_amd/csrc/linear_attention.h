@@ -27,9 +27,9 @@ struct LaArgs {
   int o_head;
   int n_tokens, n_requests, H, dk, dv, longest;
   // LA_CHANNEL and LA_MEMORY in chunks (n_chunks > 0): every chunk's request and first row, in the requests' order, and every
-  // request's first chunk, [n_chunks], [n_chunks], [n_requests + 1]
+  // request's first chunk, [n_chunks], [n_chunks], [n_requests + 1]; n_singles requests have no chunk and bring one token
   const int *chunk_req, *chunk_row0, *first_chunk;
-  int n_chunks;
+  int n_chunks, n_singles;
 };
 
 __device__ __forceinline__ float la_silu(float x) { return x / (1.0f + expf(-x)); }
@@ -50,6 +50,8 @@ __device__ __forceinline__ size_t la_max_at(const LaArgs& a, int p, int h) {
 
 // The gates of LA_MEMORY (linear_attention.hip): gates[t][h] = (decay of the state, or its logarithm; factor on what is written).
 void la_launch_gates(const LaArgs& a, float2* gates, int log_decay, hipStream_t stream);
+// The requests of one token (linear_attention.hip): all of a step, or those without a chunk.
+void la_launch_singles(int mode, const LaArgs& a, hipStream_t stream);
 // The chunked form (linear_attention_chunks.hip): whether it takes these sizes, and the call itself.
 bool la_chunks_take(int mode, int dk, int longest);
 int la_run_chunks(int mode, const LaArgs& a, hipStream_t stream);

@@ -279,7 +279,7 @@ static int la_pieces(int dk) {
 }
 
 // --------------------------------------------------------------------------
-// The same for steps in which every request brings one token: the activations are computed by the lanes that need
+// The same for requests that bring one token, all of a step's or those that decode beside prompts in chunks: the activations are computed by the lanes that need
 // them (there is no pass in front and no `rec`), with the functions of the pass above, so the sums are the same bits (up to
 // the order of LA_CHANNEL's low-rank sums: a workgroup computes its head's decays into LDS).  LA_MEMORY: every lane computes its head's two gates.
 // --------------------------------------------------------------------------
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(LA_WAVES * TK_WAVE) void linear_attention_single_ke
   const int col = blockIdx.z * (blockDim.x / LA_LANES) + grp;
   const bool live = col < columns;
   const int t = a.q_start[r];
-  if (a.q_start[r + 1] <= t) return;
+  if (a.q_start[r + 1] <= t || (a.n_chunks > 0 && a.first_chunk[r] < a.first_chunk[r + 1])) return;
   if (MODE != LA_CHANNEL && (col / LA_COLS) * LA_COLS >= columns) return;
   float* slot = a.state + (size_t)a.slots[r] * a.state_stride;
   float* s_col = slot + ((size_t)h * columns + (live ? col : 0)) * dk;
@@ -415,20 +415,33 @@ void la_launch_gates(const LaArgs& a, float2* gates, int log_decay, hipStream_t 
 }
 
 template <int MODE>
+static void la_run_singles(const LaArgs& a, hipStream_t stream) {
+  const int all_waves = (la_columns<MODE>(a.dv) + LA_COLS - 1) / LA_COLS, waves = min(LA_WAVES, all_waves), nq = la_pieces(a.dk);
+  const dim3 grid(a.H, a.n_requests, (all_waves + waves - 1) / waves), block(waves * TK_WAVE);
+#define LA_SINGLE(NQ) hipLaunchKernelGGL((linear_attention_single_kernel<NQ, MODE>), grid, block, 0, stream, a, a.proj, a.o)
+  if (nq <= 1) LA_SINGLE(1);
+  else if (nq <= 2) LA_SINGLE(2);
+  else if (nq <= 3) LA_SINGLE(3);
+  else if (nq <= 4) LA_SINGLE(4);
+  else if (nq <= 6) LA_SINGLE(6);
+  else LA_SINGLE(8);
+#undef LA_SINGLE
+}
+void la_launch_singles(int mode, const LaArgs& a, hipStream_t stream) {
+  switch (mode) {
+    case LA_CONSTANT: return la_run_singles<LA_CONSTANT>(a, stream);
+    case LA_FORGET: return la_run_singles<LA_FORGET>(a, stream);
+    case LA_CHANNEL: return la_run_singles<LA_CHANNEL>(a, stream);
+    default: return la_run_singles<LA_MEMORY>(a, stream);
+  }
+}
+
+template <int MODE>
 static int la_run(const LaArgs& a, hipStream_t stream) {
   const int columns = la_columns<MODE>(a.dv), all_waves = (columns + LA_COLS - 1) / LA_COLS;
   const int nq = la_pieces(a.dk), dkp = 64 * nq;
   if (a.longest <= 1) {
-    const int waves = min(LA_WAVES, all_waves);
-    const dim3 grid(a.H, a.n_requests, (all_waves + waves - 1) / waves), block(waves * TK_WAVE);
-#define LA_SINGLE(NQ) hipLaunchKernelGGL((linear_attention_single_kernel<NQ, MODE>), grid, block, 0, stream, a, a.proj, a.o)
-    if (nq <= 1) LA_SINGLE(1);
-    else if (nq <= 2) LA_SINGLE(2);
-    else if (nq <= 3) LA_SINGLE(3);
-    else if (nq <= 4) LA_SINGLE(4);
-    else if (nq <= 6) LA_SINGLE(6);
-    else LA_SINGLE(8);
-#undef LA_SINGLE
+    la_run_singles<MODE>(a, stream);
     TK_CHECK_LAUNCH("linear_attention");
     return 0;
   }

@@ -457,6 +457,7 @@ static int lc_run(const LaArgs& a, hipStream_t stream) {
     gates = (float2*)(a.rec + (size_t)a.n_chunks * a.H * lc_words(dkp, blocks));
     la_launch_gates(a, gates, 1, stream);
   }
+  if (a.n_singles > 0) la_launch_singles(MODE, a, stream);
   hipLaunchKernelGGL(la_chunk_factors_kernel<MODE>, dim3(a.n_chunks, a.H), dim3(256), 0, stream, a, dkp, a.proj, gates, a.rec);
   hipLaunchKernelGGL(la_chunk_states_kernel<MODE>, dim3(a.H, a.n_requests, blocks * (dkp / 16)), dim3(TK_WAVE), 0, stream, a, dkp, a.rec);
   // blocks of columns a workgroup: as many as leave two workgroups for each of 256 compute units, one of which reads its block while

@@ -1663,6 +1663,7 @@ class _LinearAttentionArgs(ctypes.Structure):
         ("o", ctypes.c_void_p), ("floor", ctypes.c_void_p), ("o_head", ctypes.c_int), ("n_tokens", ctypes.c_int),
         ("n_requests", ctypes.c_int), ("H", ctypes.c_int), ("dk", ctypes.c_int), ("dv", ctypes.c_int), ("longest", ctypes.c_int),
         ("chunk_req", ctypes.c_void_p), ("chunk_row0", ctypes.c_void_p), ("first_chunk", ctypes.c_void_p), ("n_chunks", ctypes.c_int),
+        ("n_singles", ctypes.c_int),
     ]
 
 
@@ -1680,11 +1681,12 @@ def linear_attention_state_words(heads: int, key_dim: int, value_dim: int, memor
 class ChunkPlan:
     """A step's rows (those of the requests that go in chunks) cut into chunks of so many neighbouring tokens of one request
     (``linear_attention_chunk_tokens``, ``delta_chunk_tokens``), in the requests' order: every chunk's request and first row, and
-    every request's first chunk (and, last, the number of chunks), int32."""
+    every request's first chunk (and, last, the number of chunks), int32; and how many requests have none."""
 
     req: torch.Tensor
     row0: torch.Tensor
     first: torch.Tensor
+    without: int = 0
 
 
 def linear_attention_chunk_tokens() -> int:
@@ -1730,7 +1732,7 @@ def _linear_attention(mode: int, proj: torch.Tensor, q_off: int, k_off: int, v_o
             _need(n_chunks > 0 and chunks.row0.numel() == n_chunks and chunks.first.numel() == slots.numel() + 1,
                   "linear_attention: one request and one row a chunk, one first chunk a request")
             extra = dict(extra, chunk_req=chunks.req.data_ptr(), chunk_row0=chunks.row0.data_ptr(), first_chunk=chunks.first.data_ptr(),
-                         n_chunks=n_chunks)
+                         n_chunks=n_chunks, n_singles=chunks.without)
             work = n_chunks * chunk_words + (2 * n * H if mode == LA_MEMORY else 0)
         else:
             work = n * load("core").tk_linear_attention_work_words(mode, H, dk, dv, longest)
