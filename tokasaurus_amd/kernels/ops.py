@@ -1457,7 +1457,8 @@ TILE_SHAPES = ((128, 128, 0.47, 4.3), (192, 128, 0.54, 6.5), (128, 256, 0.79, 5.
 TILES_LONGEST_STRIDE = 1 << 22  # elements between rows of x (a tile's rows lie within 32-bit bytes of its first)
 PLAIN_TILES_FROM_ROWS = 129  # (where the fit begins)
 GLU_TILES_FROM_ROWS = 65  # (up to 64 rows gate and up stream through local memory)
-# two rounds of tiles of 192 x 256: with more the chip's power bounds the step, and the library's kernel needs less of it
+# two rounds of tiles of 192 x 256: with more the chip's power bounds the step, and the library's kernel needs less of it (the line of the
+# activation by expf and a division; by the hardware's reciprocal the tiles are ahead up to two rounds of 256 x 256, see the figures below)
 GLU_TILES_MOST_SUMS = 2 * 256 * 192 * 256
 GLU_TILES_LATER_FILL = 0.95  # how much of its rounds a product fills that takes more than one
 
@@ -1468,17 +1469,19 @@ def tiles_choice(m: int, n: int, k: int, glu: bool = False) -> int:
     -1: the library's product is faster.
 
     In the gated form the tiles save the pass behind the library's product; they pay where they fill four fifths of one round of
-    the compute units, or further rounds whole, up to ``GLU_TILES_MOST_SUMS``.  us library and pass / tiles, weights from memory: 16,384 x 2,048 33.5 / 26.4 at 256 rows, 41.7 / 37.7 at 512, 70.1 /
-    61.3 at 1,024, 98.7 / 94.9 at 1,500, 117 / 120 at 2,048; 16,384 x 3,072 45.1 / 37.8 at 256, 92.0 / 81.6 at 1,024, 172 / 165 at 2,048;
-    28,672 x 4,096 105 / 102 at 512, 204 / 194 at 1,024 (fill 0.73: 262 / 279 at 1,280).  In whole steps, where power counts, us a layer that
-    tiles save on two machines: one round, 16,384 x 2,048 15 and 16 at 512 rows, 16,384 x 3,072 9 and 5 at 1,024, 28,672 x 4,096 9 and 3 at 512;
-    two rounds filled whole, 16,384 x 2,048 -0.4 and 1.0 at 1,408, -1.2 and 2.9 at 1,536 (in another model 7 and 7), but -1.7 and -5.6 at
-    2,048; filled to 0.88, 16,384 x 2,048 -6.2 and -8.9 at 1,280, -5.9 and -9.4 at 1,664, 28,672 x 4,096 -13 and -18 at 640, -4.4 and -9.2 at 896.
-    Up to 128 rows, at 65 and 128: tiles of 64 weight rows where one round holds them, 16,384 x 2,048 21.7 / 19.1 and 23.9 / 20.9 (of 128
-    weight rows, half of the units, 23.1 and 26.7), 16,384 x 3,072 29.0 / 25.9 and 30.5 / 29.3, 16,384 x 8,192 66.7 / 62.8 and 68.7 / 66.1; wider
-    weights tiles of 128, which there pay from two thirds of the units on, 22,016 x 2,048 27.5 / 24.9 and 29.9 / 28.0, 22,016 x 4,096 46.9 / 44.9
-    and 47.1 / 48.0, 24,576 x 4,096 51.9 / 45.7 and 50.6 / 48.8, 28,672 x 4,096 58.6 / 55.2 and 57.6 / 56.2 (20,480 x 2,560, fill 0.63, 36.4 / 36.1
-    and 34.6 / 37.5).
+    the compute units, or further rounds whole, up to ``GLU_TILES_MOST_SUMS``.  us library and pass / tiles, weights from memory: 16,384 x 2,048
+    35.0 / 26.9 at 256 rows, 43.0 / 36.3 at 512, 67.6 / 60.0 at 1,024, 101 / 89.6 at 1,500, 120 / 117 at 2,048, 227 / 230 at 4,096; 16,384 x 3,072
+    47.3 / 38.2 at 256, 92.8 / 86.0 at 1,024, 169 / 161 at 2,048; 28,672 x 4,096 110 / 104 at 512, 204 / 196 at 1,024 (fill 0.73: 264 / 274 at 1,280).
+    In whole steps, where power counts, us a layer that tiles save on two machines: one round, 16,384 x 2,048 6.5 and 6.4 at 512 rows, 7.4 and
+    5.7 at 1,024, 16,384 x 3,072 15 and 16 at 1,024, 28,672 x 4,096 9.2 and 9.5 at 512; two rounds filled whole, 16,384 x 2,048 6.9 and 6.3 at 1,408, 8.7 and
+    8.5 at 1,536; filled to 0.88, 16,384 x 2,048 3.0 and 1.9 at 1,280, 1.1 and -0.2 at 1,664, 28,672 x 4,096 -11 and -11 at 640, 4.9 and 4.6 at 896.
+    Beyond ``GLU_TILES_MOST_SUMS`` two rounds of 256 x 256 would save too, 3.9 and 5.5 at 2,048 rows of 16,384 x 2,048, 13 and 16 of 16,384 x 3,072, 9.1 and
+    7.8 at 1,024 of 28,672 x 4,096; four rounds 6.5 and 8.2 at 4,096 of 16,384 x 2,048, but of 28,672 x 4,096 at 2,048 rows the library's is ahead by 16.  (The
+    line was drawn with an activation of 25 instructions in the tiles' kernel, whose tiles lost 1.7 and 5.6 at 2,048 rows of 16,384 x 2,048.)
+    Up to 128 rows, at 65 and 128: tiles of 64 weight rows where one round holds them, 16,384 x 2,048 22.8 / 19.0 and 25.1 / 21.3,
+    16,384 x 3,072 28.9 / 24.6 and 33.0 / 29.7, 16,384 x 8,192 68.7 / 61.9 and 73.4 / 68.9; wider weights tiles of 128, which there pay from two
+    thirds of the units on, 22,016 x 2,048 29.7 / 25.8 and 32.4 / 29.2, 22,016 x 4,096 51.1 / 45.7 and 52.5 / 52.6, 24,576 x 4,096 55.9 / 48.5 and 57.6 / 55.0,
+    28,672 x 4,096 61.0 / 54.6 and 62.4 / 58.3 (20,480 x 2,560, fill 0.63, 35.1 / 33.7 and 36.7 / 37.2).
     A plain product in tiles is ahead of the library's where one round of tiles of 128 outputs fills the chip and the library's
     larger tiles do not, from 129 rows on (below the two are even, 32,000 x 2,048 31.6 / 32.6 at 96 rows, 28,672 x 4,096 54.3 / 55.2 and 27,648
     x 1,024 17.8 / 16.9 at 128, and steps are the library's): 3,072 x 8,192 71.8 / 65.0 at 1,280 rows, 90.4 / 78.9 at 1,792; 5,120 x 3,072 40.1 / 35.2 at 1,024; 4,096 x 4,096
