@@ -6,8 +6,9 @@ may be stacked along the output rows into one product (q|k|v, gate|up).  The bia
 to the 32-bit sums, before the product is rounded.
 
 Which kernel runs is decided by the storage type and the number of rows:
-  * float32: 32-bit multiply-adds throughout (the true 32-bit path), on the matrix cores where the sizes fit them; up to 16
-    rows (``ops.gemm_f32_few``) with the activation, or the rotation and append, in the same kernel;
+  * float32: products and sums of all 24 bits (the true 32-bit path), on the matrix cores where the sizes fit them: 32-bit
+    multiply-adds, or for many rows products of each number's three exact bfloat16 pieces with 32-bit sums, whose errors are not larger;
+    up to 16 rows (``ops.gemm_f32_few``) with the activation, or the rotation and append, in the same kernel;
   * bfloat16, few rows (decode; how many depends on the inner size, ``ops.skinny_rows``, and ``ops.glu_rows`` for gate and
     up): the hand-written matrix-core kernels that stream the weight once and fuses the epilogue; it can also fold in the
     norm in front (``Normed`` input), leave what the norm behind it needs
